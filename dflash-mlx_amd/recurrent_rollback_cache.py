@@ -177,19 +177,12 @@ class RecurrentRollbackCache:
 
     def clear_transients(self) -> None:
         self._armed = False
-        self._tape = None
-        self._tape_k = None
-        self._tape_g = None
-        self._tape_qkv = None
-        self._snapshot = None
+        self._tape = self._tape_k = self._tape_g = self._tape_qkv = self._snapshot = None
 
     def arm_rollback(self, prefix_len: int = 0) -> None:
         del prefix_len
         self._armed = True
-        self._tape = None
-        self._tape_k = None
-        self._tape_g = None
-        self._tape_qkv = None
+        self._tape = self._tape_k = self._tape_g = self._tape_qkv = None
         self.checkpoint()
 
     def record_tape(self, *, tape: torch.Tensor, k: torch.Tensor, g: torch.Tensor,
@@ -322,22 +315,27 @@ class RollbackArena:
         self.g = torch.zeros(gshape, dtype=g_dtype, device=dev)
         self.qkv = torch.zeros((L, B, T, self.C), dtype=qkv_dtype, device=dev)
         self.steps = torch.zeros((L * B,), dtype=torch.int32, device=dev)
+        # The views the per-layer calls hand out and compare against, made once: indexing a tensor
+        # costs the host 2-3 us, and a rollback of 48 layers made about 700 of them (0.85 of its
+        # 0.90 ms; the launch itself is 42 us).
+        self._state_half = [[self.state[h, layer] for layer in range(L)] for h in (0, 1)]
+        self._conv_half = [[self.conv[h, layer] for layer in range(L)] for h in (0, 1)]
+        self._slots = [(self.tape[layer], self.k[layer], self.g[layer], self.qkv[layer]) for layer in range(L)]
         self._caches: List[RecurrentRollbackCache] = []
         for layer in range(L):
             c = RecurrentRollbackCache(size=2, conv_kernel_size=conv_kernel_size)
             c._arena, c._layer = self, layer
-            c.cache = [self.conv[0, layer], self.state[0, layer]]
+            c.cache = [self._conv_half[0][layer], self._state_half[0][layer]]
             self._caches.append(c)
 
     def caches(self) -> List[RecurrentRollbackCache]:
         return list(self._caches)
 
     @staticmethod
-    def _half_of(buf: torch.Tensor, layer: int, t: Optional[torch.Tensor]) -> int:
+    def _half_of(halves: List[List[torch.Tensor]], layer: int, t: Optional[torch.Tensor]) -> int:
         """Which half of a double buffer tensor ``t`` is (0 when it is in neither)."""
-        if t is not None and t.data_ptr() == buf[1, layer].data_ptr():
-            return 1
-        return 0
+        other = halves[1][layer]
+        return 1 if t is other or (t is not None and t.data_ptr() == other.data_ptr()) else 0
 
     def _reference_entry(self, layer: int, idx: int) -> Optional[torch.Tensor]:
         c = self._caches[layer]
@@ -347,24 +345,26 @@ class RollbackArena:
     def next_state(self, layer: int) -> torch.Tensor:
         """Where a verify forward of ``layer`` should write its new state: the half of the
         double buffer that does not hold the snapshot (or, un-armed, the current state)."""
-        return self.state[1 - self._half_of(self.state, layer, self._reference_entry(layer, 1)), layer]
+        return self._state_half[1 - self._half_of(self._state_half, layer, self._reference_entry(layer, 1))][layer]
 
     def next_conv(self, layer: int) -> torch.Tensor:
-        return self.conv[1 - self._half_of(self.conv, layer, self._reference_entry(layer, 0)), layer]
+        return self._conv_half[1 - self._half_of(self._conv_half, layer, self._reference_entry(layer, 0))][layer]
 
     def tape_slots(self, layer: int):
         """Views a tape producer may fill in place: (tape, k, g, qkv) of ``layer``."""
-        return self.tape[layer], self.k[layer], self.g[layer], self.qkv[layer]
+        return self._slots[layer]
 
     # -- used by the per-layer cache objects
     def _store_tape(self, layer: int, tape, k, g, qkv):
-        dst = self.tape_slots(layer)
+        dst = self._slots[layer]
+        if tape is dst[0] and k is dst[1] and g is dst[2] and qkv is dst[3]:
+            return dst  # the producer wrote into the arena: nothing to copy, no view to make
         out = []
         for d, src, name in zip(dst, (tape, k, g, qkv), ("tape", "k", "g", "qkv")):
             steps = int(src.shape[1])
             if steps > self.T:
                 raise ValueError(f"{name} has {steps} steps, arena holds {self.T}")
-            view = d[:, :steps]
+            view = d if steps == self.T else d[:, :steps]
             if src.data_ptr() != view.data_ptr() or src.dtype != d.dtype:
                 view.copy_(src)  # converts when the producer's dtype is not the arena's
             out.append(view)
@@ -374,8 +374,9 @@ class RollbackArena:
         return self.next_conv(layer)
 
     def _replay_layer(self, layer: int, state_in: torch.Tensor, steps: int) -> torch.Tensor:
-        out = self.state[1 - self._half_of(self.state, layer, state_in), layer]
-        replay_launch(self.tape[layer], self.k[layer], self.g[layer], state_in.contiguous(), out,
+        out = self._state_half[1 - self._half_of(self._state_half, layer, state_in)][layer]
+        tape, k, g, _ = self._slots[layer]
+        replay_launch(tape, k, g, state_in.contiguous(), out,
                       steps=steps, T_alloc=self.T, slots=self.B)
         return out
 
@@ -387,6 +388,9 @@ class RollbackArena:
     def _uniform_snapshot_half(self) -> Optional[int]:
         """Half (0/1) holding every layer's snapshot state and conv window, or None when
         the layers disagree, a snapshot or tape is missing, or a tensor is foreign."""
+        def same(a: torch.Tensor, b: torch.Tensor) -> bool:
+            return a is b or a.data_ptr() == b.data_ptr()
+
         half = None
         for layer, c in enumerate(self._caches):
             if c._snapshot is None or c._tape is None or c._tape_qkv is None:
@@ -394,12 +398,9 @@ class RollbackArena:
             conv, st = c._snapshot[0], c._snapshot[1]
             if st is None or conv is None:
                 return None
-            h = self._half_of(self.state, layer, st)
-            if st.data_ptr() != self.state[h, layer].data_ptr():
-                return None
-            if conv.data_ptr() != self.conv[h, layer].data_ptr():
-                return None
-            if c._tape.data_ptr() != self.tape[layer].data_ptr():
+            h = self._half_of(self._state_half, layer, st)
+            if not (same(st, self._state_half[h][layer]) and same(conv, self._conv_half[h][layer])
+                    and same(c._tape, self._slots[layer][0])):
                 return None
             if half is None:
                 half = h
@@ -447,5 +448,5 @@ class RollbackArena:
                       T_alloc=self.T, slots=self.L * self.B,
                       conv=(self.conv[snap], self.qkv, self.conv[nxt]) if self.keep > 0 else None)
         for layer, c in enumerate(self._caches):
-            c.cache = [self.conv[nxt, layer], self.state[nxt, layer]]
+            c.cache = [self._conv_half[nxt][layer], self._state_half[nxt][layer]]
             c.clear_transients()
