@@ -12,7 +12,7 @@ from typing import Optional
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libdflash_mi355.so")
 
-ABI_VERSION = 18
+ABI_VERSION = 19
 
 BF16, FP16, FP32 = 0, 1, 2
 QMM_MMA2BIG, QMM_MMA2BIG_PIPE = 0, 1
@@ -49,6 +49,8 @@ EXPORTED_SYMBOLS = (
     "dflash_qmm_m16_packed_bytes",
     "dflash_qmm_m16_pack",
     "dflash_qmm_m16_packed",
+    "dflash_qmm_rows_workspace_bytes",
+    "dflash_qmm_rows",
     "dflash_qmm_m16_gather_workspace_bytes",
     "dflash_qmm_m16_gather",
     "dflash_tape_replay",
@@ -102,6 +104,10 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.dflash_qmm_m16_pack_gate_up.argtypes = [c.c_void_p] * 6 + [c.c_int] * 3 + [c.c_void_p]
     lib.dflash_qmm_m16_packed.restype = c.c_int
     lib.dflash_qmm_m16_packed.argtypes = [c.c_void_p] * 6 + [c.c_size_t] + [c.c_int] * 5 + [c.c_void_p]
+    lib.dflash_qmm_rows_workspace_bytes.restype = c.c_size_t
+    lib.dflash_qmm_rows_workspace_bytes.argtypes = [c.c_int] * 4
+    lib.dflash_qmm_rows.restype = c.c_int
+    lib.dflash_qmm_rows.argtypes = [c.c_void_p] * 6 + [c.c_size_t] + [c.c_int] * 6 + [c.c_void_p]
     lib.dflash_qmm_m16_gather_workspace_bytes.restype = c.c_size_t
     lib.dflash_qmm_m16_gather_workspace_bytes.argtypes = [c.c_int] * 5
     lib.dflash_qmm_m16_gather.restype = c.c_int

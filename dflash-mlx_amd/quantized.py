@@ -63,9 +63,17 @@ def dequantize(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
 def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
                      *, transpose: bool = True, group_size: int = 64, bits: int = 4,
                      mode: str = "affine") -> torch.Tensor:
-    """Stock quantized matmul: dequantise to x.dtype, then an ordinary matmul."""
+    """Stock quantized matmul: dequantise to x.dtype, then an ordinary matmul - on the device in one
+    launch (``verify_qmm.rows_matmul``), else (host tensors, shapes it does not cover,
+    ``DFLASH_STOCK_KERNEL=0``) with array operators."""
     if mode != "affine":
         raise NotImplementedError(f"quantisation mode {mode!r}")
+    if transpose and x.is_cuda and os.environ.get("DFLASH_STOCK_KERNEL", "1") != "0":
+        from .verify_qmm import rows_matmul
+
+        y = rows_matmul(x, w, scales, biases, group_size=group_size, bits=bits)
+        if y is not None:
+            return y
     wd = dequantize(w, scales, biases, group_size, bits, dtype=x.dtype)
     return x @ (wd.transpose(-1, -2) if transpose else wd)
 

@@ -478,6 +478,47 @@ def small_m_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biase
     return y[:m].reshape(*x.shape[:-1], N)
 
 
+# Scratch of the any-rows product, one per (device, stream): 64 KiB of counters, then partial tiles.
+_ROWS_WORKSPACES: Dict[Tuple[int, int], torch.Tensor] = {}
+
+
+def rows_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
+                *, group_size: int = 64, bits: int = 4) -> "torch.Tensor | None":
+    """``x @ dequant(w).T`` for any number of rows of device activations in one launch
+    (``dflash_qmm_rows``): weights are dequantised to the activation type inside the product.
+    Returns None for what the kernel does not cover (other bit widths, fp32, N not a multiple of
+    16).  No counterpart in the reference, whose stock operator is ``mx.quantized_matmul``."""
+    if (not x.is_cuda or bits != 4 or group_size not in (32, 64, 128) or x.dtype not in _DTYPE_CODE or
+            scales.dtype not in _DTYPE_CODE or biases.dtype != scales.dtype or w.ndim != 2 or not _native.is_built()):
+        return None
+    K, N = int(x.shape[-1]), int(w.shape[0])
+    M = x.numel() // K if K else 0
+    if M < 1 or N % 16 != 0 or K % group_size != 0 or int(w.shape[1]) * 8 != K:
+        return None
+    w, scales, biases = w.contiguous(), scales.contiguous(), biases.contiguous()
+    _require_operands("quantized_matmul", K, N, group_size, w, scales, biases, x.device)
+    x2 = x.reshape(M, K).contiguous()
+    if (x2.data_ptr() | w.data_ptr()) % 16:
+        return None
+    lib = _native.lib()
+    y = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    stream = _native.raw_stream(x.device)
+    need = int(lib.dflash_qmm_rows_workspace_bytes(M, K, N, group_size))
+    ws_ptr, ws_bytes = None, 0
+    if need:
+        key = (x.device.index if x.device.index is not None else torch.cuda.current_device(), stream)
+        ws = _ROWS_WORKSPACES.get(key)
+        if ws is None or ws.numel() < need:
+            ws = torch.empty(max(need, 1 << 23), dtype=torch.uint8, device=x.device)
+            ws[:1 << 16].zero_()
+            _ROWS_WORKSPACES[key] = ws
+        ws_ptr, ws_bytes = ws.data_ptr(), ws.numel()
+    rc = lib.dflash_qmm_rows(x2.data_ptr(), w.data_ptr(), scales.data_ptr(), biases.data_ptr(), y.data_ptr(), ws_ptr,
+                             ws_bytes, M, K, N, group_size, _DTYPE_CODE[x.dtype], _DTYPE_CODE[scales.dtype], stream)
+    _native.check(rc, "dflash_qmm_rows")
+    return y.reshape(*x.shape[:-1], N)
+
+
 def gather_qmm(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
                expert_ids: torch.Tensor, *, group_size: int = 64, bits: int = 4) -> torch.Tensor:
     """Per-row expert selection for MoE layers: ``y[p] = x[p] @ dequant(w[expert_ids[p]]).T``.

@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define DFLASH_ABI_VERSION 18
+#define DFLASH_ABI_VERSION 19
 
 enum {
   DFLASH_OK = 0,
@@ -244,6 +244,23 @@ int dflash_qmm_m16_pack(const uint32_t* w_q, const void* scales, const void* bia
 int dflash_qmm_m16_packed(const void* x, const void* codes, const void* scales, const void* biases,
                           void* y, void* workspace, size_t workspace_bytes, int K, int N,
                           int group_size, int act_dtype, int sb_dtype, void* stream);
+
+/*
+ * The product for any number of rows: y[M,N] = x[M,K] . round(s*q + b)^T, weights rounded to act_dtype
+ * as an array-op dequantisation does, fp32 accumulation.  What the reference leaves to
+ * mx.quantized_matmul (dflash_mlx/verify_qmm.py:277-280, 300-304, 317-321): prompts and calls outside
+ * the verify gate.  Operands as for dflash_qmm_m16 with M rows of x and y.  Requirements: M >= 1,
+ * group_size in {32,64,128}, K % group_size == 0, N % 16 == 0; x, w_q 16-byte, y 8-byte aligned.
+ * workspace: dflash_qmm_rows_workspace_bytes(...) bytes (0: none needed), 256-byte aligned, its first
+ * 64 KiB zero-filled once by the caller and handed back zero-filled; the rest holds partial tiles and
+ * need not be cleared.  NOT shareable with the other qmm entry points' workspace.  Calls that share
+ * it must not overlap in time.  Deterministic.
+ */
+size_t dflash_qmm_rows_workspace_bytes(int M, int K, int N, int group_size);
+
+int dflash_qmm_rows(const void* x, const uint32_t* w_q, const void* scales, const void* biases, void* y,
+                    void* workspace, size_t workspace_bytes, int M, int K, int N, int group_size,
+                    int act_dtype, int sb_dtype, void* stream);
 
 /*
  * Gathered per-expert M<=16-per-expert qmm for MoE layers: y[p,:] = x[p,:] . (s*q + b)^T of

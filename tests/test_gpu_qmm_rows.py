@@ -1,0 +1,43 @@
+"""The any-rows 4-bit product (prompts, calls outside the verify gate) against its operands in fp64:
+tile edges in M, N and K, every group size, both activation types, split and whole tiles."""
+import pytest
+import torch
+
+from dflash_mlx_amd.quantized import dequantize, quantized_matmul
+from dflash_mlx_amd.verify_qmm import rows_matmul
+from dflash_mlx_amd.workloads import make_qmm_case
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("M,K,N,group,dtype", [
+    (1, 64, 16, 64, torch.bfloat16), (3, 32, 48, 32, torch.bfloat16), (17, 1024, 512, 64, torch.bfloat16),
+    (33, 96, 144, 32, torch.float16), (48, 320, 1040, 64, torch.bfloat16), (64, 384, 272, 128, torch.float16),
+    (65, 4096, 256, 64, torch.bfloat16), (77, 2048, 6144, 32, torch.bfloat16), (81, 128, 64, 128, torch.bfloat16),
+    (96, 1152, 528, 128, torch.bfloat16), (97, 640, 1296, 64, torch.float16), (112, 256, 16, 64, torch.bfloat16),
+    (127, 4352, 2048, 64, torch.bfloat16), (128, 1024, 256, 64, torch.bfloat16), (129, 512, 4112, 64, torch.bfloat16),
+    (300, 3072, 528, 32, torch.float16), (1024, 1280, 1040, 128, torch.bfloat16), (1500, 64, 4096, 64, torch.bfloat16),
+])
+def test_rows_against_fp64(native_lib, M, K, N, group, dtype):
+    c = make_qmm_case(K, N, 1000 + M, group_size=group, dtype=dtype, M=M).to(DEV)
+    y = rows_matmul(c.x, c.w, c.scales, c.biases, group_size=group)
+    assert y is not None and y.shape == (M, N) and y.dtype == dtype
+    assert torch.equal(y, quantized_matmul(c.x, c.w, c.scales, c.biases, group_size=group))  # and the same every time
+    dense = dequantize(c.w, c.scales, c.biases, group, 4, dtype=dtype).double()
+    exact = c.x.double() @ dense.t().contiguous()
+    # half a unit in the last place of the result (8 and 11 significant bits), and fp32 sums of K products of size |x||w|
+    eps = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    size = c.x.double().abs() @ dense.abs().t().contiguous()
+    # (q*s is exact in fp32, so both forms round the same weight: no term for it)
+    assert ((y.double() - exact).abs() <= 1.01 * eps * exact.abs() + size * 2.0 ** -24 * K ** 0.5 + 1e-6).all()
+    assert (y.double() - exact).norm() <= eps * exact.norm()
+
+
+def test_leading_dimensions_and_switch(native_lib, monkeypatch):
+    c = make_qmm_case(512, 96, 5, M=40).to(DEV)
+    y = quantized_matmul(c.x.reshape(2, 20, 512), c.w, c.scales, c.biases)
+    assert torch.equal(y.reshape(40, 96), quantized_matmul(c.x, c.w, c.scales, c.biases))
+    monkeypatch.setenv("DFLASH_STOCK_KERNEL", "0")
+    arrays = quantized_matmul(c.x, c.w, c.scales, c.biases)
+    assert (y.reshape(40, 96).float() - arrays.float()).norm() <= 2 ** -8 * arrays.float().norm()
