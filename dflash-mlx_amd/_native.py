@@ -56,6 +56,8 @@ EXPORTED_SYMBOLS = (
     "dflash_tape_replay",
     "dflash_gdn_forward_tape",
     "dflash_gdn_forward_tape_norm",
+    "dflash_gdn_forward_workspace_bytes",
+    "dflash_gdn_forward",
     "dflash_gdn_prepare",
     "dflash_gdn_gated_norm",
     "dflash_sdpa_q16_workspace_bytes",
@@ -118,6 +120,10 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.dflash_gdn_forward_tape.argtypes = [c.c_void_p] * 10 + [c.c_int] * 11 + [c.c_void_p]
     lib.dflash_gdn_forward_tape_norm.restype = c.c_int
     lib.dflash_gdn_forward_tape_norm.argtypes = [c.c_void_p] * 12 + [c.c_int] * 12 + [c.c_float, c.c_void_p]
+    lib.dflash_gdn_forward_workspace_bytes.restype = c.c_size_t
+    lib.dflash_gdn_forward_workspace_bytes.argtypes = [c.c_int] * 8
+    lib.dflash_gdn_forward.restype = c.c_int
+    lib.dflash_gdn_forward.argtypes = [c.c_void_p] * 13 + [c.c_size_t] + [c.c_int] * 12 + [c.c_float, c.c_void_p]
     lib.dflash_gdn_prepare.restype = c.c_int
     lib.dflash_gdn_prepare.argtypes = [c.c_void_p] * 14 + [c.c_int] * 9 + [c.c_float, c.c_void_p]
     lib.dflash_gdn_gated_norm.restype = c.c_int

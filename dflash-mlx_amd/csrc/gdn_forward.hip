@@ -29,7 +29,7 @@
 //    kernel keeps S / c with c = prod g, scales the two sums and delta instead, and
 //    multiplies c back in once at the end (renormalising if c gets very small).
 // q, k, v, g, beta of the block are staged once in LDS as fp32.
-#include "dflash_common.h"
+#include "gdn_device.h"
 #include <cstdlib>
 
 namespace dflash {
@@ -50,6 +50,7 @@ struct GdnArgs {
   const uint8_t* mask;
   int T, Hk, Hv, Dk, Dv;
   int in_dtype, g_dtype, beta_dtype, state_dtype, g_per_dk;
+  int staged;  // step-by-step kernel: steps staged in LDS at a time
   // gated output norm fused behind the recurrence (block kernel only): y is then
   // silu(z) * rms_norm(recurrence output, norm_weight), z laid out like y
   const void* z;
@@ -79,28 +80,27 @@ __device__ __forceinline__ float dot4(const f32x4_t& s, const float4& k) {
 }
 
 // ---------------------------------------------------------------------------
-// Dk = Dv = 128.  LDS (floats): sQ[T][128] | sK[T][128] | sV[T][128] | sG[T][128 or 1] |
-// sBeta[T] | sKQ[T].  FOLD: keep S / prod(g) instead of applying the decay (one gate per
+// Dk = Dv = 128.  The steps come through LDS in blocks of B = a.staged: (floats) sQ[B][128] |
+// sK[B][128] | sV[B][128] | sG[B][128 or 1] | sBeta[B] | sKQ[B].  FOLD: keep S / prod(g) instead of applying the decay (one gate per
 // head, fp32 state only).
 // ---------------------------------------------------------------------------
 template <bool VECG, bool FOLD>
 __global__ __launch_bounds__(kThreads) void gdn_forward_128(GdnArgs a) {
   static_assert(!(VECG && FOLD), "the folded decay needs one gate per head");
   extern __shared__ float smem[];
-  const int T = a.T;
+  const int staged = a.staged;
   float* sQ = smem;
-  float* sK = sQ + T * 128;
-  float* sV = sK + T * 128;
-  float* sG = sV + T * 128;
-  float* sBeta = sG + T * (VECG ? 128 : 1);
-  float* sKQ = sBeta + T;
+  float* sK = sQ + staged * 128;
+  float* sV = sK + staged * 128;
+  float* sG = sV + staged * 128;
+  float* sBeta = sG + staged * (VECG ? 128 : 1);
+  float* sKQ = sBeta + staged;
 
   const int slot = blockIdx.x / a.Hv, hv = blockIdx.x % a.Hv;
   const int hk = hv / (a.Hv / a.Hk);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int c3 = lane & 7;
   const int row0 = 32 * wave + 4 * (lane >> 3);  // this lane's rows: row0 .. row0 + 3
-  const size_t slotT = (size_t)slot * T;
   const bool f32_state = FOLD || a.state_dtype == DFLASH_FP32;
 
   // ---- state in: float4 columns c3 + 8c (c = 0..3) of 4 rows --------------------------------
@@ -123,6 +123,11 @@ __global__ __launch_bounds__(kThreads) void gdn_forward_128(GdnArgs a) {
                                     a.state_dtype);
   }
 
+  float cum = 1.f;  // FOLD: the registers hold S / cum
+  for (int first = 0; first < a.T; first += staged) {
+  const int T = a.T - first < staged ? a.T - first : staged;
+  const size_t slotT = (size_t)slot * a.T + first;
+  if (first > 0) __syncthreads();  // the block before has been read
   // ---- stage the block ---------------------------------------------------------------------
   for (int i = tid; i < T * 128; i += kThreads) {
     const int t = i >> 7, d = i & 127;
@@ -147,8 +152,7 @@ __global__ __launch_bounds__(kThreads) void gdn_forward_128(GdnArgs a) {
   }
   __syncthreads();
 
-  float cum = 1.f;  // FOLD: the registers hold S / cum
-  const size_t obase = (size_t)slot * T * a.Hv * 128 + (size_t)hv * 128;  // + t * Hv * 128 + dv
+  const size_t obase = slotT * a.Hv * 128 + (size_t)hv * 128;  // + t * Hv * 128 + dv
   for (int t = 0; t < T; ++t) {
     float delta[4], yv[4];
     const bool on = a.mask == nullptr || a.mask[slotT + t] != 0;
@@ -240,6 +244,7 @@ __global__ __launch_bounds__(kThreads) void gdn_forward_128(GdnArgs a) {
       store_from_f32(a.y, o, y_out, a.in_dtype);
     }
   }
+  }
 
   // ---- state out ----------------------------------------------------------------------------
   if (f32_state) {
@@ -326,39 +331,7 @@ __device__ __forceinline__ void store4_rounded(void* p, size_t i, f32x4_t v, int
     store4_from_f32(p, i, v, dt);
   }
 }
-// ---- exact products on the 16-bit matrix cores ---------------------------------------------
-// An fp32 value is the sum of three bf16 values (its leading 8 significant bits, the next 8 of
-// what is left, and the rest: 24 bits in all, each piece cut off, not rounded, so every
-// difference is exact), and a bf16 times a bf16 is exact in fp32.  A product of an fp32 matrix
-// with a matrix whose entries are bf16 numbers can therefore run as three passes of
-// v_mfma_f32_16x16x32_bf16 (9 ns for 32 steps of the sum) instead of eight of
-// v_mfma_f32_16x16x4_f32 (16 ns for 4 steps): the same products, summed in fp32 in another order.
 typedef __attribute__((ext_vector_type(4))) short s16x4_t;
-// the upper halves of a and b (a in the low half): two bf16 numbers, cut off
-__device__ __forceinline__ uint32_t upper_halves(float a, float b) {
-  return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
-}
-__device__ __forceinline__ float below_bf16(float v) {  // v minus its leading 8 significant bits
-  return v - __uint_as_float(__float_as_uint(v) & 0xffff0000u);
-}
-template <int N>
-struct Pieces {  // three bf16 pieces of N fp32 values, packed in pairs
-  uint32_t hi[N / 2], mid[N / 2], lo[N / 2];
-};
-template <int N>
-__device__ __forceinline__ Pieces<N> split_bf16(const float (&f)[N]) {
-  Pieces<N> p;
-  float r1[N], r2[N];
-#pragma unroll
-  for (int j = 0; j < N; ++j) r1[j] = below_bf16(f[j]), r2[j] = below_bf16(r1[j]);
-#pragma unroll
-  for (int j = 0; j < N / 2; ++j) {
-    p.hi[j] = upper_halves(f[2 * j], f[2 * j + 1]);
-    p.mid[j] = upper_halves(r1[2 * j], r1[2 * j + 1]);
-    p.lo[j] = upper_halves(r2[2 * j], r2[2 * j + 1]);
-  }
-  return p;
-}
 __device__ __forceinline__ f32x4_t mfma32_bf16(const uint32_t (&a)[4], const uint32_t (&b)[4], f32x4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, uint4{a[0], a[1], a[2], a[3]}),
                                                  __builtin_bit_cast(bf16x8_t, uint4{b[0], b[1], b[2], b[3]}), c, 0, 0, 0);
@@ -815,15 +788,27 @@ __global__ __launch_bounds__(kThreads) void gdn_forward_generic(GdnArgs a) {
 }  // namespace dflash
 
 namespace dflash {
+// gdn_prompt.hip
+bool gdn_prompt_covers(int slots, int T, int Hk, int Hv, int Dk, int Dv, int in_dtype, int g_per_dk);
+size_t gdn_prompt_workspace_bytes(int slots, int T, int Hk, int Hv, int Dk);
+int gdn_prompt_launch(const void* q, const void* k, const void* v, const void* g, const void* beta, const void* state_in,
+                      void* state_out, void* y, float* tape, const uint8_t* mask, void* workspace, int slots, int T, int Hk,
+                      int Hv, int Dk, int Dv, int g_dtype, int beta_dtype, int state_dtype, hipStream_t s);
+
 namespace {
 
-// Shared body of the two entry points; z == nullptr: no output norm.
+// Shared body of the entry points; z == nullptr: no output norm.
 int gdn_forward_launch(const char* who, const void* q, const void* k, const void* v, const void* g, const void* beta,
                        const void* state_in, void* state_out, void* y, float* tape, const uint8_t* mask,
                        const void* z, const void* norm_weight, int weight_dtype, float eps, int slots, int T, int Hk,
                        int Hv, int Dk, int Dv, int in_dtype, int g_dtype, int beta_dtype, int state_dtype,
-                       int g_per_dk, void* stream) {
-  DFLASH_REQUIRE(q && k && v && g && beta && state_in && state_out && y && tape, DFLASH_ERR_ARG, "%s: null operand", who);
+                       int g_per_dk, void* stream, void* workspace = nullptr, size_t workspace_bytes = 0) {
+  const bool aligned16 = (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)y | (uintptr_t)tape |
+                           (uintptr_t)z | (uintptr_t)norm_weight) % 16) == 0;
+  const bool no_chunk = option(DFLASH_OPT_GDN_STEP_BY_STEP) != 0;  // (tests of one kernel against the other)
+  const bool prompt = workspace != nullptr && aligned16 && !no_chunk && gdn_prompt_covers(slots, T, Hk, Hv, Dk, Dv, in_dtype, g_per_dk) &&
+                      (((uintptr_t)state_in | (uintptr_t)state_out | (uintptr_t)workspace) % 16) == 0;
+  DFLASH_REQUIRE(q && k && v && g && beta && state_in && state_out && y && (tape || prompt), DFLASH_ERR_ARG, "%s: null operand", who);
   DFLASH_REQUIRE(state_in != state_out, DFLASH_ERR_ARG, "%s: state_out must not alias state_in", who);
   auto ok = [](int dt) { return dt == DFLASH_BF16 || dt == DFLASH_FP16 || dt == DFLASH_FP32; };
   DFLASH_REQUIRE(ok(in_dtype) && ok(g_dtype) && ok(beta_dtype) && ok(state_dtype) && (!z || ok(weight_dtype)),
@@ -846,16 +831,21 @@ int gdn_forward_launch(const char* who, const void* q, const void* k, const void
 
   const dim3 grid((unsigned)(slots * Hv)), block(kThreads);
   hipStream_t s = (hipStream_t)stream;
-  const size_t smem = ((size_t)T * 128 * 3 + (size_t)T * (g_per_dk ? 128 : 1) + 2 * (size_t)T) * sizeof(float);
-  const bool fast = Dk == 128 && Dv == 128 && T >= 1 && smem <= 64 * 1024 &&
+  a.staged = T < 16 ? T : 16;
+  const size_t smem = (size_t)a.staged * (3 * 128 + (g_per_dk ? 128 : 1) + 2) * sizeof(float);
+  const bool fast = Dk == 128 && Dv == 128 && T >= 1 &&
                     (state_dtype != DFLASH_FP32 ||
                      (((uintptr_t)state_in % 16) == 0 && ((uintptr_t)state_out % 16) == 0));
-  const bool no_chunk = option(DFLASH_OPT_GDN_STEP_BY_STEP) != 0;  // (tests of one kernel against the other)
-  const bool aligned16 = (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)y | (uintptr_t)tape |
-                           (uintptr_t)z | (uintptr_t)norm_weight) % 16) == 0;
   const bool chunk = fast && !g_per_dk && state_dtype == DFLASH_FP32 && T <= 16 && aligned16 && !no_chunk;
   bool norm_done = false;
-  if (chunk) {
+  if (prompt) {
+    const size_t need = gdn_prompt_workspace_bytes(slots, T, Hk, Hv, Dk);
+    DFLASH_REQUIRE(workspace_bytes >= need, DFLASH_ERR_WORKSPACE, "%s: workspace of %zu bytes needed, %zu given", who, need,
+                   workspace_bytes);
+    const int rc = gdn_prompt_launch(q, k, v, g, beta, state_in, state_out, y, tape, mask, workspace, slots, T, Hk, Hv, Dk, Dv,
+                                     g_dtype, beta_dtype, state_dtype, s);
+    if (rc != DFLASH_OK) return rc;
+  } else if (chunk) {
     const size_t lds = kChunkLdsFloats * sizeof(float);
     const bool wide = in_dtype == DFLASH_FP32;
     const bool split = in_dtype == DFLASH_BF16;  // q and k are bf16 numbers: exact products on the bf16 matrix cores
@@ -910,4 +900,19 @@ extern "C" int dflash_gdn_forward_tape_norm(const void* q, const void* k, const 
   return dflash::gdn_forward_launch("dflash_gdn_forward_tape_norm", q, k, v, g, beta, state_in, state_out, out, tape,
                                     mask, z, norm_weight, weight_dtype, eps, slots, T, Hk, Hv, Dk, Dv, in_dtype,
                                     g_dtype, beta_dtype, state_dtype, g_per_dk, stream);
+}
+
+extern "C" size_t dflash_gdn_forward_workspace_bytes(int slots, int T, int Hk, int Hv, int Dk, int Dv, int in_dtype, int g_per_dk) {
+  using namespace dflash;
+  return gdn_prompt_covers(slots, T, Hk, Hv, Dk, Dv, in_dtype, g_per_dk) ? gdn_prompt_workspace_bytes(slots, T, Hk, Hv, Dk) : 0;
+}
+
+extern "C" int dflash_gdn_forward(const void* q, const void* k, const void* v, const void* g, const void* beta,
+                                  const void* state_in, void* state_out, const void* z, const void* norm_weight, void* y,
+                                  float* tape, const uint8_t* mask, void* workspace, size_t workspace_bytes, int slots, int T,
+                                  int Hk, int Hv, int Dk, int Dv, int in_dtype, int g_dtype, int beta_dtype, int state_dtype,
+                                  int weight_dtype, int g_per_dk, float eps, void* stream) {
+  return dflash::gdn_forward_launch("dflash_gdn_forward", q, k, v, g, beta, state_in, state_out, y, tape, mask, z, norm_weight,
+                                    weight_dtype, eps, slots, T, Hk, Hv, Dk, Dv, in_dtype, g_dtype, beta_dtype, state_dtype,
+                                    g_per_dk, stream, workspace, workspace_bytes);
 }

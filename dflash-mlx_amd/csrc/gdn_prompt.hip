@@ -1,0 +1,463 @@
+// GatedDeltaNet forward over a prompt (T > 16 tokens, bf16 q / k / v, one gate per head) for gfx950.
+//
+// The recurrence of gdn_forward.hip (dflash_mlx/kernels.py:12-127) is sequential in t, and a kernel that
+// walks it token by token takes microseconds per token.  Here the tokens go through in chunks of 32 in closed
+// form.  With c_t = prod_{u<=t} g_u inside the chunk, L[t][s] = beta_t (c_t/c_s)(k_s.k_t) for s < t and
+// Lq[t][s] = (c_t/c_s)(k_s.q_t) for s <= t (masked and missing tokens: g = 1, beta = 0),
+//     Delta = M' (V - c U),   M' = (I + L)^-1 diag(beta),   U = K S0^T
+//     Y     = c (Q S0^T) + Lq Delta
+//     S^T   = c_T S0^T + K^T diag(c_T/c_s) Delta,
+// a chunk needs the state only in two products with it and one update of it.
+//
+//  * gdn_chunk_kernel, one wave per (slot, chunk, head), computes what does not depend on the state: M' and
+//    Lq, in the register order the other kernel multiplies them in, and K^T likewise.  All chunks at once.
+//  * gdn_prompt_kernel, one wave per (slot, head, 16 rows of the state), walks the chunks.  Rows of S are
+//    independent, so 32 heads of 128 x 128 fill 256 compute units with one wave each, and what bounds
+//    the kernel is that wave's chain of dependent steps.  Nothing in it crosses lanes or goes through
+//    LDS: the accumulators of U^T, Delta^T and S^T (a lane holds four consecutive rows of one column)
+//    are read as the B operand of the next product with k in the order the lane happens to have it,
+//    and the A operands (M', Lq, K^T) were laid out in that order.
+//  * fp32 factors (S, V - c U, Delta, M', Lq) are cut into three bf16 pieces (24 bits, exact); products with bf16
+//    K and Q take three matrix-core passes, products of two fp32 factors the six of relative size 2^-16 and up.
+//    The result carries fp32 accuracy, as the step-by-step kernel's does.
+//  * The operands of the next chunk are loaded into the registers of the present one as soon as these have
+//    been used for the last time; 1 wave per SIMD has registers for all of them.
+// A 16-bit state is carried in fp32 and rounded once, at the end.
+//
+// Measured, 1024 tokens, 16 / 32 heads of 128 x 128: 15 + 65 us, against 123.7 ms with one workgroup per head
+// that kept S in memory (the step-by-step kernel held 41 tokens at most).  What the second kernel
+// is bound by is its chain: 2 us per chunk, of which the 72 matrix instructions with S are half.  Chunks of
+// 32 and not 16: cutting S into pieces (176 vector instructions) is paid per chunk, and a matrix instruction
+// of depth 32 in the update is filled; 64 would need more registers than a wave has.
+#include "gdn_device.h"
+
+namespace dflash {
+namespace prompt {
+
+constexpr int kChunk = 32;
+constexpr int kMatBytes = 2 * 3 * 1024;                // [tile of 16 rows][piece][lane] 16 bytes
+constexpr int kHeadBytes = 2 * kMatBytes + 3 * kChunk * 4;  // M', Lq, then per token c (0 if masked) and c_T / c_s, then c_T
+constexpr int kPitch = 36;                             // floats per row of the 32 x 32 matrices in LDS
+
+struct Args {
+  const uint16_t* q;
+  const uint16_t* k;
+  const uint16_t* v;
+  const void* g;
+  const void* beta;
+  const void* state_in;
+  void* state_out;
+  uint16_t* y;
+  float* tape;  // may be null
+  const uint8_t* mask;
+  char* work;
+  int slots, T, chunks, Hk, Hv, Dv;
+  int g_dtype, beta_dtype, state_dtype;
+};
+
+// Token (row 0 .. 31 of a chunk) that element j = 0 .. 7 of lane group kq holds in an operand of depth 32:
+// accumulators of the two 16-row tiles, one after the other.
+__device__ __forceinline__ int token_of(int kq, int j) { return 16 * (j >> 2) + 4 * kq + (j & 3); }
+// dk that row i of 16-row tile c of S^T stands for: tiles 2C and 2C + 1 of a lane are 8 consecutive dk.
+__device__ __forceinline__ int dk_of(int c, int i) { return 32 * (c >> 1) + 8 * (i >> 2) + 4 * (c & 1) + (i & 3); }
+
+__device__ __forceinline__ f32x4_t mfma(uint4 a, const uint32_t (&b)[4], f32x4_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a),
+                                                 __builtin_bit_cast(bf16x8_t, uint4{b[0], b[1], b[2], b[3]}), c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4_t mfma(uint4 a, uint4 b, f32x4_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+}
+
+// Raw buffer descriptor: 32-bit byte offsets, accesses from `bytes` on read zero and write nothing.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00027000);
+}
+
+template <int DK>
+__device__ __forceinline__ size_t chunk_bytes(const Args& a) {
+  return (size_t)a.Hv * kHeadBytes + (size_t)a.Hk * (kChunk * DK * 2);
+}
+
+template <int DK>
+__global__ __launch_bounds__(64, 3) void gdn_chunk_kernel(Args a) {
+  constexpr int NC = DK / 32;
+  constexpr int kKRow = DK + 8;  // 16-bit elements per row of K in LDS
+  __shared__ __align__(16) float sA[kChunk * kPitch];  // k_s . k_t, then L, then M'
+  __shared__ __align__(16) float sB[kChunk * kPitch];  // k_s . q_t, then Lq
+  __shared__ __align__(16) uint16_t sK[kChunk * kKRow];
+  __shared__ float sGate[kChunk], sBeta[kChunk];
+
+  const int hv = blockIdx.x % a.Hv, rest = blockIdx.x / a.Hv;
+  const int chunk = rest % a.chunks, slot = rest / a.chunks;
+  const int per = a.Hv / a.Hk, hk = hv / per;
+  const bool writes_k = hv % per == 0;
+  const int lane = threadIdx.x, li = lane & 15, kq = lane >> 4;
+  const int t0 = chunk * kChunk;
+  const size_t slotT = (size_t)slot * a.T;
+
+  uint4 kf[2][NC], qf[2][NC];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    int t = t0 + 16 * i + li;
+    t = t < a.T ? t : a.T - 1;
+    const size_t row = ((slotT + t) * a.Hk + hk) * DK + 8 * kq;
+#pragma unroll
+    for (int C = 0; C < NC; ++C) {
+      kf[i][C] = *reinterpret_cast<const uint4*>(a.k + row + 32 * C);
+      qf[i][C] = *reinterpret_cast<const uint4*>(a.q + row + 32 * C);
+    }
+  }
+  float on_v = 0.f;
+  if (lane < kChunk) {
+    const int t = t0 + lane;
+    const bool on = t < a.T && (a.mask == nullptr || a.mask[slotT + t] != 0);
+    const size_t at = (slotT + (t < a.T ? t : a.T - 1)) * a.Hv + hv;
+    sGate[lane] = on ? load_as_f32(a.g, at, a.g_dtype) : 1.f;
+    sBeta[lane] = on ? load_as_f32(a.beta, at, a.beta_dtype) : 0.f;
+    on_v = on ? 1.f : 0.f;
+  }
+  if (writes_k) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int C = 0; C < NC; ++C) *reinterpret_cast<uint4*>(sK + (16 * i + li) * kKRow + 32 * C + 8 * kq) = kf[i][C];
+  }
+#pragma unroll
+  for (int ts = 0; ts < 2; ++ts)
+#pragma unroll
+    for (int tt = ts; tt < 2; ++tt) {
+      f32x4_t x1 = {0.f, 0.f, 0.f, 0.f}, x2 = x1;  // rows s = 16 ts + 4 kq + r, column t = 16 tt + li
+#pragma unroll
+      for (int C = 0; C < NC; ++C) {
+        x1 = mfma(kf[ts][C], kf[tt][C], x1);
+        x2 = mfma(kf[ts][C], qf[tt][C], x2);
+      }
+      *reinterpret_cast<f32x4_t*>(sA + (16 * tt + li) * kPitch + 16 * ts + 4 * kq) = x1;
+      *reinterpret_cast<f32x4_t*>(sB + (16 * tt + li) * kPitch + 16 * ts + 4 * kq) = x2;
+    }
+  __syncthreads();
+  char* const out = a.work + ((size_t)slot * a.chunks + chunk) * chunk_bytes<DK>(a) + (size_t)hv * kHeadBytes;
+  float* const vec = reinterpret_cast<float*>(out + 2 * kMatBytes);
+  {
+    // one column s per lane: the lower half of the wave L, the upper half Lq
+    const int s = lane & 31;
+    const bool lower = lane < 32;
+    float* mat = lower ? sA : sB;
+    float r = 0.f, c_mine = 0.f, c = 1.f, on_t[kChunk];
+#pragma unroll
+    for (int t = 0; t < kChunk; ++t) on_t[t] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(on_v), t));
+#pragma unroll
+    for (int t = 0; t < kChunk; ++t) {
+      const float g = sGate[t];
+      r = t == s ? 1.f : (t > s ? r * g : 0.f);
+      c *= g;
+      c_mine = t == s ? c : c_mine;
+      const float x = mat[t * kPitch + s];
+      const bool counts = lower ? t > s : t >= s && on_t[t] != 0.f;  // (a masked token's y is zero)
+      mat[t * kPitch + s] = counts ? (lower ? sBeta[t] * r * x : r * x) : 0.f;
+    }
+    if (lower) {
+      vec[s] = on_v != 0.f ? c_mine : 0.f;
+      vec[kChunk + s] = r;
+      if (s == 0) vec[2 * kChunk] = c;
+    }
+  }
+  __syncthreads();
+  {  // column j of (I + L)^-1 by forward substitution, rows of L read by all lanes at once
+    const int j = lane & 31;
+    float x[kChunk];
+    f32x4_t row[2][kChunk / 4];  // the row in use and the next one
+#pragma unroll
+    for (int t = 0; t < kChunk; ++t) {
+      if (t + 1 < kChunk) {
+#pragma unroll
+        for (int s4 = 0; s4 < t + 1; s4 += 4) row[(t + 1) & 1][s4 / 4] = *reinterpret_cast<const f32x4_t*>(sA + (t + 1) * kPitch + s4);
+      }
+      float acc0 = t == j ? 1.f : 0.f, acc1 = 0.f;
+#pragma unroll
+      for (int s = 0; s < t; ++s) {
+        if (s & 1) acc1 -= row[t & 1][s / 4][s & 3] * x[s];
+        else acc0 -= row[t & 1][s / 4][s & 3] * x[s];
+      }
+      x[t] = acc0 + acc1;
+      // row by row: all of L at once does not fit the registers
+      asm volatile("" : "+v"(x[t]));
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();
+    const float beta = sBeta[j];
+    if (lane < 32) {
+#pragma unroll
+      for (int t = 0; t < kChunk; ++t) sA[t * kPitch + j] = x[t] * beta;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    const float* mat = m == 0 ? sA : sB;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const f32x4_t lo = *reinterpret_cast<const f32x4_t*>(mat + (16 * i + li) * kPitch + 4 * kq);
+      const f32x4_t hi = *reinterpret_cast<const f32x4_t*>(mat + (16 * i + li) * kPitch + 16 + 4 * kq);
+      const float f[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      const Pieces<8> p = split_bf16(f);
+      uint4* dst = reinterpret_cast<uint4*>(out + m * kMatBytes + i * 3072) + lane;
+      dst[0] = uint4{p.hi[0], p.hi[1], p.hi[2], p.hi[3]};
+      dst[64] = uint4{p.mid[0], p.mid[1], p.mid[2], p.mid[3]};
+      dst[128] = uint4{p.lo[0], p.lo[1], p.lo[2], p.lo[3]};
+    }
+  }
+  if (writes_k) {
+    char* const kt = a.work + ((size_t)slot * a.chunks + chunk) * chunk_bytes<DK>(a) + (size_t)a.Hv * kHeadBytes +
+                     (size_t)hk * (kChunk * DK * 2);
+#pragma unroll
+    for (int c = 0; c < DK / 16; ++c) {
+      uint32_t w[4];
+#pragma unroll
+      for (int j = 0; j < 8; j += 2)
+        w[j / 2] = (uint32_t)sK[token_of(kq, j) * kKRow + dk_of(c, li)] |
+                   ((uint32_t)sK[token_of(kq, j + 1) * kKRow + dk_of(c, li)] << 16);
+      reinterpret_cast<uint4*>(kt)[c * 64 + lane] = uint4{w[0], w[1], w[2], w[3]};
+    }
+  }
+}
+
+template <int DK>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void gdn_prompt_kernel(Args a) {
+  constexpr int NC = DK / 32, NT = DK / 16;
+  const int slices = a.Dv / 16;
+  // the slices of a head read the same K, Q, M' and Lq: all of them behind one L2 (blocks go to the XCDs in turn)
+  const int heads = a.slots * a.Hv;
+  int item, slice;
+  if (heads % 8 == 0) {
+    const int b = blockIdx.x / 8;
+    item = (b / slices) * 8 + blockIdx.x % 8;
+    slice = b % slices;
+  } else {
+    item = blockIdx.x / slices;
+    slice = blockIdx.x % slices;
+  }
+  const int slot = item / a.Hv, hv = item % a.Hv, hk = hv / (a.Hv / a.Hk);
+  const int lane = threadIdx.x, li = lane & 15, kq = lane >> 4;
+  const size_t slotT = (size_t)slot * a.T;
+  const int dv = 16 * slice + li;
+
+  // S^T tile c: rows dk_of(c, 4 kq + r), column dv = this lane's; two tiles are 8 consecutive dk of a row of S
+  f32x4_t st[NT];
+  const size_t srow = ((size_t)item * a.Dv + dv) * DK + 8 * kq;
+#pragma unroll
+  for (int C = 0; C < NC; ++C)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if (a.state_dtype == DFLASH_FP32) {
+        st[2 * C + h] = *reinterpret_cast<const f32x4_t*>((const float*)a.state_in + srow + 32 * C + 4 * h);
+      } else {
+        const uint2 w = *reinterpret_cast<const uint2*>((const uint16_t*)a.state_in + srow + 32 * C + 4 * h);
+        const uint32_t b[4] = {w.x & 0xffffu, w.x >> 16, w.y & 0xffffu, w.y >> 16};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) st[2 * C + h][e] = a.state_dtype == DFLASH_BF16 ? bf16_bits_to_f32(b[e]) : f16_bits_to_f32(b[e]);
+      }
+    }
+
+  // What a chunk reads and writes by token goes through buffer descriptors of this slot: tokens past T read
+  // zeros and are not written, with no branch (a branch around a store leaves the count of requests in flight
+  // open, and the next wait for a load becomes a wait for every store).
+  const uint32_t k_bytes = (uint32_t)a.T * a.Hk * DK * 2, v_bytes = (uint32_t)a.T * a.Hv * a.Dv * 2;
+  const auto k_buf = buffer_of(a.k + slotT * a.Hk * DK, k_bytes), q_buf = buffer_of(a.q + slotT * a.Hk * DK, k_bytes);
+  const auto v_buf = buffer_of(a.v + slotT * a.Hv * a.Dv, v_bytes), y_buf = buffer_of(a.y + slotT * a.Hv * a.Dv, v_bytes);
+  const auto tape_buf = buffer_of(a.tape + slotT * a.Hv * a.Dv, a.tape != nullptr ? 2 * v_bytes : 0u);
+  const uint32_t k_step = (uint32_t)a.Hk * DK * 2, v_step = (uint32_t)a.Hv * a.Dv * 2;  // bytes per token
+  const uint32_t k_at = li * k_step + hk * (DK * 2) + 16 * kq;
+  const uint32_t v_at = 4 * kq * v_step + (hv * a.Dv + dv) * 2;
+
+  uint4 kf[2][NC], qf[2][NC], kt[NT], mf[2][3], lf[2][3];
+  uint32_t vb[8];
+  f32x4_t cv[2], cfv[2];
+  float c_last, c_next;  // (asked for with K and Q: the scheduler moves the scaling of S to the front)
+  const size_t per_chunk = chunk_bytes<DK>(a);
+  const char* const head0 = a.work + (size_t)slot * a.chunks * per_chunk + (size_t)hv * kHeadBytes;
+  const char* const kt0 = a.work + (size_t)slot * a.chunks * per_chunk + (size_t)a.Hv * kHeadBytes + (size_t)hk * (kChunk * DK * 2);
+  auto load_kq = [&](int ch) __attribute__((always_inline)) {
+    c_next = reinterpret_cast<const float*>(head0 + ch * per_chunk + 2 * kMatBytes)[2 * kChunk + (lane >> 6)];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint32_t at = k_at + (ch * kChunk + 16 * i) * k_step;
+#pragma unroll
+      for (int C = 0; C < NC; ++C) {
+        kf[i][C] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(k_buf, at + 64 * C, 0, 0));
+        qf[i][C] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(q_buf, at + 64 * C, 0, 0));
+      }
+    }
+  };
+  auto load_v = [&](int ch) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      vb[j] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(v_buf, v_at + (ch * kChunk + 16 * (j >> 2) + (j & 3)) * v_step, 0, 0);
+  };
+  auto load_mat = [&](int ch, int which, uint4 (&f)[2][3]) __attribute__((always_inline)) {
+    const uint4* src = reinterpret_cast<const uint4*>(head0 + ch * per_chunk + which * kMatBytes) + lane;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int p = 0; p < 3; ++p) f[i][p] = src[(3 * i + p) * 64];
+  };
+  auto load_kt = [&](int ch) __attribute__((always_inline)) {
+    const uint4* src = reinterpret_cast<const uint4*>(kt0 + ch * per_chunk) + lane;
+#pragma unroll
+    for (int c = 0; c < NT; ++c) kt[c] = src[c * 64];
+  };
+  auto load_vec = [&](int ch) __attribute__((always_inline)) {
+    const float* vec = reinterpret_cast<const float*>(head0 + ch * per_chunk + 2 * kMatBytes);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      cv[i] = *reinterpret_cast<const f32x4_t*>(vec + 16 * i + 4 * kq);
+      cfv[i] = *reinterpret_cast<const f32x4_t*>(vec + kChunk + 16 * i + 4 * kq);
+    }
+  };
+  // arithmetic may move across, requests to memory stay where they were written
+#define DFLASH_KEEP_REQUESTS() __builtin_amdgcn_sched_barrier(0xF)
+  load_kq(0);
+  DFLASH_KEEP_REQUESTS();  // in the order of the loop: what its first wait may leave in flight is the least of both
+  load_v(0);
+  load_mat(0, 0, mf);
+  load_kt(0);
+  load_mat(0, 1, lf);
+  load_vec(0);
+  DFLASH_KEEP_REQUESTS();
+
+  // sum of the six piece products of two fp32 factors that matter; two accumulators, smaller terms first
+  auto product6 = [&](const uint4 (&f)[3], const Pieces<8>& p, f32x4_t big) __attribute__((always_inline)) {
+    f32x4_t small = {0.f, 0.f, 0.f, 0.f};
+    small = mfma(f[0], p.lo, small);
+    big = mfma(f[0], p.mid, big);
+    small = mfma(f[2], p.hi, small);
+    big = mfma(f[1], p.hi, big);
+    small = mfma(f[1], p.mid, small);
+    big = mfma(f[0], p.hi, big);
+    return big + small;
+  };
+
+#pragma unroll 1
+  for (int ch = 0; ch < a.chunks; ++ch) {
+    const int next = ch + 1 < a.chunks ? ch + 1 : ch;
+    c_last = c_next;
+    // ---- U = K S^T, W = Q S^T: rows = tokens, column = dv ---------------------------------------
+    f32x4_t U[2], W[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) U[i] = W[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int C = 0; C < NC; ++C) {
+      const float f[8] = {st[2 * C][0],     st[2 * C][1],     st[2 * C][2],     st[2 * C][3],
+                          st[2 * C + 1][0], st[2 * C + 1][1], st[2 * C + 1][2], st[2 * C + 1][3]};
+      const Pieces<8> sp = split_bf16(f);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) U[i] = mfma(kf[i][C], sp.lo, U[i]), W[i] = mfma(qf[i][C], sp.lo, W[i]);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) U[i] = mfma(kf[i][C], sp.mid, U[i]), W[i] = mfma(qf[i][C], sp.mid, W[i]);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) U[i] = mfma(kf[i][C], sp.hi, U[i]), W[i] = mfma(qf[i][C], sp.hi, W[i]);
+    }
+    load_kq(next);
+    DFLASH_KEEP_REQUESTS();
+    // ---- Delta = M' (V - c U) ----------------------------------------------------------------------
+    float rhs[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) rhs[j] = bf16_bits_to_f32(vb[j]) - cv[j >> 2][j & 3] * U[j >> 2][j & 3];
+    load_v(next);
+    DFLASH_KEEP_REQUESTS();
+    const Pieces<8> rp = split_bf16(rhs);
+    f32x4_t D[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) D[i] = product6(mf[i], rp, f32x4_t{0.f, 0.f, 0.f, 0.f});
+    load_mat(next, 0, mf);
+    DFLASH_KEEP_REQUESTS();
+    // ---- S^T = c_T S^T + K^T diag(c_T / c_s) Delta ----------------------------------------------
+    float scaled[8], plain[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      plain[j] = D[j >> 2][j & 3];
+      scaled[j] = plain[j] * cfv[j >> 2][j & 3];
+    }
+    {
+      const Pieces<8> dp = split_bf16(scaled);
+#pragma unroll
+      for (int c = 0; c < NT; ++c) st[c] *= c_last;
+#pragma unroll
+      for (int c = 0; c < NT; ++c) st[c] = mfma(kt[c], dp.lo, st[c]);
+#pragma unroll
+      for (int c = 0; c < NT; ++c) st[c] = mfma(kt[c], dp.mid, st[c]);
+#pragma unroll
+      for (int c = 0; c < NT; ++c) st[c] = mfma(kt[c], dp.hi, st[c]);
+    }
+    load_kt(next);
+    DFLASH_KEEP_REQUESTS();
+    // ---- Y = c W + Lq Delta ------------------------------------------------------------------------
+    const Pieces<8> dq = split_bf16(plain);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const f32x4_t Y = product6(lf[i], dq, W[i] * cv[i]);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const uint32_t at = v_at + (ch * kChunk + 16 * i + r) * v_step;
+        __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(uint16_t, (__bf16)Y[r]), y_buf, at, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(D[i][r]), tape_buf, 2 * at, 0, 0);
+      }
+    }
+    load_mat(next, 1, lf);
+    load_vec(next);
+    DFLASH_KEEP_REQUESTS();
+  }
+#undef DFLASH_KEEP_REQUESTS
+
+#pragma unroll
+  for (int C = 0; C < NC; ++C)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if (a.state_dtype == DFLASH_FP32) {
+        *reinterpret_cast<f32x4_t*>((float*)a.state_out + srow + 32 * C + 4 * h) = st[2 * C + h];
+      } else {
+        uint32_t b[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          b[e] = a.state_dtype == DFLASH_BF16 ? f32_to_bf16_bits(st[2 * C + h][e]) : f32_to_f16_bits(st[2 * C + h][e]);
+        *reinterpret_cast<uint2*>((uint16_t*)a.state_out + srow + 32 * C + 4 * h) = uint2{b[0] | (b[1] << 16), b[2] | (b[3] << 16)};
+      }
+    }
+}
+
+template <int DK>
+int launch(const Args& a, hipStream_t s) {
+  hipLaunchKernelGGL((gdn_chunk_kernel<DK>), dim3((unsigned)(a.slots * a.chunks * a.Hv)), dim3(64), 0, s, a);
+  hipLaunchKernelGGL((gdn_prompt_kernel<DK>), dim3((unsigned)(a.slots * a.Hv * (a.Dv / 16))), dim3(64), 0, s, a);
+  DFLASH_HIP_OK(hipGetLastError());
+  return DFLASH_OK;
+}
+
+}  // namespace prompt
+
+// Blocks of up to 16 tokens have kernels of their own (one launch, one wave of workgroups per head).
+bool gdn_prompt_covers(int slots, int T, int Hk, int Hv, int Dk, int Dv, int in_dtype, int g_per_dk) {
+  return in_dtype == DFLASH_BF16 && !g_per_dk && T > 16 && (Dk == 64 || Dk == 128) && Dv % 16 == 0 && Hk > 0 && Hv % Hk == 0 &&
+         slots > 0 && (long long)slots * Hv * ((T + 31) / 32) < (1ll << 31) && (long long)slots * Hv * (Dv / 16) < (1ll << 31) &&
+         ((long long)T + 32) * Hv * Dv * 4 < (1ll << 31) && ((long long)T + 32) * Hk * Dk * 2 < (1ll << 31);  // (buffer offsets)
+}
+
+size_t gdn_prompt_workspace_bytes(int slots, int T, int Hk, int Hv, int Dk) {
+  const int chunks = (T + prompt::kChunk - 1) / prompt::kChunk;
+  return (size_t)slots * chunks * ((size_t)Hv * prompt::kHeadBytes + (size_t)Hk * (prompt::kChunk * Dk * 2));
+}
+
+int gdn_prompt_launch(const void* q, const void* k, const void* v, const void* g, const void* beta, const void* state_in,
+                      void* state_out, void* y, float* tape, const uint8_t* mask, void* workspace, int slots, int T, int Hk,
+                      int Hv, int Dk, int Dv, int g_dtype, int beta_dtype, int state_dtype, hipStream_t s) {
+  prompt::Args a;
+  a.q = (const uint16_t*)q; a.k = (const uint16_t*)k; a.v = (const uint16_t*)v; a.g = g; a.beta = beta;
+  a.state_in = state_in; a.state_out = state_out; a.y = (uint16_t*)y; a.tape = tape; a.mask = mask;
+  a.work = (char*)workspace;
+  a.slots = slots; a.T = T; a.chunks = (T + prompt::kChunk - 1) / prompt::kChunk;
+  a.Hk = Hk; a.Hv = Hv; a.Dv = Dv;
+  a.g_dtype = g_dtype; a.beta_dtype = beta_dtype; a.state_dtype = state_dtype;
+  return Dk == 64 ? prompt::launch<64>(a, s) : prompt::launch<128>(a, s);
+}
+}  // namespace dflash

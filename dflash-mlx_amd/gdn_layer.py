@@ -253,7 +253,7 @@ def _gdn_call(self, inputs: torch.Tensor, mask: Optional[torch.Tensor], cache: O
     fused = (isinstance(norm, RMSNormGated) and os.environ.get("DFLASH_GDN_FUSED_NORM", "1") != "0" and
              fused_output_norm_applies(q, v, state, z, norm.weight))
     out, state, innovation_tape = gated_delta_kernel_with_tape(
-        q, k, v, g, beta, state, mask, output_norm=(z, norm.weight, norm.eps) if fused else None)
+        q, k, v, g, beta, state, mask, output_norm=(z, norm.weight, norm.eps) if fused else None, with_tape=record)
     if record:
         if mask is not None:
             qkv = torch.where(mask.to(torch.bool)[..., None], qkv, torch.zeros_like(qkv))

@@ -100,7 +100,7 @@ def fused_output_norm_applies(q: torch.Tensor, v: torch.Tensor, state: torch.Ten
 def gated_delta_kernel_with_tape(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor,
                                  beta: torch.Tensor, state: torch.Tensor,
                                  mask: Optional[torch.Tensor] = None, *,
-                                 output_norm: Optional[tuple] = None):
+                                 output_norm: Optional[tuple] = None, with_tape: bool = True):
     """GatedDeltaNet forward over a block that records the innovation tape (mirror of
     dflash_mlx/kernels.py:176-224): ``(y, state_out, tape)`` with y in q's dtype, the state in
     its own dtype and an fp32 tape.  Device tensors with Dk a multiple of 32 go to the gfx950
@@ -110,7 +110,8 @@ def gated_delta_kernel_with_tape(q: torch.Tensor, k: torch.Tensor, v: torch.Tens
     ``output_norm=(z, weight, eps)`` (no counterpart in the reference, which calls the layer's
     norm right after): the first result is then ``silu(z) * rms_norm(y, weight, eps)``, computed
     by the same launch (``dflash_gdn_forward_tape_norm``); only for inputs the kernel takes -
-    callers check ``fused_output_norm_applies`` first."""
+    callers check ``fused_output_norm_applies`` first.  ``with_tape=False``: the caller has no use for the
+    tape; long prompts then leave it out (the third result may be None)."""
     B, T, hk, dk = (int(d) for d in k.shape)
     hv, dv = int(v.shape[2]), int(v.shape[3])
     if g.ndim not in (3, 4):
@@ -130,32 +131,34 @@ def gated_delta_kernel_with_tape(q: torch.Tensor, k: torch.Tensor, v: torch.Tens
     q_c, k_c, v_c, g_c, beta_c = (t.contiguous() for t in (q, k, v, g, beta))
     state_c = state.contiguous()
     y = torch.empty((B, T, hv, dv), dtype=q.dtype, device=q.device)
-    tape = torch.empty((B, T, hv, dv), dtype=torch.float32, device=q.device)
+    code, per_dk = _DTYPE_CODE[q.dtype], 1 if g.ndim == 4 else 0
+    need = int(lib.dflash_gdn_forward_workspace_bytes(B, T, hk, hv, dk, dv, code, per_dk)) if T > 16 else 0
+    if any(t.data_ptr() % 16 for t in (q_c, k_c, v_c, state_c)):
+        need = 0
+    ws = torch.empty(need, dtype=torch.uint8, device=q.device) if need else None
+    tape = None
+    if with_tape or not need or lib.dflash_get_option(_native.OPT_GDN_STEP_BY_STEP):
+        tape = torch.empty((B, T, hv, dv), dtype=torch.float32, device=q.device)
     state_out = torch.empty_like(state_c)
     mask_ptr = None
     if mask is not None:
         mask = mask.to(torch.uint8).contiguous()
         mask_ptr = mask.data_ptr()
+    z_c = w_c = None
+    eps = 0.0
     if output_norm is not None:
         z, weight, eps = output_norm
         if not fused_output_norm_applies(q, v, state, z, weight):
             raise ValueError("output_norm: shapes or dtypes the fused kernel does not take")
         z_c, w_c = z.contiguous(), weight.contiguous()
-        rc = lib.dflash_gdn_forward_tape_norm(
-            q_c.data_ptr(), k_c.data_ptr(), v_c.data_ptr(), g_c.data_ptr(), beta_c.data_ptr(),
-            state_c.data_ptr(), state_out.data_ptr(), z_c.data_ptr(), w_c.data_ptr(), y.data_ptr(), tape.data_ptr(),
-            mask_ptr, B, T, hk, hv, dk, dv, _DTYPE_CODE[q.dtype], _DTYPE_CODE[g.dtype], _DTYPE_CODE[beta.dtype],
-            _DTYPE_CODE[state.dtype], _DTYPE_CODE[weight.dtype], 1 if g.ndim == 4 else 0, float(eps),
-            _native.raw_stream(q.device))
-        _native.check(rc, "dflash_gdn_forward_tape_norm")
-        return y, state_out, tape
-    rc = lib.dflash_gdn_forward_tape(
+    rc = lib.dflash_gdn_forward(
         q_c.data_ptr(), k_c.data_ptr(), v_c.data_ptr(), g_c.data_ptr(), beta_c.data_ptr(),
-        state_c.data_ptr(), state_out.data_ptr(), y.data_ptr(), tape.data_ptr(), mask_ptr,
-        B, T, hk, hv, dk, dv, _DTYPE_CODE[q.dtype], _DTYPE_CODE[g.dtype], _DTYPE_CODE[beta.dtype],
-        _DTYPE_CODE[state.dtype], 1 if g.ndim == 4 else 0,
-        _native.raw_stream(q.device))
-    _native.check(rc, "dflash_gdn_forward_tape")
+        state_c.data_ptr(), state_out.data_ptr(), None if z_c is None else z_c.data_ptr(),
+        None if w_c is None else w_c.data_ptr(), y.data_ptr(), None if tape is None else tape.data_ptr(), mask_ptr,
+        None if ws is None else ws.data_ptr(), need, B, T, hk, hv, dk, dv, code, _DTYPE_CODE[g.dtype],
+        _DTYPE_CODE[beta.dtype], _DTYPE_CODE[state.dtype], _DTYPE_CODE[q.dtype if w_c is None else w_c.dtype], per_dk,
+        float(eps), _native.raw_stream(q.device))
+    _native.check(rc, "dflash_gdn_forward")
     return y, state_out, tape
 
 

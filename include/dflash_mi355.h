@@ -339,8 +339,7 @@ int dflash_tape_replay(const void* tape, const void* k, const void* g, const voi
  *   mask      [slots, T] uint8 or NULL
  * 128 x 128 heads take register-resident kernels: one gate per head with an fp32 state and
  * T <= 16 the block kernel on the fp32 matrix cores (closed form of the recurrence; the option
- * DFLASH_OPT_GDN_STEP_BY_STEP turns it off), the rest a step-by-step kernel
- * while T*(3*128 + (g_per_dk ? 128 : 1) + 2)*4 bytes fit 64 KiB of LDS; every other shape a
+ * DFLASH_OPT_GDN_STEP_BY_STEP turns it off), the rest a step-by-step kernel; every other shape a
  * simple kernel that keeps S in state_out.
  */
 int dflash_gdn_forward_tape(const void* q, const void* k, const void* v, const void* g,
@@ -364,6 +363,20 @@ int dflash_gdn_forward_tape_norm(const void* q, const void* k, const void* v, co
                                  const uint8_t* mask, int slots, int T, int Hk, int Hv, int Dk, int Dv,
                                  int in_dtype, int g_dtype, int beta_dtype, int state_dtype,
                                  int weight_dtype, int g_per_dk, float eps, void* stream);
+
+/*
+ * The general form of the two calls above: z NULL leaves the output norm out, and with a workspace of
+ * dflash_gdn_forward_workspace_bytes() bytes (16-byte aligned, contents irrelevant; 0 where none is used)
+ * prompts - T > 16, bf16 q / k / v, one gate per head, Dk 64 or 128, Dv a multiple of 16 - go through the
+ * matrix cores in chunks of 32 tokens.  There a 16-bit state is carried in fp32 and rounded once, behind
+ * the last token, and tape may be NULL (not recorded).
+ */
+size_t dflash_gdn_forward_workspace_bytes(int slots, int T, int Hk, int Hv, int Dk, int Dv, int in_dtype, int g_per_dk);
+int dflash_gdn_forward(const void* q, const void* k, const void* v, const void* g, const void* beta,
+                       const void* state_in, void* state_out, const void* z, const void* norm_weight, void* y,
+                       float* tape, const uint8_t* mask, void* workspace, size_t workspace_bytes, int slots, int T,
+                       int Hk, int Hv, int Dk, int Dv, int in_dtype, int g_dtype, int beta_dtype, int state_dtype,
+                       int weight_dtype, int g_per_dk, float eps, void* stream);
 
 /*
  * GatedDeltaNet layer, everything between the input projections and the recurrence, in one

@@ -217,6 +217,42 @@ def test_bf16_arrays_take_the_16_bit_matrix_cores_without_losing_a_bit(native_li
     assert np.all(diff <= 2.0 ** -20 * size), float((diff / (2.0 ** -23 * size + 1e-300)).max())
 
 
+@pytest.mark.parametrize("shape", [
+    dict(T=17), dict(T=31, Hk=1, Hv=3), dict(T=32, Dk=64, Dv=64), dict(T=33, B=1), dict(T=63, Dk=64, Dv=48, Hk=2, Hv=2),
+    dict(T=65, B=1, Hk=2, Hv=8, Dv=16), dict(T=200, B=1, Hk=1, Hv=2)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_prompts_in_chunks(native_lib, shape, masked):
+    """More than 16 tokens: chunks of 32 on the matrix cores.  One token to several chunks, last chunks
+    of one token and full ones, state slices of one and of several waves, against the fp64 oracle; the
+    three-piece products carry fp32 accuracy, so the bars are those of the 16-token kernel."""
+    args = _case(seed=50 + shape["T"], **shape)
+    B, T = args[0].shape[:2]
+    mask = None
+    if masked:
+        mask = torch.rand((B, T), generator=torch.Generator().manual_seed(T)) > 0.3
+    y, s, tape = _run(args, mask)
+    yo, so, to = O.gated_delta_ops_with_tape(*[_f64(t) for t in args], mask=None if mask is None else mask.numpy())
+    assert _rel(_f64(s), so) <= 2e-5 and _rel(_f64(tape), to) <= 2e-5
+    assert np.all(np.abs(_f64(y) - yo) <= 2.0 ** -8 * np.abs(yo) + 2e-5 * np.abs(yo).max())
+    if masked:
+        assert torch.all(tape.cpu()[~mask] == 0) and torch.all(y.cpu()[~mask] == 0)
+
+
+@pytest.mark.parametrize("state_dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("in_dtype", [torch.bfloat16, torch.float16])
+def test_prompts_with_a_low_precision_state(native_lib, state_dtype, in_dtype):
+    """bf16 arrays: the state is rounded once, behind the last token (half a unit of its type).  fp16
+    arrays take the step-by-step kernel, whose state is rounded at every one of the 70 steps."""
+    args = _case(B=1, T=70, Hk=2, Hv=2, seed=61, dtype=in_dtype, state_dtype=state_dtype)
+    y, s, tape = _run(args)
+    yo, so, to = O.gated_delta_ops_with_tape(*[_f64(t) for t in args])
+    half = 2.0 ** (-9 if state_dtype == torch.bfloat16 else -12)
+    # a rounding decays with the gates (0.2 to 0.9 a step, mean 0.5), so few steps' roundings are alive at a time
+    bar = half if in_dtype == torch.bfloat16 else 4 * half
+    assert s.dtype == state_dtype and _rel(_f64(s), so) <= bar
+    assert _rel(_f64(tape), to) <= (2e-5 if in_dtype == torch.bfloat16 else 4 * half)
+
+
 def test_errors_and_host_tensors(native_lib):
     q, k, v, gate, beta, state = _case(B=1, T=2, Hk=3, Hv=4, Dk=32, Dv=8)
     with pytest.raises(ValueError, match="Cannot align"):
