@@ -12,7 +12,7 @@ from typing import Optional
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libdflash_mi355.so")
 
-ABI_VERSION = 19
+ABI_VERSION = 20
 
 BF16, FP16, FP32 = 0, 1, 2
 QMM_MMA2BIG, QMM_MMA2BIG_PIPE = 0, 1
@@ -41,6 +41,7 @@ EXPORTED_SYMBOLS = (
     "dflash_get_option",
     "dflash_qmm_m16_workspace_bytes",
     "dflash_qmm_m16",
+    "dflash_qmm_few",
     "dflash_qmm_error",
     "dflash_qmm_m16_static",
     "dflash_qmm_m16_pack_gate_up",
@@ -90,6 +91,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.dflash_qmm_m16.argtypes = (
         [c.c_void_p] * 6 + [c.c_size_t] + [c.c_int] * 8 + [c.c_void_p]
     )
+    lib.dflash_qmm_few.restype = c.c_int
+    lib.dflash_qmm_few.argtypes = [c.c_void_p] * 6 + [c.c_size_t] + [c.c_int] * 7 + [c.c_void_p]
     lib.dflash_qmm_error.restype = c.c_int
     lib.dflash_qmm_error.argtypes = [c.c_void_p, c.POINTER(c.c_uint32), c.c_void_p]
     lib.dflash_qmm_m16_static.restype = c.c_int

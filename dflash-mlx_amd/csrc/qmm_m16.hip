@@ -97,8 +97,8 @@ template <int GS, bool ACT_FP16, bool SB_FP16, int NT>
 __global__ __launch_bounds__(kThreads) void qmm_m16_kernel(
     const uint16_t* __restrict__ x, const uint32_t* __restrict__ w,
     const uint16_t* __restrict__ scales, const uint16_t* __restrict__ biases,
-    uint16_t* __restrict__ y, float* __restrict__ partials, uint32_t* __restrict__ counters, int K,
-    int N, int k_parts) {
+    uint16_t* __restrict__ y, float* __restrict__ partials, uint32_t* __restrict__ counters, int M,
+    int K, int N, int k_parts) {
   using A = Act<ACT_FP16>;
   constexpr int WPL = GS / 32;  // packed words (= MFMA k-steps) per lane per group
 
@@ -119,7 +119,7 @@ __global__ __launch_bounds__(kThreads) void qmm_m16_kernel(
   for (int t = 0; t < NT; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
   const uint4 ones = make_uint4(A::kOnes, A::kOnes, A::kOnes, A::kOnes);
-  const uint16_t* xrow = x + (size_t)col * K + kblk * (GS / 4);
+  const uint16_t* xrow = x + (size_t)(col < M ? col : 0) * K + kblk * (GS / 4);
 
   for (int g = g_begin + wave; g < g_end; g += kWaves) {
     // x operands of this group: lane (m=col, kblk) holds k = g*GS + kblk*GS/4 + [0, GS/4).
@@ -181,7 +181,8 @@ __global__ __launch_bounds__(kThreads) void qmm_m16_kernel(
 
   if (k_parts == 1) {
 #pragma unroll
-    for (int t = 0; t < NT; ++t) y[(size_t)m * N + n0 + 16 * t + col] = (uint16_t)A::from_f32(v[t]);
+    for (int t = 0; t < NT; ++t)
+      if (m < M) y[(size_t)m * N + n0 + 16 * t + col] = (uint16_t)A::from_f32(v[t]);
     return;
   }
 
@@ -217,24 +218,24 @@ __global__ __launch_bounds__(kThreads) void qmm_m16_kernel(
       // non-zero word in a slot of its own for a partial tile that has arrived
       __hip_atomic_store(slot, 0.f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    y[(size_t)m * N + n0 + 16 * t + col] = (uint16_t)A::from_f32(sum);
+    if (m < M) y[(size_t)m * N + n0 + 16 * t + col] = (uint16_t)A::from_f32(sum);
   }
 }
 
 template <int GS, bool ACT_FP16, bool SB_FP16>
 int launch(const void* x, const uint32_t* w, const void* scales, const void* biases, void* y,
-           float* partials, uint32_t* counters, int K, int N, int k_parts, hipStream_t stream) {
+           float* partials, uint32_t* counters, int M, int K, int N, int k_parts, hipStream_t stream) {
   const dim3 block(kThreads);
   if (N % 32 == 0) {
     const dim3 grid(N / 32, k_parts);
     hipLaunchKernelGGL((qmm_m16_kernel<GS, ACT_FP16, SB_FP16, 2>), grid, block, 0, stream,
                        (const uint16_t*)x, w, (const uint16_t*)scales, (const uint16_t*)biases,
-                       (uint16_t*)y, partials, counters, K, N, k_parts);
+                       (uint16_t*)y, partials, counters, M, K, N, k_parts);
   } else {
     const dim3 grid(N / 16, k_parts);
     hipLaunchKernelGGL((qmm_m16_kernel<GS, ACT_FP16, SB_FP16, 1>), grid, block, 0, stream,
                        (const uint16_t*)x, w, (const uint16_t*)scales, (const uint16_t*)biases,
-                       (uint16_t*)y, partials, counters, K, N, k_parts);
+                       (uint16_t*)y, partials, counters, M, K, N, k_parts);
   }
   DFLASH_HIP_OK(hipGetLastError());
   return DFLASH_OK;
@@ -242,13 +243,13 @@ int launch(const void* x, const uint32_t* w, const void* scales, const void* bia
 
 template <int GS>
 int launch_gs(int act_dtype, int sb_dtype, const void* x, const uint32_t* w, const void* scales,
-              const void* biases, void* y, float* partials, uint32_t* counters, int K, int N,
+              const void* biases, void* y, float* partials, uint32_t* counters, int M, int K, int N,
               int k_parts, hipStream_t stream) {
   const bool a16 = act_dtype == DFLASH_FP16, s16 = sb_dtype == DFLASH_FP16;
-  if (!a16 && !s16) return launch<GS, false, false>(x, w, scales, biases, y, partials, counters, K, N, k_parts, stream);
-  if (!a16 && s16) return launch<GS, false, true>(x, w, scales, biases, y, partials, counters, K, N, k_parts, stream);
-  if (a16 && !s16) return launch<GS, true, false>(x, w, scales, biases, y, partials, counters, K, N, k_parts, stream);
-  return launch<GS, true, true>(x, w, scales, biases, y, partials, counters, K, N, k_parts, stream);
+  if (!a16 && !s16) return launch<GS, false, false>(x, w, scales, biases, y, partials, counters, M, K, N, k_parts, stream);
+  if (!a16 && s16) return launch<GS, false, true>(x, w, scales, biases, y, partials, counters, M, K, N, k_parts, stream);
+  if (a16 && !s16) return launch<GS, true, false>(x, w, scales, biases, y, partials, counters, M, K, N, k_parts, stream);
+  return launch<GS, true, true>(x, w, scales, biases, y, partials, counters, M, K, N, k_parts, stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -417,11 +418,12 @@ constexpr int kMaxCounterTiles = (int)(kCounterBytes / sizeof(uint32_t));
 namespace dflash {
 // qmm_m16_stream.hip
 bool qmm_stream_eligible(int K, int N, int group_size);
+bool qmm_stream_any_eligible(int K, int N, int group_size);
 size_t qmm_stream_workspace_bytes(int N, int grid);
 int qmm_stream_grid();
 int qmm_stream_launch(const void* x, const uint32_t* w, const void* scales, const void* biases,
-                      void* y, void* workspace, size_t workspace_bytes, int K, int N,
-                      int act_dtype, int sb_dtype, hipStream_t stream);
+                      void* y, void* workspace, size_t workspace_bytes, int M, int K, int N,
+                      int group_size, int act_dtype, int sb_dtype, hipStream_t stream);
 bool qmm_stream_gather_eligible(int P, int K, int N, int E, int group_size);
 int qmm_stream_gather_launch(const void* x, const int32_t* expert_ids, const uint32_t* w,
                              const void* scales, const void* biases, void* y, void* workspace,
@@ -443,18 +445,43 @@ extern "C" size_t dflash_qmm_m16_workspace_bytes(int K, int N, int group_size, i
   if (kernel != DFLASH_QMM_KERNEL_STREAM && variant == DFLASH_QMM_MMA2BIG_PIPE && k_parts > 1) {
     need = dflash::kCounterBytes + (size_t)k_parts * 16 * (size_t)N * sizeof(float);
   }
-  if (kernel != DFLASH_QMM_KERNEL_TILE && dflash::qmm_stream_eligible(K, N, group_size)) {
+  if (kernel != DFLASH_QMM_KERNEL_TILE &&
+      (dflash::qmm_stream_eligible(K, N, group_size) || dflash::qmm_stream_any_eligible(K, N, group_size))) {
     const size_t s = dflash::qmm_stream_workspace_bytes(N, dflash::qmm_stream_grid());
     need = s > need ? s : need;
   }
   return need;
 }
 
+namespace dflash {
+namespace {
+int qmm_up_to_16(const void* x, const uint32_t* w_q, const void* scales, const void* biases, void* y, void* workspace,
+                 size_t workspace_bytes, int M, int K, int N, int group_size, int act_dtype, int sb_dtype, int variant,
+                 int k_parts, int kernel, void* stream);
+}  // namespace
+}  // namespace dflash
+
 extern "C" int dflash_qmm_m16(const void* x, const uint32_t* w_q, const void* scales,
                               const void* biases, void* y, void* workspace, size_t workspace_bytes,
                               int K, int N, int group_size, int act_dtype, int sb_dtype,
                               int variant, int k_parts, int kernel, void* stream) {
-  using namespace dflash;
+  return dflash::qmm_up_to_16(x, w_q, scales, biases, y, workspace, workspace_bytes, 16, K, N, group_size, act_dtype, sb_dtype,
+                              variant, k_parts, kernel, stream);
+}
+
+extern "C" int dflash_qmm_few(const void* x, const uint32_t* w_q, const void* scales, const void* biases, void* y,
+                              void* workspace, size_t workspace_bytes, int M, int K, int N, int group_size, int act_dtype,
+                              int sb_dtype, int kernel, void* stream) {
+  DFLASH_REQUIRE(M >= 1 && M <= 16, DFLASH_ERR_SHAPE, "dflash_qmm_few: 1 to 16 rows, got %d", M);
+  return dflash::qmm_up_to_16(x, w_q, scales, biases, y, workspace, workspace_bytes, M, K, N, group_size, act_dtype, sb_dtype,
+                              DFLASH_QMM_MMA2BIG, 1, kernel, stream);
+}
+
+namespace dflash {
+namespace {
+int qmm_up_to_16(const void* x, const uint32_t* w_q, const void* scales, const void* biases, void* y, void* workspace,
+                 size_t workspace_bytes, int M, int K, int N, int group_size, int act_dtype, int sb_dtype, int variant,
+                 int k_parts, int kernel, void* stream) {
   DFLASH_REQUIRE(x && w_q && scales && biases && y, DFLASH_ERR_ARG, "dflash_qmm_m16: null operand");
   DFLASH_REQUIRE(act_dtype == DFLASH_BF16 || act_dtype == DFLASH_FP16, DFLASH_ERR_ARG,
                  "dflash_qmm_m16: act_dtype %d is not bf16/fp16", act_dtype);
@@ -475,8 +502,12 @@ extern "C" int dflash_qmm_m16(const void* x, const uint32_t* w_q, const void* sc
                  "dflash_qmm_m16: K=%d is not a multiple of 32*k_parts (k_parts=%d)", K, k_parts);
   DFLASH_REQUIRE(((uintptr_t)x % 16) == 0 && ((uintptr_t)w_q % 16) == 0, DFLASH_ERR_ARG,
                  "dflash_qmm_m16: x and w_q must be 16-byte aligned");
-  if (kernel != DFLASH_QMM_KERNEL_TILE && qmm_stream_eligible(K, N, group_size)) {
-    return qmm_stream_launch(x, w_q, scales, biases, y, workspace, workspace_bytes, K, N, act_dtype,
+  // (the C interface has always taken scales of 2-byte alignment; the ANYK loads need four)
+  const bool any = kernel == DFLASH_QMM_KERNEL_AUTO && qmm_stream_any_eligible(K, N, group_size) &&
+                   (((uintptr_t)scales | (uintptr_t)biases) % 4) == 0 && workspace != nullptr &&
+                   workspace_bytes >= qmm_stream_workspace_bytes(N, qmm_stream_grid());
+  if (kernel != DFLASH_QMM_KERNEL_TILE && (qmm_stream_eligible(K, N, group_size) || any)) {
+    return qmm_stream_launch(x, w_q, scales, biases, y, workspace, workspace_bytes, M, K, N, group_size, act_dtype,
                              sb_dtype, (hipStream_t)stream);
   }
   DFLASH_REQUIRE(kernel != DFLASH_QMM_KERNEL_STREAM, DFLASH_ERR_SHAPE,
@@ -499,13 +530,15 @@ extern "C" int dflash_qmm_m16(const void* x, const uint32_t* w_q, const void* sc
   hipStream_t s = (hipStream_t)stream;
   switch (group_size) {
     case 32:
-      return launch_gs<32>(act_dtype, sb_dtype, x, w_q, scales, biases, y, partials, counters, K, N, k_parts, s);
+      return launch_gs<32>(act_dtype, sb_dtype, x, w_q, scales, biases, y, partials, counters, M, K, N, k_parts, s);
     case 64:
-      return launch_gs<64>(act_dtype, sb_dtype, x, w_q, scales, biases, y, partials, counters, K, N, k_parts, s);
+      return launch_gs<64>(act_dtype, sb_dtype, x, w_q, scales, biases, y, partials, counters, M, K, N, k_parts, s);
     default:
-      return launch_gs<128>(act_dtype, sb_dtype, x, w_q, scales, biases, y, partials, counters, K, N, k_parts, s);
+      return launch_gs<128>(act_dtype, sb_dtype, x, w_q, scales, biases, y, partials, counters, M, K, N, k_parts, s);
   }
 }
+}  // namespace
+}  // namespace dflash
 
 // ---------------------------------------------------------------------------------
 // dflash_qmm_m16_static: the same product for callers that cannot allocate.

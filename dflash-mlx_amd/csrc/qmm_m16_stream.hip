@@ -1,7 +1,8 @@
 // Streaming M=16 int4 qmm for gfx950: persistent workgroups, LDS-staged weights.
 //
-// y[16,N] = x[16,K] . (s*q + b)^T for group_size 64, K % 512 == 0, N % 16 == 0 - the
-// shapes of the projections in the dense verify stacks - and its gathered form for MoE
+// y[M,N] = x[M,K] . (s*q + b)^T for M <= 16, group_size 64, K % 512 == 0, N % 16 == 0 - the
+// shapes of the projections in the dense verify stacks; other group sizes and K that is a multiple of
+// 64 only through variants with a little more bookkeeping (ANYK) - and its gathered form for MoE
 // layers, y[p] = x[p] . (s*q + b)^T of expert ids[p] for up to 256 rows: rows that share an
 // expert are taken 16 at a time as the M dimension, and the weights of the experts that
 // have rows are streamed like one tall matrix.  Same arithmetic as
@@ -51,7 +52,7 @@
 // Every instruction a wave issues costs it at least four cycles, scalar bookkeeping
 // included, so the per-unit paths are kept short: ring positions advance by addition,
 // and the loaders and the workers run separate loops that meet only at the barriers.
-#include <cstdlib>
+#include <type_traits>
 
 #include "dflash_common.h"
 #include "qmm_stream_device.h"
@@ -71,8 +72,9 @@ struct Params {
 #ifdef DFLASH_STREAM_STAMPS
   int stamp_slot;
 #endif
+  int M;               // rows of x and y that count (dense form), at most 16
   int K, N;
-  int stages;          // K / 256
+  int stages;          // ceil(K / 256)
   int units;           // row blocks * stages (dense form; the gathered form counts its own)
   // gathered form: x, y [P, .], row p goes through the weights of expert expert_ids[p];
   // w, scales, biases hold E matrices of [N, .] back to back
@@ -137,24 +139,34 @@ __device__ unsigned long long g_sstamps[64][256][16];
 #define DFLASH_SSTAMP(ev) do {} while (0)
 #endif
 
-// CHUNK: units per scale/bias chunk (4, or 2 when K is a multiple of 512 only).
+// GS: group size.  SBROW: bytes of scales per row and chunk, CHUNK = SBROW * GS / 512 units per chunk
+// (group 64: 4 units, or 2 when K is a multiple of 512 only).
+// ANYK: K a multiple of 64 and no more, groups of 32, 64 or 128.  A row block is ceil(K / 256) stages and
+// its last chunk may be a shorter one; that chunk is loaded from where it ends with the row (so that
+// no load leaves the array) and read that much further on.  Codes past the end of a row are some other
+// codes of the row, and the quarters of the last stage that lie past it are multiplied with scales and
+// biases masked to zero.  The tile kernel (qmm_m16.hip), which served these shapes, asks for weights in
+// the lane order of the matrix instruction, where neighbouring lanes sit in different rows: 64 cycles of
+// address work per load instead of 16.  Measured with groups of 32: 4096 x 24576 78.2 -> 21 us (3.0 TB/s),
+// 12288 x 4096 43.2 -> 12 us; the bookkeeping costs the group-64 shapes of the first two variants nothing.
 // GATHER: per-expert form.  Rows of x that share an expert are taken 16 at a time as one
 // "entry"; an entry is a matrix problem of its own, [rows, K] x [N, K]^T, and the unit
 // space is that of all entries back to back: virtual row block = entry * RB + row block.
-template <bool ACT_FP16, bool SB_FP16, int CHUNK, bool GATHER>
+template <bool ACT_FP16, bool SB_FP16, int GS, int SBROW, bool ANYK, bool GATHER>
 __global__ __launch_bounds__(kThreads, 1) void qmm_stream_kernel(Params p) {
   using A = Act<ACT_FP16>;
-  constexpr int SBROW = 8 * CHUNK;              // bytes of scales per row and chunk
-  constexpr int kChunkLoads = CHUNK == 4 ? 2 : 1;  // loads per loader and chunk
+  constexpr int CHUNK = SBROW * GS / 512;
+  constexpr int kSbUnit = SBROW / CHUNK;           // bytes of scales per row and unit
+  constexpr int kChunkLoads = SBROW == 32 ? 2 : 1;  // loads per loader and chunk
   // The first unit is what a launch waits for longest, and its scales and biases (256 pieces
   // of 32 bytes, one DRAM access each) are the last of it to land.  The worker waves, which
   // have nothing to do until that unit is in LDS, ask for it as their first instructions -
   // about a microsecond before the loader waves have their pointers set up - and the loaders
-  // start with the second unit.  CHUNK = 4: per worker lane one 16-byte load of scales or biases
-  // (wave w < 4 the scales of rows 32 w .., the others the biases), one of x (instruction w of
-  // the loaders' scheme) and two of codes (instructions 2 w, 2 w + 1).
-  constexpr bool kWorkersFetchFirstChunk = CHUNK == 4;
-  constexpr int kFirst = kWorkersFetchFirstChunk ? 1 : 0;  // units at the head of the range the loaders skip
+  // start with the second unit.  Per worker lane one 16-byte load of scales or biases (SBROW = 32:
+  // wave w < 4 the scales of rows 32 w .., the others the biases; SBROW = 16: waves 0 and 1 the scales of
+  // rows 64 w .., 2 and 3 the biases), one of x (instruction w of the loaders' scheme) and two of codes
+  // (instructions 2 w, 2 w + 1).
+  constexpr int kFirst = 1;  // units at the head of the range the loaders skip
   extern __shared__ __attribute__((aligned(1024))) char lds[];
 
   const int tid = threadIdx.x;
@@ -165,9 +177,15 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_stream_kernel(Params p) {
   if (wave == kWaves) DFLASH_SSTAMP(8);
   const int RB = (p.N + kRows - 1) / kRows;  // row blocks of one matrix
   // bytes from one unit's codes to the next unit's of the same rows, and from chunk to chunk
-  const bool packed = !GATHER && CHUNK == 4 && p.packed;
+  const bool packed = !GATHER && !ANYK && SBROW == 32 && p.packed;
   const uint32_t w_unit_stride = packed ? kPackedUnitBytes : kUnitK / 2;
-  const uint32_t sb_chunk_stride = packed ? kPackedChunkBytes : CHUNK * kGroups * 2;
+  const uint32_t sb_chunk_stride = packed ? kPackedChunkBytes : SBROW;
+  // where chunk c of a row of scales is loaded from, and how much later than there it begins
+  const int sb_last = p.K / GS * 2 - SBROW;
+  auto chunk_at = [&](int c) __attribute__((always_inline)) -> int {
+    const int at = c * (int)sb_chunk_stride;
+    return ANYK ? (at < sb_last ? at : sb_last) : at;
+  };
 
   int units = p.units;
   if (GATHER) {
@@ -260,7 +278,7 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_stream_kernel(Params p) {
       wh.expert = (int)(e & 0xFFFFu);
       wh.rows = (int)(e >> 16);
     } else {
-      wh.entry = 0, wh.rb = vrb, wh.expert = 0, wh.rows = 16;
+      wh.entry = 0, wh.rb = vrb, wh.expert = 0, wh.rows = p.M;
     }
     return wh;
   };
@@ -288,10 +306,12 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_stream_kernel(Params p) {
     //         CHUNK = 2: 2 + 2 instructions of 64 rows, one granule per row; loaders 0, 1
     //         issue the scales of rows 0..63, 64..127, loaders 2, 3 the biases
     const int ld = wave - kWaves;
-    const int G = p.K / kGS;
+    const int G = p.K / GS;
     const size_t row_bytes = (size_t)p.K >> 1;
     const int w_r = lane >> 3;
     const int w_c = (lane & 7) ^ (((w_r >> 1) & 3) << 1);
+    const int w_tail = (p.stages - 1) * (kUnitK / 2);  // byte offset of the last stage's codes in a row
+    const int w_fix = ANYK && w_tail + w_c * 16 >= (int)row_bytes ? -(w_tail + w_c * 16) : 0;
     const char* xp[2];   // x of this lane's row at stage 0
     const char* wp[4];   // codes of this lane's rows at stage 0 of the row block being issued
     const char* sbp[2];  // scales / biases of this lane's row, chunk 0 (CHUNK = 2: [0] only)
@@ -307,14 +327,14 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_stream_kernel(Params p) {
         row = row < p.N ? row : p.N - 1;
         wp[i] = (const char*)wmat + (size_t)row * row_bytes + w_c * 16;
       }
-      if (!GATHER && CHUNK == 4 && p.packed) {
+      if (packed) {
         const char* img = (const char*)p.w + (size_t)wh.rb * p.stages * kPackedUnitBytes + lane * 16;
 #pragma unroll
         for (int i = 0; i < 4; ++i) wp[i] = img + (ld + 4 * i) * 1024;
         const size_t sb_img = (size_t)wh.rb * (p.stages / 4) * kPackedChunkBytes + ld * 1024 + lane * 16;
         sbp[0] = (const char*)p.scales + sb_img;
         sbp[1] = (const char*)p.biases + sb_img;
-      } else if (CHUNK == 4) {
+      } else if (SBROW == 32) {
         int row = row0 + 32 * ld + (lane >> 1);
         row = row < p.N ? row : p.N - 1;
         sbp[0] = (const char*)(smat + (size_t)row * G) + (lane & 1) * 16;
@@ -327,11 +347,8 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_stream_kernel(Params p) {
       }
       // rows of x: the entry's rows in the order of its table; surplus rows of the MFMA tile
       // repeat the entry's first row (their results are never stored)
-      int xrow = lane & 15;
-      if (GATHER) {
-        const int m = xrow < wh.rows ? xrow : 0;
-        xrow = (int)lds_read_u16(lds0 + kTabOffset + kTabRows + 2 * (wh.entry * 16 + m));
-      }
+      int xrow = (lane & 15) < wh.rows ? lane & 15 : 0;
+      if (GATHER) xrow = (int)lds_read_u16(lds0 + kTabOffset + kTabRows + 2 * (wh.entry * 16 + xrow));
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
         const int xi = ld + 4 * i;
@@ -348,15 +365,18 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_stream_kernel(Params p) {
       ++rb_i;
     }
     int sb_slot_i = kFirst;  // scale/bias slot of the next chunk to issue
-    if (issued < u1 || !kFirst) set_row_block(rb_i);
+    if (issued < u1) set_row_block(rb_i);
+    uint32_t chunk_starts = 0;  // bit i: the unit issued i units ago came with a chunk of scales and biases
     // Issues one unit: 6 loads (2 for x, 4 for codes), plus kChunkLoads with the first unit
     // of every scale/bias chunk and with the first unit of the range.
     auto issue_next = [&]() __attribute__((always_inline)) {
       char* slot = lds + slot_i * kSlotBytes;
-      if ((st_i % CHUNK) == 0 || (!kFirst && issued == u0)) {
+      const bool starts_chunk = st_i % CHUNK == 0;
+      if (ANYK) chunk_starts = chunk_starts << 1 | (starts_chunk ? 1u : 0u);
+      if (starts_chunk) {
         char* sb = lds + kSbOffset + sb_slot_i * kSbSlotBytes;
-        const size_t off = (size_t)(st_i / CHUNK) * sb_chunk_stride;
-        if (CHUNK == 4) {
+        const size_t off = (size_t)chunk_at(st_i / CHUNK);
+        if (SBROW == 32) {
           load16_to_lds(sbp[0] + off, sb + ld * 1024);
           load16_to_lds(sbp[1] + off, sb + kSbArrayBytes + ld * 1024);
         } else {
@@ -365,11 +385,16 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_stream_kernel(Params p) {
         if (++sb_slot_i == kSbDepth) sb_slot_i = 0;
       }
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
-        load16_to_lds(xp[i] + (size_t)st_i * (kUnitK * 2), slot + kXOffset + (ld + 4 * i) * 1024);
+      for (int i = 0; i < 2; ++i) {
+        // (instruction ld + 4 i is quarter (ld + 4 i) / 2 of the stage)
+        const bool in = !ANYK || st_i * kUnitK + ((ld + 4 * i) >> 1) * 64 < p.K;
+        load16_to_lds(xp[i] + (in ? (size_t)st_i * (kUnitK * 2) : (size_t)0) - (in ? 0 : ((ld + 4 * i) >> 1) * 128),
+                      slot + kXOffset + (ld + 4 * i) * 1024);
+      }
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        load16_to_lds_stream(wp[i] + (size_t)st_i * w_unit_stride, slot + (ld + 4 * i) * 1024);
+        load16_to_lds_stream(wp[i] + (ptrdiff_t)((size_t)st_i * w_unit_stride) + (ANYK && st_i == p.stages - 1 ? w_fix : 0),
+                             slot + (ld + 4 * i) * 1024);
       ++issued;
       if (++slot_i == kDepth) slot_i = 0;
       if (++st_i == p.stages) {
@@ -385,13 +410,17 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_stream_kernel(Params p) {
     };
     // Waits until this loader's part of unit v has landed (loads retire in issue order).
     auto wait_unit = [&](int v) __attribute__((always_inline)) {
-      wait_loads(loads_through(issued - 1) - loads_through(v));
+      if (ANYK) {
+        const int n = issued - 1 - v;  // units issued behind v
+        wait_loads(6 * n + kChunkLoads * __builtin_popcount(chunk_starts & ((1u << n) - 1u)));
+      } else {
+        wait_loads(loads_through(issued - 1) - loads_through(v));
+      }
     };
 
     const int ahead = units < 4 * grid ? kAheadShort : kAhead;
     DFLASH_SSTAMP(9);
     for (int i = kFirst; i < ahead && issued < u1; ++i) issue_next();
-    if (!kFirst) wait_unit(u0);
     DFLASH_SSTAMP(10);
     asm volatile("s_barrier" ::: "memory");
     DFLASH_SSTAMP(11);
@@ -416,28 +445,27 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_stream_kernel(Params p) {
   }
 
   // ================================== worker waves ====================================
-  if (kWorkersFetchFirstChunk) {
+  {
     const Where wh = locate(rb0);
-    const int G = p.K / kGS;
-    const int part = wave & 3;
-    int row = wh.rb * kRows + 32 * part + (lane >> 1);
-    row = row < p.N ? row : p.N - 1;
-    const uint16_t* mat = (wave < 4 ? p.scales : p.biases) + (size_t)wh.expert * p.N * G;
-    const char* src = (const char*)(mat + (size_t)row * G) + (lane & 1) * 16 +
-                      (size_t)(st0 / CHUNK) * (CHUNK * kGroups * 2);
-    if (packed)
-      src = (const char*)(wave < 4 ? p.scales : p.biases) +
-            ((size_t)wh.rb * (p.stages / 4) + st0 / CHUNK) * kPackedChunkBytes + part * 1024 + lane * 16;
-    load16_to_lds(src, lds + kSbOffset + (wave < 4 ? 0 : kSbArrayBytes) + part * 1024);
-    // x: instruction `wave` of the loaders' scheme; codes: instructions 2 wave and 2 wave + 1
-    int xrow = lane & 15;
-    if (GATHER) {
-      const int m = xrow < wh.rows ? xrow : 0;
-      xrow = (int)lds_read_u16(lds0 + kTabOffset + kTabRows + 2 * (wh.entry * 16 + m));
+    const int G = p.K / GS;
+    if (SBROW == 32 || wave < 4) {
+      const int part = SBROW == 32 ? wave & 3 : wave & 1;
+      const bool is_scale = SBROW == 32 ? wave < 4 : wave < 2;
+      int row = wh.rb * kRows + (SBROW == 32 ? 32 * part + (lane >> 1) : 64 * part + lane);
+      row = row < p.N ? row : p.N - 1;
+      const uint16_t* mat = (is_scale ? p.scales : p.biases) + (size_t)wh.expert * p.N * G;
+      const char* src = (const char*)(mat + (size_t)row * G) + (SBROW == 32 ? (lane & 1) * 16 : 0) + chunk_at(st0 / CHUNK);
+      if (packed)
+        src = (const char*)(is_scale ? p.scales : p.biases) +
+              ((size_t)wh.rb * (p.stages / 4) + st0 / CHUNK) * kPackedChunkBytes + part * 1024 + lane * 16;
+      load16_to_lds(src, lds + kSbOffset + (is_scale ? 0 : kSbArrayBytes) + part * 1024);
     }
-    const char* xsrc = (const char*)(p.x + (size_t)xrow * p.K + (wave >> 1) * kGS +
-                                     (2 * (wave & 1) + (lane >> 5)) * 16 + ((lane >> 4) & 1) * 8) +
-                       (size_t)st0 * (kUnitK * 2);
+    // x: instruction `wave` of the loaders' scheme; codes: instructions 2 wave and 2 wave + 1
+    int xrow = (lane & 15) < wh.rows ? lane & 15 : 0;
+    if (GATHER) xrow = (int)lds_read_u16(lds0 + kTabOffset + kTabRows + 2 * (wh.entry * 16 + xrow));
+    const bool x_in = !ANYK || st0 * kUnitK + (wave >> 1) * 64 < p.K;
+    const char* xsrc = (const char*)(p.x + (size_t)xrow * p.K + (x_in ? (wave >> 1) * 64 + st0 * kUnitK : 0) +
+                                     (2 * (wave & 1) + (lane >> 5)) * 16 + ((lane >> 4) & 1) * 8);
     load16_to_lds(xsrc, lds + kXOffset + wave * 1024);
     const size_t row_bytes = (size_t)p.K >> 1;
     const uint32_t* wmat = p.w + (size_t)wh.expert * p.N * (row_bytes >> 2);
@@ -448,7 +476,8 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_stream_kernel(Params p) {
       const int q = 2 * wave + i;
       int wrow = wh.rb * kRows + 8 * q + w_r;
       wrow = wrow < p.N ? wrow : p.N - 1;
-      const char* wsrc = (const char*)wmat + (size_t)wrow * row_bytes + w_c * 16 + (size_t)st0 * (kUnitK / 2);
+      const int w_at = w_c * 16 + st0 * (kUnitK / 2);
+      const char* wsrc = (const char*)wmat + (size_t)wrow * row_bytes + (!ANYK || w_at < (int)row_bytes ? w_at : 0);
       if (packed)
         wsrc = (const char*)p.w + ((size_t)wh.rb * p.stages + st0) * kPackedUnitBytes + q * 1024 + lane * 16;
       load16_to_lds_stream(wsrc, lds + q * 1024);
@@ -462,26 +491,29 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_stream_kernel(Params p) {
   const int grp = wave & 3;   // quantisation group of the unit this wave works on
   const int half = wave >> 2; // rows 64*half .. 64*half + 63: tiles j = 0..3
   //   x fragment j of lane (m = col, kb = kblk) for group grp inside a slot: + j*256
-  const uint32_t xoff =
-      lds0 + kXOffset + grp * 2048 + (kblk >> 1) * 1024 + (16 * (2 * (kblk & 1)) + col) * 16;
+  //   (groups of 32: fragment 0 is k-blocks 0 .. 3 of 8, the first group, fragment 1 the second)
+  const uint32_t xoff = lds0 + kXOffset + grp * 2048 + kblk * (GS == 32 ? 256 : 512) + col * 16;
   // codes of row 64*half + 16j + col: group grp sits in the 32-byte pair grp ^ ((row >> 1) & 3),
   // which does not depend on j; tile j is 2 KiB further
   const uint32_t wrow = 64 * half + col;
-  const uint32_t woff =
-      lds0 + wrow * 128 + ((grp ^ ((wrow >> 1) & 3)) << 5) + (kblk >> 1) * 16 + (kblk & 1) * 8;
+  const uint32_t woff = lds0 + wrow * 128 + ((grp ^ ((wrow >> 1) & 3)) << 5) + kblk * (GS == 32 ? 4 : 8);
   // scale of that row: SBROW bytes per row and chunk, four 16-bit values per unit; tile j is
   // 16 rows further, biases one array further
-  const uint32_t soff = lds0 + kSbOffset + wrow * SBROW + grp * 2;
+  const uint32_t soff = lds0 + kSbOffset + wrow * SBROW + (GS == 32 ? grp * 4 : GS == 64 ? grp * 2 : (grp >> 1) * 2);
 
   // reading position: the unit whose operands are fetched next
   int rd_slot = 0;   // byte offset of its ring slot
   int rd_sb = -kSbSlotBytes;  // byte offset of its scale/bias slot
   int rd_q = st0 % CHUNK;     // its stage within the chunk
+  int rd_st = st0;            // its stage (ANYK)
+  int rd_shift = 0;           // bytes from where the chunk was loaded from to where it begins (ANYK)
+  uint32_t keep = 0xFFFFFFFFu, rd_keep = keep;  // 0: this wave's quarter of the unit in registers / read next is past K
   bool rd_first = true;
   f32x4_t acc4[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) acc4[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  Operands op[2];
+  typedef typename std::conditional<GS == 32, OperandsOf32, Operands>::type Ops;
+  Ops op[2];
 
   // addresses of the next unit's operands, and the step to the unit after it
   uint32_t rd_x, rd_w, rd_s;
@@ -490,13 +522,18 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_stream_kernel(Params p) {
       rd_sb += kSbSlotBytes;
       if (rd_sb == kSbDepth * kSbSlotBytes) rd_sb = 0;
       rd_first = false;
+      if (ANYK) rd_shift = rd_st / CHUNK * SBROW - chunk_at(rd_st / CHUNK);
     }
     rd_x = xoff + rd_slot;
     rd_w = woff + rd_slot;
-    rd_s = soff + rd_sb + rd_q * 8;
+    rd_s = soff + rd_sb + rd_q * kSbUnit + (ANYK ? rd_shift : 0);
     rd_slot += kSlotBytes;
     if (rd_slot == kDepth * kSlotBytes) rd_slot = 0;
     rd_q = (rd_q + 1) & (CHUNK - 1);
+    if (ANYK) {
+      rd_keep = rd_st * kUnitK + grp * 64 < p.K ? 0xFFFFFFFFu : 0u;
+      if (++rd_st == p.stages) rd_st = rd_q = 0;
+    }
   };
 
   // Output of a finished tile: accumulator r of lane l is (m = 4*(l/16) + r, n = 16*wave + l%16)
@@ -514,12 +551,13 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_stream_kernel(Params p) {
       }
     } else {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) p.y[(size_t)(4 * kblk + r) * p.N + n_out] = (uint16_t)A::from_f32(acc[r]);
+      for (int r = 0; r < 4; ++r)
+        if (4 * kblk + r < p.M) p.y[(size_t)(4 * kblk + r) * p.N + n_out] = (uint16_t)A::from_f32(acc[r]);
     }
   };
 
   DFLASH_SSTAMP(1);
-  if (kWorkersFetchFirstChunk) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   DFLASH_SSTAMP(2);
   asm volatile("s_barrier" ::: "memory");
   DFLASH_SSTAMP(3);
@@ -529,6 +567,7 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_stream_kernel(Params p) {
   operands_issue_piece<2, SBROW>(rd_x, rd_w, rd_s, op[0], acc4[0]);
   operands_issue_piece<3, SBROW>(rd_x, rd_w, rd_s, op[0], acc4[0]);
   operands_wait(op[0], acc4[0], acc4[1], acc4[2], acc4[3]);
+  keep = rd_keep;
 
   int left = u1 - u0;            // units still to consume, the current one included
   int rb_left = p.stages - st0;  // same, within the current row block
@@ -569,16 +608,17 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_stream_kernel(Params p) {
   while (true) {
 #pragma unroll
     for (int par = 0; par < 2; ++par) {
-      Operands& cur = op[par];
-      Operands& nxt = op[par ^ 1];
+      Ops& cur = op[par];
+      Ops& nxt = op[par ^ 1];
       asm volatile("s_barrier" ::: "memory");
       // The next unit's operands are read along the way.  After the last unit the same reads
       // are made once more, of the unit just consumed (valid LDS, results unused): with a
       // condition around them every tile would be a basic block of its own, and the compiler
       // could not run one tile's unpacking under another tile's matrix instructions.
       if (left > 1) next_addresses();
-      consume_unit<ACT_FP16, SB_FP16, SBROW>(cur, nxt, true, rd_x, rd_w, rd_s, acc4, ones, mask, magic);
+      consume_unit<ACT_FP16, SB_FP16, SBROW, ANYK>(cur, nxt, true, rd_x, rd_w, rd_s, acc4, ones, mask, magic, keep);
       operands_wait(nxt, acc4[0], acc4[1], acc4[2], acc4[3]);
+      keep = rd_keep;
       --left;
       ++in_rb;
 #ifdef DFLASH_STREAM_STAMPS
@@ -735,13 +775,25 @@ bool qmm_stream_eligible(int K, int N, int group_size) {
   return units * 1024 < (1ll << 31) && row_blocks <= (64 * 1024) / 4;
 }
 
+// K a multiple of 64 and no more, groups of 32, 64 or 128 (the ANYK kernels): what their loads ask for is
+// rows of scales that start on four bytes and hold a whole chunk.
+bool qmm_stream_any_eligible(int K, int N, int group_size) {
+  if ((group_size != 32 && group_size != 64 && group_size != 128) || K <= 0 || K % 64 != 0 || K % group_size != 0 || N <= 0 ||
+      N % 16 != 0) return false;
+  const int row = K / group_size * 2;
+  if (row % 4 != 0 || row < (group_size == 32 ? 32 : 16)) return false;
+  const long long row_blocks = (N + stream::kRows - 1) / stream::kRows;
+  const long long units = row_blocks * ((K + stream::kUnitK - 1) / stream::kUnitK);
+  return units * 1024 < (1ll << 31) && row_blocks <= (64 * 1024) / 4;
+}
+
 bool qmm_stream_gather_eligible(int P, int K, int N, int E, int group_size) {
-  if (!qmm_stream_eligible(K, N, group_size)) return false;
+  if (group_size != 64 || !(qmm_stream_eligible(K, N, group_size) || qmm_stream_any_eligible(K, N, group_size))) return false;
   const long long row_blocks = (N + stream::kRows - 1) / stream::kRows;
   // every row could be an entry of its own
   return P > 0 && P <= stream::kMaxEntries && E > 0 && E <= stream::kMaxExperts &&
          row_blocks * stream::kMaxEntries <= (64 * 1024) / 4 &&
-         row_blocks * stream::kMaxEntries * (K / stream::kUnitK) * 1024 < (1ll << 31);
+         row_blocks * stream::kMaxEntries * ((K + stream::kUnitK - 1) / stream::kUnitK) * 1024 < (1ll << 31);
 }
 
 size_t qmm_stream_workspace_bytes(int N, int grid) {
@@ -750,33 +802,41 @@ size_t qmm_stream_workspace_bytes(int N, int grid) {
 }
 
 namespace {
-template <bool GATHER>
-const void* stream_kernel_for(bool a16, bool s16, bool chunk4) {
+// Variants: group 64 with K a multiple of 1024 (0) and of 512 (1), any K with groups of 64 (2), 32 (3), 128 (4).
+constexpr int kVariants = 5;
+template <bool A16, bool S16>
+const void* stream_kernel_for(int variant, bool gather) {
   using namespace stream;
-#define DFLASH_STREAM_PICK(A16, S16)                                                      \
-  if (a16 == A16 && s16 == S16)                                                           \
-    return chunk4 ? (const void*)qmm_stream_kernel<A16, S16, 4, GATHER>                   \
-                  : (const void*)qmm_stream_kernel<A16, S16, 2, GATHER>;
-  DFLASH_STREAM_PICK(false, false)
-  DFLASH_STREAM_PICK(false, true)
-  DFLASH_STREAM_PICK(true, false)
-  DFLASH_STREAM_PICK(true, true)
-#undef DFLASH_STREAM_PICK
-  return nullptr;
+  switch (variant) {
+    case 0:
+      return gather ? (const void*)qmm_stream_kernel<A16, S16, 64, 32, false, true>
+                    : (const void*)qmm_stream_kernel<A16, S16, 64, 32, false, false>;
+    case 1:
+      return gather ? (const void*)qmm_stream_kernel<A16, S16, 64, 16, false, true>
+                    : (const void*)qmm_stream_kernel<A16, S16, 64, 16, false, false>;
+    case 2:
+      return gather ? (const void*)qmm_stream_kernel<A16, S16, 64, 16, true, true>
+                    : (const void*)qmm_stream_kernel<A16, S16, 64, 16, true, false>;
+    case 3:
+      return (const void*)qmm_stream_kernel<A16, S16, 32, 32, true, false>;
+    default:
+      return (const void*)qmm_stream_kernel<A16, S16, 128, 16, true, false>;
+  }
 }
 
-int launch_stream(stream::Params& p, bool gather, int grid, int act_dtype, int sb_dtype,
+int launch_stream(stream::Params& p, bool gather, int grid, int group_size, int act_dtype, int sb_dtype,
                   hipStream_t stream) {
   using namespace stream;
   const bool a16 = act_dtype == DFLASH_FP16, s16 = sb_dtype == DFLASH_FP16;
-  const bool chunk4 = p.K % (kUnitK * 4) == 0;
+  const int variant = group_size == 32 ? 3 : group_size == 128 ? 4 : p.K % (kUnitK * 4) == 0 ? 0 : p.K % (kUnitK * 2) == 0 ? 1 : 2;
   // (tests shorten the wait of the workgroups that add partial tiles to see them give up)
   p.spin_limit = option(DFLASH_OPT_QMM_SPIN_LIMIT) > 0 ? option(DFLASH_OPT_QMM_SPIN_LIMIT) : kSpinLimit;
-  const void* fn = gather ? stream_kernel_for<true>(a16, s16, chunk4) : stream_kernel_for<false>(a16, s16, chunk4);
+  const void* fn = a16 ? (s16 ? stream_kernel_for<true, true>(variant, gather) : stream_kernel_for<true, false>(variant, gather))
+                       : (s16 ? stream_kernel_for<false, true>(variant, gather) : stream_kernel_for<false, false>(variant, gather));
   const int lds_bytes = gather ? kLdsBytesGather : kLdsBytes;
   // the attribute belongs to the device's copy of the kernel: once per device and kernel
-  static bool attr_set[kMaxDevices][16] = {};
-  const int idx = (gather ? 8 : 0) + (chunk4 ? 4 : 0) + (a16 ? 2 : 0) + (s16 ? 1 : 0);
+  static bool attr_set[kMaxDevices][kVariants * 8] = {};
+  const int idx = variant * 8 + (gather ? 4 : 0) + (a16 ? 2 : 0) + (s16 ? 1 : 0);
   const int slot = current_device_slot();
   if (!attr_set[slot][idx] || slot == kMaxDevices - 1) {
     DFLASH_HIP_OK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes));
@@ -793,10 +853,11 @@ int launch_stream(stream::Params& p, bool gather, int grid, int act_dtype, int s
 }  // namespace
 
 int qmm_stream_launch(const void* x, const uint32_t* w, const void* scales, const void* biases,
-                      void* y, void* workspace, size_t workspace_bytes, int K, int N,
-                      int act_dtype, int sb_dtype, hipStream_t stream) {
+                      void* y, void* workspace, size_t workspace_bytes, int M, int K, int N,
+                      int group_size, int act_dtype, int sb_dtype, hipStream_t stream) {
   using namespace stream;
   Params p{};
+  p.M = M;
   p.x = (const uint16_t*)x;
   p.w = w;
   p.scales = (const uint16_t*)scales;
@@ -804,7 +865,7 @@ int qmm_stream_launch(const void* x, const uint32_t* w, const void* scales, cons
   p.y = (uint16_t*)y;
   p.K = K;
   p.N = N;
-  p.stages = K / kUnitK;
+  p.stages = (K + kUnitK - 1) / kUnitK;
   p.units = ((N + kRows - 1) / kRows) * p.stages;
   const int grid = qmm_stream_pick_grid(p.units, p.units / p.stages, qmm_stream_grid());
   const size_t need = qmm_stream_workspace_bytes(N, grid);
@@ -813,7 +874,7 @@ int qmm_stream_launch(const void* x, const uint32_t* w, const void* scales, cons
                  workspace ? workspace_bytes : (size_t)0);
   p.status = (uint32_t*)workspace;
   p.partials = (float*)((char*)workspace + 64 * 1024);
-  return launch_stream(p, false, grid, act_dtype, sb_dtype, stream);
+  return launch_stream(p, false, grid, group_size, act_dtype, sb_dtype, stream);
 }
 
 bool qmm_stream_packed_eligible(int K, int N, int group_size) {
@@ -850,8 +911,9 @@ int qmm_stream_packed_launch(const void* x, const void* w_img, const void* s_img
   p.y = (uint16_t*)y;
   p.K = K;
   p.N = N;
-  p.stages = K / kUnitK;
+  p.stages = (K + kUnitK - 1) / kUnitK;
   p.units = ((N + kRows - 1) / kRows) * p.stages;
+  p.M = 16;
   p.packed = 1;
   const int grid = qmm_stream_pick_grid(p.units, p.units / p.stages, qmm_stream_grid());
   const size_t need = qmm_stream_workspace_bytes(N, grid);
@@ -860,7 +922,7 @@ int qmm_stream_packed_launch(const void* x, const void* w_img, const void* s_img
                  workspace ? workspace_bytes : (size_t)0);
   p.status = (uint32_t*)workspace;
   p.partials = (float*)((char*)workspace + 64 * 1024);
-  return launch_stream(p, false, grid, act_dtype, sb_dtype, stream);
+  return launch_stream(p, false, grid, 64, act_dtype, sb_dtype, stream);
 }
 
 int qmm_stream_gather_launch(const void* x, const int32_t* expert_ids, const uint32_t* w,
@@ -876,7 +938,7 @@ int qmm_stream_gather_launch(const void* x, const int32_t* expert_ids, const uin
   p.y = (uint16_t*)y;
   p.K = K;
   p.N = N;
-  p.stages = K / kUnitK;
+  p.stages = (K + kUnitK - 1) / kUnitK;
   p.units = 0;  // counted on the device from the routing
   p.expert_ids = expert_ids;
   p.P = P;
@@ -889,7 +951,7 @@ int qmm_stream_gather_launch(const void* x, const int32_t* expert_ids, const uin
                  workspace ? workspace_bytes : (size_t)0);
   p.status = (uint32_t*)workspace;
   p.partials = (float*)((char*)workspace + 64 * 1024);
-  return launch_stream(p, true, grid, act_dtype, sb_dtype, stream);
+  return launch_stream(p, true, grid, 64, act_dtype, sb_dtype, stream);
 }
 
 }  // namespace dflash

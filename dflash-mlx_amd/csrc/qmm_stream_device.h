@@ -129,9 +129,19 @@ __device__ __forceinline__ uint32_t lds_address(const void* p) {
 //   f0, f1  x fragments (natural order) feeding MFMA 0 / 1
 //   wq[j]   packed codes of tile j: .x feeds MFMA 0, .y MFMA 1
 //   sv, bv  scale / bias of this lane's row in tile j, 16 bits zero-extended
+// With groups of 32 (see OperandsOf32) MFMA 0 and 1 take one group each.
 struct Operands {
+  static constexpr int kStepF1 = 256;  // bytes from x fragment 0 to 1 in LDS
   u32x4_t f0, f1;
   u32x2_t wq[4];
+  uint32_t sv[4], bv[4];
+};
+//   w0, w1  packed codes of tile j feeding MFMA 0 / 1 (lane group kb: words kb and 4 + kb of the quarter)
+//   sv, bv  scales / biases of the two groups, 16 bits each
+struct OperandsOf32 {
+  static constexpr int kStepF1 = 1024;
+  u32x4_t f0, f1;
+  uint32_t w0[4], w1[4];
   uint32_t sv[4], bv[4];
 };
 // The LDS reads of a unit's operands are started in four pieces and return at once: the
@@ -165,6 +175,31 @@ __device__ __forceinline__ void operands_issue_piece(uint32_t xaddr, uint32_t wa
         : "memory");
   }
 }
+template <int J, int SBROW>
+__device__ __forceinline__ void operands_issue_piece(uint32_t xaddr, uint32_t waddr, uint32_t saddr,
+                                                     OperandsOf32& o, f32x4_t& pin) {
+  if (J == 0) {
+    asm volatile(
+        "ds_read_b128 %0, %7\n"
+        "ds_read_b128 %1, %7 offset:1024\n"
+        "ds_read_b32 %2, %8\n"
+        "ds_read_b32 %3, %8 offset:16\n"
+        "ds_read_b32 %4, %9\n"
+        "ds_read_b32 %5, %9 offset:4096\n"
+        : "=&v"(o.f0), "=&v"(o.f1), "=&v"(o.w0[0]), "=&v"(o.w1[0]), "=&v"(o.sv[0]), "=&v"(o.bv[0]), "+v"(pin)
+        : "v"(xaddr), "v"(waddr), "v"(saddr)
+        : "memory");
+  } else {
+    asm volatile(
+        "ds_read_b32 %0, %5 offset:%7\n"
+        "ds_read_b32 %1, %5 offset:%8\n"
+        "ds_read_b32 %2, %6 offset:%9\n"
+        "ds_read_b32 %3, %6 offset:%10\n"
+        : "=&v"(o.w0[J]), "=&v"(o.w1[J]), "=&v"(o.sv[J]), "=&v"(o.bv[J]), "+v"(pin)
+        : "v"(waddr), "v"(saddr), "n"(2048 * J), "n"(2048 * J + 16), "n"(16 * SBROW * J), "n"(4096 + 16 * SBROW * J)
+        : "memory");
+  }
+}
 __device__ __forceinline__ void operands_wait(Operands& o, f32x4_t& acc0, f32x4_t& acc1,
                                               f32x4_t& acc2, f32x4_t& acc3) {
   asm volatile("s_waitcnt lgkmcnt(0)\n"
@@ -175,15 +210,27 @@ __device__ __forceinline__ void operands_wait(Operands& o, f32x4_t& acc0, f32x4_
                :
                : "memory");
 }
+__device__ __forceinline__ void operands_wait(OperandsOf32& o, f32x4_t& acc0, f32x4_t& acc1,
+                                              f32x4_t& acc2, f32x4_t& acc3) {
+  asm volatile("s_waitcnt lgkmcnt(0)\n"
+               : "+v"(o.f0), "+v"(o.f1), "+v"(o.w0[0]), "+v"(o.w0[1]), "+v"(o.w0[2]), "+v"(o.w0[3]),
+                 "+v"(o.w1[0]), "+v"(o.w1[1]), "+v"(o.w1[2]), "+v"(o.w1[3]),
+                 "+v"(o.sv[0]), "+v"(o.sv[1]), "+v"(o.sv[2]), "+v"(o.sv[3]),
+                 "+v"(o.bv[0]), "+v"(o.bv[1]), "+v"(o.bv[2]), "+v"(o.bv[3]),
+                 "+v"(acc0), "+v"(acc1), "+v"(acc2), "+v"(acc3)
+               :
+               : "memory");
+}
 
 // The arithmetic of one unit: acc[j] += (scale, bias)-corrected x . codes^T of tile j, from
 // the operands in `cur`.  With `fetch` set, the reads of the next unit's operands into `nxt`
 // are started along the way (nothing else may touch `nxt` before operands_wait).
-template <bool ACT_FP16, bool SB_FP16, int SBROW>
+// KEEP: scales and biases are masked with `keep` first (0 for k past the end of a row: nothing is added).
+template <bool ACT_FP16, bool SB_FP16, int SBROW, bool KEEP = false>
 __device__ __forceinline__ void consume_unit(const Operands& cur, Operands& nxt, bool fetch,
                                              uint32_t xaddr, uint32_t waddr, uint32_t saddr,
                                              f32x4_t (&acc)[4], uint4 ones, uint32_t mask,
-                                             uint32_t magic) {
+                                             uint32_t magic, uint32_t keep = 0xFFFFFFFFu) {
   using A = Act<ACT_FP16>;
   using SB = Act<SB_FP16>;
   if (fetch) operands_issue_piece<0, SBROW>(xaddr, waddr, saddr, nxt, acc[3]);
@@ -196,11 +243,42 @@ __device__ __forceinline__ void consume_unit(const Operands& cur, Operands& nxt,
     f32x4_t c = f32x4_t{0.f, 0.f, 0.f, 0.f};
     c = A::mfma(a0, unpack_codes(cur.wq[j].x, mask, magic), c);
     c = A::mfma(a1, unpack_codes(cur.wq[j].y, mask, magic), c);
-    const float s = SB::to_f32(cur.sv[j]);
-    const float b = SB::to_f32(cur.bv[j]);
+    const float s = SB::to_f32(KEEP ? cur.sv[j] & keep : cur.sv[j]);
+    const float b = SB::to_f32(KEEP ? cur.bv[j] & keep : cur.bv[j]);
     const float bb = __builtin_fmaf(-A::kOffset, s, b);
 #pragma unroll
     for (int r = 0; r < 4; ++r) acc[j][r] = __builtin_fmaf(bb, xs[r], __builtin_fmaf(s, c[r], acc[j][r]));
+    if (fetch) {
+      if (j == 0) operands_issue_piece<1, SBROW>(xaddr, waddr, saddr, nxt, acc[0]);
+      if (j == 1) operands_issue_piece<2, SBROW>(xaddr, waddr, saddr, nxt, acc[1]);
+      if (j == 2) operands_issue_piece<3, SBROW>(xaddr, waddr, saddr, nxt, acc[2]);
+    }
+  }
+}
+template <bool ACT_FP16, bool SB_FP16, int SBROW, bool KEEP = false>
+__device__ __forceinline__ void consume_unit(const OperandsOf32& cur, OperandsOf32& nxt, bool fetch,
+                                             uint32_t xaddr, uint32_t waddr, uint32_t saddr,
+                                             f32x4_t (&acc)[4], uint4 ones, uint32_t mask,
+                                             uint32_t magic, uint32_t keep = 0xFFFFFFFFu) {
+  using A = Act<ACT_FP16>;
+  using SB = Act<SB_FP16>;
+  if (fetch) operands_issue_piece<0, SBROW>(xaddr, waddr, saddr, nxt, acc[3]);
+  const uint4 a0 = as_uint4(permute_x(cur.f0)), a1 = as_uint4(permute_x(cur.f1));
+  const f32x4_t zero = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const f32x4_t xs0 = A::mfma(a0, ones, zero), xs1 = A::mfma(a1, ones, zero);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const f32x4_t c0 = A::mfma(a0, unpack_codes(cur.w0[j], mask, magic), zero);
+    const f32x4_t c1 = A::mfma(a1, unpack_codes(cur.w1[j], mask, magic), zero);
+    const uint32_t sv = KEEP ? cur.sv[j] & keep : cur.sv[j], bv = KEEP ? cur.bv[j] & keep : cur.bv[j];
+    const float s0 = SB::to_f32(sv & 0xFFFFu), s1 = SB::to_f32(sv >> 16);
+    const float bb0 = __builtin_fmaf(-A::kOffset, s0, SB::to_f32(bv & 0xFFFFu));
+    const float bb1 = __builtin_fmaf(-A::kOffset, s1, SB::to_f32(bv >> 16));
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      acc[j][r] = __builtin_fmaf(bb0, xs0[r], __builtin_fmaf(s0, c0[r], acc[j][r]));
+      acc[j][r] = __builtin_fmaf(bb1, xs1[r], __builtin_fmaf(s1, c1[r], acc[j][r]));
+    }
     if (fetch) {
       if (j == 0) operands_issue_piece<1, SBROW>(xaddr, waddr, saddr, nxt, acc[0]);
       if (j == 1) operands_issue_piece<2, SBROW>(xaddr, waddr, saddr, nxt, acc[1]);

@@ -451,9 +451,9 @@ def verify_matmul_packed(x: torch.Tensor, packed: PackedWeights) -> torch.Tensor
 
 def small_m_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
                    *, group_size: int = 64, bits: int = 4) -> "torch.Tensor | None":
-    """``x @ dequant(w).T`` for at most 16 rows of device activations through the M=16 kernel:
-    the rows are padded with zeros to 16 (a row of the product depends on its own row of x only,
-    so a row comes out the same whatever shares the block with it).  Covers what the C ABI covers
+    """``x @ dequant(w).T`` for at most 16 rows of device activations through the M=16 kernel (a row of
+    the product depends on its own row of x only, so a row comes out the same whatever shares the
+    block with it).  Covers what the C ABI covers
     (N a multiple of 16, K a multiple of the group size, bf16/fp16), which is more than the
     Python gate of ``verify_matmul`` lets through; returns None for anything else.  No
     counterpart in the reference, whose stock operator is a fused kernel of its own: here the
@@ -468,14 +468,25 @@ def small_m_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biase
         m *= int(d)
     if m < 1 or m > 16 or N % 16 != 0 or K % group_size != 0 or K % 32 != 0 or int(w.shape[1]) * 8 != K:
         return None
-    x2 = x.reshape(m, K)
-    if m < 16:
-        x16 = torch.zeros((16, K), dtype=x.dtype, device=x.device)
-        x16[:m] = x2
-    else:
-        x16 = x2.contiguous()
-    y = _launch(x16, w.contiguous(), scales.contiguous(), biases.contiguous(), K, N, group_size, "mma2big", 1)
-    return y[:m].reshape(*x.shape[:-1], N)
+    w, scales, biases = w.contiguous(), scales.contiguous(), biases.contiguous()
+    _require_operands("quantized_matmul", K, N, group_size, w, scales, biases, x.device)
+    x2 = x.reshape(m, K).contiguous()
+    lib = _native.lib()
+    y = torch.empty((m, N), dtype=x.dtype, device=x.device)
+    stream = _native.raw_stream(x.device)
+    kernel = _kernel_select()
+    key = (K, N, group_size, _native.QMM_MMA2BIG, 1, kernel)
+    need = _WORKSPACE_BYTES.get(key)
+    if need is None:
+        need = _WORKSPACE_BYTES[key] = int(lib.dflash_qmm_m16_workspace_bytes(*key))
+    ws_ptr, ws_bytes = None, 0
+    if need:
+        ws = _workspace(x.device, stream, need)
+        ws_ptr, ws_bytes = ws.data_ptr(), ws.numel()
+    rc = lib.dflash_qmm_few(x2.data_ptr(), w.data_ptr(), scales.data_ptr(), biases.data_ptr(), y.data_ptr(), ws_ptr, ws_bytes,
+                            m, K, N, group_size, _DTYPE_CODE[x.dtype], _DTYPE_CODE[scales.dtype], kernel, stream)
+    _native.check(rc, "dflash_qmm_few")
+    return y.reshape(*x.shape[:-1], N)
 
 
 # Scratch of the any-rows product, one per (device, stream): 64 KiB of counters, then partial tiles.

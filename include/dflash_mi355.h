@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define DFLASH_ABI_VERSION 19
+#define DFLASH_ABI_VERSION 20
 
 enum {
   DFLASH_OK = 0,
@@ -118,6 +118,15 @@ size_t dflash_qmm_m16_workspace_bytes(int K, int N, int group_size, int variant,
 int dflash_qmm_m16(const void* x, const uint32_t* w_q, const void* scales, const void* biases,
                    void* y, void* workspace, size_t workspace_bytes, int K, int N, int group_size,
                    int act_dtype, int sb_dtype, int variant, int k_parts, int kernel, void* stream);
+
+/*
+ * dflash_qmm_m16 for M = 1 .. 16 rows: x [M, K], y [M, N].  A row's result does not depend on how many
+ * rows come with it (bit for bit).  Workspace of dflash_qmm_m16_workspace_bytes(K, N, group_size,
+ * DFLASH_QMM_MMA2BIG, 1, kernel).
+ */
+int dflash_qmm_few(const void* x, const uint32_t* w_q, const void* scales, const void* biases, void* y,
+                   void* workspace, size_t workspace_bytes, int M, int K, int N, int group_size, int act_dtype,
+                   int sb_dtype, int kernel, void* stream);
 
 /*
  * dflash_qmm_m16 for callers that cannot allocate device memory: code under HIP graph

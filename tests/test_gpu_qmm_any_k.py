@@ -1,0 +1,60 @@
+"""Up to 16 rows through the streaming kernel's variants for every group size and K that is a multiple of 64
+only, against the product of the same operands in fp64: last chunks and last stages that are cut
+short in every way, ragged row blocks, one to sixteen rows, both activation types, gathered experts."""
+import pytest
+import torch
+
+from dflash_mlx_amd import verify_qmm as VQ
+from dflash_mlx_amd.quantized import dequantize, stock_matmul
+from dflash_mlx_amd.workloads import make_qmm_case
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _check(y, x, dense, K, dtype):
+    exact = x.double() @ dense.t().contiguous()
+    size = x.double().abs() @ dense.abs().t().contiguous()
+    # half a unit in the last place of the result; fp32 sums over codes offset by 128 or 1024 (up to 70 times the
+    # size of a centred code), whose errors add up like a random walk over K terms
+    eps = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    offset = 16.0 if dtype == torch.bfloat16 else 128.0
+    assert ((y.double() - exact).abs() <= 1.01 * eps * exact.abs() + size * offset * 2.0 ** -24 * 4).all()
+    assert (y.double() - exact).norm() <= eps * exact.norm()
+
+
+@pytest.mark.parametrize("K,N,group,dtype", [
+    (512, 16, 32, torch.bfloat16), (576, 48, 32, torch.bfloat16), (640, 128, 64, torch.bfloat16), (768, 144, 64, torch.float16),
+    (832, 272, 32, torch.float16), (896, 1040, 64, torch.bfloat16), (1024, 512, 32, torch.bfloat16),
+    (1024, 512, 128, torch.bfloat16), (1152, 2064, 64, torch.bfloat16), (1280, 112, 128, torch.float16),
+    (2176, 4096, 64, torch.bfloat16), (2816, 528, 128, torch.bfloat16), (4096, 6144, 32, torch.bfloat16),
+    (5376, 144, 64, torch.bfloat16), (12288, 4096, 32, torch.bfloat16), (4352, 5120, 128, torch.bfloat16)])
+def test_every_group_size_and_k(native_lib, monkeypatch, K, N, group, dtype):
+    monkeypatch.setenv("DFLASH_VERIFY_QMM", "1")
+    monkeypatch.delenv("DFLASH_QMM_KERNEL", raising=False)
+    c = make_qmm_case(K, N, 300 + K, group_size=group, dtype=dtype).to(DEV)
+    dense = dequantize(c.w, c.scales, c.biases, group, 4, dtype=torch.float64)
+    y = VQ._launch(c.x, c.w, c.scales, c.biases, K, N, group, "mma2big", 1)
+    _check(y, c.x, dense, K, dtype)
+    for rows in (1, 2, 7, 15, 16):  # and the same bits whatever shares the block with a row
+        assert torch.equal(stock_matmul(c.x[:rows], c.w, c.scales, c.biases, group_size=group), y[:rows])
+    torch.cuda.synchronize()
+    VQ.raise_on_device_errors(torch.device(DEV))
+    ws = VQ._workspace(torch.device(DEV), torch.cuda.current_stream().cuda_stream, 1)
+    assert int((ws != 0).sum()) == 0
+
+
+@pytest.mark.parametrize("K,N,E,P", [(640, 144, 4, 37), (768, 256, 3, 16), (896, 2048, 8, 128), (1152, 272, 2, 250)])
+def test_gathered_experts_of_any_k(native_lib, K, N, E, P):
+    cases = [make_qmm_case(K, N, 500 + e).to(DEV) for e in range(E)]
+    w, s, b = (torch.stack([getattr(c, n) for c in cases]) for n in ("w", "scales", "biases"))
+    gen = torch.Generator().manual_seed(K)
+    ids = torch.randint(-1, E + 1, (P,), generator=gen).to(torch.int32).to(DEV)  # some belong to no expert
+    x = torch.randn(P, K, generator=gen).to(torch.bfloat16).to(DEV)
+    y = VQ.gather_qmm(x, w, s, b, ids)
+    for e in range(E):
+        rows = ids == e
+        if bool(rows.any()):
+            _check(y[rows], x[rows], dequantize(w[e], s[e], b[e], 64, 4, dtype=torch.float64), K, torch.bfloat16)
+    assert bool((y[(ids < 0) | (ids >= E)] == 0).all())
+    assert torch.equal(y, VQ.gather_qmm(x, w, s, b, ids))
