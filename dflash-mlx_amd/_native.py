@@ -110,9 +110,9 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.dflash_qmm_m16_packed.restype = c.c_int
     lib.dflash_qmm_m16_packed.argtypes = [c.c_void_p] * 6 + [c.c_size_t] + [c.c_int] * 5 + [c.c_void_p]
     lib.dflash_qmm_rows_workspace_bytes.restype = c.c_size_t
-    lib.dflash_qmm_rows_workspace_bytes.argtypes = [c.c_int] * 4
+    lib.dflash_qmm_rows_workspace_bytes.argtypes = [c.c_int] * 7
     lib.dflash_qmm_rows.restype = c.c_int
-    lib.dflash_qmm_rows.argtypes = [c.c_void_p] * 6 + [c.c_size_t] + [c.c_int] * 6 + [c.c_void_p]
+    lib.dflash_qmm_rows.argtypes = [c.c_void_p] * 6 + [c.c_size_t] + [c.c_int] * 7 + [c.c_void_p]
     lib.dflash_qmm_m16_gather_workspace_bytes.restype = c.c_size_t
     lib.dflash_qmm_m16_gather_workspace_bytes.argtypes = [c.c_int] * 5
     lib.dflash_qmm_m16_gather.restype = c.c_int

@@ -26,7 +26,7 @@ import torch
 import torch.nn as nn
 
 from .quantized import QuantizedLinear, stock_matmul
-from .verify_qmm import (ChainProblem, QmmChain, _should_use_verify, pack_weights, packable, verify_matmul,
+from .verify_qmm import (ChainProblem, QmmChain, _should_use_verify, pack_weights, packable, rows_matmul, verify_matmul,
                          verify_matmul_packed)
 
 _VERIFY_MAX_N_DEFAULT = 100_000
@@ -129,7 +129,18 @@ class FusedProjections:
         m = 1
         for d in x.shape[:-1]:
             m *= d
-        if m != 16 or x.device != self.weight.device or not _should_use_verify(x, self.group_size, self.bits, True):
+        if m != 16 or not _should_use_verify(x, self.group_size, self.bits, True):
+            return False
+        return self._holds(parent, x)
+
+    def serves_prompt(self, parent: nn.Module, x: torch.Tensor) -> bool:
+        """The same for more rows than a block has, which take the any-rows product of the joint matrix
+        (``prompt``): device activations, outside the verify switch."""
+        return (x.is_cuda and x.ndim >= 2 and x.numel() > 16 * int(x.shape[-1]) and self.bits == 4
+                and os.environ.get("DFLASH_STOCK_KERNEL", "1") != "0" and self._holds(parent, x))
+
+    def _holds(self, parent: nn.Module, x: torch.Tensor) -> bool:
+        if x.device != self.weight.device:
             return False
         for index, name in enumerate(self.names):
             mod = getattr(parent, name, None)
@@ -167,6 +178,13 @@ class FusedProjections:
         chain()
         return out
 
+    def prompt(self, x: torch.Tensor, epilogue: Optional[str] = None) -> Optional[torch.Tensor]:
+        """The joint product (with ``epilogue="silu_mul"`` the gated activation) of any number of rows, or
+        None where that kernel does not apply."""
+        if epilogue is not None and not (len(self.bounds) == 2 and self.bounds[1] == (self.bounds[0][1], 2 * self.bounds[0][1])):
+            return None
+        return rows_matmul(x, self.weight, self.scales, self.biases, group_size=self.group_size, bits=self.bits, epilogue=epilogue)
+
     def __call__(self, x: torch.Tensor) -> Tuple[torch.Tensor, ...]:
         if self._packed is not None and x.is_cuda:
             product = verify_matmul_packed(x, self._packed)
@@ -185,13 +203,18 @@ def silu_gate_up(parent: nn.Module, x: torch.Tensor, names: Tuple[str, str] = ("
     activation and the product applied before anything is stored (``dflash_qmm_m16_chain`` with
     its silu-mul epilogue; every operator's rounding to the activation dtype is kept, the split
     of K between workgroups differs from the separate projections', so single results may
-    differ by one rounding of the array dtype).  Everything else goes through
+    differ by one rounding of the array dtype).  Prompts (more than 16 rows) take one launch of the
+    any-rows product with the same epilogue.  Everything else goes through
     ``shared_input_outputs`` and the array operators.  No counterpart in the reference, whose MLP
     is mlx-lm's ``down_proj(swiglu(gate_proj(x), up_proj(x)))``; 27B shape: gate/up/activation
     48 us with ``down_proj`` against 60 us for the four separate steps."""
     for group in getattr(parent, "_dflash_fused", ()):
         if group.names == tuple(names) and group.applies(parent, x) and group.silu_mul_ready(x):
             return group.silu_mul(x)
+        if group.names == tuple(names) and group.serves_prompt(parent, x):
+            hidden = group.prompt(x, "silu_mul")
+            if hidden is not None:
+                return hidden
     gate, up = shared_input_outputs(parent, names, x)
     return (gate * torch.sigmoid(gate)) * up   # x * sigmoid(x): the operators the epilogue follows, one rounding each
 
@@ -203,6 +226,10 @@ def shared_input_outputs(parent: nn.Module, names: Sequence[str], x: torch.Tenso
     for group in getattr(parent, "_dflash_fused", ()):
         if all(n in names for n in group.names) and group.applies(parent, x):
             outs.update(zip(group.names, group(x)))
+        elif all(n in names for n in group.names) and group.serves_prompt(parent, x):
+            product = group.prompt(x)
+            if product is not None:
+                outs.update((n, product[..., lo:hi]) for n, (lo, hi) in zip(group.names, group.bounds))
     return tuple(outs[n] if n in outs else getattr(parent, n)(x) for n in names)
 
 

@@ -493,12 +493,17 @@ def small_m_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biase
 _ROWS_WORKSPACES: Dict[Tuple[int, int], torch.Tensor] = {}
 
 
+# what dflash_qmm_rows_workspace_bytes answered per call shape
+_ROWS_WORKSPACE_BYTES: Dict[Tuple[int, ...], int] = {}
+
+
 def rows_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
-                *, group_size: int = 64, bits: int = 4) -> "torch.Tensor | None":
+                *, group_size: int = 64, bits: int = 4, epilogue: Optional[str] = None) -> "torch.Tensor | None":
     """``x @ dequant(w).T`` for any number of rows of device activations in one launch
     (``dflash_qmm_rows``): weights are dequantised to the activation type inside the product.
     Returns None for what the kernel does not cover (other bit widths, fp32, N not a multiple of
-    16).  No counterpart in the reference, whose stock operator is ``mx.quantized_matmul``."""
+    16).  ``epilogue="silu_mul"``: ``w`` holds the gate rows of an MLP followed by its up rows and the result is
+    ``silu(gate) * up``.  No counterpart in the reference, whose stock operator is ``mx.quantized_matmul``."""
     if (not x.is_cuda or bits != 4 or group_size not in (32, 64, 128) or x.dtype not in _DTYPE_CODE or
             scales.dtype not in _DTYPE_CODE or biases.dtype != scales.dtype or w.ndim != 2 or not _native.is_built()):
         return None
@@ -506,28 +511,39 @@ def rows_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: 
     M = x.numel() // K if K else 0
     if M < 1 or N % 16 != 0 or K % group_size != 0 or int(w.shape[1]) * 8 != K:
         return None
+    code = _native.QMM_EPILOGUE_NONE
+    if epilogue is not None:
+        code = _native.QMM_EPILOGUE_SILU_MUL
+        if epilogue != "silu_mul" or N % 32 != 0 or scales.dtype != x.dtype:
+            return None
     w, scales, biases = w.contiguous(), scales.contiguous(), biases.contiguous()
     _require_operands("quantized_matmul", K, N, group_size, w, scales, biases, x.device)
     x2 = x.reshape(M, K).contiguous()
     if (x2.data_ptr() | w.data_ptr()) % 16:
         return None
     lib = _native.lib()
-    y = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    cols = N if code == _native.QMM_EPILOGUE_NONE else N // 2
+    y = torch.empty((M, cols), dtype=x.dtype, device=x.device)
     stream = _native.raw_stream(x.device)
-    need = int(lib.dflash_qmm_rows_workspace_bytes(M, K, N, group_size))
+    index = x.device.index if x.device.index is not None else torch.cuda.current_device()
+    shape = (M, K, N, group_size, _DTYPE_CODE[x.dtype], _DTYPE_CODE[scales.dtype], code)
+    need = _ROWS_WORKSPACE_BYTES.get((index, *shape))
+    if need is None:
+        if len(_ROWS_WORKSPACE_BYTES) > 4096:  # prompts come in every length
+            _ROWS_WORKSPACE_BYTES.clear()
+        need = _ROWS_WORKSPACE_BYTES[(index, *shape)] = int(lib.dflash_qmm_rows_workspace_bytes(*shape))
     ws_ptr, ws_bytes = None, 0
     if need:
-        key = (x.device.index if x.device.index is not None else torch.cuda.current_device(), stream)
-        ws = _ROWS_WORKSPACES.get(key)
+        ws = _ROWS_WORKSPACES.get((index, stream))
         if ws is None or ws.numel() < need:
             ws = torch.empty(max(need, 1 << 23), dtype=torch.uint8, device=x.device)
             ws[:1 << 16].zero_()
-            _ROWS_WORKSPACES[key] = ws
+            _ROWS_WORKSPACES[(index, stream)] = ws
         ws_ptr, ws_bytes = ws.data_ptr(), ws.numel()
     rc = lib.dflash_qmm_rows(x2.data_ptr(), w.data_ptr(), scales.data_ptr(), biases.data_ptr(), y.data_ptr(), ws_ptr,
-                             ws_bytes, M, K, N, group_size, _DTYPE_CODE[x.dtype], _DTYPE_CODE[scales.dtype], stream)
+                             ws_bytes, *shape, stream)
     _native.check(rc, "dflash_qmm_rows")
-    return y.reshape(*x.shape[:-1], N)
+    return y.reshape(*x.shape[:-1], cols)
 
 
 def gather_qmm(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,

@@ -264,12 +264,14 @@ int dflash_qmm_m16_packed(const void* x, const void* codes, const void* scales, 
  * 64 KiB zero-filled once by the caller and handed back zero-filled; the rest holds partial tiles and
  * need not be cleared.  NOT shareable with the other qmm entry points' workspace.  Calls that share
  * it must not overlap in time.  Deterministic.
+ * epilogue DFLASH_QMM_EPILOGUE_SILU_MUL: w_q, scales, biases hold N/2 gate rows followed by N/2 up rows, and y
+ * [M, N/2] is silu(gate) * up with every operator's rounding to act_dtype; N % 32 == 0, act_dtype == sb_dtype.
  */
-size_t dflash_qmm_rows_workspace_bytes(int M, int K, int N, int group_size);
+size_t dflash_qmm_rows_workspace_bytes(int M, int K, int N, int group_size, int act_dtype, int sb_dtype, int epilogue);
 
 int dflash_qmm_rows(const void* x, const uint32_t* w_q, const void* scales, const void* biases, void* y,
                     void* workspace, size_t workspace_bytes, int M, int K, int N, int group_size,
-                    int act_dtype, int sb_dtype, void* stream);
+                    int act_dtype, int sb_dtype, int epilogue, void* stream);
 
 /*
  * Gathered per-expert M<=16-per-expert qmm for MoE layers: y[p,:] = x[p,:] . (s*q + b)^T of

@@ -41,3 +41,20 @@ def test_leading_dimensions_and_switch(native_lib, monkeypatch):
     monkeypatch.setenv("DFLASH_STOCK_KERNEL", "0")
     arrays = quantized_matmul(c.x, c.w, c.scales, c.biases)
     assert (y.reshape(40, 96).float() - arrays.float()).norm() <= 2 ** -8 * arrays.float().norm()
+
+
+@pytest.mark.parametrize("M,K,N,group,dtype", [
+    (17, 128, 32, 64, torch.bfloat16), (33, 1024, 544, 32, torch.float16), (77, 512, 1024, 64, torch.bfloat16),
+    (112, 640, 96, 128, torch.bfloat16), (130, 1024, 2080, 64, torch.bfloat16), (600, 256, 8192, 64, torch.float16)])
+def test_gated_activation_in_the_product(native_lib, M, K, N, group, dtype):
+    """The silu-mul epilogue: the operators applied one by one to the product of the same rows.  The two products may
+    be cut into different slices of K, so a result may differ by the rounding of a factor or two."""
+    c = make_qmm_case(K, N, 2000 + M, group_size=group, dtype=dtype, M=M).to(DEV)
+    c.scales.mul_(0.05); c.biases.mul_(0.05)
+    h = rows_matmul(c.x, c.w, c.scales, c.biases, group_size=group, epilogue="silu_mul")
+    gate, up = rows_matmul(c.x, c.w, c.scales, c.biases, group_size=group).split(N // 2, dim=-1)
+    ops = ((gate * torch.sigmoid(gate)) * up).float()
+    assert h.shape == (M, N // 2) and h.dtype == dtype
+    eps = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    assert ((h.float() - ops).abs() <= 4 * eps * ops.abs() + eps * (gate * up).abs().float() * 1e-2 + 1e-6).all()
+    assert float((h.float() != ops).float().mean()) <= 2e-2
