@@ -12,7 +12,7 @@ from typing import Optional
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libdflash_mi355.so")
 
-ABI_VERSION = 20
+ABI_VERSION = 21
 
 BF16, FP16, FP32 = 0, 1, 2
 QMM_MMA2BIG, QMM_MMA2BIG_PIPE = 0, 1
@@ -61,6 +61,8 @@ EXPORTED_SYMBOLS = (
     "dflash_gdn_forward",
     "dflash_gdn_prepare",
     "dflash_gdn_gated_norm",
+    "dflash_attn_prepare",
+    "dflash_attn_gate",
     "dflash_sdpa_q16_workspace_bytes",
     "dflash_sdpa_q16",
     "dflash_conv_state_rebuild",
@@ -131,6 +133,11 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.dflash_gdn_prepare.argtypes = [c.c_void_p] * 14 + [c.c_int] * 9 + [c.c_float, c.c_void_p]
     lib.dflash_gdn_gated_norm.restype = c.c_int
     lib.dflash_gdn_gated_norm.argtypes = [c.c_void_p] * 4 + [c.c_longlong] + [c.c_int] * 3 + [c.c_float, c.c_void_p]
+    lib.dflash_attn_prepare.restype = c.c_int
+    lib.dflash_attn_prepare.argtypes = ([c.c_void_p] * 8 + [c.c_int] * 7 + [c.POINTER(c.c_longlong)] + [c.c_float] * 3 +
+                                        [c.c_int] * 3 + [c.c_void_p])
+    lib.dflash_attn_gate.restype = c.c_int
+    lib.dflash_attn_gate.argtypes = [c.c_void_p] * 3 + [c.c_int] * 4 + [c.c_longlong] * 5 + [c.c_int, c.c_void_p]
     lib.dflash_sdpa_q16_workspace_bytes.restype = c.c_size_t
     lib.dflash_sdpa_q16_workspace_bytes.argtypes = [c.c_int] * 5
     lib.dflash_sdpa_q16.restype = c.c_int

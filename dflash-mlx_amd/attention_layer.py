@@ -10,14 +10,17 @@ k_proj, v_proj, o_proj, scale, num_attention_heads, num_key_value_heads).
 """
 from __future__ import annotations
 
+import ctypes
 from typing import Any, Optional
 
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from . import _native
+from .cache import KVCache
 from .gdn_layer import rms_norm_ops
-from .kernels import batched_sdpa_2pass_exact
+from .kernels import _DTYPE_CODE, batched_sdpa_2pass_exact
 from .verify_linear import shared_input_outputs
 
 _HYBRID_SDPA_EXACT_KV_THRESHOLD = 1024
@@ -144,6 +147,9 @@ def _project(self, x: torch.Tensor, cache: Optional[Any]):
     num_key_value_heads = _attention_num_kv_heads(self)
     # one launch for the three where fuse_shared_input_linears joined them
     q_proj_output, keys, values = shared_input_outputs(self, ("q_proj", "k_proj", "v_proj"), x)
+    on_device = _project_on_device(self, q_proj_output, keys, values, cache)
+    if on_device is not None:
+        return on_device
     queries, gate = torch.chunk(q_proj_output.reshape(B, L, num_attention_heads, -1), 2, dim=-1)
     gate = gate.reshape(B, L, -1)
     queries = self.q_norm(queries).transpose(1, 2)
@@ -160,8 +166,83 @@ def _project(self, x: torch.Tensor, cache: Optional[Any]):
     return queries, keys, values, gate, cached_prefix_len
 
 
+def _plain(*tensors: torch.Tensor) -> bool:
+    """Ordinary device tensors that nothing is differentiating, tracing or batching: what a kernel that takes
+    their addresses may stand in for the array operators on."""
+    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+        return False
+    if any(type(t) not in (torch.Tensor, nn.Parameter) or not t.is_cuda for t in tensors):
+        return False
+    return (torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None
+            and torch._C._get_tracing_state() is None and not torch.compiler.is_compiling())
+
+
+def _unhooked(module: nn.Module) -> bool:
+    return not (module._forward_hooks or module._forward_pre_hooks)
+
+
+def _project_on_device(self, q_proj_output: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, cache: Any):
+    """Everything behind the projections in one launch (``dflash_attn_prepare``), keys and values straight into
+    the cache; the gate stays where q_proj put it.  None - the caller then takes the array operators - for
+    what the kernel does not cover: other caches, norms and rotary modules than this package's, host tensors, fp32
+    activations, head sizes other than 64, 128, 192 and 256, a cache of another type or batch."""
+    q_norm, k_norm, rope = self.q_norm, self.k_norm, self.rope
+    if type(cache) is not KVCache or type(q_norm) is not HeadRMSNorm or type(k_norm) is not HeadRMSNorm \
+            or type(rope) is not RotaryEmbedding or not (_unhooked(q_norm) and _unhooked(k_norm) and _unhooked(rope)):
+        return None
+    code = _DTYPE_CODE.get(q_proj_output.dtype)
+    if code is None or code == _native.FP32 or q_proj_output.ndim != 3 or not _plain(q_proj_output, keys, values):
+        return None
+    B, L, width = q_proj_output.shape
+    Hq, Hk = _attention_num_heads(self), _attention_num_kv_heads(self)
+    D = width // (2 * Hq)
+    qw, kw, device, dtype = q_norm.weight, k_norm.weight, q_proj_output.device, q_proj_output.dtype
+    per = D // 64
+    if (D not in (64, 128, 192, 256) or width != 2 * Hq * D or not 0 < rope.dims <= D or rope.dims % (2 * per)
+            or tuple(keys.shape) != (B, L, Hk * D) or keys.shape != values.shape or B * L == 0):
+        return None
+    if not (keys.dtype == values.dtype == dtype and keys.device == values.device == device == qw.device == kw.device
+            and tuple(qw.shape) == (D,) == tuple(kw.shape) and qw.dtype in _DTYPE_CODE and kw.dtype in _DTYPE_CODE
+            and qw.is_contiguous() and kw.is_contiguous() and _plain(qw, kw)):
+        return None
+    for held in (cache.keys, cache.values):
+        if held is not None and (tuple(held.shape[:2]) != (B, Hk) or held.shape[3] != D or held.dtype != dtype
+                                 or held.device != device or held.stride(3) != 1 or not _plain(held)):
+            return None
+    if any(t.stride(2) != 1 or (t.stride(0) | t.stride(1)) % 4 or t.data_ptr() % 8 for t in (q_proj_output, keys, values)) \
+            or (qw.data_ptr() | kw.data_ptr()) % 8:
+        return None
+    for held in (cache.keys, cache.values):
+        if held is not None and (held.data_ptr() % 8 or (held.stride(0) | held.stride(1) | held.stride(2)) % 4):
+            return None
+    prev = cache._append_room(B, Hk, L, D, D, keys, values)
+    ko, vo = cache.keys, cache.values
+    queries = torch.empty((B, Hq, L, D), dtype=dtype, device=device)
+    strides = (ctypes.c_longlong * 12)(q_proj_output.stride(0), q_proj_output.stride(1), keys.stride(0), keys.stride(1),
+                                       values.stride(0), values.stride(1), *ko.stride()[:3], *vo.stride()[:3])
+    rc = _native.lib().dflash_attn_prepare(
+        q_proj_output.data_ptr(), keys.data_ptr(), values.data_ptr(), qw.data_ptr(), kw.data_ptr(), queries.data_ptr(),
+        ko.data_ptr() + 2 * prev * ko.stride(2), vo.data_ptr() + 2 * prev * vo.stride(2), B, L, Hq, Hk, D, rope.dims, prev,
+        strides, q_norm.eps, k_norm.eps, float(rope.base), code, _DTYPE_CODE[qw.dtype], _DTYPE_CODE[kw.dtype],
+        _native.raw_stream(device))
+    _native.check(rc, "dflash_attn_prepare")
+    end = prev + L
+    return queries, ko[:, :, :end], vo[:, :, :end], q_proj_output, prev
+
+
 def _finish(self, output: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
-    B, _, L, _ = output.shape
+    """``gate`` [B, L, Hq * D], or the whole output of q_proj, [B, L, Hq * 2 D], as ``_project_on_device`` leaves it."""
+    B, H, L, D = output.shape
+    if gate.shape[-1] == 2 * H * D:
+        if (output.dtype == gate.dtype and _plain(output) and output.stride(3) == 1 and output.data_ptr() % 8 == 0
+                and (output.stride(0) | output.stride(1) | output.stride(2)) % 4 == 0):
+            gated = torch.empty((B, L, H * D), dtype=output.dtype, device=output.device)
+            rc = _native.lib().dflash_attn_gate(
+                output.data_ptr(), gate.data_ptr(), gated.data_ptr(), B, L, H, D, *output.stride()[:3], gate.stride(0),
+                gate.stride(1), _DTYPE_CODE[output.dtype], _native.raw_stream(output.device))
+            _native.check(rc, "dflash_attn_gate")
+            return self.o_proj(gated)
+        gate = gate.reshape(B, L, H, 2 * D)[..., D:].reshape(B, L, -1)
     output = output.transpose(1, 2).reshape(B, L, -1)
     return self.o_proj(output * torch.sigmoid(gate))
 

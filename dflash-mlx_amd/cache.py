@@ -24,11 +24,17 @@ class KVCache:
 
     def update_and_fetch(self, keys: torch.Tensor, values: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
         """Append ``keys``/``values`` ``[B, H, S, D]`` at ``offset``; return the filled prefix."""
+        b, h, s, dk = keys.shape
+        prev = self._append_room(b, h, s, dk, values.shape[3], keys, values)
+        self.keys[:, :, prev:self.offset] = keys
+        self.values[:, :, prev:self.offset] = values
+        return self.keys[:, :, :self.offset], self.values[:, :, :self.offset]
+
+    def _append_room(self, b: int, h: int, s: int, dk: int, dv: int, keys: torch.Tensor, values: torch.Tensor) -> int:
+        """Moves ``offset`` past ``s`` more rows, growing the buffers where they are too short (types and devices
+        as ``keys`` / ``values``); returns where the new rows start."""
         prev = self.offset
-        s = keys.shape[2]
         if self.keys is None or prev + s > self.keys.shape[2]:
-            b, h, _, dk = keys.shape
-            dv = values.shape[3]
             n_steps = (self.step + s - 1) // self.step
             new_k = torch.zeros((b, h, n_steps * self.step, dk), dtype=keys.dtype, device=keys.device)
             new_v = torch.zeros((b, h, n_steps * self.step, dv), dtype=values.dtype, device=values.device)
@@ -38,9 +44,7 @@ class KVCache:
             else:
                 self.keys, self.values = new_k, new_v
         self.offset = prev + s
-        self.keys[:, :, prev:self.offset] = keys
-        self.values[:, :, prev:self.offset] = values
-        return self.keys[:, :, :self.offset], self.values[:, :, :self.offset]
+        return prev
 
     def is_trimmable(self) -> bool:
         return True

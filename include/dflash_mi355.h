@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define DFLASH_ABI_VERSION 20
+#define DFLASH_ABI_VERSION 21
 
 enum {
   DFLASH_OK = 0,
@@ -420,6 +420,31 @@ int dflash_gdn_prepare(const void* qkv, const void* conv_state, const void* conv
  */
 int dflash_gdn_gated_norm(const void* x, const void* z, const void* weight, void* y, long long rows,
                           int D, int dtype, int weight_dtype, float eps, void* stream);
+
+/*
+ * What a gated attention layer does between its projections and its attention, in one launch: replaces the
+ * array operators of dflash_mlx/runtime.py:527-556 (split of q_proj into queries and gate, head norms, rotary embedding,
+ * cache update).  One rounding to `dtype` per operator, fp32 inside.
+ *     n = rms_norm(head, weight, eps);  positions offset .. offset + L - 1, features i and i + rope_dims / 2 of the first
+ *     rope_dims turned by position * rope_base^(-2 i / rope_dims);  the rest and v as they are
+ *   q [B, L, Hq, 2 D] (a head's queries, then its gate), k, v [B, L, Hk, D]; heads and features contiguous
+ *   q_weight, k_weight [D];  q_out [B, Hq, L, D] contiguous;  k_out, v_out: rows of a cache, [B, Hk, L, D]
+ *   strides: 12 element counts - batch, row of q, k, v; batch, head, row of k_out, v_out
+ * bf16 / fp16; D a multiple of 64 up to 256, rope_dims a multiple of D / 32; pointers and rows 8-byte aligned.
+ */
+int dflash_attn_prepare(const void* q, const void* k, const void* v, const void* q_weight, const void* k_weight,
+                        void* q_out, void* k_out, void* v_out, int B, int L, int Hq, int Hk, int D, int rope_dims,
+                        int offset, const long long* strides, float q_eps, float k_eps, float rope_base, int dtype,
+                        int q_weight_dtype, int k_weight_dtype, void* stream);
+
+/*
+ * The layer's output gate: y[b, l, h, :] = o[b, h, l, :] * sigmoid(gate[b, l, h, D:]), the sigmoid and the product rounded
+ * to `dtype` (dflash_mlx/runtime.py:606-616).  o with the strides given (features contiguous), gate the q_proj output
+ * [B, L, Hq, 2 D], y [B, L, Hq, D] contiguous.  Same types, head dims and alignment as above.
+ */
+int dflash_attn_gate(const void* o, const void* gate, void* y, int B, int L, int Hq, int D, long long o_batch_stride,
+                     long long o_head_stride, long long o_row_stride, long long gate_batch_stride,
+                     long long gate_row_stride, int dtype, void* stream);
 
 /*
  * Exact attention of a verify block of 16 queries over a long KV cache.  Replaces the two

@@ -1,0 +1,104 @@
+"""The one-launch glue of a gated attention layer (dflash_attn_prepare, dflash_attn_gate) against the array operators of the
+same layer, and both against float64, at the edges of its range: one token, ragged prompts, every head size,
+partial rotation, strided projections, caches that grow."""
+import pytest
+import torch
+
+from dflash_mlx_amd import attention_layer as A
+from dflash_mlx_amd.cache import KVCache
+
+pytestmark = pytest.mark.gpu
+
+
+class _Given(torch.nn.Module):
+    """A projection whose output is given: columns lo .. hi of a joint product."""
+
+    def __init__(self, out):
+        super().__init__()
+        self.out = out
+
+    def forward(self, x):
+        return self.out
+
+
+def _layer(B, L, Hq, Hk, D, dims, dtype, wdtype, gen, joint):
+    widths = (2 * Hq * D, Hk * D, Hk * D)
+    full = torch.randn((B, L, sum(widths)), generator=gen, device="cuda").to(dtype)
+    outs = torch.split(full, widths, dim=-1)
+    if not joint:
+        outs = [o.contiguous() for o in outs]
+    attn = A.GatedAttention(num_attention_heads=Hq, num_key_value_heads=Hk, head_dim=D, q_proj=_Given(outs[0]),
+                            k_proj=_Given(outs[1]), v_proj=_Given(outs[2]), o_proj=torch.nn.Identity(), rope_dims=dims)
+    for norm in (attn.q_norm, attn.k_norm):
+        norm.weight = torch.nn.Parameter((1 + 0.2 * torch.randn(D, generator=gen, device="cuda")).to(wdtype), requires_grad=False)
+    return attn, outs
+
+
+def _exact(head, weight, dims, offset, eps=1e-6):
+    x = head.double()
+    n = x / torch.sqrt((x * x).mean(-1, keepdim=True) + eps) * weight.double()
+    half = dims // 2
+    freq = 10000.0 ** (-torch.arange(half, device=x.device, dtype=torch.float64) / half)
+    angle = torch.arange(offset, offset + x.shape[1], device=x.device, dtype=torch.float64)[:, None] * freq
+    c, s = torch.cos(angle)[None, :, None], torch.sin(angle)[None, :, None]
+    a, b = n[..., :half], n[..., half:dims]
+    return torch.cat([a * c - b * s, a * s + b * c, n[..., dims:]], dim=-1).transpose(1, 2)
+
+
+@pytest.mark.parametrize("B,L,Hq,Hk,D,dims,prefix,dtype,wdtype,joint", [
+    (1, 16, 32, 8, 256, 256, 4096, torch.bfloat16, torch.bfloat16, True),
+    (1, 16, 16, 4, 256, 64, 240, torch.bfloat16, torch.float32, True),      # quarter rotation; the cache grows here
+    (1, 1, 64, 8, 128, 128, 32700, torch.float16, torch.float16, False),    # one token, long angles
+    (2, 77, 8, 2, 64, 64, 0, torch.bfloat16, torch.bfloat16, True),         # empty cache, two sequences
+    (1, 5, 3, 1, 192, 96, 7, torch.float16, torch.bfloat16, False),         # three features per lane
+    (1, 1030, 24, 4, 256, 256, 3, torch.bfloat16, torch.bfloat16, True),    # several heads per wave
+])
+def test_prepare_equals_the_array_operators(monkeypatch, B, L, Hq, Hk, D, dims, prefix, dtype, wdtype, joint):
+    gen = torch.Generator(device="cuda").manual_seed(11)
+    attn, outs = _layer(B, L, Hq, Hk, D, dims, dtype, wdtype, gen, joint)
+    x = torch.empty((B, L, 8), device="cuda")
+    before = [torch.randn((B, Hk, prefix, D), generator=gen, device="cuda").to(dtype) for _ in range(2)]
+    caches = [KVCache(), KVCache()]
+    for c in caches:
+        if prefix:
+            c.update_and_fetch(*before)
+    queries, keys, values, gate, prev = A._project(attn, x, caches[0])
+    assert gate is not None and gate.shape[-1] == 2 * Hq * D and prev == prefix  # the kernel took it
+    monkeypatch.setattr(A, "_project_on_device", lambda *a: None)
+    ref_q, ref_k, ref_v, ref_gate, _ = A._project(attn, x, caches[1])
+    assert caches[0].offset == caches[1].offset == prefix + L and caches[0].keys.shape == caches[1].keys.shape
+    assert torch.equal(values, ref_v) and torch.equal(keys[:, :, :prefix], ref_k[:, :, :prefix])
+    # the sum of squares is taken in another order: a normed feature may fall on the next value of the type (eps of itself),
+    # a turned one is the sum of two of them, rounded once more
+    eps = torch.finfo(dtype).eps
+    for got, ref, head, norm in ((queries, ref_q, outs[0].reshape(B, L, Hq, 2 * D)[..., :D], attn.q_norm),
+                                 (keys[:, :, prefix:], ref_k[:, :, prefix:], outs[1].reshape(B, L, Hk, D), attn.k_norm)):
+        exact = _exact(head, norm.weight, dims, prefix)
+        size = exact.abs()
+        pair = size.clone()
+        pair[..., :dims // 2] += size[..., dims // 2:dims]
+        pair[..., dims // 2:dims] += size[..., :dims // 2]
+        assert ((got.double() - ref.double()).abs() <= 3 * eps * 1.5 * pair + 1e-6).all()
+        err = [((t.double() - exact).norm() / exact.norm()).item() for t in (got, ref)]
+        assert err[0] <= 1.01 * err[1]
+    out = torch.randn((B, L, Hq, D), generator=gen, device="cuda").to(dtype)
+    for o in (out.transpose(1, 2), out.transpose(1, 2).contiguous()):  # either order an attention may leave
+        assert torch.equal(A._finish(attn, o, gate), A._finish(attn, o, ref_gate))
+
+
+def test_what_the_kernel_does_not_cover_goes_to_the_array_operators():
+    gen = torch.Generator(device="cuda").manual_seed(12)
+    x = torch.empty((1, 4, 8), device="cuda")
+    for change in ("hook", "cache", "grad", "fp32", "odd"):
+        dtype = torch.float32 if change == "fp32" else torch.bfloat16
+        attn, outs = _layer(1, 4, 4, 2, 96 if change == "odd" else 128, 64, dtype, dtype, gen, True)
+        cache = KVCache()
+        if change == "hook":
+            attn.q_norm.register_forward_hook(lambda m, i, o: o)
+        if change == "cache":
+            cache = type("Other", (KVCache,), {})()
+        if change == "grad":
+            attn.q_proj.out = outs[0].clone().requires_grad_(True)
+        queries, keys, _, gate, _ = A._project(attn, x, cache)
+        assert gate.shape[-1] == queries.shape[1] * queries.shape[-1], change
+        assert queries.requires_grad == (change == "grad")
