@@ -42,6 +42,8 @@ EXPORTED_SYMBOLS = (
     "dflash_qmm_m16_workspace_bytes",
     "dflash_qmm_m16",
     "dflash_qmm_few",
+    "dflash_qmm_few_silu_mul_workspace_bytes",
+    "dflash_qmm_few_silu_mul",
     "dflash_qmm_error",
     "dflash_qmm_m16_static",
     "dflash_qmm_m16_pack_gate_up",
@@ -95,6 +97,10 @@ def _declare(lib: ctypes.CDLL) -> None:
     )
     lib.dflash_qmm_few.restype = c.c_int
     lib.dflash_qmm_few.argtypes = [c.c_void_p] * 6 + [c.c_size_t] + [c.c_int] * 7 + [c.c_void_p]
+    lib.dflash_qmm_few_silu_mul_workspace_bytes.restype = c.c_size_t
+    lib.dflash_qmm_few_silu_mul_workspace_bytes.argtypes = [c.c_int] * 3
+    lib.dflash_qmm_few_silu_mul.restype = c.c_int
+    lib.dflash_qmm_few_silu_mul.argtypes = [c.c_void_p] * 6 + [c.c_size_t] + [c.c_int] * 5 + [c.c_void_p]
     lib.dflash_qmm_error.restype = c.c_int
     lib.dflash_qmm_error.argtypes = [c.c_void_p, c.POINTER(c.c_uint32), c.c_void_p]
     lib.dflash_qmm_m16_static.restype = c.c_int

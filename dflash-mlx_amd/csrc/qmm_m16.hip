@@ -423,7 +423,7 @@ size_t qmm_stream_workspace_bytes(int N, int grid);
 int qmm_stream_grid();
 int qmm_stream_launch(const void* x, const uint32_t* w, const void* scales, const void* biases,
                       void* y, void* workspace, size_t workspace_bytes, int M, int K, int N,
-                      int group_size, int act_dtype, int sb_dtype, hipStream_t stream);
+                      int group_size, int act_dtype, int sb_dtype, bool silu_mul, hipStream_t stream);
 bool qmm_stream_gather_eligible(int P, int K, int N, int E, int group_size);
 int qmm_stream_gather_launch(const void* x, const int32_t* expert_ids, const uint32_t* w,
                              const void* scales, const void* biases, void* y, void* workspace,
@@ -477,6 +477,28 @@ extern "C" int dflash_qmm_few(const void* x, const uint32_t* w_q, const void* sc
                               DFLASH_QMM_MMA2BIG, 1, kernel, stream);
 }
 
+extern "C" size_t dflash_qmm_few_silu_mul_workspace_bytes(int K, int N, int group_size) {
+  using namespace dflash;
+  if (!qmm_stream_eligible(K, N, group_size) && !qmm_stream_any_eligible(K, N, group_size)) return 0;
+  return qmm_stream_workspace_bytes(N, qmm_stream_grid());
+}
+
+extern "C" int dflash_qmm_few_silu_mul(const void* x, const uint32_t* w_q, const void* scales, const void* biases, void* y,
+                                       void* workspace, size_t workspace_bytes, int M, int K, int N, int group_size,
+                                       int dtype, void* stream) {
+  using namespace dflash;
+  DFLASH_REQUIRE(x && w_q && scales && biases && y, DFLASH_ERR_ARG, "dflash_qmm_few_silu_mul: null operand");
+  DFLASH_REQUIRE(dtype == DFLASH_BF16 || dtype == DFLASH_FP16, DFLASH_ERR_ARG, "dflash_qmm_few_silu_mul: dtype %d is not bf16/fp16",
+                 dtype);
+  DFLASH_REQUIRE(M >= 1 && M <= 16, DFLASH_ERR_SHAPE, "dflash_qmm_few_silu_mul: 1 to 16 rows, got %d", M);
+  DFLASH_REQUIRE(qmm_stream_eligible(K, N, group_size) || qmm_stream_any_eligible(K, N, group_size), DFLASH_ERR_SHAPE,
+                 "dflash_qmm_few_silu_mul: the streaming kernel does not cover K=%d N=%d gs=%d", K, N, group_size);
+  DFLASH_REQUIRE((((uintptr_t)x | (uintptr_t)w_q) % 16) == 0 && (((uintptr_t)scales | (uintptr_t)biases) % 4) == 0,
+                 DFLASH_ERR_ARG, "dflash_qmm_few_silu_mul: x and w_q must be 16-byte aligned, scales and biases 4-byte aligned");
+  return qmm_stream_launch(x, w_q, scales, biases, y, workspace, workspace_bytes, M, K, N, group_size, dtype, dtype, true,
+                           (hipStream_t)stream);
+}
+
 namespace dflash {
 namespace {
 int qmm_up_to_16(const void* x, const uint32_t* w_q, const void* scales, const void* biases, void* y, void* workspace,
@@ -508,7 +530,7 @@ int qmm_up_to_16(const void* x, const uint32_t* w_q, const void* scales, const v
                    workspace_bytes >= qmm_stream_workspace_bytes(N, qmm_stream_grid());
   if (kernel != DFLASH_QMM_KERNEL_TILE && (qmm_stream_eligible(K, N, group_size) || any)) {
     return qmm_stream_launch(x, w_q, scales, biases, y, workspace, workspace_bytes, M, K, N, group_size, act_dtype,
-                             sb_dtype, (hipStream_t)stream);
+                             sb_dtype, false, (hipStream_t)stream);
   }
   DFLASH_REQUIRE(kernel != DFLASH_QMM_KERNEL_STREAM, DFLASH_ERR_SHAPE,
                  "dflash_qmm_m16: the streaming kernel needs group_size 64 and K %% 1024 == 0 "

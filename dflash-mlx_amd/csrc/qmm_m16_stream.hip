@@ -80,7 +80,7 @@ struct Params {
   // w, scales, biases hold E matrices of [N, .] back to back
   const int32_t* expert_ids;
   int P, E;
-  // dense form, K % 1024 == 0: w, scales, biases hold the images qmm_pack_kernel writes - per
+  // dense forms, K % 1024 == 0: w, scales, biases hold the images qmm_pack_kernel writes - per
   // (row block, unit) the 16 KiB of codes in the order of the LDS slot, per (row block, chunk)
   // 4 KiB of scales and of biases - so that every load instruction of a wave moves 1 KiB of
   // consecutive memory
@@ -152,7 +152,12 @@ __device__ unsigned long long g_sstamps[64][256][16];
 // GATHER: per-expert form.  Rows of x that share an expert are taken 16 at a time as one
 // "entry"; an entry is a matrix problem of its own, [rows, K] x [N, K]^T, and the unit
 // space is that of all entries back to back: virtual row block = entry * RB + row block.
-template <bool ACT_FP16, bool SB_FP16, int GS, int SBROW, bool ANYK, bool GATHER>
+// SILU_MUL (dense form, weights in row order): W holds the gate rows of an MLP and, behind them, its up rows, and
+// y[M, N / 2] is silu(gate) * up.  The rows of a tile of 16 are 8 gate rows and the up rows of the same columns, so that
+// lane col + 8 of a finished tile holds what lane col multiplies with: nothing else changes, and the activation
+// costs no pass of its own.  4096 x 24576 in one launch 19.5 us, where two products and three array operators took 32
+// (groups of 64, one token), 21.8 us for 32 (groups of 32, 16 tokens: a joint product and three operators).
+template <bool ACT_FP16, bool SB_FP16, int GS, int SBROW, bool ANYK, bool GATHER, bool SILU_MUL>
 __global__ __launch_bounds__(kThreads, 1) void qmm_stream_kernel(Params p) {
   using A = Act<ACT_FP16>;
   constexpr int CHUNK = SBROW * GS / 512;
@@ -180,6 +185,18 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_stream_kernel(Params p) {
   const bool packed = !GATHER && !ANYK && SBROW == 32 && p.packed;
   const uint32_t w_unit_stride = packed ? kPackedUnitBytes : kUnitK / 2;
   const uint32_t sb_chunk_stride = packed ? kPackedChunkBytes : SBROW;
+  // row of the matrix behind row v (0 .. 127) of row block rb; rows past the last one repeat it
+  auto matrix_row = [&](int rb, int v) __attribute__((always_inline)) -> int {
+    const int rows = SILU_MUL ? p.N >> 1 : p.N;
+    const int row = SILU_MUL ? rb * (kRows / 2) + (v >> 4) * 8 + (v & 7) : rb * kRows + v;
+    return (row < rows ? row : rows - 1) + (SILU_MUL && (v & 8) ? rows : 0);
+  };
+  // Packed gate/up images (qmm_pack_gate_up_kernel) hold a row block's 64 gate rows first: the instruction of them that
+  // moves rows 8 q .. 8 q + 7 of the row block, and the place of row v's 32 bytes of a chunk
+  auto image_piece = [&](int q) __attribute__((always_inline)) -> int { return SILU_MUL ? (q >> 1) + 8 * (q & 1) : q; };
+  auto image_sb = [&](int v) __attribute__((always_inline)) -> int {
+    return (SILU_MUL ? (v >> 4) * 8 + (v & 7) + 8 * (v & 8) : v) * 32 + (lane & 1) * 16;
+  };
   // where chunk c of a row of scales is loaded from, and how much later than there it begins
   const int sb_last = p.K / GS * 2 - SBROW;
   auto chunk_at = [&](int c) __attribute__((always_inline)) -> int {
@@ -317,31 +334,27 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_stream_kernel(Params p) {
     const char* sbp[2];  // scales / biases of this lane's row, chunk 0 (CHUNK = 2: [0] only)
     auto set_row_block = [&](int vrb) __attribute__((always_inline)) {
       const Where wh = locate(vrb);
-      const int row0 = wh.rb * kRows;
       const uint32_t* wmat = p.w + (size_t)wh.expert * p.N * (row_bytes >> 2);
       const uint16_t* smat = p.scales + (size_t)wh.expert * p.N * G;
       const uint16_t* bmat = p.biases + (size_t)wh.expert * p.N * G;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        int row = row0 + 8 * (ld + 4 * i) + w_r;
-        row = row < p.N ? row : p.N - 1;
+        const int row = matrix_row(wh.rb, 8 * (ld + 4 * i) + w_r);
         wp[i] = (const char*)wmat + (size_t)row * row_bytes + w_c * 16;
       }
       if (packed) {
         const char* img = (const char*)p.w + (size_t)wh.rb * p.stages * kPackedUnitBytes + lane * 16;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) wp[i] = img + (ld + 4 * i) * 1024;
-        const size_t sb_img = (size_t)wh.rb * (p.stages / 4) * kPackedChunkBytes + ld * 1024 + lane * 16;
+        for (int i = 0; i < 4; ++i) wp[i] = img + image_piece(ld + 4 * i) * 1024;
+        const size_t sb_img = (size_t)wh.rb * (p.stages / 4) * kPackedChunkBytes + image_sb(32 * ld + (lane >> 1));
         sbp[0] = (const char*)p.scales + sb_img;
         sbp[1] = (const char*)p.biases + sb_img;
       } else if (SBROW == 32) {
-        int row = row0 + 32 * ld + (lane >> 1);
-        row = row < p.N ? row : p.N - 1;
+        const int row = matrix_row(wh.rb, 32 * ld + (lane >> 1));
         sbp[0] = (const char*)(smat + (size_t)row * G) + (lane & 1) * 16;
         sbp[1] = (const char*)(bmat + (size_t)row * G) + (lane & 1) * 16;
       } else {
-        int row = row0 + 64 * (ld & 1) + lane;
-        row = row < p.N ? row : p.N - 1;
+        const int row = matrix_row(wh.rb, 64 * (ld & 1) + lane);
         sbp[0] = (const char*)(((ld & 2) ? bmat : smat) + (size_t)row * G);
         sbp[1] = sbp[0];
       }
@@ -451,13 +464,12 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_stream_kernel(Params p) {
     if (SBROW == 32 || wave < 4) {
       const int part = SBROW == 32 ? wave & 3 : wave & 1;
       const bool is_scale = SBROW == 32 ? wave < 4 : wave < 2;
-      int row = wh.rb * kRows + (SBROW == 32 ? 32 * part + (lane >> 1) : 64 * part + lane);
-      row = row < p.N ? row : p.N - 1;
+      const int row = matrix_row(wh.rb, SBROW == 32 ? 32 * part + (lane >> 1) : 64 * part + lane);
       const uint16_t* mat = (is_scale ? p.scales : p.biases) + (size_t)wh.expert * p.N * G;
       const char* src = (const char*)(mat + (size_t)row * G) + (SBROW == 32 ? (lane & 1) * 16 : 0) + chunk_at(st0 / CHUNK);
       if (packed)
         src = (const char*)(is_scale ? p.scales : p.biases) +
-              ((size_t)wh.rb * (p.stages / 4) + st0 / CHUNK) * kPackedChunkBytes + part * 1024 + lane * 16;
+              ((size_t)wh.rb * (p.stages / 4) + st0 / CHUNK) * kPackedChunkBytes + image_sb(32 * part + (lane >> 1));
       load16_to_lds(src, lds + kSbOffset + (is_scale ? 0 : kSbArrayBytes) + part * 1024);
     }
     // x: instruction `wave` of the loaders' scheme; codes: instructions 2 wave and 2 wave + 1
@@ -474,12 +486,11 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_stream_kernel(Params p) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int q = 2 * wave + i;
-      int wrow = wh.rb * kRows + 8 * q + w_r;
-      wrow = wrow < p.N ? wrow : p.N - 1;
+      const int wrow = matrix_row(wh.rb, 8 * q + w_r);
       const int w_at = w_c * 16 + st0 * (kUnitK / 2);
       const char* wsrc = (const char*)wmat + (size_t)wrow * row_bytes + (!ANYK || w_at < (int)row_bytes ? w_at : 0);
       if (packed)
-        wsrc = (const char*)p.w + ((size_t)wh.rb * p.stages + st0) * kPackedUnitBytes + q * 1024 + lane * 16;
+        wsrc = (const char*)p.w + ((size_t)wh.rb * p.stages + st0) * kPackedUnitBytes + image_piece(q) * 1024 + lane * 16;
       load16_to_lds_stream(wsrc, lds + q * 1024);
     }
   }
@@ -540,6 +551,17 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_stream_kernel(Params p) {
   // of the row block; in the gathered form m is a position in the entry's row table.
   auto emit = [&](int vrb, const f32x4_t& acc) __attribute__((always_inline)) {
     const Where wh = locate(vrb);
+    if (SILU_MUL) {
+      const int cols = p.N >> 1, n_out = wh.rb * (kRows / 2) + 8 * wave + col;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        // lane col of 16 reads lane col ^ 8 (DPP row_ror:8)
+        const float up = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(acc[r]), 0x128, 0xF, 0xF, false));
+        const float h = silu_mul<ACT_FP16>(acc[r], up);
+        if (col < 8 && n_out < cols && 4 * kblk + r < p.M) p.y[(size_t)(4 * kblk + r) * cols + n_out] = (uint16_t)A::from_f32(h);
+      }
+      return;
+    }
     const int n_out = wh.rb * kRows + 16 * wave + col;
     if (n_out >= p.N) return;
     if (GATHER) {
@@ -804,39 +826,43 @@ size_t qmm_stream_workspace_bytes(int N, int grid) {
 namespace {
 // Variants: group 64 with K a multiple of 1024 (0) and of 512 (1), any K with groups of 64 (2), 32 (3), 128 (4).
 constexpr int kVariants = 5;
-template <bool A16, bool S16>
-const void* stream_kernel_for(int variant, bool gather) {
+enum class Form { kDense, kGather, kSiluMul };
+template <bool A16, bool S16, bool SILU_MUL>
+const void* dense_kernel_for(int variant) {
   using namespace stream;
   switch (variant) {
-    case 0:
-      return gather ? (const void*)qmm_stream_kernel<A16, S16, 64, 32, false, true>
-                    : (const void*)qmm_stream_kernel<A16, S16, 64, 32, false, false>;
-    case 1:
-      return gather ? (const void*)qmm_stream_kernel<A16, S16, 64, 16, false, true>
-                    : (const void*)qmm_stream_kernel<A16, S16, 64, 16, false, false>;
-    case 2:
-      return gather ? (const void*)qmm_stream_kernel<A16, S16, 64, 16, true, true>
-                    : (const void*)qmm_stream_kernel<A16, S16, 64, 16, true, false>;
-    case 3:
-      return (const void*)qmm_stream_kernel<A16, S16, 32, 32, true, false>;
-    default:
-      return (const void*)qmm_stream_kernel<A16, S16, 128, 16, true, false>;
+    case 0: return (const void*)qmm_stream_kernel<A16, S16, 64, 32, false, false, SILU_MUL>;
+    case 1: return (const void*)qmm_stream_kernel<A16, S16, 64, 16, false, false, SILU_MUL>;
+    case 2: return (const void*)qmm_stream_kernel<A16, S16, 64, 16, true, false, SILU_MUL>;
+    case 3: return (const void*)qmm_stream_kernel<A16, S16, 32, 32, true, false, SILU_MUL>;
+    default: return (const void*)qmm_stream_kernel<A16, S16, 128, 16, true, false, SILU_MUL>;
+  }
+}
+template <bool A16, bool S16>
+const void* stream_kernel_for(int variant, Form form) {
+  using namespace stream;
+  if (form == Form::kDense) return dense_kernel_for<A16, S16, false>(variant);
+  if (form == Form::kSiluMul) return dense_kernel_for<A16, A16, true>(variant);  // (one type for both: qmm_stream_silu_mul)
+  switch (variant) {
+    case 0: return (const void*)qmm_stream_kernel<A16, S16, 64, 32, false, true, false>;
+    case 1: return (const void*)qmm_stream_kernel<A16, S16, 64, 16, false, true, false>;
+    default: return (const void*)qmm_stream_kernel<A16, S16, 64, 16, true, true, false>;
   }
 }
 
-int launch_stream(stream::Params& p, bool gather, int grid, int group_size, int act_dtype, int sb_dtype,
+int launch_stream(stream::Params& p, Form form, int grid, int group_size, int act_dtype, int sb_dtype,
                   hipStream_t stream) {
   using namespace stream;
   const bool a16 = act_dtype == DFLASH_FP16, s16 = sb_dtype == DFLASH_FP16;
   const int variant = group_size == 32 ? 3 : group_size == 128 ? 4 : p.K % (kUnitK * 4) == 0 ? 0 : p.K % (kUnitK * 2) == 0 ? 1 : 2;
   // (tests shorten the wait of the workgroups that add partial tiles to see them give up)
-  p.spin_limit = option(DFLASH_OPT_QMM_SPIN_LIMIT) > 0 ? option(DFLASH_OPT_QMM_SPIN_LIMIT) : kSpinLimit;
-  const void* fn = a16 ? (s16 ? stream_kernel_for<true, true>(variant, gather) : stream_kernel_for<true, false>(variant, gather))
-                       : (s16 ? stream_kernel_for<false, true>(variant, gather) : stream_kernel_for<false, false>(variant, gather));
-  const int lds_bytes = gather ? kLdsBytesGather : kLdsBytes;
+  if (p.spin_limit <= 0) p.spin_limit = option(DFLASH_OPT_QMM_SPIN_LIMIT) > 0 ? option(DFLASH_OPT_QMM_SPIN_LIMIT) : kSpinLimit;
+  const void* fn = a16 ? (s16 ? stream_kernel_for<true, true>(variant, form) : stream_kernel_for<true, false>(variant, form))
+                       : (s16 ? stream_kernel_for<false, true>(variant, form) : stream_kernel_for<false, false>(variant, form));
+  const int lds_bytes = form == Form::kGather ? kLdsBytesGather : kLdsBytes;
   // the attribute belongs to the device's copy of the kernel: once per device and kernel
-  static bool attr_set[kMaxDevices][kVariants * 8] = {};
-  const int idx = variant * 8 + (gather ? 4 : 0) + (a16 ? 2 : 0) + (s16 ? 1 : 0);
+  static bool attr_set[kMaxDevices][kVariants * 12] = {};
+  const int idx = variant * 12 + (int)form * 4 + (a16 ? 2 : 0) + (s16 ? 1 : 0);
   const int slot = current_device_slot();
   if (!attr_set[slot][idx] || slot == kMaxDevices - 1) {
     DFLASH_HIP_OK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes));
@@ -854,7 +880,7 @@ int launch_stream(stream::Params& p, bool gather, int grid, int group_size, int 
 
 int qmm_stream_launch(const void* x, const uint32_t* w, const void* scales, const void* biases,
                       void* y, void* workspace, size_t workspace_bytes, int M, int K, int N,
-                      int group_size, int act_dtype, int sb_dtype, hipStream_t stream) {
+                      int group_size, int act_dtype, int sb_dtype, bool silu_mul, hipStream_t stream) {
   using namespace stream;
   Params p{};
   p.M = M;
@@ -874,7 +900,36 @@ int qmm_stream_launch(const void* x, const uint32_t* w, const void* scales, cons
                  workspace ? workspace_bytes : (size_t)0);
   p.status = (uint32_t*)workspace;
   p.partials = (float*)((char*)workspace + 64 * 1024);
-  return launch_stream(p, false, grid, group_size, act_dtype, sb_dtype, stream);
+  return launch_stream(p, silu_mul ? Form::kSiluMul : Form::kDense, grid, group_size, act_dtype, sb_dtype, stream);
+}
+
+// A gate/up problem of a chained launch that stands alone: 16 rows, one type for activations and scales, K % 1024 == 0,
+// N % 128 == 0; `packed`: the images of qmm_pack_gate_up_kernel.
+int qmm_stream_gate_up_launch(const void* x, const uint32_t* w, const void* scales, const void* biases, void* y,
+                              void* workspace, size_t workspace_bytes, int K, int N, int dtype, bool packed,
+                              int spin_limit, hipStream_t stream) {
+  using namespace stream;
+  Params p{};
+  p.M = 16;
+  p.x = (const uint16_t*)x;
+  p.w = w;
+  p.scales = (const uint16_t*)scales;
+  p.biases = (const uint16_t*)biases;
+  p.y = (uint16_t*)y;
+  p.K = K;
+  p.N = N;
+  p.stages = K / kUnitK;
+  p.units = (N / kRows) * p.stages;
+  p.packed = packed ? 1 : 0;
+  p.spin_limit = spin_limit;
+  const int grid = qmm_stream_pick_grid(p.units, p.units / p.stages, qmm_stream_grid());
+  const size_t need = qmm_stream_workspace_bytes(N, grid);
+  DFLASH_REQUIRE(workspace && workspace_bytes >= need, DFLASH_ERR_WORKSPACE,
+                 "dflash_qmm_m16_chain: workspace of %zu bytes needed, %zu given", need,
+                 workspace ? workspace_bytes : (size_t)0);
+  p.status = (uint32_t*)workspace;
+  p.partials = (float*)((char*)workspace + 64 * 1024);
+  return launch_stream(p, Form::kSiluMul, grid, 64, dtype, dtype, stream);
 }
 
 bool qmm_stream_packed_eligible(int K, int N, int group_size) {
@@ -922,7 +977,7 @@ int qmm_stream_packed_launch(const void* x, const void* w_img, const void* s_img
                  workspace ? workspace_bytes : (size_t)0);
   p.status = (uint32_t*)workspace;
   p.partials = (float*)((char*)workspace + 64 * 1024);
-  return launch_stream(p, false, grid, 64, act_dtype, sb_dtype, stream);
+  return launch_stream(p, Form::kDense, grid, 64, act_dtype, sb_dtype, stream);
 }
 
 int qmm_stream_gather_launch(const void* x, const int32_t* expert_ids, const uint32_t* w,
@@ -951,7 +1006,7 @@ int qmm_stream_gather_launch(const void* x, const int32_t* expert_ids, const uin
                  workspace ? workspace_bytes : (size_t)0);
   p.status = (uint32_t*)workspace;
   p.partials = (float*)((char*)workspace + 64 * 1024);
-  return launch_stream(p, true, grid, 64, act_dtype, sb_dtype, stream);
+  return launch_stream(p, Form::kGather, grid, 64, act_dtype, sb_dtype, stream);
 }
 
 }  // namespace dflash

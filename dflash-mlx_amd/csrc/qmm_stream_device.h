@@ -289,7 +289,9 @@ __device__ __forceinline__ void consume_unit(const OperandsOf32& cur, OperandsOf
 
 // Cross-wave sum at the end of a row block: every worker hands the three tiles it does
 // not own to their owners through `base` (24 KiB: 8 owners x 3 tiles x 1 KiB), and after
-// a barrier returns the sum of its own tile and the three it receives, in a fixed order.
+// a barrier returns the sum of its own tile and the three it receives: groups g and g + 2, groups
+// g + 1 and g + 3 (mod 4), then the two sums - the same additions whichever of the four holds the tile, so
+// that a row's result does not depend on the tile it is dealt to.
 __device__ __forceinline__ void reduce_groups_write(uint32_t base, const f32x4_t (&acc)[4], int wave,
                                                     int lane) {
   const int g = wave & 3, h = wave >> 2;
@@ -318,7 +320,7 @@ __device__ __forceinline__ f32x4_t reduce_groups_read(uint32_t base, const f32x4
       : "v"(addr)
       : "memory");
 #pragma unroll
-  for (int r = 0; r < 4; ++r) own[r] = ((own[r] + v0[r]) + v1[r]) + v2[r];
+  for (int r = 0; r < 4; ++r) own[r] = (own[r] + v1[r]) + (v0[r] + v2[r]);
   return own;
 }
 
@@ -406,6 +408,20 @@ __device__ __forceinline__ u32x2_t lds_read_u64(uint32_t addr) {
   u32x2_t v;
   asm volatile("ds_read_b64 %0, %1\n s_waitcnt lgkmcnt(0)" : "=v"(v) : "v"(addr) : "memory");
   return v;
+}
+
+template <bool FP16>
+__device__ __forceinline__ float silu_mul(float g, float u) {
+  using A = Act<FP16>;
+  // silu(g) * u as the array operators x * sigmoid(x) and * give it: the factors as the
+  // activation type holds them between the projections and the activation, then the sigmoid,
+  // its product with g and the product with u each rounded to that type (the last one by the
+  // store).  Same form as the GatedDeltaNet glue kernels use.
+  g = A::to_f32(A::from_f32(g));
+  u = A::to_f32(A::from_f32(u));
+  const float sig = A::to_f32(A::from_f32(1.0f / (1.0f + expf(-g))));
+  const float s = A::to_f32(A::from_f32(g * sig));
+  return s * u;
 }
 
 }  // namespace stream

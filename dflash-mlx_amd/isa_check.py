@@ -29,7 +29,7 @@ CSRC = os.path.join(HERE, "csrc")
 
 # source, mangled-name prefix of its kernel, instantiations, LDS reads each must at least hold
 KERNELS = (
-    ("qmm_m16_stream.hip", "_ZN6dflash6stream17qmm_stream_kernel", 32, 40),  # activation x scale dtype x group size, chunk, any K x dense|gathered
+    ("qmm_m16_stream.hip", "_ZN6dflash6stream17qmm_stream_kernel", 42, 40),  # activation x scale dtype x group size, chunk, any K x dense|gathered, silu-mul
     ("qmm_m16_chain.hip", "_ZN6dflash6stream16qmm_chain_kernel", 8, 40),     # activation x scale dtype x weight layout
 )
 # source, number of counter bumps (arrival counters; the chained kernel's per-problem and exit counters too)

@@ -26,8 +26,8 @@ import torch
 import torch.nn as nn
 
 from .quantized import QuantizedLinear, stock_matmul
-from .verify_qmm import (ChainProblem, QmmChain, _should_use_verify, pack_weights, packable, rows_matmul, verify_matmul,
-                         verify_matmul_packed)
+from .verify_qmm import (ChainProblem, QmmChain, _should_use_verify, is_enabled, pack_weights, packable, rows_matmul,
+                         small_m_matmul, small_m_silu_mul, verify_matmul, verify_matmul_packed)
 
 _VERIFY_MAX_N_DEFAULT = 100_000
 
@@ -139,13 +139,21 @@ class FusedProjections:
         return (x.is_cuda and x.ndim >= 2 and x.numel() > 16 * int(x.shape[-1]) and self.bits == 4
                 and os.environ.get("DFLASH_STOCK_KERNEL", "1") != "0" and self._holds(parent, x))
 
-    def _holds(self, parent: nn.Module, x: torch.Tensor) -> bool:
+    def serves_few(self, parent: nn.Module, x: torch.Tensor) -> bool:
+        """The same for fewer rows than a block has (a token, a last short block), which members take through
+        ``small_m_matmul`` one by one.  With the verify switch on, that includes members behind a wrapper that pads to 16 rows
+        so that a token meets the kernel a block meets: the joint product is that kernel, and a row of
+        it does not depend on the rows beside it."""
+        return (x.is_cuda and x.ndim >= 2 and 0 < x.numel() < 16 * int(x.shape[-1]) and self.bits == 4
+                and os.environ.get("DFLASH_STOCK_KERNEL", "1") != "0" and self._holds(parent, x, padded=is_enabled()))
+
+    def _holds(self, parent: nn.Module, x: torch.Tensor, padded: bool = False) -> bool:
         if x.device != self.weight.device:
             return False
         for index, name in enumerate(self.names):
             mod = getattr(parent, name, None)
             if getattr(mod, "_dflash_exact_small_proj_wrapped", False):
-                if x.ndim == 3 and x.shape[1] < mod.pad_m:
+                if x.ndim == 3 and x.shape[1] < mod.pad_m and not padded:
                     return False
                 mod = mod.linear
             if getattr(mod, "_shared_input", None) != (self, index):
@@ -185,6 +193,16 @@ class FusedProjections:
             return None
         return rows_matmul(x, self.weight, self.scales, self.biases, group_size=self.group_size, bits=self.bits, epilogue=epilogue)
 
+    def few(self, x: torch.Tensor) -> Optional[torch.Tensor]:
+        """The joint product of fewer rows than a block has, or None where its kernel does not apply."""
+        return small_m_matmul(x, self.weight, self.scales, self.biases, group_size=self.group_size, bits=self.bits)
+
+    def few_silu_mul(self, x: torch.Tensor) -> Optional[torch.Tensor]:
+        """The gated activation of up to 16 rows, or None where its kernel does not apply."""
+        if not (len(self.bounds) == 2 and self.bounds[1] == (self.bounds[0][1], 2 * self.bounds[0][1])):
+            return None
+        return small_m_silu_mul(x, self.weight, self.scales, self.biases, group_size=self.group_size, bits=self.bits)
+
     def __call__(self, x: torch.Tensor) -> Tuple[torch.Tensor, ...]:
         if self._packed is not None and x.is_cuda:
             product = verify_matmul_packed(x, self._packed)
@@ -203,7 +221,8 @@ def silu_gate_up(parent: nn.Module, x: torch.Tensor, names: Tuple[str, str] = ("
     activation and the product applied before anything is stored (``dflash_qmm_m16_chain`` with
     its silu-mul epilogue; every operator's rounding to the activation dtype is kept, the split
     of K between workgroups differs from the separate projections', so single results may
-    differ by one rounding of the array dtype).  Prompts (more than 16 rows) take one launch of the
+    differ by one rounding of the array dtype).  Other group sizes and widths, and blocks of fewer than 16
+    rows, take the streaming kernel with the activation in its last step (``dflash_qmm_few_silu_mul``).  Prompts (more than 16 rows) take one launch of the
     any-rows product with the same epilogue.  Everything else goes through
     ``shared_input_outputs`` and the array operators.  No counterpart in the reference, whose MLP
     is mlx-lm's ``down_proj(swiglu(gate_proj(x), up_proj(x)))``; 27B shape: gate/up/activation
@@ -211,10 +230,13 @@ def silu_gate_up(parent: nn.Module, x: torch.Tensor, names: Tuple[str, str] = ("
     for group in getattr(parent, "_dflash_fused", ()):
         if group.names == tuple(names) and group.applies(parent, x) and group.silu_mul_ready(x):
             return group.silu_mul(x)
+        hidden = None
         if group.names == tuple(names) and group.serves_prompt(parent, x):
             hidden = group.prompt(x, "silu_mul")
-            if hidden is not None:
-                return hidden
+        elif group.names == tuple(names) and (group.serves_few(parent, x) or group.applies(parent, x)):
+            hidden = group.few_silu_mul(x)
+        if hidden is not None:
+            return hidden
     gate, up = shared_input_outputs(parent, names, x)
     return (gate * torch.sigmoid(gate)) * up   # x * sigmoid(x): the operators the epilogue follows, one rounding each
 
@@ -228,6 +250,10 @@ def shared_input_outputs(parent: nn.Module, names: Sequence[str], x: torch.Tenso
             outs.update(zip(group.names, group(x)))
         elif all(n in names for n in group.names) and group.serves_prompt(parent, x):
             product = group.prompt(x)
+            if product is not None:
+                outs.update((n, product[..., lo:hi]) for n, (lo, hi) in zip(group.names, group.bounds))
+        elif all(n in names for n in group.names) and group.serves_few(parent, x):
+            product = group.few(x)
             if product is not None:
                 outs.update((n, product[..., lo:hi]) for n, (lo, hi) in zip(group.names, group.bounds))
     return tuple(outs[n] if n in outs else getattr(parent, n)(x) for n in names)

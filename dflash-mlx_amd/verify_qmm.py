@@ -489,6 +489,41 @@ def small_m_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biase
     return y.reshape(*x.shape[:-1], N)
 
 
+def small_m_silu_mul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
+                     *, group_size: int = 64, bits: int = 4) -> "torch.Tensor | None":
+    """``silu(x @ gate.T) * (x @ up.T)`` for at most 16 rows of device activations in one launch of the streaming
+    kernel; ``w`` holds the gate rows of an MLP followed by its up rows.  None for what that kernel does not
+    cover.  No counterpart in the reference."""
+    if (not x.is_cuda or bits != 4 or x.dtype not in _DTYPE_CODE or not (scales.dtype == biases.dtype == x.dtype)
+            or w.ndim != 2 or not _native.is_built() or _kernel_select() != _native.QMM_KERNEL_AUTO):
+        return None
+    K, N = int(x.shape[-1]), int(w.shape[0])
+    m = x.numel() // K if K else 0
+    if m < 1 or m > 16 or N % 16 != 0 or int(w.shape[1]) * 8 != K:
+        return None
+    lib = _native.lib()
+    key = (K, N, group_size, -1, 1, _native.QMM_KERNEL_STREAM)  # (-1: with the activation)
+    need = _WORKSPACE_BYTES.get(key)
+    if need is None:
+        need = _WORKSPACE_BYTES[key] = int(lib.dflash_qmm_few_silu_mul_workspace_bytes(K, N, group_size))
+    if need == 0:
+        return None
+    w, scales, biases = w.contiguous(), scales.contiguous(), biases.contiguous()
+    if w.data_ptr() % 16 or (scales.data_ptr() | biases.data_ptr()) % 4:
+        return None
+    _require_operands("silu_gate_up", K, N, group_size, w, scales, biases, x.device)
+    x2 = x.reshape(m, K).contiguous()
+    if x2.data_ptr() % 16:
+        return None
+    y = torch.empty((m, N // 2), dtype=x.dtype, device=x.device)
+    stream = _native.raw_stream(x.device)
+    ws = _workspace(x.device, stream, need)
+    rc = lib.dflash_qmm_few_silu_mul(x2.data_ptr(), w.data_ptr(), scales.data_ptr(), biases.data_ptr(), y.data_ptr(), ws.data_ptr(),
+                                     ws.numel(), m, K, N, group_size, _DTYPE_CODE[x.dtype], stream)
+    _native.check(rc, "dflash_qmm_few_silu_mul")
+    return y.reshape(*x.shape[:-1], N // 2)
+
+
 # Scratch of the any-rows product, one per (device, stream): 64 KiB of counters, then partial tiles.
 _ROWS_WORKSPACES: Dict[Tuple[int, int], torch.Tensor] = {}
 

@@ -129,6 +129,17 @@ int dflash_qmm_few(const void* x, const uint32_t* w_q, const void* scales, const
                    int sb_dtype, int kernel, void* stream);
 
 /*
+ * The hidden activation of a gated MLP for M = 1 .. 16 rows: w_q holds N / 2 gate rows and, behind them, as many up rows,
+ * y [M, N / 2] = silu(x . gate^T) * (x . up^T) with every operator's rounding to `dtype` (activations and scales).
+ * Shapes of the streaming kernel: group_size 32, 64 or 128, K a multiple of 64 and of the group size, N of 16,
+ * scales and biases 4-byte aligned.  The size is 0 for what it does not cover.
+ */
+size_t dflash_qmm_few_silu_mul_workspace_bytes(int K, int N, int group_size);
+int dflash_qmm_few_silu_mul(const void* x, const uint32_t* w_q, const void* scales, const void* biases, void* y,
+                            void* workspace, size_t workspace_bytes, int M, int K, int N, int group_size, int dtype,
+                            void* stream);
+
+/*
  * dflash_qmm_m16 for callers that cannot allocate device memory: code under HIP graph
  * capture, serving loops and harnesses that forbid hipMalloc.  No counterpart in the
  * reference (MLX allocates behind every array).  The workspace is an array inside the

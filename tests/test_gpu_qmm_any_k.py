@@ -58,3 +58,73 @@ def test_gathered_experts_of_any_k(native_lib, K, N, E, P):
             _check(y[rows], x[rows], dequantize(w[e], s[e], b[e], 64, 4, dtype=torch.float64), K, torch.bfloat16)
     assert bool((y[(ids < 0) | (ids >= E)] == 0).all())
     assert torch.equal(y, VQ.gather_qmm(x, w, s, b, ids))
+
+
+@pytest.mark.parametrize("K,N,group,dtype", [
+    (512, 32, 64, torch.bfloat16), (512, 16, 32, torch.bfloat16), (576, 48, 32, torch.float16), (896, 272, 64, torch.bfloat16),
+    (1024, 1040, 64, torch.bfloat16), (1280, 112, 128, torch.float16), (1536, 4128, 64, torch.float16),
+    (4096, 24576, 32, torch.bfloat16), (5120, 34816, 64, torch.bfloat16)])
+def test_gated_activation_of_few_rows(native_lib, monkeypatch, K, N, group, dtype):
+    """The silu-mul form (8 gate rows and their 8 up rows to a tile) against the joint product of the same matrix and the array
+    operators, and both against float64."""
+    monkeypatch.setenv("DFLASH_VERIFY_QMM", "1")
+    monkeypatch.delenv("DFLASH_QMM_KERNEL", raising=False)
+    c = make_qmm_case(K, N, 700 + K, group_size=group, dtype=dtype).to(DEV)
+    x = (c.x / (K ** 0.5 * c.scales.float().abs().mean() * 4)).to(dtype)  # gates of a few units
+    assert VQ.small_m_silu_mul(x[:, :K - 64], c.w, c.scales, c.biases, group_size=group) is None
+    y = VQ.small_m_silu_mul(x, c.w, c.scales, c.biases, group_size=group)
+    assert y.shape == (16, N // 2)
+    for rows in (1, 2, 9, 15):  # the same bits whatever shares the block with a row
+        assert torch.equal(VQ.small_m_silu_mul(x[:rows], c.w, c.scales, c.biases, group_size=group), y[:rows])
+    joint = VQ.small_m_matmul(x, c.w, c.scales, c.biases, group_size=group)
+    gate, up = joint[:, :N // 2], joint[:, N // 2:]
+    ref = (gate * torch.sigmoid(gate)) * up
+    # K is cut between workgroups in other places: gate and up may fall on the next value of the type (eps of
+    # themselves) and, where they cancel, move by the error of two fp32 sums over offset codes (``_check``); the slope of
+    # silu is below 1.1, and three more roundings follow on either side
+    eps = torch.finfo(dtype).eps
+    dense = dequantize(c.w, c.scales, c.biases, group, 4, dtype=torch.float64)
+    sums = (x.double().abs() @ dense.abs().t().contiguous()) * (16.0 if dtype == torch.bfloat16 else 128.0) * 2.0 ** -24 * 4 * 2
+    g, u = gate.double(), up.double()
+    s = g * torch.sigmoid(g)
+    dg, du = eps * g.abs() + sums[:, :N // 2], eps * u.abs() + sums[:, N // 2:]
+    assert ((y.double() - ref.double()).abs() <= 1.1 * dg * (u.abs() + du) + s.abs() * du + 3 * eps * (s * u).abs() + 1e-6).all()
+    product = x.double() @ dense.t().contiguous()
+    exact = product[:, :N // 2] * torch.sigmoid(product[:, :N // 2]) * product[:, N // 2:]
+    assert (y.double() - exact).norm() <= 1.05 * (ref.double() - exact).norm()
+    torch.cuda.synchronize()
+    VQ.raise_on_device_errors(torch.device(DEV))
+    ws = VQ._workspace(torch.device(DEV), torch.cuda.current_stream().cuda_stream, 1)
+    assert int((ws != 0).sum()) == 0
+
+
+def test_few_rows_take_the_joint_launch(native_lib, monkeypatch):
+    """One token and a short block through joined projections: the rows a block of 16 gets, also for members
+    behind a wrapper that pads, and the members' own launches with DFLASH_STOCK_KERNEL=0 or once a member has left."""
+    from dflash_mlx_amd import verify_linear as VL
+    from dflash_mlx_amd.gdn_layer import _ExactSmallProjPad
+    from dflash_mlx_amd.quantized import QuantizedLinear
+
+    monkeypatch.setenv("DFLASH_VERIFY_QMM", "1")
+    monkeypatch.delenv("DFLASH_QMM_KERNEL", raising=False)
+    parent = torch.nn.Module()
+    widths = dict(in_proj_qkv=256, in_proj_z=128, in_proj_b=48, in_proj_a=48)
+    for i, (name, n) in enumerate(widths.items()):
+        c = make_qmm_case(1024, n, 900 + i).to(DEV)
+        setattr(parent, name, QuantizedLinear(c.w, c.scales, c.biases, group_size=64, bits=4))
+    parent.in_proj_b, parent.in_proj_a = _ExactSmallProjPad(parent.in_proj_b), _ExactSmallProjPad(parent.in_proj_a)
+    VL.install_verify_linears(parent)
+    assert VL.fuse_shared_input_linears(parent) == 1
+    x = make_qmm_case(1024, 32, 950).to(DEV).x.reshape(1, 16, 1024)
+    whole = VL.shared_input_outputs(parent, tuple(widths), x)
+    group = parent._dflash_fused[0]
+    for rows in (1, 5, 15):
+        assert group.serves_few(parent, x[:, :rows])
+        for got, want in zip(VL.shared_input_outputs(parent, tuple(widths), x[:, :rows]), whole):
+            assert torch.equal(got, want[:, :rows])
+    monkeypatch.setenv("DFLASH_STOCK_KERNEL", "0")
+    assert not group.serves_few(parent, x[:, :1])
+    monkeypatch.delenv("DFLASH_STOCK_KERNEL")
+    parent.in_proj_z.to(torch.device(DEV), torch.bfloat16)
+    parent.in_proj_z._apply(lambda t: t.clone())
+    assert not group.serves_few(parent, x[:, :1])
