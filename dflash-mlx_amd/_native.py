@@ -62,6 +62,7 @@ EXPORTED_SYMBOLS = (
     "dflash_gdn_forward_workspace_bytes",
     "dflash_gdn_forward",
     "dflash_gdn_prepare",
+    "dflash_gdn_prepare_rows",
     "dflash_gdn_gated_norm",
     "dflash_attn_prepare",
     "dflash_attn_gate",
@@ -134,9 +135,12 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.dflash_gdn_forward_workspace_bytes.restype = c.c_size_t
     lib.dflash_gdn_forward_workspace_bytes.argtypes = [c.c_int] * 8
     lib.dflash_gdn_forward.restype = c.c_int
-    lib.dflash_gdn_forward.argtypes = [c.c_void_p] * 13 + [c.c_size_t] + [c.c_int] * 12 + [c.c_float, c.c_void_p]
+    lib.dflash_gdn_forward.argtypes = [c.c_void_p] * 13 + [c.c_size_t] + [c.c_longlong] * 2 + [c.c_int] * 12 + [c.c_float, c.c_void_p]
     lib.dflash_gdn_prepare.restype = c.c_int
     lib.dflash_gdn_prepare.argtypes = [c.c_void_p] * 14 + [c.c_int] * 9 + [c.c_float, c.c_void_p]
+    lib.dflash_gdn_prepare_rows.restype = c.c_int
+    lib.dflash_gdn_prepare_rows.argtypes = ([c.c_void_p] * 15 + [c.POINTER(c.c_longlong)] + [c.c_int] * 9 +
+                                            [c.c_float, c.c_void_p])
     lib.dflash_gdn_gated_norm.restype = c.c_int
     lib.dflash_gdn_gated_norm.argtypes = [c.c_void_p] * 4 + [c.c_longlong] + [c.c_int] * 3 + [c.c_float, c.c_void_p]
     lib.dflash_attn_prepare.restype = c.c_int

@@ -52,8 +52,9 @@ struct GdnArgs {
   int in_dtype, g_dtype, beta_dtype, state_dtype, g_per_dk;
   int staged;  // step-by-step kernel: steps staged in LDS at a time
   // gated output norm fused behind the recurrence (block kernel only): y is then
-  // silu(z) * rms_norm(recurrence output, norm_weight), z laid out like y
-  const void* z;
+  // silu(z) * rms_norm(recurrence output, norm_weight)
+  const void* z;  // [slots, T, Hv, Dv], slots and steps with a stride (elements)
+  long long z_batch, z_row;
   const void* norm_weight;  // [Dv]
   int weight_dtype;
   float eps;
@@ -390,7 +391,7 @@ __device__ __forceinline__ void issue_item_loads(const GdnArgs& a, int item, int
     // ahead of the state, like every load whose width depends on a dtype: behind it, the branch
     // around such a load would leave the number of loads in flight unknown at the first wait
     const int tz = li < T ? li : T - 1;
-    const size_t zb = ((slotT + tz) * a.Hv + hv) * 128;
+    const size_t zb = (size_t)slot * a.z_batch + (size_t)tz * a.z_row + (size_t)hv * 128;
     const bool wwide = a.weight_dtype == DFLASH_FP32;
 #pragma unroll
     for (int t2 = 0; t2 < 2; ++t2) {
@@ -794,17 +795,23 @@ size_t gdn_prompt_workspace_bytes(int slots, int T, int Hk, int Hv, int Dk);
 int gdn_prompt_launch(const void* q, const void* k, const void* v, const void* g, const void* beta, const void* state_in,
                       void* state_out, void* y, float* tape, const uint8_t* mask, void* workspace, int slots, int T, int Hk,
                       int Hv, int Dk, int Dv, int g_dtype, int beta_dtype, int state_dtype, hipStream_t s);
+// gdn_glue.hip
+int gdn_gated_norm_launch(const void* x, const void* z, const void* weight, void* y, int B, int T, int H, int D,
+                          long long z_batch, long long z_row, int dtype, int weight_dtype, float eps, hipStream_t stream);
 
 namespace {
 
-// Shared body of the entry points; z == nullptr: no output norm.
+// Shared body of the entry points; z == nullptr: no output norm; z_row = 0: z laid out like y.
 int gdn_forward_launch(const char* who, const void* q, const void* k, const void* v, const void* g, const void* beta,
                        const void* state_in, void* state_out, void* y, float* tape, const uint8_t* mask,
                        const void* z, const void* norm_weight, int weight_dtype, float eps, int slots, int T, int Hk,
                        int Hv, int Dk, int Dv, int in_dtype, int g_dtype, int beta_dtype, int state_dtype,
-                       int g_per_dk, void* stream, void* workspace = nullptr, size_t workspace_bytes = 0) {
+                       int g_per_dk, void* stream, void* workspace = nullptr, size_t workspace_bytes = 0, long long z_batch = 0,
+                       long long z_row = 0) {
+  if (z_row == 0) z_row = (long long)Hv * Dv, z_batch = z_row * T;
+  const int z_elem = in_dtype == DFLASH_FP32 ? 4 : 2;
   const bool aligned16 = (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)y | (uintptr_t)tape |
-                           (uintptr_t)z | (uintptr_t)norm_weight) % 16) == 0;
+                           (uintptr_t)z | (uintptr_t)norm_weight | (uintptr_t)(z ? (z_batch | z_row) * z_elem : 0)) % 16) == 0;
   const bool no_chunk = option(DFLASH_OPT_GDN_STEP_BY_STEP) != 0;  // (tests of one kernel against the other)
   const bool prompt = workspace != nullptr && aligned16 && !no_chunk && gdn_prompt_covers(slots, T, Hk, Hv, Dk, Dv, in_dtype, g_per_dk) &&
                       (((uintptr_t)state_in | (uintptr_t)state_out | (uintptr_t)workspace) % 16) == 0;
@@ -819,6 +826,8 @@ int gdn_forward_launch(const char* who, const void* q, const void* k, const void
   DFLASH_REQUIRE((long long)slots * Hv < (1ll << 31), DFLASH_ERR_SHAPE, "%s: too many (slot, head) pairs", who);
   DFLASH_REQUIRE(!z || (norm_weight && Dv % 64 == 0 && Dv <= 256), DFLASH_ERR_SHAPE,
                  "%s: the output norm needs a weight and a row length that is a multiple of 64 up to 256, got %d", who, Dv);
+  DFLASH_REQUIRE(!z || (z_batch >= 0 && z_row >= 0 && (long long)slots * T * Hv < (1ll << 31)), DFLASH_ERR_SHAPE,
+                 "%s: z needs non-negative strides and fewer than 2^31 rows", who);
   if (slots == 0) return DFLASH_OK;
 
   GdnArgs a;
@@ -827,7 +836,7 @@ int gdn_forward_launch(const char* who, const void* q, const void* k, const void
   a.T = T; a.Hk = Hk; a.Hv = Hv; a.Dk = Dk; a.Dv = Dv;
   a.in_dtype = in_dtype; a.g_dtype = g_dtype; a.beta_dtype = beta_dtype; a.state_dtype = state_dtype;
   a.g_per_dk = g_per_dk ? 1 : 0;
-  a.z = z; a.norm_weight = norm_weight; a.weight_dtype = weight_dtype; a.eps = eps;
+  a.z = z; a.z_batch = z_batch; a.z_row = z_row; a.norm_weight = norm_weight; a.weight_dtype = weight_dtype; a.eps = eps;
 
   const dim3 grid((unsigned)(slots * Hv)), block(kThreads);
   hipStream_t s = (hipStream_t)stream;
@@ -872,8 +881,8 @@ int gdn_forward_launch(const char* who, const void* q, const void* k, const void
   }
   DFLASH_HIP_OK(hipGetLastError());
   if (z && !norm_done)  // the other kernels leave the recurrence's output in y: normalise it in place
-    return dflash_gdn_gated_norm(y, z, norm_weight, y, (long long)slots * T * Hv, Dv, in_dtype, weight_dtype, eps,
-                                 stream);
+    return T == 0 ? DFLASH_OK : gdn_gated_norm_launch(y, z, norm_weight, y, slots, T, Hv, Dv, z_batch, z_row, in_dtype, weight_dtype,
+                                                      eps, s);
   return DFLASH_OK;
 }
 
@@ -909,10 +918,11 @@ extern "C" size_t dflash_gdn_forward_workspace_bytes(int slots, int T, int Hk, i
 
 extern "C" int dflash_gdn_forward(const void* q, const void* k, const void* v, const void* g, const void* beta,
                                   const void* state_in, void* state_out, const void* z, const void* norm_weight, void* y,
-                                  float* tape, const uint8_t* mask, void* workspace, size_t workspace_bytes, int slots, int T,
+                                  float* tape, const uint8_t* mask, void* workspace, size_t workspace_bytes,
+                                  long long z_batch_stride, long long z_row_stride, int slots, int T,
                                   int Hk, int Hv, int Dk, int Dv, int in_dtype, int g_dtype, int beta_dtype, int state_dtype,
                                   int weight_dtype, int g_per_dk, float eps, void* stream) {
   return dflash::gdn_forward_launch("dflash_gdn_forward", q, k, v, g, beta, state_in, state_out, y, tape, mask, z, norm_weight,
                                     weight_dtype, eps, slots, T, Hk, Hv, Dk, Dv, in_dtype, g_dtype, beta_dtype, state_dtype,
-                                    g_per_dk, stream, workspace, workspace_bytes);
+                                    g_per_dk, stream, workspace, workspace_bytes, z_batch_stride, z_row_stride);
 }

@@ -8,9 +8,14 @@
 // then rms_norm(out, weight) * silu(z).  Every array-level operator of that sequence rounds
 // to the array dtype once; the arithmetic inside an operator is fp32.
 //
-// These operators are a few hundred KB of data per layer: the point of fusing them is the
-// launch count (two launches instead of about twenty elementwise kernels per layer and
-// verify step), not bandwidth.
+// For a verify block these operators are a few hundred KB per layer, and the point of fusing them is the launch
+// count (two launches instead of about twenty elementwise kernels).  For a prompt they are bound by the vector
+// instructions per element (the sigmoid's exponential and division, the roundings): a wave takes several tokens
+// of its head in turn, so that a row of qkv is read and unpacked once and not once per tap, the taps once per wave, and
+// the gates of all its tokens are computed side by side, one token per lane.  1024 tokens of 16 + 16 + 32 heads of
+// 128: 62 us with a wave per token and head, 28.6 us; the gated norm 15 -> 13.6 us.  The projections are read where a joint product
+// left them (rows with a stride), which saves four copies per layer call (25 us of the same prompt, 12 us of a
+// verify block).
 #include "glue_device.h"
 
 #include <cmath>
@@ -22,11 +27,11 @@ constexpr int kWavesPerGroup = 4;
 constexpr int kMaxPerLane = 4;  // head dims up to 256
 
 struct PrepareArgs {
-  const void* qkv;         // [B, S, C]
+  const void* qkv;         // [B, S, C], rows and batches with a stride
   const void* conv_state;  // [B, K-1, C] or null (zeros)
   const void* conv_w;      // [C, K]
-  const void* a;           // [B, S, Hv]
-  const void* b;           // [B, S, Hv]
+  const void* a;           // [B, S, Hv], likewise
+  const void* b;           // [B, S, Hv], likewise
   const void* A_log;       // [Hv]
   const void* dt_bias;     // [Hv]
   const uint8_t* mask;     // [B, S] or null
@@ -36,179 +41,214 @@ struct PrepareArgs {
   void* v;                 // [B, S, Hv, Dv]
   float* g;                // [B, S, Hv]
   void* beta;              // [B, S, Hv]
-  int B, S, Hk, Hv, Dk, Dv, K, dt, param_dt;
+  void* qkv_out;           // [B, S, C]: qkv with masked rows zeroed, or null
+  long long qkv_batch, qkv_row, a_batch, a_row, b_batch, b_row;  // strides, elements
+  int tokens;              // per wave
+  int B, S, Hk, Hv, Dk, Dv, param_dt;
   float eps, scale_q, scale_k;  // scales already rounded to the array dtype
 };
 
-// One wave per (batch, step, head); heads 0..Hk-1 are q, Hk..2Hk-1 are k, the rest v.  A lane
+// One wave per (batch, run of tokens, head); heads 0..Hk-1 are q, Hk..2Hk-1 are k, the rest v.  A lane
 // holds PER = D / 64 adjacent channels of its head, so a row of the head is one access per lane
-// and the K taps of those channels are PER * K adjacent weights.  All loads of a wave are issued
-// before anything is computed: the kernel moves a few hundred KB and lives on latency.
-template <int PER, int K>
-__device__ __forceinline__ void prepare_head(const PrepareArgs& p, int b, int s, int h, int lane) {
+// and the K taps of those channels are PER * K adjacent weights.  All loads the first token needs are issued
+// before anything is computed, the next token's row while the present one is worked on.
+template <int DT, int PER, int K>
+__device__ __forceinline__ void prepare_head(const PrepareArgs& p, int b, int s0, int s1, int h, int lane) {
   const int key_dim = p.Hk * p.Dk;
   const int C = 2 * key_dim + p.Hv * p.Dv;
   constexpr int keep = K - 1;
+  constexpr bool wide = DT == DFLASH_FP32;
   const bool is_v = h >= 2 * p.Hk;
   const int D = PER * 64;
   const int cb = is_v ? 2 * key_dim + (h - 2 * p.Hk) * p.Dv : h * p.Dk;  // q and k heads are contiguous
   const int c = cb + PER * lane;
-
-  const bool wide = p.dt == DFLASH_FP32, pwide = p.param_dt == DFLASH_FP32;
+  const int hv = is_v ? h - 2 * p.Hk : 0;
+  const bool pwide = p.param_dt == DFLASH_FP32;
+  const size_t qkv0 = (size_t)b * p.qkv_batch + c, token0 = (size_t)b * p.S;
+  // the mask byte of a row of qkv; without a mask some byte that is not looked at
+  auto mask_at = [&](int s) __attribute__((always_inline)) -> uint32_t {
+    return *(p.mask != nullptr ? p.mask + token0 + s : (const uint8_t*)p.qkv);
+  };
   // Every load below is unconditional: which row of which array a tap comes from, and whether it
   // counts at all, is decided by selecting the address (a tap that does not count reads some
   // readable row and is zeroed afterwards).  Loads inside branches, with the registers they
   // write preset to zero, make the compiler wait for earlier loads that used the same registers.
   uint32_t xr[K][PER], wr[PER * K], mask_byte[K];
-  bool counts[K];
 #pragma unroll
   for (int j = 0; j < K; ++j) {
-    const int r = s + j;  // row of [conv_state | qkv]
-    const bool from_state = r < keep;
-    counts[j] = !from_state || p.conv_state != nullptr;
-    const void* base = (from_state && p.conv_state != nullptr) ? p.conv_state : p.qkv;
-    const size_t row = !counts[j] ? (size_t)b * p.S
-                                  : from_state ? (size_t)b * keep + r : (size_t)b * p.S + (r - keep);
-    load_adjacent_raw<PER>(base, row * C + c, wide, xr[j]);
-    // the mask byte of a qkv row; without a mask (or for a state row) some byte that is not looked at
-    const uint8_t* mp = (p.mask != nullptr && !from_state) ? p.mask + (size_t)b * p.S + (r - keep)
-                                                           : (const uint8_t*)p.qkv;
-    mask_byte[j] = *mp;
+    const int r = s0 + j;  // row of [conv_state | qkv]
+    const bool from_state = r < keep, stored = from_state && p.conv_state != nullptr;
+    const int s = from_state ? 0 : r - keep;
+    load_adjacent_raw<PER>(stored ? p.conv_state : p.qkv,
+                           stored ? ((size_t)b * keep + r) * C + c : qkv0 + (size_t)s * p.qkv_row, wide, xr[j]);
+    mask_byte[j] = mask_at(s);
   }
   load_adjacent_raw<PER * K>(p.conv_w, (size_t)c * K, wide, wr);
-  const int hv = h - 2 * p.Hk;
-  const size_t vrow = ((size_t)b * p.S + s) * p.Hv + (is_v ? hv : 0);
-  // gates of the value head (key heads read head 0's and do not use them)
-  const uint32_t a_bits = load_bits(p.a, vrow, wide);
-  const uint32_t b_bits = load_bits(p.b, vrow, wide);
-  const uint32_t a_log_bits = load_bits(p.A_log, is_v ? hv : 0, pwide);
-  const uint32_t bias_bits = load_bits(p.dt_bias, is_v ? hv : 0, pwide);
+  // gates of the value head's tokens, one per lane (key heads read some and do not use them)
+  const int gate_token = s0 + lane < s1 ? s0 + lane : s1 - 1;
+  const uint32_t a_bits = load_bits(p.a, (size_t)b * p.a_batch + (size_t)gate_token * p.a_row + hv, wide);
+  const uint32_t b_bits = load_bits(p.b, (size_t)b * p.b_batch + (size_t)gate_token * p.b_row + hv, wide);
+  const uint32_t a_log_bits = load_bits(p.A_log, hv, pwide);
+  const uint32_t bias_bits = load_bits(p.dt_bias, hv, pwide);
   asm volatile("" ::: "memory");  // every request above is out before the first value is interpreted
   float x[K][PER], w[PER * K];
 #pragma unroll
-  for (int j = 0; j < K; ++j) {
-    unpack_adjacent<PER>(xr[j], p.dt, x[j]);
-    {
-      const bool from_state = s + j < keep;
-      const bool on = counts[j] && (p.mask == nullptr || from_state || mask_byte[j] != 0);
+  for (int j = 0; j < keep; ++j) {
+    unpack_adjacent<PER>(xr[j], DT, x[j]);
+    const bool from_state = s0 + j < keep;
+    const bool on = from_state ? p.conv_state != nullptr : p.mask == nullptr || mask_byte[j] != 0;
 #pragma unroll
-      for (int e = 0; e < PER; ++e) x[j][e] = on ? x[j][e] : 0.f;
-    }
+    for (int e = 0; e < PER; ++e) x[j][e] = on ? x[j][e] : 0.f;
   }
-  unpack_adjacent<PER * K>(wr, p.dt, w);
-  const float gate_a = bits_as_f32(a_bits, p.dt), gate_b = bits_as_f32(b_bits, p.dt);
-  const float a_log = bits_as_f32(a_log_bits, p.param_dt), bias = bits_as_f32(bias_bits, p.param_dt);
-
-  // the last `keep` rows of [conv_state | qkv] are the next conv state
-  if (s + keep >= p.S) store_adjacent<PER>(p.conv_next, ((size_t)b * keep + (s + keep - p.S)) * C + c, p.dt, x[K - 1]);
-  if (s == 0) {
+  unpack_adjacent<PER * K>(wr, DT, w);
+  if (is_v && lane < s1 - s0) {
+    const float gate_a = bits_as_f32(a_bits, DT), gate_b = bits_as_f32(b_bits, DT);
+    const float a_log = bits_as_f32(a_log_bits, p.param_dt), bias = bits_as_f32(bias_bits, p.param_dt);
+    // a + dt_bias and the softplus live in the promoted dtype of the two operands
+    const int sum_dt = pwide ? DFLASH_FP32 : DT;
+    const float apb = round_through(gate_a + bias, sum_dt);
+    const float sp = round_through(fmaxf(apb, 0.f) + log1pf(expf(-fabsf(apb))), sum_dt);
+    const size_t at = (token0 + gate_token) * p.Hv + hv;
+    p.g[at] = expf(-expf(a_log) * sp);
+    store_from_f32(p.beta, at, sigmoid_f32(gate_b), DT);
+  }
+  if (s0 == 0) {
     for (int r = p.S; r < keep; ++r) {  // blocks shorter than the state: old rows move up
       float old[PER];
 #pragma unroll
       for (int e = 0; e < PER; ++e) old[e] = 0.f;
-      if (p.conv_state) load_adjacent<PER>(p.conv_state, ((size_t)b * keep + r) * C + c, p.dt, old);
-      store_adjacent<PER>(p.conv_next, ((size_t)b * keep + (r - p.S)) * C + c, p.dt, old);
+      if (p.conv_state) load_adjacent<PER>(p.conv_state, ((size_t)b * keep + r) * C + c, DT, old);
+      store_adjacent<PER>(p.conv_next, ((size_t)b * keep + (r - p.S)) * C + c, DT, old);
     }
   }
 
-  float act[PER];
-  float ss = 0.f;
+#pragma unroll 1
+  for (int s = s0; s < s1; ++s) {
+    unpack_adjacent<PER>(xr[keep], DT, x[keep]);
+    const bool on = p.mask == nullptr || mask_byte[keep] != 0;
 #pragma unroll
-  for (int e = 0; e < PER; ++e) {
-    float acc = 0.f;
-#pragma unroll
-    for (int j = 0; j < K; ++j) acc += x[j][e] * w[e * K + j];
-    act[e] = silu_rounded(round_through(acc, p.dt), p.dt);
-    ss += act[e] * act[e];
-  }
-
-  if (is_v) {
-    store_adjacent<PER>(p.v, vrow * p.Dv + PER * lane, p.dt, act);
-    if (lane == 0) {
-      // a + dt_bias and the softplus live in the promoted dtype of the two operands
-      const int sum_dt = p.param_dt == DFLASH_FP32 ? DFLASH_FP32 : p.dt;
-      const float apb = round_through(gate_a + bias, sum_dt);
-      const float sp = round_through(fmaxf(apb, 0.f) + log1pf(expf(-fabsf(apb))), sum_dt);
-      p.g[vrow] = expf(-expf(a_log) * sp);
-      store_from_f32(p.beta, vrow, sigmoid_f32(gate_b), p.dt);
+    for (int e = 0; e < PER; ++e) x[keep][e] = on ? x[keep][e] : 0.f;
+    if (s + 1 < s1) {
+      load_adjacent_raw<PER>(p.qkv, qkv0 + (size_t)(s + 1) * p.qkv_row, wide, xr[keep]);
+      mask_byte[keep] = mask_at(s + 1);
     }
-    return;
-  }
+    // the last `keep` rows of [conv_state | qkv] are the next conv state
+    if (s + keep >= p.S) store_adjacent<PER>(p.conv_next, ((size_t)b * keep + (s + keep - p.S)) * C + c, DT, x[keep]);
+    if (p.qkv_out != nullptr) store_adjacent<PER>(p.qkv_out, (token0 + s) * C + c, DT, x[keep]);
 
-  const float inv_rms = 1.0f / sqrtf(wave_sum(ss) / (float)D + p.eps);
-  const bool is_q = h < p.Hk;
-  const float scale = is_q ? p.scale_q : p.scale_k;
-  void* out = is_q ? p.q : p.k;
-  const size_t row = ((size_t)b * p.S + s) * p.Hk + (is_q ? h : h - p.Hk);
-  float scaled[PER];
+    float act[PER];
+    float ss = 0.f;
 #pragma unroll
-  for (int e = 0; e < PER; ++e) scaled[e] = scale * round_through(act[e] * inv_rms, p.dt);
-  store_adjacent<PER>(out, row * p.Dk + PER * lane, p.dt, scaled);
+    for (int e = 0; e < PER; ++e) {
+      float acc = 0.f;
+#pragma unroll
+      for (int j = 0; j < K; ++j) acc += x[j][e] * w[e * K + j];
+      act[e] = silu_rounded(round_through(acc, DT), DT);
+      ss += act[e] * act[e];
+    }
+#pragma unroll
+    for (int j = 0; j < keep; ++j)
+#pragma unroll
+      for (int e = 0; e < PER; ++e) x[j][e] = x[j + 1][e];
+
+    if (is_v) {
+      store_adjacent<PER>(p.v, ((token0 + s) * p.Hv + hv) * p.Dv + PER * lane, DT, act);
+      continue;
+    }
+    const float inv_rms = 1.0f / sqrtf(wave_sum(ss) / (float)D + p.eps);
+    const bool is_q = h < p.Hk;
+    const float scale = is_q ? p.scale_q : p.scale_k;
+    void* out = is_q ? p.q : p.k;
+    const size_t row = (token0 + s) * p.Hk + (is_q ? h : h - p.Hk);
+    float scaled[PER];
+#pragma unroll
+    for (int e = 0; e < PER; ++e) scaled[e] = scale * round_through(act[e] * inv_rms, DT);
+    store_adjacent<PER>(out, row * p.Dk + PER * lane, DT, scaled);
+  }
 }
 
-template <int K>
+template <int DT, int K>
 __global__ __launch_bounds__(kWavesPerGroup * 64) void gdn_prepare_kernel(PrepareArgs p) {
   const int lane = threadIdx.x & 63;
-  const int heads = 2 * p.Hk + p.Hv;
-  const long long w = (long long)blockIdx.x * kWavesPerGroup + (threadIdx.x >> 6);
-  if (w >= (long long)p.B * p.S * heads) return;
-  const int h = (int)(w % heads);
-  const int s = (int)((w / heads) % p.S);
-  const int b = (int)(w / ((long long)heads * p.S));
+  const int heads = 2 * p.Hk + p.Hv, runs = (p.S + p.tokens - 1) / p.tokens;
+  const int w = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * kWavesPerGroup + (threadIdx.x >> 6)));
+  if (w >= p.B * runs * heads) return;
+  const int h = w % heads, run = w / heads;
+  const int b = run / runs, s0 = (run - b * runs) * p.tokens;
+  const int s1 = s0 + p.tokens < p.S ? s0 + p.tokens : p.S;
   switch ((h >= 2 * p.Hk ? p.Dv : p.Dk) / 64) {
-    case 1: prepare_head<1, K>(p, b, s, h, lane); break;
-    case 2: prepare_head<2, K>(p, b, s, h, lane); break;
-    case 3: prepare_head<3, K>(p, b, s, h, lane); break;
-    default: prepare_head<4, K>(p, b, s, h, lane); break;
+    case 1: prepare_head<DT, 1, K>(p, b, s0, s1, h, lane); break;
+    case 2: prepare_head<DT, 2, K>(p, b, s0, s1, h, lane); break;
+    case 3: prepare_head<DT, 3, K>(p, b, s0, s1, h, lane); break;
+    default: prepare_head<DT, 4, K>(p, b, s0, s1, h, lane); break;
   }
+}
+template <int DT>
+const void* prepare_kernel_for(int conv_kernel) {
+  return conv_kernel == 4   ? (const void*)gdn_prepare_kernel<DT, 4>
+         : conv_kernel == 3 ? (const void*)gdn_prepare_kernel<DT, 3>
+                            : (const void*)gdn_prepare_kernel<DT, 2>;
 }
 
 struct NormArgs {
-  const void* x;       // [rows, D]
-  const void* z;       // [rows, D]
+  const void* x;       // [B, T, H, D]
+  const void* z;       // [B, T, H, D], tokens and batches with a stride
   const void* weight;  // [D]
-  void* y;             // [rows, D]
-  long long rows;
-  int D, dt, weight_dt;
+  void* y;             // like x
+  long long z_batch, z_row;
+  int rows, T, H;      // rows = B T H
+  int per_wave;        // rows of a wave
+  int D, weight_dt;
   float eps;
 };
 
-// One wave per row: rms_norm(x, weight) * silu(z); a lane holds PER = D / 64 adjacent elements.
-template <int PER>
-__device__ __forceinline__ void gated_norm_row(const NormArgs& p, long long row, int lane) {
-  const bool wide = p.dt == DFLASH_FP32;
-  const size_t at = (size_t)row * p.D + PER * lane;
+// One wave for a few rows: rms_norm(x, weight) * silu(z); a lane holds PER = D / 64 adjacent elements.
+template <int DT, int PER>
+__device__ __forceinline__ void gated_norm_rows(const NormArgs& p, int row, int end, int lane) {
+  constexpr bool wide = DT == DFLASH_FP32;
   uint32_t xr[PER], zr[PER], wr[PER];
-  load_adjacent_raw<PER>(p.x, at, wide, xr);
-  load_adjacent_raw<PER>(p.z, at, wide, zr);
+  auto load = [&](int r) __attribute__((always_inline)) {
+    const int token = r / p.H, h = r - token * p.H, b = token / p.T, t = token - b * p.T;
+    load_adjacent_raw<PER>(p.x, (size_t)r * p.D + PER * lane, wide, xr);
+    load_adjacent_raw<PER>(p.z, (size_t)b * p.z_batch + (size_t)t * p.z_row + (size_t)h * p.D + PER * lane, wide, zr);
+  };
+  load(row);
   load_adjacent_raw<PER>(p.weight, PER * lane, p.weight_dt == DFLASH_FP32, wr);
   asm volatile("" ::: "memory");  // all three requests are out before the first value is interpreted
-  float x[PER], z[PER], wt[PER];
-  unpack_adjacent<PER>(xr, p.dt, x);
-  unpack_adjacent<PER>(zr, p.dt, z);
+  float wt[PER];
   unpack_adjacent<PER>(wr, p.weight_dt, wt);
-  float ss = 0.f;
+#pragma unroll 1
+  for (; row < end; ++row) {
+    float x[PER], z[PER];
+    unpack_adjacent<PER>(xr, DT, x);
+    unpack_adjacent<PER>(zr, DT, z);
+    if (row + 1 < end) load(row + 1);
+    float ss = 0.f;
 #pragma unroll
-  for (int e = 0; e < PER; ++e) ss += x[e] * x[e];
-  const float inv_rms = 1.0f / sqrtf(wave_sum(ss) / (float)p.D + p.eps);
-  float y[PER];
+    for (int e = 0; e < PER; ++e) ss += x[e] * x[e];
+    const float inv_rms = 1.0f / sqrtf(wave_sum(ss) / (float)p.D + p.eps);
+    float y[PER];
 #pragma unroll
-  for (int e = 0; e < PER; ++e) {
-    const float normed = round_through(x[e] * inv_rms * wt[e], p.dt);
-    y[e] = silu_rounded(z[e], p.dt) * normed;
+    for (int e = 0; e < PER; ++e) {
+      const float normed = round_through(x[e] * inv_rms * wt[e], DT);
+      y[e] = silu_rounded(z[e], DT) * normed;
+    }
+    store_adjacent<PER>(p.y, (size_t)row * p.D + PER * lane, DT, y);
   }
-  store_adjacent<PER>(p.y, at, p.dt, y);
 }
 
+template <int DT>
 __global__ __launch_bounds__(kWavesPerGroup * 64) void gdn_gated_norm_kernel(NormArgs p) {
   const int lane = threadIdx.x & 63;
-  const long long row = (long long)blockIdx.x * kWavesPerGroup + (threadIdx.x >> 6);
-  if (row >= p.rows) return;
+  const int w = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * kWavesPerGroup + (threadIdx.x >> 6)));
+  const long long first = (long long)w * p.per_wave;
+  if (first >= p.rows) return;
+  const int row = (int)first, end = p.rows - row < p.per_wave ? p.rows : row + p.per_wave;
   switch (p.D / 64) {
-    case 1: gated_norm_row<1>(p, row, lane); break;
-    case 2: gated_norm_row<2>(p, row, lane); break;
-    case 3: gated_norm_row<3>(p, row, lane); break;
-    default: gated_norm_row<4>(p, row, lane); break;
+    case 1: gated_norm_rows<DT, 1>(p, row, end, lane); break;
+    case 2: gated_norm_rows<DT, 2>(p, row, end, lane); break;
+    case 3: gated_norm_rows<DT, 3>(p, row, end, lane); break;
+    default: gated_norm_rows<DT, 4>(p, row, end, lane); break;
   }
 }
 
@@ -234,13 +274,13 @@ float as_array_scalar(double v, int dt) {
 }  // namespace
 }  // namespace dflash
 
-extern "C" int dflash_gdn_prepare(const void* qkv, const void* conv_state, const void* conv_w, const void* a,
-                                  const void* b, const void* A_log, const void* dt_bias, const uint8_t* mask,
-                                  void* conv_next, void* q, void* k, void* v, float* g, void* beta, int B,
-                                  int S, int Hk, int Hv, int Dk, int Dv, int conv_kernel, int dtype,
-                                  int param_dtype, float eps, void* stream) {
+extern "C" int dflash_gdn_prepare_rows(const void* qkv, const void* conv_state, const void* conv_w, const void* a,
+                                       const void* b, const void* A_log, const void* dt_bias, const uint8_t* mask,
+                                       void* conv_next, void* q, void* k, void* v, float* g, void* beta, void* qkv_out,
+                                       const long long* strides, int B, int S, int Hk, int Hv, int Dk, int Dv,
+                                       int conv_kernel, int dtype, int param_dtype, float eps, void* stream) {
   using namespace dflash;
-  DFLASH_REQUIRE(qkv && conv_w && a && b && A_log && dt_bias && conv_next && q && k && v && g && beta,
+  DFLASH_REQUIRE(qkv && conv_w && a && b && A_log && dt_bias && conv_next && q && k && v && g && beta && strides,
                  DFLASH_ERR_ARG, "dflash_gdn_prepare: null operand");
   DFLASH_REQUIRE(known_dtype(dtype) && known_dtype(param_dtype), DFLASH_ERR_ARG,
                  "dflash_gdn_prepare: unknown dtype code");
@@ -248,30 +288,65 @@ extern "C" int dflash_gdn_prepare(const void* qkv, const void* conv_state, const
                  "dflash_gdn_prepare: bad dimension (conv kernels of 2 to 4 taps)");
   DFLASH_REQUIRE(head_dim_ok(Dk) && head_dim_ok(Dv), DFLASH_ERR_SHAPE,
                  "dflash_gdn_prepare: head dims must be multiples of 64 up to 256, got %d and %d", Dk, Dv);
-  const long long waves = (long long)B * S * (2 * Hk + Hv);
-  DFLASH_REQUIRE(waves < (1ll << 31), DFLASH_ERR_SHAPE, "dflash_gdn_prepare: too many rows");
+  const int heads = 2 * Hk + Hv;
+  DFLASH_REQUIRE((long long)B * S * heads < (1ll << 31), DFLASH_ERR_SHAPE, "dflash_gdn_prepare: too many rows");
   if (B == 0) return DFLASH_OK;
   DFLASH_REQUIRE(S > 0, DFLASH_ERR_SHAPE, "dflash_gdn_prepare: empty block");
+  for (int i = 0; i < 6; ++i) DFLASH_REQUIRE(strides[i] >= 0, DFLASH_ERR_SHAPE, "dflash_gdn_prepare: negative stride");
   PrepareArgs p;
   p.qkv = qkv; p.conv_state = conv_state; p.conv_w = conv_w; p.a = a; p.b = b; p.A_log = A_log;
   p.dt_bias = dt_bias; p.mask = mask; p.conv_next = conv_next; p.q = q; p.k = k; p.v = v; p.g = g;
-  p.beta = beta; p.B = B; p.S = S; p.Hk = Hk; p.Hv = Hv; p.Dk = Dk; p.Dv = Dv; p.K = conv_kernel;
-  p.dt = dtype; p.param_dt = param_dtype; p.eps = eps;
+  p.beta = beta; p.qkv_out = qkv_out; p.B = B; p.S = S; p.Hk = Hk; p.Hv = Hv; p.Dk = Dk; p.Dv = Dv;
+  p.qkv_batch = strides[0]; p.qkv_row = strides[1]; p.a_batch = strides[2]; p.a_row = strides[3];
+  p.b_batch = strides[4]; p.b_row = strides[5];
+  p.param_dt = param_dtype; p.eps = eps;
   const double inv_scale = 1.0 / sqrt((double)Dk);
   p.scale_q = as_array_scalar(inv_scale * inv_scale, dtype);
   p.scale_k = as_array_scalar(inv_scale, dtype);
+  // as many tokens per wave as leave 8 waves per SIMD: below that a wave's latency counts, not its instructions
+  const long long per = (long long)B * S * heads / 8192;
+  p.tokens = per < 1 ? 1 : per > 16 ? 16 : (int)per;
+  const long long waves = (long long)B * ((S + p.tokens - 1) / p.tokens) * heads;
   const unsigned groups = (unsigned)((waves + kWavesPerGroup - 1) / kWavesPerGroup);
-  const dim3 grid(groups), block(kWavesPerGroup * 64);
-  if (conv_kernel == 4) {
-    hipLaunchKernelGGL(gdn_prepare_kernel<4>, grid, block, 0, (hipStream_t)stream, p);
-  } else if (conv_kernel == 3) {
-    hipLaunchKernelGGL(gdn_prepare_kernel<3>, grid, block, 0, (hipStream_t)stream, p);
-  } else {
-    hipLaunchKernelGGL(gdn_prepare_kernel<2>, grid, block, 0, (hipStream_t)stream, p);
-  }
-  DFLASH_HIP_OK(hipGetLastError());
+  const void* fn = dtype == DFLASH_BF16   ? prepare_kernel_for<DFLASH_BF16>(conv_kernel)
+                   : dtype == DFLASH_FP16 ? prepare_kernel_for<DFLASH_FP16>(conv_kernel)
+                                          : prepare_kernel_for<DFLASH_FP32>(conv_kernel);
+  void* args[] = {&p};
+  DFLASH_HIP_OK(hipLaunchKernel(fn, dim3(groups), dim3(kWavesPerGroup * 64), args, 0, (hipStream_t)stream));
   return DFLASH_OK;
 }
+
+extern "C" int dflash_gdn_prepare(const void* qkv, const void* conv_state, const void* conv_w, const void* a,
+                                  const void* b, const void* A_log, const void* dt_bias, const uint8_t* mask,
+                                  void* conv_next, void* q, void* k, void* v, float* g, void* beta, int B,
+                                  int S, int Hk, int Hv, int Dk, int Dv, int conv_kernel, int dtype,
+                                  int param_dtype, float eps, void* stream) {
+  const long long row = 2ll * Hk * Dk + (long long)Hv * Dv;
+  const long long strides[6] = {S * row, row, (long long)S * Hv, Hv, (long long)S * Hv, Hv};
+  return dflash_gdn_prepare_rows(qkv, conv_state, conv_w, a, b, A_log, dt_bias, mask, conv_next, q, k, v, g, beta, nullptr, strides,
+                                 B, S, Hk, Hv, Dk, Dv, conv_kernel, dtype, param_dtype, eps, stream);
+}
+
+namespace dflash {
+// x, y [B, T, H, D] contiguous, z with these strides (also called by gdn_forward.hip)
+int gdn_gated_norm_launch(const void* x, const void* z, const void* weight, void* y, int B, int T, int H, int D,
+                          long long z_batch, long long z_row, int dtype, int weight_dtype, float eps, hipStream_t stream) {
+  NormArgs p;
+  p.x = x; p.z = z; p.weight = weight; p.y = y;
+  p.z_batch = z_batch; p.z_row = z_row;
+  p.rows = B * T * H; p.T = T; p.H = H; p.D = D;
+  p.weight_dt = weight_dtype; p.eps = eps;
+  p.per_wave = p.rows / 8192 < 1 ? 1 : p.rows / 8192 > 16 ? 16 : p.rows / 8192;
+  const long long waves = ((long long)p.rows + p.per_wave - 1) / p.per_wave;
+  const unsigned groups = (unsigned)((waves + kWavesPerGroup - 1) / kWavesPerGroup);
+  const void* fn = dtype == DFLASH_BF16   ? (const void*)gdn_gated_norm_kernel<DFLASH_BF16>
+                   : dtype == DFLASH_FP16 ? (const void*)gdn_gated_norm_kernel<DFLASH_FP16>
+                                          : (const void*)gdn_gated_norm_kernel<DFLASH_FP32>;
+  void* args[] = {&p};
+  DFLASH_HIP_OK(hipLaunchKernel(fn, dim3(groups), dim3(kWavesPerGroup * 64), args, 0, stream));
+  return DFLASH_OK;
+}
+}  // namespace dflash
 
 extern "C" int dflash_gdn_gated_norm(const void* x, const void* z, const void* weight, void* y, long long rows,
                                      int D, int dtype, int weight_dtype, float eps, void* stream) {
@@ -283,11 +358,5 @@ extern "C" int dflash_gdn_gated_norm(const void* x, const void* z, const void* w
   DFLASH_REQUIRE(head_dim_ok(D), DFLASH_ERR_SHAPE,
                  "dflash_gdn_gated_norm: row length must be a multiple of 64 up to 256, got %d", D);
   if (rows == 0) return DFLASH_OK;
-  NormArgs p;
-  p.x = x; p.z = z; p.weight = weight; p.y = y; p.rows = rows; p.D = D; p.dt = dtype;
-  p.weight_dt = weight_dtype; p.eps = eps;
-  const unsigned groups = (unsigned)((rows + kWavesPerGroup - 1) / kWavesPerGroup);
-  hipLaunchKernelGGL(gdn_gated_norm_kernel, dim3(groups), dim3(kWavesPerGroup * 64), 0, (hipStream_t)stream, p);
-  DFLASH_HIP_OK(hipGetLastError());
-  return DFLASH_OK;
+  return gdn_gated_norm_launch(x, z, weight, y, 1, 1, (int)rows, D, 0, 0, dtype, weight_dtype, eps, (hipStream_t)stream);
 }

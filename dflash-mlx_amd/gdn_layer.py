@@ -21,6 +21,7 @@ out_proj); its own ``forward`` is the plain, non-speculative call.
 """
 from __future__ import annotations
 
+import ctypes
 import os
 from typing import Any, Optional, Tuple
 
@@ -99,10 +100,11 @@ def _kernel_covers(x: torch.Tensor, *dims: int) -> bool:
 
 def gdn_prepare(qkv: torch.Tensor, conv_state: Optional[torch.Tensor], conv_w: torch.Tensor, a: torch.Tensor,
                 b: torch.Tensor, A_log: torch.Tensor, dt_bias: torch.Tensor, mask: Optional[torch.Tensor] = None,
-                *, Hk: int, Hv: int, Dk: int, Dv: int, eps: float = 1e-6
+                *, Hk: int, Hv: int, Dk: int, Dv: int, eps: float = 1e-6, qkv_out: Optional[torch.Tensor] = None
                 ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
     """Mask, conv, silu, split, norms and gates of a GatedDeltaNet call in one launch:
-    (conv_next [B,K-1,C], q, k [B,S,Hk,Dk], v [B,S,Hv,Dv], g [B,S,Hv] fp32, beta [B,S,Hv])."""
+    (conv_next [B,K-1,C], q, k [B,S,Hk,Dk], v [B,S,Hv,Dv], g [B,S,Hv] fp32, beta [B,S,Hv]).  qkv, a and b are read where
+    they are (columns of a joint product).  ``qkv_out`` [B,S,C], contiguous, receives qkv with masked rows zeroed."""
     B, S, C = (int(d) for d in qkv.shape)
     if conv_w.ndim == 3:            # mlx conv1d weight [C, K, 1]
         conv_w = conv_w.reshape(conv_w.shape[0], conv_w.shape[1])
@@ -112,6 +114,8 @@ def gdn_prepare(qkv: torch.Tensor, conv_state: Optional[torch.Tensor], conv_w: t
     same = (conv_w.dtype == a.dtype == b.dtype == qkv.dtype and A_log.dtype == dt_bias.dtype and
             A_log.dtype in _DTYPE_CODE and (conv_state is None or conv_state.dtype == qkv.dtype))
     if not (_kernel_covers(qkv, Dk, Dv) and same and S > 0 and 2 <= K <= 4):
+        if qkv_out is not None:
+            qkv_out.copy_(qkv if mask is None else torch.where(mask.to(torch.bool)[..., None], qkv, torch.zeros_like(qkv)))
         return gdn_prepare_ops(qkv, conv_state, conv_w, a, b, A_log, dt_bias, mask,
                                Hk=Hk, Hv=Hv, Dk=Dk, Dv=Dv, eps=eps)
     lib = _native.lib()
@@ -127,7 +131,15 @@ def gdn_prepare(qkv: torch.Tensor, conv_state: Optional[torch.Tensor], conv_w: t
             raise ValueError(f"gdn_prepare: {name} must be {list(shape)} on {dev}, got {list(t.shape)} on {t.device}")
     if mask is not None and (mask.numel() != B * S or mask.device != dev):
         raise ValueError(f"gdn_prepare: mask must hold {B} x {S} entries on {dev}")
-    qkv_c, w_c, a_c, b_c = qkv.contiguous(), conv_w.contiguous(), a.contiguous(), b.contiguous()
+    if qkv_out is not None and not (qkv_out.shape == qkv.shape and qkv_out.dtype == dt and qkv_out.device == dev
+                                    and qkv_out.is_contiguous()):
+        raise ValueError(f"gdn_prepare: qkv_out must be a contiguous {list(qkv.shape)} of {dt} on {dev}")
+    step = qkv.element_size()
+    in_place = qkv.stride(2) == 1 and (qkv.data_ptr() | qkv.stride(0) * step | qkv.stride(1) * step) % 8 == 0
+    qkv_c, w_c = qkv if in_place else qkv.contiguous(), conv_w.contiguous()
+    a_c, b_c = (t if t.stride(2) == 1 else t.contiguous() for t in (a, b))
+    strides = (ctypes.c_longlong * 6)(qkv_c.stride(0), qkv_c.stride(1), a_c.stride(0), a_c.stride(1), b_c.stride(0),
+                                      b_c.stride(1))
     cs = None if conv_state is None else conv_state.contiguous()
     mask_c = None if mask is None else mask.to(torch.uint8).contiguous()
     conv_next = torch.empty((B, K - 1, C), dtype=dt, device=dev)
@@ -136,11 +148,12 @@ def gdn_prepare(qkv: torch.Tensor, conv_state: Optional[torch.Tensor], conv_w: t
     v = torch.empty((B, S, Hv, Dv), dtype=dt, device=dev)
     g = torch.empty((B, S, Hv), dtype=torch.float32, device=dev)
     beta = torch.empty((B, S, Hv), dtype=dt, device=dev)
-    rc = lib.dflash_gdn_prepare(
+    rc = lib.dflash_gdn_prepare_rows(
         qkv_c.data_ptr(), None if cs is None else cs.data_ptr(), w_c.data_ptr(), a_c.data_ptr(), b_c.data_ptr(),
         A_log.contiguous().data_ptr(), dt_bias.contiguous().data_ptr(),
         None if mask_c is None else mask_c.data_ptr(), conv_next.data_ptr(), q.data_ptr(), k.data_ptr(),
-        v.data_ptr(), g.data_ptr(), beta.data_ptr(), B, S, Hk, Hv, Dk, Dv, K, _DTYPE_CODE[dt],
+        v.data_ptr(), g.data_ptr(), beta.data_ptr(), None if qkv_out is None else qkv_out.data_ptr(), strides, B, S, Hk, Hv,
+        Dk, Dv, K, _DTYPE_CODE[dt],
         _DTYPE_CODE[A_log.dtype], float(eps), _native.raw_stream(dev))
     _native.check(rc, "dflash_gdn_prepare")
     return conv_next, q, k, v, g, beta
@@ -239,9 +252,14 @@ def _gdn_call(self, inputs: torch.Tensor, mask: Optional[torch.Tensor], cache: O
     z = z.reshape(B, S, self.num_v_heads, self.head_v_dim)
 
     conv_state = cache[0] if cache is not None else None
+    # the rollback wants qkv in one piece, without what the mask hides
+    tape_qkv = qkv
+    if record and (mask is not None or not qkv.is_contiguous()):
+        tape_qkv = torch.empty(qkv.shape, dtype=qkv.dtype, device=qkv.device)
     conv_next, q, k, v, g, beta = gdn_prepare(
         qkv, conv_state, self.conv1d.weight, a, b, self.A_log, self.dt_bias, mask,
-        Hk=self.num_k_heads, Hv=self.num_v_heads, Dk=self.head_k_dim, Dv=self.head_v_dim)
+        Hk=self.num_k_heads, Hv=self.num_v_heads, Dk=self.head_k_dim, Dv=self.head_v_dim,
+        qkv_out=None if tape_qkv is qkv else tape_qkv)
     if cache is not None:
         cache[0] = conv_next
 
@@ -255,9 +273,7 @@ def _gdn_call(self, inputs: torch.Tensor, mask: Optional[torch.Tensor], cache: O
     out, state, innovation_tape = gated_delta_kernel_with_tape(
         q, k, v, g, beta, state, mask, output_norm=(z, norm.weight, norm.eps) if fused else None, with_tape=record)
     if record:
-        if mask is not None:
-            qkv = torch.where(mask.to(torch.bool)[..., None], qkv, torch.zeros_like(qkv))
-        cache.record_tape(tape=innovation_tape, k=k, g=g, qkv=qkv)
+        cache.record_tape(tape=innovation_tape, k=k, g=g, qkv=tape_qkv)
     if cache is not None:
         cache[1] = state
     if not fused:

@@ -150,12 +150,17 @@ def gated_delta_kernel_with_tape(q: torch.Tensor, k: torch.Tensor, v: torch.Tens
         z, weight, eps = output_norm
         if not fused_output_norm_applies(q, v, state, z, weight):
             raise ValueError("output_norm: shapes or dtypes the fused kernel does not take")
-        z_c, w_c = z.contiguous(), weight.contiguous()
+        z_c, w_c = z, weight.contiguous()
+        # steps and slots may have a stride (columns of a joint product); heads and columns lie together
+        if z_c.stride(3) != 1 or z_c.stride(2) != dv or z_c.stride(1) == 0 or z_c.data_ptr() % 16 \
+                or (z_c.stride(0) | z_c.stride(1)) * z_c.element_size() % 16:
+            z_c = z_c.contiguous()
     rc = lib.dflash_gdn_forward(
         q_c.data_ptr(), k_c.data_ptr(), v_c.data_ptr(), g_c.data_ptr(), beta_c.data_ptr(),
         state_c.data_ptr(), state_out.data_ptr(), None if z_c is None else z_c.data_ptr(),
         None if w_c is None else w_c.data_ptr(), y.data_ptr(), None if tape is None else tape.data_ptr(), mask_ptr,
-        None if ws is None else ws.data_ptr(), need, B, T, hk, hv, dk, dv, code, _DTYPE_CODE[g.dtype],
+        None if ws is None else ws.data_ptr(), need,
+        0 if z_c is None else z_c.stride(0), 0 if z_c is None else z_c.stride(1), B, T, hk, hv, dk, dv, code, _DTYPE_CODE[g.dtype],
         _DTYPE_CODE[beta.dtype], _DTYPE_CODE[state.dtype], _DTYPE_CODE[q.dtype if w_c is None else w_c.dtype], per_dk,
         float(eps), _native.raw_stream(q.device))
     _native.check(rc, "dflash_gdn_forward")

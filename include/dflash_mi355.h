@@ -391,14 +391,16 @@ int dflash_gdn_forward_tape_norm(const void* q, const void* k, const void* v, co
  * dflash_gdn_forward_workspace_bytes() bytes (16-byte aligned, contents irrelevant; 0 where none is used)
  * prompts - T > 16, bf16 q / k / v, one gate per head, Dk 64 or 128, Dv a multiple of 16 - go through the
  * matrix cores in chunks of 32 tokens.  There a 16-bit state is carried in fp32 and rounded once, behind
- * the last token, and tape may be NULL (not recorded).
+ * the last token, and tape may be NULL (not recorded).  z_row_stride, z_batch_stride: elements from a step's z to the
+ * next one's and from slot to slot (heads and columns contiguous, rows at least 8-byte aligned); 0: z [slots, T, Hv, Dv].
  */
 size_t dflash_gdn_forward_workspace_bytes(int slots, int T, int Hk, int Hv, int Dk, int Dv, int in_dtype, int g_per_dk);
 int dflash_gdn_forward(const void* q, const void* k, const void* v, const void* g, const void* beta,
                        const void* state_in, void* state_out, const void* z, const void* norm_weight, void* y,
-                       float* tape, const uint8_t* mask, void* workspace, size_t workspace_bytes, int slots, int T,
-                       int Hk, int Hv, int Dk, int Dv, int in_dtype, int g_dtype, int beta_dtype, int state_dtype,
-                       int weight_dtype, int g_per_dk, float eps, void* stream);
+                       float* tape, const uint8_t* mask, void* workspace, size_t workspace_bytes,
+                       long long z_batch_stride, long long z_row_stride, int slots, int T, int Hk, int Hv, int Dk, int Dv,
+                       int in_dtype, int g_dtype, int beta_dtype, int state_dtype, int weight_dtype, int g_per_dk,
+                       float eps, void* stream);
 
 /*
  * GatedDeltaNet layer, everything between the input projections and the recurrence, in one
@@ -423,6 +425,17 @@ int dflash_gdn_prepare(const void* qkv, const void* conv_state, const void* conv
                        void* conv_next, void* q, void* k, void* v, float* g, void* beta, int B,
                        int S, int Hk, int Hv, int Dk, int Dv, int conv_kernel, int dtype,
                        int param_dtype, float eps, void* stream);
+
+/*
+ * dflash_gdn_prepare on projections as a joint product leaves them.  strides: 6 element counts - batch and row of qkv, a,
+ * b (channels and heads contiguous; rows of 16-bit qkv at least 8-byte aligned).  qkv_out [B, S, C] contiguous receives
+ * qkv with masked rows zeroed, or NULL.
+ */
+int dflash_gdn_prepare_rows(const void* qkv, const void* conv_state, const void* conv_w, const void* a,
+                            const void* b, const void* A_log, const void* dt_bias, const uint8_t* mask,
+                            void* conv_next, void* q, void* k, void* v, float* g, void* beta, void* qkv_out,
+                            const long long* strides, int B, int S, int Hk, int Hv, int Dk, int Dv,
+                            int conv_kernel, int dtype, int param_dtype, float eps, void* stream);
 
 /*
  * Gated output norm of a GatedDeltaNet layer: y = silu(z) * rms_norm(x, weight, eps) over rows of

@@ -190,3 +190,59 @@ def test_layer_hook_with_an_arena_cache_matches_the_per_layer_cache(native_lib, 
     torch.cuda.synchronize()
     assert torch.equal(y_arena, y_plain)
     assert torch.equal(cache[1], plain[1]) and torch.equal(cache[0], plain[0])
+
+
+@pytest.mark.parametrize("name", ["bf16", "fp16", "fp32"])
+@pytest.mark.parametrize("B,S,Hk,Hv,Dk,Dv,K,masked", [(1, 1030, 16, 32, 128, 128, 4, False), (2, 333, 8, 16, 64, 192, 3, True),
+                                                      (1, 700, 4, 8, 256, 64, 2, True), (3, 17, 2, 2, 128, 128, 4, True)])
+def test_long_prompts_and_strided_projections(native_lib, name, B, S, Hk, Hv, Dk, Dv, K, masked):
+    """Several tokens per wave and rows with a stride: the bits of blocks of at most 16 tokens (one token per wave) of
+    contiguous arrays, their conv windows handed on; qkv_out is qkv without what the mask hides."""
+    dt = TORCH[name]
+    gen = torch.Generator(device=DEV).manual_seed(S)
+    C = 2 * Hk * Dk + Hv * Dv
+    joint = torch.randn((B, S, C + 64 + 2 * Hv), generator=gen, device=DEV).to(dt)
+    qkv, b, a = joint[..., :C], joint[..., C + 64:C + 64 + Hv], joint[..., C + 64 + Hv:]
+    conv_w = (torch.randn((C, K), generator=gen, device=DEV) * 0.5).to(dt)
+    A_log, dt_bias = torch.randn(Hv, generator=gen, device=DEV).to(dt), torch.randn(Hv, generator=gen, device=DEV).to(dt)
+    mask = torch.rand((B, S), generator=gen, device=DEV) > 0.2 if masked else None
+    state = torch.randn((B, K - 1, C), generator=gen, device=DEV).to(dt)
+    dims = dict(Hk=Hk, Hv=Hv, Dk=Dk, Dv=Dv)
+    kept = torch.full((B, S, C), 7.0, dtype=dt, device=DEV)
+    got = G.gdn_prepare(qkv, state, conv_w, a, b, A_log, dt_bias, mask, **dims, qkv_out=kept)
+    assert torch.equal(kept, qkv if mask is None else torch.where(mask[..., None], qkv, torch.zeros_like(qkv)))
+    pieces, window = [], state
+    for s in range(0, S, 16):
+        cut = slice(s, min(s + 16, S))
+        part = G.gdn_prepare(qkv[:, cut].contiguous(), window, conv_w, a[:, cut].contiguous(), b[:, cut].contiguous(), A_log,
+                             dt_bias, None if mask is None else mask[:, cut].contiguous(), **dims)
+        window = part[0]
+        pieces.append(part[1:])
+    assert torch.equal(got[0], window)
+    for whole, *parts in zip(got[1:], *pieces):
+        assert torch.equal(whole, torch.cat(parts, dim=1))
+
+
+@pytest.mark.parametrize("name", ["bf16", "fp32"])
+@pytest.mark.parametrize("B,T,Hv,Dv,state", [(1, 16, 32, 128, "fp32"), (2, 16, 8, 128, "bf16"), (1, 1030, 16, 128, "fp32"),
+                                             (2, 21, 4, 64, "fp32")])
+def test_output_norm_reads_a_strided_gate(native_lib, name, B, T, Hv, Dv, state):
+    """z as the columns of a joint product, through the block kernel, the prompt kernels and the norm of its own."""
+    from dflash_mlx_amd.kernels import gated_delta_kernel_with_tape
+
+    dt = TORCH[name]
+    gen = torch.Generator(device=DEV).manual_seed(T)
+    r = lambda *s: torch.randn(s, generator=gen, device=DEV)  # noqa: E731
+    q, k, v = (r(B, T, h, Dv).mul(0.1).to(dt) for h in (Hv, Hv, Hv))
+    g, beta = torch.rand((B, T, Hv), generator=gen, device=DEV), torch.sigmoid(r(B, T, Hv)).to(dt)
+    joint = r(B, T, 96 + Hv * Dv + 32).to(dt)
+    z = joint[..., 96:96 + Hv * Dv].reshape(B, T, Hv, Dv)
+    assert not z.is_contiguous()
+    weight, s0 = (1 + 0.1 * r(Dv)).to(dt), r(B, Hv, Dv, Dv).to(TORCH[state])
+    got = gated_delta_kernel_with_tape(q, k, v, g, beta, s0, output_norm=(z, weight, 1e-6))
+    want = gated_delta_kernel_with_tape(q, k, v, g, beta, s0, output_norm=(z.contiguous(), weight, 1e-6))
+    assert all(torch.equal(x, y) for x, y in zip(got, want))
+    plain = gated_delta_kernel_with_tape(q, k, v, g, beta, s0)[0]
+    pieces = [G.gated_norm(plain[:, t:t + 16], z[:, t:t + 16], weight) for t in range(0, T, 16)]
+    assert torch.equal(G.gated_norm(plain, z, weight), torch.cat(pieces, dim=1))
+    assert torch.allclose(got[0].float(), torch.cat(pieces, dim=1).float(), rtol=4 * ULP[name], atol=1e-4)
