@@ -44,12 +44,11 @@ typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 
 __device__ __forceinline__ float bf16_bits_to_f32(uint32_t h) { return __uint_as_float(h << 16); }
 
-// Round-to-nearest-even fp32 -> bf16 bit pattern (NaN kept quiet).
+// Round-to-nearest-even fp32 -> bf16 bit pattern (NaN kept quiet): one v_cvt_pk_bf16_f32, where the
+// add-and-shift form with its test for NaN is seven instructions.  GatedDeltaNet glue of 1024 tokens, which rounds every
+// element five times: prepare 28.6 -> 23.3 us, gated norm 13.6 -> 12.3 us.
 __device__ __forceinline__ uint32_t f32_to_bf16_bits(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return 0x7fc0u;
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return u >> 16;
+  return __builtin_bit_cast(uint16_t, (__bf16)f);
 }
 
 __device__ __forceinline__ float f16_bits_to_f32(uint32_t h) {
