@@ -23,8 +23,10 @@
 //    wave are dealt to its tiles so that a lane ends up with 4*NT consecutive columns of one row.
 //  * Where the tiles do not fill the chip, K is cut into slices: workgroups leave fp32 partial tiles in
 //    the workspace, and whoever arrives last at a tile adds them in order of k.  Nobody waits.  Deterministic.
+//    Of more tiles than the chip takes at once, only those of the last, incomplete round are cut: 1088 tiles of
+//    5120 x 34816 are 4 rounds and a quarter instead of 5 (a 27B layer over 1024 tokens 787 -> 758 us).
 //
-// Measured (kernel time, group 64): 1024 rows of 5120 x 34816 415 us (880 TFLOP/s; torch's bf16 product of weights
+// Measured (kernel time, group 64, before that cut): 1024 rows of 5120 x 34816 415 us (880 TFLOP/s; torch's bf16 product of weights
 // that are already dense 411 us), 17408 x 5120 204 us (237), 5120 x 5120 71 us (62); 77 rows of
 // 4096 x 24576 42 us, 12288 x 4096 22 us.  The form with codes in registers took 540, 260, 105 and 87, 31 us for
 // the same tiles.  What bounds it at many rows is shared: matrix instructions 45 % of the cycles,
@@ -45,11 +47,12 @@ struct Args {
   const uint16_t* scales;
   const uint16_t* biases;
   uint16_t* y;
-  float* partials;      // [tile][slice][tile of 16x16 in the workgroup][thread][4]
-  uint32_t* counters;   // one per tile, zero between calls
+  float* partials;      // [cut tile][slice][tile of 16x16 in the workgroup][thread][4]
+  uint32_t* counters;   // one per cut tile, zero between calls
   int M, K, N;
   int group_shift;      // log2(group size)
-  int tiles_m, tiles, slices;
+  int tiles_m, tiles;
+  int whole, slices;    // tiles computed in one piece; slices of K of the others
   int stages;           // ceil(K / (64 KG))
 };
 
@@ -116,11 +119,13 @@ __global__ __launch_bounds__(256 * KG, 2) void qmm_rows_kernel(Args a) {
   const int wave = __builtin_amdgcn_readfirstlane((tid >> 6) & 3);
   const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
   const int li = lane & 15, kq = lane >> 4;
-  const int grid = (int)gridDim.x;
-  // neighbours in tile order (same columns, other rows) behind one L2
-  const int wg = grid % 8 == 0 ? (int)(blockIdx.x % 8) * (grid / 8) + (int)(blockIdx.x / 8) : (int)blockIdx.x;
-  const int slice = wg % a.slices, tile = wg / a.slices;
-  const int st0 = (int)((long long)a.stages * slice / a.slices), st1 = (int)((long long)a.stages * (slice + 1) / a.slices);
+  // neighbours in tile order (same columns, other rows) behind one L2; the whole tiles are dispatched first
+  const bool cut = (int)blockIdx.x >= a.whole;
+  const int part = cut ? (int)gridDim.x - a.whole : a.whole, at = (int)blockIdx.x - (cut ? a.whole : 0);
+  const int wg = part % 8 == 0 ? (at % 8) * (part / 8) + at / 8 : at;
+  const int slices = cut ? a.slices : 1, slice = wg % slices, cut_tile = wg / slices;
+  const int tile = cut ? a.whole + cut_tile : wg;
+  const int st0 = (int)((long long)a.stages * slice / slices), st1 = (int)((long long)a.stages * (slice + 1) / slices);
   const int nb = tile / a.tiles_m, mb = tile - nb * a.tiles_m;
   const int m0 = mb * BM, n0 = nb * BN;
   const int G = a.K >> a.group_shift;
@@ -378,7 +383,7 @@ __global__ __launch_bounds__(256 * KG, 2) void qmm_rows_kernel(Args a) {
       if (n + 4 * t < out_cols) *reinterpret_cast<uint2*>(dst + 4 * t) = w;
     }
   };
-  if (a.slices == 1) {
+  if (slices == 1) {
     if (kg == 0) {
 #pragma unroll
       for (int i = 0; i < MT; ++i) emit(i, acc[i]);
@@ -387,7 +392,7 @@ __global__ __launch_bounds__(256 * KG, 2) void qmm_rows_kernel(Args a) {
   }
   // Partial tiles are written through to and read from the level all XCDs share (sc1, as in the streaming kernel).
   constexpr size_t kTileFloats = (size_t)BM * BN;
-  float* const first = a.partials + (size_t)tile * a.slices * kTileFloats;
+  float* const first = a.partials + (size_t)cut_tile * slices * kTileFloats;
   if (kg == 0) {
     float* mine = first + slice * kTileFloats + (tid & 255) * 4;
 #pragma unroll
@@ -398,7 +403,7 @@ __global__ __launch_bounds__(256 * KG, 2) void qmm_rows_kernel(Args a) {
   // every wave's stores are acknowledged before the arrival is counted
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  if (tid == 0) s_last = atomicInc(&a.counters[tile], (uint32_t)(a.slices - 1)) == (uint32_t)(a.slices - 1);
+  if (tid == 0) s_last = atomicInc(&a.counters[cut_tile], (uint32_t)(slices - 1)) == (uint32_t)(slices - 1);
   __syncthreads();
   if (!s_last || kg != 0) return;
   // in order of k; a row of tiles of every slice is asked for before the first is looked at
@@ -408,11 +413,11 @@ __global__ __launch_bounds__(256 * KG, 2) void qmm_rows_kernel(Args a) {
     f32x4_t sum[NT];
 #pragma unroll
     for (int t = 0; t < NT; ++t) sum[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    for (int c0 = 0; c0 < a.slices; c0 += 4) {
+    for (int c0 = 0; c0 < slices; c0 += 4) {
       f32x4_t v[4][NT];
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        const int cc = c0 + c < a.slices ? c0 + c : a.slices - 1;
+        const int cc = c0 + c < slices ? c0 + c : slices - 1;
 #pragma unroll
         for (int t = 0; t < NT; ++t)
           v[c][t] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(
@@ -420,7 +425,7 @@ __global__ __launch_bounds__(256 * KG, 2) void qmm_rows_kernel(Args a) {
       }
 #pragma unroll
       for (int c = 0; c < 4; ++c)
-        if (c0 + c < a.slices) {
+        if (c0 + c < slices) {
 #pragma unroll
           for (int t = 0; t < NT; ++t) sum[t] += v[c][t];
         }
@@ -459,7 +464,7 @@ const void* kernel_for(int mt, int nt, int kg, bool mixed, bool silu_mul) {
 constexpr int lds_bytes(int mt, int nt, int kg) { return kg * (2 * 16 * mt * 128 + 3 * 64 * nt * 32) + 2 * 2 * 64 * nt * 16; }
 
 struct Plan {
-  int mt, nt, kg, slices, tiles_m, tiles, stages, grid;
+  int mt, nt, kg, whole, slices, tiles_m, tiles, stages, grid;
   size_t workspace;
 };
 
@@ -490,21 +495,24 @@ Plan make_plan(int M, int K, int N, int cus, bool mixed, bool silu_mul) {
         p.stages = (K + kStageK * kg - 1) / (kStageK * kg);
         const int slots = cus * (kg == 1 ? 2 : 1);
         const double stage = 0.134 + 0.1256 * nt + 0.0463 * mt + 0.0342 * mt * nt;
-        for (int slices = 1; slices <= 16 && slices <= p.stages; ++slices) {
-          if (slices > 1 && (p.tiles * slices > slots || p.tiles > (int)(kCounterBytes / 4))) break;
+        const int whole = p.tiles / slots * slots, cut = p.tiles - whole;
+        for (int slices = 1; slices <= 16 && slices <= p.stages && (slices == 1 || cut > 0); ++slices) {
+          if (slices > 1 && (cut * slices > (whole > 0 ? 2 : 1) * slots || cut > (int)(kCounterBytes / 4))) break;
           p.slices = slices;
-          p.grid = p.tiles * slices;
-          const int full = p.grid / slots, rest = p.grid - full * slots;
+          p.whole = slices > 1 ? whole : p.tiles;
+          p.grid = slices > 1 ? whole + cut * slices : p.tiles;
+          const int full = cut * slices / slots, rest = cut * slices - full * slots;
           // a last round with one workgroup per CU where there is room for two is the faster one
           const double rounds = full + (rest == 0 ? 0. : kg == 1 && rest <= cus ? 0.62 : 1.);
-          const double us = 7.55 + rounds * ((p.stages + slices - 1) / slices * stage - 2.89) +
+          const double us = 7.55 + whole / slots * (p.stages * stage - 2.89) +
+                            rounds * ((p.stages + slices - 1) / slices * stage - 2.89) +
                             (slices > 1 ? 1.48 + 0.113 * slices * mt * nt : 0.);
           if (best.grid == 0 || us < best_us) best = p, best_us = us;
         }
       }
     }
   }
-  best.workspace = best.slices > 1 ? kCounterBytes + (size_t)best.grid * (16 * best.mt) * (64 * best.nt) * sizeof(float) : 0;
+  best.workspace = best.slices > 1 ? kCounterBytes + (size_t)(best.grid - best.whole) * (16 * best.mt) * (64 * best.nt) * sizeof(float) : 0;
   return best;
 }
 
@@ -556,7 +564,7 @@ extern "C" int dflash_qmm_rows(const void* x, const uint32_t* w_q, const void* s
   a.partials = workspace ? (float*)((char*)workspace + rows::kCounterBytes) : nullptr;
   a.M = M; a.K = K; a.N = N;
   a.group_shift = group_size == 32 ? 5 : group_size == 64 ? 6 : 7;
-  a.tiles_m = p.tiles_m; a.tiles = p.tiles; a.slices = p.slices; a.stages = p.stages;
+  a.tiles_m = p.tiles_m; a.tiles = p.tiles; a.whole = p.whole; a.slices = p.slices; a.stages = p.stages;
   const bool fp16 = act_dtype == DFLASH_FP16;
   const void* fn = fp16 ? rows::kernel_for<true>(p.mt, p.nt, p.kg, mixed, silu_mul)
                         : rows::kernel_for<false>(p.mt, p.nt, p.kg, mixed, silu_mul);

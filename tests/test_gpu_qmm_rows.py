@@ -58,3 +58,20 @@ def test_gated_activation_in_the_product(native_lib, M, K, N, group, dtype):
     eps = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
     assert ((h.float() - ops).abs() <= 4 * eps * ops.abs() + eps * (gate * up).abs().float() * 1e-2 + 1e-6).all()
     assert float((h.float() != ops).float().mean()) <= 2e-2
+
+
+@pytest.mark.parametrize("M,K,N,group,dtype", [
+    (1024, 1024, 12352, 64, torch.bfloat16),   # 392 tiles of 128 x 256: one round whole, the rest in slices
+    (1000, 5120, 10000, 64, torch.bfloat16), (520, 2176, 33040, 32, torch.float16), (2048, 640, 17408, 128, torch.bfloat16)])
+def test_more_tiles_than_the_chip_takes_at_once(native_lib, M, K, N, group, dtype):
+    c = make_qmm_case(K, N, 3000 + M, group_size=group, dtype=dtype, M=M).to(DEV)
+    y = rows_matmul(c.x, c.w, c.scales, c.biases, group_size=group)
+    assert torch.equal(y, rows_matmul(c.x, c.w, c.scales, c.biases, group_size=group))
+    dense = dequantize(c.w, c.scales, c.biases, group, 4, dtype=dtype).double()
+    eps = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    for lo in range(0, N, 4096):  # (as in the test above, some columns at a time)
+        part = dense[lo:lo + 4096].t().contiguous()
+        exact, size = c.x.double() @ part, c.x.double().abs() @ part.abs()
+        got = y[:, lo:lo + 4096].double()
+        assert ((got - exact).abs() <= 1.01 * eps * exact.abs() + size * 2.0 ** -24 * K ** 0.5 + 1e-6).all()
+        assert (got - exact).norm() <= eps * exact.norm()
