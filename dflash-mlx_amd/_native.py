@@ -9,6 +9,8 @@ import ctypes
 import os
 from typing import Optional
 
+import torch
+
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libdflash_mi355.so")
 
@@ -191,11 +193,19 @@ def is_built() -> bool:
     return os.path.exists(LIB_PATH)
 
 
+def env(key: bytes) -> Optional[bytes]:
+    """Value of an environment variable as the process holds it now (``os.environ.get`` encodes the name and
+    decodes the value, 1 us a look; a launch looks at three)."""
+    try:
+        return os.environ._data.get(key)
+    except AttributeError:  # an os.environ of another make
+        value = os.environ.get(os.fsdecode(key))
+        return None if value is None else os.fsencode(value)
+
+
 def raw_stream(device) -> int:
     """Handle of the current stream of ``device`` (torch's Stream object costs microseconds per
     call to build; the handle is all the C ABI takes)."""
-    import torch
-
     index = device.index if device.index is not None else torch.cuda.current_device()
     try:
         return torch._C._cuda_getCurrentRawStream(index)

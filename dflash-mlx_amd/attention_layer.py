@@ -16,6 +16,7 @@ from typing import Any, Optional
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from . import _native
 from .cache import KVCache
@@ -24,6 +25,7 @@ from .kernels import _DTYPE_CODE, batched_sdpa_2pass_exact
 from .verify_linear import shared_input_outputs
 
 _HYBRID_SDPA_EXACT_KV_THRESHOLD = 1024
+_functorch_level, _tracing = torch._C._functorch.peek_interpreter_stack, torch._C._get_tracing_state
 
 
 def _attention_num_heads(attn: Any) -> int:
@@ -169,12 +171,14 @@ def _project(self, x: torch.Tensor, cache: Optional[Any]):
 def _plain(*tensors: torch.Tensor) -> bool:
     """Ordinary device tensors that nothing is differentiating, tracing or batching: what a kernel that takes
     their addresses may stand in for the array operators on."""
-    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+    if (forward_ad._current_level >= 0 or _functorch_level() is not None or _tracing() is not None
+            or torch.compiler.is_compiling()):
         return False
-    if any(type(t) not in (torch.Tensor, nn.Parameter) or not t.is_cuda for t in tensors):
-        return False
-    return (torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None
-            and torch._C._get_tracing_state() is None and not torch.compiler.is_compiling())
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if (type(t) is not torch.Tensor and type(t) is not nn.Parameter) or not t.is_cuda or (grad and t.requires_grad):
+            return False
+    return True
 
 
 def _unhooked(module: nn.Module) -> bool:
@@ -191,7 +195,7 @@ def _project_on_device(self, q_proj_output: torch.Tensor, keys: torch.Tensor, va
             or type(rope) is not RotaryEmbedding or not (_unhooked(q_norm) and _unhooked(k_norm) and _unhooked(rope)):
         return None
     code = _DTYPE_CODE.get(q_proj_output.dtype)
-    if code is None or code == _native.FP32 or q_proj_output.ndim != 3 or not _plain(q_proj_output, keys, values):
+    if code is None or code == _native.FP32 or q_proj_output.ndim != 3:
         return None
     B, L, width = q_proj_output.shape
     Hq, Hk = _attention_num_heads(self), _attention_num_kv_heads(self)
@@ -199,27 +203,29 @@ def _project_on_device(self, q_proj_output: torch.Tensor, keys: torch.Tensor, va
     qw, kw, device, dtype = q_norm.weight, k_norm.weight, q_proj_output.device, q_proj_output.dtype
     per = D // 64
     if (D not in (64, 128, 192, 256) or width != 2 * Hq * D or not 0 < rope.dims <= D or rope.dims % (2 * per)
-            or tuple(keys.shape) != (B, L, Hk * D) or keys.shape != values.shape or B * L == 0):
+            or keys.shape != (B, L, Hk * D) or keys.shape != values.shape or B * L == 0):
+        return None
+    held = () if cache.keys is None else (cache.keys, cache.values)
+    if not _plain(q_proj_output, keys, values, qw, kw, *held):
         return None
     if not (keys.dtype == values.dtype == dtype and keys.device == values.device == device == qw.device == kw.device
-            and tuple(qw.shape) == (D,) == tuple(kw.shape) and qw.dtype in _DTYPE_CODE and kw.dtype in _DTYPE_CODE
-            and qw.is_contiguous() and kw.is_contiguous() and _plain(qw, kw)):
+            and qw.shape == (D,) == kw.shape and qw.dtype in _DTYPE_CODE and kw.dtype in _DTYPE_CODE
+            and qw.is_contiguous() and kw.is_contiguous() and (qw.data_ptr() | kw.data_ptr()) % 8 == 0):
         return None
-    for held in (cache.keys, cache.values):
-        if held is not None and (tuple(held.shape[:2]) != (B, Hk) or held.shape[3] != D or held.dtype != dtype
-                                 or held.device != device or held.stride(3) != 1 or not _plain(held)):
+    for t in (q_proj_output, keys, values):
+        s0, s1, s2 = t.stride()
+        if s2 != 1 or (s0 | s1) % 4 or t.data_ptr() % 8:
             return None
-    if any(t.stride(2) != 1 or (t.stride(0) | t.stride(1)) % 4 or t.data_ptr() % 8 for t in (q_proj_output, keys, values)) \
-            or (qw.data_ptr() | kw.data_ptr()) % 8:
-        return None
-    for held in (cache.keys, cache.values):
-        if held is not None and (held.data_ptr() % 8 or (held.stride(0) | held.stride(1) | held.stride(2)) % 4):
+    for t in held:
+        s0, s1, s2, s3 = t.stride()
+        if (t.shape[0] != B or t.shape[1] != Hk or t.shape[3] != D or t.dtype != dtype or t.device != device or s3 != 1
+                or (s0 | s1 | s2) % 4 or t.data_ptr() % 8):
             return None
     prev = cache._append_room(B, Hk, L, D, D, keys, values)
     ko, vo = cache.keys, cache.values
     queries = torch.empty((B, Hq, L, D), dtype=dtype, device=device)
-    strides = (ctypes.c_longlong * 12)(q_proj_output.stride(0), q_proj_output.stride(1), keys.stride(0), keys.stride(1),
-                                       values.stride(0), values.stride(1), *ko.stride()[:3], *vo.stride()[:3])
+    strides = (ctypes.c_longlong * 12)(*q_proj_output.stride()[:2], *keys.stride()[:2], *values.stride()[:2],
+                                       *ko.stride()[:3], *vo.stride()[:3])
     rc = _native.lib().dflash_attn_prepare(
         q_proj_output.data_ptr(), keys.data_ptr(), values.data_ptr(), qw.data_ptr(), kw.data_ptr(), queries.data_ptr(),
         ko.data_ptr() + 2 * prev * ko.stride(2), vo.data_ptr() + 2 * prev * vo.stride(2), B, L, Hq, Hk, D, rope.dims, prev,

@@ -22,7 +22,6 @@ out_proj); its own ``forward`` is the plain, non-speculative call.
 from __future__ import annotations
 
 import ctypes
-import os
 from typing import Any, Optional, Tuple
 
 import torch
@@ -127,7 +126,7 @@ def gdn_prepare(qkv: torch.Tensor, conv_state: Optional[torch.Tensor], conv_w: t
     if conv_state is not None:
         expect["conv_state"] = (conv_state, (B, K - 1, C))
     for name, (t, shape) in expect.items():
-        if tuple(t.shape) != shape or t.device != dev:
+        if t.shape != shape or t.device != dev:
             raise ValueError(f"gdn_prepare: {name} must be {list(shape)} on {dev}, got {list(t.shape)} on {t.device}")
     if mask is not None and (mask.numel() != B * S or mask.device != dev):
         raise ValueError(f"gdn_prepare: mask must hold {B} x {S} entries on {dev}")
@@ -268,7 +267,7 @@ def _gdn_call(self, inputs: torch.Tensor, mask: Optional[torch.Tensor], cache: O
         state = torch.zeros((B, self.num_v_heads, self.head_v_dim, self.head_k_dim), dtype=q.dtype, device=q.device)
     # the layer's output norm rides on the recurrence's launch where the kernel takes it
     norm = self.norm
-    fused = (isinstance(norm, RMSNormGated) and os.environ.get("DFLASH_GDN_FUSED_NORM", "1") != "0" and
+    fused = (isinstance(norm, RMSNormGated) and _native.env(b"DFLASH_GDN_FUSED_NORM") != b"0" and
              fused_output_norm_applies(q, v, state, z, norm.weight))
     out, state, innovation_tape = gated_delta_kernel_with_tape(
         q, k, v, g, beta, state, mask, output_norm=(z, norm.weight, norm.eps) if fused else None, with_tape=record)

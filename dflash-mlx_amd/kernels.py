@@ -12,7 +12,6 @@ state [B,Hv,Dv,Dk]; mask [B,T] bool.
 """
 from __future__ import annotations
 
-import os
 from typing import Optional, Union
 
 import torch
@@ -27,7 +26,7 @@ def _require_extents(who: str, device: torch.device, **operands) -> None:
     one operand, so every other operand must have exactly the extents that follow from them, and
     live on the same device.  Anything else is an error here instead of a stray access there."""
     for name, (t, shape) in operands.items():
-        if tuple(t.shape) != tuple(shape) or t.device != device:
+        if t.shape != shape or t.device != device:
             raise ValueError(f"{who}: {name} must be {list(shape)} on {device}, got {list(t.shape)} on {t.device}")
 
 
@@ -168,7 +167,7 @@ def gated_delta_kernel_with_tape(q: torch.Tensor, k: torch.Tensor, v: torch.Tens
 
 
 def _exact_order() -> bool:
-    return os.environ.get("DFLASH_REPLAY_EXACT", "") == "1"
+    return _native.env(b"DFLASH_REPLAY_EXACT") == b"1"
 
 
 def _slot_major(t: torch.Tensor, inner: int) -> tuple:

@@ -12,12 +12,12 @@ holding elements ``8*(k>>3) .. +7`` of row n, element k in bits ``4*(k&7) .. +3`
 """
 from __future__ import annotations
 
-import os
-
 from typing import Optional, Tuple
 
 import torch
 import torch.nn as nn
+
+from . import _native
 
 _WORD_DTYPES = tuple(d for d in (torch.int32, getattr(torch, "uint32", None)) if d is not None)
 
@@ -68,7 +68,7 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
     ``DFLASH_STOCK_KERNEL=0``) with array operators."""
     if mode != "affine":
         raise NotImplementedError(f"quantisation mode {mode!r}")
-    if transpose and x.is_cuda and os.environ.get("DFLASH_STOCK_KERNEL", "1") != "0":
+    if transpose and x.is_cuda and _native.env(b"DFLASH_STOCK_KERNEL") != b"0":
         from .verify_qmm import rows_matmul
 
         y = rows_matmul(x, w, scales, biases, group_size=group_size, bits=bits)
@@ -85,7 +85,7 @@ def stock_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases:
     (``verify_qmm.small_m_matmul``) instead of dequantising the whole matrix - one-token steps
     and the narrow projections that the verify gate does not admit.  ``DFLASH_STOCK_KERNEL=0``
     keeps every such call on the array-op form."""
-    if transpose and mode == "affine" and x.is_cuda and os.environ.get("DFLASH_STOCK_KERNEL", "1") != "0":
+    if transpose and mode == "affine" and x.is_cuda and _native.env(b"DFLASH_STOCK_KERNEL") != b"0":
         from .verify_qmm import small_m_matmul
 
         y = small_m_matmul(x, w, scales, biases, group_size=group_size, bits=bits)

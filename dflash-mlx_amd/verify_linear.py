@@ -25,6 +25,7 @@ from typing import Callable, List, Optional, Sequence, Tuple
 import torch
 import torch.nn as nn
 
+from . import _native
 from .quantized import QuantizedLinear, stock_matmul
 from .verify_qmm import (ChainProblem, QmmChain, _should_use_verify, is_enabled, pack_weights, packable, rows_matmul,
                          small_m_matmul, small_m_silu_mul, verify_matmul, verify_matmul_packed)
@@ -126,10 +127,7 @@ class FusedProjections:
         verify path, on the device the joint matrix lives on, every member still a view into it
         (a module moved with ``.to()``, or replaced, has left) and behind no wrapper that would
         pad this input."""
-        m = 1
-        for d in x.shape[:-1]:
-            m *= d
-        if m != 16 or not _should_use_verify(x, self.group_size, self.bits, True):
+        if x.numel() != 16 * x.shape[-1] or not _should_use_verify(x, self.group_size, self.bits, True):
             return False
         return self._holds(parent, x)
 
@@ -137,7 +135,7 @@ class FusedProjections:
         """The same for more rows than a block has, which take the any-rows product of the joint matrix
         (``prompt``): device activations, outside the verify switch."""
         return (x.is_cuda and x.ndim >= 2 and x.numel() > 16 * int(x.shape[-1]) and self.bits == 4
-                and os.environ.get("DFLASH_STOCK_KERNEL", "1") != "0" and self._holds(parent, x))
+                and _native.env(b"DFLASH_STOCK_KERNEL") != b"0" and self._holds(parent, x))
 
     def serves_few(self, parent: nn.Module, x: torch.Tensor) -> bool:
         """The same for fewer rows than a block has (a token, a last short block), which members take through
@@ -145,18 +143,20 @@ class FusedProjections:
         so that a token meets the kernel a block meets: the joint product is that kernel, and a row of
         it does not depend on the rows beside it."""
         return (x.is_cuda and x.ndim >= 2 and 0 < x.numel() < 16 * int(x.shape[-1]) and self.bits == 4
-                and os.environ.get("DFLASH_STOCK_KERNEL", "1") != "0" and self._holds(parent, x, padded=is_enabled()))
+                and _native.env(b"DFLASH_STOCK_KERNEL") != b"0" and self._holds(parent, x, padded=is_enabled()))
 
     def _holds(self, parent: nn.Module, x: torch.Tensor, padded: bool = False) -> bool:
         if x.device != self.weight.device:
             return False
         for index, name in enumerate(self.names):
-            mod = getattr(parent, name, None)
-            if getattr(mod, "_dflash_exact_small_proj_wrapped", False):
+            # (submodules and their marks by the dictionaries they live in: getattr() looks there last)
+            mod = parent._modules.get(name)
+            if mod is not None and "_dflash_exact_small_proj_wrapped" in mod.__dict__:
                 if x.ndim == 3 and x.shape[1] < mod.pad_m and not padded:
                     return False
-                mod = mod.linear
-            if getattr(mod, "_shared_input", None) != (self, index):
+                mod = mod._modules.get("linear")
+            joined = None if mod is None else mod.__dict__.get("_shared_input")
+            if joined is None or joined[0] is not self or joined[1] != index:
                 return False
         return True
 

@@ -37,16 +37,19 @@ _KERNEL_CODE = {"auto": _native.QMM_KERNEL_AUTO, "tile": _native.QMM_KERNEL_TILE
 def _kernel_select() -> int:
     """``DFLASH_QMM_KERNEL`` in {auto, tile, stream}: which device kernel serves eligible
     calls (auto: the streaming kernel wherever it applies, the tile kernel elsewhere)."""
-    return _KERNEL_CODE.get(os.environ.get("DFLASH_QMM_KERNEL", "auto").strip().lower(),
-                            _native.QMM_KERNEL_AUTO)
+    chosen = _native.env(b"DFLASH_QMM_KERNEL")
+    if chosen is None:
+        return _native.QMM_KERNEL_AUTO
+    return _KERNEL_CODE.get(os.fsdecode(chosen).strip().lower(), _native.QMM_KERNEL_AUTO)
 
 
 def is_enabled() -> bool:
-    return os.environ.get("DFLASH_VERIFY_QMM", "") == "1"
+    return _native.env(b"DFLASH_VERIFY_QMM") == b"1"
 
 
 def _variant() -> str:
-    return os.environ.get("DFLASH_VERIFY_VARIANT", "auto")
+    chosen = _native.env(b"DFLASH_VERIFY_VARIANT")
+    return "auto" if chosen is None else os.fsdecode(chosen)
 
 
 def _auto_variant(K: int, N: int) -> Tuple[str, int]:
@@ -117,8 +120,8 @@ def _require_operands(who: str, K: int, N: int, group_size: int, w: torch.Tensor
     """The kernels read what K, N and the group size say: weights of any other extent, word size
     or device must not reach them (``lead``: leading extents, the experts of the gathered form)."""
     groups = lead + (N, K // group_size)
-    if (tuple(w.shape) != lead + (N, K // 8) or w.element_size() != 4 or tuple(scales.shape) != groups
-            or tuple(biases.shape) != groups or scales.dtype not in _DTYPE_CODE or biases.dtype != scales.dtype
+    if (w.shape != lead + (N, K // 8) or w.element_size() != 4 or scales.shape != groups
+            or biases.shape != groups or scales.dtype not in _DTYPE_CODE or biases.dtype != scales.dtype
             or not (w.device == scales.device == biases.device == device)):
         raise ValueError(f"{who}: K={K}, N={N} need w {list(lead + (N, K // 8))} of 32-bit words and bf16/fp16 scales, "
                          f"biases {list(groups)} on {device}; got {tuple(w.shape)} {w.dtype}, {tuple(scales.shape)} "
@@ -462,11 +465,9 @@ def small_m_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biase
     if (not x.is_cuda or bits != 4 or group_size not in (32, 64, 128) or x.dtype not in _DTYPE_CODE or
             scales.dtype not in _DTYPE_CODE or biases.dtype != scales.dtype or w.ndim != 2 or not _native.is_built()):
         return None
-    K, N = int(x.shape[-1]), int(w.shape[0])
-    m = 1
-    for d in x.shape[:-1]:
-        m *= int(d)
-    if m < 1 or m > 16 or N % 16 != 0 or K % group_size != 0 or K % 32 != 0 or int(w.shape[1]) * 8 != K:
+    K, N = x.shape[-1], w.shape[0]
+    m = x.numel() // K if K else 0
+    if m < 1 or m > 16 or N % 16 != 0 or K % group_size != 0 or K % 32 != 0 or w.shape[1] * 8 != K:
         return None
     w, scales, biases = w.contiguous(), scales.contiguous(), biases.contiguous()
     _require_operands("quantized_matmul", K, N, group_size, w, scales, biases, x.device)
