@@ -125,7 +125,7 @@ __global__ __launch_bounds__(256 * KG, 2) void qmm_rows_kernel(Args a) {
   const int wg = part % 8 == 0 ? (at % 8) * (part / 8) + at / 8 : at;
   const int slices = cut ? a.slices : 1, slice = wg % slices, cut_tile = wg / slices;
   const int tile = cut ? a.whole + cut_tile : wg;
-  const int st0 = (int)((long long)a.stages * slice / slices), st1 = (int)((long long)a.stages * (slice + 1) / slices);
+  const int st0 = a.stages * slice / slices, st1 = a.stages * (slice + 1) / slices;  // (at most 16 slices)
   const int nb = tile / a.tiles_m, mb = tile - nb * a.tiles_m;
   const int m0 = mb * BM, n0 = nb * BN;
   const int G = a.K >> a.group_shift;
@@ -481,35 +481,54 @@ bool covers(int M, int K, int N, int group_size, bool mixed, int epilogue) {
 // average, 12 % at worst).  A stage of 64 KG columns of K costs a fixed part (barrier, latency) and parts that go with
 // the columns (codes to dequantise), the rows (x) and their product (matrix work); a workgroup with two sets of waves
 // has a CU to itself, those with one share it in pairs.
+// The last round of more tiles than fit at once is cut with the tile left as it is: matrix work that fills the chip
+// runs against its power, so a smaller tile that fills it better gains nothing (5120 x 12352 over 1024 rows: 65 x 8
+// tiles of 192 columns, 8 of them cut, 190 us; 49 x 8 of 256, uncut, 179).  Partial tiles behind whole rounds meet the
+// memory busy, 3 TB/s for their way out and back: of 5120 x 34816, 64 of 1088 in four slices save 24 us, of
+// 5120 x 12352, 136 of 392 in three slices nothing.
 Plan make_plan(int M, int K, int N, int cus, bool mixed, bool silu_mul) {
+  auto microseconds = [cus](const Plan& p) {
+    const int slots = cus * (p.kg == 1 ? 2 : 1);
+    const double stage = 0.134 + 0.1256 * p.nt + 0.0463 * p.mt + 0.0342 * p.mt * p.nt;
+    const int whole = p.slices > 1 ? p.whole / slots : p.tiles / slots;  // rounds
+    const int parts = p.grid - whole * slots, full = parts / slots, rest = parts - full * slots;
+    // a last round with one workgroup per CU where there is room for two is the faster one
+    const double rounds = full + (rest == 0 ? 0. : p.kg == 1 && rest <= cus ? 0.62 : 1.);
+    double us = 7.55 + whole * (p.stages * stage - 2.89) + rounds * ((p.stages + p.slices - 1) / p.slices * stage - 2.89);
+    if (p.slices > 1) us += 1.48 + 0.113 * p.slices * p.mt * p.nt;
+    if (p.slices > 1 && whole > 0) us += parts * (16. * p.mt * 64 * p.nt * 8) / 3e6;
+    return us;
+  };
   Plan best{};
   double best_us = 0.;
   for (int mt = 1; mt <= 8; ++mt) {
     for (int nt = 1; nt <= 4; ++nt) {
       for (int kg = 1; kg <= 2; ++kg) {
         if (kernel_for<false>(mt, nt, kg, mixed, silu_mul) == nullptr) continue;
-        Plan p;
+        Plan p{};
         p.mt = mt, p.nt = nt, p.kg = kg;
         p.tiles_m = (M + 16 * mt - 1) / (16 * mt);
         p.tiles = p.tiles_m * ((N + 64 * nt - 1) / (64 * nt));
         p.stages = (K + kStageK * kg - 1) / (kStageK * kg);
         const int slots = cus * (kg == 1 ? 2 : 1);
-        const double stage = 0.134 + 0.1256 * nt + 0.0463 * mt + 0.0342 * mt * nt;
-        const int whole = p.tiles / slots * slots, cut = p.tiles - whole;
-        for (int slices = 1; slices <= 16 && slices <= p.stages && (slices == 1 || cut > 0); ++slices) {
-          if (slices > 1 && (cut * slices > (whole > 0 ? 2 : 1) * slots || cut > (int)(kCounterBytes / 4))) break;
-          p.slices = slices;
-          p.whole = slices > 1 ? whole : p.tiles;
-          p.grid = slices > 1 ? whole + cut * slices : p.tiles;
-          const int full = cut * slices / slots, rest = cut * slices - full * slots;
-          // a last round with one workgroup per CU where there is room for two is the faster one
-          const double rounds = full + (rest == 0 ? 0. : kg == 1 && rest <= cus ? 0.62 : 1.);
-          const double us = 7.55 + whole / slots * (p.stages * stage - 2.89) +
-                            rounds * ((p.stages + slices - 1) / slices * stage - 2.89) +
-                            (slices > 1 ? 1.48 + 0.113 * slices * mt * nt : 0.);
+        for (p.slices = 1; p.slices <= 16 && p.slices <= p.stages; ++p.slices) {
+          if (p.slices > 1 && (p.tiles * p.slices > slots || p.tiles > (int)(kCounterBytes / 4))) break;
+          p.whole = p.slices > 1 ? 0 : p.tiles;
+          p.grid = p.tiles * p.slices;
+          const double us = microseconds(p);
           if (best.grid == 0 || us < best_us) best = p, best_us = us;
         }
       }
+    }
+  }
+  const int slots = cus * (best.kg == 1 ? 2 : 1), cut = best.tiles % slots;
+  if (best.slices == 1 && best.tiles > slots && cut > 0) {
+    Plan p = best;
+    p.whole = best.tiles - cut;
+    for (p.slices = 2; p.slices <= 16 && p.slices <= p.stages && cut * p.slices <= 2 * slots; ++p.slices) {
+      p.grid = p.whole + cut * p.slices;
+      const double us = microseconds(p);
+      if (us < best_us) best = p, best_us = us;
     }
   }
   best.workspace = best.slices > 1 ? kCounterBytes + (size_t)(best.grid - best.whole) * (16 * best.mt) * (64 * best.nt) * sizeof(float) : 0;
