@@ -70,6 +70,7 @@ EXPORTED_SYMBOLS = (
     "dflash_attn_gate",
     "dflash_sdpa_q16_workspace_bytes",
     "dflash_sdpa_q16",
+    "dflash_sdpa_q16_gated",
     "dflash_conv_state_rebuild",
     "dflash_rollback_layer",
 )
@@ -155,6 +156,9 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.dflash_sdpa_q16.restype = c.c_int
     lib.dflash_sdpa_q16.argtypes = ([c.c_void_p] * 6 + [c.c_size_t] + [c.c_int] * 5 + [c.c_longlong] * 6 +
                                     [c.c_float, c.c_int, c.c_void_p])
+    lib.dflash_sdpa_q16_gated.restype = c.c_int
+    lib.dflash_sdpa_q16_gated.argtypes = ([c.c_void_p] * 7 + [c.c_size_t] + [c.c_int] * 5 + [c.c_longlong] * 8 +
+                                          [c.c_float, c.c_int, c.c_void_p])
     lib.dflash_tape_replay.restype = c.c_int
     lib.dflash_tape_replay.argtypes = (
         [c.c_void_p] * 6 + [c.c_int] + [c.c_void_p] + [c.c_int] * 12 + [c.c_void_p]

@@ -237,7 +237,7 @@ def _project_on_device(self, q_proj_output: torch.Tensor, keys: torch.Tensor, va
 
 
 def _finish(self, output: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
-    """``gate`` [B, L, Hq * D], or the whole output of q_proj, [B, L, Hq * 2 D], as ``_project_on_device`` leaves it."""
+    """Gate and output projection.  ``gate`` [B, L, Hq * D], or the whole output of q_proj, [B, L, Hq * 2 D], as ``_project_on_device`` leaves it."""
     B, H, L, D = output.shape
     if gate.shape[-1] == 2 * H * D:
         if (output.dtype == gate.dtype and _plain(output) and output.stride(3) == 1 and output.data_ptr() % 8 == 0
@@ -277,8 +277,11 @@ def _install_split_full_attention_hook(attn: Any) -> None:
                                     int(queries.shape[-1]) in (128, 256) and int(values.shape[-1]) in (128, 256))
         output = None
         if should_use_batched_2pass:
+            in_one = gate.shape[-1] == 2 * queries.shape[1] * queries.shape[3]  # as _project_on_device leaves it
             output = batched_sdpa_2pass_exact(queries=queries, keys=keys, values=values, scale=self.scale,
-                                              mask=mask if is_array else None)
+                                              mask=mask if is_array else None, q_proj_output=gate if in_one else None)
+            if output is not None and output.ndim == 3:
+                return self.o_proj(output)  # gated
         if output is None and should_split:
             output = _split_sdpa_output(queries=queries, keys=keys, values=values, scale=self.scale, mask=mask,
                                         chunk_size=1, cached_prefix_len=cached_prefix_len)

@@ -9,7 +9,8 @@
 // What bounds it is neither bandwidth (a block of 16 tokens is about 1 MB) nor arithmetic: as array operators the
 // same steps were 70 launches, 2 to 5 us each on the device and about 400 us of host time per layer call.
 // Measured, 16 tokens of 32 + 8 heads of 256: layer call over 4 112 or 32 716 keys
-// 498 -> 109 us (host time: the kernels are 62 and 102 us); this kernel 6.8 us, the gate 4 us.
+// 498 -> 109 us (host time: the kernels are 62 and 102 us); this kernel 6.8 us, the gate 4 us (a verify block over a
+// long cache has it in the merge of sdpa_q16.hip instead).
 #include "glue_device.h"
 
 #include <cmath>

@@ -54,7 +54,9 @@ struct SdpaArgs {
   const uint16_t* k;     // [B, Hk, N, D] through strides (elements), D contiguous
   const uint16_t* v;
   const uint16_t* mask;  // [B, Hq, 16, N] additive, in the input dtype, or null
-  uint16_t* out;         // [B, Hq, 16, D]
+  uint16_t* out;         // [B, Hq, 16, D], gated: [B, 16, Hq, D]
+  const uint16_t* gate;  // [B, 16, Hq, 2 D] with these strides (elements), the gate behind the queries of a head; or null
+  long long gate_batch_stride, gate_row_stride;
   uint16_t* part_o;      // [splits, B * Hq, 16, D] in the input dtype, as the reference keeps them
   float* part_ml;        // [splits, B * Hq, 16, 2]  (max, sum)
   long long k_batch_stride, k_head_stride, k_seq_stride;
@@ -302,6 +304,11 @@ __global__ __launch_bounds__(256) void sdpa_q16_merge_kernel(SdpaArgs a, int D) 
     }
   };
   issue_round(g);
+  // (b, hq, i) of the row; the gate is asked for with the partial results
+  const int i = (int)(row % 16), hq = (int)(row / 16 % a.Hq), b = (int)(row / (16 * (size_t)a.Hq));
+  uint2 gate = uint2{0u, 0u};
+  if (a.gate != nullptr && g == 0 && col)
+    gate = *reinterpret_cast<const uint2*>(a.gate + b * a.gate_batch_stride + i * a.gate_row_stride + (size_t)hq * 2 * D + D + 4 * c4);
   if (tid < 64) {
     f32x2_t ml[kMaxSplits / 64];
 #pragma unroll
@@ -348,8 +355,22 @@ __global__ __launch_bounds__(256) void sdpa_q16_merge_kernel(SdpaArgs a, int D) 
   if (g == 0 && col) {
     o = acc[0][c4] + acc[1][c4] + acc[2][c4] + acc[3][c4];
     const float inv = total > 0.f ? 1.f / total : 1.f;
-    const uint2 packed = {pack2<FP16>(o[0] * inv, o[1] * inv), pack2<FP16>(o[2] * inv, o[3] * inv)};
-    *reinterpret_cast<uint2*>(a.out + row * D + 4 * c4) = packed;
+    uint2 packed = {pack2<FP16>(o[0] * inv, o[1] * inv), pack2<FP16>(o[2] * inv, o[3] * inv)};
+    size_t to = row;
+    if (a.gate != nullptr) {
+      // output * sigmoid(gate) as the array operators give it: output, sigmoid and product each of the array's type
+      const uint32_t gw[4] = {gate.x & 0xFFFFu, gate.x >> 16, gate.y & 0xFFFFu, gate.y >> 16};
+      const uint32_t ow[4] = {packed.x & 0xFFFFu, packed.x >> 16, packed.y & 0xFFFFu, packed.y >> 16};
+      float y[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float sig = 1.0f / (1.0f + expf(-elem_to_f32<FP16>((uint16_t)gw[e])));
+        y[e] = elem_to_f32<FP16>((uint16_t)ow[e]) * elem_to_f32<FP16>((uint16_t)pack2<FP16>(sig, 0.f));
+      }
+      packed = uint2{pack2<FP16>(y[0], y[1]), pack2<FP16>(y[2], y[3])};
+      to = ((size_t)b * 16 + i) * a.Hq + hq;
+    }
+    *reinterpret_cast<uint2*>(a.out + to * D + 4 * c4) = packed;
   }
 }
 
@@ -381,12 +402,13 @@ extern "C" size_t dflash_sdpa_q16_workspace_bytes(int B, int Hq, int Hk, int N, 
   return (size_t)splits * B * Hq * 16 * (D * sizeof(uint16_t) + 2 * sizeof(float));
 }
 
-extern "C" int dflash_sdpa_q16(const void* q, const void* k, const void* v, const void* mask, void* out,
-                               void* workspace, size_t workspace_bytes, int B, int Hq, int Hk, int N, int D,
-                               long long k_batch_stride, long long k_head_stride, long long k_seq_stride,
-                               long long v_batch_stride, long long v_head_stride, long long v_seq_stride,
-                               float scale, int dtype, void* stream) {
-  using namespace dflash;
+namespace dflash {
+namespace {
+int sdpa_launch(const void* q, const void* k, const void* v, const void* mask, const void* gate, void* out,
+                void* workspace, size_t workspace_bytes, int B, int Hq, int Hk, int N, int D,
+                long long k_batch_stride, long long k_head_stride, long long k_seq_stride,
+                long long v_batch_stride, long long v_head_stride, long long v_seq_stride,
+                long long gate_batch_stride, long long gate_row_stride, float scale, int dtype, void* stream) {
   DFLASH_REQUIRE(q && k && v && out, DFLASH_ERR_ARG, "dflash_sdpa_q16: null operand");
   DFLASH_REQUIRE(dtype == DFLASH_BF16 || dtype == DFLASH_FP16, DFLASH_ERR_ARG,
                  "dflash_sdpa_q16: bf16 or fp16 only");
@@ -412,6 +434,9 @@ extern "C" int dflash_sdpa_q16(const void* q, const void* k, const void* v, cons
   a.splits = pick_splits(B, Hk, N, &a.keys_per_split);
   a.scale = scale;
   a.lowest = dtype == DFLASH_FP16 ? -65504.0f : -3.3895313892515355e38f;
+  a.gate = (const uint16_t*)gate;
+  a.gate_batch_stride = gate_batch_stride; a.gate_row_stride = gate_row_stride;
+  DFLASH_REQUIRE(!gate || a.splits > 1, DFLASH_ERR_SHAPE, "dflash_sdpa_q16_gated: the gate rides on the merge of key ranges");
   a.part_o = nullptr;
   a.part_ml = nullptr;
   if (a.splits > 1) {
@@ -461,4 +486,33 @@ extern "C" int dflash_sdpa_q16(const void* q, const void* k, const void* v, cons
     DFLASH_HIP_OK(hipGetLastError());
   }
   return DFLASH_OK;
+}
+}  // namespace
+}  // namespace dflash
+
+extern "C" int dflash_sdpa_q16(const void* q, const void* k, const void* v, const void* mask, void* out,
+                               void* workspace, size_t workspace_bytes, int B, int Hq, int Hk, int N, int D,
+                               long long k_batch_stride, long long k_head_stride, long long k_seq_stride,
+                               long long v_batch_stride, long long v_head_stride, long long v_seq_stride,
+                               float scale, int dtype, void* stream) {
+  return dflash::sdpa_launch(q, k, v, mask, nullptr, out, workspace, workspace_bytes, B, Hq, Hk, N, D, k_batch_stride,
+                             k_head_stride, k_seq_stride, v_batch_stride, v_head_stride, v_seq_stride, 0, 0, scale, dtype, stream);
+}
+
+// A launch of its own for the gate (dflash_attn_gate) cost 4 us on the device and 10 us of host time behind an attention
+// of 15 us (4 112 keys): layer call 92 -> 86 us, over 32 716 keys 99 -> 96 us.
+extern "C" int dflash_sdpa_q16_gated(const void* q, const void* k, const void* v, const void* mask, const void* gate,
+                                     void* out, void* workspace, size_t workspace_bytes, int B, int Hq, int Hk, int N,
+                                     int D, long long k_batch_stride, long long k_head_stride, long long k_seq_stride,
+                                     long long v_batch_stride, long long v_head_stride, long long v_seq_stride,
+                                     long long gate_batch_stride, long long gate_row_stride, float scale, int dtype,
+                                     void* stream) {
+  using namespace dflash;
+  DFLASH_REQUIRE(gate, DFLASH_ERR_ARG, "dflash_sdpa_q16_gated: null gate");
+  DFLASH_REQUIRE(gate_batch_stride >= 0 && gate_row_stride >= 0 &&
+                     (((uintptr_t)gate | (uintptr_t)(gate_batch_stride * 2) | (uintptr_t)(gate_row_stride * 2)) % 8) == 0,
+                 DFLASH_ERR_ARG, "dflash_sdpa_q16_gated: rows of the gate must be 8-byte aligned");
+  return sdpa_launch(q, k, v, mask, gate, out, workspace, workspace_bytes, B, Hq, Hk, N, D, k_batch_stride, k_head_stride,
+                     k_seq_stride, v_batch_stride, v_head_stride, v_seq_stride, gate_batch_stride, gate_row_stride, scale, dtype,
+                     stream);
 }

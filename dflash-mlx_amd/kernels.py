@@ -352,14 +352,19 @@ def _sdpa_workspace(device: torch.device, nbytes: int) -> torch.Tensor:
 
 
 def batched_sdpa_2pass_exact(queries: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, scale: float,
-                             mask: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+                             mask: Optional[torch.Tensor] = None, *,
+                             q_proj_output: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """Exact attention of a 16-token verify block over a long KV cache (mirror of
     dflash_mlx/kernels.py:658-761): queries [B,Hq,16,D], keys / values [B,Hk,N,D] (views of a
     cache are read in place), mask None, bool or additive, broadcastable to [B,Hq,16,N].
     Query i attends to keys n <= N - 16 + i.  Returns None - the caller then takes its
     general attention - for everything the kernel does not cover, as the reference does:
     host tensors, q_len != 16, dtypes other than bf16 / fp16, head dims other than 128 / 256,
-    more than 8 query heads per key/value head."""
+    more than 8 query heads per key/value head.
+
+    ``q_proj_output`` [B,16,Hq*2D] (no counterpart in the reference, which gates with array operators): the result is
+    [B,16,Hq*D], every head times the sigmoid of the second half of its part of q_proj_output, where the same launch can do
+    it; where it cannot (one range of keys), the plain result."""
     if queries.ndim != 4 or keys.ndim != 4 or values.ndim != 4 or not queries.is_cuda:
         return None
     bsz, hq, q_len, d = (int(x) for x in queries.shape)
@@ -392,9 +397,21 @@ def batched_sdpa_2pass_exact(queries: torch.Tensor, keys: torch.Tensor, values: 
         mask_tensor = torch.broadcast_to(mask_tensor.to(queries.device), (bsz, hq, q_len, n_kv)).contiguous()
 
     lib = _native.lib()
-    out = torch.empty_like(queries)
     need = int(lib.dflash_sdpa_q16_workspace_bytes(bsz, hq, hk, n_kv, d))
     ws = _sdpa_workspace(queries.device, need) if need else None
+    gate = q_proj_output
+    if gate is not None and need and gate.shape == (bsz, q_len, hq * 2 * d) and gate.dtype == queries.dtype \
+            and gate.device == queries.device and gate.stride(2) == 1 and (gate.stride(0) | gate.stride(1)) % 4 == 0 \
+            and gate.data_ptr() % 8 == 0:
+        out = torch.empty((bsz, q_len, hq * d), dtype=queries.dtype, device=queries.device)
+        rc = lib.dflash_sdpa_q16_gated(
+            queries.data_ptr(), keys.data_ptr(), values.data_ptr(),
+            None if mask_tensor is None else mask_tensor.data_ptr(), gate.data_ptr(), out.data_ptr(), ws.data_ptr(),
+            ws.numel(), bsz, hq, hk, n_kv, d, *keys.stride()[:3], *values.stride()[:3], gate.stride(0), gate.stride(1),
+            float(scale), _DTYPE_CODE[queries.dtype], _native.raw_stream(queries.device))
+        _native.check(rc, "dflash_sdpa_q16_gated")
+        return out
+    out = torch.empty_like(queries)
     rc = lib.dflash_sdpa_q16(
         queries.data_ptr(), keys.data_ptr(), values.data_ptr(),
         None if mask_tensor is None else mask_tensor.data_ptr(), out.data_ptr(),

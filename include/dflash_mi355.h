@@ -494,6 +494,18 @@ int dflash_sdpa_q16(const void* q, const void* k, const void* v, const void* mas
                     float scale, int dtype, void* stream);
 
 /*
+ * The same with the layer's output gate applied where the key ranges meet (only where the workspace size is not 0):
+ * out [B, 16, Hq, D] = attention * sigmoid(gate), attention, sigmoid and product each rounded to `dtype`.
+ *   gate  the q_proj output [B, 16, Hq, 2 D] (a head's queries, then its gate), batches and rows with strides in elements,
+ *         rows 8-byte aligned
+ */
+int dflash_sdpa_q16_gated(const void* q, const void* k, const void* v, const void* mask, const void* gate, void* out,
+                          void* workspace, size_t workspace_bytes, int B, int Hq, int Hk, int N, int D,
+                          long long k_batch_stride, long long k_head_stride, long long k_seq_stride,
+                          long long v_batch_stride, long long v_head_stride, long long v_seq_stride,
+                          long long gate_batch_stride, long long gate_row_stride, float scale, int dtype, void* stream);
+
+/*
  * Conv-window rebuild of a GatedDeltaNet layer after a partial acceptance: output
  * row j of a slot is row steps+j of concat([conv_prev, qkv], axis=rows).  Replaces the
  * array ops of dflash_mlx/recurrent_rollback_cache.py:129-146 (zeros stand in for a

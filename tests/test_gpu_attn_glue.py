@@ -102,3 +102,23 @@ def test_what_the_kernel_does_not_cover_goes_to_the_array_operators():
         queries, keys, _, gate, _ = A._project(attn, x, cache)
         assert gate.shape[-1] == queries.shape[1] * queries.shape[-1], change
         assert queries.requires_grad == (change == "grad")
+
+
+@pytest.mark.parametrize("B,Hq,Hk,D,N,dtype,masked,joint", [
+    (1, 32, 8, 256, 4112, torch.bfloat16, False, True), (2, 16, 2, 128, 257, torch.float16, False, False),
+    (1, 24, 4, 256, 1040, torch.bfloat16, True, True), (3, 5, 1, 128, 300, torch.bfloat16, False, True)])
+def test_gate_behind_the_attention(B, Hq, Hk, D, N, dtype, masked, joint):
+    """The gate where the key ranges meet: the bits of the attention followed by the gate of its own."""
+    from dflash_mlx_amd.kernels import batched_sdpa_2pass_exact
+
+    gen = torch.Generator(device="cuda").manual_seed(13)
+    attn, outs = _layer(B, 16, Hq, Hk, D, D, dtype, dtype, gen, joint)
+    q = torch.randn((B, Hq, 16, D), generator=gen, device="cuda").to(dtype)
+    k, v = (torch.randn((B, Hk, N, D), generator=gen, device="cuda").to(dtype) for _ in range(2))
+    mask = torch.randn((B, 1, 16, N), generator=gen, device="cuda").to(dtype) if masked else None
+    plain = batched_sdpa_2pass_exact(q, k, v, D ** -0.5, mask)
+    gated = batched_sdpa_2pass_exact(q, k, v, D ** -0.5, mask, q_proj_output=outs[0])
+    assert gated.shape == (B, 16, Hq * D) and torch.equal(gated, A._finish(attn, plain, outs[0]))
+    # one range of keys: nothing to ride on, the plain result
+    short = batched_sdpa_2pass_exact(q, k[:, :, :100], v[:, :, :100], D ** -0.5, q_proj_output=outs[0])
+    assert torch.equal(short, batched_sdpa_2pass_exact(q, k[:, :, :100], v[:, :, :100], D ** -0.5))
