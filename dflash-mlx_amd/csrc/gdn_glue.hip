@@ -13,7 +13,7 @@
 // instructions per element (the sigmoid's exponential and division, the roundings): a wave takes several tokens
 // of its head in turn, so that a row of qkv is read and unpacked once and not once per tap, the taps once per wave, and
 // the gates of all its tokens are computed side by side, one token per lane.  1024 tokens of 16 + 16 + 32 heads of
-// 128: 62 us with a wave per token and head, 28.6 us; the gated norm 15 -> 13.6 us.  The projections are read where a joint product
+// 128: 62 us with a wave per token and head, now 20.3 us; the gated norm 15 -> 10.1 us.  The projections are read where a joint product
 // left them (rows with a stride), which saves four copies per layer call (25 us of the same prompt, 12 us of a
 // verify block).
 #include "glue_device.h"
@@ -25,6 +25,28 @@ namespace {
 
 constexpr int kWavesPerGroup = 4;
 constexpr int kMaxPerLane = 4;  // head dims up to 256
+
+// Sum of the squares of a head: PER elements in each of LANES lanes (a power of two).  Adjacent elements first and in
+// sixty-fourths of the head whatever LANES is, so that a row has the same sum in the wide and the narrow kernels.
+template <int PER, int LANES>
+__device__ __forceinline__ float sum_of_squares(const float (&v)[PER]) {
+  constexpr int kEach = PER * LANES / 64, kParts = PER / kEach;
+  float part[kParts];
+#pragma unroll
+  for (int i = 0; i < kParts; ++i) {
+    part[i] = 0.f;
+#pragma unroll
+    for (int e = 0; e < kEach; ++e) part[i] += v[i * kEach + e] * v[i * kEach + e];
+  }
+#pragma unroll
+  for (int n = kParts / 2; n >= 1; n /= 2)
+#pragma unroll
+    for (int i = 0; i < n; ++i) part[i] = part[2 * i] + part[2 * i + 1];
+  float sum = part[0];
+#pragma unroll
+  for (int off = 1; off < LANES; off <<= 1) sum += __shfl_xor(sum, off, 64);
+  return sum;
+}
 
 struct PrepareArgs {
   const void* qkv;         // [B, S, C], rows and batches with a stride
@@ -48,18 +70,17 @@ struct PrepareArgs {
   float eps, scale_q, scale_k;  // scales already rounded to the array dtype
 };
 
-// One wave per (batch, run of tokens, head); heads 0..Hk-1 are q, Hk..2Hk-1 are k, the rest v.  A lane
-// holds PER = D / 64 adjacent channels of its head, so a row of the head is one access per lane
+// LANES lanes per (batch, run of tokens, head); heads 0..Hk-1 are q, Hk..2Hk-1 are k, the rest v, those of a wave of
+// one kind.  A lane holds PER = D / LANES adjacent channels of its head, so a row of the head is one access per lane
 // and the K taps of those channels are PER * K adjacent weights.  All loads the first token needs are issued
 // before anything is computed, the next token's row while the present one is worked on.
-template <int DT, int PER, int K>
-__device__ __forceinline__ void prepare_head(const PrepareArgs& p, int b, int s0, int s1, int h, int lane) {
+template <int DT, int PER, int K, int LANES>
+__device__ __forceinline__ void prepare_head(const PrepareArgs& p, int b, int s0, int s1, bool is_v, int h, int lane) {
   const int key_dim = p.Hk * p.Dk;
   const int C = 2 * key_dim + p.Hv * p.Dv;
   constexpr int keep = K - 1;
   constexpr bool wide = DT == DFLASH_FP32;
-  const bool is_v = h >= 2 * p.Hk;
-  const int D = PER * 64;
+  const int D = PER * LANES;
   const int cb = is_v ? 2 * key_dim + (h - 2 * p.Hk) * p.Dv : h * p.Dk;  // q and k heads are contiguous
   const int c = cb + PER * lane;
   const int hv = is_v ? h - 2 * p.Hk : 0;
@@ -137,14 +158,12 @@ __device__ __forceinline__ void prepare_head(const PrepareArgs& p, int b, int s0
     if (p.qkv_out != nullptr) store_adjacent<PER>(p.qkv_out, (token0 + s) * C + c, DT, x[keep]);
 
     float act[PER];
-    float ss = 0.f;
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
       float acc = 0.f;
 #pragma unroll
       for (int j = 0; j < K; ++j) acc += x[j][e] * w[e * K + j];
       act[e] = silu_rounded(round_through(acc, DT), DT);
-      ss += act[e] * act[e];
     }
 #pragma unroll
     for (int j = 0; j < keep; ++j)
@@ -155,7 +174,7 @@ __device__ __forceinline__ void prepare_head(const PrepareArgs& p, int b, int s0
       store_adjacent<PER>(p.v, ((token0 + s) * p.Hv + hv) * p.Dv + PER * lane, DT, act);
       continue;
     }
-    const float inv_rms = 1.0f / sqrtf(wave_sum(ss) / (float)D + p.eps);
+    const float inv_rms = 1.0f / sqrtf(sum_of_squares<PER, LANES>(act) / (float)D + p.eps);
     const bool is_q = h < p.Hk;
     const float scale = is_q ? p.scale_q : p.scale_k;
     void* out = is_q ? p.q : p.k;
@@ -176,18 +195,43 @@ __global__ __launch_bounds__(kWavesPerGroup * 64) void gdn_prepare_kernel(Prepar
   const int h = w % heads, run = w / heads;
   const int b = run / runs, s0 = (run - b * runs) * p.tokens;
   const int s1 = s0 + p.tokens < p.S ? s0 + p.tokens : p.S;
-  switch ((h >= 2 * p.Hk ? p.Dv : p.Dk) / 64) {
-    case 1: prepare_head<DT, 1, K>(p, b, s0, s1, h, lane); break;
-    case 2: prepare_head<DT, 2, K>(p, b, s0, s1, h, lane); break;
-    case 3: prepare_head<DT, 3, K>(p, b, s0, s1, h, lane); break;
-    default: prepare_head<DT, 4, K>(p, b, s0, s1, h, lane); break;
+  const bool is_v = h >= 2 * p.Hk;
+  switch ((is_v ? p.Dv : p.Dk) / 64) {
+    case 1: prepare_head<DT, 1, K, 64>(p, b, s0, s1, is_v, h, lane); break;
+    case 2: prepare_head<DT, 2, K, 64>(p, b, s0, s1, is_v, h, lane); break;
+    case 3: prepare_head<DT, 3, K, 64>(p, b, s0, s1, is_v, h, lane); break;
+    default: prepare_head<DT, 4, K, 64>(p, b, s0, s1, is_v, h, lane); break;
   }
+}
+// Eight channels per lane, several heads per wave: Dk = Dv = 64, 128 or 256, the heads of either kind a multiple of those
+// of a wave, 16-bit arrays.
+template <int DT, int K, int LANES>
+__global__ __launch_bounds__(kWavesPerGroup * 64) void gdn_prepare_wide_kernel(PrepareArgs p) {
+  constexpr int kHeads = 64 / LANES;
+  const int lane = threadIdx.x & 63;
+  const int groups = (2 * p.Hk + p.Hv) / kHeads, runs = (p.S + p.tokens - 1) / p.tokens;
+  const int w = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * kWavesPerGroup + (threadIdx.x >> 6)));
+  if (w >= p.B * runs * groups) return;
+  const int h0 = w % groups * kHeads, run = w / groups;
+  const int b = run / runs, s0 = (run - b * runs) * p.tokens;
+  const int s1 = s0 + p.tokens < p.S ? s0 + p.tokens : p.S;
+  prepare_head<DT, 8, K, LANES>(p, b, s0, s1, h0 >= 2 * p.Hk, h0 + lane / LANES, lane % LANES);
 }
 template <int DT>
 const void* prepare_kernel_for(int conv_kernel) {
   return conv_kernel == 4   ? (const void*)gdn_prepare_kernel<DT, 4>
          : conv_kernel == 3 ? (const void*)gdn_prepare_kernel<DT, 3>
                             : (const void*)gdn_prepare_kernel<DT, 2>;
+}
+template <int DT, int K>
+const void* wide_kernel_for(int D) {
+  return D == 64    ? (const void*)gdn_prepare_wide_kernel<DT, K, 8>
+         : D == 128 ? (const void*)gdn_prepare_wide_kernel<DT, K, 16>
+                    : (const void*)gdn_prepare_wide_kernel<DT, K, 32>;
+}
+template <int DT>
+const void* wide_kernel_for(int D, int conv_kernel) {
+  return conv_kernel == 4 ? wide_kernel_for<DT, 4>(D) : conv_kernel == 3 ? wide_kernel_for<DT, 3>(D) : wide_kernel_for<DT, 2>(D);
 }
 
 struct NormArgs {
@@ -202,9 +246,9 @@ struct NormArgs {
   float eps;
 };
 
-// One wave for a few rows: rms_norm(x, weight) * silu(z); a lane holds PER = D / 64 adjacent elements.
-template <int DT, int PER>
-__device__ __forceinline__ void gated_norm_rows(const NormArgs& p, int row, int end, int lane) {
+// LANES lanes for a few rows, `step` apart: rms_norm(x, weight) * silu(z); a lane holds PER = D / LANES adjacent elements.
+template <int DT, int PER, int LANES>
+__device__ __forceinline__ void gated_norm_rows(const NormArgs& p, int row, int end, int step, int lane) {
   constexpr bool wide = DT == DFLASH_FP32;
   uint32_t xr[PER], zr[PER], wr[PER];
   auto load = [&](int r) __attribute__((always_inline)) {
@@ -212,21 +256,18 @@ __device__ __forceinline__ void gated_norm_rows(const NormArgs& p, int row, int 
     load_adjacent_raw<PER>(p.x, (size_t)r * p.D + PER * lane, wide, xr);
     load_adjacent_raw<PER>(p.z, (size_t)b * p.z_batch + (size_t)t * p.z_row + (size_t)h * p.D + PER * lane, wide, zr);
   };
-  load(row);
+  load(row < end ? row : end - 1);
   load_adjacent_raw<PER>(p.weight, PER * lane, p.weight_dt == DFLASH_FP32, wr);
   asm volatile("" ::: "memory");  // all three requests are out before the first value is interpreted
   float wt[PER];
   unpack_adjacent<PER>(wr, p.weight_dt, wt);
 #pragma unroll 1
-  for (; row < end; ++row) {
+  for (; row < end; row += step) {
     float x[PER], z[PER];
     unpack_adjacent<PER>(xr, DT, x);
     unpack_adjacent<PER>(zr, DT, z);
-    if (row + 1 < end) load(row + 1);
-    float ss = 0.f;
-#pragma unroll
-    for (int e = 0; e < PER; ++e) ss += x[e] * x[e];
-    const float inv_rms = 1.0f / sqrtf(wave_sum(ss) / (float)p.D + p.eps);
+    if (row + step < end) load(row + step);
+    const float inv_rms = 1.0f / sqrtf(sum_of_squares<PER, LANES>(x) / (float)(PER * LANES) + p.eps);
     float y[PER];
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
@@ -245,11 +286,28 @@ __global__ __launch_bounds__(kWavesPerGroup * 64) void gdn_gated_norm_kernel(Nor
   if (first >= p.rows) return;
   const int row = (int)first, end = p.rows - row < p.per_wave ? p.rows : row + p.per_wave;
   switch (p.D / 64) {
-    case 1: gated_norm_rows<DT, 1>(p, row, end, lane); break;
-    case 2: gated_norm_rows<DT, 2>(p, row, end, lane); break;
-    case 3: gated_norm_rows<DT, 3>(p, row, end, lane); break;
-    default: gated_norm_rows<DT, 4>(p, row, end, lane); break;
+    case 1: gated_norm_rows<DT, 1, 64>(p, row, end, 1, lane); break;
+    case 2: gated_norm_rows<DT, 2, 64>(p, row, end, 1, lane); break;
+    case 3: gated_norm_rows<DT, 3, 64>(p, row, end, 1, lane); break;
+    default: gated_norm_rows<DT, 4, 64>(p, row, end, 1, lane); break;
   }
+}
+
+template <int DT, int LANES>
+__global__ __launch_bounds__(kWavesPerGroup * 64) void gdn_gated_norm_wide_kernel(NormArgs p) {
+  constexpr int kRows = 64 / LANES;
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * kWavesPerGroup + (threadIdx.x >> 6)));
+  const long long first = (long long)w * p.per_wave;
+  if (first >= p.rows) return;
+  const int row = (int)first, end = p.rows - row < p.per_wave ? p.rows : row + p.per_wave;
+  gated_norm_rows<DT, 8, LANES>(p, row + lane / LANES, end, kRows, lane % LANES);
+}
+template <int DT>
+const void* wide_norm_for(int D) {
+  return D == 64    ? (const void*)gdn_gated_norm_wide_kernel<DT, 8>
+         : D == 128 ? (const void*)gdn_gated_norm_wide_kernel<DT, 16>
+                    : (const void*)gdn_gated_norm_wide_kernel<DT, 32>;
 }
 
 bool known_dtype(int dt) { return dt == DFLASH_BF16 || dt == DFLASH_FP16 || dt == DFLASH_FP32; }
@@ -306,9 +364,20 @@ extern "C" int dflash_gdn_prepare_rows(const void* qkv, const void* conv_state, 
   // as many tokens per wave as leave 8 waves per SIMD: below that a wave's latency counts, not its instructions
   const long long per = (long long)B * S * heads / 8192;
   p.tokens = per < 1 ? 1 : per > 16 ? 16 : (int)per;
-  const long long waves = (long long)B * ((S + p.tokens - 1) / p.tokens) * heads;
+  // Eight channels per lane once that leaves 4 waves per SIMD: the sums, roots and addresses of a row are then paid for
+  // four heads of 128 at a time, 1024 tokens 23.3 -> 20.3 us.
+  const int per_wave = 512 / Dk;  // heads
+  const bool wide = dtype != DFLASH_FP32 && Dk == Dv && Dk != 192 && Hk % per_wave == 0 && Hv % per_wave == 0 &&
+                    (long long)B * S * heads / per_wave >= 4096;
+  if (wide) {
+    const long long each = (long long)B * S * heads / per_wave / 4096, most = Dk / 8 < 16 ? Dk / 8 : 16;
+    p.tokens = (int)(each > most ? most : each);  // (a lane of the head computes a token's gates)
+  }
+  const long long waves = (long long)B * ((S + p.tokens - 1) / p.tokens) * (wide ? heads / per_wave : heads);
   const unsigned groups = (unsigned)((waves + kWavesPerGroup - 1) / kWavesPerGroup);
-  const void* fn = dtype == DFLASH_BF16   ? prepare_kernel_for<DFLASH_BF16>(conv_kernel)
+  const void* fn = wide ? (dtype == DFLASH_BF16 ? wide_kernel_for<DFLASH_BF16>(Dk, conv_kernel)
+                                                : wide_kernel_for<DFLASH_FP16>(Dk, conv_kernel))
+                   : dtype == DFLASH_BF16 ? prepare_kernel_for<DFLASH_BF16>(conv_kernel)
                    : dtype == DFLASH_FP16 ? prepare_kernel_for<DFLASH_FP16>(conv_kernel)
                                           : prepare_kernel_for<DFLASH_FP32>(conv_kernel);
   void* args[] = {&p};
@@ -337,9 +406,16 @@ int gdn_gated_norm_launch(const void* x, const void* z, const void* weight, void
   p.rows = B * T * H; p.T = T; p.H = H; p.D = D;
   p.weight_dt = weight_dtype; p.eps = eps;
   p.per_wave = p.rows / 8192 < 1 ? 1 : p.rows / 8192 > 16 ? 16 : p.rows / 8192;
+  // eight elements per lane and several rows per wave where that leaves 4 waves per SIMD: 12.3 -> 10.1 us (32 768 rows of 128)
+  const bool wide = dtype != DFLASH_FP32 && D != 192 && p.rows / (512 / D) >= 4096;
+  if (wide) {
+    const int passes = p.rows / (512 / D) / 4096;
+    p.per_wave = 512 / D * (passes > 8 ? 8 : passes);
+  }
   const long long waves = ((long long)p.rows + p.per_wave - 1) / p.per_wave;
   const unsigned groups = (unsigned)((waves + kWavesPerGroup - 1) / kWavesPerGroup);
-  const void* fn = dtype == DFLASH_BF16   ? (const void*)gdn_gated_norm_kernel<DFLASH_BF16>
+  const void* fn = wide ? (dtype == DFLASH_BF16 ? wide_norm_for<DFLASH_BF16>(D) : wide_norm_for<DFLASH_FP16>(D))
+                   : dtype == DFLASH_BF16 ? (const void*)gdn_gated_norm_kernel<DFLASH_BF16>
                    : dtype == DFLASH_FP16 ? (const void*)gdn_gated_norm_kernel<DFLASH_FP16>
                                           : (const void*)gdn_gated_norm_kernel<DFLASH_FP32>;
   void* args[] = {&p};
