@@ -206,6 +206,11 @@ def _project_on_device(self, q_proj_output: torch.Tensor, keys: torch.Tensor, va
             or keys.shape != (B, L, Hk * D) or keys.shape != values.shape or B * L == 0):
         return None
     held = () if cache.keys is None else (cache.keys, cache.values)
+    # the kernel writes rows offset .. offset + L - 1 of both buffers: an offset outside them, or buffers of two
+    # lengths, are left to the array operators, which refuse them
+    capacity = cache.keys.shape[2] if held and cache.keys.ndim == 4 else 0
+    if not 0 <= cache.offset <= capacity:
+        return None
     if not _plain(q_proj_output, keys, values, qw, kw, *held):
         return None
     if not (keys.dtype == values.dtype == dtype and keys.device == values.device == device == qw.device == kw.device
@@ -217,6 +222,8 @@ def _project_on_device(self, q_proj_output: torch.Tensor, keys: torch.Tensor, va
         if s2 != 1 or (s0 | s1) % 4 or t.data_ptr() % 8:
             return None
     for t in held:
+        if t.ndim != 4 or t.shape[2] != capacity:
+            return None
         s0, s1, s2, s3 = t.stride()
         if (t.shape[0] != B or t.shape[1] != Hk or t.shape[3] != D or t.dtype != dtype or t.device != device or s3 != 1
                 or (s0 | s1 | s2) % 4 or t.data_ptr() % 8):

@@ -104,6 +104,34 @@ def test_what_the_kernel_does_not_cover_goes_to_the_array_operators():
         assert queries.requires_grad == (change == "grad")
 
 
+@pytest.mark.parametrize("broken", ["values shorter", "offset behind the end", "offset without buffers", "negative offset"])
+def test_rows_outside_the_cache_are_left_to_the_array_operators(monkeypatch, broken):
+    """Buffers and offsets that do not belong together never reach the kernel: the caller gets what the array operators
+    make of them, an error where the rows do not fit."""
+    gen = torch.Generator(device="cuda").manual_seed(14)
+    attn, _ = _layer(1, 16, 4, 2, 128, 128, torch.bfloat16, torch.bfloat16, gen, True)
+    x = torch.empty((1, 16, 8), device="cuda")
+
+    def launched(*args):
+        raise AssertionError("the kernel was launched")
+
+    monkeypatch.setattr(A._native.lib(), "dflash_attn_prepare", launched)
+    cache = KVCache()
+    if broken != "offset without buffers":
+        cache.update_and_fetch(*(torch.zeros((1, 2, 100, 128), dtype=torch.bfloat16, device="cuda") for _ in range(2)))
+    if broken == "values shorter":
+        cache.values = cache.values[:, :, :100].contiguous()
+    elif broken == "negative offset":
+        cache.offset = -20
+    else:
+        cache.offset = 1000
+    if broken == "negative offset":  # (they count from the end)
+        assert A._project(attn, x, cache)[4] == -20 and cache.offset == -4
+        return
+    with pytest.raises(RuntimeError):
+        A._project(attn, x, cache)
+
+
 @pytest.mark.parametrize("B,Hq,Hk,D,N,dtype,masked,joint", [
     (1, 32, 8, 256, 4112, torch.bfloat16, False, True), (2, 16, 2, 128, 257, torch.float16, False, False),
     (1, 24, 4, 256, 1040, torch.bfloat16, True, True), (3, 5, 1, 128, 300, torch.bfloat16, False, True)])
