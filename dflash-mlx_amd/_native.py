@@ -10,6 +10,7 @@ import os
 from typing import Optional
 
 import torch
+from torch.autograd import forward_ad
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libdflash_mi355.so")
@@ -205,6 +206,24 @@ def env(key: bytes) -> Optional[bytes]:
     except AttributeError:  # an os.environ of another make
         value = os.environ.get(os.fsdecode(key))
         return None if value is None else os.fsencode(value)
+
+
+_functorch_level, _tracing = torch._C._functorch.peek_interpreter_stack, torch._C._get_tracing_state
+_dispatch_modes, _compiling = torch._C._len_torch_dispatch_stack, torch.compiler.is_compiling
+
+
+def plain(*tensors: torch.Tensor) -> bool:
+    """Ordinary tensors that nothing is differentiating, tracing or batching: what a kernel that takes
+    their addresses may stand in for array operators on.  The results of such a kernel have no graph, no tangent and
+    no place in a trace, so every call that the array operators could also answer asks here first."""
+    if (_compiling() or forward_ad._current_level >= 0 or _functorch_level() is not None or _tracing() is not None
+            or _dispatch_modes()):
+        return False
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if (type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter) or (grad and t.requires_grad):
+            return False
+    return True
 
 
 def raw_stream(device) -> int:

@@ -16,7 +16,6 @@ from typing import Any, Optional
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
-from torch.autograd import forward_ad
 
 from . import _native
 from .cache import KVCache
@@ -25,7 +24,6 @@ from .kernels import _DTYPE_CODE, batched_sdpa_2pass_exact
 from .verify_linear import shared_input_outputs
 
 _HYBRID_SDPA_EXACT_KV_THRESHOLD = 1024
-_functorch_level, _tracing = torch._C._functorch.peek_interpreter_stack, torch._C._get_tracing_state
 
 
 def _attention_num_heads(attn: Any) -> int:
@@ -168,19 +166,6 @@ def _project(self, x: torch.Tensor, cache: Optional[Any]):
     return queries, keys, values, gate, cached_prefix_len
 
 
-def _plain(*tensors: torch.Tensor) -> bool:
-    """Ordinary device tensors that nothing is differentiating, tracing or batching: what a kernel that takes
-    their addresses may stand in for the array operators on."""
-    if (forward_ad._current_level >= 0 or _functorch_level() is not None or _tracing() is not None
-            or torch.compiler.is_compiling()):
-        return False
-    grad = torch.is_grad_enabled()
-    for t in tensors:
-        if (type(t) is not torch.Tensor and type(t) is not nn.Parameter) or not t.is_cuda or (grad and t.requires_grad):
-            return False
-    return True
-
-
 def _unhooked(module: nn.Module) -> bool:
     return not (module._forward_hooks or module._forward_pre_hooks)
 
@@ -211,7 +196,7 @@ def _project_on_device(self, q_proj_output: torch.Tensor, keys: torch.Tensor, va
     capacity = cache.keys.shape[2] if held and cache.keys.ndim == 4 else 0
     if not 0 <= cache.offset <= capacity:
         return None
-    if not _plain(q_proj_output, keys, values, qw, kw, *held):
+    if not q_proj_output.is_cuda or not _native.plain(q_proj_output, keys, values, qw, kw, *held):
         return None
     if not (keys.dtype == values.dtype == dtype and keys.device == values.device == device == qw.device == kw.device
             and qw.shape == (D,) == kw.shape and qw.dtype in _DTYPE_CODE and kw.dtype in _DTYPE_CODE
@@ -247,7 +232,7 @@ def _finish(self, output: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
     """Gate and output projection.  ``gate`` [B, L, Hq * D], or the whole output of q_proj, [B, L, Hq * 2 D], as ``_project_on_device`` leaves it."""
     B, H, L, D = output.shape
     if gate.shape[-1] == 2 * H * D:
-        if (output.dtype == gate.dtype and _plain(output) and output.stride(3) == 1 and output.data_ptr() % 8 == 0
+        if (output.dtype == gate.dtype and output.is_cuda and _native.plain(output) and output.stride(3) == 1 and output.data_ptr() % 8 == 0
                 and (output.stride(0) | output.stride(1) | output.stride(2)) % 4 == 0):
             gated = torch.empty((B, L, H * D), dtype=output.dtype, device=output.device)
             rc = _native.lib().dflash_attn_gate(

@@ -64,8 +64,8 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
                      *, transpose: bool = True, group_size: int = 64, bits: int = 4,
                      mode: str = "affine") -> torch.Tensor:
     """Stock quantized matmul: dequantise to x.dtype, then an ordinary matmul - on the device in one
-    launch (``verify_qmm.rows_matmul``), else (host tensors, shapes it does not cover,
-    ``DFLASH_STOCK_KERNEL=0``) with array operators."""
+    launch (``verify_qmm.rows_matmul``), else (host tensors, shapes it does not cover, operands that
+    something differentiates, ``DFLASH_STOCK_KERNEL=0``) with array operators."""
     if mode != "affine":
         raise NotImplementedError(f"quantisation mode {mode!r}")
     if transpose and x.is_cuda and _native.env(b"DFLASH_STOCK_KERNEL") != b"0":
@@ -81,7 +81,7 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
 def stock_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
                  *, transpose: bool = True, group_size: int = 64, bits: int = 4, mode: str = "affine") -> torch.Tensor:
     """What a quantized module computes outside the verify switch: ``quantized_matmul``, except
-    that at most 16 rows of device activations take the M=16 kernel on zero-padded rows
+    that at most 16 rows of device activations take the M=16 kernel on the rows there are
     (``verify_qmm.small_m_matmul``) instead of dequantising the whole matrix - one-token steps
     and the narrow projections that the verify gate does not admit.  ``DFLASH_STOCK_KERNEL=0``
     keeps every such call on the array-op form."""

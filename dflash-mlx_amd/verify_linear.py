@@ -148,6 +148,7 @@ class FusedProjections:
     def _holds(self, parent: nn.Module, x: torch.Tensor, padded: bool = False) -> bool:
         if x.device != self.weight.device:
             return False
+        grad = torch.is_grad_enabled()
         for index, name in enumerate(self.names):
             # (submodules and their marks by the dictionaries they live in: getattr() looks there last)
             mod = parent._modules.get(name)
@@ -157,6 +158,9 @@ class FusedProjections:
                 mod = mod._modules.get("linear")
             joined = None if mod is None else mod.__dict__.get("_shared_input")
             if joined is None or joined[0] is not self or joined[1] != index:
+                return False
+            # (the joint matrix is not what a member's own scales, made leaves, would get their gradient from)
+            if grad and (mod._buffers["scales"].requires_grad or mod._buffers["biases"].requires_grad):
                 return False
         return True
 

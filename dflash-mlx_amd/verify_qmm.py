@@ -458,12 +458,14 @@ def small_m_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biase
     the product depends on its own row of x only, so a row comes out the same whatever shares the
     block with it).  Covers what the C ABI covers
     (N a multiple of 16, K a multiple of the group size, bf16/fp16), which is more than the
-    Python gate of ``verify_matmul`` lets through; returns None for anything else.  No
+    Python gate of ``verify_matmul`` lets through; returns None for anything else, and for calls that
+    something differentiates, traces or batches (``_native.plain``).  No
     counterpart in the reference, whose stock operator is a fused kernel of its own: here the
     stock operator dequantises the whole matrix with array ops, which for a one-token step or a
     48-row projection costs far more than the product itself."""
-    if (not x.is_cuda or bits != 4 or group_size not in (32, 64, 128) or x.dtype not in _DTYPE_CODE or
-            scales.dtype not in _DTYPE_CODE or biases.dtype != scales.dtype or w.ndim != 2 or not _native.is_built()):
+    if (not x.is_cuda or not _native.plain(x, w, scales, biases) or bits != 4 or group_size not in (32, 64, 128) or
+            x.dtype not in _DTYPE_CODE or scales.dtype not in _DTYPE_CODE or biases.dtype != scales.dtype or
+            w.ndim != 2 or not _native.is_built()):
         return None
     K, N = x.shape[-1], w.shape[0]
     m = x.numel() // K if K else 0
@@ -494,9 +496,10 @@ def small_m_silu_mul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
                      *, group_size: int = 64, bits: int = 4) -> "torch.Tensor | None":
     """``silu(x @ gate.T) * (x @ up.T)`` for at most 16 rows of device activations in one launch of the streaming
     kernel; ``w`` holds the gate rows of an MLP followed by its up rows.  None for what that kernel does not
-    cover.  No counterpart in the reference."""
-    if (not x.is_cuda or bits != 4 or x.dtype not in _DTYPE_CODE or not (scales.dtype == biases.dtype == x.dtype)
-            or w.ndim != 2 or not _native.is_built() or _kernel_select() != _native.QMM_KERNEL_AUTO):
+    cover or ``small_m_matmul`` leaves to the array operators.  No counterpart in the reference."""
+    if (not x.is_cuda or not _native.plain(x, w, scales, biases) or bits != 4 or x.dtype not in _DTYPE_CODE
+            or not (scales.dtype == biases.dtype == x.dtype) or w.ndim != 2 or not _native.is_built()
+            or _kernel_select() != _native.QMM_KERNEL_AUTO):
         return None
     K, N = int(x.shape[-1]), int(w.shape[0])
     m = x.numel() // K if K else 0
@@ -538,10 +541,12 @@ def rows_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: 
     """``x @ dequant(w).T`` for any number of rows of device activations in one launch
     (``dflash_qmm_rows``): weights are dequantised to the activation type inside the product.
     Returns None for what the kernel does not cover (other bit widths, fp32, N not a multiple of
-    16).  ``epilogue="silu_mul"``: ``w`` holds the gate rows of an MLP followed by its up rows and the result is
+    16) and for calls that something differentiates, traces or batches (``_native.plain``).
+    ``epilogue="silu_mul"``: ``w`` holds the gate rows of an MLP followed by its up rows and the result is
     ``silu(gate) * up``.  No counterpart in the reference, whose stock operator is ``mx.quantized_matmul``."""
-    if (not x.is_cuda or bits != 4 or group_size not in (32, 64, 128) or x.dtype not in _DTYPE_CODE or
-            scales.dtype not in _DTYPE_CODE or biases.dtype != scales.dtype or w.ndim != 2 or not _native.is_built()):
+    if (not x.is_cuda or not _native.plain(x, w, scales, biases) or bits != 4 or group_size not in (32, 64, 128) or
+            x.dtype not in _DTYPE_CODE or scales.dtype not in _DTYPE_CODE or biases.dtype != scales.dtype or
+            w.ndim != 2 or not _native.is_built()):
         return None
     K, N = int(x.shape[-1]), int(w.shape[0])
     M = x.numel() // K if K else 0

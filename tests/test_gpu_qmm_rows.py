@@ -3,7 +3,7 @@ tile edges in M, N and K, every group size, both activation types, split and who
 import pytest
 import torch
 
-from dflash_mlx_amd.quantized import dequantize, quantized_matmul
+from dflash_mlx_amd.quantized import QuantizedLinear, dequantize, quantized_matmul
 from dflash_mlx_amd.verify_qmm import rows_matmul
 from dflash_mlx_amd.workloads import make_qmm_case
 
@@ -75,3 +75,79 @@ def test_more_tiles_than_the_chip_takes_at_once(native_lib, M, K, N, group, dtyp
         got = y[:, lo:lo + 4096].double()
         assert ((got - exact).abs() <= 1.01 * eps * exact.abs() + size * 2.0 ** -24 * K ** 0.5 + 1e-6).all()
         assert (got - exact).norm() <= eps * exact.norm()
+
+
+def _layer(widths, K, seed, dtype=torch.bfloat16):
+    """A parent module whose swapped projections were joined."""
+    from dflash_mlx_amd import verify_linear as VL
+
+    parent = torch.nn.Module()
+    for i, (name, n) in enumerate(widths.items()):
+        c = make_qmm_case(K, n, seed + i, dtype=dtype).to(DEV)
+        c.scales.mul_(0.05); c.biases.mul_(0.05)
+        setattr(parent, name, QuantizedLinear(c.w, c.scales, c.biases, group_size=64, bits=4))
+    VL.install_verify_linears(parent)
+    assert VL.fuse_shared_input_linears(parent) == 1
+    return parent
+
+
+@pytest.mark.parametrize("rows", [1, 15, 17, 77])
+def test_gradients_reach_the_activations(native_lib, rows):
+    """A call that something differentiates keeps the array operators, whose graph autograd has: x + layer(x), joined
+    projections, the gated activation, and the scales themselves."""
+    from dflash_mlx_amd import verify_linear as VL
+
+    c = make_qmm_case(512, 512, 50 + rows, M=rows).to(DEV)
+    dense = dequantize(c.w, c.scales, c.biases, 64, 4, dtype=torch.bfloat16).double()
+    x, g = c.x.clone().requires_grad_(True), torch.randn_like(c.x)
+    layer = QuantizedLinear(c.w, c.scales, c.biases, group_size=64, bits=4)
+    (x + layer(x)).backward(g)
+    want = g.double() + g.double() @ dense
+    # one rounding each of the product's part of the gradient and of the sum
+    assert (x.grad.double() - want).norm() <= 2 * 2.0 ** -8 * want.norm()
+    scales = c.scales.clone().requires_grad_(True)
+    quantized_matmul(c.x, c.w, scales, c.biases).backward(g)
+    assert scales.grad is not None and bool((scales.grad != 0).any())
+
+    parent = _layer(dict(gate_proj=256, up_proj=256), 512, 60)
+    for fn in (lambda v: VL.shared_input_outputs(parent, ("gate_proj", "up_proj"), v)[1], lambda v: VL.silu_gate_up(parent, v)):
+        x.grad = None
+        fn(x).float().square().sum().backward()
+        assert x.grad is not None and bool((x.grad != 0).any())
+    if rows > 16:
+        parent.up_proj.scales.requires_grad_(True)
+        VL.silu_gate_up(parent, c.x).float().square().sum().backward()
+        assert parent.up_proj.scales.grad is not None
+
+
+@pytest.mark.parametrize("rows", [5, 40])
+def test_tangents_and_batched_calls_keep_the_array_operators(native_lib, rows):
+    from torch.autograd import forward_ad
+
+    from dflash_mlx_amd.verify_qmm import small_m_matmul, small_m_silu_mul
+
+    c = make_qmm_case(512, 512, 70 + rows, M=rows).to(DEV)
+    t = torch.randn_like(c.x)
+    with forward_ad.dual_level():
+        y = quantized_matmul(forward_ad.make_dual(c.x, t), c.w, c.scales, c.biases)
+        tangent = forward_ad.unpack_dual(y).tangent
+    assert tangent is not None
+    want = t.double() @ dequantize(c.w, c.scales, c.biases, 64, 4, dtype=torch.bfloat16).double().t().contiguous()
+    assert (tangent.double() - want).norm() <= 2.0 ** -8 * want.norm()
+
+    def none_of_the_kernels(v):
+        for kernel in (rows_matmul, small_m_matmul, small_m_silu_mul):
+            assert kernel(v, c.w, c.scales, c.biases) is None
+        return v
+
+    torch.func.vmap(none_of_the_kernels)(torch.stack([c.x, t]))
+
+    class Tagged(torch.Tensor):
+        pass
+
+    none_of_the_kernels(c.x.as_subclass(Tagged))
+    assert rows_matmul(c.x, c.w, c.scales, c.biases) is not None
+
+    layer = QuantizedLinear(c.w, c.scales, c.biases, group_size=64, bits=4)
+    whole = torch.compile(layer, backend="eager", fullgraph=True)  # one graph of array operators, no break at a launch
+    assert (whole(c.x).float() - layer(c.x).float()).norm() <= 2.0 ** -8 * layer(c.x).float().norm()
