@@ -22,6 +22,11 @@
 //    The result carries fp32 accuracy, as the step-by-step kernel's does.
 //  * The operands of the next chunk are loaded into the registers of the present one as soon as these have
 //    been used for the last time; 1 wave per SIMD has registers for all of them.
+//  * The closed form is for finite numbers: in a product over all tokens of a chunk, a NaN or an infinity meets the
+//    zeros of M' and Lq and spoils tokens and rows of the state that it must not reach, and products of k with k
+//    may overflow where the recurrence does not.  Both kernels look at what they computed (a sum of 0 x stays zero
+//    as long as every x is finite), and such a chunk is walked token by token instead, by the same wave.  What a masked
+//    token holds never enters a product: its rows of K and Q are zeros, its element of V - c U as well.
 // A 16-bit state is carried in fp32 and rounded once, at the end.
 //
 // Measured, 1024 tokens, 16 / 32 heads of 128 x 128: 15 + 65 us, against 123.7 ms with one workgroup per head
@@ -36,7 +41,8 @@ namespace prompt {
 
 constexpr int kChunk = 32;
 constexpr int kMatBytes = 2 * 3 * 1024;                // [tile of 16 rows][piece][lane] 16 bytes
-constexpr int kHeadBytes = 2 * kMatBytes + 3 * kChunk * 4;  // M', Lq, then per token c (0 if masked) and c_T / c_s, then c_T
+constexpr int kHeadBytes = 2 * kMatBytes + 3 * kChunk * 4;  // M', Lq, then per token c (0 if masked) and c_T / c_s, then kTail:
+constexpr int kTail = 2 * kChunk;                      // four words: c_T, 0 or (numbers that are not finite) NaN, one bit per token that counts, -
 constexpr int kPitch = 36;                             // floats per row of the 32 x 32 matrices in LDS
 
 struct Args {
@@ -100,21 +106,27 @@ __global__ __launch_bounds__(64, 3) void gdn_chunk_kernel(Args a) {
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     int t = t0 + 16 * i + li;
-    t = t < a.T ? t : a.T - 1;
+    const bool past = t >= a.T;
+    t = past ? a.T - 1 : t;
     const size_t row = ((slotT + t) * a.Hk + hk) * DK + 8 * kq;
+    const bool on = !past && (a.mask == nullptr || a.mask[slotT + t] != 0);
 #pragma unroll
     for (int C = 0; C < NC; ++C) {
       kf[i][C] = *reinterpret_cast<const uint4*>(a.k + row + 32 * C);
       qf[i][C] = *reinterpret_cast<const uint4*>(a.q + row + 32 * C);
+      if (!on) kf[i][C] = qf[i][C] = uint4{0u, 0u, 0u, 0u};
     }
   }
+  float finite = 0.f;  // stays zero
   float on_v = 0.f;
   if (lane < kChunk) {
     const int t = t0 + lane;
     const bool on = t < a.T && (a.mask == nullptr || a.mask[slotT + t] != 0);
     const size_t at = (slotT + (t < a.T ? t : a.T - 1)) * a.Hv + hv;
-    sGate[lane] = on ? load_as_f32(a.g, at, a.g_dtype) : 1.f;
-    sBeta[lane] = on ? load_as_f32(a.beta, at, a.beta_dtype) : 0.f;
+    const float g = on ? load_as_f32(a.g, at, a.g_dtype) : 1.f, beta = on ? load_as_f32(a.beta, at, a.beta_dtype) : 0.f;
+    sGate[lane] = g;
+    sBeta[lane] = beta;
+    finite = fmaf(g, 0.f, beta * 0.f);
     on_v = on ? 1.f : 0.f;
   }
   if (writes_k) {
@@ -133,6 +145,9 @@ __global__ __launch_bounds__(64, 3) void gdn_chunk_kernel(Args a) {
         x1 = mfma(kf[ts][C], kf[tt][C], x1);
         x2 = mfma(kf[ts][C], qf[tt][C], x2);
       }
+      // (with the diagonals k . k and k . q among them: nothing that is not finite in K or Q stays unseen)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) finite = fmaf(x1[e], 0.f, fmaf(x2[e], 0.f, finite));
       *reinterpret_cast<f32x4_t*>(sA + (16 * tt + li) * kPitch + 16 * ts + 4 * kq) = x1;
       *reinterpret_cast<f32x4_t*>(sB + (16 * tt + li) * kPitch + 16 * ts + 4 * kq) = x2;
     }
@@ -155,12 +170,15 @@ __global__ __launch_bounds__(64, 3) void gdn_chunk_kernel(Args a) {
       c_mine = t == s ? c : c_mine;
       const float x = mat[t * kPitch + s];
       const bool counts = lower ? t > s : t >= s && on_t[t] != 0.f;  // (a masked token's y is zero)
-      mat[t * kPitch + s] = counts ? (lower ? sBeta[t] * r * x : r * x) : 0.f;
+      const float entry = counts ? (lower ? sBeta[t] * r * x : r * x) : 0.f;
+      mat[t * kPitch + s] = entry;
+      finite = fmaf(entry, 0.f, finite);
     }
+    finite = fmaf(r, 0.f, fmaf(c, 0.f, finite));
     if (lower) {
       vec[s] = on_v != 0.f ? c_mine : 0.f;
       vec[kChunk + s] = r;
-      if (s == 0) vec[2 * kChunk] = c;
+      if (s == 0) vec[kTail] = c;
     }
   }
   __syncthreads();
@@ -187,10 +205,17 @@ __global__ __launch_bounds__(64, 3) void gdn_chunk_kernel(Args a) {
     }
     __syncthreads();
     const float beta = sBeta[j];
+#pragma unroll
+    for (int t = 0; t < kChunk; ++t) finite = fmaf(x[t] * beta, 0.f, finite);
     if (lane < 32) {
 #pragma unroll
       for (int t = 0; t < kChunk; ++t) sA[t * kPitch + j] = x[t] * beta;
     }
+  }
+  {
+    const bool all_finite = __all(finite == 0.f);
+    const uint32_t on_bits = (uint32_t)__ballot(on_v != 0.f);
+    if (lane == 0) vec[kTail + 1] = all_finite ? 0.f : __builtin_nanf(""), vec[kTail + 2] = __uint_as_float(on_bits);
   }
   __syncthreads();
 #pragma unroll
@@ -223,7 +248,8 @@ __global__ __launch_bounds__(64, 3) void gdn_chunk_kernel(Args a) {
   }
 }
 
-template <int DK>
+// MASKED: some tokens may not count (those past T read zeros and need no looking after).
+template <int DK, bool MASKED>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void gdn_prompt_kernel(Args a) {
   constexpr int NC = DK / 32, NT = DK / 16;
   const int slices = a.Dv / 16;
@@ -274,12 +300,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
   uint4 kf[2][NC], qf[2][NC], kt[NT], mf[2][3], lf[2][3];
   uint32_t vb[8];
   f32x4_t cv[2], cfv[2];
-  float c_last, c_next;  // (asked for with K and Q: the scheduler moves the scaling of S to the front)
+  f32x4_t tail_next;  // (asked for with K and Q: the scheduler moves the scaling of S to the front)
   const size_t per_chunk = chunk_bytes<DK>(a);
   const char* const head0 = a.work + (size_t)slot * a.chunks * per_chunk + (size_t)hv * kHeadBytes;
   const char* const kt0 = a.work + (size_t)slot * a.chunks * per_chunk + (size_t)a.Hv * kHeadBytes + (size_t)hk * (kChunk * DK * 2);
   auto load_kq = [&](int ch) __attribute__((always_inline)) {
-    c_next = reinterpret_cast<const float*>(head0 + ch * per_chunk + 2 * kMatBytes)[2 * kChunk + (lane >> 6)];
+    tail_next = reinterpret_cast<const f32x4_t*>(head0 + ch * per_chunk + 2 * kMatBytes + 4 * kTail)[lane >> 6];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const uint32_t at = k_at + (ch * kChunk + 16 * i) * k_step;
@@ -317,15 +343,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
   };
   // arithmetic may move across, requests to memory stay where they were written
 #define DFLASH_KEEP_REQUESTS() __builtin_amdgcn_sched_barrier(0xF)
-  load_kq(0);
-  DFLASH_KEEP_REQUESTS();  // in the order of the loop: what its first wait may leave in flight is the least of both
-  load_v(0);
-  load_mat(0, 0, mf);
-  load_kt(0);
-  load_mat(0, 1, lf);
-  load_vec(0);
-  DFLASH_KEEP_REQUESTS();
-
   // sum of the six piece products of two fp32 factors that matter; two accumulators, smaller terms first
   auto product6 = [&](const uint4 (&f)[3], const Pieces<8>& p, f32x4_t big) __attribute__((always_inline)) {
     f32x4_t small = {0.f, 0.f, 0.f, 0.f};
@@ -338,75 +355,153 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
     return big + small;
   };
 
+  // The recurrence itself, for a chunk with numbers that are not finite.
+  auto token_by_token = [&](int ch) __attribute__((always_inline)) {
+    const int end = (ch + 1) * kChunk < a.T ? (ch + 1) * kChunk : a.T;
 #pragma unroll 1
-  for (int ch = 0; ch < a.chunks; ++ch) {
-    const int next = ch + 1 < a.chunks ? ch + 1 : ch;
-    c_last = c_next;
-    // ---- U = K S^T, W = Q S^T: rows = tokens, column = dv ---------------------------------------
-    f32x4_t U[2], W[2];
+    for (int t = ch * kChunk; t < end; ++t) {
+      const uint32_t at = (uint32_t)t * v_step + (hv * a.Dv + dv) * 2;
+      float delta = 0.f, y = 0.f;
+      if (a.mask == nullptr || a.mask[slotT + t] != 0) {
+        const float g = load_as_f32(a.g, (slotT + t) * a.Hv + hv, a.g_dtype);
+        const float beta = load_as_f32(a.beta, (slotT + t) * a.Hv + hv, a.beta_dtype);
+        const float v = bf16_bits_to_f32((uint16_t)__builtin_amdgcn_raw_buffer_load_b16(v_buf, at, 0, 0));
+        const size_t row = ((slotT + t) * a.Hk + hk) * DK + 8 * kq;
+        auto element = [](uint4 w, int e) __attribute__((always_inline)) {  // 0 .. 7
+          const uint32_t half[4] = {w.x, w.y, w.z, w.w};
+          return __uint_as_float(e & 1 ? half[e >> 1] & 0xffff0000u : half[e >> 1] << 16);
+        };
+        uint4 kw[NC], qw[NC];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) U[i] = W[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        for (int C = 0; C < NC; ++C) {
+          kw[C] = *reinterpret_cast<const uint4*>(a.k + row + 32 * C);
+          qw[C] = *reinterpret_cast<const uint4*>(a.q + row + 32 * C);
+        }
+        float known = 0.f;  // S k, summed over the four lanes that hold a row of S
 #pragma unroll
-    for (int C = 0; C < NC; ++C) {
-      const float f[8] = {st[2 * C][0],     st[2 * C][1],     st[2 * C][2],     st[2 * C][3],
-                          st[2 * C + 1][0], st[2 * C + 1][1], st[2 * C + 1][2], st[2 * C + 1][3]};
-      const Pieces<8> sp = split_bf16(f);
+        for (int C = 0; C < NC; ++C)
 #pragma unroll
-      for (int i = 0; i < 2; ++i) U[i] = mfma(kf[i][C], sp.lo, U[i]), W[i] = mfma(qf[i][C], sp.lo, W[i]);
+          for (int e = 0; e < 8; ++e) {
+            f32x4_t& entry = st[2 * C + (e >> 2)];
+            entry[e & 3] *= g;
+            known = fmaf(entry[e & 3], element(kw[C], e), known);
+          }
+        known += __shfl_xor(known, 16, 64);
+        known += __shfl_xor(known, 32, 64);
+        delta = (v - known) * beta;
 #pragma unroll
-      for (int i = 0; i < 2; ++i) U[i] = mfma(kf[i][C], sp.mid, U[i]), W[i] = mfma(qf[i][C], sp.mid, W[i]);
+        for (int C = 0; C < NC; ++C)
 #pragma unroll
-      for (int i = 0; i < 2; ++i) U[i] = mfma(kf[i][C], sp.hi, U[i]), W[i] = mfma(qf[i][C], sp.hi, W[i]);
-    }
-    load_kq(next);
-    DFLASH_KEEP_REQUESTS();
-    // ---- Delta = M' (V - c U) ----------------------------------------------------------------------
-    float rhs[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) rhs[j] = bf16_bits_to_f32(vb[j]) - cv[j >> 2][j & 3] * U[j >> 2][j & 3];
-    load_v(next);
-    DFLASH_KEEP_REQUESTS();
-    const Pieces<8> rp = split_bf16(rhs);
-    f32x4_t D[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) D[i] = product6(mf[i], rp, f32x4_t{0.f, 0.f, 0.f, 0.f});
-    load_mat(next, 0, mf);
-    DFLASH_KEEP_REQUESTS();
-    // ---- S^T = c_T S^T + K^T diag(c_T / c_s) Delta ----------------------------------------------
-    float scaled[8], plain[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      plain[j] = D[j >> 2][j & 3];
-      scaled[j] = plain[j] * cfv[j >> 2][j & 3];
-    }
-    {
-      const Pieces<8> dp = split_bf16(scaled);
-#pragma unroll
-      for (int c = 0; c < NT; ++c) st[c] *= c_last;
-#pragma unroll
-      for (int c = 0; c < NT; ++c) st[c] = mfma(kt[c], dp.lo, st[c]);
-#pragma unroll
-      for (int c = 0; c < NT; ++c) st[c] = mfma(kt[c], dp.mid, st[c]);
-#pragma unroll
-      for (int c = 0; c < NT; ++c) st[c] = mfma(kt[c], dp.hi, st[c]);
-    }
-    load_kt(next);
-    DFLASH_KEEP_REQUESTS();
-    // ---- Y = c W + Lq Delta ------------------------------------------------------------------------
-    const Pieces<8> dq = split_bf16(plain);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const f32x4_t Y = product6(lf[i], dq, W[i] * cv[i]);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const uint32_t at = v_at + (ch * kChunk + 16 * i + r) * v_step;
-        __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(uint16_t, (__bf16)Y[r]), y_buf, at, 0, 0);
-        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(D[i][r]), tape_buf, 2 * at, 0, 0);
+          for (int e = 0; e < 8; ++e) {
+            f32x4_t& entry = st[2 * C + (e >> 2)];
+            entry[e & 3] = fmaf(element(kw[C], e), delta, entry[e & 3]);
+            y = fmaf(entry[e & 3], element(qw[C], e), y);
+          }
+        y += __shfl_xor(y, 16, 64);
+        y += __shfl_xor(y, 32, 64);
+      }
+      if (kq == 0) {
+        __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(uint16_t, (__bf16)y), y_buf, at, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(delta), tape_buf, 2 * at, 0, 0);
       }
     }
-    load_mat(next, 1, lf);
-    load_vec(next);
+  };
+
+  // (the way to the token-by-token form leaves the loop: the loop itself stays without a branch around its stores)
+  int ch = 0;
+  while (ch < a.chunks) {
+    load_kq(ch);
+    DFLASH_KEEP_REQUESTS();  // in the order of the loop: what its first wait may leave in flight is the least of both
+    load_v(ch);
+    load_mat(ch, 0, mf);
+    load_kt(ch);
+    load_mat(ch, 1, lf);
+    load_vec(ch);
     DFLASH_KEEP_REQUESTS();
+#pragma unroll 1
+    for (; ch < a.chunks; ++ch) {
+      const int next = ch + 1 < a.chunks ? ch + 1 : ch;
+      const float c_last = tail_next[0];
+      float finite = tail_next[1];  // stays zero
+      int keep[8];  // all bits of the tokens of this lane that count
+#pragma unroll
+      for (int j = 0; j < 8; ++j) keep[j] = MASKED ? -(int)((__float_as_uint(tail_next[2]) >> token_of(kq, j)) & 1u) : -1;
+      // ---- U = K S^T, W = Q S^T: rows = tokens, column = dv ---------------------------------------
+      f32x4_t U[2], W[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) U[i] = W[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int C = 0; C < NC; ++C) {
+        const float f[8] = {st[2 * C][0],     st[2 * C][1],     st[2 * C][2],     st[2 * C][3],
+                            st[2 * C + 1][0], st[2 * C + 1][1], st[2 * C + 1][2], st[2 * C + 1][3]};
+        const Pieces<8> sp = split_bf16(f);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) U[i] = mfma(kf[i][C], sp.lo, U[i]), W[i] = mfma(qf[i][C], sp.lo, W[i]);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) U[i] = mfma(kf[i][C], sp.mid, U[i]), W[i] = mfma(qf[i][C], sp.mid, W[i]);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) U[i] = mfma(kf[i][C], sp.hi, U[i]), W[i] = mfma(qf[i][C], sp.hi, W[i]);
+      }
+      load_kq(next);
+      DFLASH_KEEP_REQUESTS();
+      // ---- Delta = M' (V - c U) ----------------------------------------------------------------------
+      float rhs[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        rhs[j] = bf16_bits_to_f32(vb[j]) - cv[j >> 2][j & 3] * U[j >> 2][j & 3];
+        if (MASKED) rhs[j] = __int_as_float(__float_as_int(rhs[j]) & keep[j]);
+      }
+      load_v(next);
+      DFLASH_KEEP_REQUESTS();
+      const Pieces<8> rp = split_bf16(rhs);
+      f32x4_t D[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) D[i] = product6(mf[i], rp, f32x4_t{0.f, 0.f, 0.f, 0.f});
+      load_mat(next, 0, mf);
+      DFLASH_KEEP_REQUESTS();
+      // a number that is not finite in V, U (and so in S) or M' is one in every Delta of its column
+#pragma unroll
+      for (int j = 0; j < 8; ++j) finite = fmaf(D[j >> 2][j & 3], 0.f, finite);
+      if (!__all(finite == 0.f)) break;
+      // ---- S^T = c_T S^T + K^T diag(c_T / c_s) Delta ----------------------------------------------
+      float scaled[8], plain[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        plain[j] = D[j >> 2][j & 3];
+        scaled[j] = plain[j] * cfv[j >> 2][j & 3];
+      }
+      {
+        const Pieces<8> dp = split_bf16(scaled);
+#pragma unroll
+        for (int c = 0; c < NT; ++c) st[c] *= c_last;
+#pragma unroll
+        for (int c = 0; c < NT; ++c) st[c] = mfma(kt[c], dp.lo, st[c]);
+#pragma unroll
+        for (int c = 0; c < NT; ++c) st[c] = mfma(kt[c], dp.mid, st[c]);
+#pragma unroll
+        for (int c = 0; c < NT; ++c) st[c] = mfma(kt[c], dp.hi, st[c]);
+      }
+      load_kt(next);
+      DFLASH_KEEP_REQUESTS();
+      // ---- Y = c W + Lq Delta ------------------------------------------------------------------------
+      const Pieces<8> dq = split_bf16(plain);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const f32x4_t Y = product6(lf[i], dq, W[i] * cv[i]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const uint32_t at = v_at + (ch * kChunk + 16 * i + r) * v_step;
+          uint16_t y = __builtin_bit_cast(uint16_t, (__bf16)Y[r]);
+          if (MASKED) y &= (uint16_t)keep[4 * i + r];
+          __builtin_amdgcn_raw_buffer_store_b16(y, y_buf, at, 0, 0);
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(D[i][r]), tape_buf, 2 * at, 0, 0);
+        }
+      }
+      load_mat(next, 1, lf);
+      load_vec(next);
+      DFLASH_KEEP_REQUESTS();
+    }
+    if (ch < a.chunks) token_by_token(ch++);
   }
 #undef DFLASH_KEEP_REQUESTS
 
@@ -429,7 +524,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
 template <int DK>
 int launch(const Args& a, hipStream_t s) {
   hipLaunchKernelGGL((gdn_chunk_kernel<DK>), dim3((unsigned)(a.slots * a.chunks * a.Hv)), dim3(64), 0, s, a);
-  hipLaunchKernelGGL((gdn_prompt_kernel<DK>), dim3((unsigned)(a.slots * a.Hv * (a.Dv / 16))), dim3(64), 0, s, a);
+  const dim3 grid((unsigned)(a.slots * a.Hv * (a.Dv / 16)));
+  if (a.mask != nullptr) hipLaunchKernelGGL((gdn_prompt_kernel<DK, true>), grid, dim3(64), 0, s, a);
+  else hipLaunchKernelGGL((gdn_prompt_kernel<DK, false>), grid, dim3(64), 0, s, a);
   DFLASH_HIP_OK(hipGetLastError());
   return DFLASH_OK;
 }

@@ -334,3 +334,73 @@ def test_output_norm_in_the_same_launch(native_lib, dtype, wdtype, state_dtype, 
     assert not fused_output_norm_applies(args[0], args[2], args[5], z[..., :64], weight)
     with pytest.raises(ValueError):
         gated_delta_kernel_with_tape(*args, output_norm=(z[..., :64], weight, 1e-6))
+
+
+def _same_values(got, want, bar):
+    """NaN where the other has NaN, the same infinities, and finite values within ``bar`` of their norm."""
+    got, want = got.detach().cpu().double(), want.detach().cpu().double()
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(torch.isinf(got), torch.isinf(want)) and torch.equal(got[torch.isinf(got)], want[torch.isinf(want)])
+    ok = torch.isfinite(want)
+    assert float((got[ok] - want[ok]).norm()) <= bar * max(float(want[ok].norm()), 1e-30)
+
+
+@pytest.mark.parametrize("shape", [dict(T=70, B=2), dict(T=100, B=1, Dk=64, Dv=48, Hk=2, Hv=2)])
+@pytest.mark.parametrize("what", ["v", "k", "q", "g", "beta", "state"])
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), -float("inf")])
+def test_a_non_finite_value_in_a_prompt_reaches_what_comes_after_it(native_lib, shape, what, value):
+    """Token by token, a NaN or an infinity at one token touches that token and the ones behind it, in the rows of the state
+    it enters; chunks of tokens must not hand it to the ones before or to other rows.  Against the array operators on the host."""
+    args = list(_case(seed=70, **shape))
+    for at in (5, 37):  # in the first chunk and in one that a state is carried into
+        new = [t.clone() for t in args]
+        which = ["q", "k", "v", "g", "beta", "state"].index(what)
+        if what == "state":
+            new[which][0, 1, 3, 7] = value
+        elif what in ("g", "beta"):
+            new[which][0, at, 1] = value
+        else:
+            new[which][0, at, 1, 9] = value
+        y, s, tape = _run(new)
+        wide = [t.double() for t in new]
+        yo, so, to = _gated_delta_ops_with_tape(*wide)
+        _same_values(y, yo, 4e-3)
+        _same_values(s, so, 2e-5)
+        _same_values(tape, to, 2e-5)
+
+
+@pytest.mark.parametrize("T", [17, 70])
+def test_what_a_mask_hides_in_a_prompt_has_no_effect(native_lib, T):
+    """A masked token is skipped whatever it holds: the same bits as with ordinary values in its place."""
+    args = _case(seed=71, T=T)
+    mask = torch.rand((2, T), generator=torch.Generator().manual_seed(T)) > 0.4
+    mask[:, 3], mask[:, 16] = False, False
+    plain = _run(args, mask)
+    for value in (float("nan"), float("inf")):
+        hidden = [t.clone() for t in args]
+        for t in hidden[:5]:
+            t[~mask] = value
+        for a, b in zip(_run(hidden, mask), plain):
+            assert torch.equal(a, b)
+    # and together with a value that counts
+    last = int(torch.nonzero(mask[0])[-1])
+    hidden[2][0, last, 1, 5] = float("nan")
+    y, s, tape = _run(hidden, mask)
+    assert bool(torch.isnan(s[0, 1, 5]).all()) and int(torch.isnan(s).sum()) == 128
+    assert int(torch.isnan(y).sum()) == 1 and int(torch.isnan(tape).sum()) == 1
+
+
+def test_magnitudes_whose_products_leave_the_range_of_fp32(native_lib):
+    """Keys and values of 1e20 overflow in the closed form of a chunk (k . k) before they do token by token."""
+    q, k, v, g, beta, state = _case(seed=72, T=40, Hk=2, Hv=2)
+    k[0, 20] *= 1e20
+    v[1, 30] *= 1e30
+    wide = [t.float() for t in (q, k, v, g, beta, state)]
+    yo, so, to = _gated_delta_ops_with_tape(*wide)
+    y, s, tape = _run((q, k, v, g, beta, state))
+    for before, (a, b) in ((20, (y[0], yo[0])), (20, (tape[0], to[0]))):
+        _same_values(a[:before], b[:before], 4e-3)
+        assert bool(torch.isfinite(a[:before]).all())
+    _same_values(y[1], yo[1], 4e-3)
+    _same_values(tape[1], to[1], 2e-5)
+    _same_values(s[1], so[1], 2e-5)
