@@ -474,6 +474,8 @@ def small_m_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biase
     w, scales, biases = w.contiguous(), scales.contiguous(), biases.contiguous()
     _require_operands("quantized_matmul", K, N, group_size, w, scales, biases, x.device)
     x2 = x.reshape(m, K).contiguous()
+    if m < 16 and x2.data_ptr() % 16:  # (the kernel loads 16 bytes at a time; it refuses a whole block that starts elsewhere)
+        x2 = x2.clone()
     lib = _native.lib()
     y = torch.empty((m, N), dtype=x.dtype, device=x.device)
     stream = _native.raw_stream(x.device)

@@ -128,3 +128,18 @@ def test_few_rows_take_the_joint_launch(native_lib, monkeypatch):
     parent.in_proj_z.to(torch.device(DEV), torch.bfloat16)
     parent.in_proj_z._apply(lambda t: t.clone())
     assert not group.serves_few(parent, x[:, :1])
+
+
+@pytest.mark.parametrize("rows", [1, 3, 15])
+def test_few_rows_that_start_anywhere(native_lib, monkeypatch, rows):
+    """The kernel loads x in pieces of 16 bytes; fewer rows than a block may start on any element all the same."""
+    monkeypatch.delenv("DFLASH_QMM_KERNEL", raising=False)
+    for group, K, N in ((64, 1024, 256), (32, 576, 48), (128, 128, 16)):
+        c = make_qmm_case(K, N, 960 + rows, group_size=group, M=rows).to(DEV)
+        want = stock_matmul(c.x, c.w, c.scales, c.biases, group_size=group)
+        for shift in (1, 4):
+            held = torch.empty(rows * K + shift, dtype=c.x.dtype, device=DEV)
+            x = held[shift:].view(rows, K)
+            x.copy_(c.x)
+            assert x.data_ptr() % 16 and x.is_contiguous()
+            assert torch.equal(stock_matmul(x, c.w, c.scales, c.biases, group_size=group), want)
