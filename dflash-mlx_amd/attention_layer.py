@@ -21,7 +21,7 @@ from . import _native
 from .cache import KVCache
 from .gdn_layer import rms_norm_ops
 from .kernels import _DTYPE_CODE, batched_sdpa_2pass_exact
-from .verify_linear import shared_input_outputs
+from .verify_linear import shared_input_outputs, unhooked
 
 _HYBRID_SDPA_EXACT_KV_THRESHOLD = 1024
 
@@ -166,10 +166,6 @@ def _project(self, x: torch.Tensor, cache: Optional[Any]):
     return queries, keys, values, gate, cached_prefix_len
 
 
-def _unhooked(module: nn.Module) -> bool:
-    return not (module._forward_hooks or module._forward_pre_hooks)
-
-
 def _project_on_device(self, q_proj_output: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, cache: Any):
     """Everything behind the projections in one launch (``dflash_attn_prepare``), keys and values straight into
     the cache; the gate stays where q_proj put it.  None - the caller then takes the array operators - for
@@ -177,7 +173,7 @@ def _project_on_device(self, q_proj_output: torch.Tensor, keys: torch.Tensor, va
     activations, head sizes other than 64, 128, 192 and 256, a cache of another type or batch."""
     q_norm, k_norm, rope = self.q_norm, self.k_norm, self.rope
     if type(cache) is not KVCache or type(q_norm) is not HeadRMSNorm or type(k_norm) is not HeadRMSNorm \
-            or type(rope) is not RotaryEmbedding or not (_unhooked(q_norm) and _unhooked(k_norm) and _unhooked(rope)):
+            or type(rope) is not RotaryEmbedding or not unhooked(q_norm, k_norm, rope):
         return None
     code = _DTYPE_CODE.get(q_proj_output.dtype)
     if code is None or code == _native.FP32 or q_proj_output.ndim != 3:

@@ -24,6 +24,7 @@ from typing import Callable, List, Optional, Sequence, Tuple
 
 import torch
 import torch.nn as nn
+from torch.nn.modules import module as _every_module
 
 from . import _native
 from .quantized import QuantizedLinear, stock_matmul
@@ -92,6 +93,17 @@ def is_verify_eligible(ql, path: str = "") -> bool:
     return True
 
 
+def unhooked(*modules: nn.Module) -> bool:
+    """Whether calling these modules does what their classes' ``forward`` does and nothing else: no hooks of their
+    own or of every module, no ``forward`` put on the instance.  Only then may a launch stand in for the calls."""
+    if _every_module._global_forward_hooks or _every_module._global_forward_pre_hooks:
+        return False
+    for m in modules:
+        if m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__:
+            return False
+    return True
+
+
 # Sibling projections that read the same input in the decoder layers the reference serves.
 SHARED_INPUT_GROUPS: Tuple[Tuple[str, ...], ...] = (
     ("gate_proj", "up_proj"),
@@ -125,8 +137,8 @@ class FusedProjections:
     def applies(self, parent: nn.Module, x: torch.Tensor) -> bool:
         """The joint launch gives what ``parent``'s members would give one by one: 16 rows on the
         verify path, on the device the joint matrix lives on, every member still a view into it
-        (a module moved with ``.to()``, or replaced, has left) and behind no wrapper that would
-        pad this input."""
+        (a module moved with ``.to()``, or replaced, has left), behind no wrapper that would
+        pad this input and without hooks."""
         if x.numel() != 16 * x.shape[-1] or not _should_use_verify(x, self.group_size, self.bits, True):
             return False
         return self._holds(parent, x)
@@ -155,9 +167,11 @@ class FusedProjections:
             if mod is not None and "_dflash_exact_small_proj_wrapped" in mod.__dict__:
                 if x.ndim == 3 and x.shape[1] < mod.pad_m and not padded:
                     return False
+                if not unhooked(mod):
+                    return False
                 mod = mod._modules.get("linear")
             joined = None if mod is None else mod.__dict__.get("_shared_input")
-            if joined is None or joined[0] is not self or joined[1] != index:
+            if joined is None or joined[0] is not self or joined[1] != index or not unhooked(mod):
                 return False
             # (the joint matrix is not what a member's own scales, made leaves, would get their gradient from)
             if grad and (mod._buffers["scales"].requires_grad or mod._buffers["biases"].requires_grad):

@@ -143,3 +143,51 @@ def test_few_rows_that_start_anywhere(native_lib, monkeypatch, rows):
             x.copy_(c.x)
             assert x.data_ptr() % 16 and x.is_contiguous()
             assert torch.equal(stock_matmul(x, c.w, c.scales, c.biases, group_size=group), want)
+
+
+def test_hooks_of_joined_projections_run(native_lib, monkeypatch):
+    """A member with a hook, or with a forward of its own, answers for itself; every length of call, the wrapper that pads
+    included."""
+    from dflash_mlx_amd import verify_linear as VL
+    from dflash_mlx_amd.gdn_layer import _ExactSmallProjPad
+    from dflash_mlx_amd.quantized import QuantizedLinear
+
+    monkeypatch.setenv("DFLASH_VERIFY_QMM", "1")
+    monkeypatch.delenv("DFLASH_QMM_KERNEL", raising=False)
+    parent = torch.nn.Module()
+    widths = dict(in_proj_qkv=256, in_proj_z=128, in_proj_b=48, in_proj_a=48)
+    for i, (name, n) in enumerate(widths.items()):
+        c = make_qmm_case(1024, n, 980 + i).to(DEV)
+        setattr(parent, name, QuantizedLinear(c.w, c.scales, c.biases, group_size=64, bits=4))
+    parent.in_proj_b, parent.in_proj_a = _ExactSmallProjPad(parent.in_proj_b), _ExactSmallProjPad(parent.in_proj_a)
+    VL.install_verify_linears(parent)
+    assert VL.fuse_shared_input_linears(parent) == 1
+    seen = []
+
+    def hook(module, args, *output):
+        seen.append(module)
+
+    places = [(parent.in_proj_z, "register_forward_hook"), (parent.in_proj_qkv, "register_forward_pre_hook"),
+              (parent.in_proj_b, "register_forward_hook"), (parent.in_proj_b.linear, "register_forward_hook")]
+    for rows in (1, 5, 16, 77):
+        x = make_qmm_case(1024, 32, 990, M=rows).to(DEV).x.reshape(1, rows, 1024)
+        for module, register in places:
+            handle = getattr(module, register)(hook)
+            VL.shared_input_outputs(parent, tuple(widths), x)
+            handle.remove()
+            assert seen == [module], (rows, register)
+            seen.clear()
+        every = torch.nn.modules.module.register_module_forward_hook(hook)
+        VL.shared_input_outputs(parent, tuple(widths), x)
+        every.remove()
+        assert {id(m) for m in seen if isinstance(m, VL.VerifyQuantizedLinear)} == \
+            {id(m) for m in (parent.in_proj_qkv, parent.in_proj_z, parent.in_proj_b.linear, parent.in_proj_a.linear)}
+        seen.clear()
+        z = parent.in_proj_z
+        z.forward = lambda v: seen.append(z) or type(z).forward(z, v)  # as wrappers of a module's forward leave it
+        VL.shared_input_outputs(parent, tuple(widths), x)
+        del z.forward
+        assert seen == [z]
+        seen.clear()
+        VL.shared_input_outputs(parent, tuple(widths), x)
+        assert parent._dflash_fused[0]._holds(parent, x, padded=True) and not seen
