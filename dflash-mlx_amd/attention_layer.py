@@ -146,10 +146,12 @@ def _project(self, x: torch.Tensor, cache: Optional[Any]):
     num_attention_heads = _attention_num_heads(self)
     num_key_value_heads = _attention_num_kv_heads(self)
     # one launch for the three where fuse_shared_input_linears joined them
-    q_proj_output, keys, values = shared_input_outputs(self, ("q_proj", "k_proj", "v_proj"), x)
+    q_proj_output, keys, values = shared_input_outputs(self, ("q_proj", "k_proj", "v_proj"), x, columns=True)
     on_device = _project_on_device(self, q_proj_output, keys, values, cache)
     if on_device is not None:
         return on_device
+    # (norms, rotation and caches of any make see what the projections by themselves would give them)
+    q_proj_output, keys, values = q_proj_output.contiguous(), keys.contiguous(), values.contiguous()
     queries, gate = torch.chunk(q_proj_output.reshape(B, L, num_attention_heads, -1), 2, dim=-1)
     gate = gate.reshape(B, L, -1)
     queries = self.q_norm(queries).transpose(1, 2)
@@ -228,8 +230,8 @@ def _finish(self, output: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
     """Gate and output projection.  ``gate`` [B, L, Hq * D], or the whole output of q_proj, [B, L, Hq * 2 D], as ``_project_on_device`` leaves it."""
     B, H, L, D = output.shape
     if gate.shape[-1] == 2 * H * D:
-        if (output.dtype == gate.dtype and output.is_cuda and _native.plain(output) and output.stride(3) == 1 and output.data_ptr() % 8 == 0
-                and (output.stride(0) | output.stride(1) | output.stride(2)) % 4 == 0):
+        if (output.dtype == gate.dtype and output.is_cuda and _native.plain(output) and output.stride(3) == 1
+                and output.data_ptr() % 8 == 0 and (output.stride(0) | output.stride(1) | output.stride(2)) % 4 == 0):
             gated = torch.empty((B, L, H * D), dtype=output.dtype, device=output.device)
             rc = _native.lib().dflash_attn_gate(
                 output.data_ptr(), gate.data_ptr(), gated.data_ptr(), B, L, H, D, *output.stride()[:3], gate.stride(0),

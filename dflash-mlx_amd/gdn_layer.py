@@ -247,7 +247,7 @@ def _gdn_call(self, inputs: torch.Tensor, mask: Optional[torch.Tensor], cache: O
     """The body shared by the plain and the speculative call (dflash_mlx/runtime.py:359-453)."""
     B, S, _ = inputs.shape
     # one launch for those of the four that fuse_shared_input_linears joined
-    qkv, z, b, a = shared_input_outputs(self, ("in_proj_qkv", "in_proj_z", "in_proj_b", "in_proj_a"), inputs)
+    qkv, z, b, a = shared_input_outputs(self, ("in_proj_qkv", "in_proj_z", "in_proj_b", "in_proj_a"), inputs, columns=True)
     z = z.reshape(B, S, self.num_v_heads, self.head_v_dim)
 
     conv_state = cache[0] if cache is not None else None
@@ -276,7 +276,7 @@ def _gdn_call(self, inputs: torch.Tensor, mask: Optional[torch.Tensor], cache: O
     if cache is not None:
         cache[1] = state
     if not fused:
-        out = self.norm(out, z)
+        out = self.norm(out, z.contiguous())
     return self.out_proj(out.reshape(B, S, -1))
 
 

@@ -255,25 +255,30 @@ def silu_gate_up(parent: nn.Module, x: torch.Tensor, names: Tuple[str, str] = ("
             hidden = group.few_silu_mul(x)
         if hidden is not None:
             return hidden
-    gate, up = shared_input_outputs(parent, names, x)
+    gate, up = shared_input_outputs(parent, names, x, columns=True)
     return (gate * torch.sigmoid(gate)) * up   # x * sigmoid(x): the operators the epilogue follows, one rounding each
 
 
-def shared_input_outputs(parent: nn.Module, names: Sequence[str], x: torch.Tensor) -> Tuple[torch.Tensor, ...]:
+def shared_input_outputs(parent: nn.Module, names: Sequence[str], x: torch.Tensor, *,
+                         columns: bool = False) -> Tuple[torch.Tensor, ...]:
     """``tuple(getattr(parent, n)(x) for n in names)``, with the projections that
-    ``fuse_shared_input_linears`` joined under ``parent`` served by their one launch."""
+    ``fuse_shared_input_linears`` joined under ``parent`` served by their one launch.  The results of a verify block are
+    columns of the joint product; so are those of other lengths for a caller that reads them with their strides
+    (``columns=True``), every other caller gets them as tensors of their own, as the projections would return them."""
     outs = {}
     for group in getattr(parent, "_dflash_fused", ()):
-        if all(n in names for n in group.names) and group.applies(parent, x):
+        if not all(n in names for n in group.names):
+            continue
+        product = None
+        if group.applies(parent, x):
             outs.update(zip(group.names, group(x)))
-        elif all(n in names for n in group.names) and group.serves_prompt(parent, x):
+        elif group.serves_prompt(parent, x):
             product = group.prompt(x)
-            if product is not None:
-                outs.update((n, product[..., lo:hi]) for n, (lo, hi) in zip(group.names, group.bounds))
-        elif all(n in names for n in group.names) and group.serves_few(parent, x):
+        elif group.serves_few(parent, x):
             product = group.few(x)
-            if product is not None:
-                outs.update((n, product[..., lo:hi]) for n, (lo, hi) in zip(group.names, group.bounds))
+        if product is not None:
+            parts = (product[..., lo:hi] for lo, hi in group.bounds)
+            outs.update(zip(group.names, parts if columns else (part.contiguous() for part in parts)))
     return tuple(outs[n] if n in outs else getattr(parent, n)(x) for n in names)
 
 

@@ -191,3 +191,39 @@ def test_hooks_of_joined_projections_run(native_lib, monkeypatch):
         seen.clear()
         VL.shared_input_outputs(parent, tuple(widths), x)
         assert parent._dflash_fused[0]._holds(parent, x, padded=True) and not seen
+
+
+@pytest.mark.parametrize("rows", [1, 5, 77])
+def test_joined_outputs_of_prompts_and_short_blocks_are_tensors_of_their_own(native_lib, monkeypatch, rows):
+    from dflash_mlx_amd import verify_linear as VL
+    from dflash_mlx_amd.quantized import QuantizedLinear
+
+    monkeypatch.setenv("DFLASH_VERIFY_QMM", "1")
+    monkeypatch.delenv("DFLASH_QMM_KERNEL", raising=False)
+    parent = torch.nn.Module()
+    for i, (name, n) in enumerate(dict(q_proj=256, k_proj=64, v_proj=64).items()):
+        c = make_qmm_case(512, n, 970 + i).to(DEV)
+        setattr(parent, name, QuantizedLinear(c.w, c.scales, c.biases, group_size=64, bits=4))
+    VL.install_verify_linears(parent)
+    assert VL.fuse_shared_input_linears(parent) == 1
+    x = make_qmm_case(512, 32, 975, M=rows).to(DEV).x.reshape(1, rows, 512)
+    names = ("q_proj", "k_proj", "v_proj")
+    for name, y in zip(names, VL.shared_input_outputs(parent, names, x)):
+        n = getattr(parent, name).weight.shape[0]
+        assert y.view(rows, n // 32, 32).shape == (rows, n // 32, 32) and y.is_contiguous()
+
+    class Norm(torch.nn.Module):  # somebody's own
+        def __init__(self, weight):
+            super().__init__()
+            self.weight = weight
+
+        def forward(self, v):
+            return v.view(-1, v.shape[-1]).view(v.shape) if v.shape[2] == 2 else v
+
+    from dflash_mlx_amd.attention_layer import GatedAttention
+
+    attn = GatedAttention(num_attention_heads=4, num_key_value_heads=2, head_dim=32, q_proj=parent.q_proj, k_proj=parent.k_proj,
+                          v_proj=parent.v_proj, o_proj=torch.nn.Identity())
+    object.__setattr__(attn, "_dflash_fused", parent._dflash_fused)
+    attn.q_norm, attn.k_norm = Norm(attn.q_norm.weight), Norm(attn.k_norm.weight)
+    assert attn(x).shape == (1, rows, 128)
