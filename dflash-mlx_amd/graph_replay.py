@@ -4,8 +4,8 @@ No counterpart in the reference (MLX builds its graph lazily by itself).  On thi
 through the Python surface costs the host 10-30 microseconds, as much as the device needs for a
 layer kernel, so a serving loop replays the verify step instead of launching it call by call.
 The kernels allow it: nothing in them depends on host state from the time of capture (split-K
-arrival counters return to zero by themselves, accepted lengths can be device tensors,
-workspaces belong to the stream).
+arrival counters return to zero by themselves, accepted lengths can be device tensors, scratch of prompts is the graph's own,
+other workspaces belong to the stream).
 """
 from __future__ import annotations
 

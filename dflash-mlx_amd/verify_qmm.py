@@ -532,6 +532,20 @@ def small_m_silu_mul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
 
 # Scratch of the any-rows product, one per (device, stream): 64 KiB of counters, then partial tiles.
 _ROWS_WORKSPACES: Dict[Tuple[int, int], torch.Tensor] = {}
+_ROWS_COUNTER_BYTES = 1 << 16
+
+
+def _rows_workspace(device: torch.device, key: Tuple[int, int], need: int, recording: bool) -> torch.Tensor:
+    """Counters at zero, then room for partial tiles; every call leaves the counters at zero again.  The buffer of a stream
+    grows with its prompts, and the one it had is freed: a launch that is being recorded has scratch of its own, from the
+    graph's memory, and the clearing of its counters is recorded with it."""
+    ws = None if recording else _ROWS_WORKSPACES.get(key)
+    if ws is None or ws.numel() < need:
+        ws = torch.empty(need if recording else max(need, 1 << 23), dtype=torch.uint8, device=device)
+        ws[:_ROWS_COUNTER_BYTES].zero_()
+        if not recording:
+            _ROWS_WORKSPACES[key] = ws
+    return ws
 
 
 # what dflash_qmm_rows_workspace_bytes answered per call shape
@@ -577,11 +591,7 @@ def rows_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: 
         need = _ROWS_WORKSPACE_BYTES[(index, *shape)] = int(lib.dflash_qmm_rows_workspace_bytes(*shape))
     ws_ptr, ws_bytes = None, 0
     if need:
-        ws = _ROWS_WORKSPACES.get((index, stream))
-        if ws is None or ws.numel() < need:
-            ws = torch.empty(max(need, 1 << 23), dtype=torch.uint8, device=x.device)
-            ws[:1 << 16].zero_()
-            _ROWS_WORKSPACES[(index, stream)] = ws
+        ws = _rows_workspace(x.device, (index, stream), need, torch.cuda.is_current_stream_capturing())
         ws_ptr, ws_bytes = ws.data_ptr(), ws.numel()
     rc = lib.dflash_qmm_rows(x2.data_ptr(), w.data_ptr(), scales.data_ptr(), biases.data_ptr(), y.data_ptr(), ws_ptr,
                              ws_bytes, *shape, stream)

@@ -161,3 +161,43 @@ def test_attention_kernel_replays(native_lib):
         cache_k[:, :, N - 16:N].copy_(torch.randn((1, Hk, 16, D), generator=gen, device=DEV).to(torch.bfloat16))
 
     _replays_match(graph, captured, run, refill)
+
+
+def test_products_of_prompts_replay_beside_longer_ones(native_lib):
+    """Products of more than 16 rows whose K is cut into slices: the recorded launches keep scratch of their own when the
+    same stream goes on to longer prompts, whose scratch replaces the stream's, and its old memory is used for something else."""
+    cases = [make_qmm_case(4096, 1040, seed_for(0, 101), M=77).to(DEV), make_qmm_case(2048, 512, seed_for(0, 102), M=33).to(DEV),
+             make_qmm_case(5120, 12352, seed_for(0, 103), M=1000).to(DEV)]
+
+    def run():
+        return [VQ.rows_matmul(c.x, c.w, c.scales, c.biases) for c in cases[:2]] + [
+            VQ.rows_matmul(cases[0].x, cases[0].w[:1024], cases[0].scales[:1024], cases[0].biases[:1024], epilogue="silu_mul")]
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    graph, key = torch.cuda.CUDAGraph(), (torch.device(DEV).index, side.cuda_stream)
+    VQ._ROWS_WORKSPACES.pop(key, None)
+    with torch.cuda.stream(side):
+        run()
+        first = VQ._ROWS_WORKSPACES[key]  # (the shapes do need it)
+        side.synchronize()
+        with torch.cuda.graph(graph, stream=side):
+            captured = run()
+        assert VQ._ROWS_WORKSPACES[key] is first
+        VQ._ROWS_WORKSPACES[key] = first[:1 << 16].clone()  # too small for anything: the next call replaces it
+        size = first.numel()
+        del first
+        litter = [torch.full((size,), 255, dtype=torch.uint8, device=DEV) for _ in range(2)]
+        VQ.rows_matmul(cases[2].x, cases[2].w, cases[2].scales, cases[2].biases)
+    torch.cuda.synchronize()
+    gen = torch.Generator(device=DEV).manual_seed(7)
+
+    def refill(r):
+        for c in cases[:2]:
+            c.x.copy_(torch.randn(c.x.shape, generator=gen, device=DEV).to(c.x.dtype))
+        with torch.cuda.stream(side):
+            for t in litter:
+                t.fill_(255 - r)
+            run()
+
+    _replays_match(graph, captured, run, refill, rounds=4)

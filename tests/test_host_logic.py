@@ -559,3 +559,17 @@ def test_narrow_projections_join_a_shared_input_group(monkeypatch):
     del m.linear_attn.in_proj_z, m.linear_attn.in_proj_a
     install_verify_linears(m)
     assert fuse_shared_input_linears(m) == 0 and type(m.linear_attn.in_proj_b) is QuantizedLinear
+
+
+def test_scratch_of_recorded_prompts_is_not_shared(monkeypatch):
+    """The buffer of a stream is replaced by a larger one and freed; a recorded launch keeps its addresses, so it must
+    never be given that buffer."""
+    monkeypatch.setattr(VQ, "_ROWS_WORKSPACES", {})
+    cpu, key = torch.device("cpu"), (0, 0)
+    eager = VQ._rows_workspace(cpu, key, 1 << 20, False)
+    assert VQ._rows_workspace(cpu, key, 1 << 19, False) is eager
+    recorded = VQ._rows_workspace(cpu, key, 1 << 20, True)
+    assert recorded is not eager and VQ._rows_workspace(cpu, key, 1 << 20, True).data_ptr() != recorded.data_ptr()
+    assert recorded.numel() >= 1 << 20 and not recorded[:VQ._ROWS_COUNTER_BYTES].any()
+    larger = VQ._rows_workspace(cpu, key, 1 << 24, False)
+    assert larger is not eager and VQ._ROWS_WORKSPACES == {key: larger} and not larger[:VQ._ROWS_COUNTER_BYTES].any()
