@@ -211,7 +211,7 @@ def _project_on_device(self, q_proj_output: torch.Tensor, keys: torch.Tensor, va
         if (t.shape[0] != B or t.shape[1] != Hk or t.shape[3] != D or t.dtype != dtype or t.device != device or s3 != 1
                 or (s0 | s1 | s2) % 4 or t.data_ptr() % 8):
             return None
-    prev = cache._append_room(B, Hk, L, D, D, keys, values)
+    prev = cache._make_room(B, Hk, L, D, D, keys, values)
     ko, vo = cache.keys, cache.values
     queries = torch.empty((B, Hq, L, D), dtype=dtype, device=device)
     strides = (ctypes.c_longlong * 12)(*q_proj_output.stride()[:2], *keys.stride()[:2], *values.stride()[:2],
@@ -222,7 +222,7 @@ def _project_on_device(self, q_proj_output: torch.Tensor, keys: torch.Tensor, va
         strides, q_norm.eps, k_norm.eps, float(rope.base), code, _DTYPE_CODE[qw.dtype], _DTYPE_CODE[kw.dtype],
         _native.raw_stream(device))
     _native.check(rc, "dflash_attn_prepare")
-    end = prev + L
+    end = cache.offset = prev + L  # the rows are on their way: not before
     return queries, ko[:, :, :end], vo[:, :, :end], q_proj_output, prev
 
 

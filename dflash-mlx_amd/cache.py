@@ -25,14 +25,15 @@ class KVCache:
     def update_and_fetch(self, keys: torch.Tensor, values: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
         """Append ``keys``/``values`` ``[B, H, S, D]`` at ``offset``; return the filled prefix."""
         b, h, s, dk = keys.shape
-        prev = self._append_room(b, h, s, dk, values.shape[3], keys, values)
+        prev = self._make_room(b, h, s, dk, values.shape[3], keys, values)
+        self.offset = prev + s
         self.keys[:, :, prev:self.offset] = keys
         self.values[:, :, prev:self.offset] = values
         return self.keys[:, :, :self.offset], self.values[:, :, :self.offset]
 
-    def _append_room(self, b: int, h: int, s: int, dk: int, dv: int, keys: torch.Tensor, values: torch.Tensor) -> int:
-        """Moves ``offset`` past ``s`` more rows, growing the buffers where they are too short (types and devices
-        as ``keys`` / ``values``); returns where the new rows start."""
+    def _make_room(self, b: int, h: int, s: int, dk: int, dv: int, keys: torch.Tensor, values: torch.Tensor) -> int:
+        """Grows the buffers where they are too short for ``s`` more rows (types and devices as ``keys`` / ``values``);
+        returns where the new rows start.  Whoever writes them moves ``offset``."""
         prev = self.offset
         if self.keys is None or prev + s > self.keys.shape[2]:
             n_steps = (self.step + s - 1) // self.step
@@ -43,7 +44,6 @@ class KVCache:
                 self.values = torch.cat([self.values[:, :, :prev], new_v], dim=2)
             else:
                 self.keys, self.values = new_k, new_v
-        self.offset = prev + s
         return prev
 
     def is_trimmable(self) -> bool:

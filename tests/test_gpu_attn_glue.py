@@ -150,3 +150,23 @@ def test_gate_behind_the_attention(B, Hq, Hk, D, N, dtype, masked, joint):
     # one range of keys: nothing to ride on, the plain result
     short = batched_sdpa_2pass_exact(q, k[:, :, :100], v[:, :, :100], D ** -0.5, q_proj_output=outs[0])
     assert torch.equal(short, batched_sdpa_2pass_exact(q, k[:, :, :100], v[:, :, :100], D ** -0.5))
+
+
+def test_a_refused_launch_leaves_the_cache_where_it_was(monkeypatch):
+    gen = torch.Generator(device="cuda").manual_seed(15)
+    attn, _ = _layer(1, 16, 4, 2, 128, 128, torch.bfloat16, torch.bfloat16, gen, True)
+    x = torch.empty((1, 16, 8), device="cuda")
+    for prefix in (0, 250):  # no buffers yet; buffers that are too short for the block
+        cache = KVCache()
+        before = [torch.randn((1, 2, prefix, 128), generator=gen, device="cuda").to(torch.bfloat16) for _ in range(2)]
+        if prefix:
+            cache.update_and_fetch(*before)
+        with monkeypatch.context() as m:
+            m.setattr(A._native.lib(), "dflash_attn_prepare", lambda *args: -1)
+            with pytest.raises(A._native.NativeLibraryError):
+                A._project(attn, x, cache)
+        assert cache.offset == prefix
+        _, keys, _, _, at = A._project(attn, x, cache)
+        assert at == prefix and cache.offset == prefix + 16 and keys.shape[2] == prefix + 16
+        if prefix:
+            assert torch.equal(keys[:, :, :prefix], before[0])
