@@ -78,7 +78,8 @@ __device__ __forceinline__ void attn_prepare_token(const AttnPrepareArgs& p, int
     unpack_adjacent<PER>(wraw, wdt, w);
 #pragma unroll
     for (int e = 0; e < PER; ++e) ss += x[e] * x[e];
-    const float inv_rms = 1.0f / sqrtf(wave_sum(ss) / (float)D + (is_q ? p.q_eps : p.k_eps));
+    // (the array operators divide by a number by multiplying with its reciprocal: the mean here, the exponents above)
+    const float inv_rms = 1.0f / sqrtf(wave_sum(ss) * (1.0f / (float)D) + (is_q ? p.q_eps : p.k_eps));
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
       x[e] = round_through(x[e] * inv_rms * w[e], p.dt);

@@ -170,3 +170,24 @@ def test_a_refused_launch_leaves_the_cache_where_it_was(monkeypatch):
         assert at == prefix and cache.offset == prefix + 16 and keys.shape[2] == prefix + 16
         if prefix:
             assert torch.equal(keys[:, :, :prefix], before[0])
+
+
+@pytest.mark.parametrize("D,dims", [(128, 128), (128, 96), (192, 192), (192, 96), (256, 104), (64, 20)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_bits_of_the_array_operators_where_the_norms_sum_is_exact(monkeypatch, D, dims, dtype):
+    """Small whole numbers: their squares add up exactly in any order, so that every bit that is left to differ is
+    the rotation's or a rounding's."""
+    gen = torch.Generator(device="cuda").manual_seed(16)
+    attn, outs = _layer(1, 40, 6, 2, D, dims, dtype, dtype, gen, True)
+    for o in outs:
+        o.copy_(torch.randint(-8, 9, o.shape, generator=gen, device="cuda"))
+    x = torch.empty((1, 40, 8), device="cuda")
+    caches = [KVCache(), KVCache()]
+    for c in caches:
+        c.update_and_fetch(*(torch.zeros((1, 2, 3001, D), dtype=dtype, device="cuda") for _ in range(2)))
+    got = A._project(attn, x, caches[0])
+    assert got[3].shape[-1] == 2 * 6 * D  # the kernel took it
+    monkeypatch.setattr(A, "_project_on_device", lambda *a: None)
+    want = A._project(attn, x, caches[1])
+    for a, b in zip(got[:3], want[:3]):
+        assert torch.equal(a, b)
