@@ -195,7 +195,7 @@ def lib() -> ctypes.CDLL:
 
 
 def is_built() -> bool:
-    return os.path.exists(LIB_PATH)
+    return _lib is not None or os.path.exists(LIB_PATH)  # (a look at the file costs a microsecond)
 
 
 def env(key: bytes) -> Optional[bytes]:
@@ -210,6 +210,7 @@ def env(key: bytes) -> Optional[bytes]:
 
 _functorch_level, _tracing = torch._C._functorch.peek_interpreter_stack, torch._C._get_tracing_state
 _dispatch_modes, _compiling = torch._C._len_torch_dispatch_stack, torch.compiler.is_compiling
+_grad_enabled, _Tensor, _Parameter = torch.is_grad_enabled, torch.Tensor, torch.nn.Parameter
 
 
 def plain(*tensors: torch.Tensor) -> bool:
@@ -219,10 +220,14 @@ def plain(*tensors: torch.Tensor) -> bool:
     if (_compiling() or forward_ad._current_level >= 0 or _functorch_level() is not None or _tracing() is not None
             or _dispatch_modes()):
         return False
-    grad = torch.is_grad_enabled()
     for t in tensors:
-        if (type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter) or (grad and t.requires_grad):
+        made = type(t)
+        if made is not _Tensor and made is not _Parameter:
             return False
+    if _grad_enabled():
+        for t in tensors:
+            if t.requires_grad:
+                return False
     return True
 
 

@@ -93,13 +93,17 @@ def is_verify_eligible(ql, path: str = "") -> bool:
     return True
 
 
+_HOOKS_OF_EVERY, _PRE_HOOKS_OF_EVERY = _every_module._global_forward_hooks, _every_module._global_forward_pre_hooks
+
+
 def unhooked(*modules: nn.Module) -> bool:
     """Whether calling these modules does what their classes' ``forward`` does and nothing else: no hooks of their
     own or of every module, no ``forward`` put on the instance.  Only then may a launch stand in for the calls."""
-    if _every_module._global_forward_hooks or _every_module._global_forward_pre_hooks:
+    if _HOOKS_OF_EVERY or _PRE_HOOKS_OF_EVERY:
         return False
     for m in modules:
-        if m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__:
+        own = m.__dict__
+        if own["_forward_hooks"] or own["_forward_pre_hooks"] or "forward" in own:
             return False
     return True
 

@@ -463,13 +463,14 @@ def small_m_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biase
     counterpart in the reference, whose stock operator is a fused kernel of its own: here the
     stock operator dequantises the whole matrix with array ops, which for a one-token step or a
     48-row projection costs far more than the product itself."""
-    if (not x.is_cuda or not _native.plain(x, w, scales, biases) or bits != 4 or group_size not in (32, 64, 128) or
-            x.dtype not in _DTYPE_CODE or scales.dtype not in _DTYPE_CODE or biases.dtype != scales.dtype or
-            w.ndim != 2 or not _native.is_built()):
+    if (not x.is_cuda or bits != 4 or group_size not in (32, 64, 128) or x.dtype not in _DTYPE_CODE or
+            scales.dtype not in _DTYPE_CODE or biases.dtype != scales.dtype or w.ndim != 2):
         return None
     K, N = x.shape[-1], w.shape[0]
     m = x.numel() // K if K else 0
     if m < 1 or m > 16 or N % 16 != 0 or K % group_size != 0 or K % 32 != 0 or w.shape[1] * 8 != K:
+        return None
+    if not _native.plain(x, w, scales, biases) or not _native.is_built():
         return None
     w, scales, biases = w.contiguous(), scales.contiguous(), biases.contiguous()
     _require_operands("quantized_matmul", K, N, group_size, w, scales, biases, x.device)
@@ -499,13 +500,14 @@ def small_m_silu_mul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
     """``silu(x @ gate.T) * (x @ up.T)`` for at most 16 rows of device activations in one launch of the streaming
     kernel; ``w`` holds the gate rows of an MLP followed by its up rows.  None for what that kernel does not
     cover or ``small_m_matmul`` leaves to the array operators.  No counterpart in the reference."""
-    if (not x.is_cuda or not _native.plain(x, w, scales, biases) or bits != 4 or x.dtype not in _DTYPE_CODE
-            or not (scales.dtype == biases.dtype == x.dtype) or w.ndim != 2 or not _native.is_built()
-            or _kernel_select() != _native.QMM_KERNEL_AUTO):
+    if (not x.is_cuda or bits != 4 or x.dtype not in _DTYPE_CODE or not (scales.dtype == biases.dtype == x.dtype)
+            or w.ndim != 2 or _kernel_select() != _native.QMM_KERNEL_AUTO):
         return None
     K, N = int(x.shape[-1]), int(w.shape[0])
     m = x.numel() // K if K else 0
     if m < 1 or m > 16 or N % 16 != 0 or int(w.shape[1]) * 8 != K:
+        return None
+    if not _native.plain(x, w, scales, biases) or not _native.is_built():
         return None
     lib = _native.lib()
     key = (K, N, group_size, -1, 1, _native.QMM_KERNEL_STREAM)  # (-1: with the activation)
@@ -560,13 +562,14 @@ def rows_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: 
     16) and for calls that something differentiates, traces or batches (``_native.plain``).
     ``epilogue="silu_mul"``: ``w`` holds the gate rows of an MLP followed by its up rows and the result is
     ``silu(gate) * up``.  No counterpart in the reference, whose stock operator is ``mx.quantized_matmul``."""
-    if (not x.is_cuda or not _native.plain(x, w, scales, biases) or bits != 4 or group_size not in (32, 64, 128) or
-            x.dtype not in _DTYPE_CODE or scales.dtype not in _DTYPE_CODE or biases.dtype != scales.dtype or
-            w.ndim != 2 or not _native.is_built()):
+    if (not x.is_cuda or bits != 4 or group_size not in (32, 64, 128) or x.dtype not in _DTYPE_CODE or
+            scales.dtype not in _DTYPE_CODE or biases.dtype != scales.dtype or w.ndim != 2):
         return None
     K, N = int(x.shape[-1]), int(w.shape[0])
     M = x.numel() // K if K else 0
     if M < 1 or N % 16 != 0 or K % group_size != 0 or int(w.shape[1]) * 8 != K:
+        return None
+    if not _native.plain(x, w, scales, biases) or not _native.is_built():
         return None
     code = _native.QMM_EPILOGUE_NONE
     if epilogue is not None:
