@@ -375,7 +375,7 @@ __global__ __launch_bounds__(256 * KG, 2) void qmm_rows_kernel(Args a) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const float g = round16<FP16>(v[t][r]), u = round16<FP16>(v[t + kTiles][r]);
-          const float s = round16<FP16>(1.0f / (1.0f + __expf(-g)));
+          const float s = round16<FP16>(1.0f / (1.0f + expf(-g)));
           o[r] = round16<FP16>(g * s) * u;
         }
       }

@@ -151,3 +151,16 @@ def test_tangents_and_batched_calls_keep_the_array_operators(native_lib, rows):
     layer = QuantizedLinear(c.w, c.scales, c.biases, group_size=64, bits=4)
     whole = torch.compile(layer, backend="eager", fullgraph=True)  # one graph of array operators, no break at a launch
     assert (whole(c.x).float() - layer(c.x).float()).norm() <= 2.0 ** -8 * layer(c.x).float().norm()
+
+
+def test_activation_takes_the_bits_of_the_array_operators(native_lib):
+    """Rows with a single 1 make every product exact (a dequantised weight), so that nothing but the activation is left to
+    differ: every 16-bit gate a checkpoint's codes give, against the operators one by one."""
+    for dtype in (torch.bfloat16, torch.float16):
+        c = make_qmm_case(512, 2048, 80, dtype=dtype).to(DEV)
+        c.scales.mul_(0.2); c.biases.mul_(0.2)
+        x = torch.eye(512, dtype=dtype, device=DEV)
+        gate, up = rows_matmul(x, c.w, c.scales, c.biases).split(1024, dim=-1)
+        assert torch.equal(torch.cat([gate, up], dim=-1), dequantize(c.w, c.scales, c.biases, 64, 4, dtype=dtype).t())
+        h = rows_matmul(x, c.w, c.scales, c.biases, epilogue="silu_mul")
+        assert torch.equal(h, (gate * torch.sigmoid(gate)) * up)
