@@ -533,7 +533,7 @@ int qmm_up_to_16(const void* x, const uint32_t* w_q, const void* scales, const v
                              sb_dtype, false, (hipStream_t)stream);
   }
   DFLASH_REQUIRE(kernel != DFLASH_QMM_KERNEL_STREAM, DFLASH_ERR_SHAPE,
-                 "dflash_qmm_m16: the streaming kernel needs group_size 64 and K %% 1024 == 0 "
+                 "dflash_qmm_m16: the streaming kernel, asked for by name, needs group_size 64 and K %% 512 == 0 "
                  "(K=%d gs=%d)", K, group_size);
   float* partials = nullptr;
   uint32_t* counters = nullptr;

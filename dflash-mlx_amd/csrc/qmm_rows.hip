@@ -29,9 +29,12 @@
 // Measured (kernel time, group 64, before that cut): 1024 rows of 5120 x 34816 415 us (880 TFLOP/s; torch's bf16 product of weights
 // that are already dense 411 us), 17408 x 5120 204 us (237), 5120 x 5120 71 us (62); 77 rows of
 // 4096 x 24576 42 us, 12288 x 4096 22 us.  The form with codes in registers took 540, 260, 105 and 87, 31 us for
-// the same tiles.  What bounds it at many rows is shared: matrix instructions 45 % of the cycles,
-// vector instructions 38 %, at 2.0 of 2.4 GHz (power); with no dequantisation at all the same loop is 20 % faster.
-// At few rows it is latency: two memory round trips before the first product and one for the slices.
+// the same tiles.  What bounds it at many rows is shared (counters, the first of these shapes with the
+// activation): matrix instructions 42 % of the SIMDs' cycles, other vector instructions 38 %, the LDS busy for 50 % - half of that
+// bank conflicts - at 1.9 of 2.4 GHz (power); with no dequantisation at all the same loop is 20 % faster.
+// At few rows it is latency - two memory round trips before the first product and one for the slices, a third of the
+// waves' time - and the LDS: 77 rows of 4096 x 24576 matrix 24 %, vector 37 %, LDS 51 %.
+// The activation's exponential is expf as in its other forms; 64 of them per lane behind the last stage cost 1 %.
 #include "dflash_common.h"
 #include "qmm_stream_device.h"
 

@@ -13,7 +13,8 @@ and shape dispatch, with the device work done by the gfx950 kernel behind
 * ``DFLASH_VERIFY_VARIANT`` in {auto, mma2big, mma2big_pipe} and
   ``DFLASH_VERIFY_QMM_KPARTS`` select the variant (:15-22, 292-297).
 * ``DFLASH_QMM_KERNEL`` in {auto, tile, stream} picks the device kernel (no counterpart
-  in the reference; auto uses the streaming kernel for group 64 and K % 512 == 0).
+  in the reference; auto uses the streaming kernel, whose every-K form takes all group sizes and K a multiple of 64,
+  wherever it applies).
 * An eligible call needs device tensors and the built HIP library; there is no
   software fallback for it.
 """

@@ -46,7 +46,8 @@ enum { DFLASH_QMM_MMA2BIG = 0, DFLASH_QMM_MMA2BIG_PIPE = 1 };
  * per K slice, K cut into k_parts slices for the pipe variant.  STREAM: persistent
  * workgroups that divide the weight matrix evenly and stream it through LDS; needs
  * group_size 64 and K % 512 == 0, and decides the K split itself (variant and k_parts
- * then only name the caller's dispatch decision).  AUTO: STREAM where it applies.
+ * then only name the caller's dispatch decision).  AUTO: STREAM where it applies, and its
+ * form for every group size and K a multiple of 64 where scales and biases start on 4 bytes.
  */
 enum { DFLASH_QMM_KERNEL_AUTO = 0, DFLASH_QMM_KERNEL_TILE = 1, DFLASH_QMM_KERNEL_STREAM = 2 };
 
