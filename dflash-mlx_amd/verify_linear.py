@@ -178,7 +178,7 @@ class FusedProjections:
             if joined is None or joined[0] is not self or joined[1] != index or not unhooked(mod):
                 return False
             # (the joint matrix is not what a member's own scales, made leaves, would get their gradient from)
-            if grad and (mod._buffers["scales"].requires_grad or mod._buffers["biases"].requires_grad):
+            if grad and any(t is not None and t.requires_grad for t in (mod.scales, mod.biases)):
                 return False
         return True
 

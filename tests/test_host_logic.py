@@ -573,3 +573,18 @@ def test_scratch_of_recorded_prompts_is_not_shared(monkeypatch):
     assert recorded.numel() >= 1 << 20 and not recorded[:VQ._ROWS_COUNTER_BYTES].any()
     larger = VQ._rows_workspace(cpu, key, 1 << 24, False)
     assert larger is not eager and VQ._ROWS_WORKSPACES == {key: larger} and not larger[:VQ._ROWS_COUNTER_BYTES].any()
+
+
+def test_members_whose_scales_are_learnt_leave_the_joint_product(monkeypatch):
+    """As leaves, in place or as parameters put where the buffers were: only while gradients are on."""
+    monkeypatch.delenv("DFLASH_VERIFY_QMM", raising=False)
+    m = _SharedInputToy()
+    install_verify_linears(m)
+    fuse_shared_input_linears(m)
+    group, x = m.mlp.gate_proj._shared_input[0], torch.randn(40, 512).to(torch.bfloat16)
+    assert group._holds(m.mlp, x)
+    for make in (lambda t: t.requires_grad_(True), lambda t: nn.Parameter(t.detach().clone())):
+        m.mlp.up_proj.scales = make(m.mlp.up_proj.scales)
+        assert not group._holds(m.mlp, x)
+        with torch.no_grad():
+            assert group._holds(m.mlp, x)
