@@ -130,6 +130,51 @@ __device__ __forceinline__ void raw8_to_lds(const Raw8<WIDE>& r, int dt, float* 
   reinterpret_cast<float4*>(dst)[0] = float4{o[0], o[1], o[2], o[3]};
   reinterpret_cast<float4*>(dst)[1] = float4{o[4], o[5], o[6], o[7]};
 }
+// N consecutive elements (N a power of two) of an array of 4-byte (wide) or 2-byte elements, as the bits they are;
+// element i is a multiple of N and the array 16-byte aligned.
+template <int N>
+__device__ __forceinline__ void load_bits(const void* p, size_t i, bool wide, uint32_t (&raw)[N]) {
+  if (wide) {
+    __builtin_memcpy(raw, __builtin_assume_aligned((const uint32_t*)p + i, N < 4 ? 4 * N : 16), 4 * N);
+  } else {
+    __builtin_memcpy(raw, __builtin_assume_aligned((const uint16_t*)p + i, N < 8 ? 2 * N : 16), 2 * N);
+  }
+}
+// ... and element e of them as a number
+template <int N>
+__device__ __forceinline__ float bits_element(const uint32_t (&raw)[N], int e, int dt) {
+  if (dt == DFLASH_FP32) return __uint_as_float(raw[e]);
+  const uint32_t h = e & 1 ? raw[e >> 1] >> 16 : raw[e >> 1] & 0xffffu;
+  return dt == DFLASH_BF16 ? bf16_bits_to_f32(h) : f16_bits_to_f32(h);
+}
+
+// Where element e of a row of D fp32 values sits in LDS when lanes read eight consecutive ones each: the lower and the
+// upper four of every eight in planes of their own, so that 16 lanes reading 16 bytes each read 256 consecutive ones.
+template <int D>
+__device__ __forceinline__ constexpr int plane_index(int e) {
+  return ((e >> 2) & 1) * (D / 2) + 4 * (e >> 3) + (e & 3);
+}
+
+typedef __attribute__((ext_vector_type(4))) unsigned int u32x4_t;
+typedef __attribute__((ext_vector_type(2))) float f32x2_t;
+typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
+typedef __attribute__((ext_vector_type(2))) _Float16 f16x2_t;
+// Two fp32 values rounded to a 16-bit type, the first in the low half, and the way back.
+template <int DT>
+__device__ __forceinline__ uint32_t pack_pair(float a, float b) {
+  if constexpr (DT == DFLASH_BF16) return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t{a, b}), bf16x2_t));
+  else return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t{a, b}), f16x2_t));
+}
+template <int DT>
+__device__ __forceinline__ float pair_lo(uint32_t w) {
+  if constexpr (DT == DFLASH_BF16) return __uint_as_float(w << 16);
+  else return (float)__builtin_bit_cast(f16x2_t, w)[0];
+}
+template <int DT>
+__device__ __forceinline__ float pair_hi(uint32_t w) {
+  if constexpr (DT == DFLASH_BF16) return __uint_as_float(w & 0xffff0000u);
+  else return (float)__builtin_bit_cast(f16x2_t, w)[1];
+}
 __device__ __forceinline__ f32x4_t mfma4(float x, float y, f32x4_t acc) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, acc, 0, 0, 0);
 }

@@ -59,10 +59,6 @@ struct Args {
   int stages;           // ceil(K / (64 KG))
 };
 
-typedef __attribute__((ext_vector_type(2))) float f32x2_t;
-typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
-typedef __attribute__((ext_vector_type(2))) _Float16 f16x2_t;
-
 template <bool FP16>
 __device__ __forceinline__ uint32_t pack2(float a, float b) {
   if constexpr (FP16) {

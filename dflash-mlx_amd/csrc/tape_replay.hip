@@ -17,7 +17,7 @@
 //    that is a rank-16 update which runs on the fp32 matrix cores; as scalar
 //    FMAs it costs more time than the memory traffic of the head.  bf16/fp16
 //    states, which the reference rounds after every step (kernels.py:281-283),
-//    and callers that ask for it keep the step-by-step order;
+//    and callers that ask for it keep the step-by-step order (replay_rows, replay_generic);
 //  * the accepted length is read per slot from device memory, so a rollback
 //    does not need the host to know it, and one launch covers all layers.
 #include "dflash_common.h"
@@ -44,7 +44,7 @@ struct ReplayArgs {
   char* conv_out;
   size_t conv_row_bytes;
   int conv_keep, conv_vec16;
-  int replay_blocks;  // slots * Hv
+  int replay_blocks;  // workgroups of the replay itself
 };
 
 // LDS layout (floats): sA[Dv][T] (delta, t contiguous) | sK[T][Dk] | sG[T][Dk or 1] | sGt[Dk]
@@ -203,7 +203,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3, 3))
   const bool g_wide = a.g_dtype == DFLASH_FP32;
   // raw bytes and bits in plain registers; nothing is computed from them until the state has
   // been asked for (see the fence below)
-  typedef __attribute__((ext_vector_type(4))) unsigned int u32x4_t;
   u32x4_t rd0 = {0u, 0u, 0u, 0u}, rd1 = rd0, rk0 = rd0, rk1 = rd0, rg0 = rd0, rg1 = rd0;
   uint32_t mask_t = 1u, mask_g = 1u, g1_bits = 0u;
   {
@@ -325,6 +324,158 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3, 3))
 }
 
 // ---------------------------------------------------------------------------
+// Dk = 64 or 128, T <= 16, one gate per head: a thread keeps 8 consecutive columns of R rows of S in registers from
+// the first step to the last.  STATE = bf16 / fp16: step by step, rounded to that type after every step, three
+// and a half vector instructions per element and step (unpack, product, fma, half a conversion of two).  STATE =
+// fp32: the folded single sweep, for the head sizes the matrix-core kernel above does not have.
+//  * One request of 16 bytes per row and lane; the tape is asked for first, the state right behind it, and nothing
+//    is looked at before all of it is on its way (see replay_f32_128).
+//  * k of a step is read from LDS once for the R rows; a wave's reads of it are 512 consecutive bytes.
+//  * Bound by its vector instructions: 128 x 128 at 16 steps are 3.6 k of them per wave of a head that one workgroup
+//    computes, so a launch of few heads is spread over 32 rows per workgroup (R = 2, 64 x 64 heads: R = 1).
+// Measured against replay_generic, which served these before (one workgroup per head, 2-byte accesses, a division
+// per element), bf16 states, 16 / 6 steps, us: 32 heads of 128 x 128 97.8 / 45.6 -> 5.1 / 3.9, 1536 heads 148 / 69 -> 44 / 21;
+// 32 heads of 64 x 64 26.6 / 13.4 -> 4.0 / 3.2, 1536 heads 39 / 21 -> 12.3 / 7.9.
+// ---------------------------------------------------------------------------
+template <int STATE, int DK, int R>
+__global__ __launch_bounds__(kThreads) void replay_rows(ReplayArgs a) {
+  constexpr bool kWide = STATE == DFLASH_FP32;
+  constexpr int kLanes = DK / 8, kPass = kThreads / kLanes, kRows = kPass * R;  // lanes of a row, rows of a pass, of the workgroup
+  constexpr int kD = kRows / 16, kK = DK / 16;  // elements of delta and k that a thread brings
+  __shared__ __align__(16) float sK[16 * DK];
+  __shared__ __align__(16) float sD[16 * kRows];
+  __shared__ float sG[16];
+  if (conv_window_workgroup(a)) return;
+  const int per = a.Dv / kRows, head = (int)blockIdx.x / per, row0 = ((int)blockIdx.x - head * per) * kRows;
+  const int slot = head / a.Hv, hv = head % a.Hv, hk = hv / (a.Hv / a.Hk);
+  const int n = slot_steps(a, slot);
+  const int tid = threadIdx.x, t = tid >> 4, seg = tid & 15;
+  const size_t slotT = (size_t)slot * a.T;
+
+  // (every row below T exists, accepted or not)
+  uint32_t rd[kD] = {}, rk[kK] = {}, mask_t = 1u, mask_g = 1u, g_bits = 0u;
+  if (t < a.T) {
+    load_bits<kD>(a.tape, ((slotT + t) * a.Hv + hv) * a.Dv + row0 + kD * seg, a.tape_dtype == DFLASH_FP32, rd);
+    load_bits<kK>(a.k, ((slotT + t) * a.Hk + hk) * DK + kK * seg, a.k_dtype == DFLASH_FP32, rk);
+    if (a.mask != nullptr) mask_t = a.mask[slotT + t];
+  }
+  if (tid < a.T) {  // thread t < 16 also fetches the gate of step t
+    const size_t at = (slotT + tid) * a.Hv + hv;
+    if (a.g_dtype == DFLASH_FP32) g_bits = ((const uint32_t*)a.g)[at];
+    else g_bits = ((const uint16_t*)a.g)[at];
+    if (a.mask != nullptr) mask_g = a.mask[slotT + tid];
+  }
+  const int rr = tid / kLanes, c8 = tid % kLanes;
+  const size_t at0 = ((size_t)head * a.Dv + row0 + rr) * DK + 8 * c8;
+  u32x4_t raw[R][kWide ? 2 : 1];
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const size_t at = at0 + (size_t)i * kPass * DK;
+    if (kWide) {
+      const u32x4_t* src = reinterpret_cast<const u32x4_t*>((const float*)a.state_in + at);
+      raw[i][0] = __builtin_nontemporal_load(src);
+      raw[i][kWide ? 1 : 0] = __builtin_nontemporal_load(src + 1);
+    } else {
+      raw[i][0] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>((const uint16_t*)a.state_in + at));
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < kD; ++e) asm volatile("" : "+v"(rd[e])::"memory");
+#pragma unroll
+  for (int e = 0; e < kK; ++e) asm volatile("" : "+v"(rk[e])::"memory");
+  asm volatile("" : "+v"(mask_t), "+v"(mask_g), "+v"(g_bits)::"memory");
+
+  // masked and missing steps are (delta = 0, k = 0, g = 1): no-op steps
+  {
+    const bool keep = t < n && mask_t != 0;
+#pragma unroll
+    for (int e = 0; e < kD; ++e) sD[t * kRows + kD * seg + e] = keep ? bits_element(rd, e, a.tape_dtype) : 0.f;
+#pragma unroll
+    for (int e = 0; e < kK; ++e) sK[t * DK + plane_index<DK>(kK * seg + e)] = keep ? bits_element(rk, e, a.k_dtype) : 0.f;
+    if (tid < 16) {
+      const uint32_t bits[1] = {g_bits};
+      sG[tid] = tid < n && mask_g != 0 ? bits_element(bits, 0, a.g_dtype) : 1.f;
+    }
+  }
+  __syncthreads();
+  float total = 1.f;
+  if (kWide) {  // suffix products of the gates into the k rows
+    for (int s = n - 1; s >= 0; --s) {
+      if (tid < DK) sK[s * DK + tid] *= total;
+      total *= sG[s];
+    }
+    __syncthreads();
+  }
+
+  if constexpr (kWide) {
+    float v[R][8];
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[i][e] = __uint_as_float(raw[i][kWide ? e >> 2 : 0][e & 3]) * total;
+#pragma unroll 2
+    for (int s = 0; s < n; ++s) {
+      float k8[8];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const float4 k4 = *reinterpret_cast<const float4*>(sK + s * DK + h * (DK / 2) + 4 * c8);
+        k8[4 * h] = k4.x, k8[4 * h + 1] = k4.y, k8[4 * h + 2] = k4.z, k8[4 * h + 3] = k4.w;
+      }
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        const float d = sD[s * kRows + i * kPass + rr];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[i][e] = fmaf(d, k8[e], v[i][e]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) raw[i][kWide ? e >> 2 : 0][e & 3] = __float_as_uint(v[i][e]);
+  } else {
+#pragma unroll 2
+    for (int s = 0; s < n; ++s) {
+      float k8[8];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const float4 k4 = *reinterpret_cast<const float4*>(sK + s * DK + h * (DK / 2) + 4 * c8);
+        k8[4 * h] = k4.x, k8[4 * h + 1] = k4.y, k8[4 * h + 2] = k4.z, k8[4 * h + 3] = k4.w;
+      }
+      const float g = sG[s];
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        const float d = sD[s * kRows + i * kPass + rr];
+#pragma unroll
+        for (int p = 0; p < 4; ++p)
+          raw[i][0][p] = pack_pair<STATE>(fmaf(pair_lo<STATE>(raw[i][0][p]), g, k8[2 * p] * d),
+                                          fmaf(pair_hi<STATE>(raw[i][0][p]), g, k8[2 * p + 1] * d));
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const size_t at = at0 + (size_t)i * kPass * DK;
+    if (kWide) {
+      u32x4_t* dst = reinterpret_cast<u32x4_t*>((float*)a.state_out + at);
+      __builtin_nontemporal_store(raw[i][0], dst);
+      __builtin_nontemporal_store(raw[i][kWide ? 1 : 0], dst + 1);
+    } else {
+      __builtin_nontemporal_store(raw[i][0], reinterpret_cast<u32x4_t*>((uint16_t*)a.state_out + at));
+    }
+  }
+}
+
+// The form of replay_rows for a head size and state type; rows: how many a workgroup computes.
+template <int STATE>
+const void* replay_rows_for(int Dk, int Dv, bool many, int* rows) {
+  if (Dk == 128 && many && Dv % 128 == 0) return *rows = 128, (const void*)replay_rows<STATE, 128, 8>;
+  if (Dk == 128 && Dv % 32 == 0) return *rows = 32, (const void*)replay_rows<STATE, 128, 2>;
+  if (Dk == 64 && many && Dv % 64 == 0) return *rows = 64, (const void*)replay_rows<STATE, 64, 2>;
+  if (Dk == 64 && Dv % 32 == 0) return *rows = 32, (const void*)replay_rows<STATE, 64, 1>;
+  return nullptr;
+}
+
+// ---------------------------------------------------------------------------
 // Generic shapes / dtypes.  EXACT = step-by-step order with a round-trip through
 // the state dtype after every step; otherwise the folded single sweep (fp32 state).
 // ---------------------------------------------------------------------------
@@ -422,9 +573,23 @@ int replay_launch(const void* tape, const void* k, const void* g, const void* st
   // the 128 x 128 kernel fetches tape, k and per-element gates 16 bytes at a time
   const bool aligned16 = (((uintptr_t)tape | (uintptr_t)k | (g_per_dk ? (uintptr_t)g : 0)) % 16) == 0;
   const bool fast = !exact && Dk == 128 && Dv == 128 && T <= 16 && aligned16;
+  // 16-bit states step by step and fp32 states of the other head sizes.  A whole head per workgroup from 1024 heads on: k
+  // is staged once for more rows, but at 16 steps fewer waves cover each other's waits (128 x 128, 16 / 6 steps, us, split and
+  // whole: 512 heads 16.0 / 10.0 and 19.3 / 10.3, 1024 heads 28.6 / 16.8 and 31.9 / 15.4, 1536 heads 41.6 / 25.4 and 44.4 / 20.5;
+  // 64 x 64 at 1024 heads 10.6 / 7.2 and 9.6 / 6.1).
+  const void* by_rows = nullptr;
+  int rows = Dv;
+  if (!fast && !g_per_dk && T >= 1 && T <= 16 && aligned16 && (((uintptr_t)state_in | (uintptr_t)state_out) % 16) == 0 &&
+      (!exact || state_dtype != DFLASH_FP32)) {
+    const bool many = (long long)slots * Hv >= 1024;
+    by_rows = state_dtype == DFLASH_BF16   ? replay_rows_for<DFLASH_BF16>(Dk, Dv, many, &rows)
+              : state_dtype == DFLASH_FP16 ? replay_rows_for<DFLASH_FP16>(Dk, Dv, many, &rows)
+                                           : replay_rows_for<DFLASH_FP32>(Dk, Dv, many, &rows);
+  }
   const size_t Tl = fast ? 16 : (size_t)T;
-  const size_t smem_floats = fast ? replay_f32_128_lds_floats(g_per_dk != 0)
-                                  : (size_t)Dv * Tl + Tl * Dk + Tl * (g_per_dk ? Dk : 1) + (size_t)Dk;
+  const size_t smem_floats = by_rows ? 0
+                             : fast  ? replay_f32_128_lds_floats(g_per_dk != 0)
+                                     : (size_t)Dv * Tl + Tl * Dk + Tl * (g_per_dk ? Dk : 1) + (size_t)Dk;
   const size_t smem = smem_floats * sizeof(float);
   DFLASH_REQUIRE(state_dtype != DFLASH_FP32 ||
                      (((uintptr_t)state_in % 16) == 0 && ((uintptr_t)state_out % 16) == 0),
@@ -441,7 +606,9 @@ int replay_launch(const void* tape, const void* k, const void* g, const void* st
   a.T = T; a.Hk = Hk; a.Hv = Hv; a.Dk = Dk; a.Dv = Dv;
   a.state_dtype = state_dtype; a.tape_dtype = tape_dtype; a.k_dtype = k_dtype;
   a.g_dtype = g_dtype; a.g_per_dk = g_per_dk ? 1 : 0;
-  a.replay_blocks = slots * Hv;
+  const long long blocks = (long long)slots * Hv * (by_rows ? Dv / rows : 1);
+  DFLASH_REQUIRE(blocks < (1ll << 31), DFLASH_ERR_SHAPE, "dflash_tape_replay: too many workgroups");
+  a.replay_blocks = (int)blocks;
   a.conv_prev = a.conv_qkv = nullptr; a.conv_out = nullptr; a.conv_row_bytes = 0; a.conv_keep = a.conv_vec16 = 0;
   long long conv_blocks = 0;
   if (qkv != nullptr) {
@@ -455,12 +622,17 @@ int replay_launch(const void* tape, const void* k, const void* g, const void* st
     a.conv_vec16 = a.conv_row_bytes % 16 == 0 && (uintptr_t)qkv % 16 == 0 && (uintptr_t)conv_out % 16 == 0 &&
                    (uintptr_t)conv_prev % 16 == 0;
     conv_blocks = (long long)slots * keep;
-    DFLASH_REQUIRE((long long)slots * Hv + conv_blocks < (1ll << 31), DFLASH_ERR_SHAPE,
+    DFLASH_REQUIRE(blocks + conv_blocks < (1ll << 31), DFLASH_ERR_SHAPE,
                    "dflash_rollback_layer: too many workgroups");
   }
 
-  const dim3 grid((unsigned)(slots * Hv + conv_blocks)), block(kThreads);
+  const dim3 grid((unsigned)(blocks + conv_blocks)), block(kThreads);
   hipStream_t s = (hipStream_t)stream;
+  if (by_rows != nullptr) {
+    void* args[] = {&a};
+    DFLASH_HIP_OK(hipLaunchKernel(by_rows, grid, block, args, 0, s));
+    return DFLASH_OK;
+  }
   if (exact) {
     hipLaunchKernelGGL(replay_generic<true>, grid, block, smem, s, a);
   } else if (fast) {

@@ -411,3 +411,34 @@ def test_arena_takes_per_batch_row_acceptance_and_other_tape_dtypes(native_lib):
         for l, c in enumerate(caches):
             c.record_tape(tape=case.tape[l].to(DEV), k=case.k[l].to(DEV), g=case.g[l].to(DEV), qkv=qkv[l].to(DEV))
         arena.rollback_all(torch.zeros(5, dtype=torch.int32, device=DEV))
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("Dk,Dv,layers,T", [(128, 32, 2, 16), (128, 96, 1, 5), (128, 128, 3, 16), (128, 128, 130, 16), (64, 32, 2, 16),
+                                            (64, 64, 3, 1), (64, 192, 2, 16), (64, 64, 130, 9)])
+def test_states_held_in_registers(native_lib, dt, Dk, Dv, layers, T):
+    """The kernel that keeps 16-bit states (and fp32 ones of other head sizes than 128 x 128) in registers, few and many
+    heads, with a mask and per-slot lengths: 16-bit states bit for bit what the walk through memory gives, which
+    serves the same call when an operand does not start on 16 bytes; fp32 states against the oracle."""
+    case = make_replay_case(layers, batch=2, T=T, Hk=2, Hv=4, Dk=Dk, Dv=Dv, steps=T, seed=Dk + Dv + T, tape_dtype=torch.float32)
+    case.state = case.state.to(dt)
+    slots = 2 * layers
+    rng = np.random.default_rng(T)
+    mask = rng.integers(0, 4, (slots, T)) > 0
+    steps = torch.from_numpy(rng.integers(0, T + 1, slots).astype(np.int32))
+    steps[0], steps[-1] = 0, T
+    for m in (None, mask):
+        out = _launch(case, steps, mask=m)
+        assert out.dtype == dt
+        if dt == torch.float32:
+            want = _oracle_slots(case, steps.numpy(), m)
+            for s in range(slots):
+                assert _rel_l2(_np(out).reshape(slots, -1)[s], want.reshape(slots, -1)[s]) <= TOL, (s, m is not None)
+            continue
+        d = case.to(DEV)
+        apart = torch.empty(d.k.numel() + 1, dtype=d.k.dtype, device=DEV)[1:].view(d.k.shape)  # starts on its second element
+        apart.copy_(d.k)
+        walked = torch.empty_like(d.state)
+        mm = None if m is None else torch.from_numpy(m.astype(np.uint8)).to(DEV)
+        replay_launch(d.tape, apart, d.g, d.state, walked, steps=steps.to(DEV), T_alloc=T, mask=mm, slots=slots)
+        assert torch.equal(out, walked)
