@@ -270,6 +270,195 @@ __global__ __launch_bounds__(kThreads) void gdn_forward_128(GdnArgs a) {
 }
 
 // ---------------------------------------------------------------------------
+// Dk = 64 or 128, one gate per head, step by step: 16-bit states (which are rounded after every step, so the closed
+// form below does not apply) and fp32 states of the head sizes the other kernels do not have.
+//  * Rows of S are independent, and a step is a chain (two sums over dk, then the update): what bounds a
+//    call of few heads is that chain, so a head is spread over workgroups of 16 R (Dk = 64: 32 R) rows.  A lane
+//    holds 8 columns of R rows, a row is 16 (8) neighbouring lanes, its sums are four (three) DPP steps.
+//  * k and q of the next step are read from LDS (planes of four, see plane_index) while the present one computes; tape
+//    and y leave through LDS, 16 steps at a time.
+// Measured against one workgroup per head with 2-byte accesses and the types sorted out per element, bf16 states,
+// 16 steps / 1 step, us: 32 heads of 128 x 128 73.9 / 21.7 -> 7.6 / 3.9, 1024 heads 184 / 53 -> 69 / 19; of 64 x 64, whose
+// state went through memory at every step, 913 / 77.7 -> 6.8 / 3.4 and 1158 / 105 -> 21 / 5.9.
+// ---------------------------------------------------------------------------
+template <int STATE, int DK, int R>
+__global__ __launch_bounds__(kThreads) void gdn_forward_rows(GdnArgs a) {
+  constexpr bool kWide = STATE == DFLASH_FP32;
+  constexpr int kLanes = DK / 8, kPass = kThreads / kLanes, kRows = kPass * R;  // lanes of a row, rows of a pass, of the workgroup
+  constexpr int kD = kRows / 16, kK = DK / 16;  // elements of v and of k, q that a thread brings
+  __shared__ __align__(16) float sQ[16 * DK];
+  __shared__ __align__(16) float sK[16 * DK];
+  __shared__ __align__(16) float sV[16 * kRows];  // v, then (row by row, once it has been read) the tape
+  __shared__ __align__(16) float sY[16 * kRows];
+  __shared__ __align__(16) float sS[16 * 4];      // gate, beta, k . q of a step
+  const int per = a.Dv / kRows, head = (int)blockIdx.x / per, row0 = ((int)blockIdx.x - head * per) * kRows;
+  const int slot = head / a.Hv, hv = head % a.Hv, hk = hv / (a.Hv / a.Hk);
+  const int tid = threadIdx.x, t16 = tid >> 4, seg = tid & 15;
+  const int rr = tid / kLanes, c8 = tid % kLanes;
+  const bool wide = a.in_dtype == DFLASH_FP32;
+
+  const size_t at0 = ((size_t)head * a.Dv + row0 + rr) * DK + 8 * c8;
+  u32x4_t raw[R][kWide ? 2 : 1];
+  float st[R][8];
+  for (int first = 0; first < a.T; first += 16) {
+    const int T = a.T - first < 16 ? a.T - first : 16;
+    const size_t slotT = (size_t)slot * a.T + first;
+    // the block's operands first, the state behind them, nothing looked at before all of it is on its way
+    uint32_t rq[kK] = {}, rk[kK] = {}, rv[kD] = {}, g_bits = 0u, beta_bits = 0u;
+    if (t16 < T) {
+      load_bits<kK>(a.q, ((slotT + t16) * a.Hk + hk) * DK + kK * seg, wide, rq);
+      load_bits<kK>(a.k, ((slotT + t16) * a.Hk + hk) * DK + kK * seg, wide, rk);
+      load_bits<kD>(a.v, ((slotT + t16) * a.Hv + hv) * a.Dv + row0 + kD * seg, wide, rv);
+    }
+    if (tid < T) {
+      const size_t at = (slotT + tid) * a.Hv + hv;
+      if (a.g_dtype == DFLASH_FP32) g_bits = ((const uint32_t*)a.g)[at];
+      else g_bits = ((const uint16_t*)a.g)[at];
+      if (a.beta_dtype == DFLASH_FP32) beta_bits = ((const uint32_t*)a.beta)[at];
+      else beta_bits = ((const uint16_t*)a.beta)[at];
+    }
+    if (first == 0) {
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        const size_t at = at0 + (size_t)i * kPass * DK;
+        if (kWide) {
+          const u32x4_t* src = reinterpret_cast<const u32x4_t*>((const float*)a.state_in + at);
+          raw[i][0] = __builtin_nontemporal_load(src);
+          raw[i][kWide ? 1 : 0] = __builtin_nontemporal_load(src + 1);
+        } else {
+          raw[i][0] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>((const uint16_t*)a.state_in + at));
+        }
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < kK; ++e) asm volatile("" : "+v"(rq[e]), "+v"(rk[e])::"memory");
+#pragma unroll
+    for (int e = 0; e < kD; ++e) asm volatile("" : "+v"(rv[e])::"memory");
+    asm volatile("" : "+v"(g_bits), "+v"(beta_bits)::"memory");
+    float kq = 0.f;  // k . q of step t16: 16 lanes, kK products each
+#pragma unroll
+    for (int e = 0; e < kK; ++e) {
+      const float q = bits_element(rq, e, a.in_dtype), k = bits_element(rk, e, a.in_dtype);
+      sQ[t16 * DK + plane_index<DK>(kK * seg + e)] = q;
+      sK[t16 * DK + plane_index<DK>(kK * seg + e)] = k;
+      kq = fmaf(k, q, kq);
+    }
+    kq = sum_over_16(kq);
+    if (seg == 0) sS[4 * t16 + 2] = kq;
+#pragma unroll
+    for (int e = 0; e < kD; ++e) sV[t16 * kRows + kD * seg + e] = bits_element(rv, e, a.in_dtype);
+    if (tid < 16) {
+      const uint32_t g1[1] = {g_bits}, b1[1] = {beta_bits};
+      sS[4 * tid] = bits_element(g1, 0, a.g_dtype);
+      sS[4 * tid + 1] = bits_element(b1, 0, a.beta_dtype);
+    }
+    if (first == 0) {
+#pragma unroll
+      for (int i = 0; i < R; ++i)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          if constexpr (kWide) st[i][e] = __uint_as_float(raw[i][kWide ? e >> 2 : 0][e & 3]);
+          else st[i][e] = e & 1 ? pair_hi<STATE>(raw[i][0][e >> 1]) : pair_lo<STATE>(raw[i][0][e >> 1]);
+        }
+    }
+    __syncthreads();
+
+    f32x4_t k4[2], q4[2], s4;
+    float v[R];
+    auto fetch = [&](int t) __attribute__((always_inline)) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        k4[h] = *reinterpret_cast<const f32x4_t*>(sK + t * DK + h * (DK / 2) + 4 * c8);
+        q4[h] = *reinterpret_cast<const f32x4_t*>(sQ + t * DK + h * (DK / 2) + 4 * c8);
+      }
+      s4 = *reinterpret_cast<const f32x4_t*>(sS + 4 * t);
+#pragma unroll
+      for (int i = 0; i < R; ++i) v[i] = sV[t * kRows + i * kPass + rr];
+    };
+    fetch(0);
+    for (int t = 0; t < T; ++t) {
+      float kk[8], qq[8], vv[R], delta[R], y[R];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) kk[e] = k4[e >> 2][e & 3], qq[e] = q4[e >> 2][e & 3];
+      const float g = s4[0], beta = s4[1], kdotq = s4[2];
+#pragma unroll
+      for (int i = 0; i < R; ++i) vv[i] = v[i], delta[i] = y[i] = 0.f;
+      fetch(t + 1 < T ? t + 1 : t);
+      if (a.mask == nullptr || a.mask[slotT + t] != 0) {
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+          float pk[2] = {0.f, 0.f}, pq[2] = {0.f, 0.f};
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            st[i][e] *= g;
+            pk[e & 1] = fmaf(st[i][e], kk[e], pk[e & 1]);
+            pq[e & 1] = fmaf(st[i][e], qq[e], pq[e & 1]);
+          }
+          const float sk = pk[0] + pk[1], sq = pq[0] + pq[1];
+          delta[i] = (vv[i] - (kLanes == 16 ? sum_over_16(sk) : sum_over_8(sk))) * beta;
+          y[i] = fmaf(kdotq, delta[i], kLanes == 16 ? sum_over_16(sq) : sum_over_8(sq));
+#pragma unroll
+          for (int e = 0; e < 8; ++e) st[i][e] = fmaf(kk[e], delta[i], st[i][e]);
+          if constexpr (!kWide) {
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+              const uint32_t w = pack_pair<STATE>(st[i][2 * p], st[i][2 * p + 1]);
+              st[i][2 * p] = pair_lo<STATE>(w), st[i][2 * p + 1] = pair_hi<STATE>(w);
+            }
+          }
+        }
+      }
+      if (c8 == 0) {  // (nobody else reads these elements of v, and this wave has)
+#pragma unroll
+        for (int i = 0; i < R; ++i) sV[t * kRows + i * kPass + rr] = delta[i], sY[t * kRows + i * kPass + rr] = y[i];
+      }
+    }
+    __syncthreads();
+    if (t16 < T) {
+      const size_t o = ((slotT + t16) * a.Hv + hv) * a.Dv + row0 + kD * seg;
+      float d[kD], y[kD];
+#pragma unroll
+      for (int e = 0; e < kD; ++e) d[e] = sV[t16 * kRows + kD * seg + e], y[e] = sY[t16 * kRows + kD * seg + e];
+      __builtin_memcpy(__builtin_assume_aligned(a.tape + o, kD < 4 ? 4 * kD : 16), d, 4 * kD);
+      if (wide) {
+        __builtin_memcpy(__builtin_assume_aligned((float*)a.y + o, kD < 4 ? 4 * kD : 16), y, 4 * kD);
+      } else {
+        uint16_t h[kD];
+#pragma unroll
+        for (int e = 0; e < kD; ++e) h[e] = (uint16_t)(a.in_dtype == DFLASH_BF16 ? f32_to_bf16_bits(y[e]) : f32_to_f16_bits(y[e]));
+        __builtin_memcpy(__builtin_assume_aligned((uint16_t*)a.y + o, kD < 8 ? 2 * kD : 16), h, 2 * kD);
+      }
+    }
+    if (first + 16 < a.T) __syncthreads();  // the next block is staged where this one's results are read
+  }
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const size_t at = at0 + (size_t)i * kPass * DK;
+    if constexpr (kWide) {
+      f32x4_t* dst = reinterpret_cast<f32x4_t*>((float*)a.state_out + at);
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        __builtin_nontemporal_store(f32x4_t{st[i][4 * h], st[i][4 * h + 1], st[i][4 * h + 2], st[i][4 * h + 3]}, dst + h);
+    } else {
+      u32x4_t w;
+#pragma unroll
+      for (int p = 0; p < 4; ++p) w[p] = pack_pair<STATE>(st[i][2 * p], st[i][2 * p + 1]);  // (exact: rounded already)
+      __builtin_nontemporal_store(w, reinterpret_cast<u32x4_t*>((uint16_t*)a.state_out + at));
+    }
+  }
+}
+
+// The form of gdn_forward_rows for a head size and state type; rows: how many a workgroup computes.
+template <int STATE>
+const void* forward_rows_for(int Dk, int Dv, bool many, int* rows) {
+  if (Dk == 128 && many && Dv % 32 == 0) return *rows = 32, (const void*)gdn_forward_rows<STATE, 128, 2>;
+  if (Dk == 128 && Dv % 16 == 0) return *rows = 16, (const void*)gdn_forward_rows<STATE, 128, 1>;
+  if (Dk == 64 && many && Dv % 64 == 0) return *rows = 64, (const void*)gdn_forward_rows<STATE, 64, 2>;
+  if (Dk == 64 && Dv % 32 == 0) return *rows = 32, (const void*)gdn_forward_rows<STATE, 64, 1>;
+  return nullptr;
+}
+
+// ---------------------------------------------------------------------------
 // Dk = Dv = 128, T <= 16, one gate per head, fp32 state: the block in closed form.
 // With c_t = prod_{u<=t} g_u (masked steps: g = 1, beta = 0) the recurrence unrolls to
 //     kv_t    = c_t (S0 k_t) + sum_{s<t}  (c_t/c_s) (k_s.k_t) delta_s
@@ -748,7 +937,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3, 3))
 // ---------------------------------------------------------------------------
 // Any Dk, Dv: one workgroup per (slot, head), a thread walks whole rows of S, which lives in
 // state_out between steps (so it is rounded through the state dtype after every step by
-// construction).  Slow and simple; the 128 x 128 kernel above is the one that is measured.
+// construction).  Slow and simple; the kernels above have the head sizes of the models served.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(kThreads) void gdn_forward_generic(GdnArgs a) {
   const int slot = blockIdx.x / a.Hv, hv = blockIdx.x % a.Hv;
@@ -846,6 +1035,19 @@ int gdn_forward_launch(const char* who, const void* q, const void* k, const void
                     (state_dtype != DFLASH_FP32 ||
                      (((uintptr_t)state_in % 16) == 0 && ((uintptr_t)state_out % 16) == 0));
   const bool chunk = fast && !g_per_dk && state_dtype == DFLASH_FP32 && T <= 16 && aligned16 && !no_chunk;
+  // Step by step in registers.  Two rows per lane, which share the reads of k and q, from 32 K rows on (128 x 128 at 16
+  // steps, us, one and two rows: 96 heads 11.3 and 12.9, 256 heads 23.7 and 21.5, 1024 heads 77 and 69; 64 x 64, 512 heads 12.9 and 13.2,
+  // 1024 heads 22.3 and 21.2).
+  const void* by_rows = nullptr;
+  int rows = Dv;
+  if (!prompt && !chunk && !g_per_dk && T >= 1 && aligned16 && (((uintptr_t)state_in | (uintptr_t)state_out) % 16) == 0 &&
+      !(fast && state_dtype == DFLASH_FP32)) {
+    const bool many = (long long)slots * Hv * Dv >= 32768;
+    by_rows = state_dtype == DFLASH_BF16   ? forward_rows_for<DFLASH_BF16>(Dk, Dv, many, &rows)
+              : state_dtype == DFLASH_FP16 ? forward_rows_for<DFLASH_FP16>(Dk, Dv, many, &rows)
+                                           : forward_rows_for<DFLASH_FP32>(Dk, Dv, many, &rows);
+    if ((long long)slots * Hv * (Dv / rows) >= (1ll << 31)) by_rows = nullptr;
+  }
   bool norm_done = false;
   if (prompt) {
     const size_t need = gdn_prompt_workspace_bytes(slots, T, Hk, Hv, Dk);
@@ -868,6 +1070,9 @@ int gdn_forward_launch(const char* who, const void* q, const void* k, const void
       else if (split) hipLaunchKernelGGL((gdn_forward_chunk_128<false, false, true>), grid, block, lds, s, a);
       else hipLaunchKernelGGL((gdn_forward_chunk_128<false, false, false>), grid, block, lds, s, a);
     }
+  } else if (by_rows != nullptr) {
+    void* args[] = {&a};
+    DFLASH_HIP_OK(hipLaunchKernel(by_rows, dim3((unsigned)(slots * Hv * (Dv / rows))), block, args, 0, s));
   } else if (fast) {
     if (g_per_dk) {
       hipLaunchKernelGGL((gdn_forward_128<true, false>), grid, block, smem, s, a);

@@ -404,3 +404,33 @@ def test_magnitudes_whose_products_leave_the_range_of_fp32(native_lib):
     _same_values(y[1], yo[1], 4e-3)
     _same_values(tape[1], to[1], 2e-5)
     _same_values(s[1], so[1], 2e-5)
+
+
+@pytest.mark.parametrize("state_dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("B,T,Hk,Hv,Dk,Dv,dtype", [(1, 1, 2, 4, 128, 128, torch.bfloat16), (2, 16, 2, 4, 128, 48, torch.bfloat16),
+                                                   (9, 7, 8, 16, 128, 128, torch.bfloat16), (1, 16, 4, 8, 64, 64, torch.bfloat16),
+                                                   (1, 33, 1, 2, 64, 96, torch.float16), (9, 16, 16, 32, 64, 64, torch.float32),
+                                                   (2, 17, 2, 2, 128, 64, torch.float32)])
+def test_rows_of_the_state_in_registers(native_lib, state_dtype, B, T, Hk, Hv, Dk, Dv, dtype):
+    """The kernel that spreads a head over workgroups of some of its rows: one and two rows per lane, blocks of 16
+    steps and what is left of them, masked steps; against the recurrence in fp64 with the state rounded after every step."""
+    args = _case(B=B, T=T, Hk=Hk, Hv=Hv, Dk=Dk, Dv=Dv, seed=B + T + Dk + Dv, dtype=dtype, state_dtype=state_dtype)
+    q, k, v, gate, beta, state = (t.double() for t in args)
+    mask = torch.rand((B, T), generator=torch.Generator().manual_seed(T)) > 0.25
+    mask[0, -1] = True
+    for m in (None, mask):
+        y, s, tape = _run(args, m)
+        assert s.dtype == state_dtype and y.dtype == dtype
+        S, ys, tapes = state, [], []
+        for t in range(T):
+            yt, S, tp = _gated_delta_ops_with_tape(q[:, t:t + 1], k[:, t:t + 1], v[:, t:t + 1], gate[:, t:t + 1], beta[:, t:t + 1], S,
+                                                   None if m is None else m[:, t:t + 1])
+            S = S.to(state_dtype).double()
+            ys.append(yt)
+            tapes.append(tp)
+        # one unit of a 16-bit state here and there (as for whole heads above); y is rounded to its own type
+        tol = 2e-5 if state_dtype == torch.float32 else 2e-3
+        tol_y = max(tol, {torch.bfloat16: 4e-3, torch.float16: 5e-4, torch.float32: 0.0}[dtype])
+        assert _rel(_f64(s), _f64(S)) <= tol
+        assert _rel(_f64(tape), _f64(torch.cat(tapes, dim=1))) <= tol
+        assert _rel(_f64(y), _f64(torch.cat(ys, dim=1))) <= tol_y
