@@ -5,44 +5,44 @@
 // dequantised to the activation type as the array-op form of this package does it (s*q + b in
 // fp32, rounded once) and multiplied on the matrix cores with fp32 accumulation.
 //
-//  * A wave owns whole columns: a workgroup is 4 waves side by side, each 16*NT columns wide and all
-//    16*MT rows high, so that a weight is dequantised once per 16*MT rows.  With KG = 2 a second
-//    set of four waves takes the other half of every stage of K and the two halves meet in LDS
-//    at the end: two waves per SIMD, so that one dequantises while the other multiplies, without
-//    cutting the result any smaller.
-//  * Codes, scales and x all go through LDS.  Read by the lanes that multiply them, neighbouring lanes would
-//    ask for different rows, and a load that touches 16 or 64 rows costs the address unit 64 cycles
-//    instead of 16: that, not arithmetic, bounded the form of this kernel that kept codes in
-//    registers (4 + 8 such loads per 64 k and wave, 3072 cycles of address work per 1024 cycles of
-//    matrix work).  Loads go to registers at the start of a stage and to the other LDS buffer at its end.
+//  * A wave owns whole columns: W waves side by side, each 32*NT columns wide and all 32*MT rows high, so that a
+//    weight is dequantised once per 32*MT rows.  KG sets of such waves take 64 k of every stage each and add
+//    their sums up through LDS at the end: eight waves on a CU without cutting the result any smaller.
+//  * Matrix instructions of 32 x 32 x 16.  One takes the issue port of its SIMD for 8 cycles and the matrix pipe for
+//    32 (16 x 16 x 32: 8 and 16, for half the work), and a vector instruction takes the port for 4: six of them hide beside a large
+//    one, two beside a small one (measured: 33.9 and 42.7 cycles with 6 and 8 beside a large one; 17.4, 21.8 and 25.7 with 2, 3 and 4
+//    beside a small one).  Dequantisation is 5 to 6 for MT = 4.  The order of instructions is spelled out per step
+//    of 16 k: a few vector instructions behind each matrix instruction.
+//  * x and codes go from memory to LDS past the registers: a write of 16 bytes per lane takes the LDS 14 cycles, a read 4,
+//    and the form of this kernel that loaded to registers spent an eighth of its time on the writes.  Lane i of a request lands
+//    at 16 i, so the places that keep reads free of bank conflicts are made by what each lane asks for.  A read of 16
+//    bytes per lane serves lanes {0-3, 12-15, 20-23, 24-27} together, then {4-7, 8-11, 16-19, 28-31} and so on.
 //  * dequantisation: code q sits in the low bits of a half word; as an fp16 subnormal that half is
 //    q 2^-24, so fma_mix(half, s 2^24, b) is s q + b in one instruction and exact up to its one
 //    rounding; the conversion to the activation type packs two at a time: 19 vector instructions per
-//    8 weights, 60 % of the matrix instructions' time at MT = 8.
+//    8 weights.
 //  * W is the A operand (rows of the tile = columns of y), x the B operand, and the columns of a
-//    wave are dealt to its tiles so that a lane ends up with 4*NT consecutive columns of one row.
+//    tile are dealt so that a lane ends up with 16 consecutive columns of one row.
 //  * Where the tiles do not fill the chip, K is cut into slices: workgroups leave fp32 partial tiles in
 //    the workspace, and whoever arrives last at a tile adds them in order of k.  Nobody waits.  Deterministic.
-//    Of more tiles than the chip takes at once, only those of the last, incomplete round are cut: 1088 tiles of
-//    5120 x 34816 are 4 rounds and a quarter instead of 5 (a 27B layer over 1024 tokens 787 -> 758 us).
+//    Of more tiles than the chip takes at once, only those of the last, incomplete round are cut.
 //
-// Measured (kernel time, group 64, before that cut): 1024 rows of 5120 x 34816 415 us (880 TFLOP/s; torch's bf16 product of weights
-// that are already dense 411 us), 17408 x 5120 204 us (237), 5120 x 5120 71 us (62); 77 rows of
-// 4096 x 24576 42 us, 12288 x 4096 22 us.  The form with codes in registers took 540, 260, 105 and 87, 31 us for
-// the same tiles.  What bounds it at many rows is shared (counters, the first of these shapes with the
-// activation): matrix instructions 42 % of the SIMDs' cycles, other vector instructions 38 %, the LDS busy for 50 % - half of that
-// bank conflicts - at 1.9 of 2.4 GHz (power); with no dequantisation at all the same loop is 20 % faster.
-// At few rows it is latency - two memory round trips before the first product and one for the slices, a third of the
-// waves' time - and the LDS: 77 rows of 4096 x 24576 matrix 24 %, vector 37 %, LDS 51 %.
-// The activation's exponential is expf as in its other forms; 64 of them per lane behind the last stage cost 1 %.
+// Measured (us, group 64; before: 16 x 16 x 32 instructions, loads to registers): 1024 rows of 5120 x 34816 with the
+// activation 398 -> 344 (1.06 PFLOP/s), 17408 x 5120 207 -> 184, 5120 x 12352 164 -> 134; 200 rows of 4096 x 4096 22.6 -> 17.5; 77 rows
+// of 4096 x 24576 with the activation 36.4 -> 30.8, 12288 x 4096 24.9 -> 21.2; 20 rows of 5120 x 12352 21.4 -> 18.4, of 2048 x 2048 7.1 -> 7.4.
+// What bounds it at many rows: the matrix pipes are busy for 60 to 66 % of the cycles at 2.0 to 2.1 of 2.4 GHz (power); with no requests
+// to memory at all the same loop is 15 to 20 % faster, with no dequantisation on top 2 to 10 %.  At few rows:
+// 3300 cycles of setup, requests and their latency before the first product, 1500 a stage of (1,1,2,4), where four dependent steps take 1050 and
+// the barrier the rest, and 5000 and more for the slices.
 #include "dflash_common.h"
+
 #include "qmm_stream_device.h"
+#include <algorithm>
 
 namespace dflash {
 namespace rows {
 
-constexpr int kWaves = 4;      // side by side
-constexpr int kStageK = 64;    // k per stage and set of waves
+constexpr int kStageK = 64;  // k per stage and set of waves
 
 struct Args {
   const uint16_t* x;
@@ -76,48 +76,73 @@ __device__ __forceinline__ float code_fma(uint32_t pair, int hi, float s24, floa
   const f16x2_t h = __builtin_bit_cast(f16x2_t, pair);
   return __builtin_fmaf((float)h[hi], s24, b);
 }
-// eight codes of one word (k ascending from the low nibble) -> eight values of the activation type; s24 and s20
+// Codes 2 p and 2 p + 1 of one word (k ascending from the low nibble) -> two values of the activation type; s24 and s20
 // are the scale times 2^24 and 2^20 (a code in bits 4 .. 7 of a half word is 16 times one in bits 0 .. 3)
 template <bool FP16>
+__device__ __forceinline__ uint32_t dequant2(uint32_t w, int p, float s24, float s20, float b, uint32_t mask0, uint32_t mask4) {
+  const uint32_t v = p & 1 ? w >> 8 : w;  // halves (k0, k4), (k1, k5) or (k2, k6), (k3, k7)
+  return pack2<FP16>(code_fma(v & mask0, p >> 1, s24, b), code_fma(v & mask4, p >> 1, s20, b));
+}
+template <bool FP16>
 __device__ __forceinline__ uint4 dequant8(uint32_t w, float s24, float s20, float b, uint32_t mask0, uint32_t mask4) {
-  const uint32_t w8 = w >> 8;
-  const uint32_t p0 = w & mask0, p1 = w & mask4, p2 = w8 & mask0, p3 = w8 & mask4;  // (k0,k4) (k1,k5) ..
-  uint4 r;
-  r.x = pack2<FP16>(code_fma(p0, 0, s24, b), code_fma(p1, 0, s20, b));
-  r.y = pack2<FP16>(code_fma(p2, 0, s24, b), code_fma(p3, 0, s20, b));
-  r.z = pack2<FP16>(code_fma(p0, 1, s24, b), code_fma(p1, 1, s20, b));
-  r.w = pack2<FP16>(code_fma(p2, 1, s24, b), code_fma(p3, 1, s20, b));
-  return r;
+  return make_uint4(dequant2<FP16>(w, 0, s24, s20, b, mask0, mask4), dequant2<FP16>(w, 1, s24, s20, b, mask0, mask4),
+                    dequant2<FP16>(w, 2, s24, s20, b, mask0, mask4), dequant2<FP16>(w, 3, s24, s20, b, mask0, mask4));
 }
 template <bool FP16>
 __device__ __forceinline__ float sb_value(uint32_t h) {
   return FP16 ? f16_bits_to_f32(h) : bf16_bits_to_f32(h);
 }
 
-// KG: sets of four waves, each with its 64 k of a stage.
-// SILU_MUL: W holds the gate rows and, behind them, the up rows of an MLP, y[M, N / 2] is silu(gate) * up with every
-// operator's rounding to the activation type.  Half of a wave's tiles are gate columns, the others the up
-// columns of the same lanes.
-template <bool FP16, bool SB_FP16, int MT, int NT, int KG, bool SILU_MUL>
-__global__ __launch_bounds__(256 * KG, 2) void qmm_rows_kernel(Args a) {
-  using A = stream::Act<FP16>;
-  constexpr int kThreads = 256 * KG;
-  constexpr int BM = 16 * MT, BN = kWaves * 16 * NT;
-  constexpr int kXBytes = KG * BM * 128, kWBytes = KG * BN * 32;
-  constexpr int kFrontBytes = 2 * kXBytes + 3 * kWBytes;
-  constexpr int kSbBytes = 2 * BN * 16;  // scales and biases of eight groups
-  constexpr int kXRows = kThreads / (8 * KG), XL = (BM + kXRows - 1) / kXRows;  // 16-byte pieces of x per thread
-  constexpr int kWRows = kThreads / (2 * KG), WL = (BN + kWRows - 1) / kWRows;  // ... of codes
-  constexpr int SL = (2 * BN + kThreads - 1) / kThreads;                        // ... of scales and biases
-  extern __shared__ __attribute__((aligned(1024))) char lds[];  // x of 2 stages, codes of 3, 2 chunks of scales and biases
-  __shared__ uint32_t s_last;
-  char* const w_lds = lds + 2 * kXBytes;
-  char* const sb_lds = lds + kFrontBytes;
+typedef __attribute__((ext_vector_type(16))) float f32x16_t;
 
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane((tid >> 6) & 3);
-  const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
-  const int li = lane & 15, kq = lane >> 4;
+template <bool FP16>
+__device__ __forceinline__ f32x16_t mfma32(uint4 w, uint4 x, f32x16_t c) {
+  if constexpr (FP16) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, w), __builtin_bit_cast(f16x8_t, x), c, 0, 0, 0);
+  } else {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, w), __builtin_bit_cast(bf16x8_t, x), c, 0, 0, 0);
+  }
+}
+
+// Lane i of the wave: 16 bytes from rsrc + voff + soff to LDS at lds + 16 i, past the registers.  The compiler counts neither the
+// request nor what it writes: whoever reads that place waits with stage_done() first.
+__device__ __forceinline__ void request16(__amdgpu_buffer_rsrc_t rsrc, uint32_t lds, uint32_t voff, uint32_t soff) {
+  asm volatile("s_mov_b32 m0, %0\n s_nop 0\n buffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "m0");
+}
+// All but the last LEFT requests of this wave have landed, its writes to LDS are done, and so have and are every other wave's.
+template <int LEFT>
+__device__ __forceinline__ void stage_done() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n s_barrier" ::"n"(LEFT) : "memory");
+}
+
+template <int MT, int NT, int W, int KG>
+struct Tile {
+  static constexpr int kThreads = 64 * W * KG, BM = 32 * MT, BN = 32 * NT * W;
+  static constexpr int kGroups = KG < 4 ? 8 : 4 * KG;  // whose scales and biases are brought at a time: two stages at least
+  static constexpr int kXBytes = KG * BM * 128, kWBytes = KG * BN * 32, kSbBytes = 4 * BN * kGroups;
+  static constexpr int kXBufs = 2, kWBufs = 3;  // (a third buffer of x changes nothing: 17408 x 5120 over 1024 rows 201 and 203 us)
+  static constexpr int kFrontBytes = kXBufs * kXBytes + kWBufs * kWBytes;
+  static constexpr int kLdsBytes = kFrontBytes + 2 * kSbBytes;
+};
+
+// KG: sets of W waves, each with its 64 k of a stage.
+// SILU_MUL: W holds the gate rows and, behind them, the up rows of an MLP, y[M, N / 2] is silu(gate) * up with every
+// operator's rounding to the activation type.  A wave's first tile is gate columns, its second the up columns of the same lanes.
+template <bool FP16, bool SB_FP16, int MT, int NT, int W, int KG, bool SILU_MUL>
+__global__ __launch_bounds__(64 * W * KG, 2) void qmm_rows_kernel(Args a) {
+  using T = Tile<MT, NT, W, KG>;
+  constexpr int BM = T::BM, BN = T::BN, kThreads = T::kThreads, kSet = 64 * W, kGroups = T::kGroups;
+  constexpr int XB = T::kXBufs, WB = T::kWBufs;
+  constexpr int kXReq = BM / (8 * W), kWReq = NT;  // requests of a wave for a stage: 8 rows of x, 64 / (2 KG) rows of codes each
+  static_assert(BM % (8 * W) == 0 && (!SILU_MUL || NT == 2), "whole requests; gate and up tiles come in pairs");
+  extern __shared__ __attribute__((aligned(1024))) char lds[];  // x [buffer][set][row] 128 bytes, codes [buffer][row] 32 KG bytes, scales and biases [2]
+  char* const w_lds = lds + XB * T::kXBytes;
+  char* const sb_lds = lds + T::kFrontBytes;
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane(stream::lds_address(lds));
+
+  const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, kq = lane >> 5;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = wid % W, kg = wid / W;
   // neighbours in tile order (same columns, other rows) behind one L2; the whole tiles are dispatched first
   const bool cut = (int)blockIdx.x >= a.whole;
   const int part = cut ? (int)gridDim.x - a.whole : a.whole, at = (int)blockIdx.x - (cut ? a.whole : 0);
@@ -130,340 +155,396 @@ __global__ __launch_bounds__(256 * KG, 2) void qmm_rows_kernel(Args a) {
   const int G = a.K >> a.group_shift;
   uint32_t mask0 = 0x000F000Fu, mask4 = 0x00F000F0u;
   asm volatile("" : "+s"(mask0), "+s"(mask4));
-
-  constexpr int kTiles = SILU_MUL ? NT / 2 : NT;  // tiles of output columns per wave
-  static_assert(!SILU_MUL || NT % 2 == 0, "gate and up tiles come in pairs");
   const int out_cols = SILU_MUL ? a.N / 2 : a.N;
-  // Where row r of the workgroup's part of W sits in LDS: tile t of a wave holds rows 4 T (i / 4) + 4 t + i % 4 of its 16 T
-  // (T = kTiles), i = 0 .. 15, one after the other.
-  auto position = [](int r) __attribute__((always_inline)) {
-    const int half = SILU_MUL ? r / (BN / 2) : 0;
-    r -= half * (BN / 2);
-    const int w = r / (16 * kTiles), c = r % (16 * kTiles);
-    return w * (16 * NT) + (half * kTiles + (c >> 2) % kTiles) * 16 + (c / (4 * kTiles)) * 4 + (c & 3);
+  // Row of W at place p of the workgroup's (tile p / 32, row i = p % 32 of it): accumulator r of lane (lr, kq) is row
+  // i = 8 (r / 4) + 4 kq + r % 4, which stands for column 16 kq + r of the tile, so that a lane has 16 consecutive ones.
+  auto first_row = [&](int t) __attribute__((always_inline)) {  // of tile t
+    return SILU_MUL ? n0 / 2 + (t >> 1) * 32 + (t & 1) * out_cols : n0 + t * 32;
   };
-  // ... and which row of W it is
-  auto row_of_w = [&](int r) __attribute__((always_inline)) {
-    const int half = SILU_MUL ? r / (BN / 2) : 0;
-    int n = (SILU_MUL ? n0 / 2 : n0) + r - half * (BN / 2);
-    n = n < out_cols ? n : out_cols - 1;
-    return n + half * out_cols;
-  };
+  auto row_in_tile = [](int i) __attribute__((always_inline)) { return 16 * ((i >> 2) & 1) + 4 * (i >> 3) + (i & 3); };
 
-  // this thread's pieces of a stage: uniform bases, 32-bit byte offsets from them
-  const char* const xbase = (const char*)(a.x + (size_t)m0 * a.K);
-  const char* const wbase = (const char*)a.w + (size_t)(SILU_MUL ? 0 : n0) * (a.K >> 1);
-  const int xg = tid % (8 * KG), xr = tid / (8 * KG), wg16 = tid % (2 * KG), wr = tid / (2 * KG);
-  uint32_t xo[XL];
-  size_t wo[WL];
+  // ---- what this wave requests: x by descriptors of the workgroup's rows, codes of one tile at a time ---------------------
+  const int rows_here = a.M - m0 < BM ? a.M - m0 : BM;
+  const auto x_buf = __builtin_amdgcn_make_buffer_rsrc((void*)(a.x + (size_t)m0 * a.K), 0, (int)((uint32_t)rows_here * (uint32_t)a.K * 2u), 0x00027000);
+  // x: request j brings rows 8 (kXReq wave + j) .. + 7 of this wave's set, piece c of a row to place c ^ (row / 2 % 8)
+  uint32_t xo[kXReq];
 #pragma unroll
-  for (int i = 0; i < XL; ++i) {
-    int row = xr + kXRows * i;
-    row = m0 + row < a.M ? row : a.M - 1 - m0;
-    xo[i] = (uint32_t)row * (uint32_t)a.K * 2u;
+  for (int j = 0; j < kXReq; ++j) {
+    const int row = 8 * (kXReq * wave + j) + (lane >> 3), c = (lane & 7) ^ ((row >> 1) & 7);
+    xo[j] = (uint32_t)(row < rows_here ? row : rows_here - 1) * (uint32_t)a.K * 2u + 128u * kg + 16u * c;
   }
+  const uint32_t x_to = lds0 + kg * (BM * 128) + 1024 * kXReq * wave;
+  const int tail = a.K % (kStageK * KG) != 0 ? a.stages - 1 : -1;
+  // codes: a row has 2 KG pieces (32 k each); request j brings 32 / KG rows, piece u of row p to place u ^ f(p)
+  constexpr int kPieces = 2 * KG, kWRows = 64 / kPieces;
+  auto code_place = [](int p) __attribute__((always_inline)) { return KG == 8 ? p & 15 : KG == 4 ? (p >> 1) & 7 : KG == 2 ? (p >> 2) & 3 : (p >> 3) & 1; };
+  uint32_t wo[kWReq];
+  __amdgpu_buffer_rsrc_t w_buf[kWReq];
 #pragma unroll
-  for (int i = 0; i < WL; ++i) {
-    const int row = row_of_w(wr + kWRows * i < BN ? wr + kWRows * i : BN - 1) - (SILU_MUL ? 0 : n0);
-    wo[i] = (size_t)row * ((uint32_t)a.K >> 1);
+  for (int j = 0; j < kWReq; ++j) {
+    const int p0 = kWRows * (kWReq * wid + j), p = p0 + lane / kPieces, u = (lane % kPieces) ^ code_place(p);
+    const int first = __builtin_amdgcn_readfirstlane(first_row(p0 >> 5));
+    int here = (SILU_MUL && first >= out_cols ? a.N : out_cols) - first;  // rows there are
+    const bool none = here <= 0;
+    here = here > 32 ? 32 : here;
+    const int row = row_in_tile(p & 31);
+    wo[j] = (uint32_t)(row < here ? row : none ? 0 : here - 1) * ((uint32_t)a.K >> 1) + 16u * u;
+    const int from = none ? 0 : first;
+    w_buf[j] = __builtin_amdgcn_make_buffer_rsrc((void*)((const char*)a.w + (size_t)from * (a.K >> 1)), 0,
+                                                 (int)((uint32_t)(none ? 1 : here) * ((uint32_t)a.K >> 1)), 0x00027000);
   }
-  static_assert(WL <= 2, "two pieces of codes per thread at most");
-  uint4 xv[XL], wv0, wv1, sv[SL];
-  auto load_x = [&](int st) __attribute__((always_inline)) {
-    const int kx = st * (kStageK * KG) + 8 * xg;
-    const uint32_t xk = kx < a.K ? 2u * kx : 0u;
-#pragma unroll
-    for (int i = 0; i < XL; ++i) xv[i] = *reinterpret_cast<const uint4*>(xbase + (xo[i] + xk));
-    if (kx >= a.K) {  // k past the end of the rows: zeros on this side are enough
-#pragma unroll
-      for (int i = 0; i < XL; ++i) xv[i] = make_uint4(0u, 0u, 0u, 0u);
-    }
+  const uint32_t w_to = lds0 + XB * T::kXBytes + 1024 * kWReq * wid;
+  // Stages behind the last one are the last one again; k past the end of the rows reads zeros (an offset behind all of them).
+  auto request_x = [&](int st, int buf, int j) __attribute__((always_inline)) {
+    st = st < a.stages ? st : a.stages - 1;
+    const int row = 8 * (kXReq * wave + j) + (lane >> 3), c = (lane & 7) ^ ((row >> 1) & 7);
+    const bool past = st == tail && (st * KG + kg) * kStageK + 8 * c >= a.K;
+    request16(x_buf, x_to + buf * T::kXBytes + 1024 * j, past ? 0x80000000u : xo[j], st * (2 * kStageK * KG));
   };
-  auto load_w = [&](int st) __attribute__((always_inline)) {
-    const int kw = st * (kStageK * KG) + 32 * wg16;
-    const uint32_t wk = kw < a.K ? (uint32_t)kw >> 1 : 0u;
-    wv0 = *reinterpret_cast<const uint4*>(wbase + (wo[0] + wk));
-    if constexpr (WL == 2) wv1 = *reinterpret_cast<const uint4*>(wbase + (wo[WL - 1] + wk));
+  auto request_w = [&](int st, int buf, int j) __attribute__((always_inline)) {
+    st = st < a.stages ? st : a.stages - 1;
+    const int p = kWRows * (kWReq * wid + j) + lane / kPieces, u = (lane % kPieces) ^ code_place(p);
+    const bool past = st == tail && st * (kStageK * KG) + 32 * u >= a.K;
+    request16(w_buf[j], w_to + buf * T::kWBytes + 1024 * j, past ? 0x80000000u : wo[j], st * (kStageK * KG / 2));
   };
-  auto store_x = [&](int buf) __attribute__((always_inline)) {
-    char* const xs = lds + buf * kXBytes + (xg >> 3) * (BM * 128);
-#pragma unroll
-    for (int i = 0; i < XL; ++i) {
-      const int row = xr + kXRows * i;
-      if (BM % kXRows == 0 || row < BM) *reinterpret_cast<uint4*>(xs + row * 128 + (((xg & 7) ^ ((row >> 1) & 7)) << 4)) = xv[i];
-    }
-  };
-  auto store_w = [&](int buf) __attribute__((always_inline)) {
-    char* const ws = w_lds + buf * kWBytes + (wg16 >> 1) * (BN * 32) + (wg16 & 1) * 16;
-    if (BN >= kWRows || wr < BN) *reinterpret_cast<uint4*>(ws + position(wr) * 32) = wv0;
-    if constexpr (WL == 2) {
-      if (BN % kWRows == 0 || wr + kWRows < BN) *reinterpret_cast<uint4*>(ws + position(wr + kWRows) * 32) = wv1;
-    }
-  };
-  // a chunk is the scales and biases of eight groups (16 bytes) of every row
-  auto load_chunk = [&](int chunk) __attribute__((always_inline)) {
+  // a chunk is the scales and biases of kGroups groups of every row, 16 bytes for eight of them
+  constexpr int kSbPieces = kGroups / 4 * BN, SL = (kSbPieces + kThreads - 1) / kThreads;
+  uint4 sv[SL];
+  auto load_chunk = [&](int chunk, uint4 (&sv)[SL]) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < SL; ++i) {
-      const int e = tid + kThreads * i, r = e % BN;
-      const int n = row_of_w(r);
-      const uint16_t* src = (e < BN ? a.scales : a.biases) + (size_t)n * G;
-      if (8 * chunk + 8 <= G) {
+      const int e = tid + kThreads * i, p = e % BN, g0 = kGroups * chunk + (e / (2 * BN)) * 8;
+      int n = first_row(p >> 5) + row_in_tile(p & 31);
+      const int end = SILU_MUL && ((p >> 5) & 1) ? a.N : out_cols;
+      n = n < end ? n : end - 1;
+      const uint16_t* src = ((e / BN) % 2 == 0 ? a.scales : a.biases) + (size_t)n * G;
+      if (g0 + 8 <= G) {
         struct __attribute__((packed, aligned(2))) Loose { uint32_t a, b, c, d; };  // (rows of scales start on any element)
-        const Loose v = *reinterpret_cast<const Loose*>(src + 8 * chunk);
+        const Loose v = *reinterpret_cast<const Loose*>(src + g0);
         sv[i] = make_uint4(v.a, v.b, v.c, v.d);
       } else {
         uint32_t h[8];
 #pragma unroll
-        for (int g = 0; g < 8; ++g) h[g] = src[8 * chunk + g < G ? 8 * chunk + g : G - 1];
+        for (int g = 0; g < 8; ++g) h[g] = src[g0 + g < G ? g0 + g : G - 1];
         sv[i] = make_uint4(h[0] | h[1] << 16, h[2] | h[3] << 16, h[4] | h[5] << 16, h[6] | h[7] << 16);
       }
     }
   };
-  auto store_chunk = [&](int buf) __attribute__((always_inline)) {
+  auto store_chunk = [&](int buf, const uint4 (&sv)[SL]) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < SL; ++i) {
       const int e = tid + kThreads * i;
-      if ((2 * BN) % kThreads == 0 || e < 2 * BN)
-        *reinterpret_cast<uint4*>(sb_lds + buf * kSbBytes + (e < BN ? 0 : BN * 16) + position(e % BN) * 16) = sv[i];
+      if (kSbPieces % kThreads == 0 || e < kSbPieces) *reinterpret_cast<uint4*>(sb_lds + buf * T::kSbBytes + e * 16) = sv[i];
     }
   };
-  const int stages_per_chunk = (8 << a.group_shift) / (kStageK * KG);
+  const int stages_per_chunk = (kGroups << a.group_shift) / (kStageK * KG);
 
-  f32x4_t acc[MT][NT];
+  f32x16_t acc[MT][NT];
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int t = 0; t < NT; ++t) acc[i][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][t][r] = 0.f;
 
   int chunk = st0 / stages_per_chunk;  // of the stage whose codes are read next, and its place in the chunk
   int in_chunk = st0 - chunk * stages_per_chunk;
   const int last_chunk = (a.stages - 1) / stages_per_chunk;
   int cbuf = 0, wbuf = 0;  // buffers of that stage
-  // lane addresses inside a stage
-  const char* const xrd = lds + kg * (BM * 128) + li * 128;
-  const char* const wrd = w_lds + kg * (BN * 32) + (wave * (16 * NT) + li) * 32 + kq * 8;
-  const char* const srd = sb_lds + (wave * (16 * NT) + li) * 16;
-  uint2 wc[NT];
+  // Lane (lr, kq) multiplies k = 32 kq .. 32 kq + 31 of its set's 64: step s of a stage 32 kq + 8 s .. + 7.
+  const char* xrd[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) xrd[s] = lds + kg * (BM * 128) + lr * 128 + (((4 * kq + s) ^ ((lr >> 1) & 7)) << 4);
+  const char* const wrd = w_lds + (wave * (32 * NT) + lr) * (32 * KG) + (((2 * kg + kq) ^ code_place(lr)) << 4);
+  const char* const srd = sb_lds + (wave * (32 * NT) + lr) * 16;
+  uint4 wc[NT];
+  uint32_t sraw[NT], braw[NT];
   float sc[NT], sc16[NT], bc[NT];
   auto read_codes = [&]() __attribute__((always_inline)) {
-    // lane group kq multiplies k = 16 kq .. 16 kq + 15 of its 64: words 2 kq and 2 kq + 1 of a row
-    const int g = ((in_chunk * KG + kg) * kStageK + 16 * kq) >> a.group_shift;
-    const char* const sp = srd + cbuf * kSbBytes + g * 2;
+    const int g = ((in_chunk * KG + kg) * kStageK + 32 * kq) >> a.group_shift;
+    const char* const sp = srd + cbuf * T::kSbBytes + (kGroups == 8 ? 0 : (g >> 3) * (32 * BN)) + (kGroups == 8 ? g : g & 7) * 2;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      wc[t] = *reinterpret_cast<const uint2*>(wrd + wbuf * kWBytes + t * 512);
-      const float scale = sb_value<SB_FP16>(*reinterpret_cast<const uint16_t*>(sp + t * 256));
+      wc[t] = *reinterpret_cast<const uint4*>(wrd + wbuf * T::kWBytes + t * (1024 * KG));
+      sraw[t] = *reinterpret_cast<const uint16_t*>(sp + t * 512);
+      braw[t] = *reinterpret_cast<const uint16_t*>(sp + BN * 16 + t * 512);
+    }
+  };
+  auto take_scales = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const float scale = sb_value<SB_FP16>(sraw[t]);
       sc[t] = scale * 16777216.0f, sc16[t] = scale * 1048576.0f;
-      bc[t] = sb_value<SB_FP16>(*reinterpret_cast<const uint16_t*>(sp + BN * 16 + t * 256));
+      bc[t] = sb_value<SB_FP16>(braw[t]);
     }
   };
-  uint4 wf[2][NT];
-  // Half a stage: the products with the weights in wf[j] and, spread over their matrix instructions, the
-  // dequantisation of the other half.  x is read two rows of tiles ahead.
-  constexpr int kAhead = NT == 4 ? 2 : 4;  // rows of tiles of x read ahead
-  uint4 xf[kAhead + 1];
-  auto first_x = [&](int j, int xbuf) __attribute__((always_inline)) -> const char* {
-    const char* const xp = xrd + xbuf * kXBytes + (((2 * kq + j) ^ (li >> 1)) << 4);
+  constexpr int kAhead = MT == 1 ? 3 : 1;  // steps that x is read ahead: a step of few products is shorter than the way to LDS
+  uint4 wf[2][NT], xf[kAhead + 1][MT];
+  auto read_x = [&](int s, int buf) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < kAhead && i < MT; ++i) xf[i] = *reinterpret_cast<const uint4*>(xp + i * 2048);
-    return xp;
-  };
-  auto half_stage = [&](int j, const char* xp) __attribute__((always_inline)) {
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int i = 0; i < MT; ++i) {
-      if (i + kAhead < MT) xf[(i + kAhead) % (kAhead + 1)] = *reinterpret_cast<const uint4*>(xp + (i + kAhead) * 2048);
-#pragma unroll
-      for (int t = 0; t < NT; ++t) acc[i][t] = A::mfma(wf[j][t], xf[i % (kAhead + 1)], acc[i][t]);
-    }
-#pragma unroll
-    for (int t = 0; t < NT; ++t) wf[j ^ 1][t] = dequant8<FP16>(j == 0 ? wc[t].y : wc[t].x, sc[t], sc16[t], bc[t], mask0, mask4);
-#pragma unroll
-    for (int i = 0; i < MT; ++i) {
-      if (i + kAhead < MT) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x2, (20 + MT - 1) / MT, 0);
-      }
-    }
-    // (used in the next stage only, the weights would be dequantised there)
-#pragma unroll
-    for (int t = 0; t < NT; ++t) asm volatile("" : "+v"(wf[j ^ 1][t].x), "+v"(wf[j ^ 1][t].y), "+v"(wf[j ^ 1][t].z), "+v"(wf[j ^ 1][t].w));
-    __builtin_amdgcn_sched_barrier(0);
+    for (int i = 0; i < MT; ++i) xf[s & kAhead][i] = *reinterpret_cast<const uint4*>(xrd[s] + buf * T::kXBytes + i * 4096);
   };
 
-  load_chunk(chunk);
-  load_w(st0);
-  load_x(st0);
-  store_chunk(0);
-  store_w(0);
-  load_w(st0 + 1);
-  store_x(0);
-  store_w(1);
-  if (chunk < last_chunk) {
-    load_chunk(chunk + 1);
-    store_chunk(1);
-  }
-  load_x(st0 + 1);
-  load_w(st0 + 2);
-  __syncthreads();
+  // ---- prologue ------------------------------------------------------------------------------------------------------------
+#pragma unroll
+  for (int j = 0; j < kWReq; ++j) request_w(st0, 0, j);
+#pragma unroll
+  for (int j = 0; j < kXReq; ++j) request_x(st0, 0, j);
+#pragma unroll
+  for (int b = 1; b < WB; ++b)
+#pragma unroll
+    for (int j = 0; j < kWReq; ++j) request_w(st0 + b, b, j);
+  uint4 sv_next[SL];
+  const bool two_chunks = (chunk + 1) * stages_per_chunk < st1;
+  load_chunk(chunk, sv);
+  if (two_chunks) load_chunk(chunk + 1, sv_next);
+  store_chunk(0, sv);
+  if (two_chunks) store_chunk(1, sv_next);
+  stage_done<0>();
   read_codes();
 #pragma unroll
+  for (int s = 0; s < kAhead; ++s) read_x(s, 0);
+  take_scales();
+#pragma unroll
   for (int t = 0; t < NT; ++t) wf[0][t] = dequant8<FP16>(wc[t].x, sc[t], sc16[t], bc[t], mask0, mask4);
+
+  int xbuf = 0;
   for (int st = st0; st < st1; ++st) {
-    const int xbuf = (st - st0) & 1;
     const bool brings_chunk = in_chunk == 0 && st != st0 && chunk < last_chunk;
-    if (brings_chunk) load_chunk(chunk + 1);
-    half_stage(0, first_x(0, xbuf));
-    // What was asked for a stage ago goes to LDS in the middle of this one, and the next requests leave: a
-    // whole stage for the latency of memory, and no wave waits at the barrier for another one's loads.
-    // (Behind the last stage: loads of valid addresses, stores to buffers that nobody reads.)
-    store_x(xbuf ^ 1);
-    store_w(wbuf == 0 ? 2 : wbuf - 1);
-    load_x(st + 2);
-    load_w(st + 3);
-    // the codes of the next stage (behind the last one: of some stage that is in LDS, not used)
-    const int cbuf_now = cbuf;
-    if (++wbuf == 3) wbuf = 0;
+    if (brings_chunk) load_chunk(chunk + 1, sv);
+    const int cbuf_now = cbuf, wbuf_now = wbuf;
+    if (++wbuf == WB) wbuf = 0;
     if (++in_chunk == stages_per_chunk) {
       in_chunk = 0;
       ++chunk;
       cbuf ^= 1;
     }
-    const char* const xp = first_x(1, xbuf);
-    read_codes();
-    half_stage(1, xp);
-    if (brings_chunk) store_chunk(cbuf_now ^ 1);
-    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      __builtin_amdgcn_sched_barrier(0);
+      // the next step's x; requests for later stages; the next stage's codes, whose first word the last step dequantises
+      if (s + kAhead < 4) read_x(s + kAhead, xbuf);
+      if (s == 0) {
+#pragma unroll
+        for (int j = 0; j < kXReq; ++j) request_x(st + 1, xbuf ^ 1, j);
+      }
+      if (s == 1) {
+#pragma unroll
+        for (int j = 0; j < kWReq; ++j) request_w(st + WB, wbuf_now, j);
+      }
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[i][t] = mfma32<FP16>(wf[s & 1][t], xf[s & kAhead][i], acc[i][t]);
+      if (s == 3) take_scales();
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        wf[(s + 1) & 1][t] = dequant8<FP16>(s == 0 ? wc[t].y : s == 1 ? wc[t].z : s == 2 ? wc[t].w : wc[t].x, sc[t], sc16[t], bc[t], mask0, mask4);
+      constexpr int kVector = (20 + MT - 1) / MT;
+#pragma unroll
+      for (int i = 0; i < MT * NT; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x2, kVector, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      // (used in the next step only, the weights would be dequantised there)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        asm volatile("" : "+v"(wf[(s + 1) & 1][t].x), "+v"(wf[(s + 1) & 1][t].y), "+v"(wf[(s + 1) & 1][t].z), "+v"(wf[(s + 1) & 1][t].w));
+      if (s == 2) read_codes();
+    }
+    if (brings_chunk) store_chunk(cbuf_now ^ 1, sv);
+    stage_done<kWReq>();  // (the codes asked for in this stage may take another one)
+    xbuf ^= 1;
+#pragma unroll
+    for (int s = 0; s < kAhead; ++s) read_x(s, xbuf);
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the requests that nobody reads: LDS is used for other things, or the workgroup leaves
 
-  if constexpr (KG == 2) {
-    // the second set hands its sums over through LDS, as many rows of tiles at a time as fit the stages
-    constexpr int kPer = kFrontBytes / (4096 * NT) < MT ? kFrontBytes / (4096 * NT) : MT;
-    f32x4_t* const red = reinterpret_cast<f32x4_t*>(lds);
-    const int t256 = tid & 255;
+  auto mine = [&](int i) __attribute__((always_inline)) { return KG == 1 || i % KG == kg; };
+  if constexpr (KG > 1) {
+    // Row of tiles i is finished by set i % KG: the others hand their sums over through LDS, as many rows of tiles at a
+    // time as fit the stages.
+    constexpr int kRow = (KG - 1) * NT * 4 * kSet;  // 16-byte pieces that are handed over for a row of tiles
+    constexpr int kPer = T::kFrontBytes / (16 * kRow) < MT ? T::kFrontBytes / (16 * kRow) : MT;
+    static_assert(kPer > 0, "the stages hold the sums of a row of tiles");
+    f32x4_t* const red = reinterpret_cast<f32x4_t*>(lds) + tid % kSet;
+    __syncthreads();
 #pragma unroll
     for (int i0 = 0; i0 < MT; i0 += kPer) {
       if (i0 > 0) __syncthreads();
-      if (kg == 1) {
 #pragma unroll
-        for (int i = i0; i < i0 + kPer && i < MT; ++i)
+      for (int i = i0; i < i0 + kPer && i < MT; ++i) {
+        if (mine(i)) continue;
+        f32x4_t* const to = red + (i - i0) * kRow + (kg - (kg > i % KG ? 1 : 0)) * (NT * 4 * kSet);
 #pragma unroll
-          for (int t = 0; t < NT; ++t) red[((i - i0) * NT + t) * 256 + t256] = acc[i][t];
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            to[(4 * t + q) * kSet] = f32x4_t{acc[i][t][4 * q], acc[i][t][4 * q + 1], acc[i][t][4 * q + 2], acc[i][t][4 * q + 3]};
       }
       __syncthreads();
-      if (kg == 0) {
 #pragma unroll
-        for (int i = i0; i < i0 + kPer && i < MT; ++i)
+      for (int i = i0; i < i0 + kPer && i < MT; ++i) {
+        if (!mine(i)) continue;
 #pragma unroll
-          for (int t = 0; t < NT; ++t) acc[i][t] += red[((i - i0) * NT + t) * 256 + t256];
+        for (int o = 0; o < KG - 1; ++o)
+#pragma unroll
+          for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              const f32x4_t v = red[(i - i0) * kRow + ((o * NT + t) * 4 + q) * kSet];
+#pragma unroll
+              for (int r = 0; r < 4; ++r) acc[i][t][4 * q + r] += v[r];
+            }
       }
     }
   }
 
-  // accumulator r of lane (li, kq), tile (i, t): row m0 + 16 i + li, column 16 T wave + 4 T kq + 4 t + r of the workgroup's
-  auto emit = [&](int i, const f32x4_t (&v)[NT]) __attribute__((always_inline)) {
-    const int m = m0 + 16 * i + li, n = (SILU_MUL ? n0 / 2 : n0) + wave * (16 * kTiles) + 4 * kTiles * kq;
-    if (m >= a.M) return;
-    uint16_t* dst = a.y + (size_t)m * out_cols + n;
+  // accumulator r of lane (lr, kq), tile (i, t): row m0 + 32 i + lr, column 16 kq + r of the tile; the tiles of one piece of the
+  // result: one, or those of gate and up
+  constexpr int kTiles = SILU_MUL ? NT : 1, kUnits = MT * NT / kTiles;
+  auto emit = [&](int i, int t, const f32x4_t (&v)[kTiles][4]) __attribute__((always_inline)) {
+    const int m = m0 + 32 * i + lr, n = (SILU_MUL ? n0 / 2 + wave * 32 : n0 + (wave * NT + t) * 32) + 16 * kq;
+    if (m >= a.M || n >= out_cols) return;
+    uint32_t w[8];
 #pragma unroll
-    for (int t = 0; t < kTiles; ++t) {
-      f32x4_t o = v[t];
-      if constexpr (SILU_MUL) {
+    for (int p = 0; p < 8; ++p) {
+      float o[2];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float g = round16<FP16>(v[t][r]), u = round16<FP16>(v[t + kTiles][r]);
-          const float s = round16<FP16>(1.0f / (1.0f + expf(-g)));
-          o[r] = round16<FP16>(g * s) * u;
+      for (int h = 0; h < 2; ++h) {
+        const int r = 2 * p + h;
+        o[h] = v[0][r >> 2][r & 3];
+        if constexpr (SILU_MUL) {
+          const float g = round16<FP16>(o[h]), u = round16<FP16>(v[kTiles - 1][r >> 2][r & 3]);
+          const float sg = round16<FP16>(1.0f / (1.0f + expf(-g)));
+          o[h] = round16<FP16>(g * sg) * u;
         }
       }
-      const uint2 w = make_uint2(pack2<FP16>(o[0], o[1]), pack2<FP16>(o[2], o[3]));
-      if (n + 4 * t < out_cols) *reinterpret_cast<uint2*>(dst + 4 * t) = w;
+      w[p] = pack2<FP16>(o[0], o[1]);
     }
+    struct __attribute__((packed, aligned(8))) Loose { uint32_t w[4]; };  // (y starts on 8 bytes)
+    Loose* const dst = reinterpret_cast<Loose*>(a.y + (size_t)m * out_cols + n);
+    dst[0] = Loose{{w[0], w[1], w[2], w[3]}};
+    dst[1] = Loose{{w[4], w[5], w[6], w[7]}};
   };
   if (slices == 1) {
-    if (kg == 0) {
 #pragma unroll
-      for (int i = 0; i < MT; ++i) emit(i, acc[i]);
+    for (int i = 0; i < MT; ++i) {
+      if (!mine(i)) continue;
+#pragma unroll
+      for (int t0 = 0; t0 < NT; t0 += kTiles) {
+        f32x4_t v[kTiles][4];
+#pragma unroll
+        for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[t][q][r] = acc[i][t0 + t][4 * q + r];
+        emit(i, t0, v);
+      }
     }
     return;
   }
   // Partial tiles are written through to and read from the level all XCDs share (sc1, as in the streaming kernel).
   constexpr size_t kTileFloats = (size_t)BM * BN;
   float* const first = a.partials + (size_t)cut_tile * slices * kTileFloats;
-  if (kg == 0) {
-    float* mine = first + slice * kTileFloats + (tid & 255) * 4;
+  float* const part_of = first + slice * kTileFloats + (tid % kSet) * 4;
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
+  for (int i = 0; i < MT; ++i) {
+    if (!mine(i)) continue;
 #pragma unroll
-      for (int t = 0; t < NT; ++t) stream::store_partial(mine + (i * NT + t) * 1024, acc[i][t]);
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        stream::store_partial(part_of + ((i * NT + t) * 4 + q) * (4 * kSet),
+                              f32x4_t{acc[i][t][4 * q], acc[i][t][4 * q + 1], acc[i][t][4 * q + 2], acc[i][t][4 * q + 3]});
   }
   // every wave's stores are acknowledged before the arrival is counted
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  if (tid == 0) s_last = atomicInc(&a.counters[cut_tile], (uint32_t)(slices - 1)) == (uint32_t)(slices - 1);
+  uint32_t* const s_last = reinterpret_cast<uint32_t*>(lds);  // (what was handed over has been read)
+  if (tid == 0) *s_last = atomicInc(&a.counters[cut_tile], (uint32_t)(slices - 1)) == (uint32_t)(slices - 1);
   __syncthreads();
-  if (!s_last || kg != 0) return;
-  // in order of k; a row of tiles of every slice is asked for before the first is looked at
+  if (!*s_last) return;
+  // In order of k, the pieces of the result dealt to the sets; what a thread needs of several slices is asked for before the first
+  // is looked at.
+  constexpr int kAtOnce = kTiles == 1 || MT == 2 || MT == 3 ? 4 : 2;
   const auto parts = __builtin_amdgcn_make_buffer_rsrc(first, 0, 0x7FFFFFFF, 0x00027000);
+#pragma unroll 1
+  for (int u = kg; u < kUnits; u += KG) {
+    const int i = SILU_MUL ? u : u / NT, t0 = SILU_MUL ? 0 : u % NT;
+    f32x4_t sum[kTiles][4];
 #pragma unroll
-  for (int i = 0; i < MT; ++i) {
-    f32x4_t sum[NT];
+    for (int t = 0; t < kTiles; ++t)
 #pragma unroll
-    for (int t = 0; t < NT; ++t) sum[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    for (int c0 = 0; c0 < slices; c0 += 4) {
-      f32x4_t v[4][NT];
+      for (int q = 0; q < 4; ++q) sum[t][q] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int c0 = 0; c0 < slices; c0 += kAtOnce) {
+      f32x4_t v[kAtOnce][kTiles][4];
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
+      for (int c = 0; c < kAtOnce; ++c) {
         const int cc = c0 + c < slices ? c0 + c : slices - 1;
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
-          v[c][t] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(
-              parts, (uint32_t)(tid * 16 + (i * NT + t) * 4096 + cc * (kTileFloats * 4)), 0, 16));
+        for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            v[c][t][q] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(
+                parts, (uint32_t)((tid % kSet) * 16 + ((i * NT + t0 + t) * 4 + q) * (16 * kSet) + cc * (kTileFloats * 4)), 0, 16));
       }
 #pragma unroll
-      for (int c = 0; c < 4; ++c)
+      for (int c = 0; c < kAtOnce; ++c)
         if (c0 + c < slices) {
 #pragma unroll
-          for (int t = 0; t < NT; ++t) sum[t] += v[c][t];
+          for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) sum[t][q] += v[c][t][q];
         }
     }
-    emit(i, sum);
+    emit(i, t0, sum);
   }
 }
 
-// The tile shapes there are: columns (16 NT a wave) for a height, and the one with a single set of waves for calls with
-// many tiles.
-template <bool FP16>
-const void* kernel_for(int mt, int nt, int kg, bool mixed, bool silu_mul) {
-#define DFLASH_ROWS_PICK(MT, NT, KG) \
-  if (mt == MT && nt == NT && kg == KG && !mixed && !silu_mul) return (const void*)qmm_rows_kernel<FP16, FP16, MT, NT, KG, false>;
-#define DFLASH_ROWS_PICK_SILU(MT, NT, KG) \
-  if (mt == MT && nt == NT && kg == KG && !mixed && silu_mul) return (const void*)qmm_rows_kernel<FP16, FP16, MT, NT, KG, true>;
-#define DFLASH_ROWS_PICK_MIXED(MT, NT, KG) \
-  if (mt == MT && nt == NT && kg == KG && mixed && !silu_mul) return (const void*)qmm_rows_kernel<FP16, !FP16, MT, NT, KG, false>;
-  DFLASH_ROWS_PICK(1, 1, 2)
-  DFLASH_ROWS_PICK(2, 1, 2) DFLASH_ROWS_PICK(2, 2, 2) DFLASH_ROWS_PICK_SILU(2, 2, 2)
-  DFLASH_ROWS_PICK(3, 1, 2) DFLASH_ROWS_PICK(3, 2, 2) DFLASH_ROWS_PICK_SILU(3, 2, 2)
-  DFLASH_ROWS_PICK(4, 1, 2) DFLASH_ROWS_PICK(4, 2, 2) DFLASH_ROWS_PICK_SILU(4, 2, 2)
-  DFLASH_ROWS_PICK(5, 1, 2) DFLASH_ROWS_PICK(5, 2, 2) DFLASH_ROWS_PICK_SILU(5, 2, 2)
-  DFLASH_ROWS_PICK(6, 1, 2) DFLASH_ROWS_PICK(6, 2, 2) DFLASH_ROWS_PICK_SILU(6, 2, 2)
-  DFLASH_ROWS_PICK(7, 1, 2) DFLASH_ROWS_PICK(7, 2, 2) DFLASH_ROWS_PICK_SILU(7, 2, 2)
-  DFLASH_ROWS_PICK(8, 1, 2) DFLASH_ROWS_PICK(8, 2, 2) DFLASH_ROWS_PICK_SILU(8, 2, 2)
-  DFLASH_ROWS_PICK(8, 3, 2) DFLASH_ROWS_PICK(8, 4, 2) DFLASH_ROWS_PICK_SILU(8, 4, 2)
-  DFLASH_ROWS_PICK(8, 3, 1) DFLASH_ROWS_PICK(8, 4, 1) DFLASH_ROWS_PICK_SILU(8, 4, 1)
-  // scales of the other 16-bit type: a few shapes
-  DFLASH_ROWS_PICK_MIXED(2, 1, 2) DFLASH_ROWS_PICK_MIXED(4, 2, 2) DFLASH_ROWS_PICK_MIXED(8, 2, 2)
-#undef DFLASH_ROWS_PICK
-#undef DFLASH_ROWS_PICK_SILU
-#undef DFLASH_ROWS_PICK_MIXED
-  return nullptr;
+// A tile shape: what it takes, how long a stage takes it, and its kernels.
+struct Shape {
+  int mt, nt, w, kg, lds;
+  int together;        // workgroups that a CU has room for
+  double alone, busy;  // us per stage: of one workgroup on a CU, and of each where they share it
+  const void* kernel[2][3];  // [fp16][plain, scales of the other type, silu-mul]; null: there is none
+  int rows() const { return 32 * mt; }
+  int columns() const { return 32 * nt * w; }
+};
+template <int MT, int NT, int W, int KG, bool MIXED = false>
+Shape shape(int together, double alone, double busy) {
+  Shape s{MT, NT, W, KG, Tile<MT, NT, W, KG>::kLdsBytes, together, alone, busy, {}};
+  s.kernel[0][0] = (const void*)qmm_rows_kernel<false, false, MT, NT, W, KG, false>;
+  s.kernel[1][0] = (const void*)qmm_rows_kernel<true, true, MT, NT, W, KG, false>;
+  if constexpr (MIXED) {
+    s.kernel[0][1] = (const void*)qmm_rows_kernel<false, true, MT, NT, W, KG, false>;
+    s.kernel[1][1] = (const void*)qmm_rows_kernel<true, false, MT, NT, W, KG, false>;
+  }
+  if constexpr (NT == 2) {
+    s.kernel[0][2] = (const void*)qmm_rows_kernel<false, false, MT, NT, W, KG, true>;
+    s.kernel[1][2] = (const void*)qmm_rows_kernel<true, true, MT, NT, W, KG, true>;
+  }
+  return s;
 }
-constexpr int lds_bytes(int mt, int nt, int kg) { return kg * (2 * 16 * mt * 128 + 3 * 64 * nt * 32) + 2 * 2 * 64 * nt * 16; }
+// (1,1,4,2), (2,1,4,2), (3,1,4,2), (4,1,4,2), (2,2,2,2), (2,2,4,2), (3,2,4,1), (2,2,8,1) and (4,2,8,1) were measured as well:
+// without them the best of the rest is 0.3 % slower on average.
+constexpr int kShapes = 14;
+const Shape* shapes() {
+  static const Shape all[kShapes] = {
+      shape<1, 1, 1, 8>(1, 0.600, 0.571),       shape<2, 1, 1, 8>(1, 0.925, 0.454),
+      shape<1, 1, 2, 4, true>(2, 0.540, 0.472), shape<2, 1, 2, 4>(1, 0.709, 0.447),       shape<3, 1, 2, 4>(1, 0.910, 0.307),
+      shape<1, 2, 2, 4>(1, 0.924, 0.508),       shape<2, 2, 2, 4, true>(1, 1.100, 0.401), shape<3, 2, 2, 4>(1, 1.367, 0.390),
+      shape<1, 2, 4, 2>(2, 0.905, 0.750),       shape<3, 2, 4, 2>(1, 1.274, 0.363),       shape<4, 2, 4, 2, true>(1, 1.533, 0.524),
+      shape<4, 2, 2, 2>(1, 0.879, 0.546),       shape<2, 2, 4, 1>(2, 0.650, 0.535),       shape<4, 2, 4, 1>(2, 0.834, 0.767)};
+  return all;
+}
 
 struct Plan {
-  int mt, nt, kg, whole, slices, tiles_m, tiles, stages, grid;
+  const Shape* shape;
+  int whole, slices, tiles_m, tiles, stages, grid;
   size_t workspace;
 };
 
@@ -475,76 +556,69 @@ bool covers(int M, int K, int N, int group_size, bool mixed, int epilogue) {
          N % 16 == 0;
 }
 
-// Which tile, how many slices of K: the least of a model of the time, fitted to 2757 measured combinations (8 shapes of
-// 1 to 178 M weights, 20 to 1024 rows; 8 % rms, and what it picks is within 1 % of the best measured one on
-// average, 12 % at worst).  A stage of 64 KG columns of K costs a fixed part (barrier, latency) and parts that go with
-// the columns (codes to dequantise), the rows (x) and their product (matrix work); a workgroup with two sets of waves
-// has a CU to itself, those with one share it in pairs.
-// The last round of more tiles than fit at once is cut with the tile left as it is: matrix work that fills the chip
-// runs against its power, so a smaller tile that fills it better gains nothing (5120 x 12352 over 1024 rows: 65 x 8
-// tiles of 192 columns, 8 of them cut, 190 us; 49 x 8 of 256, uncut, 179).  Partial tiles behind whole rounds meet the
-// memory busy, 3 TB/s for their way out and back: of 5120 x 34816, 64 of 1088 in four slices save 24 us, of
-// 5120 x 12352, 136 of 392 in three slices nothing.
-Plan make_plan(int M, int K, int N, int cus, bool mixed, bool silu_mul) {
-  auto microseconds = [cus](const Plan& p) {
-    const int slots = cus * (p.kg == 1 ? 2 : 1);
-    const double stage = 0.134 + 0.1256 * p.nt + 0.0463 * p.mt + 0.0342 * p.mt * p.nt;
-    const int whole = p.slices > 1 ? p.whole / slots : p.tiles / slots;  // rounds
-    const int parts = p.grid - whole * slots, full = parts / slots, rest = parts - full * slots;
-    // a last round with one workgroup per CU where there is room for two is the faster one
-    const double rounds = full + (rest == 0 ? 0. : p.kg == 1 && rest <= cus ? 0.62 : 1.);
-    double us = 7.55 + whole * (p.stages * stage - 2.89) + rounds * ((p.stages + p.slices - 1) / p.slices * stage - 2.89);
-    if (p.slices > 1) us += 1.48 + 0.113 * p.slices * p.mt * p.nt;
-    if (p.slices > 1 && whole > 0) us += parts * (16. * p.mt * 64 * p.nt * 8) / 3e6;
+// Which tile, how many slices of K: the least of a model of the time, fitted to measured combinations (13 matrices of 1 to 178 M
+// weights, 20 to 1024 rows; the 2053 within 30 % of the best of their call: 5 % rms, and what it picks is within 0.5 % of the best on
+// average, 12 % at worst).  A workgroup takes `alone` for a stage, or `busy` times those that share its CU; a chip that is full runs
+// against its power.  Adding slices up takes trips to memory and traffic at 3 TB/s and more.
+// Slices only while all of them find room at once.  Of more tiles than that, those of the last, incomplete round may be
+// cut, with the tile left as it is (5120 x 34816 over 1024 rows: 1088 tiles, two to a CU, the last 64 in slices, 344 us; uncut 382).
+Plan make_plan(int M, int K, int N, int cus, bool fp16, bool mixed, bool silu_mul) {
+  const int form = silu_mul ? 2 : mixed ? 1 : 0;
+  auto ceil_div = [](long long a, long long b) { return (int)((a + b - 1) / b); };
+  auto microseconds = [&](const Plan& p) {
+    const Shape& sh = *p.shape;
+    const int slots = cus * sh.together, parts = p.grid - p.whole;
+    auto stretch = [&](int on_a_cu, int stages) {  // workgroups one after the other and beside each other
+      const int rounds = ceil_div(on_a_cu, sh.together);
+      return rounds * 4.47 + stages * std::max(sh.alone * rounds, sh.busy * on_a_cu);
+    };
+    const int rounds = p.whole / slots;
+    double us = stretch(rounds * sh.together, p.stages) + stretch(ceil_div(parts, cus), ceil_div(p.stages, p.slices));
+    us *= 1 + 0.17 * (std::min(1.0, (double)p.grid / cus) - 0.5);
+    us += 0.88 + (silu_mul ? 2.02 : 0.0);
+    const int pieces = silu_mul ? sh.mt : sh.mt * sh.nt, at_once = silu_mul && (sh.mt == 1 || sh.mt == 4) ? 2 : 4;
+    if (p.slices > 1)
+      us += 0.94 + 0.715 * ceil_div(pieces, sh.kg) * ceil_div(p.slices, at_once) + 0.392 * parts * (sh.rows() * 8.0 * sh.columns()) / 3e6;
     return us;
   };
   Plan best{};
   double best_us = 0.;
-  for (int mt = 1; mt <= 8; ++mt) {
-    for (int nt = 1; nt <= 4; ++nt) {
-      for (int kg = 1; kg <= 2; ++kg) {
-        if (kernel_for<false>(mt, nt, kg, mixed, silu_mul) == nullptr) continue;
-        Plan p{};
-        p.mt = mt, p.nt = nt, p.kg = kg;
-        p.tiles_m = (M + 16 * mt - 1) / (16 * mt);
-        p.tiles = p.tiles_m * ((N + 64 * nt - 1) / (64 * nt));
-        p.stages = (K + kStageK * kg - 1) / (kStageK * kg);
-        const int slots = cus * (kg == 1 ? 2 : 1);
-        for (p.slices = 1; p.slices <= 16 && p.slices <= p.stages; ++p.slices) {
-          if (p.slices > 1 && (p.tiles * p.slices > slots || p.tiles > (int)(kCounterBytes / 4))) break;
-          p.whole = p.slices > 1 ? 0 : p.tiles;
-          p.grid = p.tiles * p.slices;
-          const double us = microseconds(p);
-          if (best.grid == 0 || us < best_us) best = p, best_us = us;
-        }
-      }
-    }
-  }
-  const int slots = cus * (best.kg == 1 ? 2 : 1), cut = best.tiles % slots;
-  if (best.slices == 1 && best.tiles > slots && cut > 0) {
-    Plan p = best;
-    p.whole = best.tiles - cut;
-    for (p.slices = 2; p.slices <= 16 && p.slices <= p.stages && cut * p.slices <= 2 * slots; ++p.slices) {
-      p.grid = p.whole + cut * p.slices;
+  for (int i = 0; i < kShapes; ++i) {
+    const Shape& sh = shapes()[i];
+    if (sh.kernel[fp16][form] == nullptr) continue;
+    Plan p{};
+    p.shape = &sh;
+    p.tiles_m = ceil_div(M, sh.rows());
+    const long long tiles = (long long)p.tiles_m * ceil_div(N, sh.columns());
+    if (tiles > 0x7fffffff / 16) continue;
+    p.tiles = (int)tiles;
+    p.stages = ceil_div(K, kStageK * sh.kg);
+    const int slots = cus * sh.together, most = sh.kg == 1 ? 4 : 16;
+    const int rest = p.tiles % slots;
+    for (p.slices = 1; p.slices <= 16 && p.slices <= p.stages; ++p.slices) {
+      const bool all = p.tiles < slots;
+      if (p.slices > 1 && (all ? p.tiles * p.slices > slots || p.slices > most : rest == 0 || rest * p.slices > 2 * slots)) break;
+      p.whole = p.tiles - rest;
+      p.grid = p.whole + rest * p.slices;
       const double us = microseconds(p);
-      if (us < best_us) best = p, best_us = us;
+      if (best.grid == 0 || us < best_us) best = p, best_us = us;
     }
   }
-  best.workspace = best.slices > 1 ? kCounterBytes + (size_t)(best.grid - best.whole) * (16 * best.mt) * (64 * best.nt) * sizeof(float) : 0;
+  best.workspace = best.slices > 1 ? kCounterBytes + (size_t)(best.grid - best.whole) * best.shape->rows() * best.shape->columns() * sizeof(float) : 0;
   return best;
 }
 
 // The last few plans of this thread: a model asks for the same ones over and over.
-const Plan& plan(int M, int K, int N, int cus, bool mixed, bool silu_mul) {
+const Plan& plan(int M, int K, int N, int cus, bool fp16, bool mixed, bool silu_mul) {
   struct Entry {
     int M, K, N, cus, flags;
     Plan p;
   };
   static thread_local Entry cache[64] = {};
-  const int flags = (mixed ? 2 : 0) | (silu_mul ? 1 : 0);
+  const int flags = (fp16 ? 4 : 0) | (mixed ? 2 : 0) | (silu_mul ? 1 : 0);
   Entry& e = cache[((unsigned)M * 2654435761u + (unsigned)K * 40503u + (unsigned)N * 69069u + (unsigned)flags) >> 26];
   if (e.M != M || e.K != K || e.N != N || e.cus != cus || e.flags != flags)
-    e = Entry{M, K, N, cus, flags, make_plan(M, K, N, cus, mixed, silu_mul)};
+    e = Entry{M, K, N, cus, flags, make_plan(M, K, N, cus, fp16, mixed, silu_mul)};
   return e.p;
 }
 
@@ -556,7 +630,7 @@ int qmm_stream_grid();
 extern "C" size_t dflash_qmm_rows_workspace_bytes(int M, int K, int N, int group_size, int act_dtype, int sb_dtype, int epilogue) {
   using namespace dflash;
   if (!rows::covers(M, K, N, group_size, act_dtype != sb_dtype, epilogue)) return 0;
-  return rows::plan(M, K, N, qmm_stream_grid(), act_dtype != sb_dtype, epilogue != DFLASH_QMM_EPILOGUE_NONE).workspace;
+  return rows::plan(M, K, N, qmm_stream_grid(), act_dtype == DFLASH_FP16, act_dtype != sb_dtype, epilogue != DFLASH_QMM_EPILOGUE_NONE).workspace;
 }
 
 extern "C" int dflash_qmm_rows(const void* x, const uint32_t* w_q, const void* scales, const void* biases, void* y,
@@ -572,7 +646,7 @@ extern "C" int dflash_qmm_rows(const void* x, const uint32_t* w_q, const void* s
                  "with the silu-mul epilogue) (M=%d K=%d N=%d gs=%d)", M, K, N, group_size);
   DFLASH_REQUIRE(((uintptr_t)x % 16) == 0 && ((uintptr_t)w_q % 16) == 0 && ((uintptr_t)y % 8) == 0, DFLASH_ERR_ARG,
                  "dflash_qmm_rows: x and w_q must be 16-byte aligned");
-  const rows::Plan& p = rows::plan(M, K, N, qmm_stream_grid(), mixed, silu_mul);
+  const rows::Plan& p = rows::plan(M, K, N, qmm_stream_grid(), act_dtype == DFLASH_FP16, mixed, silu_mul);
   DFLASH_REQUIRE(p.workspace == 0 || (workspace && workspace_bytes >= p.workspace), DFLASH_ERR_WORKSPACE,
                  "dflash_qmm_rows: workspace of %zu bytes needed, %zu given", p.workspace, workspace ? workspace_bytes : (size_t)0);
   rows::Args a;
@@ -584,19 +658,19 @@ extern "C" int dflash_qmm_rows(const void* x, const uint32_t* w_q, const void* s
   a.group_shift = group_size == 32 ? 5 : group_size == 64 ? 6 : 7;
   a.tiles_m = p.tiles_m; a.tiles = p.tiles; a.whole = p.whole; a.slices = p.slices; a.stages = p.stages;
   const bool fp16 = act_dtype == DFLASH_FP16;
-  const void* fn = fp16 ? rows::kernel_for<true>(p.mt, p.nt, p.kg, mixed, silu_mul)
-                        : rows::kernel_for<false>(p.mt, p.nt, p.kg, mixed, silu_mul);
-  const int lds_bytes = rows::lds_bytes(p.mt, p.nt, p.kg);
-  static bool attr_set[kMaxDevices][8][9][5][3] = {};
+  const int form = silu_mul ? 2 : mixed ? 1 : 0;
+  const void* const fn = p.shape->kernel[fp16][form];
+  const int lds_bytes = p.shape->lds;
+  static bool attr_set[kMaxDevices][rows::kShapes][2][3] = {};
   const int dev = current_device_slot();
   if (lds_bytes > 48 * 1024) {
-    bool& set = attr_set[dev][4 * silu_mul + 2 * fp16 + mixed][p.mt][p.nt][p.kg];
+    bool& set = attr_set[dev][p.shape - rows::shapes()][fp16][form];
     if (!set || dev == kMaxDevices - 1) {
       DFLASH_HIP_OK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes));
       set = true;
     }
   }
   void* args[] = {&a};
-  DFLASH_HIP_OK(hipLaunchKernel(fn, dim3((unsigned)p.grid), dim3(256 * p.kg), args, (size_t)lds_bytes, (hipStream_t)stream));
+  DFLASH_HIP_OK(hipLaunchKernel(fn, dim3((unsigned)p.grid), dim3(64 * p.shape->w * p.shape->kg), args, (size_t)lds_bytes, (hipStream_t)stream));
   return DFLASH_OK;
 }

@@ -34,6 +34,37 @@ def test_rows_against_fp64(native_lib, M, K, N, group, dtype):
     assert (y.double() - exact).norm() <= eps * exact.norm()
 
 
+# a call for every tile shape there is: K that ends inside a stage, N and M that end inside a tile, whole and sliced
+TILE_SHAPES = [(17, 288, 16, 32), (17, 2080, 48, 32), (20, 96, 528, 32), (17, 160, 8208, 32), (17, 96, 6160, 32), (33, 288, 2064, 32),
+               (45, 96, 2064, 32), (33, 160, 12432, 32), (65, 160, 3088, 32), (129, 160, 6160, 32), (129, 96, 12432, 32), (65, 96, 1552, 32),
+               (400, 160, 8208, 32), (300, 96, 12432, 32), (97, 4416, 2064, 64), (200, 3136, 1552, 64), (1000, 1664, 5136, 128)]
+TILE_SHAPES_SILU = [(17, 160, 32, 32), (31, 1056, 96, 32), (20, 96, 544, 32), (33, 160, 6176, 32), (40, 2080, 4128, 32), (400, 96, 16416, 32),
+                    (65, 160, 6176, 32), (77, 2080, 4128, 32), (33, 96, 24864, 32), (193, 160, 16416, 32), (1000, 96, 16416, 32),
+                    (200, 96, 16416, 32), (130, 1984, 4256, 64)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,K,N,group,silu", [(*t, False) for t in TILE_SHAPES] + [(*t, True) for t in TILE_SHAPES_SILU])
+def test_every_tile_shape_at_its_edges(native_lib, M, K, N, group, silu, dtype):
+    c = make_qmm_case(K, N, 4000 + M, group_size=group, dtype=dtype, M=M).to(DEV)
+    if silu:
+        c.scales.mul_(0.05); c.biases.mul_(0.05)
+    y = rows_matmul(c.x, c.w, c.scales, c.biases, group_size=group, epilogue="silu_mul" if silu else None)
+    assert torch.equal(y, rows_matmul(c.x, c.w, c.scales, c.biases, group_size=group, epilogue="silu_mul" if silu else None))
+    dense = dequantize(c.w, c.scales, c.biases, group, 4, dtype=dtype).double()
+    exact, size = c.x.double() @ dense.t().contiguous(), c.x.double().abs() @ dense.abs().t().contiguous()
+    eps = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    err = size * 2.0 ** -24 * K ** 0.5 + 1e-6
+    if silu:  # five roundings between the sums and the result, the sums' own errors with the slopes of the factors (silu's is below 1.1)
+        (gate, up), (eg, eu) = exact.split(N // 2, dim=-1), err.split(N // 2, dim=-1)
+        act = gate * torch.sigmoid(gate)
+        err = 5 * eps * ((act * up).abs() + (gate * up).abs() * 0.25) + 1.1 * eg * up.abs() + eu * act.abs() + 1e-6
+        exact = act * up
+    else:
+        err = err + 1.01 * eps * exact.abs()
+    assert ((y.double() - exact).abs() <= err).all()
+
+
 def test_leading_dimensions_and_switch(native_lib, monkeypatch):
     c = make_qmm_case(512, 96, 5, M=40).to(DEV)
     y = quantized_matmul(c.x.reshape(2, 20, 512), c.w, c.scales, c.biases)
