@@ -1,4 +1,5 @@
-"""ctypes binding of libdflash_mi355.so (the C ABI declared in include/dflash_mi355.h).
+"""ctypes binding of libdflash_mi355.so (the C ABI declared in include/dflash_mi355.h), and the module
+that issues its common launches from native code (``host``, csrc/host.cpp).
 
 There is no software fallback: if the library has not been built, or an entry
 point reports an error, the caller gets an exception.
@@ -6,6 +7,7 @@ point reports an error, the caller gets an exception.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 from typing import Optional
 
@@ -14,6 +16,7 @@ from torch.autograd import forward_ad
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libdflash_mi355.so")
+HOST_PATH = os.path.join(_HERE, "_dflash_host.so")
 
 ABI_VERSION = 21
 
@@ -194,8 +197,31 @@ def lib() -> ctypes.CDLL:
     return loaded
 
 
+_host = None
+
+
+def host():
+    """The native launch path (csrc/host.cpp).  Its functions serve the ordinary form of a call and return
+    None for everything else, which the Python that asked then does by itself."""
+    return _host if _host is not None else _load_host()
+
+
+def _load_host():
+    global _host
+    lib()  # (the module is linked against it)
+    if not os.path.exists(HOST_PATH):
+        raise NativeLibraryError(f"{HOST_PATH} not found: build it with `python dflash-mlx_amd/build_ext.py`")
+    spec = importlib.util.spec_from_file_location("_dflash_host", HOST_PATH)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    module.bind(NativeLibraryError)
+    _host = module
+    return module
+
+
 def is_built() -> bool:
-    return _lib is not None or os.path.exists(LIB_PATH)  # (a look at the file costs a microsecond)
+    # (a look at the files costs microseconds)
+    return _lib is not None or (os.path.exists(LIB_PATH) and os.path.exists(HOST_PATH))
 
 
 def env(key: bytes) -> Optional[bytes]:

@@ -1,0 +1,565 @@
+// Host side of the launches, native: the checks, allocations and argument lists of the calls a decoding step is made of.
+//
+// A 16-row projection takes 6 to 20 us of device time, and issued from Python its launch took 12 us around the 3.5 us of
+// the HIP runtime: extents and types compared one attribute at a time, results allocated through the argument parser, every
+// pointer and number converted for ctypes.  Here the same is done on the tensors themselves.  One verify_matmul of
+// 1024 x 512 13.9 -> 6.9 us (its device time: 6.0), a GatedDeltaNet layer's verify block with its rollback 106 -> 51 us (49),
+// the attention layer of one over 4096 keys 81 -> 54 us, one token through the projections of a 9B-shaped layer 61 -> 44 us.
+//
+// Each function serves the ordinary form of a call - strided device tensors of the exact extents, in one piece - and
+// returns None for every other form and for whatever it would have to refuse: the Python function that asked then goes on
+// as if it had not, copying, falling back to the array operators, or raising.  So nothing is decided here about what a
+// call means, only how fast the common form of it gets to the device.  What Python holds (workspaces, options in the
+// environment) is passed in, never kept; tensors are only held while a function runs.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/Device.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/object_ptr.h>
+#include <torch/csrc/utils/pybind.h>
+
+#include <initializer_list>
+
+#include "dflash_mi355.h"
+
+namespace {
+
+PyObject* g_error = nullptr;  // _native.NativeLibraryError
+
+using at::Tensor;
+
+constexpr int kNoCode = -1;
+
+int dtype_code(at::ScalarType t) {
+  return t == at::kBFloat16 ? DFLASH_BF16 : t == at::kHalf ? DFLASH_FP16 : t == at::kFloat ? DFLASH_FP32 : kNoCode;
+}
+int half_code(at::ScalarType t) { return t == at::kFloat ? kNoCode : dtype_code(t); }
+
+// A tensor that is memory on the device and nothing else: no subclass, no wrapper of a transform, no lazy conjugate.
+const Tensor* device_tensor(PyObject* o) {
+  if (!THPVariable_CheckExact(o)) return nullptr;
+  const Tensor& t = THPVariable_Unpack(o);
+  static const c10::DispatchKeySet ordinary =
+      c10::DispatchKeySet({c10::DispatchKey::Dense, c10::DispatchKey::ADInplaceOrView, c10::DispatchKey::AutogradFunctionality,
+                           c10::DispatchKey::AutocastCUDA}) | c10::DispatchKeySet(c10::BackendComponent::CUDABit);
+  if (!t.defined() || (t.key_set().raw_repr() & ~ordinary.raw_repr()) != 0 || !t.is_cuda() || !t.has_storage()) return nullptr;
+  return &t;
+}
+bool is_matrix(const Tensor& t, int64_t a, int64_t b) { return t.dim() == 2 && t.size(0) == a && t.size(1) == b && t.is_contiguous(); }
+bool has_shape(const Tensor& t, std::initializer_list<int64_t> shape) { return t.sizes() == at::IntArrayRef(shape); }
+bool aligned(const void* p, uintptr_t n) { return (reinterpret_cast<uintptr_t>(p) & (n - 1)) == 0; }
+const void* at_of(const Tensor& t) { return t.const_data_ptr(); }
+
+void* stream_of(const Tensor& t) { return (void*)c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+
+bool integer(PyObject* o, long* out) {
+  if (!PyLong_CheckExact(o)) return false;
+  int overflow = 0;
+  *out = PyLong_AsLongAndOverflow(o, &overflow);
+  return overflow == 0 && *out >= 0 && *out < (1l << 31);
+}
+bool integer(PyObject* o, int* out) {
+  long v = 0;
+  if (!integer(o, &v)) return false;
+  *out = (int)v;
+  return true;
+}
+
+// The scratch that Python keeps for a key in one of its dictionaries, if there is enough of it; undefined if not.
+Tensor kept_workspace(PyObject* held, PyObject* key, size_t need) {
+  Tensor ws;
+  if (key != nullptr && PyDict_CheckExact(held)) {
+    PyObject* entry = PyDict_GetItemWithError(held, key);
+    const Tensor* t = entry == nullptr ? nullptr : device_tensor(entry);
+    if (t != nullptr && (size_t)t->nbytes() >= need && t->is_contiguous()) ws = *t;
+  }
+  Py_XDECREF(key);
+  if (PyErr_Occurred()) PyErr_Clear();
+  return ws;
+}
+PyObject* by_index(const Tensor& x, void* stream) {
+  return Py_BuildValue("(iK)", (int)x.device().index(), (unsigned long long)(uintptr_t)stream);
+}
+
+PyObject* fail(int rc, const char* what) {
+  PyErr_Format(g_error == nullptr ? PyExc_RuntimeError : g_error, "%s failed (code %d): %s", what, rc, dflash_last_error());
+  return nullptr;
+}
+
+// Runs `work` (allocations and launches) without the interpreter lock, as the calls did that this replaces.
+template <class F>
+int released(F&& work) {
+  pybind11::gil_scoped_release release;
+  return work();
+}
+
+std::vector<int64_t> rows_by(const Tensor& x, int64_t n) {
+  std::vector<int64_t> shape(x.sizes().begin(), x.sizes().end());
+  shape.back() = n;
+  return shape;
+}
+
+// ---- 4-bit products -------------------------------------------------------------------------------------------------
+struct Product {
+  const Tensor *x, *w, *s, *b;
+  int64_t rows;
+  int K, N, group, act, sb;
+};
+
+// x [.., K], w [N, K/8] of 32-bit words, scales and biases [N, K/group], all in one piece on one device.
+bool product_of(PyObject* const* a, Product* p) {
+  p->x = device_tensor(a[0]), p->w = device_tensor(a[1]), p->s = device_tensor(a[2]), p->b = device_tensor(a[3]);
+  if (!p->x || !p->w || !p->s || !p->b || !integer(a[4], &p->group)) return false;
+  const Tensor &x = *p->x, &w = *p->w, &s = *p->s, &b = *p->b;
+  if (p->group != 32 && p->group != 64 && p->group != 128) return false;
+  if (x.dim() < 1 || w.dim() != 2 || w.element_size() != 4) return false;
+  const int64_t K = x.size(-1), N = w.size(0);
+  if (K < p->group || K >= (1 << 30) || N < 1 || N >= (1 << 30) || K % p->group != 0 || N % 16 != 0) return false;
+  p->K = (int)K, p->N = (int)N, p->rows = x.numel() / K;
+  p->act = half_code(x.scalar_type()), p->sb = half_code(s.scalar_type());
+  return p->rows >= 1 && p->rows < (1 << 30) && p->act != kNoCode && p->sb != kNoCode && b.scalar_type() == s.scalar_type() &&
+         x.is_contiguous() && is_matrix(w, N, K / 8) && is_matrix(s, N, K / p->group) && is_matrix(b, N, K / p->group) &&
+         w.device() == x.device() && s.device() == x.device() && b.device() == x.device();
+}
+
+// qmm_m16(x, w, scales, biases, group_size, kernel, workspaces): the verify product of 16 rows, variant chosen as "auto" does.
+PyObject* qmm_m16(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Product p;
+  int kernel;
+  if (n != 7 || !product_of(a, &p) || p.rows != 16 || !integer(a[5], &kernel)) Py_RETURN_NONE;
+  const bool pipe = p.K >= 8192 || p.N <= 8192;
+  const int variant = pipe ? DFLASH_QMM_MMA2BIG_PIPE : DFLASH_QMM_MMA2BIG, parts = pipe ? 8 : 1;
+  if (p.N % 32 != 0 || p.K % (32 * parts) != 0) Py_RETURN_NONE;
+  void* stream = stream_of(*p.x);
+  const size_t need = dflash_qmm_m16_workspace_bytes(p.K, p.N, p.group, variant, parts, kernel);
+  Tensor ws, y;
+  if (need != 0 && !(ws = kept_workspace(a[6], by_index(*p.x, stream), need)).defined()) Py_RETURN_NONE;
+  const int rc = released([&] {
+    y = at::empty(rows_by(*p.x, p.N), p.x->options());
+    return dflash_qmm_m16(at_of(*p.x), (const uint32_t*)at_of(*p.w), at_of(*p.s), at_of(*p.b), y.mutable_data_ptr(),
+                          need ? ws.mutable_data_ptr() : nullptr, need ? ws.nbytes() : 0, p.K, p.N, p.group, p.act, p.sb,
+                          variant, parts, kernel, stream);
+  });
+  return rc != 0 ? fail(rc, "dflash_qmm_m16") : THPVariable_Wrap(std::move(y));
+  END_HANDLE_TH_ERRORS
+}
+
+// qmm_packed(x, codes, scales, biases, K, N, group_size, workspaces): the same on images of pack_weights.
+PyObject* qmm_packed(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 8) Py_RETURN_NONE;
+  const Tensor *x = device_tensor(a[0]), *w = device_tensor(a[1]), *s = device_tensor(a[2]), *b = device_tensor(a[3]);
+  int K, N, group;
+  if (!x || !w || !s || !b || !integer(a[4], &K) || !integer(a[5], &N) || !integer(a[6], &group)) Py_RETURN_NONE;
+  const int act = half_code(x->scalar_type()), sb = half_code(s->scalar_type());
+  if (act == kNoCode || sb == kNoCode || x->dim() < 1 || x->size(-1) != K || x->numel() != 16 * (int64_t)K ||
+      !x->is_contiguous() || w->device() != x->device())
+    Py_RETURN_NONE;
+  void* stream = stream_of(*x);
+  const size_t need = dflash_qmm_m16_workspace_bytes(K, N, group, DFLASH_QMM_MMA2BIG, 1, DFLASH_QMM_KERNEL_STREAM);
+  Tensor y, ws = kept_workspace(a[7], by_index(*x, stream), need);
+  if (!ws.defined()) Py_RETURN_NONE;
+  const int rc = released([&] {
+    y = at::empty(rows_by(*x, N), x->options());
+    return dflash_qmm_m16_packed(at_of(*x), at_of(*w), at_of(*s), at_of(*b), y.mutable_data_ptr(), ws.mutable_data_ptr(),
+                                 ws.nbytes(), K, N, group, act, sb, stream);
+  });
+  return rc != 0 ? fail(rc, "dflash_qmm_m16_packed") : THPVariable_Wrap(std::move(y));
+  END_HANDLE_TH_ERRORS
+}
+
+// qmm_few(x, w, scales, biases, group_size, kernel, workspaces): 1 to 16 rows outside the verify switch.
+PyObject* qmm_few(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Product p;
+  int kernel;
+  if (n != 7 || !product_of(a, &p) || p.rows > 16 || !integer(a[5], &kernel)) Py_RETURN_NONE;
+  if (p.rows < 16 && !aligned(at_of(*p.x), 16)) Py_RETURN_NONE;
+  void* stream = stream_of(*p.x);
+  const size_t need = dflash_qmm_m16_workspace_bytes(p.K, p.N, p.group, DFLASH_QMM_MMA2BIG, 1, kernel);
+  Tensor ws, y;
+  if (need != 0 && !(ws = kept_workspace(a[6], by_index(*p.x, stream), need)).defined()) Py_RETURN_NONE;
+  const int rc = released([&] {
+    y = at::empty(rows_by(*p.x, p.N), p.x->options());
+    return dflash_qmm_few(at_of(*p.x), (const uint32_t*)at_of(*p.w), at_of(*p.s), at_of(*p.b), y.mutable_data_ptr(),
+                          need ? ws.mutable_data_ptr() : nullptr, need ? ws.nbytes() : 0, (int)p.rows, p.K, p.N, p.group,
+                          p.act, p.sb, kernel, stream);
+  });
+  return rc != 0 ? fail(rc, "dflash_qmm_few") : THPVariable_Wrap(std::move(y));
+  END_HANDLE_TH_ERRORS
+}
+
+// qmm_few_silu_mul(x, w, scales, biases, group_size, workspaces): the gated activation of 1 to 16 rows.
+PyObject* qmm_few_silu_mul(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Product p;
+  if (n != 6 || !product_of(a, &p) || p.rows > 16 || p.act != p.sb) Py_RETURN_NONE;
+  if (!aligned(at_of(*p.x), 16) || !aligned(at_of(*p.w), 16) || !aligned(at_of(*p.s), 4) || !aligned(at_of(*p.b), 4)) Py_RETURN_NONE;
+  const size_t need = dflash_qmm_few_silu_mul_workspace_bytes(p.K, p.N, p.group);
+  if (need == 0) Py_RETURN_NONE;
+  void* stream = stream_of(*p.x);
+  Tensor y, ws = kept_workspace(a[5], by_index(*p.x, stream), need);
+  if (!ws.defined()) Py_RETURN_NONE;
+  const int rc = released([&] {
+    y = at::empty(rows_by(*p.x, p.N / 2), p.x->options());
+    return dflash_qmm_few_silu_mul(at_of(*p.x), (const uint32_t*)at_of(*p.w), at_of(*p.s), at_of(*p.b), y.mutable_data_ptr(),
+                                   ws.mutable_data_ptr(), ws.nbytes(), (int)p.rows, p.K, p.N, p.group, p.act, stream);
+  });
+  return rc != 0 ? fail(rc, "dflash_qmm_few_silu_mul") : THPVariable_Wrap(std::move(y));
+  END_HANDLE_TH_ERRORS
+}
+
+// qmm_rows(x, w, scales, biases, group_size, epilogue, workspaces): any number of rows.  Not on a stream that records: the
+// scratch of a recorded launch is its own, which Python sees to.
+PyObject* qmm_rows(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Product p;
+  int epilogue;
+  if (n != 7 || !product_of(a, &p) || !integer(a[5], &epilogue)) Py_RETURN_NONE;
+  const bool silu = epilogue == DFLASH_QMM_EPILOGUE_SILU_MUL;
+  if ((silu && (p.N % 32 != 0 || p.act != p.sb)) || !aligned(at_of(*p.x), 16) || !aligned(at_of(*p.w), 16)) Py_RETURN_NONE;
+  void* stream = stream_of(*p.x);
+  const size_t need = dflash_qmm_rows_workspace_bytes((int)p.rows, p.K, p.N, p.group, p.act, p.sb, epilogue);
+  Tensor y, ws;
+  if (need != 0) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing((hipStream_t)stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone) Py_RETURN_NONE;
+    if (!(ws = kept_workspace(a[6], by_index(*p.x, stream), need)).defined()) Py_RETURN_NONE;
+  }
+  const int rc = released([&] {
+    y = at::empty(rows_by(*p.x, silu ? p.N / 2 : p.N), p.x->options());
+    return dflash_qmm_rows(at_of(*p.x), (const uint32_t*)at_of(*p.w), at_of(*p.s), at_of(*p.b), y.mutable_data_ptr(),
+                           need ? ws.mutable_data_ptr() : nullptr, need ? ws.nbytes() : 0, (int)p.rows, p.K, p.N, p.group,
+                           p.act, p.sb, epilogue, stream);
+  });
+  return rc != 0 ? fail(rc, "dflash_qmm_rows") : THPVariable_Wrap(std::move(y));
+  END_HANDLE_TH_ERRORS
+}
+
+// gather(x, w, scales, biases, ids, group_size, streaming, workspaces): a row of x with the expert ids names, w [E, N, K/8].
+PyObject* gather(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 8) Py_RETURN_NONE;
+  const Tensor *x = device_tensor(a[0]), *w = device_tensor(a[1]), *s = device_tensor(a[2]), *b = device_tensor(a[3]),
+               *ids = device_tensor(a[4]);
+  int group;
+  if (!x || !w || !s || !b || !ids || !integer(a[5], &group) || group < 1 || x->dim() < 1 || w->dim() != 3) Py_RETURN_NONE;
+  const int64_t K = x->size(-1), E = w->size(0), N = w->size(1);
+  if (K < group || K >= (1 << 30) || E < 1 || E >= (1 << 30) || N < 1 || N >= (1 << 30)) Py_RETURN_NONE;
+  const int64_t P = x->numel() / K;
+  const int act = half_code(x->scalar_type()), sb = half_code(s->scalar_type());
+  if (P < 1 || P >= (1 << 30) || act == kNoCode || sb == kNoCode || b->scalar_type() != s->scalar_type() || w->element_size() != 4 ||
+      ids->scalar_type() != at::kInt || ids->numel() != P || !has_shape(*w, {E, N, K / 8}) ||
+      !has_shape(*s, {E, N, K / group}) || !has_shape(*b, {E, N, K / group}))
+    Py_RETURN_NONE;
+  for (const Tensor* t : {x, w, s, b, ids})
+    if (!t->is_contiguous() || t->device() != x->device()) Py_RETURN_NONE;
+  void* stream = stream_of(*x);
+  const size_t need =
+      a[6] == Py_True ? dflash_qmm_m16_gather_workspace_bytes((int)P, (int)K, (int)N, (int)E, group) : 0;
+  Tensor ws, y;
+  if (need != 0 && !(ws = kept_workspace(a[7], by_index(*x, stream), need)).defined()) Py_RETURN_NONE;
+  const int rc = released([&] {
+    y = at::empty(rows_by(*x, N), x->options());
+    return dflash_qmm_m16_gather(at_of(*x), (const int32_t*)at_of(*ids), (const uint32_t*)at_of(*w), at_of(*s), at_of(*b),
+                                 y.mutable_data_ptr(), need ? ws.mutable_data_ptr() : nullptr, need ? ws.nbytes() : 0, (int)P,
+                                 (int)K, (int)N, (int)E, group, act, sb, stream);
+  });
+  return rc != 0 ? fail(rc, "dflash_qmm_m16_gather") : THPVariable_Wrap(std::move(y));
+  END_HANDLE_TH_ERRORS
+}
+
+// chain_bind(problem, x, x_before, columns): points a planned one-problem launch at other rows and at a result of their
+// shape, which it returns.  problem: address of the caller's dflash_qmm_problem; x_before: rows of the type it was planned for.
+PyObject* chain_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 4 || !PyLong_CheckExact(a[0])) Py_RETURN_NONE;
+  const Tensor *x = device_tensor(a[1]), *before = device_tensor(a[2]);
+  int cols;
+  if (!x || !before || !integer(a[3], &cols)) Py_RETURN_NONE;
+  auto* problem = (dflash_qmm_problem*)PyLong_AsVoidPtr(a[0]);
+  if (problem == nullptr || problem->wait_for >= 0 || x->dim() < 1 || x->size(-1) != problem->K || x->numel() != 16 * (int64_t)problem->K ||
+      !x->is_contiguous() || x->scalar_type() != before->scalar_type() || x->device() != before->device())
+    Py_RETURN_NONE;
+  Tensor out = at::empty(rows_by(*x, cols), x->options());
+  problem->x = at_of(*x);
+  problem->y = out.mutable_data_ptr();
+  return THPVariable_Wrap(std::move(out));
+  END_HANDLE_TH_ERRORS
+}
+
+// chain_launch(problems, count, need, group_size, act, scales, spin_limit, flags, x, workspaces): the workspace it used.
+PyObject* chain_launch(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 10 || !PyLong_CheckExact(a[0])) Py_RETURN_NONE;
+  int count, group, act, sb, spin, flags;
+  long need;
+  const Tensor* x = device_tensor(a[8]);
+  if (!x || !integer(a[1], &count) || !integer(a[2], &need) || !integer(a[3], &group) || !integer(a[4], &act) ||
+      !integer(a[5], &sb) || !integer(a[6], &spin) || !integer(a[7], &flags))
+    Py_RETURN_NONE;
+  const auto* problems = (const dflash_qmm_problem*)PyLong_AsVoidPtr(a[0]);
+  void* stream = stream_of(*x);
+  Tensor ws = kept_workspace(a[9], by_index(*x, stream), (size_t)need);
+  if (problems == nullptr || !ws.defined()) Py_RETURN_NONE;
+  const int rc = released([&] {
+    return dflash_qmm_m16_chain(problems, count, ws.mutable_data_ptr(), ws.nbytes(), group, act, sb, spin, flags, stream);
+  });
+  return rc != 0 ? fail(rc, "dflash_qmm_m16_chain") : THPVariable_Wrap(std::move(ws));
+  END_HANDLE_TH_ERRORS
+}
+
+// columns(product, bounds): product[..., lo:hi] for every pair of bounds.
+PyObject* columns(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  const Tensor* t = n == 2 ? device_tensor(a[0]) : nullptr;
+  if (t == nullptr || t->dim() < 1 || !PyList_CheckExact(a[1])) Py_RETURN_NONE;
+  const Py_ssize_t count = PyList_GET_SIZE(a[1]);
+  const int64_t width = t->size(-1);
+  THPObjectPtr out(PyTuple_New(count));
+  if (!out) return nullptr;
+  for (Py_ssize_t i = 0; i < count; ++i) {
+    PyObject* pair = PyList_GET_ITEM(a[1], i);
+    long lo, hi;
+    if (!PyTuple_CheckExact(pair) || PyTuple_GET_SIZE(pair) != 2 || !integer(PyTuple_GET_ITEM(pair, 0), &lo) ||
+        !integer(PyTuple_GET_ITEM(pair, 1), &hi) || lo > hi || hi > width)
+      Py_RETURN_NONE;
+    PyObject* part = THPVariable_Wrap(t->narrow(-1, lo, hi - lo));
+    if (part == nullptr) return nullptr;
+    PyTuple_SET_ITEM(out.get(), i, part);
+  }
+  return out.release();
+  END_HANDLE_TH_ERRORS
+}
+
+// ---- GatedDeltaNet ----------------------------------------------------------------------------------------------------
+// gdn_prepare(qkv, conv_state, conv_w, a, b, A_log, dt_bias, qkv_out, Hk, Hv, Dk, Dv, eps): without a mask;
+// (conv_next, q, k, v, g, beta).
+PyObject* gdn_prepare(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 13) Py_RETURN_NONE;
+  const Tensor *qkv = device_tensor(a[0]), *cs = nullptr, *w = device_tensor(a[2]), *ga = device_tensor(a[3]),
+               *gb = device_tensor(a[4]), *A = device_tensor(a[5]), *dt = device_tensor(a[6]), *out = nullptr;
+  if (!qkv || !w || !ga || !gb || !A || !dt || qkv->dim() != 3) Py_RETURN_NONE;
+  if (a[1] != Py_None && !(cs = device_tensor(a[1]))) Py_RETURN_NONE;
+  if (a[7] != Py_None && !(out = device_tensor(a[7]))) Py_RETURN_NONE;
+  int Hk, Hv, Dk, Dv;
+  if (!integer(a[8], &Hk) || !integer(a[9], &Hv) || !integer(a[10], &Dk) || !integer(a[11], &Dv) || !PyFloat_CheckExact(a[12]))
+    Py_RETURN_NONE;
+  const auto covers = [](int d) { return d > 0 && d <= 256 && d % 64 == 0; };
+  const int code = dtype_code(qkv->scalar_type()), param = dtype_code(A->scalar_type());
+  const int64_t B = qkv->size(0), S = qkv->size(1), C = qkv->size(2);
+  if (code == kNoCode || param == kNoCode || !covers(Dk) || !covers(Dv) || B < 1 || S < 1 || B * S >= (1 << 30) ||
+      Hk > (1 << 15) || Hv > (1 << 15) || C != 2 * (int64_t)Hk * Dk + (int64_t)Hv * Dv)
+    Py_RETURN_NONE;
+  if (w->dim() < 2 || w->dim() > 3 || w->size(0) != C || (w->dim() == 3 && w->size(2) != 1) || !w->is_contiguous()) Py_RETURN_NONE;
+  const int64_t K = w->size(1);
+  const auto type = qkv->scalar_type();
+  const auto device = qkv->device();
+  if (K < 2 || K > 4 || w->scalar_type() != type || ga->scalar_type() != type || gb->scalar_type() != type ||
+      dt->scalar_type() != A->scalar_type() || !has_shape(*ga, {B, S, Hv}) || !has_shape(*gb, {B, S, Hv}) ||
+      !has_shape(*A, {Hv}) || !has_shape(*dt, {Hv}) || !A->is_contiguous() || !dt->is_contiguous() || w->device() != device ||
+      ga->device() != device || gb->device() != device || A->device() != device || dt->device() != device)
+    Py_RETURN_NONE;
+  if (cs && (cs->scalar_type() != type || !has_shape(*cs, {B, K - 1, C}) || cs->device() != device || !cs->is_contiguous()))
+    Py_RETURN_NONE;
+  if (out && (out->scalar_type() != type || !has_shape(*out, {B, S, C}) || out->device() != device || !out->is_contiguous()))
+    Py_RETURN_NONE;
+  const int64_t step = qkv->element_size();
+  if (qkv->stride(2) != 1 || ((int64_t)(uintptr_t)at_of(*qkv) | qkv->stride(0) * step | qkv->stride(1) * step) % 8 != 0 ||
+      ga->stride(2) != 1 || gb->stride(2) != 1)
+    Py_RETURN_NONE;
+  const long long strides[6] = {qkv->stride(0), qkv->stride(1), ga->stride(0), ga->stride(1), gb->stride(0), gb->stride(1)};
+  void* stream = stream_of(*qkv);
+  const float eps = (float)PyFloat_AS_DOUBLE(a[12]);
+  Tensor next, q, k, v, g, beta;
+  const int rc = released([&] {
+    const auto options = qkv->options();
+    next = at::empty({B, K - 1, C}, options);
+    q = at::empty({B, S, Hk, Dk}, options);
+    k = at::empty({B, S, Hk, Dk}, options);
+    v = at::empty({B, S, Hv, Dv}, options);
+    g = at::empty({B, S, Hv}, options.dtype(at::kFloat));
+    beta = at::empty({B, S, Hv}, options);
+    return dflash_gdn_prepare_rows(at_of(*qkv), cs ? at_of(*cs) : nullptr, at_of(*w), at_of(*ga), at_of(*gb), at_of(*A), at_of(*dt),
+                                   nullptr, next.mutable_data_ptr(), q.mutable_data_ptr(), k.mutable_data_ptr(),
+                                   v.mutable_data_ptr(), (float*)g.mutable_data_ptr(), beta.mutable_data_ptr(),
+                                   out ? out->mutable_data_ptr() : nullptr, strides, (int)B, (int)S, Hk, Hv, Dk, Dv, (int)K, code,
+                                   param, eps, stream);
+  });
+  if (rc != 0) return fail(rc, "dflash_gdn_prepare");
+  return Py_BuildValue("(NNNNNN)", THPVariable_Wrap(std::move(next)), THPVariable_Wrap(std::move(q)), THPVariable_Wrap(std::move(k)),
+                       THPVariable_Wrap(std::move(v)), THPVariable_Wrap(std::move(g)), THPVariable_Wrap(std::move(beta)));
+  END_HANDLE_TH_ERRORS
+}
+
+// gdn_forward(q, k, v, g, beta, state, z, weight, eps, with_tape): without a mask, gates per head; z and weight None, or the
+// gate and the weight of the output norm.  (y, state, tape or None).
+PyObject* gdn_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 10) Py_RETURN_NONE;
+  const Tensor *q = device_tensor(a[0]), *k = device_tensor(a[1]), *v = device_tensor(a[2]), *g = device_tensor(a[3]),
+               *beta = device_tensor(a[4]), *state = device_tensor(a[5]), *z = nullptr, *w = nullptr;
+  if (!q || !k || !v || !g || !beta || !state || k->dim() != 4 || v->dim() != 4 || !PyFloat_CheckExact(a[8])) Py_RETURN_NONE;
+  if (a[6] != Py_None && (!(z = device_tensor(a[6])) || !(w = device_tensor(a[7])))) Py_RETURN_NONE;
+  const int64_t B = k->size(0), T = k->size(1), hk = k->size(2), dk = k->size(3), hv = v->size(2), dv = v->size(3);
+  const int code = dtype_code(q->scalar_type()), g_code = dtype_code(g->scalar_type()), b_code = dtype_code(beta->scalar_type()),
+            s_code = dtype_code(state->scalar_type());
+  if (B < 1 || T < 1 || hk < 1 || hv < 1 || dv < 1 || hv % hk != 0 || dk < 32 || dk % 32 != 0 || B * T * hv >= (1 << 30) ||
+      code == kNoCode || g_code == kNoCode || b_code == kNoCode || s_code == kNoCode || k->scalar_type() != q->scalar_type() ||
+      v->scalar_type() != q->scalar_type())
+    Py_RETURN_NONE;
+  if (!has_shape(*q, {B, T, hk, dk}) || !has_shape(*v, {B, T, hv, dv}) || !has_shape(*g, {B, T, hv}) ||
+      !has_shape(*beta, {B, T, hv}) || !has_shape(*state, {B, hv, dv, dk}))
+    Py_RETURN_NONE;
+  for (const Tensor* t : {q, k, v, g, beta, state})
+    if (!t->is_contiguous() || t->device() != state->device()) Py_RETURN_NONE;
+  int w_code = code;
+  if (z != nullptr) {
+    w_code = dtype_code(w->scalar_type());
+    const int64_t step = z->element_size();
+    if (w_code == kNoCode || z->scalar_type() != q->scalar_type() || !has_shape(*z, {B, T, hv, dv}) ||
+        z->device() != state->device() || w->device() != state->device() || w->numel() != dv || !w->is_contiguous() ||
+        dv % 64 != 0 || dv > 256)
+      Py_RETURN_NONE;
+    if (z->stride(3) != 1 || z->stride(2) != dv || z->stride(1) == 0 || !aligned(at_of(*z), 16) ||
+        (z->stride(0) | z->stride(1)) * step % 16 != 0)
+      Py_RETURN_NONE;
+  }
+  size_t need = T > 16 ? dflash_gdn_forward_workspace_bytes((int)B, (int)T, (int)hk, (int)hv, (int)dk, (int)dv, code, 0) : 0;
+  for (const Tensor* t : {q, k, v, state})
+    if (!aligned(at_of(*t), 16)) need = 0;
+  const bool with_tape = a[9] == Py_True || need == 0 || dflash_get_option(DFLASH_OPT_GDN_STEP_BY_STEP) != 0;
+  void* stream = stream_of(*q);
+  const float eps = (float)PyFloat_AS_DOUBLE(a[8]);
+  Tensor y, next, tape, ws;
+  const int rc = released([&] {
+    const auto options = q->options();
+    y = at::empty({B, T, hv, dv}, options);
+    if (need != 0) ws = at::empty({(int64_t)need}, options.dtype(at::kByte));
+    if (with_tape) tape = at::empty({B, T, hv, dv}, options.dtype(at::kFloat));
+    next = at::empty({B, hv, dv, dk}, state->options());
+    return dflash_gdn_forward(at_of(*q), at_of(*k), at_of(*v), at_of(*g), at_of(*beta), at_of(*state), next.mutable_data_ptr(),
+                              z ? at_of(*z) : nullptr, z ? at_of(*w) : nullptr, y.mutable_data_ptr(),
+                              with_tape ? (float*)tape.mutable_data_ptr() : nullptr, nullptr,
+                              need ? ws.mutable_data_ptr() : nullptr, need, z ? z->stride(0) : 0, z ? z->stride(1) : 0, (int)B,
+                              (int)T, (int)hk, (int)hv, (int)dk, (int)dv, code, g_code, b_code, s_code, w_code, 0, eps, stream);
+  });
+  if (rc != 0) return fail(rc, "dflash_gdn_forward");
+  PyObject* tape_out = with_tape ? THPVariable_Wrap(std::move(tape)) : (Py_INCREF(Py_None), Py_None);
+  return Py_BuildValue("(NNN)", THPVariable_Wrap(std::move(y)), THPVariable_Wrap(std::move(next)), tape_out);
+  END_HANDLE_TH_ERRORS
+}
+
+// rollback_layer(tape, k, g, qkv, state, conv_prev, steps, keep, exact): replay and conv window of one cache's tape;
+// (state, conv window).
+PyObject* rollback_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 9) Py_RETURN_NONE;
+  const Tensor *tape = device_tensor(a[0]), *k = device_tensor(a[1]), *g = device_tensor(a[2]), *qkv = device_tensor(a[3]),
+               *state = device_tensor(a[4]), *prev = nullptr;
+  int steps, keep, exact;
+  if (!tape || !k || !g || !qkv || !state || tape->dim() != 4 || k->dim() != 4 || g->dim() != 3 || qkv->dim() != 3 ||
+      !integer(a[6], &steps) || !integer(a[7], &keep) || !integer(a[8], &exact) || keep < 1)
+    Py_RETURN_NONE;
+  if (a[5] != Py_None && !(prev = device_tensor(a[5]))) Py_RETURN_NONE;
+  const int64_t B = tape->size(0), T = tape->size(1), hv = tape->size(2), dv = tape->size(3), hk = k->size(2), dk = k->size(3),
+                C = qkv->size(2);
+  if (hk < 1 || steps > T || !has_shape(*k, {B, T, hk, dk}) || !has_shape(*g, {B, T, hv}) || !has_shape(*qkv, {B, T, C}) ||
+      !has_shape(*state, {B, hv, dv, dk}) || dk < 32 || dk % 32 != 0 || hv % hk != 0 ||
+      T * (dv + 2 * dk + 1) * 4 + dk * 4 > 64 * 1024)
+    Py_RETURN_NONE;
+  for (const Tensor* t : {tape, k, g, qkv, state})
+    if (!t->is_contiguous() || t->device() != state->device()) Py_RETURN_NONE;
+  if (prev && (prev->device() != qkv->device() || !prev->is_contiguous() || prev->scalar_type() != qkv->scalar_type() ||
+               !has_shape(*prev, {B, keep, C})))
+    Py_RETURN_NONE;
+  const int t_code = dtype_code(tape->scalar_type()), k_code = dtype_code(k->scalar_type()), g_code = dtype_code(g->scalar_type()),
+            s_code = dtype_code(state->scalar_type());
+  if (t_code == kNoCode || k_code == kNoCode || g_code == kNoCode || s_code == kNoCode) Py_RETURN_NONE;
+  void* stream = stream_of(*state);
+  Tensor next, conv;
+  const int rc = released([&] {
+    next = at::empty({B, hv, dv, dk}, state->options());
+    conv = at::empty({B, keep, C}, qkv->options());
+    return dflash_rollback_layer(at_of(*tape), at_of(*k), at_of(*g), at_of(*state), next.mutable_data_ptr(),
+                                 prev ? at_of(*prev) : nullptr, at_of(*qkv), conv.mutable_data_ptr(), nullptr, steps, (int)B,
+                                 (int)T, (int)hk, (int)hv, (int)dk, (int)dv, s_code, t_code, k_code, g_code, 0, exact, keep,
+                                 (int)C, (int)qkv->element_size(), stream);
+  });
+  if (rc != 0) return fail(rc, "dflash_rollback_layer");
+  return Py_BuildValue("(NN)", THPVariable_Wrap(std::move(next)), THPVariable_Wrap(std::move(conv)));
+  END_HANDLE_TH_ERRORS
+}
+
+// ---- attention --------------------------------------------------------------------------------------------------------
+// sdpa_q16(queries, keys, values, scale, gate, workspaces): a block of 16 queries without a mask; gate None, or the output
+// of the projection that carries it.
+PyObject* sdpa_q16(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 6) Py_RETURN_NONE;
+  const Tensor *q = device_tensor(a[0]), *k = device_tensor(a[1]), *v = device_tensor(a[2]), *gate = nullptr;
+  if (!q || !k || !v || q->dim() != 4 || k->dim() != 4 || v->dim() != 4 || !PyFloat_CheckExact(a[3])) Py_RETURN_NONE;
+  if (a[4] != Py_None && !(gate = device_tensor(a[4]))) Py_RETURN_NONE;
+  const int64_t B = q->size(0), hq = q->size(1), d = q->size(3), hk = k->size(1), N = k->size(2);
+  const int code = half_code(q->scalar_type());
+  if (code == kNoCode || q->size(2) != 16 || (d != 128 && d != 256) || hk < 1 || hq % hk != 0 || hq / hk > 8 || N < 16 ||
+      N >= (1 << 30) || k->scalar_type() != q->scalar_type() || v->scalar_type() != q->scalar_type() ||
+      !has_shape(*k, {B, hk, N, d}) || !has_shape(*v, {B, hk, N, d}) || k->device() != q->device() || v->device() != q->device() ||
+      !q->is_contiguous())
+    Py_RETURN_NONE;
+  for (const Tensor* t : {k, v})
+    if (t->stride(3) != 1 || (t->stride(0) | t->stride(1) | t->stride(2)) % 8 != 0 || !aligned(at_of(*t), 16)) Py_RETURN_NONE;
+  const size_t need = dflash_sdpa_q16_workspace_bytes((int)B, (int)hq, (int)hk, (int)N, (int)d);
+  void* stream = stream_of(*q);
+  Tensor out, ws;
+  if (need != 0) {
+    PyObject* key = Py_BuildValue("(NK)", THPDevice_New(q->device()), (unsigned long long)(uintptr_t)stream);
+    if (!(ws = kept_workspace(a[5], key, need)).defined()) Py_RETURN_NONE;
+  }
+  const bool gated = gate != nullptr && need != 0 && has_shape(*gate, {B, 16, hq * 2 * d}) &&
+                     gate->scalar_type() == q->scalar_type() && gate->device() == q->device() && gate->stride(2) == 1 &&
+                     (gate->stride(0) | gate->stride(1)) % 4 == 0 && aligned(at_of(*gate), 8);
+  const float scale = (float)PyFloat_AS_DOUBLE(a[3]);
+  const int rc = released([&] {
+    const auto options = q->options();
+    void* scratch = need ? ws.mutable_data_ptr() : nullptr;
+    const size_t bytes = need ? ws.nbytes() : 0;
+    if (gated) {
+      out = at::empty({B, 16, hq * d}, options);
+      return dflash_sdpa_q16_gated(at_of(*q), at_of(*k), at_of(*v), nullptr, at_of(*gate), out.mutable_data_ptr(), scratch, bytes,
+                                   (int)B, (int)hq, (int)hk, (int)N, (int)d, k->stride(0), k->stride(1), k->stride(2),
+                                   v->stride(0), v->stride(1), v->stride(2), gate->stride(0), gate->stride(1), scale, code, stream);
+    }
+    out = at::empty({B, hq, 16, d}, options);
+    return dflash_sdpa_q16(at_of(*q), at_of(*k), at_of(*v), nullptr, out.mutable_data_ptr(), scratch, bytes, (int)B, (int)hq,
+                           (int)hk, (int)N, (int)d, k->stride(0), k->stride(1), k->stride(2), v->stride(0), v->stride(1),
+                           v->stride(2), scale, code, stream);
+  });
+  return rc != 0 ? fail(rc, gated ? "dflash_sdpa_q16_gated" : "dflash_sdpa_q16") : THPVariable_Wrap(std::move(out));
+  END_HANDLE_TH_ERRORS
+}
+
+// ---- module -----------------------------------------------------------------------------------------------------------
+PyObject* bind(PyObject*, PyObject* error) {  // the class that failed launches raise
+  Py_INCREF(error);
+  Py_XDECREF(g_error);
+  g_error = error;
+  Py_RETURN_NONE;
+}
+
+#define DFLASH_HOST(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
+PyMethodDef kMethods[] = {DFLASH_HOST(qmm_m16), DFLASH_HOST(qmm_packed), DFLASH_HOST(qmm_few), DFLASH_HOST(qmm_few_silu_mul),
+                          DFLASH_HOST(qmm_rows), DFLASH_HOST(columns), DFLASH_HOST(gather), DFLASH_HOST(chain_bind), DFLASH_HOST(chain_launch), DFLASH_HOST(gdn_prepare), DFLASH_HOST(gdn_forward),
+                          DFLASH_HOST(rollback_layer), DFLASH_HOST(sdpa_q16), {"bind", bind, METH_O, nullptr},
+                          {nullptr, nullptr, 0, nullptr}};
+PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_dflash_host", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__dflash_host() { return PyModule_Create(&kModule); }

@@ -104,6 +104,10 @@ def gdn_prepare(qkv: torch.Tensor, conv_state: Optional[torch.Tensor], conv_w: t
     """Mask, conv, silu, split, norms and gates of a GatedDeltaNet call in one launch:
     (conv_next [B,K-1,C], q, k [B,S,Hk,Dk], v [B,S,Hv,Dv], g [B,S,Hv] fp32, beta [B,S,Hv]).  qkv, a and b are read where
     they are (columns of a joint product).  ``qkv_out`` [B,S,C], contiguous, receives qkv with masked rows zeroed."""
+    if mask is None and qkv.is_cuda:
+        made = _native.host().gdn_prepare(qkv, conv_state, conv_w, a, b, A_log, dt_bias, qkv_out, Hk, Hv, Dk, Dv, float(eps))
+        if made is not None:
+            return made
     B, S, C = (int(d) for d in qkv.shape)
     if conv_w.ndim == 3:            # mlx conv1d weight [C, K, 1]
         conv_w = conv_w.reshape(conv_w.shape[0], conv_w.shape[1])

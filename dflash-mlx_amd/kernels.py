@@ -111,6 +111,11 @@ def gated_delta_kernel_with_tape(q: torch.Tensor, k: torch.Tensor, v: torch.Tens
     by the same launch (``dflash_gdn_forward_tape_norm``); only for inputs the kernel takes -
     callers check ``fused_output_norm_applies`` first.  ``with_tape=False``: the caller has no use for the
     tape; long prompts then leave it out (the third result may be None)."""
+    if mask is None and state.is_cuda:
+        z, weight, eps = (None, None, 0.0) if output_norm is None else output_norm
+        made = _native.host().gdn_forward(q, k, v, g, beta, state, z, weight, float(eps), bool(with_tape))
+        if made is not None:
+            return made
     B, T, hk, dk = (int(d) for d in k.shape)
     hv, dv = int(v.shape[2]), int(v.shape[3])
     if g.ndim not in (3, 4):
@@ -365,6 +370,10 @@ def batched_sdpa_2pass_exact(queries: torch.Tensor, keys: torch.Tensor, values: 
     ``q_proj_output`` [B,16,Hq*2D] (no counterpart in the reference, which gates with array operators): the result is
     [B,16,Hq*D], every head times the sigmoid of the second half of its part of q_proj_output, where the same launch can do
     it; where it cannot (one range of keys), the plain result."""
+    if mask is None and queries.is_cuda:
+        out = _native.host().sdpa_q16(queries, keys, values, float(scale), q_proj_output, _SDPA_WORKSPACE)
+        if out is not None:
+            return out
     if queries.ndim != 4 or keys.ndim != 4 or values.ndim != 4 or not queries.is_cuda:
         return None
     bsz, hq, q_len, d = (int(x) for x in queries.shape)

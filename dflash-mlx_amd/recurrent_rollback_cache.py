@@ -187,9 +187,12 @@ class RecurrentRollbackCache:
 
     def record_tape(self, *, tape: torch.Tensor, k: torch.Tensor, g: torch.Tensor,
                     qkv: torch.Tensor) -> None:
-        if self._arena is not None:
-            self._tape, self._tape_k, self._tape_g, self._tape_qkv = self._arena._store_tape(
-                self._layer, tape, k, g, qkv)
+        arena = self._arena
+        if arena is not None:
+            kept = arena._slots[self._layer]
+            if not (tape is kept[0] and k is kept[1] and g is kept[2] and qkv is kept[3]):  # else: written where it belongs
+                kept = arena._store_tape(self._layer, tape, k, g, qkv)
+            self._tape, self._tape_k, self._tape_g, self._tape_qkv = kept
             return
         self._tape = tape.contiguous()
         self._tape_k = k.contiguous()
@@ -222,6 +225,12 @@ class RecurrentRollbackCache:
         them.  False (nothing done) for anything else, which takes the two wrappers below."""
         tape, k, g, qkv, state = self._tape, self._tape_k, self._tape_g, self._tape_qkv, self.cache[1]
         keep = self.conv_kernel_size - 1
+        if qkv is not None and state.is_cuda:
+            made = _native.host().rollback_layer(tape, k, g, qkv, state, self._snapshot[0], accepted_steps, keep,
+                                                 1 if _exact_order() else 0)
+            if made is not None:
+                self.cache[1], self.cache[0] = made
+                return True
         if (qkv is None or keep <= 0 or not (state.is_cuda and qkv.is_cuda) or tape.ndim != 4 or k.ndim != 4
                 or g.ndim != 3 or qkv.ndim != 3):
             return False
@@ -320,6 +329,7 @@ class RollbackArena:
         # 0.90 ms; the launch itself is 42 us).
         self._state_half = [[self.state[h, layer] for layer in range(L)] for h in (0, 1)]
         self._conv_half = [[self.conv[h, layer] for layer in range(L)] for h in (0, 1)]
+        self._halves = [(self.state[h], self.conv[h]) for h in (0, 1)]
         self._slots = [(self.tape[layer], self.k[layer], self.g[layer], self.qkv[layer]) for layer in range(L)]
         self._caches: List[RecurrentRollbackCache] = []
         for layer in range(L):
@@ -357,8 +367,6 @@ class RollbackArena:
     # -- used by the per-layer cache objects
     def _store_tape(self, layer: int, tape, k, g, qkv):
         dst = self._slots[layer]
-        if tape is dst[0] and k is dst[1] and g is dst[2] and qkv is dst[3]:
-            return dst  # the producer wrote into the arena: nothing to copy, no view to make
         out = []
         for d, src, name in zip(dst, (tape, k, g, qkv), ("tape", "k", "g", "qkv")):
             steps = int(src.shape[1])
@@ -391,6 +399,15 @@ class RollbackArena:
         def same(a: torch.Tensor, b: torch.Tensor) -> bool:
             return a is b or a.data_ptr() == b.data_ptr()
 
+        # the caches hold the arena's own views, all of one half: what a whole-model step leaves (48 layers: 4 us, by
+        # address and half below 20 us)
+        for half in (0, 1):
+            for c, conv, st, slots in zip(self._caches, self._conv_half[half], self._state_half[half], self._slots):
+                snap = c._snapshot
+                if snap is None or snap[0] is not conv or snap[1] is not st or c._tape is not slots[0] or c._tape_qkv is None:
+                    break
+            else:
+                return half
         half = None
         for layer, c in enumerate(self._caches):
             if c._snapshot is None or c._tape is None or c._tape_qkv is None:
@@ -444,9 +461,9 @@ class RollbackArena:
             self.steps.copy_(acc)
             steps = self.steps
         # every layer's state and conv window in one launch
-        replay_launch(self.tape, self.k, self.g, self.state[snap], self.state[nxt], steps=steps,
-                      T_alloc=self.T, slots=self.L * self.B,
-                      conv=(self.conv[snap], self.qkv, self.conv[nxt]) if self.keep > 0 else None)
-        for layer, c in enumerate(self._caches):
-            c.cache = [self._conv_half[nxt][layer], self._state_half[nxt][layer]]
+        (state_in, conv_in), (state_out, conv_out) = self._halves[snap], self._halves[nxt]
+        replay_launch(self.tape, self.k, self.g, state_in, state_out, steps=steps, T_alloc=self.T, slots=self.L * self.B,
+                      conv=(conv_in, self.qkv, conv_out) if self.keep > 0 else None)
+        for c, conv, st in zip(self._caches, self._conv_half[nxt], self._state_half[nxt]):
+            c.cache = [conv, st]
             c.clear_transients()

@@ -193,8 +193,13 @@ class FusedProjections:
     def silu_mul(self, x: torch.Tensor) -> torch.Tensor:
         """``silu(x @ W_0^T) * (x @ W_1^T)`` in one launch; a new tensor per call."""
         rows = self.bounds[0][1]
-        out = torch.empty((*x.shape[:-1], rows), dtype=x.dtype, device=x.device)
         chain = self._silu_chain
+        if chain is not None:
+            out = chain._bind_rows(x, rows)
+            if out is not None:
+                chain()
+                return out
+        out = torch.empty((*x.shape[:-1], rows), dtype=x.dtype, device=x.device)
         if chain is None:
             if self._packed_silu is not None:
                 problem = ChainProblem(x.reshape(16, -1), self._packed_silu, epilogue="silu_mul", out=out.view(16, rows))
@@ -231,7 +236,11 @@ class FusedProjections:
         else:
             product = verify_matmul(x, self.weight, self.scales, self.biases, transpose=True,
                                     group_size=self.group_size, bits=self.bits)
-        return tuple(product[..., lo:hi] for lo, hi in self.bounds)
+        return self._columns(product)
+
+    def _columns(self, product: torch.Tensor) -> Tuple[torch.Tensor, ...]:
+        parts = _native.host().columns(product, self.bounds) if product.is_cuda else None
+        return parts if parts is not None else tuple(product[..., lo:hi] for lo, hi in self.bounds)
 
 
 def silu_gate_up(parent: nn.Module, x: torch.Tensor, names: Tuple[str, str] = ("gate_proj", "up_proj")) -> torch.Tensor:
@@ -281,7 +290,7 @@ def shared_input_outputs(parent: nn.Module, names: Sequence[str], x: torch.Tenso
         elif group.serves_few(parent, x):
             product = group.few(x)
         if product is not None:
-            parts = (product[..., lo:hi] for lo, hi in group.bounds)
+            parts = group._columns(product)
             outs.update(zip(group.names, parts if columns else (part.contiguous() for part in parts)))
     return tuple(outs[n] if n in outs else getattr(parent, n)(x) for n in names)
 

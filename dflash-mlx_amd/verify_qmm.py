@@ -165,6 +165,10 @@ def verify_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases
     if not _should_use_verify(x, group_size, bits, transpose):
         return quantized_matmul(x, w, scales, biases, transpose=transpose,
                                 group_size=group_size, bits=bits)
+    if x.is_cuda and _native.env(b"DFLASH_VERIFY_VARIANT") is None:
+        y = _native.host().qmm_m16(x, w, scales, biases, group_size, _kernel_select(), _WORKSPACES)
+        if y is not None:
+            return y
 
     orig_shape = x.shape
     x2 = x.reshape(16, orig_shape[-1]).contiguous()
@@ -321,6 +325,11 @@ class QmmChain:
                              "(group 64, K % 1024 == 0, N % 32 == 0; N % 128 == 0 with an epilogue)")
 
     def __call__(self):
+        ws = _native.host().chain_launch(ctypes.addressof(self._table), self._count, self._need, self._group, self._act,
+                                         self._sb, self._spin, self._flags, self._keep[0][0], _WORKSPACES)
+        if ws is not None:
+            self._ws = ws
+            return self.outputs
         stream = _native.raw_stream(self._device)
         ws = _workspace(self._device, stream, self._need)
         self._ws = ws
@@ -353,6 +362,12 @@ class QmmChain:
                 raise ValueError(f"QmmChain.rebind: out must be a contiguous {tuple(y_old.shape)} tensor of {y_old.dtype}")
             t.y = out.data_ptr()
             self.outputs[index] = out
+
+    def _bind_rows(self, x: torch.Tensor, columns: int) -> Optional[torch.Tensor]:
+        """Points a chain of one projection at the rows of ``x`` and at a new tensor for their ``columns`` results, which is
+        returned; None (nothing done) where ``rebind`` has to look at them.  For a caller that binds before every launch: the chain
+        does not hold what it was pointed at."""
+        return _native.host().chain_bind(ctypes.addressof(self._table), x, self._keep[0][0], columns)
 
     def error_word(self) -> int:
         """0, or 1 + the index of a projection whose wait for its input was given up (read back
@@ -431,6 +446,10 @@ def verify_matmul_packed(x: torch.Tensor, packed: PackedWeights) -> torch.Tensor
     K, N = packed.K, packed.N
     if packed.gate_up:
         raise ValueError("verify_matmul_packed: these images are ordered for the silu-mul epilogue of a chain")
+    if x.is_cuda:
+        y = _native.host().qmm_packed(x, packed.codes, packed.scales, packed.biases, K, N, packed.group_size, _WORKSPACES)
+        if y is not None:
+            return y
     m = 1
     for d in x.shape[:-1]:
         m *= int(d)
@@ -464,6 +483,10 @@ def small_m_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biase
     counterpart in the reference, whose stock operator is a fused kernel of its own: here the
     stock operator dequantises the whole matrix with array ops, which for a one-token step or a
     48-row projection costs far more than the product itself."""
+    if bits == 4 and x.is_cuda and _native.plain(x, w, scales, biases) and _native.is_built():
+        y = _native.host().qmm_few(x, w, scales, biases, group_size, _kernel_select(), _WORKSPACES)
+        if y is not None:
+            return y
     if (not x.is_cuda or bits != 4 or group_size not in (32, 64, 128) or x.dtype not in _DTYPE_CODE or
             scales.dtype not in _DTYPE_CODE or biases.dtype != scales.dtype or w.ndim != 2):
         return None
@@ -501,6 +524,11 @@ def small_m_silu_mul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
     """``silu(x @ gate.T) * (x @ up.T)`` for at most 16 rows of device activations in one launch of the streaming
     kernel; ``w`` holds the gate rows of an MLP followed by its up rows.  None for what that kernel does not
     cover or ``small_m_matmul`` leaves to the array operators.  No counterpart in the reference."""
+    if (bits == 4 and x.is_cuda and _kernel_select() == _native.QMM_KERNEL_AUTO and _native.plain(x, w, scales, biases)
+            and _native.is_built()):
+        y = _native.host().qmm_few_silu_mul(x, w, scales, biases, group_size, _WORKSPACES)
+        if y is not None:
+            return y
     if (not x.is_cuda or bits != 4 or x.dtype not in _DTYPE_CODE or not (scales.dtype == biases.dtype == x.dtype)
             or w.ndim != 2 or _kernel_select() != _native.QMM_KERNEL_AUTO):
         return None
@@ -563,6 +591,12 @@ def rows_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: 
     16) and for calls that something differentiates, traces or batches (``_native.plain``).
     ``epilogue="silu_mul"``: ``w`` holds the gate rows of an MLP followed by its up rows and the result is
     ``silu(gate) * up``.  No counterpart in the reference, whose stock operator is ``mx.quantized_matmul``."""
+    if (bits == 4 and x.is_cuda and (epilogue is None or epilogue == "silu_mul") and _native.plain(x, w, scales, biases)
+            and _native.is_built()):
+        y = _native.host().qmm_rows(x, w, scales, biases, group_size, _native.QMM_EPILOGUE_NONE if epilogue is None
+                                    else _native.QMM_EPILOGUE_SILU_MUL, _ROWS_WORKSPACES)
+        if y is not None:
+            return y
     if (not x.is_cuda or bits != 4 or group_size not in (32, 64, 128) or x.dtype not in _DTYPE_CODE or
             scales.dtype not in _DTYPE_CODE or biases.dtype != scales.dtype or w.ndim != 2):
         return None
@@ -614,6 +648,10 @@ def gather_qmm(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: t
         raise NotImplementedError("only 4-bit codes are implemented")
     if not x.is_cuda:
         raise _native.NativeLibraryError("gather_qmm runs on the GPU only")
+    y = _native.host().gather(x, w, scales, biases, expert_ids, group_size, _kernel_select() != _native.QMM_KERNEL_TILE,
+                              _WORKSPACES)
+    if y is not None:
+        return y
     lib = _native.lib()
     x2 = x.reshape(-1, x.shape[-1]).contiguous()
     ids = expert_ids.reshape(-1).to(torch.int32).contiguous()
