@@ -125,6 +125,7 @@ class FusedProjections:
         first = members[0]
         self.names = tuple(names)
         self.group_size, self.bits = first.group_size, first.bits
+        self._any_variant = int(first.weight.shape[1]) * (32 // first.bits) % 512 == 0
         self.weight = torch.cat([m.weight for m in members], dim=0).contiguous()
         self.scales = torch.cat([m.scales for m in members], dim=0).contiguous()
         self.biases = torch.cat([m.biases for m in members], dim=0).contiguous()
@@ -145,7 +146,8 @@ class FusedProjections:
         pad this input and without hooks."""
         if x.numel() != 16 * x.shape[-1] or not _should_use_verify(x, self.group_size, self.bits, True):
             return False
-        return self._holds(parent, x)
+        # (a variant asked for by name may leave other widths to the stock operator: the members', then)
+        return (self._any_variant or _native.env(b"DFLASH_VERIFY_VARIANT") is None) and self._holds(parent, x)
 
     def serves_prompt(self, parent: nn.Module, x: torch.Tensor) -> bool:
         """The same for more rows than a block has, which take the any-rows product of the joint matrix
@@ -412,7 +414,7 @@ def fuse_shared_input_linears(model: nn.Module, *,
                               groups: Sequence[Sequence[str]] = SHARED_INPUT_GROUPS) -> int:
     """Joins, under every parent module, the swapped projections named by one of ``groups``
     (those present, when at least two of them are and they agree in K, group size, dtype and
-    device, K is a multiple of 512, the rows add up to a multiple of 32 and none adds a bias vector)
+    device, K is a multiple of 256, the rows add up to a multiple of 32 and none adds a bias vector)
     into a ``FusedProjections`` kept in ``parent._dflash_fused`` for ``shared_input_outputs``; narrow
     projections left out of the swap (N a multiple of 16) join too.  Call it after
     ``install_verify_linears`` and after the model sits on its device.  Returns the number of
@@ -447,10 +449,12 @@ def fuse_shared_input_linears(model: nn.Module, *,
                        m.weight.dtype == ref.weight.dtype and m.weight.device == ref.weight.device
                        for _, _, _, m in found)
             rows = sum(int(m.weight.shape[0]) for _, _, _, m in found)
-            # K a multiple of 512: no variant's divisibility guard can send the joint product
-            # to the stock operator, whose rounding differs between one matrix and several
+            # K a multiple of 256: the divisibility guard of the variant that is chosen by itself cannot send the joint
+            # product to the stock operator, whose rounding differs between one matrix and several.  (With multiples of
+            # 512 only: one token through the dense layer of a model 2304 wide 50 us of device time, joined 35; a verify
+            # block 51 and 38; one token through a GatedDeltaNet layer 3328 wide, with its padded gates, 61 and 30.)
             k = int(ref.weight.shape[1]) * (32 // ref.bits)
-            if not same or k % 512 != 0 or rows % 32 != 0 or \
+            if not same or k % 256 != 0 or rows % 32 != 0 or \
                     rows >= _env_int("DFLASH_VERIFY_MAX_N", _VERIFY_MAX_N_DEFAULT):
                 continue
             members = []

@@ -227,3 +227,36 @@ def test_joined_outputs_of_prompts_and_short_blocks_are_tensors_of_their_own(nat
     object.__setattr__(attn, "_dflash_fused", parent._dflash_fused)
     attn.q_norm, attn.k_norm = Norm(attn.q_norm.weight), Norm(attn.k_norm.weight)
     assert attn(x).shape == (1, rows, 128)
+
+
+@pytest.mark.parametrize("K,group", [(256, 64), (768, 32), (1280, 128), (2304, 64)])
+def test_projections_join_where_k_is_a_multiple_of_256(verify_env, K, group):
+    """The joint product against the members' own: two orders of the same fp32 sums (each within the bound of
+    ``_check``), each rounded once to the array type.  The activation on top of that: its slope is below 1.1, its four operators
+    round once each.  A variant asked for by name: the members themselves, bit for bit."""
+    from dflash_mlx_amd.quantized import QuantizedLinear
+    from dflash_mlx_amd.verify_linear import fuse_shared_input_linears, install_verify_linears, shared_input_outputs, silu_gate_up
+
+    mlp, names = torch.nn.Module(), ("gate_proj", "up_proj")
+    for i, name in enumerate(names):
+        c = make_qmm_case(K, 288, 300 + i, group_size=group).to(DEV)
+        setattr(mlp, name, QuantizedLinear(c.w, c.scales * 0.1, c.biases * 0.1, group_size=group, bits=4))
+    model = torch.nn.Module()
+    model.mlp = mlp
+    assert install_verify_linears(model) == 2 and fuse_shared_input_linears(model) == 1
+    for rows in (1, 5, 16, 40):
+        x = (torch.randn((rows, K), generator=torch.Generator().manual_seed(rows)) * 0.5).to(torch.bfloat16).to(DEV)
+        own = [getattr(model.mlp, n)(x) for n in names]
+        dense = [dequantize(m.weight, m.scales, m.biases, group, 4, torch.float32) for m in (model.mlp.gate_proj, model.mlp.up_proj)]
+        apart = [2.0 ** -7 * y.float().abs() + x.float().abs() @ w.abs().T * 16.0 * 2.0 ** -24 * 8 for y, w in zip(own, dense)]
+        for got, want, slack in zip(shared_input_outputs(model.mlp, names, x), own, apart):
+            assert ((got.float() - want.float()).abs() <= slack).all()
+        gate, up = (y.float() for y in own)
+        act = gate * torch.sigmoid(gate)
+        slack = 1.1 * up.abs() * apart[0] + (act.abs() + apart[0]) * apart[1] + 5 * 2.0 ** -8 * (act * up).abs()
+        assert ((silu_gate_up(model.mlp, x).float() - act * up).abs() <= slack).all()
+    verify_env.setenv("DFLASH_VERIFY_VARIANT", "mma2big_pipe")
+    x = torch.randn((16, K), generator=torch.Generator().manual_seed(9)).to(torch.bfloat16).to(DEV)
+    joined = model._modules["mlp"]._dflash_fused[0].applies(model.mlp, x)
+    assert joined == (K % 512 == 0)
+    assert all(torch.equal(a, getattr(model.mlp, n)(x)) for n, a in zip(names, shared_input_outputs(model.mlp, names, x)))
