@@ -11,17 +11,19 @@
 //
 //  * gdn_chunk_kernel, one wave per (slot, chunk, head), computes what does not depend on the state: M' and
 //    Lq, in the register order the other kernel multiplies them in, and K^T likewise.  All chunks at once.
-//  * gdn_prompt_kernel, one wave per (slot, head, 16 rows of the state), walks the chunks.  Rows of S are
-//    independent, so 32 heads of 128 x 128 fill 256 compute units with one wave each, and what bounds
-//    the kernel is that wave's chain of dependent steps.  Nothing in it crosses lanes or goes through
-//    LDS: the accumulators of U^T, Delta^T and S^T (a lane holds four consecutive rows of one column)
-//    are read as the B operand of the next product with k in the order the lane happens to have it,
-//    and the A operands (M', Lq, K^T) were laid out in that order.
+//  * gdn_prompt_kernel, one workgroup per (slot, head, 16 rows of the state), walks the chunks.  Rows of S are
+//    independent, so 32 heads of 128 x 128 fill 256 compute units with one workgroup each, and what bounds
+//    the kernel is its chain of dependent steps.  Nothing in it crosses lanes: the accumulators of U^T, Delta^T and S^T (a
+//    lane holds four consecutive rows of one column) are read as the B operand of the next product with k in the order the
+//    lane happens to have it, and the A operands (M', Lq, K^T) were laid out in that order.
+//  * Where that leaves the chip with one wave per compute unit, a row's elements are divided among as many waves as it has
+//    32ths: each cuts its part of S into pieces, multiplies and updates it, and the parts of U and Q S0^T meet in LDS,
+//    one barrier per chunk.  Delta is computed by all of them, from the same sums in the same order, Y by one each.
 //  * fp32 factors (S, V - c U, Delta, M', Lq) are cut into three bf16 pieces (24 bits, exact); products with bf16
 //    K and Q take three matrix-core passes, products of two fp32 factors the six of relative size 2^-16 and up.
 //    The result carries fp32 accuracy, as the step-by-step kernel's does.
 //  * The operands of the next chunk are loaded into the registers of the present one as soon as these have
-//    been used for the last time; 1 wave per SIMD has registers for all of them.
+//    been used for the last time; 1 or 2 waves per SIMD have registers for all of them.
 //  * The closed form is for finite numbers: in a product over all tokens of a chunk, a NaN or an infinity meets the
 //    zeros of M' and Lq and spoils tokens and rows of the state that it must not reach, and products of k with k
 //    may overflow where the recurrence does not.  Both kernels look at what they computed (a sum of 0 x stays zero
@@ -29,10 +31,12 @@
 //    token holds never enters a product: its rows of K and Q are zeros, its element of V - c U as well.
 // A 16-bit state is carried in fp32 and rounded once, at the end.
 //
-// Measured, 1024 tokens, 16 / 32 heads of 128 x 128: 15 + 64 us, against 123.7 ms with one workgroup per head
-// that kept S in memory (the step-by-step kernel held 41 tokens at most).  What the second kernel
-// is bound by is its chain, 4560 cycles (2 us) per chunk by its counters: 605 vector instructions (53 %), 96 matrix
-// instructions (34 %; 72 of them with S), waits 16 %.  Chunks of
+// Measured, 1024 tokens, 16 / 32 heads of 128 x 128: 15 + 51 us (64 with one wave per 16 rows), against 123.7 ms with one
+// workgroup per head that kept S in memory (the step-by-step kernel held 41 tokens at most); 678 tokens of 16 heads both kernels
+// 46 us (55).  What the second kernel is bound by is its chain.  One wave: 4560 cycles (2 us) per chunk by its counters, 605
+// vector instructions (53 %), 96 matrix instructions (34 %; 72 of them with S), waits 16 %.  Four: 3500 cycles, 315 vector and
+// 36 matrix instructions a wave; with no loads in the loop at all it takes 2900, the rest is the hand-over and results that the next
+// instruction waits for.  Chunks of
 // 32 and not 16: cutting S into pieces (176 vector instructions) is paid per chunk, and a matrix instruction
 // of depth 32 in the update is filled; 64 would need more registers than a wave has.  The look for numbers that are not
 // finite costs 0.3 % of a layer call, a chunk token by token what 32 steps of one wave cost.
@@ -46,6 +50,10 @@ constexpr int kMatBytes = 2 * 3 * 1024;                // [tile of 16 rows][piec
 constexpr int kHeadBytes = 2 * kMatBytes + 3 * kChunk * 4;  // M', Lq, then per token c (0 if masked) and c_T / c_s, then kTail:
 constexpr int kTail = 2 * kChunk;                      // four words: c_T, 0 or (numbers that are not finite) NaN, one bit per token that counts, -
 constexpr int kPitch = 36;                             // floats per row of the 32 x 32 matrices in LDS
+// Up to as many (head, 16 rows) as there are compute units, the 32ths of a row on a wave each.  With more of them the units
+// are shared, and what the waves of a row do twice (Delta, the pieces of it) costs more than their chain is shorter: us per
+// 1024 tokens with the chunk kernel, one wave and four, 32 heads of 128 x 128 78 and 66, 48 heads 88 and 90, 64 heads 89 and 94.
+constexpr int kSpread = 256;
 
 struct Args {
   const uint16_t* q;
@@ -250,10 +258,18 @@ __global__ __launch_bounds__(64, 3) void gdn_chunk_kernel(Args a) {
   }
 }
 
-// MASKED: some tokens may not count (those past T read zeros and need no looking after).
-template <int DK, bool MASKED>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void gdn_prompt_kernel(Args a) {
-  constexpr int NC = DK / 32, NT = DK / 16;
+// MASKED: some tokens may not count (those past T read zeros and need no looking after).  WAVES: of a workgroup, which
+// divide the DK elements of a row among themselves, 1 or DK / 32.
+template <int DK, bool MASKED, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(1, WAVES == 1 ? 1 : 2)))
+void gdn_prompt_kernel(Args a) {
+  constexpr int NC = DK / 32 / WAVES, NT = 2 * NC;  // pieces of 32 and of 16 dk that a wave has
+  constexpr int kTiles = WAVES == 1 ? 2 : 1;         // of the tokens whose Y it computes
+  constexpr bool kEarly = WAVES > 1;                 // c and c_T / c_s of the next chunk are asked for at their last use, not last
+  constexpr int kStored = WAVES == 4 ? 2 : 4;        // tokens of a lane's four there whose results it writes
+  // the waves' parts of U (two tiles) and W, those of a chunk while the ones before may still be read
+  __shared__ f32x4_t parts[2][WAVES][4][WAVES == 1 ? 1 : 64];
+  __shared__ float sums[WAVES][16];  // (token by token: their parts of one row each)
   const int slices = a.Dv / 16;
   // the slices of a head read the same K, Q, M' and Lq: all of them behind one L2 (blocks go to the XCDs in turn)
   const int heads = a.slots * a.Hv;
@@ -267,13 +283,17 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
     slice = blockIdx.x % slices;
   }
   const int slot = item / a.Hv, hv = item % a.Hv, hk = hv / (a.Hv / a.Hk);
-  const int lane = threadIdx.x, li = lane & 15, kq = lane >> 4;
+  const int lane = threadIdx.x & 63, li = lane & 15, kq = lane >> 4;
+  const int wave = WAVES == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tile0 = WAVES == 4 ? wave >> 1 : wave;          // the first (or only) tile of tokens whose Y it computes
+  const int first = WAVES == 4 ? 2 * (wave & 1) : 0;        // of a lane's four tokens there
   const size_t slotT = (size_t)slot * a.T;
   const int dv = 16 * slice + li;
 
-  // S^T tile c: rows dk_of(c, 4 kq + r), column dv = this lane's; two tiles are 8 consecutive dk of a row of S
+  // S^T tile c of this wave: rows dk_of(NT wave + c, 4 kq + r), column dv = this lane's; two tiles are 8 consecutive dk of a
+  // row of S
   f32x4_t st[NT];
-  const size_t srow = ((size_t)item * a.Dv + dv) * DK + 8 * kq;
+  const size_t srow = ((size_t)item * a.Dv + dv) * DK + 32 * NC * wave + 8 * kq;
 #pragma unroll
   for (int C = 0; C < NC; ++C)
 #pragma unroll
@@ -296,10 +316,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
   const auto v_buf = buffer_of(a.v + slotT * a.Hv * a.Dv, v_bytes), y_buf = buffer_of(a.y + slotT * a.Hv * a.Dv, v_bytes);
   const auto tape_buf = buffer_of(a.tape + slotT * a.Hv * a.Dv, a.tape != nullptr ? 2 * v_bytes : 0u);
   const uint32_t k_step = (uint32_t)a.Hk * DK * 2, v_step = (uint32_t)a.Hv * a.Dv * 2;  // bytes per token
-  const uint32_t k_at = li * k_step + hk * (DK * 2) + 16 * kq;
+  const uint32_t k_at = li * k_step + hk * (DK * 2) + 64 * NC * wave + 16 * kq;
   const uint32_t v_at = 4 * kq * v_step + (hv * a.Dv + dv) * 2;
 
-  uint4 kf[2][NC], qf[2][NC], kt[NT], mf[2][3], lf[2][3];
+  uint4 kf[2][NC], qf[2][NC], kt[NT], mf[2][3], lf[kTiles][3];
   uint32_t vb[8];
   f32x4_t cv[2], cfv[2];
   f32x4_t tail_next;  // (asked for with K and Q: the scheduler moves the scaling of S to the front)
@@ -323,28 +343,34 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
     for (int j = 0; j < 8; ++j)
       vb[j] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(v_buf, v_at + (ch * kChunk + 16 * (j >> 2) + (j & 3)) * v_step, 0, 0);
   };
-  auto load_mat = [&](int ch, int which, uint4 (&f)[2][3]) __attribute__((always_inline)) {
-    const uint4* src = reinterpret_cast<const uint4*>(head0 + ch * per_chunk + which * kMatBytes) + lane;
+  auto load_m = [&](int ch) __attribute__((always_inline)) {
+    const uint4* src = reinterpret_cast<const uint4*>(head0 + ch * per_chunk) + lane;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int p = 0; p < 3; ++p) f[i][p] = src[(3 * i + p) * 64];
+      for (int p = 0; p < 3; ++p) mf[i][p] = src[(3 * i + p) * 64];
+  };
+  auto load_l = [&](int ch) __attribute__((always_inline)) {
+    const uint4* src = reinterpret_cast<const uint4*>(head0 + ch * per_chunk + kMatBytes) + 3 * tile0 * 64 + lane;
+#pragma unroll
+    for (int i = 0; i < kTiles; ++i)
+#pragma unroll
+      for (int p = 0; p < 3; ++p) lf[i][p] = src[(3 * i + p) * 64];
   };
   auto load_kt = [&](int ch) __attribute__((always_inline)) {
-    const uint4* src = reinterpret_cast<const uint4*>(kt0 + ch * per_chunk) + lane;
+    const uint4* src = reinterpret_cast<const uint4*>(kt0 + ch * per_chunk) + NT * wave * 64 + lane;
 #pragma unroll
     for (int c = 0; c < NT; ++c) kt[c] = src[c * 64];
   };
-  auto load_vec = [&](int ch) __attribute__((always_inline)) {
-    const float* vec = reinterpret_cast<const float*>(head0 + ch * per_chunk + 2 * kMatBytes);
+  auto load_vec = [&](int ch, int which, f32x4_t (&f)[2]) __attribute__((always_inline)) {
+    const float* vec = reinterpret_cast<const float*>(head0 + ch * per_chunk + 2 * kMatBytes) + which * kChunk;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      cv[i] = *reinterpret_cast<const f32x4_t*>(vec + 16 * i + 4 * kq);
-      cfv[i] = *reinterpret_cast<const f32x4_t*>(vec + kChunk + 16 * i + 4 * kq);
-    }
+    for (int i = 0; i < 2; ++i) f[i] = *reinterpret_cast<const f32x4_t*>(vec + 16 * i + 4 * kq);
   };
   // arithmetic may move across, requests to memory stay where they were written
 #define DFLASH_KEEP_REQUESTS() __builtin_amdgcn_sched_barrier(0xF)
+  // a barrier for what the waves hand over through LDS; requests to memory stay in flight
+  auto meet = [&]() __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
   // sum of the six piece products of two fp32 factors that matter; two accumulators, smaller terms first
   auto product6 = [&](const uint4 (&f)[3], const Pieces<8>& p, f32x4_t big) __attribute__((always_inline)) {
     f32x4_t small = {0.f, 0.f, 0.f, 0.f};
@@ -355,6 +381,19 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
     small = mfma(f[1], p.mid, small);
     big = mfma(f[0], p.hi, big);
     return big + small;
+  };
+  // sum over all waves of what each has for the lane's row of S, in the order of the waves
+  auto over_waves = [&](float x) __attribute__((always_inline)) -> float {
+    x += __shfl_xor(x, 16, 64);
+    x += __shfl_xor(x, 32, 64);
+    if (WAVES == 1) return x;
+    if (kq == 0) sums[wave][li] = x;
+    meet();
+    float sum = sums[0][li];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) sum += sums[w][li];
+    meet();
+    return sum;
   };
 
   // The recurrence itself, for a chunk with numbers that are not finite.
@@ -368,7 +407,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
         const float g = load_as_f32(a.g, (slotT + t) * a.Hv + hv, a.g_dtype);
         const float beta = load_as_f32(a.beta, (slotT + t) * a.Hv + hv, a.beta_dtype);
         const float v = bf16_bits_to_f32((uint16_t)__builtin_amdgcn_raw_buffer_load_b16(v_buf, at, 0, 0));
-        const size_t row = ((slotT + t) * a.Hk + hk) * DK + 8 * kq;
+        const size_t row = ((slotT + t) * a.Hk + hk) * DK + 32 * NC * wave + 8 * kq;
         auto element = [](uint4 w, int e) __attribute__((always_inline)) {  // 0 .. 7
           const uint32_t half[4] = {w.x, w.y, w.z, w.w};
           return __uint_as_float(e & 1 ? half[e >> 1] & 0xffff0000u : half[e >> 1] << 16);
@@ -379,7 +418,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
           kw[C] = *reinterpret_cast<const uint4*>(a.k + row + 32 * C);
           qw[C] = *reinterpret_cast<const uint4*>(a.q + row + 32 * C);
         }
-        float known = 0.f;  // S k, summed over the four lanes that hold a row of S
+        float known = 0.f;  // S k, summed over the four lanes of every wave that hold a row of S
 #pragma unroll
         for (int C = 0; C < NC; ++C)
 #pragma unroll
@@ -388,9 +427,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
             entry[e & 3] *= g;
             known = fmaf(entry[e & 3], element(kw[C], e), known);
           }
-        known += __shfl_xor(known, 16, 64);
-        known += __shfl_xor(known, 32, 64);
-        delta = (v - known) * beta;
+        delta = (v - over_waves(known)) * beta;
 #pragma unroll
         for (int C = 0; C < NC; ++C)
 #pragma unroll
@@ -399,35 +436,35 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
             entry[e & 3] = fmaf(element(kw[C], e), delta, entry[e & 3]);
             y = fmaf(entry[e & 3], element(qw[C], e), y);
           }
-        y += __shfl_xor(y, 16, 64);
-        y += __shfl_xor(y, 32, 64);
+        y = over_waves(y);
       }
-      if (kq == 0) {
+      if (kq == 0 && wave == 0) {
         __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(uint16_t, (__bf16)y), y_buf, at, 0, 0);
         __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(delta), tape_buf, 2 * at, 0, 0);
       }
     }
   };
 
-  // (the way to the token-by-token form leaves the loop: the loop itself stays without a branch around its stores)
+  // (the way to the token-by-token form leaves the loop: the loop itself stays without a branch around its stores.  Every
+  // wave leaves it at the same chunk: what they look at, Delta, is the same numbers in all of them.)
   int ch = 0;
   while (ch < a.chunks) {
     load_kq(ch);
     DFLASH_KEEP_REQUESTS();  // in the order of the loop: what its first wait may leave in flight is the least of both
     load_v(ch);
-    load_mat(ch, 0, mf);
+    if (kEarly) load_vec(ch, 0, cv);
+    load_m(ch);
+    if (kEarly) load_vec(ch, 1, cfv);
     load_kt(ch);
-    load_mat(ch, 1, lf);
-    load_vec(ch);
+    load_l(ch);
+    if (!kEarly) load_vec(ch, 0, cv), load_vec(ch, 1, cfv);
     DFLASH_KEEP_REQUESTS();
 #pragma unroll 1
     for (; ch < a.chunks; ++ch) {
       const int next = ch + 1 < a.chunks ? ch + 1 : ch;
       const float c_last = tail_next[0];
       float finite = tail_next[1];  // stays zero
-      int keep[8];  // all bits of the tokens of this lane that count
-#pragma unroll
-      for (int j = 0; j < 8; ++j) keep[j] = MASKED ? -(int)((__float_as_uint(tail_next[2]) >> token_of(kq, j)) & 1u) : -1;
+      const uint32_t on_bits = __float_as_uint(tail_next[2]);
       // ---- U = K S^T, W = Q S^T: rows = tokens, column = dv ---------------------------------------
       f32x4_t U[2], W[2];
 #pragma unroll
@@ -444,22 +481,38 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
 #pragma unroll
         for (int i = 0; i < 2; ++i) U[i] = mfma(kf[i][C], sp.hi, U[i]), W[i] = mfma(qf[i][C], sp.hi, W[i]);
       }
+      if constexpr (WAVES > 1) {  // the sums over the waves, in their order: the same numbers in every wave
+#pragma unroll
+        for (int i = 0; i < 2; ++i) parts[ch & 1][wave][i][lane] = U[i], parts[ch & 1][wave][2 + i][lane] = W[i];
+      }
       load_kq(next);
       DFLASH_KEEP_REQUESTS();
+      if constexpr (WAVES > 1) {
+        meet();
+        auto total = [&](int part) __attribute__((always_inline)) -> f32x4_t {
+          f32x4_t sum = parts[ch & 1][0][part][lane];
+#pragma unroll
+          for (int w = 1; w < WAVES; ++w) sum += parts[ch & 1][w][part][lane];
+          return sum;
+        };
+        U[0] = total(0), U[1] = total(1), W[0] = total(2 + tile0);
+      }
       // ---- Delta = M' (V - c U) ----------------------------------------------------------------------
       float rhs[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         rhs[j] = bf16_bits_to_f32(vb[j]) - cv[j >> 2][j & 3] * U[j >> 2][j & 3];
-        if (MASKED) rhs[j] = __int_as_float(__float_as_int(rhs[j]) & keep[j]);
+        if (MASKED) rhs[j] = __int_as_float(__float_as_int(rhs[j]) & -(int)((on_bits >> token_of(kq, j)) & 1u));
       }
+      if (kEarly) W[0] *= tile0 ? cv[1] : cv[0];
       load_v(next);
+      if (kEarly) load_vec(next, 0, cv);
       DFLASH_KEEP_REQUESTS();
       const Pieces<8> rp = split_bf16(rhs);
       f32x4_t D[2];
 #pragma unroll
       for (int i = 0; i < 2; ++i) D[i] = product6(mf[i], rp, f32x4_t{0.f, 0.f, 0.f, 0.f});
-      load_mat(next, 0, mf);
+      load_m(next);
       DFLASH_KEEP_REQUESTS();
       // a number that is not finite in V, U (and so in S) or M' is one in every Delta of its column
 #pragma unroll
@@ -471,6 +524,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
       for (int j = 0; j < 8; ++j) {
         plain[j] = D[j >> 2][j & 3];
         scaled[j] = plain[j] * cfv[j >> 2][j & 3];
+      }
+      if (kEarly) {
+        load_vec(next, 1, cfv);
+        DFLASH_KEEP_REQUESTS();
       }
       {
         const Pieces<8> dp = split_bf16(scaled);
@@ -485,22 +542,24 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
       }
       load_kt(next);
       DFLASH_KEEP_REQUESTS();
-      // ---- Y = c W + Lq Delta ------------------------------------------------------------------------
+      // ---- Y = c W + Lq Delta, for the tokens of this wave's tiles -------------------------------------
       const Pieces<8> dq = split_bf16(plain);
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const f32x4_t Y = product6(lf[i], dq, W[i] * cv[i]);
+      for (int i = 0; i < kTiles; ++i) {
+        const f32x4_t Y = product6(lf[i], dq, kEarly ? W[i] : W[i] * cv[i]), mine = i == 1 || (WAVES > 1 && tile0) ? D[1] : D[0];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const uint32_t at = v_at + (ch * kChunk + 16 * i + r) * v_step;
-          uint16_t y = __builtin_bit_cast(uint16_t, (__bf16)Y[r]);
-          if (MASKED) y &= (uint16_t)keep[4 * i + r];
+        for (int r = 0; r < kStored; ++r) {
+          const float y_r = kStored == 2 && first ? Y[(r + 2) & 3] : Y[r], d_r = kStored == 2 && first ? mine[(r + 2) & 3] : mine[r];
+          const int t = 16 * (tile0 + i) + first + r;  // and 4 kq, which v_at holds
+          const uint32_t at = v_at + (ch * kChunk + t) * v_step;
+          uint16_t y = __builtin_bit_cast(uint16_t, (__bf16)y_r);
+          if (MASKED) y &= (uint16_t)-(int)((on_bits >> (t + 4 * kq)) & 1u);
           __builtin_amdgcn_raw_buffer_store_b16(y, y_buf, at, 0, 0);
-          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(D[i][r]), tape_buf, 2 * at, 0, 0);
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(d_r), tape_buf, 2 * at, 0, 0);
         }
       }
-      load_mat(next, 1, lf);
-      load_vec(next);
+      load_l(next);
+      if (!kEarly) load_vec(next, 0, cv), load_vec(next, 1, cfv);
       DFLASH_KEEP_REQUESTS();
     }
     if (ch < a.chunks) token_by_token(ch++);
@@ -511,13 +570,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
   for (int C = 0; C < NC; ++C)
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
+      const f32x4_t entry = st[2 * C + h];
       if (a.state_dtype == DFLASH_FP32) {
-        *reinterpret_cast<f32x4_t*>((float*)a.state_out + srow + 32 * C + 4 * h) = st[2 * C + h];
+        *reinterpret_cast<f32x4_t*>((float*)a.state_out + srow + 32 * C + 4 * h) = entry;
       } else {
         uint32_t b[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          b[e] = a.state_dtype == DFLASH_BF16 ? f32_to_bf16_bits(st[2 * C + h][e]) : f32_to_f16_bits(st[2 * C + h][e]);
+        for (int e = 0; e < 4; ++e) b[e] = a.state_dtype == DFLASH_BF16 ? f32_to_bf16_bits(entry[e]) : f32_to_f16_bits(entry[e]);
         *reinterpret_cast<uint2*>((uint16_t*)a.state_out + srow + 32 * C + 4 * h) = uint2{b[0] | (b[1] << 16), b[2] | (b[3] << 16)};
       }
     }
@@ -526,9 +585,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
 template <int DK>
 int launch(const Args& a, hipStream_t s) {
   hipLaunchKernelGGL((gdn_chunk_kernel<DK>), dim3((unsigned)(a.slots * a.chunks * a.Hv)), dim3(64), 0, s, a);
-  const dim3 grid((unsigned)(a.slots * a.Hv * (a.Dv / 16)));
-  if (a.mask != nullptr) hipLaunchKernelGGL((gdn_prompt_kernel<DK, true>), grid, dim3(64), 0, s, a);
-  else hipLaunchKernelGGL((gdn_prompt_kernel<DK, false>), grid, dim3(64), 0, s, a);
+  const int groups = a.slots * a.Hv * (a.Dv / 16);
+  const bool spread = groups <= kSpread;
+  const void* fn = a.mask != nullptr ? (spread ? (const void*)gdn_prompt_kernel<DK, true, DK / 32> : (const void*)gdn_prompt_kernel<DK, true, 1>)
+                                     : (spread ? (const void*)gdn_prompt_kernel<DK, false, DK / 32> : (const void*)gdn_prompt_kernel<DK, false, 1>);
+  Args args = a;
+  void* argv[] = {&args};
+  DFLASH_HIP_OK(hipLaunchKernel(fn, dim3((unsigned)groups), dim3(spread ? 2 * DK : 64), argv, 0, s));
   DFLASH_HIP_OK(hipGetLastError());
   return DFLASH_OK;
 }

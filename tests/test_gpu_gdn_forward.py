@@ -434,3 +434,28 @@ def test_rows_of_the_state_in_registers(native_lib, state_dtype, B, T, Hk, Hv, D
         assert _rel(_f64(s), _f64(S)) <= tol
         assert _rel(_f64(tape), _f64(torch.cat(tapes, dim=1))) <= tol
         assert _rel(_f64(y), _f64(torch.cat(ys, dim=1))) <= tol_y
+
+
+@pytest.mark.parametrize("shape", [dict(T=70, B=2), dict(T=33, B=4, Dk=64, Dv=48), dict(T=40, B=2, Hk=1, Hv=1, Dv=16)])
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("value", [0.5, float("nan"), float("inf")])
+def test_prompts_of_few_heads_and_of_many(native_lib, shape, masked, value):
+    """Up to 256 (head, 16 rows) a row of the state is spread over the waves of a workgroup, above that one wave holds it.  Batches of
+    one kind, repeated into the other: sums in another order, each within the bar against fp64 (twice it between them),
+    and one rounding of y each."""
+    args = _case(seed=80 + shape["T"], **shape)
+    args[2][0, 11, 0, 5] = value
+    B, T, Hv, Dv = args[2].shape
+    few, mask = B * Hv * (Dv // 16), None
+    times = 256 // few + 1
+    assert few <= 256 < few * times
+    if masked:
+        mask = torch.rand((B, T), generator=torch.Generator().manual_seed(T)) > 0.3
+        mask[0, 11] = True
+    y, s, tape = _run(args, mask)
+    many = _run([torch.cat([t] * times) for t in args], None if mask is None else torch.cat([mask] * times))
+    for i in range(times):
+        y2, s2, tape2 = (t[i * B:(i + 1) * B] for t in many)
+        _same_values(s2, s, 4e-5)
+        _same_values(tape2, tape, 4e-5)
+        _same_values(y2, y, 2.0 ** -7)
