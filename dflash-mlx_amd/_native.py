@@ -18,7 +18,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libdflash_mi355.so")
 HOST_PATH = os.path.join(_HERE, "_dflash_host.so")
 
-ABI_VERSION = 21
+ABI_VERSION = 22
 
 BF16, FP16, FP32 = 0, 1, 2
 QMM_MMA2BIG, QMM_MMA2BIG_PIPE = 0, 1
@@ -69,6 +69,7 @@ EXPORTED_SYMBOLS = (
     "dflash_gdn_forward",
     "dflash_gdn_prepare",
     "dflash_gdn_prepare_rows",
+    "dflash_gdn_block",
     "dflash_gdn_gated_norm",
     "dflash_attn_prepare",
     "dflash_attn_gate",
@@ -148,6 +149,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.dflash_gdn_prepare_rows.restype = c.c_int
     lib.dflash_gdn_prepare_rows.argtypes = ([c.c_void_p] * 15 + [c.POINTER(c.c_longlong)] + [c.c_int] * 9 +
                                             [c.c_float, c.c_void_p])
+    lib.dflash_gdn_block.restype = c.c_int
+    lib.dflash_gdn_block.argtypes = [c.c_void_p] * 2
     lib.dflash_gdn_gated_norm.restype = c.c_int
     lib.dflash_gdn_gated_norm.argtypes = [c.c_void_p] * 4 + [c.c_longlong] + [c.c_int] * 3 + [c.c_float, c.c_void_p]
     lib.dflash_attn_prepare.restype = c.c_int

@@ -1,0 +1,161 @@
+// A GatedDeltaNet block as its projections leave it: the conv, the activation, the norms and the gates of
+// gdn_glue.hip's prepare kernel, for kernels that go on with the recurrence themselves (bf16 arrays, four taps).  Operator for
+// operator and sum for sum as there, so that both ways give the same bits.
+#pragma once
+
+#include "glue_device.h"
+
+namespace dflash {
+namespace {
+
+// Sum of the squares of a head: PER elements in each of LANES lanes (a power of two).  Adjacent elements first and in
+// sixty-fourths of the head whatever LANES is, so that a row has the same sum in every kernel.
+template <int PER, int LANES>
+__device__ __forceinline__ float sum_of_squares(const float (&v)[PER]) {
+  constexpr int kEach = PER * LANES / 64, kParts = PER / kEach;
+  float part[kParts];
+#pragma unroll
+  for (int i = 0; i < kParts; ++i) {
+    part[i] = 0.f;
+#pragma unroll
+    for (int e = 0; e < kEach; ++e) part[i] += v[i * kEach + e] * v[i * kEach + e];
+  }
+#pragma unroll
+  for (int n = kParts / 2; n >= 1; n /= 2)
+#pragma unroll
+    for (int i = 0; i < n; ++i) part[i] = part[2 * i] + part[2 * i + 1];
+  float sum = part[0];
+#pragma unroll
+  for (int off = 1; off < LANES; off <<= 1) sum += __shfl_xor(sum, off, 64);
+  return sum;
+}
+
+// Gate of a value head: a + dt_bias and the softplus live in the promoted dtype of the two operands.
+__device__ __forceinline__ float decay_of(float a, float a_log, float bias, int sum_dt) {
+  const float apb = round_through(a + bias, sum_dt);
+  const float sp = round_through(fmaxf(apb, 0.f) + log1pf(expf(-fabsf(apb))), sum_dt);
+  return expf(-expf(a_log) * sp);
+}
+
+constexpr int kTaps = 4, kKeep = kTaps - 1;
+
+struct BlockArgs {
+  const uint16_t* qkv;         // [slots, T, C], rows and slots with a stride (elements)
+  const uint16_t* conv_state;  // [slots, 3, C] or null (zeros)
+  const uint16_t* conv_w;      // [C, 4]
+  const uint16_t *a, *b;       // [slots, T, Hv], likewise with strides
+  const void *A_log, *dt_bias;  // [Hv]
+  uint16_t *conv_next, *k_out, *qkv_out;  // [slots, 3, C]; [slots, T, Hk, D] and [slots, T, C] or null
+  float* g_out;                           // [slots, T, Hv] or null
+  long long qkv_slot, qkv_row, a_slot, a_row, b_slot, b_row;
+  int param_dt;
+  float eps, scale_q, scale_k;  // scales already rounded to bf16
+};
+
+// The words of a bf16 load, stored as they are.
+template <int PER>
+__device__ __forceinline__ void store_words(uint16_t* dst, const uint32_t (&raw)[PER]) {
+  if constexpr (PER % 4 == 0) {
+#pragma unroll
+    for (int e = 0; e < PER; e += 4) *reinterpret_cast<uint2*>(dst + e) = uint2{raw[e / 2], raw[e / 2 + 1]};
+  } else if constexpr (PER == 2) {
+    *reinterpret_cast<uint32_t*>(dst) = raw[0];
+  } else {
+    *dst = (uint16_t)raw[0];
+  }
+}
+
+// bf16 numbers held as floats, stored.
+template <int PER>
+__device__ __forceinline__ void store_exact(uint16_t* dst, const float (&v)[PER]) {
+  uint32_t words[PER] = {};
+#pragma unroll
+  for (int e = 0; e + 1 < PER; e += 2) words[e / 2] = __builtin_amdgcn_perm(__float_as_uint(v[e + 1]), __float_as_uint(v[e]), 0x07060302u);
+  if constexpr (PER == 1) words[0] = __float_as_uint(v[0]) >> 16;
+  store_words<PER>(dst, words);
+}
+
+// PER adjacent channels (from c on) at one step t: rows t .. t + 3 of [conv_state | qkv] and the taps, as loaded.
+template <int PER>
+struct ConvRows {
+  uint32_t x[kTaps][PER], w[PER * kTaps];
+};
+// Every load is unconditional: a row that does not count (no conv state, steps past the block) is some readable row.
+template <int PER>
+__device__ __forceinline__ void request_rows(const BlockArgs& p, int slot, int t, int T, int C, int c, ConvRows<PER>& r) {
+  const uint16_t* const qkv = p.qkv + (size_t)slot * p.qkv_slot;
+  const uint16_t* const before = p.conv_state + (size_t)slot * kKeep * C;
+  const uint32_t pitch = (uint32_t)p.qkv_row;  // (16 rows of it are within 32 bits: checked where the launch is)
+#pragma unroll
+  for (int j = 0; j < kTaps; ++j) {
+    const int row = t + j, s = row - kKeep < T ? row - kKeep : T - 1;
+    if (j == kKeep) {
+      load_adjacent_raw<PER>(qkv, (uint32_t)s * pitch + (uint32_t)c, false, r.x[j]);
+    } else {
+      const bool stored = row < kKeep && p.conv_state != nullptr;
+      load_adjacent_raw<PER>(stored ? before : qkv, (stored ? (uint32_t)row * (uint32_t)C : (uint32_t)(s < 0 ? 0 : s) * pitch) + (uint32_t)c, false,
+                             r.x[j]);
+    }
+  }
+  load_adjacent_raw<PER * kTaps>(p.conv_w, (size_t)c * kTaps, false, r.w);
+}
+
+// silu(conv), and what the rows leave behind where `keeps`: the next conv state and qkv in one piece.
+template <int PER>
+__device__ __forceinline__ void convolve(const BlockArgs& p, int slot, int t, int T, int C, int c, bool keeps, ConvRows<PER>& r,
+                                         float (&act)[PER]) {
+  if (p.conv_state == nullptr) {
+#pragma unroll
+    for (int j = 0; j < kKeep; ++j)
+#pragma unroll
+      for (int e = 0; e < PER; ++e) r.x[j][e] = t + j >= kKeep ? r.x[j][e] : 0u;
+  }
+  float x[kTaps][PER], w[PER * kTaps];
+#pragma unroll
+  for (int j = 0; j < kTaps; ++j) unpack_adjacent<PER>(r.x[j], DFLASH_BF16, x[j]);
+  unpack_adjacent<PER * kTaps>(r.w, DFLASH_BF16, w);
+#pragma unroll
+  for (int e = 0; e < PER; ++e) {
+    float acc = 0.f;
+#pragma unroll
+    for (int j = 0; j < kTaps; ++j) acc += x[j][e] * w[e * kTaps + j];
+    act[e] = silu_rounded(round_through(acc, DFLASH_BF16), DFLASH_BF16);
+  }
+  if (!keeps || t >= T) return;
+  uint16_t* const next = p.conv_next + (size_t)slot * kKeep * C + c;
+  if (t == 0) {  // blocks shorter than the state: old rows move up
+#pragma unroll
+    for (int row = 1; row < kKeep; ++row)
+      if (row >= T) store_words<PER>(next + (size_t)(row - T) * C, r.x[row]);
+  }
+  if (t + kKeep >= T) store_words<PER>(next + (size_t)(t + kKeep - T) * C, r.x[kKeep]);
+  if (p.qkv_out != nullptr) store_words<PER>(p.qkv_out + ((size_t)slot * T + t) * C + c, r.x[kKeep]);
+}
+
+// q or k of the head from its activation: scale * rms_norm, rounded as the array it would be stored in.
+template <int PER, int LANES>
+__device__ __forceinline__ void normalise(float (&v)[PER], float scale, float eps) {
+  const float inv_rms = 1.0f / sqrtf(sum_of_squares<PER, LANES>(v) / (float)(PER * LANES) + eps);
+#pragma unroll
+  for (int e = 0; e < PER; ++e) v[e] = round_through(scale * round_through(v[e] * inv_rms, DFLASH_BF16), DFLASH_BF16);
+}
+
+// The gate and beta of step t of value head hv, as loaded and as the recurrence reads them.
+struct GateBits {
+  uint32_t a, b, a_log, bias;
+};
+__device__ __forceinline__ GateBits request_gates(const BlockArgs& p, int slot, int t, int hv) {
+  const bool wide = p.param_dt == DFLASH_FP32;
+  return {p.a[(size_t)slot * p.a_slot + (size_t)t * p.a_row + hv], p.b[(size_t)slot * p.b_slot + (size_t)t * p.b_row + hv],
+          load_one(p.A_log, hv, wide), load_one(p.dt_bias, hv, wide)};
+}
+__device__ __forceinline__ float gate_of(const BlockArgs& p, const GateBits& r) {
+  return decay_of(bits_as_f32(r.a, DFLASH_BF16), bits_as_f32(r.a_log, p.param_dt), bits_as_f32(r.bias, p.param_dt),
+                  p.param_dt == DFLASH_FP32 ? DFLASH_FP32 : DFLASH_BF16);
+}
+__device__ __forceinline__ float beta_of(const GateBits& r) {
+  return round_through(sigmoid_for(bits_as_f32(r.b, DFLASH_BF16), DFLASH_BF16), DFLASH_BF16);
+}
+
+}  // namespace
+}  // namespace dflash

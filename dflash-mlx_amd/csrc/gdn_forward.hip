@@ -30,6 +30,7 @@
 //    multiplies c back in once at the end (renormalising if c gets very small).
 // q, k, v, g, beta of the block are staged once in LDS as fp32.
 #include "gdn_device.h"
+#include "gdn_block_device.h"
 #include <cstdlib>
 
 namespace dflash {
@@ -58,6 +59,7 @@ struct GdnArgs {
   const void* norm_weight;  // [Dv]
   int weight_dtype;
   float eps;
+  BlockArgs block;  // kernels with BLOCK: the block's projections, in place of q, k, v, g and beta
 };
 
 // v + (v of the lane the DPP control names): butterfly steps inside a row of 16 lanes -
@@ -281,7 +283,7 @@ __global__ __launch_bounds__(kThreads) void gdn_forward_128(GdnArgs a) {
 // 16 steps / 1 step, us: 32 heads of 128 x 128 73.9 / 21.7 -> 7.6 / 3.9, 1024 heads 184 / 53 -> 69 / 19; of 64 x 64, whose
 // state went through memory at every step, 913 / 77.7 -> 6.8 / 3.4 and 1158 / 105 -> 21 / 5.9.
 // ---------------------------------------------------------------------------
-template <int STATE, int DK, int R>
+template <int STATE, int DK, int R, bool BLOCK>
 __global__ __launch_bounds__(kThreads) void gdn_forward_rows(GdnArgs a) {
   constexpr bool kWide = STATE == DFLASH_FP32;
   constexpr int kLanes = DK / 8, kPass = kThreads / kLanes, kRows = kPass * R;  // lanes of a row, rows of a pass, of the workgroup
@@ -305,12 +307,25 @@ __global__ __launch_bounds__(kThreads) void gdn_forward_rows(GdnArgs a) {
     const size_t slotT = (size_t)slot * a.T + first;
     // the block's operands first, the state behind them, nothing looked at before all of it is on its way
     uint32_t rq[kK] = {}, rk[kK] = {}, rv[kD] = {}, g_bits = 0u, beta_bits = 0u;
-    if (t16 < T) {
+    // BLOCK: every wave its four steps of q, k and v, of up to four steps in all one of the three; the gates the last wave
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, C = 2 * a.Hk * DK + a.Hv * a.Dv;
+    const bool few = T <= 4;
+    const int t_b = few ? lane >> 4 : t16, c_q = hk * DK + kK * seg, c_k = c_q + a.Hk * DK, c_v = 2 * a.Hk * DK + hv * a.Dv + row0 + kD * seg;
+    auto mine = [&](int which) __attribute__((always_inline)) { return few ? wave == which : 4 * wave < T; };
+    ConvRows<kK> b_q, b_k;
+    ConvRows<kD> b_v;
+    GateBits gates;
+    if constexpr (BLOCK) {
+      request_rows(a.block, slot, t_b, T, C, c_q, b_q);
+      request_rows(a.block, slot, t_b, T, C, c_k, b_k);
+      request_rows(a.block, slot, t_b, T, C, c_v, b_v);
+      gates = request_gates(a.block, slot, lane < T ? lane : T - 1, hv);
+    } else if (t16 < T) {
       load_bits<kK>(a.q, ((slotT + t16) * a.Hk + hk) * DK + kK * seg, wide, rq);
       load_bits<kK>(a.k, ((slotT + t16) * a.Hk + hk) * DK + kK * seg, wide, rk);
       load_bits<kD>(a.v, ((slotT + t16) * a.Hv + hv) * a.Dv + row0 + kD * seg, wide, rv);
     }
-    if (tid < T) {
+    if (!BLOCK && tid < T) {
       const size_t at = (slotT + tid) * a.Hv + hv;
       if (a.g_dtype == DFLASH_FP32) g_bits = ((const uint32_t*)a.g)[at];
       else g_bits = ((const uint16_t*)a.g)[at];
@@ -330,24 +345,61 @@ __global__ __launch_bounds__(kThreads) void gdn_forward_rows(GdnArgs a) {
         }
       }
     }
+    if constexpr (BLOCK) {
+      asm volatile("" ::: "memory");  // every request above is out before the first value is interpreted
+      // rows of v are one workgroup's, a key head is kept by the first of its value heads and of its first rows
+      const bool keeps = row0 == 0 && hv % (a.Hv / a.Hk) == 0;
+      if (mine(0)) {
+        float x[kK];
+        convolve(a.block, slot, t_b, T, C, c_q, keeps, b_q, x);
+        normalise<kK, 16>(x, a.block.scale_q, a.block.eps);
 #pragma unroll
-    for (int e = 0; e < kK; ++e) asm volatile("" : "+v"(rq[e]), "+v"(rk[e])::"memory");
+        for (int e = 0; e < kK; ++e) sQ[t_b * DK + plane_index<DK>(kK * seg + e)] = x[e];
+      }
+      if (mine(1)) {
+        float x[kK];
+        convolve(a.block, slot, t_b, T, C, c_k, keeps, b_k, x);
+        normalise<kK, 16>(x, a.block.scale_k, a.block.eps);
 #pragma unroll
-    for (int e = 0; e < kD; ++e) asm volatile("" : "+v"(rv[e])::"memory");
-    asm volatile("" : "+v"(g_bits), "+v"(beta_bits)::"memory");
+        for (int e = 0; e < kK; ++e) sK[t_b * DK + plane_index<DK>(kK * seg + e)] = x[e];
+        if (keeps && t_b < T && a.block.k_out != nullptr)
+          store_exact<kK>(a.block.k_out + ((slotT + t_b) * a.Hk + hk) * DK + kK * seg, x);
+      }
+      if (mine(2)) {
+        float x[kD];
+        convolve(a.block, slot, t_b, T, C, c_v, true, b_v, x);
+#pragma unroll
+        for (int e = 0; e < kD; ++e) sV[t_b * kRows + kD * seg + e] = x[e];
+      }
+      if (wave == 3 && lane < T) {
+        const float g = gate_of(a.block, gates);
+        if (row0 == 0 && a.block.g_out != nullptr) a.block.g_out[(slotT + lane) * a.Hv + hv] = g;
+        sS[4 * lane] = g;
+        sS[4 * lane + 1] = beta_of(gates);
+      }
+      __syncthreads();
+    } else {
+#pragma unroll
+      for (int e = 0; e < kK; ++e) asm volatile("" : "+v"(rq[e]), "+v"(rk[e])::"memory");
+#pragma unroll
+      for (int e = 0; e < kD; ++e) asm volatile("" : "+v"(rv[e])::"memory");
+      asm volatile("" : "+v"(g_bits), "+v"(beta_bits)::"memory");
+    }
     float kq = 0.f;  // k . q of step t16: 16 lanes, kK products each
 #pragma unroll
     for (int e = 0; e < kK; ++e) {
-      const float q = bits_element(rq, e, a.in_dtype), k = bits_element(rk, e, a.in_dtype);
-      sQ[t16 * DK + plane_index<DK>(kK * seg + e)] = q;
-      sK[t16 * DK + plane_index<DK>(kK * seg + e)] = k;
+      const int at = t16 * DK + plane_index<DK>(kK * seg + e);
+      const float q = BLOCK ? sQ[at] : bits_element(rq, e, a.in_dtype), k = BLOCK ? sK[at] : bits_element(rk, e, a.in_dtype);
+      if (!BLOCK) sQ[at] = q, sK[at] = k;
       kq = fmaf(k, q, kq);
     }
     kq = sum_over_16(kq);
     if (seg == 0) sS[4 * t16 + 2] = kq;
+    if (!BLOCK) {
 #pragma unroll
-    for (int e = 0; e < kD; ++e) sV[t16 * kRows + kD * seg + e] = bits_element(rv, e, a.in_dtype);
-    if (tid < 16) {
+      for (int e = 0; e < kD; ++e) sV[t16 * kRows + kD * seg + e] = bits_element(rv, e, a.in_dtype);
+    }
+    if (!BLOCK && tid < 16) {
       const uint32_t g1[1] = {g_bits}, b1[1] = {beta_bits};
       sS[4 * tid] = bits_element(g1, 0, a.g_dtype);
       sS[4 * tid + 1] = bits_element(b1, 0, a.beta_dtype);
@@ -449,13 +501,23 @@ __global__ __launch_bounds__(kThreads) void gdn_forward_rows(GdnArgs a) {
 }
 
 // The form of gdn_forward_rows for a head size and state type; rows: how many a workgroup computes.
-template <int STATE>
+template <int STATE, bool BLOCK>
 const void* forward_rows_for(int Dk, int Dv, bool many, int* rows) {
-  if (Dk == 128 && many && Dv % 32 == 0) return *rows = 32, (const void*)gdn_forward_rows<STATE, 128, 2>;
-  if (Dk == 128 && Dv % 16 == 0) return *rows = 16, (const void*)gdn_forward_rows<STATE, 128, 1>;
-  if (Dk == 64 && many && Dv % 64 == 0) return *rows = 64, (const void*)gdn_forward_rows<STATE, 64, 2>;
-  if (Dk == 64 && Dv % 32 == 0) return *rows = 32, (const void*)gdn_forward_rows<STATE, 64, 1>;
+  if (Dk == 128 && many && Dv % 32 == 0) return *rows = 32, (const void*)gdn_forward_rows<STATE, 128, 2, BLOCK>;
+  if (Dk == 128 && Dv % 16 == 0) return *rows = 16, (const void*)gdn_forward_rows<STATE, 128, 1, BLOCK>;
+  if (Dk == 64 && many && Dv % 64 == 0) return *rows = 64, (const void*)gdn_forward_rows<STATE, 64, 2, BLOCK>;
+  if (Dk == 64 && Dv % 32 == 0) return *rows = 32, (const void*)gdn_forward_rows<STATE, 64, 1, BLOCK>;
   return nullptr;
+}
+// Step by step in registers.  Two rows per lane, which share the reads of k and q, from 32 K rows on (128 x 128 at 16
+// steps, us, one and two rows: 96 heads 11.3 and 12.9, 256 heads 23.7 and 21.5, 1024 heads 77 and 69; 64 x 64, 512 heads 12.9 and 13.2,
+// 1024 heads 22.3 and 21.2).
+template <bool BLOCK>
+const void* forward_rows_for(int state_dtype, int slots, int Hv, int Dk, int Dv, int* rows) {
+  const bool many = (long long)slots * Hv * Dv >= 32768;
+  return state_dtype == DFLASH_BF16   ? forward_rows_for<DFLASH_BF16, BLOCK>(Dk, Dv, many, rows)
+         : state_dtype == DFLASH_FP16 ? forward_rows_for<DFLASH_FP16, BLOCK>(Dk, Dv, many, rows)
+                                      : forward_rows_for<DFLASH_FP32, BLOCK>(Dk, Dv, many, rows);
 }
 
 // ---------------------------------------------------------------------------
@@ -541,17 +603,30 @@ struct Incoming {
   f32x4_t z4[2], w4[2];  // fp32 elements
   f32x4_t st[2][8];
 };
-template <bool WIDE, bool NORM>
-__device__ __forceinline__ void issue_item_loads(const GdnArgs& a, int item, int tid, Incoming<WIDE>& in) {
+struct BlockIncoming {
+  ConvRows<8> rows[3];  // q, k, v
+  GateBits gates;
+};
+// Channel of lane group `seg` in q (0), k (1) or v (2).
+__device__ __forceinline__ int block_channel(const GdnArgs& a, int which, int hv, int hk, int seg) {
+  return (which == 0 ? hk : which == 1 ? a.Hk + hk : 2 * a.Hk + hv) * 128 + 8 * seg;
+}
+template <bool WIDE, bool NORM, bool BLOCK>
+__device__ __forceinline__ void issue_item_loads(const GdnArgs& a, int item, int tid, Incoming<WIDE>& in, BlockIncoming& block) {
   const int T = a.T;
   const int slot = item / a.Hv, hv = item % a.Hv, hk = hv / (a.Hv / a.Hk);
   const size_t slotT = (size_t)slot * T;
-  const int lane = tid & 63, wave = tid >> 6, li = lane & 15, kq = lane >> 4;
+  const int lane = tid & 63, wave = BLOCK ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6, li = lane & 15, kq = lane >> 4;
   // the block's operands first, the state behind them: loads complete in order
 #pragma unroll
   for (int j = 0; j < (WIDE ? 2 : 1); ++j) in.k.w[j] = in.q.w[j] = in.v.w[j] = uint4{0u, 0u, 0u, 0u};
   const int t = tid >> 4, seg = tid & 15;
-  if (t < T) {
+  if constexpr (BLOCK) {
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+      request_rows(a.block, slot, T <= 4 ? lane >> 4 : t, T, (2 * a.Hk + a.Hv) * 128, block_channel(a, j, hv, hk, seg), block.rows[j]);
+    block.gates = request_gates(a.block, slot, lane < T ? lane : T - 1, hv);
+  } else if (t < T) {
     const size_t kq_at = ((slotT + t) * a.Hk + hk) * 128 + 8 * seg;
     const size_t v_at = ((slotT + t) * a.Hv + hv) * 128 + 8 * seg;
     in.k = load8_raw<WIDE>(a.k, kq_at);
@@ -562,7 +637,7 @@ __device__ __forceinline__ void issue_item_loads(const GdnArgs& a, int item, int
   // state has been asked for, so that no request waits for another one's answer
   in.gate_bits = in.beta_bits = 0u;
   in.mask_byte = 1u;
-  if (tid < T && tid < 16) {
+  if (!BLOCK && tid < T && tid < 16) {
     const size_t at = (slotT + tid) * a.Hv + hv;
     if (a.g_dtype == DFLASH_FP32) {
       in.gate_bits = ((const uint32_t*)a.g)[at];
@@ -606,15 +681,18 @@ __device__ __forceinline__ void issue_item_loads(const GdnArgs& a, int item, int
   // Fence: everything above is on its way before the first of these values is looked at.
   asm volatile("" : "+v"(in.gate_bits), "+v"(in.beta_bits), "+v"(in.mask_byte)::"memory");
 }
-__device__ __forceinline__ float bits_as_f32(uint32_t bits, int dt) {
-  return dt == DFLASH_BF16 ? bf16_bits_to_f32(bits) : dt == DFLASH_FP16 ? f16_bits_to_f32(bits) : __uint_as_float(bits);
-}
-
 // One workgroup per (slot, head); the register cap keeps at least three on a compute unit.
 // SPLIT: q and k are bf16 arrays; the products with S0 and the state update run on the bf16
 // matrix cores with the fp32 factor in three exact pieces (see split_bf16).
-template <bool WIDE, bool NORM, bool SPLIT>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3, 3))) void gdn_forward_chunk_128(GdnArgs a) {
+// BLOCK: q, k, v, the gates and beta are made here, from the block's projections (gdn_block_device.h), while the state is on its
+// way.  A launch of the prepare kernel before this one took 5.4 us for what is 0.4 MB, and a microsecond to the next; here it is
+// 3.3 us of vector instructions (32 of 256 compute units have a head to work on): 16 tokens of 32 heads 13.3 + 5.4 -> 16.6 us, the
+// layer's verify block with its rollback 49.2 -> 47.1 us of device time, one token through a layer of 16-bit states (gdn_forward_rows)
+// 30.0 -> 25.1.  256 registers instead of 168: the rows, the taps and the state are all in flight at once, and a launch
+// this small has no second workgroup for a compute unit.
+template <bool WIDE, bool NORM, bool SPLIT, bool BLOCK>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(BLOCK ? 2 : 3, BLOCK ? 2 : 3)))
+void gdn_forward_chunk_128(GdnArgs a) {
   extern __shared__ __align__(16) float smem[];
   float* sK = smem + kOffK;
   float* sQ = smem + kOffQ;
@@ -637,20 +715,58 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3, 3))
 
   Incoming<WIDE> cur;
   const int item = blockIdx.x;
-  issue_item_loads<WIDE, NORM>(a, item, tid, cur);
+  BlockIncoming block;
+  issue_item_loads<WIDE, NORM, BLOCK>(a, item, tid, cur, block);
   const int slot = item / a.Hv, hv = item % a.Hv;
   const size_t slotT = (size_t)slot * T;
   const size_t sbase = (size_t)item * 128 * 128;
   f32x4_t (&st)[2][8] = cur.st;
   uint2 (&z2)[2] = cur.z2, (&w2)[2] = cur.w2;
   f32x4_t (&z4)[2] = cur.z4, (&w4)[2] = cur.w4;
-  {
+  if constexpr (BLOCK) {
+    const int seg = tid & 15, per = a.Hv / a.Hk, hk = hv / per, C = (2 * a.Hk + a.Hv) * 128;
+    // every wave its four steps of q, k and v, of up to four steps in all one of the three
+    const bool few = T <= 4;
+    const int t = few ? lane >> 4 : tid >> 4;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      float* const dst = j == 0 ? sQ : j == 1 ? sK : sV;
+      const int pitch = j == 2 ? 128 : kKPad;
+      float x[8] = {};
+      if (few ? wave == j : 4 * wave < T) {
+        const bool keeps = j == 2 || hv % per == 0;  // a key head's: by the first of its value heads
+        convolve(a.block, slot, t, T, C, block_channel(a, j, hv, hk, seg), keeps, block.rows[j], x);
+        if (j < 2) normalise<8, 16>(x, j == 1 ? a.block.scale_k : a.block.scale_q, a.block.eps);
+        if (j == 1 && keeps && t < T && a.block.k_out != nullptr)
+          store_exact<8>(a.block.k_out + ((slotT + t) * a.Hk + hk) * 128 + 8 * seg, x);
+      }
+      const auto put = [&](int step, bool on) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 8; e += 4)
+          *reinterpret_cast<f32x4_t*>(dst + step * pitch + 8 * seg + e) =
+              on ? f32x4_t{x[e], x[e + 1], x[e + 2], x[e + 3]} : f32x4_t{0.f, 0.f, 0.f, 0.f};
+      };
+      if (!few) {
+        put(t, t < T);
+      } else if (wave == j) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) put(4 * i + t, i == 0 && t < T);
+      }
+    }
+    if (wave == 3 && lane < 16) {
+      const float g = lane < T ? gate_of(a.block, block.gates) : 1.f;
+      if (lane < T && a.block.g_out != nullptr) a.block.g_out[(slotT + lane) * a.Hv + hv] = g;
+      sGate[lane] = g;
+      sBeta[lane] = lane < T ? beta_of(block.gates) : 0.f;
+      sOn[lane] = lane < T ? 1.f : 0.f;
+    }
+  } else {
     const int t = tid >> 4, seg = tid & 15;
     raw8_to_lds(cur.k, a.in_dtype, sK + t * kKPad + 8 * seg);
     raw8_to_lds(cur.q, a.in_dtype, sQ + t * kKPad + 8 * seg);
     raw8_to_lds(cur.v, a.in_dtype, sV + t * 128 + 8 * seg);
   }
-  if (tid < 16) {
+  if (!BLOCK && tid < 16) {
     const bool on = tid < T && cur.mask_byte != 0;  // masked and missing steps: gate 1, beta 0
     sGate[tid] = on ? bits_as_f32(cur.gate_bits, a.g_dtype) : 1.f;
     sBeta[tid] = on ? bits_as_f32(cur.beta_bits, a.beta_dtype) : 0.f;
@@ -1035,17 +1151,11 @@ int gdn_forward_launch(const char* who, const void* q, const void* k, const void
                     (state_dtype != DFLASH_FP32 ||
                      (((uintptr_t)state_in % 16) == 0 && ((uintptr_t)state_out % 16) == 0));
   const bool chunk = fast && !g_per_dk && state_dtype == DFLASH_FP32 && T <= 16 && aligned16 && !no_chunk;
-  // Step by step in registers.  Two rows per lane, which share the reads of k and q, from 32 K rows on (128 x 128 at 16
-  // steps, us, one and two rows: 96 heads 11.3 and 12.9, 256 heads 23.7 and 21.5, 1024 heads 77 and 69; 64 x 64, 512 heads 12.9 and 13.2,
-  // 1024 heads 22.3 and 21.2).
   const void* by_rows = nullptr;
   int rows = Dv;
   if (!prompt && !chunk && !g_per_dk && T >= 1 && aligned16 && (((uintptr_t)state_in | (uintptr_t)state_out) % 16) == 0 &&
       !(fast && state_dtype == DFLASH_FP32)) {
-    const bool many = (long long)slots * Hv * Dv >= 32768;
-    by_rows = state_dtype == DFLASH_BF16   ? forward_rows_for<DFLASH_BF16>(Dk, Dv, many, &rows)
-              : state_dtype == DFLASH_FP16 ? forward_rows_for<DFLASH_FP16>(Dk, Dv, many, &rows)
-                                           : forward_rows_for<DFLASH_FP32>(Dk, Dv, many, &rows);
+    by_rows = forward_rows_for<false>(state_dtype, slots, Hv, Dk, Dv, &rows);
     if ((long long)slots * Hv * (Dv / rows) >= (1ll << 31)) by_rows = nullptr;
   }
   bool norm_done = false;
@@ -1061,14 +1171,14 @@ int gdn_forward_launch(const char* who, const void* q, const void* k, const void
     const bool wide = in_dtype == DFLASH_FP32;
     const bool split = in_dtype == DFLASH_BF16;  // q and k are bf16 numbers: exact products on the bf16 matrix cores
     if (z) {
-      if (wide) hipLaunchKernelGGL((gdn_forward_chunk_128<true, true, false>), grid, block, lds, s, a);
-      else if (split) hipLaunchKernelGGL((gdn_forward_chunk_128<false, true, true>), grid, block, lds, s, a);
-      else hipLaunchKernelGGL((gdn_forward_chunk_128<false, true, false>), grid, block, lds, s, a);
+      if (wide) hipLaunchKernelGGL((gdn_forward_chunk_128<true, true, false, false>), grid, block, lds, s, a);
+      else if (split) hipLaunchKernelGGL((gdn_forward_chunk_128<false, true, true, false>), grid, block, lds, s, a);
+      else hipLaunchKernelGGL((gdn_forward_chunk_128<false, true, false, false>), grid, block, lds, s, a);
       norm_done = true;
     } else {
-      if (wide) hipLaunchKernelGGL((gdn_forward_chunk_128<true, false, false>), grid, block, lds, s, a);
-      else if (split) hipLaunchKernelGGL((gdn_forward_chunk_128<false, false, true>), grid, block, lds, s, a);
-      else hipLaunchKernelGGL((gdn_forward_chunk_128<false, false, false>), grid, block, lds, s, a);
+      if (wide) hipLaunchKernelGGL((gdn_forward_chunk_128<true, false, false, false>), grid, block, lds, s, a);
+      else if (split) hipLaunchKernelGGL((gdn_forward_chunk_128<false, false, true, false>), grid, block, lds, s, a);
+      else hipLaunchKernelGGL((gdn_forward_chunk_128<false, false, false, false>), grid, block, lds, s, a);
     }
   } else if (by_rows != nullptr) {
     void* args[] = {&a};
@@ -1091,8 +1201,79 @@ int gdn_forward_launch(const char* who, const void* q, const void* k, const void
   return DFLASH_OK;
 }
 
+// The value a Python float takes when it meets a bf16 array.
+float as_bf16_scalar(double v) {
+  const float f = (float)v;
+  uint32_t u;
+  __builtin_memcpy(&u, &f, 4);
+  u += 0x7fffu + ((u >> 16) & 1u);
+  u &= 0xffff0000u;
+  float r;
+  __builtin_memcpy(&r, &u, 4);
+  return r;
+}
+
 }  // namespace
 }  // namespace dflash
+
+extern "C" int dflash_gdn_block(const dflash_gdn_block_args* p, void* stream) {
+  using namespace dflash;
+  const char* who = "dflash_gdn_block";
+  DFLASH_REQUIRE(p && p->qkv && p->conv_w && p->a && p->b && p->A_log && p->dt_bias && p->conv_next && p->state_in && p->state_out &&
+                     p->y && p->tape && (!p->z || p->norm_weight),
+                 DFLASH_ERR_ARG, "%s: null operand", who);
+  DFLASH_REQUIRE(p->state_in != p->state_out, DFLASH_ERR_ARG, "%s: state_out must not alias state_in", who);
+  auto ok = [](int dt) { return dt == DFLASH_BF16 || dt == DFLASH_FP16 || dt == DFLASH_FP32; };
+  DFLASH_REQUIRE(ok(p->param_dtype) && ok(p->state_dtype) && (!p->z || ok(p->weight_dtype)), DFLASH_ERR_ARG, "%s: unknown dtype code", who);
+  const int slots = p->slots, T = p->T, Hk = p->Hk, Hv = p->Hv, D = p->D;
+  DFLASH_REQUIRE(slots >= 0 && T >= 1 && T <= 16 && Hk > 0 && Hv > 0 && Hv % Hk == 0 && (D == 64 || D == 128), DFLASH_ERR_SHAPE,
+                 "%s: 1 to 16 steps of heads of 64 or 128, whole groups of value heads; got %d steps, %d and %d heads of %d", who, T, Hk,
+                 Hv, D);
+  DFLASH_REQUIRE(p->qkv_row < (1ll << 26), DFLASH_ERR_SHAPE, "%s: rows of %lld elements", who, p->qkv_row);
+  DFLASH_REQUIRE((long long)slots * Hv * 8 < (1ll << 31) && (long long)slots * T * (2ll * Hk + Hv) * D < (1ll << 31), DFLASH_ERR_SHAPE,
+                 "%s: too many (slot, head) pairs", who);
+  uintptr_t strides = 0;
+  for (long long v : {p->qkv_slot, p->qkv_row, p->a_slot, p->a_row, p->b_slot, p->b_row, p->z_slot, p->z_row})
+    DFLASH_REQUIRE(v >= 0, DFLASH_ERR_SHAPE, "%s: negative stride", who);
+  strides = (uintptr_t)(p->qkv_slot | p->qkv_row) * 2;
+  DFLASH_REQUIRE((((uintptr_t)p->qkv | (uintptr_t)p->conv_state | (uintptr_t)p->conv_w | (uintptr_t)p->conv_next | (uintptr_t)p->k |
+                   (uintptr_t)p->qkv_out | strides) % 8) == 0,
+                 DFLASH_ERR_ARG, "%s: projections, conv arrays and k must be 8-byte aligned", who);
+  DFLASH_REQUIRE((((uintptr_t)p->state_in | (uintptr_t)p->state_out | (uintptr_t)p->y | (uintptr_t)p->tape | (uintptr_t)p->z |
+                   (uintptr_t)p->norm_weight | (p->z ? (uintptr_t)(p->z_slot | p->z_row) * 2 : 0)) % 16) == 0,
+                 DFLASH_ERR_ARG, "%s: states, y, tape, z and the norm weight must be 16-byte aligned", who);
+  if (slots == 0) return DFLASH_OK;
+
+  GdnArgs a = {};
+  a.state_in = p->state_in; a.state_out = p->state_out; a.y = p->y; a.tape = p->tape;
+  a.T = T; a.Hk = Hk; a.Hv = Hv; a.Dk = a.Dv = D;
+  a.in_dtype = a.g_dtype = a.beta_dtype = DFLASH_BF16; a.state_dtype = p->state_dtype;
+  a.z = p->z; a.z_batch = p->z_slot; a.z_row = p->z_row; a.norm_weight = p->norm_weight; a.weight_dtype = p->weight_dtype;
+  a.eps = p->norm_eps;
+  BlockArgs& b = a.block;
+  b.qkv = (const uint16_t*)p->qkv; b.conv_state = (const uint16_t*)p->conv_state; b.conv_w = (const uint16_t*)p->conv_w;
+  b.a = (const uint16_t*)p->a; b.b = (const uint16_t*)p->b; b.A_log = p->A_log; b.dt_bias = p->dt_bias;
+  b.conv_next = (uint16_t*)p->conv_next; b.k_out = (uint16_t*)p->k; b.qkv_out = (uint16_t*)p->qkv_out; b.g_out = p->g;
+  b.qkv_slot = p->qkv_slot; b.qkv_row = p->qkv_row; b.a_slot = p->a_slot; b.a_row = p->a_row; b.b_slot = p->b_slot; b.b_row = p->b_row;
+  b.param_dt = p->param_dtype; b.eps = p->eps;
+  const double inv_scale = 1.0 / sqrt((double)D);
+  b.scale_q = as_bf16_scalar(inv_scale * inv_scale);
+  b.scale_k = as_bf16_scalar(inv_scale);
+
+  hipStream_t s = (hipStream_t)stream;
+  void* args[] = {&a};
+  if (D == 128 && p->state_dtype == DFLASH_FP32) {  // the closed form, its output norm in the same launch
+    const void* fn = p->z ? (const void*)gdn_forward_chunk_128<false, true, true, true> : (const void*)gdn_forward_chunk_128<false, false, true, true>;
+    DFLASH_HIP_OK(hipLaunchKernel(fn, dim3((unsigned)(slots * Hv)), dim3(kThreads), args, kChunkLdsFloats * sizeof(float), s));
+    return DFLASH_OK;
+  }
+  int rows = D;
+  const void* fn = forward_rows_for<true>(p->state_dtype, slots, Hv, D, D, &rows);
+  DFLASH_HIP_OK(hipLaunchKernel(fn, dim3((unsigned)(slots * Hv * (D / rows))), dim3(kThreads), args, 0, s));
+  return p->z ? gdn_gated_norm_launch(p->y, p->z, p->norm_weight, p->y, slots, T, Hv, D, p->z_slot, p->z_row, DFLASH_BF16, p->weight_dtype,
+                                      p->norm_eps, s)
+              : DFLASH_OK;
+}
 
 extern "C" int dflash_gdn_forward_tape(const void* q, const void* k, const void* v, const void* g,
                                        const void* beta, const void* state_in, void* state_out,

@@ -9,14 +9,16 @@
 // to the array dtype once; the arithmetic inside an operator is fp32.
 //
 // For a verify block these operators are a few hundred KB per layer, and the point of fusing them is the launch
-// count (two launches instead of about twenty elementwise kernels).  For a prompt they are bound by the vector
+// count (two launches instead of about twenty elementwise kernels; none of their own where gdn_forward.hip takes the
+// projections as they are).  For a prompt they are bound by the vector
 // instructions per element (the sigmoid's exponential and division, the roundings): a wave takes several tokens
 // of its head in turn, so that a row of qkv is read and unpacked once and not once per tap, the taps once per wave, and
 // the gates of all its tokens are computed side by side, one token per lane.  1024 tokens of 16 + 16 + 32 heads of
-// 128: 62 us with a wave per token and head, now 20.3 us; the gated norm 15 -> 10.1 us.  The projections are read where a joint product
+// 128: 62 us with a wave per token and head, 21.4 us with several tokens and the library's exponential and division, 17.5 us with
+// the hardware's for 16-bit arrays (errors against fp64 the same in six digits); the gated norm 15 -> 10.1 -> 8.6 us.  The projections are read where a joint product
 // left them (rows with a stride), which saves four copies per layer call (25 us of the same prompt, 12 us of a
 // verify block).
-#include "glue_device.h"
+#include "gdn_block_device.h"
 
 #include <cmath>
 
@@ -25,28 +27,6 @@ namespace {
 
 constexpr int kWavesPerGroup = 4;
 constexpr int kMaxPerLane = 4;  // head dims up to 256
-
-// Sum of the squares of a head: PER elements in each of LANES lanes (a power of two).  Adjacent elements first and in
-// sixty-fourths of the head whatever LANES is, so that a row has the same sum in the wide and the narrow kernels.
-template <int PER, int LANES>
-__device__ __forceinline__ float sum_of_squares(const float (&v)[PER]) {
-  constexpr int kEach = PER * LANES / 64, kParts = PER / kEach;
-  float part[kParts];
-#pragma unroll
-  for (int i = 0; i < kParts; ++i) {
-    part[i] = 0.f;
-#pragma unroll
-    for (int e = 0; e < kEach; ++e) part[i] += v[i * kEach + e] * v[i * kEach + e];
-  }
-#pragma unroll
-  for (int n = kParts / 2; n >= 1; n /= 2)
-#pragma unroll
-    for (int i = 0; i < n; ++i) part[i] = part[2 * i] + part[2 * i + 1];
-  float sum = part[0];
-#pragma unroll
-  for (int off = 1; off < LANES; off <<= 1) sum += __shfl_xor(sum, off, 64);
-  return sum;
-}
 
 struct PrepareArgs {
   const void* qkv;         // [B, S, C], rows and batches with a stride
@@ -107,10 +87,10 @@ __device__ __forceinline__ void prepare_head(const PrepareArgs& p, int b, int s0
   load_adjacent_raw<PER * K>(p.conv_w, (size_t)c * K, wide, wr);
   // gates of the value head's tokens, one per lane (key heads read some and do not use them)
   const int gate_token = s0 + lane < s1 ? s0 + lane : s1 - 1;
-  const uint32_t a_bits = load_bits(p.a, (size_t)b * p.a_batch + (size_t)gate_token * p.a_row + hv, wide);
-  const uint32_t b_bits = load_bits(p.b, (size_t)b * p.b_batch + (size_t)gate_token * p.b_row + hv, wide);
-  const uint32_t a_log_bits = load_bits(p.A_log, hv, pwide);
-  const uint32_t bias_bits = load_bits(p.dt_bias, hv, pwide);
+  const uint32_t a_bits = load_one(p.a, (size_t)b * p.a_batch + (size_t)gate_token * p.a_row + hv, wide);
+  const uint32_t b_bits = load_one(p.b, (size_t)b * p.b_batch + (size_t)gate_token * p.b_row + hv, wide);
+  const uint32_t a_log_bits = load_one(p.A_log, hv, pwide);
+  const uint32_t bias_bits = load_one(p.dt_bias, hv, pwide);
   asm volatile("" ::: "memory");  // every request above is out before the first value is interpreted
   float x[K][PER], w[PER * K];
 #pragma unroll
@@ -125,13 +105,9 @@ __device__ __forceinline__ void prepare_head(const PrepareArgs& p, int b, int s0
   if (is_v && lane < s1 - s0) {
     const float gate_a = bits_as_f32(a_bits, DT), gate_b = bits_as_f32(b_bits, DT);
     const float a_log = bits_as_f32(a_log_bits, p.param_dt), bias = bits_as_f32(bias_bits, p.param_dt);
-    // a + dt_bias and the softplus live in the promoted dtype of the two operands
-    const int sum_dt = pwide ? DFLASH_FP32 : DT;
-    const float apb = round_through(gate_a + bias, sum_dt);
-    const float sp = round_through(fmaxf(apb, 0.f) + log1pf(expf(-fabsf(apb))), sum_dt);
     const size_t at = (token0 + gate_token) * p.Hv + hv;
-    p.g[at] = expf(-expf(a_log) * sp);
-    store_from_f32(p.beta, at, sigmoid_f32(gate_b), DT);
+    p.g[at] = decay_of(gate_a, a_log, bias, pwide ? DFLASH_FP32 : DT);
+    store_from_f32(p.beta, at, sigmoid_for(gate_b, DT), DT);
   }
   if (s0 == 0) {
     for (int r = p.S; r < keep; ++r) {  // blocks shorter than the state: old rows move up

@@ -456,6 +456,90 @@ PyObject* gdn_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// gdn_block(qkv, conv_state, conv_w, a, b, A_log, dt_bias, z, weight, state, Hk, Hv, Dk, Dv, eps, norm_eps, record): a block of
+// up to 16 tokens without a mask in one launch, where that has a form for it; z [B, S, Hv Dv] and the norm's weight None, or what
+// the output norm takes.  (y, state, conv_next, tape, k, g, qkv in one piece); the last three None unless recorded, the last
+// one also where qkv is in one piece already.
+PyObject* gdn_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 17) Py_RETURN_NONE;
+  const Tensor *qkv = device_tensor(a[0]), *cs = nullptr, *w = device_tensor(a[2]), *ga = device_tensor(a[3]),
+               *gb = device_tensor(a[4]), *A = device_tensor(a[5]), *dt = device_tensor(a[6]), *z = nullptr, *weight = nullptr,
+               *state = device_tensor(a[9]);
+  if (!qkv || !w || !ga || !gb || !A || !dt || !state || qkv->dim() != 3) Py_RETURN_NONE;
+  if (a[1] != Py_None && !(cs = device_tensor(a[1]))) Py_RETURN_NONE;
+  if (a[7] != Py_None && (!(z = device_tensor(a[7])) || !(weight = device_tensor(a[8])))) Py_RETURN_NONE;
+  int Hk, Hv, D, Dv;
+  if (!integer(a[10], &Hk) || !integer(a[11], &Hv) || !integer(a[12], &D) || !integer(a[13], &Dv) || !PyFloat_CheckExact(a[14]) ||
+      !PyFloat_CheckExact(a[15]))
+    Py_RETURN_NONE;
+  const bool record = a[16] == Py_True;
+  const int64_t B = qkv->size(0), S = qkv->size(1), C = qkv->size(2);
+  const auto type = at::kBFloat16;
+  const auto device = qkv->device();
+  const int param = dtype_code(A->scalar_type()), s_code = dtype_code(state->scalar_type());
+  if (qkv->scalar_type() != type || param == kNoCode || s_code == kNoCode || D != Dv || (D != 64 && D != 128) || B < 1 || S < 1 ||
+      S > 16 || Hk < 1 || Hv < 1 || Hk > (1 << 15) || Hv > (1 << 15) || Hv % Hk != 0 || C != 2 * (int64_t)Hk * D + (int64_t)Hv * D ||
+      B * S * (2 * Hk + Hv) * D >= (1ll << 31) || dflash_get_option(DFLASH_OPT_GDN_STEP_BY_STEP) != 0)
+    Py_RETURN_NONE;
+  if (w->dim() < 2 || w->dim() > 3 || w->size(0) != C || w->size(1) != 4 || (w->dim() == 3 && w->size(2) != 1) ||
+      !w->is_contiguous() || w->scalar_type() != type || ga->scalar_type() != type || gb->scalar_type() != type ||
+      dt->scalar_type() != A->scalar_type() || !has_shape(*ga, {B, S, Hv}) || !has_shape(*gb, {B, S, Hv}) || !has_shape(*A, {Hv}) ||
+      !has_shape(*dt, {Hv}) || !A->is_contiguous() || !dt->is_contiguous() || !has_shape(*state, {B, Hv, D, D}) ||
+      !state->is_contiguous() || !aligned(at_of(*state), 16))
+    Py_RETURN_NONE;
+  for (const Tensor* t : {w, ga, gb, A, dt, state})
+    if (t->device() != device) Py_RETURN_NONE;
+  if (cs && (cs->scalar_type() != type || !has_shape(*cs, {B, 3, C}) || cs->device() != device || !cs->is_contiguous() ||
+             !aligned(at_of(*cs), 8)))
+    Py_RETURN_NONE;
+  if (qkv->stride(2) != 1 || !aligned(at_of(*qkv), 8) || (qkv->stride(0) | qkv->stride(1)) % 4 != 0 || qkv->stride(1) >= (1 << 26) || !aligned(at_of(*w), 8) ||
+      ga->stride(2) != 1 || gb->stride(2) != 1)
+    Py_RETURN_NONE;
+  if (z && (z->scalar_type() != type || !has_shape(*z, {B, S, (int64_t)Hv * D}) || z->device() != device || z->stride(2) != 1 ||
+            (z->stride(0) | z->stride(1)) % 8 != 0 || !aligned(at_of(*z), 16) || dtype_code(weight->scalar_type()) == kNoCode ||
+            weight->numel() != D || !weight->is_contiguous() || weight->device() != device || !aligned(at_of(*weight), 16)))
+    Py_RETURN_NONE;
+  dflash_gdn_block_args p = {};
+  p.qkv = at_of(*qkv), p.conv_state = cs ? at_of(*cs) : nullptr, p.conv_w = at_of(*w), p.a = at_of(*ga), p.b = at_of(*gb);
+  p.A_log = at_of(*A), p.dt_bias = at_of(*dt), p.state_in = at_of(*state);
+  p.qkv_slot = qkv->stride(0), p.qkv_row = qkv->stride(1), p.a_slot = ga->stride(0), p.a_row = ga->stride(1);
+  p.b_slot = gb->stride(0), p.b_row = gb->stride(1);
+  if (z) p.z = at_of(*z), p.norm_weight = at_of(*weight), p.z_slot = z->stride(0), p.z_row = z->stride(1);
+  p.slots = (int)B, p.T = (int)S, p.Hk = Hk, p.Hv = Hv, p.D = D, p.param_dtype = param, p.state_dtype = s_code;
+  p.weight_dtype = z ? dtype_code(weight->scalar_type()) : DFLASH_BF16;
+  p.eps = (float)PyFloat_AS_DOUBLE(a[14]), p.norm_eps = (float)PyFloat_AS_DOUBLE(a[15]);
+  void* stream = stream_of(*qkv);
+  Tensor y, next, conv, tape, k, g, one;
+  const int rc = released([&] {
+    const auto options = qkv->options();
+    y = at::empty({B, S, Hv, D}, options);
+    next = at::empty({B, Hv, D, D}, state->options());
+    conv = at::empty({B, 3, C}, options);
+    tape = at::empty({B, S, Hv, D}, options.dtype(at::kFloat));
+    p.y = y.mutable_data_ptr(), p.state_out = next.mutable_data_ptr(), p.conv_next = conv.mutable_data_ptr();
+    p.tape = (float*)tape.mutable_data_ptr();
+    if (record) {
+      k = at::empty({B, S, Hk, D}, options);
+      g = at::empty({B, S, Hv}, options.dtype(at::kFloat));
+      p.k = k.mutable_data_ptr(), p.g = (float*)g.mutable_data_ptr();
+      if (!qkv->is_contiguous()) {
+        one = at::empty({B, S, C}, options);
+        p.qkv_out = one.mutable_data_ptr();
+      }
+    }
+    return dflash_gdn_block(&p, stream);
+  });
+  if (rc != 0) return fail(rc, "dflash_gdn_block");
+  const auto wrapped = [](Tensor&& t) -> PyObject* {
+    if (!t.defined()) Py_RETURN_NONE;
+    return THPVariable_Wrap(std::move(t));
+  };
+  return Py_BuildValue("(NNNNNNN)", wrapped(std::move(y)), wrapped(std::move(next)), wrapped(std::move(conv)), wrapped(std::move(tape)),
+                       wrapped(std::move(k)), wrapped(std::move(g)), wrapped(std::move(one)));
+  END_HANDLE_TH_ERRORS
+}
+
 // rollback_layer(tape, k, g, qkv, state, conv_prev, steps, keep, exact): replay and conv window of one cache's tape;
 // (state, conv window).
 PyObject* rollback_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -555,7 +639,7 @@ PyObject* bind(PyObject*, PyObject* error) {  // the class that failed launches 
 
 #define DFLASH_HOST(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
 PyMethodDef kMethods[] = {DFLASH_HOST(qmm_m16), DFLASH_HOST(qmm_packed), DFLASH_HOST(qmm_few), DFLASH_HOST(qmm_few_silu_mul),
-                          DFLASH_HOST(qmm_rows), DFLASH_HOST(columns), DFLASH_HOST(gather), DFLASH_HOST(chain_bind), DFLASH_HOST(chain_launch), DFLASH_HOST(gdn_prepare), DFLASH_HOST(gdn_forward),
+                          DFLASH_HOST(qmm_rows), DFLASH_HOST(columns), DFLASH_HOST(gather), DFLASH_HOST(chain_bind), DFLASH_HOST(chain_launch), DFLASH_HOST(gdn_prepare), DFLASH_HOST(gdn_forward), DFLASH_HOST(gdn_block),
                           DFLASH_HOST(rollback_layer), DFLASH_HOST(sdpa_q16), {"bind", bind, METH_O, nullptr},
                           {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_dflash_host", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};

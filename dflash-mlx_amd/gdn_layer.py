@@ -252,9 +252,30 @@ def _gdn_call(self, inputs: torch.Tensor, mask: Optional[torch.Tensor], cache: O
     B, S, _ = inputs.shape
     # one launch for those of the four that fuse_shared_input_linears joined
     qkv, z, b, a = shared_input_outputs(self, ("in_proj_qkv", "in_proj_z", "in_proj_b", "in_proj_a"), inputs, columns=True)
+    conv_state = cache[0] if cache is not None else None
+    norm = self.norm
+    normed = isinstance(norm, RMSNormGated) and _native.env(b"DFLASH_GDN_FUSED_NORM") != b"0"
+    if mask is None and S <= 16 and qkv.is_cuda:
+        # a block: conv, gates, recurrence and norm in one launch, where there is one for these sizes and types
+        state = cache[1] if cache is not None else None
+        if state is None:
+            state = torch.zeros((B, self.num_v_heads, self.head_v_dim, self.head_k_dim), dtype=qkv.dtype, device=qkv.device)
+        made = _native.host().gdn_block(
+            qkv, conv_state, self.conv1d.weight, a, b, self.A_log, self.dt_bias, z if normed else None, norm.weight if normed else None,
+            state, self.num_k_heads, self.num_v_heads, self.head_k_dim, self.head_v_dim, 1e-6, norm.eps if normed else 0.0, bool(record))
+        if made is not None:
+            out, state, conv_next, tape, k, g, tape_qkv = made
+            if cache is not None:
+                cache[0] = conv_next
+            if record:
+                cache.record_tape(tape=tape, k=k, g=g, qkv=qkv if tape_qkv is None else tape_qkv)
+            if cache is not None:
+                cache[1] = state
+            if not normed:
+                out = norm(out, z.reshape(B, S, self.num_v_heads, self.head_v_dim).contiguous())
+            return self.out_proj(out.view(B, S, -1))
     z = z.reshape(B, S, self.num_v_heads, self.head_v_dim)
 
-    conv_state = cache[0] if cache is not None else None
     # the rollback wants qkv in one piece, without what the mask hides
     tape_qkv = qkv
     if record and (mask is not None or not qkv.is_contiguous()):
@@ -270,9 +291,7 @@ def _gdn_call(self, inputs: torch.Tensor, mask: Optional[torch.Tensor], cache: O
     if state is None:
         state = torch.zeros((B, self.num_v_heads, self.head_v_dim, self.head_k_dim), dtype=q.dtype, device=q.device)
     # the layer's output norm rides on the recurrence's launch where the kernel takes it
-    norm = self.norm
-    fused = (isinstance(norm, RMSNormGated) and _native.env(b"DFLASH_GDN_FUSED_NORM") != b"0" and
-             fused_output_norm_applies(q, v, state, z, norm.weight))
+    fused = normed and fused_output_norm_applies(q, v, state, z, norm.weight)
     out, state, innovation_tape = gated_delta_kernel_with_tape(
         q, k, v, g, beta, state, mask, output_norm=(z, norm.weight, norm.eps) if fused else None, with_tape=record)
     if record:

@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define DFLASH_ABI_VERSION 21
+#define DFLASH_ABI_VERSION 22
 
 enum {
   DFLASH_OK = 0,
@@ -437,6 +437,30 @@ int dflash_gdn_prepare_rows(const void* qkv, const void* conv_state, const void*
                             void* conv_next, void* q, void* k, void* v, float* g, void* beta, void* qkv_out,
                             const long long* strides, int B, int S, int Hk, int Hv, int Dk, int Dv,
                             int conv_kernel, int dtype, int param_dtype, float eps, void* stream);
+
+/*
+ * A block of up to 16 tokens of a GatedDeltaNet layer from its projections to its (normed) output in one launch: what
+ * dflash_gdn_prepare_rows and dflash_gdn_forward do one after the other, bit for bit, for bf16 arrays, 4 taps, Dk = Dv = D of
+ * 64 or 128, no mask.  (16-bit states and heads of 64 have the output norm in a launch of its own.)
+ *   qkv, a, b     rows and slots with strides in elements, qkv 8-byte aligned;  conv_state NULL: zeros
+ *   conv_next     [slots, 3, C];  k [slots, T, Hk, D], qkv_out [slots, T, C] and g [slots, T, Hv]: NULL where not wanted
+ *   z             [slots, T, Hv, D] with strides, 16-byte aligned, norm_weight [D]; z NULL: y is the recurrence's output
+ *   state_in, state_out [slots, Hv, D, D], y bf16 [slots, T, Hv, D], tape fp32 likewise: 16-byte aligned
+ */
+typedef struct dflash_gdn_block_args {
+  const void *qkv, *conv_state, *conv_w, *a, *b, *A_log, *dt_bias;
+  long long qkv_slot, qkv_row, a_slot, a_row, b_slot, b_row;
+  void *conv_next, *k, *qkv_out;
+  float* g;
+  const void *z, *norm_weight;
+  long long z_slot, z_row;
+  const void* state_in;
+  void *state_out, *y;
+  float* tape;
+  int slots, T, Hk, Hv, D, param_dtype, state_dtype, weight_dtype;
+  float eps, norm_eps;
+} dflash_gdn_block_args;
+int dflash_gdn_block(const dflash_gdn_block_args* args, void* stream);
 
 /*
  * Gated output norm of a GatedDeltaNet layer: y = silu(z) * rms_norm(x, weight, eps) over rows of

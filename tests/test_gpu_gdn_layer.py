@@ -246,3 +246,92 @@ def test_output_norm_reads_a_strided_gate(native_lib, name, B, T, Hv, Dv, state)
     pieces = [G.gated_norm(plain[:, t:t + 16], z[:, t:t + 16], weight) for t in range(0, T, 16)]
     assert torch.equal(G.gated_norm(plain, z, weight), torch.cat(pieces, dim=1))
     assert torch.allclose(got[0].float(), torch.cat(pieces, dim=1).float(), rtol=4 * ULP[name], atol=1e-4)
+
+
+class _Given(torch.nn.Module):
+    def __init__(self, out):
+        super().__init__()
+        self.out = out
+
+    def forward(self, x):
+        return self.out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("state_dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,S,Hk,Hv,D,joint", [(1, 1, 2, 4, 128, True), (2, 16, 2, 2, 128, True), (1, 5, 1, 3, 128, False), (1, 2, 2, 4, 64, True),
+                                               (3, 16, 1, 2, 64, False), (1, 15, 2, 4, 64, True), (1, 3, 4, 256, 128, True),
+                                               (1, 16, 16, 512, 64, True)])
+def test_a_block_in_one_launch(monkeypatch, state_dtype, B, S, Hk, Hv, D, joint):
+    """The bits of the prepare kernel followed by the recurrence, for every state type, tokens fewer than taps, one row per lane and
+    two, with and without windows, tapes, norms, joint products and fp32 gates; forms it does not have are left to them."""
+    import dflash_mlx_amd._native as nat
+    from dflash_mlx_amd import gdn_layer as G
+    from dflash_mlx_amd.recurrent_rollback_cache import RecurrentRollbackCache
+
+    gen = torch.Generator("cuda").manual_seed(S + D)
+
+    def r(*shape, std=1.0, to=torch.bfloat16):
+        return (torch.randn(shape, generator=gen, device="cuda") * std).to(to)
+
+    C = 2 * Hk * D + Hv * D
+    cut = (C, Hv * D, Hv, Hv)
+    parts = r(B, S, sum(cut) + 8 - sum(cut) % 8)[..., :sum(cut)].split(cut, dim=-1) if joint else [r(B, S, n) for n in cut]
+    mixer = G.GatedDeltaNet(8, num_k_heads=Hk, num_v_heads=Hv, head_k_dim=D, head_v_dim=D, in_proj_qkv=_Given(parts[0]),
+                            in_proj_z=_Given(parts[1]), in_proj_b=_Given(parts[2]), in_proj_a=_Given(parts[3]),
+                            out_proj=torch.nn.Identity()).cuda()
+    mixer.conv1d.weight.data = r(C, 4, 1, std=0.5)
+    mixer.norm.weight.data = 1 + r(D, std=0.1)
+    x, window, state = torch.zeros((B, S, 8), device="cuda"), r(B, 3, C), r(B, Hv, D, D, std=0.1, to=state_dtype)
+    served = []
+
+    class Watched:
+        def __init__(self, block):
+            self.block = block
+
+        def __call__(self):
+            return self
+
+        def __getattr__(self, name):
+            def call(*args):
+                out = None if name == "gdn_block" and not self.block else getattr(real, name)(*args)
+                if name == "gdn_block" and self.block:
+                    served.append(out is not None)
+                return out
+
+            return call
+
+    real = nat.host()
+
+    def run(block, window, state, record, mask=None):
+        cache = RecurrentRollbackCache(size=2, conv_kernel_size=4)
+        cache[0], cache[1] = window, state
+        with monkeypatch.context() as m:
+            m.setattr(nat, "host", Watched(block))
+            if record:
+                cache.arm_rollback()
+            y = G._gdn_call(mixer, x, mask, cache, record)
+        return y, cache[0], cache[1], cache._tape, cache._tape_k, cache._tape_g, cache._tape_qkv
+
+    def same(expected, *args):
+        del served[:]
+        for got, want in zip(run(True, *args), run(False, *args)):
+            assert (got is None) == (want is None)
+            assert got is None or (got.shape == want.shape and got.dtype == want.dtype and torch.equal(got, want))
+        assert served == expected
+
+    for record in (True, False):
+        same([True], window, state, record)
+        same([True], None, None if state_dtype == torch.bfloat16 else state, record)
+    for dtype in (torch.float32, torch.bfloat16):
+        mixer.A_log.data, mixer.dt_bias.data = r(Hv, to=dtype), r(Hv, std=0.3, to=dtype)
+        same([True], window, state, True)
+    mixer.norm.weight.data = mixer.norm.weight.data.float()
+    same([True], window, state, False)
+    monkeypatch.setenv("DFLASH_GDN_FUSED_NORM", "0")
+    same([True], window, state, False)
+    monkeypatch.delenv("DFLASH_GDN_FUSED_NORM")
+    same([], window, state, True, torch.ones((B, S), dtype=torch.bool, device="cuda"))
+    shifted = torch.zeros(state.numel() + 1, dtype=state.dtype, device="cuda")
+    shifted[1:] = state.reshape(-1)
+    same([False], window, shifted[1:].view(state.shape), True)
