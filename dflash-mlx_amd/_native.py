@@ -18,7 +18,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libdflash_mi355.so")
 HOST_PATH = os.path.join(_HERE, "_dflash_host.so")
 
-ABI_VERSION = 22
+ABI_VERSION = 23
 
 BF16, FP16, FP32 = 0, 1, 2
 QMM_MMA2BIG, QMM_MMA2BIG_PIPE = 0, 1
@@ -58,6 +58,7 @@ EXPORTED_SYMBOLS = (
     "dflash_qmm_m16_packed_bytes",
     "dflash_qmm_m16_pack",
     "dflash_qmm_m16_packed",
+    "dflash_qmm_m16_packed_by",
     "dflash_qmm_rows_workspace_bytes",
     "dflash_qmm_rows",
     "dflash_qmm_m16_gather_workspace_bytes",
@@ -126,6 +127,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.dflash_qmm_m16_pack_gate_up.argtypes = [c.c_void_p] * 6 + [c.c_int] * 3 + [c.c_void_p]
     lib.dflash_qmm_m16_packed.restype = c.c_int
     lib.dflash_qmm_m16_packed.argtypes = [c.c_void_p] * 6 + [c.c_size_t] + [c.c_int] * 5 + [c.c_void_p]
+    lib.dflash_qmm_m16_packed_by.restype = c.c_int
+    lib.dflash_qmm_m16_packed_by.argtypes = [c.c_void_p] * 6 + [c.c_size_t] + [c.c_int] * 6 + [c.c_void_p]
     lib.dflash_qmm_rows_workspace_bytes.restype = c.c_size_t
     lib.dflash_qmm_rows_workspace_bytes.argtypes = [c.c_int] * 7
     lib.dflash_qmm_rows.restype = c.c_int

@@ -149,25 +149,25 @@ PyObject* qmm_m16(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// qmm_packed(x, codes, scales, biases, K, N, group_size, workspaces): the same on images of pack_weights.
+// qmm_packed(x, codes, scales, biases, K, N, group_size, kernel, workspaces): the same on images of pack_weights.
 PyObject* qmm_packed(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 8) Py_RETURN_NONE;
+  if (n != 9) Py_RETURN_NONE;
   const Tensor *x = device_tensor(a[0]), *w = device_tensor(a[1]), *s = device_tensor(a[2]), *b = device_tensor(a[3]);
-  int K, N, group;
-  if (!x || !w || !s || !b || !integer(a[4], &K) || !integer(a[5], &N) || !integer(a[6], &group)) Py_RETURN_NONE;
+  int K, N, group, kernel;
+  if (!x || !w || !s || !b || !integer(a[4], &K) || !integer(a[5], &N) || !integer(a[6], &group) || !integer(a[7], &kernel)) Py_RETURN_NONE;
   const int act = half_code(x->scalar_type()), sb = half_code(s->scalar_type());
   if (act == kNoCode || sb == kNoCode || x->dim() < 1 || x->size(-1) != K || x->numel() != 16 * (int64_t)K ||
       !x->is_contiguous() || w->device() != x->device())
     Py_RETURN_NONE;
   void* stream = stream_of(*x);
   const size_t need = dflash_qmm_m16_workspace_bytes(K, N, group, DFLASH_QMM_MMA2BIG, 1, DFLASH_QMM_KERNEL_STREAM);
-  Tensor y, ws = kept_workspace(a[7], by_index(*x, stream), need);
+  Tensor y, ws = kept_workspace(a[8], by_index(*x, stream), need);
   if (!ws.defined()) Py_RETURN_NONE;
   const int rc = released([&] {
     y = at::empty(rows_by(*x, N), x->options());
-    return dflash_qmm_m16_packed(at_of(*x), at_of(*w), at_of(*s), at_of(*b), y.mutable_data_ptr(), ws.mutable_data_ptr(),
-                                 ws.nbytes(), K, N, group, act, sb, stream);
+    return dflash_qmm_m16_packed_by(at_of(*x), at_of(*w), at_of(*s), at_of(*b), y.mutable_data_ptr(), ws.mutable_data_ptr(),
+                                    ws.nbytes(), K, N, group, act, sb, kernel, stream);
   });
   return rc != 0 ? fail(rc, "dflash_qmm_m16_packed") : THPVariable_Wrap(std::move(y));
   END_HANDLE_TH_ERRORS

@@ -430,6 +430,10 @@ int qmm_stream_gather_launch(const void* x, const int32_t* expert_ids, const uin
                              size_t workspace_bytes, int P, int K, int N, int E, int act_dtype,
                              int sb_dtype, hipStream_t stream);
 bool qmm_stream_packed_eligible(int K, int N, int group_size);
+// qmm_narrow.hip: x and w 16-byte aligned, up to 16 rows
+bool qmm_narrow_covers(const void* scales, const void* biases, int K, int N, int group_size, bool silu_mul);
+int qmm_narrow_launch(const void* x, const void* w, const void* scales, const void* biases, void* y, int M, int K, int N, int group_size,
+                      int act_dtype, int sb_dtype, bool silu_mul, bool packed, hipStream_t stream);
 void qmm_stream_packed_bytes(int K, int N, size_t* w_bytes, size_t* sb_bytes);
 int qmm_stream_pack(const uint32_t* w, const void* scales, const void* biases, void* w_out,
                     void* s_out, void* b_out, int K, int N, hipStream_t stream);
@@ -495,6 +499,8 @@ extern "C" int dflash_qmm_few_silu_mul(const void* x, const uint32_t* w_q, const
                  "dflash_qmm_few_silu_mul: the streaming kernel does not cover K=%d N=%d gs=%d", K, N, group_size);
   DFLASH_REQUIRE((((uintptr_t)x | (uintptr_t)w_q) % 16) == 0 && (((uintptr_t)scales | (uintptr_t)biases) % 4) == 0,
                  DFLASH_ERR_ARG, "dflash_qmm_few_silu_mul: x and w_q must be 16-byte aligned, scales and biases 4-byte aligned");
+  if (qmm_narrow_covers(scales, biases, K, N, group_size, true))
+    return qmm_narrow_launch(x, w_q, scales, biases, y, M, K, N, group_size, dtype, dtype, true, false, (hipStream_t)stream);
   return qmm_stream_launch(x, w_q, scales, biases, y, workspace, workspace_bytes, M, K, N, group_size, dtype, dtype, true,
                            (hipStream_t)stream);
 }
@@ -524,6 +530,8 @@ int qmm_up_to_16(const void* x, const uint32_t* w_q, const void* scales, const v
                  "dflash_qmm_m16: K=%d is not a multiple of 32*k_parts (k_parts=%d)", K, k_parts);
   DFLASH_REQUIRE(((uintptr_t)x % 16) == 0 && ((uintptr_t)w_q % 16) == 0, DFLASH_ERR_ARG,
                  "dflash_qmm_m16: x and w_q must be 16-byte aligned");
+  if (kernel == DFLASH_QMM_KERNEL_AUTO && qmm_narrow_covers(scales, biases, K, N, group_size, false))
+    return qmm_narrow_launch(x, w_q, scales, biases, y, M, K, N, group_size, act_dtype, sb_dtype, false, false, (hipStream_t)stream);
   // (the C interface has always taken scales of 2-byte alignment; the ANYK loads need four)
   const bool any = kernel == DFLASH_QMM_KERNEL_AUTO && qmm_stream_any_eligible(K, N, group_size) &&
                    (((uintptr_t)scales | (uintptr_t)biases) % 4) == 0 && workspace != nullptr &&
@@ -645,7 +653,16 @@ extern "C" int dflash_qmm_m16_packed(const void* x, const void* codes, const voi
                                      const void* biases, void* y, void* workspace,
                                      size_t workspace_bytes, int K, int N, int group_size,
                                      int act_dtype, int sb_dtype, void* stream) {
+  return dflash_qmm_m16_packed_by(x, codes, scales, biases, y, workspace, workspace_bytes, K, N, group_size, act_dtype, sb_dtype,
+                                  DFLASH_QMM_KERNEL_STREAM, stream);
+}
+
+extern "C" int dflash_qmm_m16_packed_by(const void* x, const void* codes, const void* scales, const void* biases, void* y,
+                                        void* workspace, size_t workspace_bytes, int K, int N, int group_size, int act_dtype,
+                                        int sb_dtype, int kernel, void* stream) {
   using namespace dflash;
+  DFLASH_REQUIRE(kernel == DFLASH_QMM_KERNEL_AUTO || kernel == DFLASH_QMM_KERNEL_STREAM, DFLASH_ERR_ARG,
+                 "dflash_qmm_m16_packed: no packed form of kernel %d", kernel);
   DFLASH_REQUIRE(x && codes && scales && biases && y, DFLASH_ERR_ARG, "dflash_qmm_m16_packed: null operand");
   DFLASH_REQUIRE(act_dtype == DFLASH_BF16 || act_dtype == DFLASH_FP16, DFLASH_ERR_ARG,
                  "dflash_qmm_m16_packed: act_dtype %d is not bf16/fp16", act_dtype);
@@ -657,6 +674,8 @@ extern "C" int dflash_qmm_m16_packed(const void* x, const void* codes, const voi
   DFLASH_REQUIRE(((uintptr_t)x % 16) == 0 && ((uintptr_t)codes % 16) == 0 && ((uintptr_t)scales % 16) == 0 &&
                      ((uintptr_t)biases % 16) == 0,
                  DFLASH_ERR_ARG, "dflash_qmm_m16_packed: operands must be 16-byte aligned");
+  if (kernel == DFLASH_QMM_KERNEL_AUTO && qmm_narrow_covers(scales, biases, K, N, group_size, false))
+    return qmm_narrow_launch(x, codes, scales, biases, y, 16, K, N, group_size, act_dtype, sb_dtype, false, true, (hipStream_t)stream);
   return qmm_stream_packed_launch(x, codes, scales, biases, y, workspace, workspace_bytes, K, N,
                                   act_dtype, sb_dtype, (hipStream_t)stream);
 }

@@ -13,8 +13,8 @@ and shape dispatch, with the device work done by the gfx950 kernel behind
 * ``DFLASH_VERIFY_VARIANT`` in {auto, mma2big, mma2big_pipe} and
   ``DFLASH_VERIFY_QMM_KPARTS`` select the variant (:15-22, 292-297).
 * ``DFLASH_QMM_KERNEL`` in {auto, tile, stream} picks the device kernel (no counterpart
-  in the reference; auto uses the streaming kernel, whose every-K form takes all group sizes and K a multiple of 64,
-  wherever it applies).
+  in the reference; auto takes matrices of few weights through a kernel of their own, csrc/qmm_narrow.hip, and the rest through the
+  streaming kernel, whose every-K form takes all group sizes and K a multiple of 64, wherever it applies).
 * An eligible call needs device tensors and the built HIP library; there is no
   software fallback for it.
 """
@@ -440,14 +440,20 @@ def pack_weights(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor, *,
     return PackedWeights(codes, s_img, b_img, K, N, group_size, gate_up)
 
 
+def _packed_kernel() -> int:
+    """The kernel that packed weights go through: the tile kernel has no packed form."""
+    return _native.QMM_KERNEL_AUTO if _kernel_select() == _native.QMM_KERNEL_AUTO else _native.QMM_KERNEL_STREAM
+
+
 def verify_matmul_packed(x: torch.Tensor, packed: PackedWeights) -> torch.Tensor:
     """``verify_matmul`` on packed weights: 16 rows of bf16/fp16 device activations; the result is
-    bit for bit that of the streaming kernel on the triple the weights were packed from."""
+    bit for bit ``verify_matmul``'s on the triple the weights were packed from."""
     K, N = packed.K, packed.N
     if packed.gate_up:
         raise ValueError("verify_matmul_packed: these images are ordered for the silu-mul epilogue of a chain")
     if x.is_cuda:
-        y = _native.host().qmm_packed(x, packed.codes, packed.scales, packed.biases, K, N, packed.group_size, _WORKSPACES)
+        y = _native.host().qmm_packed(x, packed.codes, packed.scales, packed.biases, K, N, packed.group_size, _packed_kernel(),
+                                      _WORKSPACES)
         if y is not None:
             return y
     m = 1
@@ -464,10 +470,10 @@ def verify_matmul_packed(x: torch.Tensor, packed: PackedWeights) -> torch.Tensor
     if need is None:
         need = _WORKSPACE_BYTES[key] = int(lib.dflash_qmm_m16_workspace_bytes(*key))
     ws = _workspace(x2.device, stream, need)
-    rc = lib.dflash_qmm_m16_packed(x2.data_ptr(), packed.codes.data_ptr(), packed.scales.data_ptr(),
-                                   packed.biases.data_ptr(), y.data_ptr(), ws.data_ptr(), ws.numel(),
-                                   K, N, packed.group_size, _DTYPE_CODE[x2.dtype],
-                                   _DTYPE_CODE[packed.scales.dtype], stream)
+    rc = lib.dflash_qmm_m16_packed_by(x2.data_ptr(), packed.codes.data_ptr(), packed.scales.data_ptr(),
+                                      packed.biases.data_ptr(), y.data_ptr(), ws.data_ptr(), ws.numel(),
+                                      K, N, packed.group_size, _DTYPE_CODE[x2.dtype],
+                                      _DTYPE_CODE[packed.scales.dtype], _packed_kernel(), stream)
     _native.check(rc, "dflash_qmm_m16_packed")
     return y.reshape(*x.shape[:-1], N)
 

@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define DFLASH_ABI_VERSION 22
+#define DFLASH_ABI_VERSION 23
 
 enum {
   DFLASH_OK = 0,
@@ -253,7 +253,7 @@ int dflash_qmm_m16_chain(const dflash_qmm_problem* problems, int count, void* wo
  * Requirements: group_size 64, K % 1024 == 0, N % 16 == 0; all pointers 16-byte aligned; the
  * workspace of dflash_qmm_m16 (kernel = DFLASH_QMM_KERNEL_STREAM) with the same rules.
  * dflash_qmm_m16_packed returns bit for bit what dflash_qmm_m16 returns through the streaming
- * kernel for the unpacked operands.
+ * kernel for the unpacked operands, dflash_qmm_m16_packed_by what it returns for `kernel` (AUTO or STREAM).
  */
 int dflash_qmm_m16_packed_bytes(int K, int N, int group_size, size_t* codes_bytes,
                                 size_t* scales_bytes /* = biases bytes */);
@@ -265,6 +265,9 @@ int dflash_qmm_m16_pack(const uint32_t* w_q, const void* scales, const void* bia
 int dflash_qmm_m16_packed(const void* x, const void* codes, const void* scales, const void* biases,
                           void* y, void* workspace, size_t workspace_bytes, int K, int N,
                           int group_size, int act_dtype, int sb_dtype, void* stream);
+int dflash_qmm_m16_packed_by(const void* x, const void* codes, const void* scales, const void* biases,
+                             void* y, void* workspace, size_t workspace_bytes, int K, int N,
+                             int group_size, int act_dtype, int sb_dtype, int kernel, void* stream);
 
 /*
  * The product for any number of rows: y[M,N] = x[M,K] . round(s*q + b)^T, weights rounded to act_dtype
