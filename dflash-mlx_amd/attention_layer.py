@@ -177,18 +177,31 @@ def _project_on_device(self, q_proj_output: torch.Tensor, keys: torch.Tensor, va
     if type(cache) is not KVCache or type(q_norm) is not HeadRMSNorm or type(k_norm) is not HeadRMSNorm \
             or type(rope) is not RotaryEmbedding or not unhooked(q_norm, k_norm, rope):
         return None
+    held = () if cache.keys is None else (cache.keys, cache.values)
+    qw, kw = q_norm.weight, k_norm.weight
+    if held and q_proj_output.is_cuda and _native.plain(q_proj_output, keys, values, qw, kw, *held):
+        # room for the block: the ordinary case
+        prev = cache.offset
+        made = _native.host().attn_prepare(q_proj_output, keys, values, qw, kw, *held, _attention_num_heads(self),
+                                           _attention_num_kv_heads(self), rope.dims, prev)
+        if made is not None:
+            queries, all_keys, all_values, args, strides, codes = made
+            rc = _native.lib().dflash_attn_prepare(*args, (ctypes.c_longlong * 12)(*strides), q_norm.eps, k_norm.eps, float(rope.base),
+                                                   *codes, _native.raw_stream(q_proj_output.device))
+            _native.check(rc, "dflash_attn_prepare")
+            cache.offset = int(all_keys.shape[2])  # the rows are on their way: not before
+            return queries, all_keys, all_values, q_proj_output, prev
     code = _DTYPE_CODE.get(q_proj_output.dtype)
     if code is None or code == _native.FP32 or q_proj_output.ndim != 3:
         return None
     B, L, width = q_proj_output.shape
     Hq, Hk = _attention_num_heads(self), _attention_num_kv_heads(self)
     D = width // (2 * Hq)
-    qw, kw, device, dtype = q_norm.weight, k_norm.weight, q_proj_output.device, q_proj_output.dtype
+    device, dtype = q_proj_output.device, q_proj_output.dtype
     per = D // 64
     if (D not in (64, 128, 192, 256) or width != 2 * Hq * D or not 0 < rope.dims <= D or rope.dims % (2 * per)
             or keys.shape != (B, L, Hk * D) or keys.shape != values.shape or B * L == 0):
         return None
-    held = () if cache.keys is None else (cache.keys, cache.values)
     # the kernel writes rows offset .. offset + L - 1 of both buffers: an offset outside them, or buffers of two
     # lengths, are left to the array operators, which refuse them
     capacity = cache.keys.shape[2] if held and cache.keys.ndim == 4 else 0

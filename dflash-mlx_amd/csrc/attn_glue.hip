@@ -9,7 +9,8 @@
 // What bounds it is neither bandwidth (a block of 16 tokens is about 1 MB) nor arithmetic: as array operators the
 // same steps were 70 launches, 2 to 5 us each on the device and about 400 us of host time per layer call.
 // Measured, 16 tokens of 32 + 8 heads of 256: layer call over 4 112 or 32 716 keys
-// 498 -> 109 us (host time: the kernels are 62 and 102 us); this kernel 6.8 us, the gate 4 us (a verify block over a
+// 498 -> 109 us (host time: the kernels are 62 and 102 us); this kernel 5.8 us, 4.5 with the angles once per workgroup (300 tokens of
+// 16 + 2 heads 12.8 -> 7.8), the gate 4 us (a verify block over a
 // long cache has it in the merge of sdpa_q16.hip instead).
 #include "glue_device.h"
 
@@ -32,29 +33,48 @@ struct AttnPrepareArgs {
   float q_eps, k_eps, base, inv_half;
 };
 
+// A workgroup has one token: its angles, the same for every head, are computed once, one per thread, while the first rows are on
+// their way (before, each wave for itself: four powers, cosines and sines per lane of a head of 256, more than half of a wave's
+// instructions).
 template <int PER>
-__device__ __forceinline__ void attn_prepare_token(const AttnPrepareArgs& p, int b, int l, int first, int lane) {
+__global__ __launch_bounds__(kWavesPerGroup * 64) void attn_prepare_kernel(AttnPrepareArgs p) {
 #pragma clang fp contract(off)
   constexpr int D = 64 * PER;
-  const int c = PER * lane, rotated = p.Hq + p.Hk, heads = rotated + p.Hk;
+  __shared__ float2 turn[D / 2];  // cosine and sine
+  const int rotated = p.Hq + p.Hk, heads = rotated + p.Hk, groups = (p.waves + kWavesPerGroup - 1) / kWavesPerGroup;
+  const int token = (int)(blockIdx.x / (unsigned)groups), b = token / p.L, l = token - b * p.L;
+  const int first = (int)(blockIdx.x - (unsigned)token * (unsigned)groups) * kWavesPerGroup + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, c = PER * lane;
   const bool rotates = c < 2 * p.half, upper = c >= p.half;
   const int other = rotates ? (upper ? lane - p.half / PER : lane + p.half / PER) : lane;
+  uint32_t raw[PER], wraw[PER];
+  auto request = [&](int h) __attribute__((always_inline)) {
+    const int hk = h - p.Hq;
+    const bool is_q = h < p.Hq, is_v = h >= rotated;
+    const uint16_t* const src = is_q   ? p.q + b * p.q_batch + l * p.q_row + (size_t)h * (2 * D)
+                                : is_v ? p.v + b * p.v_batch + l * p.v_row + (size_t)(h - rotated) * D
+                                       : p.k + b * p.k_batch + l * p.k_row + (size_t)hk * D;
+    load_adjacent_raw<PER>(src, c, false, raw);
+    load_adjacent_raw<PER>(is_q ? p.q_weight : p.k_weight, c, (is_q ? p.q_weight_dt : p.k_weight_dt) == DFLASH_FP32, wraw);
+  };
+  const bool busy = first < p.waves && first < heads;
+  if (busy) request(first);
+  asm volatile("" ::: "memory");  // on their way before the angles
+  if ((int)threadIdx.x < p.half) {
+    const float angle = (float)(p.offset + l) * powf(p.base, -(float)(int)threadIdx.x * p.inv_half);
+    turn[threadIdx.x] = make_float2(cosf(angle), sinf(angle));
+  }
+  __syncthreads();
+  if (!busy) return;
   float cs[PER], sn[PER];
-  if (first < rotated) {  // the same for every head of the token
-    const float position = (float)(p.offset + l);
 #pragma unroll
-    for (int e = 0; e < PER; ++e) {
-      const int i = rotates ? (upper ? c - p.half : c) + e : 0;
-      const float angle = position * powf(p.base, -(float)i * p.inv_half);
-      cs[e] = cosf(angle), sn[e] = sinf(angle);
-    }
+  for (int e = 0; e < PER; ++e) {
+    const float2 t = turn[rotates ? (upper ? c - p.half : c) + e : 0];
+    cs[e] = t.x, sn[e] = t.y;
   }
   for (int h = first; h < heads; h += p.waves) {
-    uint32_t raw[PER];
     if (h >= rotated) {
-      const int hv = h - rotated;
-      load_adjacent_raw<PER>(p.v + b * p.v_batch + l * p.v_row, (size_t)hv * D + c, false, raw);
-      uint16_t* const dst = p.v_out + b * p.vo_batch + hv * p.vo_head + l * p.vo_row + c;
+      uint16_t* const dst = p.v_out + b * p.vo_batch + (h - rotated) * p.vo_head + l * p.vo_row + c;
       if constexpr (PER == 4) {
         *reinterpret_cast<uint2*>(dst) = make_uint2(raw[0], raw[1]);
       } else if constexpr (PER == 2) {
@@ -63,19 +83,15 @@ __device__ __forceinline__ void attn_prepare_token(const AttnPrepareArgs& p, int
 #pragma unroll
         for (int e = 0; e < PER; ++e) dst[e] = (uint16_t)raw[e];
       }
+      if (h + p.waves < heads) request(h + p.waves);
       continue;
     }
     const bool is_q = h < p.Hq;
     const int hk = h - p.Hq;
-    const uint16_t* const src = is_q ? p.q + b * p.q_batch + l * p.q_row + (size_t)h * (2 * D)
-                                     : p.k + b * p.k_batch + l * p.k_row + (size_t)hk * D;
-    uint32_t wraw[PER];
-    load_adjacent_raw<PER>(src, c, false, raw);
-    const int wdt = is_q ? p.q_weight_dt : p.k_weight_dt;
-    load_adjacent_raw<PER>(is_q ? p.q_weight : p.k_weight, c, wdt == DFLASH_FP32, wraw);
     float x[PER], w[PER], ss = 0.f;
     unpack_adjacent<PER>(raw, p.dt, x);
-    unpack_adjacent<PER>(wraw, wdt, w);
+    unpack_adjacent<PER>(wraw, is_q ? p.q_weight_dt : p.k_weight_dt, w);
+    if (h + p.waves < heads) request(h + p.waves);
 #pragma unroll
     for (int e = 0; e < PER; ++e) ss += x[e] * x[e];
     // (the array operators divide by a number by multiplying with its reciprocal: the mean here, the exponents above)
@@ -95,14 +111,6 @@ __device__ __forceinline__ void attn_prepare_token(const AttnPrepareArgs& p, int
       store_adjacent<PER>(p.k_out + b * p.ko_batch + hk * p.ko_head + l * p.ko_row, c, p.dt, x);
     }
   }
-}
-
-template <int PER>
-__global__ __launch_bounds__(kWavesPerGroup * 64) void attn_prepare_kernel(AttnPrepareArgs p) {
-  const long long w = (long long)blockIdx.x * kWavesPerGroup + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  if (w >= (long long)p.B * p.L * p.waves) return;
-  const long long token = w / p.waves;
-  attn_prepare_token<PER>(p, (int)(token / p.L), (int)(token % p.L), (int)(w % p.waves), threadIdx.x & 63);
 }
 
 struct AttnGateArgs {
@@ -172,13 +180,12 @@ extern "C" int dflash_attn_prepare(const void* q, const void* k, const void* v, 
   p.B = B; p.L = L; p.Hq = Hq; p.Hk = Hk; p.half = rope_dims / 2; p.offset = offset;
   p.dt = dtype; p.q_weight_dt = q_weight_dtype; p.k_weight_dt = k_weight_dtype;
   p.q_eps = q_eps; p.k_eps = k_eps; p.base = rope_base; p.inv_half = 1.0f / (float)p.half;
-  // A token's angles cost about as much as three of its heads: one wave per head while that leaves the chip
-  // with fewer than 8 waves per SIMD, beyond that several heads per wave.
+  // One wave per head while that leaves the chip with fewer than 8 waves per SIMD, beyond that several heads per wave.
   const long long tokens = (long long)B * L, want = (8192 + tokens - 1) / tokens;
   p.waves = want < Hq + 2 * Hk ? (int)want : Hq + 2 * Hk;
-  const long long waves = tokens * p.waves;
-  DFLASH_REQUIRE(waves < (1ll << 31), DFLASH_ERR_SHAPE, "dflash_attn_prepare: too many rows");
-  const dim3 grid((unsigned)((waves + kWavesPerGroup - 1) / kWavesPerGroup)), block(kWavesPerGroup * 64);
+  const long long groups = tokens * ((p.waves + kWavesPerGroup - 1) / kWavesPerGroup);
+  DFLASH_REQUIRE(groups * kWavesPerGroup < (1ll << 31), DFLASH_ERR_SHAPE, "dflash_attn_prepare: too many rows");
+  const dim3 grid((unsigned)groups), block(kWavesPerGroup * 64);
   switch (per) {
     case 1: hipLaunchKernelGGL(attn_prepare_kernel<1>, grid, block, 0, (hipStream_t)stream, p); break;
     case 2: hipLaunchKernelGGL(attn_prepare_kernel<2>, grid, block, 0, (hipStream_t)stream, p); break;

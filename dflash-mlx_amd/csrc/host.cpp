@@ -582,6 +582,50 @@ PyObject* rollback_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 // ---- attention --------------------------------------------------------------------------------------------------------
+// attn_prepare(q_proj_output, keys, values, q_weight, k_weight, cache_keys, cache_values, Hq, Hk, rope_dims, offset): what a
+// launch of dflash_attn_prepare into a cache with room for the block takes: (queries, the cache's keys and values up to the block's
+// end, the arguments from q to offset, the strides, the three dtype codes).  The caller launches.
+PyObject* attn_prepare(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 11) Py_RETURN_NONE;
+  const Tensor* t[7];
+  for (int i = 0; i < 7; ++i)
+    if (!(t[i] = device_tensor(a[i]))) Py_RETURN_NONE;
+  const Tensor &q = *t[0], &k = *t[1], &v = *t[2], &qw = *t[3], &kw = *t[4], &ck = *t[5], &cv = *t[6];
+  int Hq, Hk, rope, offset;
+  if (!integer(a[7], &Hq) || !integer(a[8], &Hk) || !integer(a[9], &rope) || !integer(a[10], &offset) || Hq < 1 || Hk < 1 ||
+      q.dim() != 3 || ck.dim() != 4 || cv.dim() != 4)
+    Py_RETURN_NONE;
+  const int64_t B = q.size(0), L = q.size(1), D = q.size(2) / (2 * (int64_t)Hq), per = D / 64, capacity = ck.size(2);
+  const int code = half_code(q.scalar_type()), q_code = dtype_code(qw.scalar_type()), k_code = dtype_code(kw.scalar_type());
+  if (code == kNoCode || q_code == kNoCode || k_code == kNoCode || (D != 64 && D != 128 && D != 192 && D != 256) ||
+      q.size(2) != 2 * (int64_t)Hq * D || rope < 1 || rope > D || rope % (2 * per) != 0 || B < 1 || L < 1 || B * L >= (1 << 30) ||
+      offset + L > capacity || !has_shape(k, {B, L, Hk * D}) || !has_shape(v, {B, L, Hk * D}) || !has_shape(qw, {D}) ||
+      !has_shape(kw, {D}) || !qw.is_contiguous() || !kw.is_contiguous() || !aligned(at_of(qw), 8) || !aligned(at_of(kw), 8) ||
+      !has_shape(ck, {B, Hk, capacity, D}) || !has_shape(cv, {B, Hk, capacity, D}))
+    Py_RETURN_NONE;
+  for (const Tensor* x : {&k, &v, &ck, &cv})
+    if (x->scalar_type() != q.scalar_type() || x->device() != q.device()) Py_RETURN_NONE;
+  if (qw.device() != q.device() || kw.device() != q.device()) Py_RETURN_NONE;
+  for (const Tensor* x : {&q, &k, &v})
+    if (x->stride(2) != 1 || (x->stride(0) | x->stride(1)) % 4 != 0 || !aligned(at_of(*x), 8)) Py_RETURN_NONE;
+  for (const Tensor* x : {&ck, &cv})
+    if (x->stride(3) != 1 || (x->stride(0) | x->stride(1) | x->stride(2)) % 4 != 0 || !aligned(at_of(*x), 8)) Py_RETURN_NONE;
+  Tensor queries = at::empty({B, Hq, L, D}, q.options());
+  const auto address = [](const void* p, int64_t elements) { return (unsigned long long)(uintptr_t)p + 2 * (unsigned long long)elements; };
+  PyObject* args = Py_BuildValue("(KKKKKKKKiiiiiii)", address(at_of(q), 0), address(at_of(k), 0), address(at_of(v), 0), address(at_of(qw), 0),
+                                 address(at_of(kw), 0), address(queries.mutable_data_ptr(), 0),
+                                 address(ck.mutable_data_ptr(), offset * ck.stride(2)), address(cv.mutable_data_ptr(), offset * cv.stride(2)),
+                                 (int)B, (int)L, Hq, Hk, (int)D, rope, offset);
+  PyObject* strides = Py_BuildValue("(LLLLLLLLLLLL)", (long long)q.stride(0), (long long)q.stride(1), (long long)k.stride(0),
+                                    (long long)k.stride(1), (long long)v.stride(0), (long long)v.stride(1), (long long)ck.stride(0),
+                                    (long long)ck.stride(1), (long long)ck.stride(2), (long long)cv.stride(0), (long long)cv.stride(1),
+                                    (long long)cv.stride(2));
+  return Py_BuildValue("(NNNNN(iii))", THPVariable_Wrap(std::move(queries)), THPVariable_Wrap(ck.narrow(2, 0, offset + L)),
+                       THPVariable_Wrap(cv.narrow(2, 0, offset + L)), args, strides, code, q_code, k_code);
+  END_HANDLE_TH_ERRORS
+}
+
 // sdpa_q16(queries, keys, values, scale, gate, workspaces): a block of 16 queries without a mask; gate None, or the output
 // of the projection that carries it.
 PyObject* sdpa_q16(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -640,7 +684,7 @@ PyObject* bind(PyObject*, PyObject* error) {  // the class that failed launches 
 #define DFLASH_HOST(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
 PyMethodDef kMethods[] = {DFLASH_HOST(qmm_m16), DFLASH_HOST(qmm_packed), DFLASH_HOST(qmm_few), DFLASH_HOST(qmm_few_silu_mul),
                           DFLASH_HOST(qmm_rows), DFLASH_HOST(columns), DFLASH_HOST(gather), DFLASH_HOST(chain_bind), DFLASH_HOST(chain_launch), DFLASH_HOST(gdn_prepare), DFLASH_HOST(gdn_forward), DFLASH_HOST(gdn_block),
-                          DFLASH_HOST(rollback_layer), DFLASH_HOST(sdpa_q16), {"bind", bind, METH_O, nullptr},
+                          DFLASH_HOST(rollback_layer), DFLASH_HOST(attn_prepare), DFLASH_HOST(sdpa_q16), {"bind", bind, METH_O, nullptr},
                           {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_dflash_host", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
 

@@ -250,7 +250,39 @@ def test_host_tensors_and_strangers_are_left_alone(native_lib):
     host, x = nat.host(), torch.zeros(16, 64)
     for name, count in (("qmm_m16", 7), ("qmm_packed", 9), ("qmm_few", 7), ("qmm_few_silu_mul", 6), ("qmm_rows", 7), ("columns", 2),
                         ("gather", 8), ("chain_bind", 4), ("chain_launch", 10), ("gdn_prepare", 13), ("gdn_forward", 10),
-                        ("rollback_layer", 9), ("sdpa_q16", 6)):
+                        ("rollback_layer", 9), ("sdpa_q16", 6), ("attn_prepare", 11)):
         for value in (x, x.to("meta"), None, 1, -1, 2 ** 70, 1.5, "x", {}):
             assert getattr(host, name)(*[value] * count) is None
         assert getattr(host, name)() is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,L,Hq,Hk,D,rope,prefix", [(1, 16, 8, 2, 256, 256, 300), (2, 1, 4, 4, 128, 64, 5), (1, 40, 6, 3, 64, 32, 0),
+                                                     (1, 16, 4, 2, 192, 192, 240)])
+def test_what_stands_before_the_attention(monkeypatch, B, L, Hq, Hk, D, rope, prefix):
+    from test_gpu_attn_glue import _layer
+
+    from dflash_mlx_amd import attention_layer as A
+    from dflash_mlx_amd.cache import KVCache
+
+    gen = torch.Generator("cuda").manual_seed(4)
+    attn, _ = _layer(B, L, Hq, Hk, D, rope, BF, BF, gen, True)
+    x = torch.empty((B, L, 8), device="cuda")
+    before = [torch.randn((B, Hk, prefix, D), generator=gen, device="cuda").to(BF) for _ in range(2)]
+
+    def projected(served, change=None):
+        cache = KVCache()
+        if prefix:
+            cache.update_and_fetch(*before)
+        if change == "types":
+            cache.keys, cache.values = cache.keys.to(HF), cache.values.to(HF)
+        elif change == "order":
+            cache.keys = cache.keys.transpose(2, 3).contiguous().transpose(2, 3)
+        q, k, v, gate, at = A._project(attn, x, cache)
+        return q, k.clone(), v.clone(), gate, torch.tensor([at, cache.offset])
+
+    room = 0 < prefix and prefix + L <= -(-prefix // 256) * 256
+    _same(monkeypatch, lambda: projected(room), "attn_prepare", room)
+    if prefix:
+        for change in ("types", "order"):
+            _same(monkeypatch, lambda: projected(False, change), "attn_prepare", False)
