@@ -1120,7 +1120,7 @@ int gdn_forward_launch(const char* who, const void* q, const void* k, const void
   const bool no_chunk = option(DFLASH_OPT_GDN_STEP_BY_STEP) != 0;  // (tests of one kernel against the other)
   const bool prompt = workspace != nullptr && aligned16 && !no_chunk && gdn_prompt_covers(slots, T, Hk, Hv, Dk, Dv, in_dtype, g_per_dk) &&
                       (((uintptr_t)state_in | (uintptr_t)state_out | (uintptr_t)workspace) % 16) == 0;
-  DFLASH_REQUIRE(q && k && v && g && beta && state_in && state_out && y && (tape || prompt), DFLASH_ERR_ARG, "%s: null operand", who);
+  DFLASH_REQUIRE(q && k && v && g && beta && state_out && y && ((state_in && tape) || prompt), DFLASH_ERR_ARG, "%s: null operand", who);
   DFLASH_REQUIRE(state_in != state_out, DFLASH_ERR_ARG, "%s: state_out must not alias state_in", who);
   auto ok = [](int dt) { return dt == DFLASH_BF16 || dt == DFLASH_FP16 || dt == DFLASH_FP32; };
   DFLASH_REQUIRE(ok(in_dtype) && ok(g_dtype) && ok(beta_dtype) && ok(state_dtype) && (!z || ok(weight_dtype)),

@@ -61,7 +61,7 @@ struct Args {
   const uint16_t* v;
   const void* g;
   const void* beta;
-  const void* state_in;
+  const void* state_in;  // null: zeros
   void* state_out;
   uint16_t* y;
   float* tape;  // may be null
@@ -298,7 +298,9 @@ void gdn_prompt_kernel(Args a) {
   for (int C = 0; C < NC; ++C)
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      if (a.state_dtype == DFLASH_FP32) {
+      if (a.state_in == nullptr) {
+        st[2 * C + h] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      } else if (a.state_dtype == DFLASH_FP32) {
         st[2 * C + h] = *reinterpret_cast<const f32x4_t*>((const float*)a.state_in + srow + 32 * C + 4 * h);
       } else {
         const uint2 w = *reinterpret_cast<const uint2*>((const uint16_t*)a.state_in + srow + 32 * C + 4 * h);

@@ -399,32 +399,35 @@ PyObject* gdn_prepare(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 // gdn_forward(q, k, v, g, beta, state, z, weight, eps, with_tape): without a mask, gates per head; z and weight None, or the
-// gate and the weight of the output norm.  (y, state, tape or None).
+// gate and the weight of the output norm.  state None: zeros of q's type, for prompts that a kernel starts with them.
+// (y, state, tape or None).
 PyObject* gdn_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (n != 10) Py_RETURN_NONE;
   const Tensor *q = device_tensor(a[0]), *k = device_tensor(a[1]), *v = device_tensor(a[2]), *g = device_tensor(a[3]),
-               *beta = device_tensor(a[4]), *state = device_tensor(a[5]), *z = nullptr, *w = nullptr;
-  if (!q || !k || !v || !g || !beta || !state || k->dim() != 4 || v->dim() != 4 || !PyFloat_CheckExact(a[8])) Py_RETURN_NONE;
+               *beta = device_tensor(a[4]), *state = nullptr, *z = nullptr, *w = nullptr;
+  if (a[5] != Py_None && !(state = device_tensor(a[5]))) Py_RETURN_NONE;
+  if (!q || !k || !v || !g || !beta || k->dim() != 4 || v->dim() != 4 || !PyFloat_CheckExact(a[8])) Py_RETURN_NONE;
   if (a[6] != Py_None && (!(z = device_tensor(a[6])) || !(w = device_tensor(a[7])))) Py_RETURN_NONE;
   const int64_t B = k->size(0), T = k->size(1), hk = k->size(2), dk = k->size(3), hv = v->size(2), dv = v->size(3);
   const int code = dtype_code(q->scalar_type()), g_code = dtype_code(g->scalar_type()), b_code = dtype_code(beta->scalar_type()),
-            s_code = dtype_code(state->scalar_type());
+            s_code = state ? dtype_code(state->scalar_type()) : code;
   if (B < 1 || T < 1 || hk < 1 || hv < 1 || dv < 1 || hv % hk != 0 || dk < 32 || dk % 32 != 0 || B * T * hv >= (1 << 30) ||
       code == kNoCode || g_code == kNoCode || b_code == kNoCode || s_code == kNoCode || k->scalar_type() != q->scalar_type() ||
       v->scalar_type() != q->scalar_type())
     Py_RETURN_NONE;
   if (!has_shape(*q, {B, T, hk, dk}) || !has_shape(*v, {B, T, hv, dv}) || !has_shape(*g, {B, T, hv}) ||
-      !has_shape(*beta, {B, T, hv}) || !has_shape(*state, {B, hv, dv, dk}))
+      !has_shape(*beta, {B, T, hv}))
     Py_RETURN_NONE;
-  for (const Tensor* t : {q, k, v, g, beta, state})
-    if (!t->is_contiguous() || t->device() != state->device()) Py_RETURN_NONE;
+  if (state && (!has_shape(*state, {B, hv, dv, dk}) || !state->is_contiguous() || state->device() != q->device())) Py_RETURN_NONE;
+  for (const Tensor* t : {q, k, v, g, beta})
+    if (!t->is_contiguous() || t->device() != q->device()) Py_RETURN_NONE;
   int w_code = code;
   if (z != nullptr) {
     w_code = dtype_code(w->scalar_type());
     const int64_t step = z->element_size();
     if (w_code == kNoCode || z->scalar_type() != q->scalar_type() || !has_shape(*z, {B, T, hv, dv}) ||
-        z->device() != state->device() || w->device() != state->device() || w->numel() != dv || !w->is_contiguous() ||
+        z->device() != q->device() || w->device() != q->device() || w->numel() != dv || !w->is_contiguous() ||
         dv % 64 != 0 || dv > 256)
       Py_RETURN_NONE;
     if (z->stride(3) != 1 || z->stride(2) != dv || z->stride(1) == 0 || !aligned(at_of(*z), 16) ||
@@ -433,7 +436,8 @@ PyObject* gdn_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   }
   size_t need = T > 16 ? dflash_gdn_forward_workspace_bytes((int)B, (int)T, (int)hk, (int)hv, (int)dk, (int)dv, code, 0) : 0;
   for (const Tensor* t : {q, k, v, state})
-    if (!aligned(at_of(*t), 16)) need = 0;
+    if (t != nullptr && !aligned(at_of(*t), 16)) need = 0;
+  if (state == nullptr && (need == 0 || dflash_get_option(DFLASH_OPT_GDN_STEP_BY_STEP) != 0)) Py_RETURN_NONE;
   const bool with_tape = a[9] == Py_True || need == 0 || dflash_get_option(DFLASH_OPT_GDN_STEP_BY_STEP) != 0;
   void* stream = stream_of(*q);
   const float eps = (float)PyFloat_AS_DOUBLE(a[8]);
@@ -443,8 +447,8 @@ PyObject* gdn_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
     y = at::empty({B, T, hv, dv}, options);
     if (need != 0) ws = at::empty({(int64_t)need}, options.dtype(at::kByte));
     if (with_tape) tape = at::empty({B, T, hv, dv}, options.dtype(at::kFloat));
-    next = at::empty({B, hv, dv, dk}, state->options());
-    return dflash_gdn_forward(at_of(*q), at_of(*k), at_of(*v), at_of(*g), at_of(*beta), at_of(*state), next.mutable_data_ptr(),
+    next = at::empty({B, hv, dv, dk}, state ? state->options() : options);
+    return dflash_gdn_forward(at_of(*q), at_of(*k), at_of(*v), at_of(*g), at_of(*beta), state ? at_of(*state) : nullptr, next.mutable_data_ptr(),
                               z ? at_of(*z) : nullptr, z ? at_of(*w) : nullptr, y.mutable_data_ptr(),
                               with_tape ? (float*)tape.mutable_data_ptr() : nullptr, nullptr,
                               need ? ws.mutable_data_ptr() : nullptr, need, z ? z->stride(0) : 0, z ? z->stride(1) : 0, (int)B,

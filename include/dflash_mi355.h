@@ -395,7 +395,7 @@ int dflash_gdn_forward_tape_norm(const void* q, const void* k, const void* v, co
  * dflash_gdn_forward_workspace_bytes() bytes (16-byte aligned, contents irrelevant; 0 where none is used)
  * prompts - T > 16, bf16 q / k / v, one gate per head, Dk 64 or 128, Dv a multiple of 16 - go through the
  * matrix cores in chunks of 32 tokens.  There a 16-bit state is carried in fp32 and rounded once, behind
- * the last token, and tape may be NULL (not recorded).  z_row_stride, z_batch_stride: elements from a step's z to the
+ * the last token, tape may be NULL (not recorded) and state_in as well (zeros).  z_row_stride, z_batch_stride: elements from a step's z to the
  * next one's and from slot to slot (heads and columns contiguous, rows at least 8-byte aligned); 0: z [slots, T, Hv, Dv].
  */
 size_t dflash_gdn_forward_workspace_bytes(int slots, int T, int Hk, int Hv, int Dk, int Dv, int in_dtype, int g_per_dk);

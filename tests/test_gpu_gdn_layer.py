@@ -335,3 +335,23 @@ def test_a_block_in_one_launch(monkeypatch, state_dtype, B, S, Hk, Hv, D, joint)
     shifted = torch.zeros(state.numel() + 1, dtype=state.dtype, device="cuda")
     shifted[1:] = state.reshape(-1)
     same([False], window, shifted[1:].view(state.shape), True)
+
+
+@pytest.mark.parametrize("T,D,times", [(17, 128, 1), (40, 64, 1), (33, 128, 40)])
+@pytest.mark.parametrize("normed", [True, False])
+def test_a_prompt_that_starts_from_nothing(native_lib, T, D, times, normed):
+    """No state is the state of zeros, bit for bit; what cannot start without one is left to the caller."""
+    import dflash_mlx_amd._native as nat
+
+    gen = torch.Generator("cuda").manual_seed(T)
+    B, Hk, Hv = times, 1, 2
+    q, k, v = (torch.randn((B, T, h, D), generator=gen, device=DEV).to(torch.bfloat16) * D ** -0.5 for h in (Hk, Hk, Hv))
+    g, beta = torch.rand((B, T, Hv), generator=gen, device=DEV), torch.rand((B, T, Hv), generator=gen, device=DEV).to(torch.bfloat16)
+    z, weight = torch.randn((B, T, Hv, D), generator=gen, device=DEV).to(torch.bfloat16), torch.ones(D, device=DEV, dtype=torch.bfloat16)
+    norm = (z, weight, 1e-6) if normed else (None, None, 0.0)
+    run = lambda state, *cut: nat.host().gdn_forward(*(t[:, :cut[0]].contiguous() if cut else t for t in (q, k, v, g, beta)), state,  # noqa: E731
+                                                     *(norm if not cut else (None, None, 0.0)), True)
+    zeros = torch.zeros((B, Hv, D, D), dtype=torch.bfloat16, device=DEV)
+    for a, b in zip(run(None), run(zeros)):
+        assert a.dtype == b.dtype and torch.equal(a, b)
+    assert run(None, 16) is None and run(zeros, 16) is not None
