@@ -3,7 +3,7 @@
 // y[M,N] = x[M,K] . (s*q + b)^T for M <= 16, group_size 64, K % 512 == 0, N % 16 == 0 - the
 // shapes of the projections in the dense verify stacks; other group sizes and K that is a multiple of
 // 64 only through variants with a little more bookkeeping (ANYK) - and its gathered form for MoE
-// layers, y[p] = x[p] . (s*q + b)^T of expert ids[p] for up to 256 rows: rows that share an
+// layers, y[p] = x[p] . (s*q + b)^T of expert ids[p] for up to 2048 rows: rows that share an
 // expert are taken 16 at a time as the M dimension, and the weights of the experts that
 // have rows are streamed like one tall matrix.  Same arithmetic as
 // qmm_m16.hip (MFMA 16x16x32 on raw codes, scale/bias applied per (column, group) to
@@ -80,6 +80,7 @@ struct Params {
   // w, scales, biases hold E matrices of [N, .] back to back
   const int32_t* expert_ids;
   int P, E;
+  Tables tab;
   // dense forms, K % 1024 == 0: w, scales, biases hold the images qmm_pack_kernel writes - per
   // (row block, unit) the 16 KiB of codes in the order of the LDS slot, per (row block, chunk)
   // 4 KiB of scales and of biases - so that every load instruction of a wave moves 1 KiB of
@@ -151,7 +152,10 @@ __device__ unsigned long long g_sstamps[64][256][16];
 // 12288 x 4096 43.2 -> 12 us; the bookkeeping costs the group-64 shapes of the first two variants nothing.
 // GATHER: per-expert form.  Rows of x that share an expert are taken 16 at a time as one
 // "entry"; an entry is a matrix problem of its own, [rows, K] x [N, K]^T, and the unit
-// space is that of all entries back to back: virtual row block = entry * RB + row block.
+// space is that of all entries back to back: virtual row block = entry * RB + row block.  An expert with many rows has its
+// weights read once per entry, from the caches after the first: up to 2048 rows that is still the better way by far than
+// a workgroup per (32 columns, expert) that walks its rows alone (us, 64 experts of 2048 x 2048, 512 / 2048 rows 124 / 300 -> 34 / 84;
+// 8 of 3072 x 2048 87 / 344 -> 25 / 87; 256 of 1024 x 2048 179 / 283 -> 57 / 68; 32 of 768 x 1536, 320 rows 15.7 -> 11.6).
 // SILU_MUL (dense form, weights in row order): W holds the gate rows of an MLP and, behind them, its up rows, and
 // y[M, N / 2] is silu(gate) * up.  The rows of a tile of 16 are 8 gate rows and the up rows of the same columns, so that
 // lane col + 8 of a finished tile holds what lane col multiplies with: nothing else changes, and the activation
@@ -207,18 +211,24 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_stream_kernel(Params p) {
   int units = p.units;
   if (GATHER) {
     // ---- entry tables (ordinary code: no direct-to-LDS load has been issued yet) ----------
-    uint32_t* t_count = reinterpret_cast<uint32_t*>(lds + kTabOffset + kTabCount);
-    uint32_t* t_entry = reinterpret_cast<uint32_t*>(lds + kTabOffset + kTabEntry);
-    uint16_t* t_rows = reinterpret_cast<uint16_t*>(lds + kTabOffset + kTabRows);
-    uint32_t* t_total = reinterpret_cast<uint32_t*>(lds + kTabOffset + kTabTotal);
+    uint32_t* t_count = reinterpret_cast<uint32_t*>(lds + kTabOffset);
+    uint32_t* t_entry = reinterpret_cast<uint32_t*>(lds + kTabOffset + p.tab.entry);
+    uint16_t* t_rows = reinterpret_cast<uint16_t*>(lds + kTabOffset + p.tab.rows);
+    uint32_t* t_total = reinterpret_cast<uint32_t*>(lds + kTabOffset + p.tab.total);
+    // a thread's rows: tid, tid + kThreads, ..
+    constexpr int kRounds = (kMaxGatherRows + kThreads - 1) / kThreads, kAllWaves = kThreads / 64;
     // Every workgroup builds the same tables: a row's place among the rows of its expert is
     // its rank by row index, not the order in which threads happen to get there (partial
     // tiles of one row block come from several workgroups and must agree on the rows).
     for (int e = tid; e < p.E; e += kThreads) t_count[e] = 0;
-    int my_e = -1;
-    if (tid < p.P) {
-      const int e = p.expert_ids[tid];
-      if (e >= 0 && e < p.E) my_e = e;
+    int my_e[kRounds];
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+      my_e[r] = -1;
+      if (r * kThreads < p.P && r * kThreads + tid < p.P) {
+        const int e = p.expert_ids[r * kThreads + tid];
+        if (e >= 0 && e < p.E) my_e[r] = e;
+      }
     }
     __syncthreads();
     // Rank among the rows of the same expert: inside a wave by a match of the ids, a ballot per bit; the waves
@@ -226,24 +236,29 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_stream_kernel(Params p) {
     // the earlier equal ids one by one and scanning through LDS permutes were 2 us of a launch: 128 rows on 103 of 256 experts of
     // 512 x 32, where little else happens, 9.4 -> 7.1 us; 2048 x 1024 33.8 -> 32.9, 512 x 2048 24.1 -> 21.7 us; 256 rows on 62 of 64
     // experts 26.4 -> 23.1 and 20.4 -> 16.6 us.)
-    int my_pos = 0, same_expert = 0;
-    if (wave * 64 < p.P) {
-      unsigned long long same = __builtin_amdgcn_ballot_w64(my_e >= 0);
+    int my_pos[kRounds] = {}, same_expert[kRounds] = {};
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+      if (r * kThreads + wave * 64 >= p.P) continue;
+      unsigned long long same = __builtin_amdgcn_ballot_w64(my_e[r] >= 0);
       for (int bit = 0; (1 << bit) < p.E; ++bit) {
-        const bool one = (my_e >> bit) & 1;
+        const bool one = (my_e[r] >> bit) & 1;
         const unsigned long long ones = __builtin_amdgcn_ballot_w64(one);
         same &= one ? ones : ~ones;
       }
-      my_pos = __builtin_popcountll(same & ((1ull << lane) - 1ull));
-      same_expert = __builtin_popcountll(same);
+      my_pos[r] = __builtin_popcountll(same & ((1ull << lane) - 1ull));
+      same_expert[r] = __builtin_popcountll(same);
     }
-    for (int w = 0; w * 64 < p.P; ++w) {
-      if (wave == w && my_e >= 0) {
-        const uint32_t before = t_count[my_e];  // (read by all lanes of the wave before the first of each expert adds)
-        if (my_pos == 0) t_count[my_e] = before + (uint32_t)same_expert;
-        my_pos += (int)before;
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+      for (int w = 0; w < kAllWaves && (r * kAllWaves + w) * 64 < p.P; ++w) {
+        if (wave == w && my_e[r] >= 0) {
+          const uint32_t before = t_count[my_e[r]];  // (read by all lanes of the wave before the first of each expert adds)
+          if (my_pos[r] == 0) t_count[my_e[r]] = before + (uint32_t)same_expert[r];
+          my_pos[r] += (int)before;
+        }
+        __syncthreads();
       }
-      __syncthreads();
     }
     if (wave == 0) {
       // exclusive scan of ceil(rows / 16) over the experts: first entry of each expert
@@ -265,22 +280,29 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_stream_kernel(Params p) {
       if (lane == 0) *t_total = (uint32_t)carry;
     }
     __syncthreads();
-    if (my_e >= 0) {
-      const uint32_t c = t_count[my_e];
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+      if (r * kThreads >= p.P || my_e[r] < 0) continue;
+      const uint32_t c = t_count[my_e[r]];
       const int rows = (int)(c >> 16), first = (int)(c & 0xFFFFu);
-      const int ent = first + (my_pos >> 4), m = my_pos & 15;
-      t_rows[ent * 16 + m] = (uint16_t)tid;
+      const int ent = first + (my_pos[r] >> 4), m = my_pos[r] & 15;
+      t_rows[ent * 16 + m] = (uint16_t)(r * kThreads + tid);
       if (m == 0) {
-        const int left_rows = rows - (my_pos & ~15);
-        t_entry[ent] = ((uint32_t)(left_rows < 16 ? left_rows : 16) << 16) | (uint32_t)my_e;
+        const int left_rows = rows - (my_pos[r] & ~15);
+        t_entry[ent] = ((uint32_t)(left_rows < 16 ? left_rows : 16) << 16) | (uint32_t)my_e[r];
       }
     }
     __syncthreads();
     units = (int)*t_total * RB * p.stages;
     // A row whose expert id is outside [0, E) belongs to no entry: its output is zero (written
     // here, by the first workgroup, so that no row of y is left as it was found).
-    if (blockIdx.x == 0 && tid < p.P && my_e < 0) {
-      for (int n = 0; n < p.N; ++n) p.y[(size_t)tid * p.N + n] = 0;
+    if (blockIdx.x == 0) {
+#pragma unroll
+      for (int r = 0; r < kRounds; ++r) {
+        const int row = r * kThreads + tid;
+        if (r * kThreads >= p.P || row >= p.P || my_e[r] >= 0) continue;
+        for (int n = 0; n < p.N; ++n) p.y[(size_t)row * p.N + n] = 0;
+      }
     }
   }
 
@@ -309,7 +331,7 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_stream_kernel(Params p) {
     if (GATHER) {
       wh.entry = vrb / RB;
       wh.rb = vrb - wh.entry * RB;
-      const uint32_t e = lds_read_u32(lds0 + kTabOffset + kTabEntry + 4 * wh.entry);
+      const uint32_t e = lds_read_u32(lds0 + kTabOffset + p.tab.entry + 4 * wh.entry);
       wh.expert = (int)(e & 0xFFFFu);
       wh.rows = (int)(e >> 16);
     } else {
@@ -379,7 +401,7 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_stream_kernel(Params p) {
       // rows of x: the entry's rows in the order of its table; surplus rows of the MFMA tile
       // repeat the entry's first row (their results are never stored)
       int xrow = (lane & 15) < wh.rows ? lane & 15 : 0;
-      if (GATHER) xrow = (int)lds_read_u16(lds0 + kTabOffset + kTabRows + 2 * (wh.entry * 16 + xrow));
+      if (GATHER) xrow = (int)lds_read_u16(lds0 + kTabOffset + p.tab.rows + 2 * (wh.entry * 16 + xrow));
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
         const int xi = ld + 4 * i;
@@ -492,7 +514,7 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_stream_kernel(Params p) {
     }
     // x: instruction `wave` of the loaders' scheme; codes: instructions 2 wave and 2 wave + 1
     int xrow = (lane & 15) < wh.rows ? lane & 15 : 0;
-    if (GATHER) xrow = (int)lds_read_u16(lds0 + kTabOffset + kTabRows + 2 * (wh.entry * 16 + xrow));
+    if (GATHER) xrow = (int)lds_read_u16(lds0 + kTabOffset + p.tab.rows + 2 * (wh.entry * 16 + xrow));
     const bool x_in = !ANYK || st0 * kUnitK + (wave >> 1) * 64 < p.K;
     const char* xsrc = (const char*)(p.x + (size_t)xrow * p.K + (x_in ? (wave >> 1) * 64 + st0 * kUnitK : 0) +
                                      (2 * (wave & 1) + (lane >> 5)) * 16 + ((lane >> 4) & 1) * 8);
@@ -583,7 +605,7 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_stream_kernel(Params p) {
     const int n_out = wh.rb * kRows + 16 * wave + col;
     if (n_out >= p.N) return;
     if (GATHER) {
-      const u32x2_t rr = lds_read_u64(lds0 + kTabOffset + kTabRows + 2 * (wh.entry * 16 + 4 * kblk));
+      const u32x2_t rr = lds_read_u64(lds0 + kTabOffset + p.tab.rows + 2 * (wh.entry * 16 + 4 * kblk));
       const uint32_t rows4[4] = {rr.x & 0xFFFFu, rr.x >> 16, rr.y & 0xFFFFu, rr.y >> 16};
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
@@ -830,10 +852,11 @@ bool qmm_stream_any_eligible(int K, int N, int group_size) {
 bool qmm_stream_gather_eligible(int P, int K, int N, int E, int group_size) {
   if (group_size != 64 || !(qmm_stream_eligible(K, N, group_size) || qmm_stream_any_eligible(K, N, group_size))) return false;
   const long long row_blocks = (N + stream::kRows - 1) / stream::kRows;
-  // every row could be an entry of its own
-  return P > 0 && P <= stream::kMaxEntries && E > 0 && E <= stream::kMaxExperts &&
-         row_blocks * stream::kMaxEntries <= (64 * 1024) / 4 &&
-         row_blocks * stream::kMaxEntries * ((K + stream::kUnitK - 1) / stream::kUnitK) * 1024 < (1ll << 31);
+  if (P <= 0 || P > stream::kMaxGatherRows || E <= 0 || E > stream::kMaxExperts) return false;
+  // (up to 256 rows every one could be an entry of its own; what decides below is then the matrix alone)
+  const long long most = P <= 256 ? 256 : stream::most_entries(P, E);
+  return row_blocks * most <= (64 * 1024) / 4 && row_blocks * most * ((K + stream::kUnitK - 1) / stream::kUnitK) * 1024 < (1ll << 31) &&
+         stream::kTabOffset + stream::Tables(E, (int)most).bytes <= 160 * 1024;
 }
 
 size_t qmm_stream_workspace_bytes(int N, int grid) {
@@ -877,13 +900,13 @@ int launch_stream(stream::Params& p, Form form, int grid, int group_size, int ac
   if (p.spin_limit <= 0) p.spin_limit = option(DFLASH_OPT_QMM_SPIN_LIMIT) > 0 ? option(DFLASH_OPT_QMM_SPIN_LIMIT) : kSpinLimit;
   const void* fn = a16 ? (s16 ? stream_kernel_for<true, true>(variant, form) : stream_kernel_for<true, false>(variant, form))
                        : (s16 ? stream_kernel_for<false, true>(variant, form) : stream_kernel_for<false, false>(variant, form));
-  const int lds_bytes = form == Form::kGather ? kLdsBytesGather : kLdsBytes;
+  const int lds_bytes = form == Form::kGather ? kTabOffset + p.tab.bytes : kLdsBytes;
   // the attribute belongs to the device's copy of the kernel: once per device and kernel
   static bool attr_set[kMaxDevices][kVariants * 12] = {};
   const int idx = variant * 12 + (int)form * 4 + (a16 ? 2 : 0) + (s16 ? 1 : 0);
   const int slot = current_device_slot();
   if (!attr_set[slot][idx] || slot == kMaxDevices - 1) {
-    DFLASH_HIP_OK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes));
+    DFLASH_HIP_OK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, form == Form::kGather ? 160 * 1024 : lds_bytes));
     attr_set[slot][idx] = true;
   }
 #ifdef DFLASH_STREAM_STAMPS
@@ -1016,6 +1039,7 @@ int qmm_stream_gather_launch(const void* x, const int32_t* expert_ids, const uin
   p.expert_ids = expert_ids;
   p.P = P;
   p.E = E;
+  p.tab = Tables(E, most_entries(P, E));
   // the number of entries is not known here: a full grid, workgroups without units leave
   const int grid = qmm_stream_grid();
   const size_t need = qmm_stream_workspace_bytes(N, grid);

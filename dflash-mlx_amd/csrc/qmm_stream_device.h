@@ -44,14 +44,23 @@ constexpr int kLdsBytes = kSbOffset + kSbDepth * kSbSlotBytes;  // 144 KiB
 constexpr int kPartialFloats = 16 * kRows;
 // Gathered (per-expert) form: tables built in LDS by every workgroup at kernel start.
 //   an "entry" is up to 16 rows of x that go through the same expert's weights
-constexpr int kMaxEntries = 256;  // hence at most 256 rows of x
 constexpr int kMaxExperts = 1024;
+constexpr int kMaxGatherRows = 2048;
 constexpr int kTabOffset = kLdsBytes;
-constexpr int kTabCount = 0;                        // u32 [kMaxExperts]: rows << 16 | first entry
-constexpr int kTabEntry = kTabCount + 4 * kMaxExperts;   // u32 [kMaxEntries]: rows << 16 | expert
-constexpr int kTabRows = kTabEntry + 4 * kMaxEntries;    // u16 [kMaxEntries][16]: row of x, y
-constexpr int kTabTotal = kTabRows + 2 * 16 * kMaxEntries;  // u32: number of entries
-constexpr int kLdsBytesGather = kTabOffset + kTabTotal + 64;  // 157.1 KiB
+struct Tables {  // byte offsets behind kTabOffset, for E experts and up to n entries
+  int entry;     // behind u32 [E]: rows << 16 | first entry.  u32 [n]: rows << 16 | expert
+  int rows;      // u16 [n][16]: row of x, y
+  int total;     // u32: number of entries
+  int bytes;
+  Tables() = default;
+  __host__ __device__ Tables(int E, int n)
+      : entry(4 * E), rows((entry + 4 * n + 15) & ~15), total(rows + 32 * n), bytes(total + 64) {}
+};
+// Most entries that P rows on E experts can make: an expert's rows are cut into sixteens, the last of which may hold one.
+constexpr int most_entries(int P, int E) {
+  const int busy = P < E ? P : E, n = (P + 15 * busy) / 16;
+  return n < P ? n : P;
+}
 
 template <bool FP16>
 struct Act;

@@ -300,7 +300,8 @@ int dflash_qmm_rows(const void* x, const uint32_t* w_q, const void* scales, cons
  *   workspace               optional (may be NULL): >= dflash_qmm_m16_gather_workspace_bytes(...)
  *                           bytes, same rules as the workspace of dflash_qmm_m16 (zero-filled
  *                           once, reusable, shareable with it).  With a workspace, calls with
- *                           group_size 64, K % 512 == 0, P <= 256 and E <= 1024 are served by
+ *                           group_size 64, E <= 1024 and not too many rows and experts together
+ *                           (2048 rows: 280 experts; the size is 0 for others) are served by
  *                           the streaming kernel: the weights of the experts that have rows
  *                           are streamed through LDS by persistent workgroups, as for the
  *                           dense form.  Without one, or for other shapes, one workgroup per

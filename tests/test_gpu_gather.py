@@ -171,3 +171,26 @@ def test_argument_checks(native_lib):
     with pytest.raises(nat.NativeLibraryError):
         c = make_moe_case(64, 32, 1, experts=2, tokens=2, top_k=1)
         gather_qmm(c.x, c.w, c.scales, c.biases, c.expert_ids)
+
+
+@pytest.mark.parametrize("P,E,K,N", [(257, 8, 512, 96), (768, 256, 512, 32), (769, 64, 1024, 144), (1536, 1, 512, 128), (1537, 5, 1536, 160),
+                                     (2048, 3, 640, 272), (2048, 256, 512, 16), (2048, 1000, 512, 16)])
+def test_more_rows_than_a_workgroup_has_threads(native_lib, P, E, K, N):
+    """Up to 2048 rows in one launch of the streaming kernel: rows of a thread's second and third round, experts with many entries and
+    with none, ids that belong to no expert, tables that just fit (and, the last case, that do not: the other kernel)."""
+    from dflash_mlx_amd.quantized import dequantize
+    from test_gpu_qmm_any_k import _check
+
+    gen = torch.Generator("cuda").manual_seed(P + E)
+    w = torch.randint(-2 ** 31, 2 ** 31, (E, N, K // 8), generator=gen, device="cuda", dtype=torch.int32)
+    s = (torch.rand((E, N, K // 64), generator=gen, device="cuda") * 0.02 + 1e-4).to(torch.bfloat16)
+    b = (s.float() * -8).to(torch.bfloat16)
+    x = torch.randn((P, K), generator=gen, device="cuda").to(torch.bfloat16)
+    ids = torch.randint(-1, E + 1, (P,), generator=gen, device="cuda", dtype=torch.int32)
+    y = gather_qmm(x, w, s, b, ids)
+    assert torch.equal(y, gather_qmm(x, w, s, b, ids))
+    assert (y[(ids < 0) | (ids >= E)] == 0).all()
+    for e in range(0, E, max(1, E // 40)):
+        mine = ids == e
+        if mine.any():
+            _check(y[mine], x[mine], dequantize(w[e], s[e], b[e], 64, 4, torch.float64), K, torch.bfloat16)
