@@ -8,15 +8,14 @@
 //
 // The operation moves 2*Dv*Dk*4 bytes of state per head and almost nothing
 // else, so it is laid out for HBM streaming:
-//  * one workgroup per (slot, value head); the whole 64 KiB tile of a 128x128
-//    head is in flight at once, in and out in full 128-byte lines;
+//  * a workgroup has a head, or 32 or 64 rows of one; all of its part of the state
+//    is in flight at once, in and out in full 128-byte lines;
 //  * the tape (k, delta, g of <= T steps) is staged once into LDS as fp32;
 //  * for an fp32 state the T sequential sweeps are folded into a single one,
 //      S_a = (prod g) S0 + sum_t delta_t (x) (c_t k_t),  c_t = prod_{u>t} g_u
-//    (c_t folded into the staged k rows, per-Dk gates included).  For 128x128
-//    that is a rank-16 update which runs on the fp32 matrix cores; as scalar
-//    FMAs it costs more time than the memory traffic of the head.  bf16/fp16
-//    states, which the reference rounds after every step (kernels.py:281-283),
+//    (c_t folded into the staged k rows, per-Dk gates included), in registers
+//    (replay_rows) or, 128x128 heads with per-Dk gates, as a rank-16 update on the
+//    fp32 matrix cores (replay_f32_128).  bf16/fp16 states, which the reference rounds after every step (kernels.py:281-283),
 //    and callers that ask for it keep the step-by-step order (replay_rows, replay_generic);
 //  * the accepted length is read per slot from device memory, so a rollback
 //    does not need the host to know it, and one launch covers all layers.
@@ -135,18 +134,14 @@ __device__ __forceinline__ bool conv_window_workgroup(const ReplayArgs& a) {
 }
 
 // ---------------------------------------------------------------------------
-// fp32 state, Dk = Dv = 128, T <= 16: the folded sweep as a rank-16 update on the matrix cores.
+// fp32 state, Dk = Dv = 128, T <= 16, a gate per element of a row: the folded sweep as a rank-16 update on the matrix cores.
 //   S_out^T = diag(prod g) S_in^T + K'^T Delta,   K'[t][dk] = c_t[dk] k_t[dk]  (16 steps = 4 MFMAs
-// of 16 x 16 x 4 fp32 per 16 x 16 tile).  As scalar FMAs the update costs a wave 1024
-// instructions (4400 cycles) per head; with every workgroup of a CU reaching that phase at the
-// same time the memory pipes idle meanwhile.  The state sits in registers in accumulator layout
+// of 16 x 16 x 4 fp32 per 16 x 16 tile).  The state sits in registers in accumulator layout
 // (see swap_row_bit) and goes in and out in full 128-byte lines.
-// LDS (floats): sK[16][kPad] | sD[16][kPad] | sG[16][128] or [16] | sGt[128]
+// LDS (floats): sK[16][kPad] | sD[16][kPad] | sG[16][128] | sGt[128]
 // ---------------------------------------------------------------------------
 constexpr int kPad = 132;  // row stride of the staged tables: step rows fall on different banks
-constexpr size_t replay_f32_128_lds_floats(bool g_per_dk) {
-  return 2 * 16 * kPad + (g_per_dk ? 16 * 128 : 16) + 128;
-}
+constexpr size_t kReplayF32LdsFloats = 2 * 16 * kPad + 16 * 128 + 128;
 
 // st (accumulator layout) <- diag(sGt) st + K'^T Delta over the first 4 NB steps; MFMA j of a tile
 // covers steps 4 j + kq.
@@ -181,7 +176,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3, 3))
   float* sK = smem;
   float* sD = sK + 16 * kPad;
   float* sG = sD + 16 * kPad;
-  float* sGt = sG + (a.g_per_dk ? 16 * 128 : 16);
+  float* sGt = sG + 16 * 128;
   if (conv_window_workgroup(a)) return;
   const int slot = blockIdx.x / a.Hv, hv = blockIdx.x % a.Hv;
   const int n = slot_steps(a, slot);
@@ -204,7 +199,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3, 3))
   // raw bytes and bits in plain registers; nothing is computed from them until the state has
   // been asked for (see the fence below)
   u32x4_t rd0 = {0u, 0u, 0u, 0u}, rd1 = rd0, rk0 = rd0, rk1 = rd0, rg0 = rd0, rg1 = rd0;
-  uint32_t mask_t = 1u, mask_g = 1u, g1_bits = 0u;
+  uint32_t mask_t = 1u;
   {
     const int hk = hv / (a.Hv / a.Hk);
     const size_t slotT = (size_t)slot * a.T;
@@ -224,23 +219,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3, 3))
         rk0 = *reinterpret_cast<const u32x4_t*>((const uint16_t*)a.k + k_at);
       }
       if (a.mask != nullptr) mask_t = a.mask[slotT + t];
-      if (a.g_per_dk) {
-        if (g_wide) {
-          rg0 = reinterpret_cast<const u32x4_t*>((const float*)a.g + d_at)[0];
-          rg1 = reinterpret_cast<const u32x4_t*>((const float*)a.g + d_at)[1];
-        } else {
-          rg0 = *reinterpret_cast<const u32x4_t*>((const uint16_t*)a.g + d_at);
-        }
-      }
-    }
-    if (!a.g_per_dk && tid < a.T && tid < 16) {  // thread t < 16 also fetches the gate of step t
-      const size_t at = (slotT + tid) * a.Hv + hv;
       if (g_wide) {
-        g1_bits = ((const uint32_t*)a.g)[at];
+        rg0 = reinterpret_cast<const u32x4_t*>((const float*)a.g + d_at)[0];
+        rg1 = reinterpret_cast<const u32x4_t*>((const float*)a.g + d_at)[1];
       } else {
-        g1_bits = ((const uint16_t*)a.g)[at];
+        rg0 = *reinterpret_cast<const u32x4_t*>((const uint16_t*)a.g + d_at);
       }
-      if (a.mask != nullptr) mask_g = a.mask[slotT + tid];
     }
   }
 
@@ -252,8 +236,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3, 3))
 
   // Fence: the state's loads are out before any of the tape's values is looked at, so the
   // wait that the first use brings covers the tape only (loads return in issue order).
-  asm volatile("" : "+v"(rd0), "+v"(rd1), "+v"(rk0), "+v"(rk1), "+v"(rg0), "+v"(rg1), "+v"(mask_t), "+v"(mask_g),
-               "+v"(g1_bits)::"memory");
+  asm volatile("" : "+v"(rd0), "+v"(rd1), "+v"(rk0), "+v"(rk1), "+v"(rg0), "+v"(rg1), "+v"(mask_t)::"memory");
 
   // masked and missing steps are (delta = 0, k = 0, g = 1): no-op steps
   {
@@ -268,23 +251,17 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3, 3))
     rk.w[K_WIDE ? 1 : 0] = as_uint4(keep ? (K_WIDE ? rk1 : rk0) : zero);
     raw8_to_lds<TAPE_WIDE>(rd, a.tape_dtype, sD + t * kPad + 8 * seg);
     raw8_to_lds<K_WIDE>(rk, a.k_dtype, sK + t * kPad + 8 * seg);
-    if (a.g_per_dk) {
-      float* dst = sG + t * 128 + 8 * seg;
-      if (!keep) {
-        reinterpret_cast<float4*>(dst)[0] = reinterpret_cast<float4*>(dst)[1] = float4{1.f, 1.f, 1.f, 1.f};
-      } else if (g_wide) {
-        Raw8<true> rg;
-        rg.w[0] = as_uint4(rg0), rg.w[1] = as_uint4(rg1);
-        raw8_to_lds<true>(rg, a.g_dtype, dst);
-      } else {
-        Raw8<false> rg;
-        rg.w[0] = as_uint4(rg0);
-        raw8_to_lds<false>(rg, a.g_dtype, dst);
-      }
-    } else if (tid < 16) {
-      const bool on = tid < n && mask_g != 0;
-      sG[tid] = !on ? 1.f : a.g_dtype == DFLASH_BF16 ? bf16_bits_to_f32(g1_bits)
-                          : a.g_dtype == DFLASH_FP16 ? f16_bits_to_f32(g1_bits) : __uint_as_float(g1_bits);
+    float* dst = sG + t * 128 + 8 * seg;
+    if (!keep) {
+      reinterpret_cast<float4*>(dst)[0] = reinterpret_cast<float4*>(dst)[1] = float4{1.f, 1.f, 1.f, 1.f};
+    } else if (g_wide) {
+      Raw8<true> rg;
+      rg.w[0] = as_uint4(rg0), rg.w[1] = as_uint4(rg1);
+      raw8_to_lds<true>(rg, a.g_dtype, dst);
+    } else {
+      Raw8<false> rg;
+      rg.w[0] = as_uint4(rg0);
+      raw8_to_lds<false>(rg, a.g_dtype, dst);
     }
   }
   __syncthreads();
@@ -293,7 +270,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3, 3))
     float c = 1.f;
     for (int t = n - 1; t >= 0; --t) {
       sK[t * kPad + tid] *= c;
-      c *= a.g_per_dk ? sG[t * 128 + tid] : sG[t];
+      c *= sG[t * 128 + tid];
     }
     sGt[tid] = c;
   }
@@ -327,7 +304,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3, 3))
 // Dk = 64 or 128, T <= 16, one gate per head: a thread keeps 8 consecutive columns of R rows of S in registers from
 // the first step to the last.  STATE = bf16 / fp16: step by step, rounded to that type after every step, three
 // and a half vector instructions per element and step (unpack, product, fma, half a conversion of two).  STATE =
-// fp32: the folded single sweep, for the head sizes the matrix-core kernel above does not have.
+// fp32: the folded single sweep.  Each wave multiplies the gates up by itself, out of the lanes that fetched them, and k is
+// scaled on its way to LDS: with the products made there, one dependent read per step, and a barrier, 32 heads took 6.0 us.
 //  * One request of 16 bytes per row and lane; the tape is asked for first, the state right behind it, and nothing
 //    is looked at before all of it is on its way (see replay_f32_128).
 //  * k of a step is read from LDS once for the R rows; a wave's reads of it are 512 consecutive bytes.
@@ -335,7 +313,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3, 3))
 //    computes, so a launch of few heads is spread over 32 rows per workgroup (R = 2, 64 x 64 heads: R = 1).
 // Measured against replay_generic, which served these before (one workgroup per head, 2-byte accesses, a division
 // per element), bf16 states, 16 / 6 steps, us: 32 heads of 128 x 128 97.8 / 45.6 -> 5.1 / 3.9, 1536 heads 148 / 69 -> 44 / 21;
-// 32 heads of 64 x 64 26.6 / 13.4 -> 4.0 / 3.2, 1536 heads 39 / 21 -> 12.3 / 7.9.
+// 32 heads of 64 x 64 26.6 / 13.4 -> 4.0 / 3.2, 1536 heads 39 / 21 -> 12.3 / 7.9.  fp32 states of 128 x 128 against a rank-16 update on
+// the fp32 matrix cores, a workgroup per head (the form replay_f32_128 keeps for gates per element; same bits): 1 head 6.7 / 6.2 -> 4.0 / 3.5,
+// 32 heads 7.4 / 6.8 -> 4.4 / 3.9, 192 heads 8.3 / 7.4 -> 6.9 / 6.3, 1536 heads 40.9 / 39.7 -> 37.2 / 35.7 (5.7 TB/s); of 64 x 64, 32 heads
+// 4.7 / 3.9 -> 3.5 / 3.2, 1536 heads 14.5 / 13.1 -> 11.8 / 11.6.
 // ---------------------------------------------------------------------------
 template <int STATE, int DK, int R>
 __global__ __launch_bounds__(kThreads) void replay_rows(ReplayArgs a) {
@@ -359,14 +340,17 @@ __global__ __launch_bounds__(kThreads) void replay_rows(ReplayArgs a) {
     load_bits<kK>(a.k, ((slotT + t) * a.Hk + hk) * DK + kK * seg, a.k_dtype == DFLASH_FP32, rk);
     if (a.mask != nullptr) mask_t = a.mask[slotT + t];
   }
-  if (tid < a.T) {  // thread t < 16 also fetches the gate of step t
-    const size_t at = (slotT + tid) * a.Hv + hv;
+  // thread t < 16 also fetches the gate of step t; fp32 states: lanes t, 16 + t, .. of every wave
+  const int gt = kWide ? tid & 15 : tid;
+  if (gt < a.T) {
+    const size_t at = (slotT + gt) * a.Hv + hv;
     if (a.g_dtype == DFLASH_FP32) g_bits = ((const uint32_t*)a.g)[at];
     else g_bits = ((const uint16_t*)a.g)[at];
-    if (a.mask != nullptr) mask_g = a.mask[slotT + tid];
+    if (a.mask != nullptr) mask_g = a.mask[slotT + gt];
   }
   const int rr = tid / kLanes, c8 = tid % kLanes;
-  const size_t at0 = ((size_t)head * a.Dv + row0 + rr) * DK + 8 * c8;
+  // fp32: a lane's columns are four of either half of the row, so that every access of a row is in one piece
+  const size_t at0 = ((size_t)head * a.Dv + row0 + rr) * DK + (kWide ? 4 : 8) * c8;
   u32x4_t raw[R][kWide ? 2 : 1];
 #pragma unroll
   for (int i = 0; i < R; ++i) {
@@ -374,7 +358,7 @@ __global__ __launch_bounds__(kThreads) void replay_rows(ReplayArgs a) {
     if (kWide) {
       const u32x4_t* src = reinterpret_cast<const u32x4_t*>((const float*)a.state_in + at);
       raw[i][0] = __builtin_nontemporal_load(src);
-      raw[i][kWide ? 1 : 0] = __builtin_nontemporal_load(src + 1);
+      raw[i][kWide ? 1 : 0] = __builtin_nontemporal_load(src + DK / 8);
     } else {
       raw[i][0] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>((const uint16_t*)a.state_in + at));
     }
@@ -386,26 +370,24 @@ __global__ __launch_bounds__(kThreads) void replay_rows(ReplayArgs a) {
   asm volatile("" : "+v"(mask_t), "+v"(mask_g), "+v"(g_bits)::"memory");
 
   // masked and missing steps are (delta = 0, k = 0, g = 1): no-op steps
-  {
-    const bool keep = t < n && mask_t != 0;
+  const uint32_t g_word[1] = {g_bits};
+  const float gate = gt < n && mask_g != 0 ? bits_element(g_word, 0, a.g_dtype) : 1.f;
+  float total = 1.f, after = 1.f;  // products of all gates and of those behind step t, which goes into k
+  if (kWide) {
 #pragma unroll
-    for (int e = 0; e < kD; ++e) sD[t * kRows + kD * seg + e] = keep ? bits_element(rd, e, a.tape_dtype) : 0.f;
-#pragma unroll
-    for (int e = 0; e < kK; ++e) sK[t * DK + plane_index<DK>(kK * seg + e)] = keep ? bits_element(rk, e, a.k_dtype) : 0.f;
-    if (tid < 16) {
-      const uint32_t bits[1] = {g_bits};
-      sG[tid] = tid < n && mask_g != 0 ? bits_element(bits, 0, a.g_dtype) : 1.f;
+    for (int s = 15; s >= 0; --s) {
+      after = t == s ? total : after;
+      total *= __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(gate), s));
     }
+  } else if (tid < 16) {
+    sG[tid] = gate;
   }
+  const bool keep = t < n && mask_t != 0;
+#pragma unroll
+  for (int e = 0; e < kD; ++e) sD[t * kRows + kD * seg + e] = keep ? bits_element(rd, e, a.tape_dtype) : 0.f;
+#pragma unroll
+  for (int e = 0; e < kK; ++e) sK[t * DK + (kWide ? kK * seg + e : plane_index<DK>(kK * seg + e))] = keep ? bits_element(rk, e, a.k_dtype) * after : 0.f;
   __syncthreads();
-  float total = 1.f;
-  if (kWide) {  // suffix products of the gates into the k rows
-    for (int s = n - 1; s >= 0; --s) {
-      if (tid < DK) sK[s * DK + tid] *= total;
-      total *= sG[s];
-    }
-    __syncthreads();
-  }
 
   if constexpr (kWide) {
     float v[R][8];
@@ -413,19 +395,21 @@ __global__ __launch_bounds__(kThreads) void replay_rows(ReplayArgs a) {
     for (int i = 0; i < R; ++i)
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[i][e] = __uint_as_float(raw[i][kWide ? e >> 2 : 0][e & 3]) * total;
-#pragma unroll 2
-    for (int s = 0; s < n; ++s) {
-      float k8[8];
+    for (int s0 = 0; s0 < n; s0 += 4) {  // (steps from n on are no-op steps)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const float4 k4 = *reinterpret_cast<const float4*>(sK + s * DK + h * (DK / 2) + 4 * c8);
-        k8[4 * h] = k4.x, k8[4 * h + 1] = k4.y, k8[4 * h + 2] = k4.z, k8[4 * h + 3] = k4.w;
-      }
+      for (int s = s0; s < s0 + 4; ++s) {
+        float k8[8];
 #pragma unroll
-      for (int i = 0; i < R; ++i) {
-        const float d = sD[s * kRows + i * kPass + rr];
+        for (int h = 0; h < 2; ++h) {
+          const float4 k4 = *reinterpret_cast<const float4*>(sK + s * DK + h * (DK / 2) + 4 * c8);
+          k8[4 * h] = k4.x, k8[4 * h + 1] = k4.y, k8[4 * h + 2] = k4.z, k8[4 * h + 3] = k4.w;
+        }
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[i][e] = fmaf(d, k8[e], v[i][e]);
+        for (int i = 0; i < R; ++i) {
+          const float d = sD[s * kRows + i * kPass + rr];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[i][e] = fmaf(d, k8[e], v[i][e]);
+        }
       }
     }
 #pragma unroll
@@ -458,17 +442,26 @@ __global__ __launch_bounds__(kThreads) void replay_rows(ReplayArgs a) {
     if (kWide) {
       u32x4_t* dst = reinterpret_cast<u32x4_t*>((float*)a.state_out + at);
       __builtin_nontemporal_store(raw[i][0], dst);
-      __builtin_nontemporal_store(raw[i][kWide ? 1 : 0], dst + 1);
+      __builtin_nontemporal_store(raw[i][kWide ? 1 : 0], dst + DK / 8);
     } else {
       __builtin_nontemporal_store(raw[i][0], reinterpret_cast<u32x4_t*>((uint16_t*)a.state_out + at));
     }
   }
 }
 
-// The form of replay_rows for a head size and state type; rows: how many a workgroup computes.
+// The form of replay_rows for a head size and state type; rows: how many a workgroup computes.  heads: of all slots.  The lines
+// of the fp32 states (16 bf16 steps, us with one / two / four / eight rows of a pass): 128 x 128, 32 heads 4.5 / 4.4 / 5.1 / 7.2,
+// 192 heads 8.9 / 6.9 / 7.3 / 8.6, 256 heads 11.0 / 7.9 / 7.9 / 9.7, 384 heads 14.9 / 11.6 / 9.8 / 11.2, 1536 heads 42.6 / 39.5 / 37.2 / 39.9;
+// 64 x 64, 32 heads 3.5 / 4.0, 96 heads 4.1 / 4.2, 256 heads 5.1 / 4.5, 1536 heads 13.8 / 11.8.  Of the 16-bit ones: a whole head per
+// workgroup from 1024 heads on, where k is staged once for more rows, but at 16 steps fewer waves cover each other's waits (128 x 128, 16 / 6
+// steps, us, split and whole: 512 heads 16.0 / 10.0 and 19.3 / 10.3, 1024 heads 28.6 / 16.8 and 31.9 / 15.4, 1536 heads 41.6 / 25.4
+// and 44.4 / 20.5; 64 x 64 at 1024 heads 10.6 / 7.2 and 9.6 / 6.1).
 template <int STATE>
-const void* replay_rows_for(int Dk, int Dv, bool many, int* rows) {
-  if (Dk == 128 && many && Dv % 128 == 0) return *rows = 128, (const void*)replay_rows<STATE, 128, 8>;
+const void* replay_rows_for(int Dk, int Dv, long long heads, int* rows) {
+  constexpr bool kWide = STATE == DFLASH_FP32;
+  const bool many = kWide ? heads > (Dk == 128 ? 192 : 96) : heads >= 1024;
+  constexpr int kMany = kWide ? 4 : 8;
+  if (Dk == 128 && many && Dv % (16 * kMany) == 0) return *rows = 16 * kMany, (const void*)replay_rows<STATE, 128, kMany>;
   if (Dk == 128 && Dv % 32 == 0) return *rows = 32, (const void*)replay_rows<STATE, 128, 2>;
   if (Dk == 64 && many && Dv % 64 == 0) return *rows = 64, (const void*)replay_rows<STATE, 64, 2>;
   if (Dk == 64 && Dv % 32 == 0) return *rows = 32, (const void*)replay_rows<STATE, 64, 1>;
@@ -572,23 +565,21 @@ int replay_launch(const void* tape, const void* k, const void* g, const void* st
   const bool exact = exact_order != 0 || state_dtype != DFLASH_FP32;
   // the 128 x 128 kernel fetches tape, k and per-element gates 16 bytes at a time
   const bool aligned16 = (((uintptr_t)tape | (uintptr_t)k | (g_per_dk ? (uintptr_t)g : 0)) % 16) == 0;
-  const bool fast = !exact && Dk == 128 && Dv == 128 && T <= 16 && aligned16;
-  // 16-bit states step by step and fp32 states of the other head sizes.  A whole head per workgroup from 1024 heads on: k
-  // is staged once for more rows, but at 16 steps fewer waves cover each other's waits (128 x 128, 16 / 6 steps, us, split and
-  // whole: 512 heads 16.0 / 10.0 and 19.3 / 10.3, 1024 heads 28.6 / 16.8 and 31.9 / 15.4, 1536 heads 41.6 / 25.4 and 44.4 / 20.5;
-  // 64 x 64 at 1024 heads 10.6 / 7.2 and 9.6 / 6.1).
+  // one gate per head, at least a step: step by step for 16-bit states, folded for fp32 ones
   const void* by_rows = nullptr;
   int rows = Dv;
-  if (!fast && !g_per_dk && T >= 1 && T <= 16 && aligned16 && (((uintptr_t)state_in | (uintptr_t)state_out) % 16) == 0 &&
+  if (!g_per_dk && T >= 1 && T <= 16 && aligned16 && (((uintptr_t)state_in | (uintptr_t)state_out) % 16) == 0 &&
       (!exact || state_dtype != DFLASH_FP32)) {
-    const bool many = (long long)slots * Hv >= 1024;
-    by_rows = state_dtype == DFLASH_BF16   ? replay_rows_for<DFLASH_BF16>(Dk, Dv, many, &rows)
-              : state_dtype == DFLASH_FP16 ? replay_rows_for<DFLASH_FP16>(Dk, Dv, many, &rows)
-                                           : replay_rows_for<DFLASH_FP32>(Dk, Dv, many, &rows);
+    const long long heads = (long long)slots * Hv;
+    by_rows = state_dtype == DFLASH_BF16   ? replay_rows_for<DFLASH_BF16>(Dk, Dv, heads, &rows)
+              : state_dtype == DFLASH_FP16 ? replay_rows_for<DFLASH_FP16>(Dk, Dv, heads, &rows)
+                                           : replay_rows_for<DFLASH_FP32>(Dk, Dv, heads, &rows);
   }
+  // gates per element of a row: the matrix-core form
+  const bool fast = !exact && g_per_dk && Dk == 128 && Dv == 128 && T <= 16 && aligned16;
   const size_t Tl = fast ? 16 : (size_t)T;
   const size_t smem_floats = by_rows ? 0
-                             : fast  ? replay_f32_128_lds_floats(g_per_dk != 0)
+                             : fast  ? kReplayF32LdsFloats
                                      : (size_t)Dv * Tl + Tl * Dk + Tl * (g_per_dk ? Dk : 1) + (size_t)Dk;
   const size_t smem = smem_floats * sizeof(float);
   DFLASH_REQUIRE(state_dtype != DFLASH_FP32 ||

@@ -442,3 +442,19 @@ def test_states_held_in_registers(native_lib, dt, Dk, Dv, layers, T):
         mm = None if m is None else torch.from_numpy(m.astype(np.uint8)).to(DEV)
         replay_launch(d.tape, apart, d.g, d.state, walked, steps=steps.to(DEV), T_alloc=T, mask=mm, slots=slots)
         assert torch.equal(out, walked)
+
+
+@pytest.mark.parametrize("D,slots", [(128, 6), (128, 7), (64, 3), (64, 4)])
+def test_a_slot_alone_and_among_many(native_lib, D, slots):
+    """fp32 states: how many rows of a head a workgroup takes depends on the heads of the launch (up to and beyond 192 of
+    128 x 128, 96 of 64 x 64), the order of a row's sum does not: the same bits, steps past the accepted ones left out."""
+    case = make_replay_case(slots, Hk=16, Hv=32, Dk=D, Dv=D, steps=16, seed=90 + slots)
+    steps = torch.tensor([16, 0, 1, 7, 4, 13, 5][:slots], dtype=torch.int32)
+    out = _launch(case, steps)
+    want = _oracle_slots(case, steps.numpy())
+    d = case.to(DEV)
+    for s in range(slots):
+        assert _rel_l2(_np(out).reshape(slots, -1)[s], want.reshape(slots, -1)[s]) <= TOL, s
+        one = torch.empty_like(d.state[s:s + 1])
+        replay_launch(d.tape[s:s + 1], d.k[s:s + 1], d.g[s:s + 1], d.state[s:s + 1], one, steps=int(steps[s]), T_alloc=16, slots=1)
+        assert torch.equal(one[0], out[s]), s
