@@ -9,7 +9,8 @@ namespace dflash {
 namespace {
 
 // Sum of the squares of a head: PER elements in each of LANES lanes (a power of two).  Adjacent elements first and in
-// sixty-fourths of the head whatever LANES is, so that a row has the same sum in every kernel.
+// sixty-fourths of the head whatever LANES is, so that a row has the same sum in every kernel (fmaf by name: of a sum of two
+// products either may be the one that is rounded).
 template <int PER, int LANES>
 __device__ __forceinline__ float sum_of_squares(const float (&v)[PER]) {
   constexpr int kEach = PER * LANES / 64, kParts = PER / kEach;
@@ -18,7 +19,7 @@ __device__ __forceinline__ float sum_of_squares(const float (&v)[PER]) {
   for (int i = 0; i < kParts; ++i) {
     part[i] = 0.f;
 #pragma unroll
-    for (int e = 0; e < kEach; ++e) part[i] += v[i * kEach + e] * v[i * kEach + e];
+    for (int e = 0; e < kEach; ++e) part[i] = fmaf(v[i * kEach + e], v[i * kEach + e], part[i]);
   }
 #pragma unroll
   for (int n = kParts / 2; n >= 1; n /= 2)

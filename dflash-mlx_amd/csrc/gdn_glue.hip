@@ -15,7 +15,8 @@
 // of its head in turn, so that a row of qkv is read and unpacked once and not once per tap, the taps once per wave, and
 // the gates of all its tokens are computed side by side, one token per lane.  1024 tokens of 16 + 16 + 32 heads of
 // 128: 62 us with a wave per token and head, 21.4 us with several tokens and the library's exponential and division, 17.5 us with
-// the hardware's for 16-bit arrays (errors against fp64 the same in six digits); the gated norm 15 -> 10.1 -> 8.6 us.  The projections are read where a joint product
+// the hardware's for 16-bit arrays (errors against fp64 the same in six digits), 14.8 us with rows asked for two tokens
+// ahead (4096 tokens 47.5 -> 40.8); the gated norm 15 -> 10.1 -> 8.6 us.  The projections are read where a joint product
 // left them (rows with a stride), which saves four copies per layer call (25 us of the same prompt, 12 us of a
 // verify block).
 #include "gdn_block_device.h"
@@ -53,7 +54,7 @@ struct PrepareArgs {
 // LANES lanes per (batch, run of tokens, head); heads 0..Hk-1 are q, Hk..2Hk-1 are k, the rest v, those of a wave of
 // one kind.  A lane holds PER = D / LANES adjacent channels of its head, so a row of the head is one access per lane
 // and the K taps of those channels are PER * K adjacent weights.  All loads the first token needs are issued
-// before anything is computed, the next token's row while the present one is worked on.
+// before anything is computed, and the row of the token after the next while one is worked on.
 template <int DT, int PER, int K, int LANES>
 __device__ __forceinline__ void prepare_head(const PrepareArgs& p, int b, int s0, int s1, bool is_v, int h, int lane) {
   const int key_dim = p.Hk * p.Dk;
@@ -83,6 +84,12 @@ __device__ __forceinline__ void prepare_head(const PrepareArgs& p, int b, int s0
     load_adjacent_raw<PER>(stored ? p.conv_state : p.qkv,
                            stored ? ((size_t)b * keep + r) * C + c : qkv0 + (size_t)s * p.qkv_row, wide, xr[j]);
     mask_byte[j] = mask_at(s);
+  }
+  uint32_t ahead[PER], mask_ahead;  // of the second token
+  {
+    const int s = s0 + 1 < s1 ? s0 + 1 : s0;
+    load_adjacent_raw<PER>(p.qkv, qkv0 + (size_t)s * p.qkv_row, wide, ahead);
+    mask_ahead = mask_at(s);
   }
   load_adjacent_raw<PER * K>(p.conv_w, (size_t)c * K, wide, wr);
   // gates of the value head's tokens, one per lane (key heads read some and do not use them)
@@ -119,15 +126,20 @@ __device__ __forceinline__ void prepare_head(const PrepareArgs& p, int b, int s0
     }
   }
 
-#pragma unroll 1
-  for (int s = s0; s < s1; ++s) {
-    unpack_adjacent<PER>(xr[keep], DT, x[keep]);
-    const bool on = p.mask == nullptr || mask_byte[keep] != 0;
+  // A product of fp32 numbers, before it is rounded to fp16: the compiler makes one instruction, with one rounding, of
+  // some products and their conversion and not of others, and a row has the same bits wherever it is computed.
+  auto whole = [](float v) __attribute__((always_inline)) {
+    if (DT == DFLASH_FP16) asm("" : "+v"(v));
+    return v;
+  };
+  auto token = [&](int s, uint32_t (&row)[PER], uint32_t& mask_of_row) __attribute__((always_inline)) {
+    unpack_adjacent<PER>(row, DT, x[keep]);
+    const bool on = p.mask == nullptr || mask_of_row != 0;
 #pragma unroll
     for (int e = 0; e < PER; ++e) x[keep][e] = on ? x[keep][e] : 0.f;
-    if (s + 1 < s1) {
-      load_adjacent_raw<PER>(p.qkv, qkv0 + (size_t)(s + 1) * p.qkv_row, wide, xr[keep]);
-      mask_byte[keep] = mask_at(s + 1);
+    if (s + 2 < s1) {
+      load_adjacent_raw<PER>(p.qkv, qkv0 + (size_t)(s + 2) * p.qkv_row, wide, row);
+      mask_of_row = mask_at(s + 2);
     }
     // the last `keep` rows of [conv_state | qkv] are the next conv state
     if (s + keep >= p.S) store_adjacent<PER>(p.conv_next, ((size_t)b * keep + (s + keep - p.S)) * C + c, DT, x[keep]);
@@ -139,7 +151,8 @@ __device__ __forceinline__ void prepare_head(const PrepareArgs& p, int b, int s0
       float acc = 0.f;
 #pragma unroll
       for (int j = 0; j < K; ++j) acc += x[j][e] * w[e * K + j];
-      act[e] = silu_rounded(round_through(acc, DT), DT);
+      const float c = round_through(whole(acc), DT);
+      act[e] = round_through(whole(c * round_through(whole(sigmoid_for(c, DT)), DT)), DT);
     }
 #pragma unroll
     for (int j = 0; j < keep; ++j)
@@ -148,17 +161,22 @@ __device__ __forceinline__ void prepare_head(const PrepareArgs& p, int b, int s0
 
     if (is_v) {
       store_adjacent<PER>(p.v, ((token0 + s) * p.Hv + hv) * p.Dv + PER * lane, DT, act);
-      continue;
+      return;
     }
     const float inv_rms = 1.0f / sqrtf(sum_of_squares<PER, LANES>(act) / (float)D + p.eps);
     const bool is_q = h < p.Hk;
     const float scale = is_q ? p.scale_q : p.scale_k;
     void* out = is_q ? p.q : p.k;
-    const size_t row = (token0 + s) * p.Hk + (is_q ? h : h - p.Hk);
+    const size_t at = (token0 + s) * p.Hk + (is_q ? h : h - p.Hk);
     float scaled[PER];
 #pragma unroll
-    for (int e = 0; e < PER; ++e) scaled[e] = scale * round_through(act[e] * inv_rms, DT);
-    store_adjacent<PER>(out, row * p.Dk + PER * lane, DT, scaled);
+    for (int e = 0; e < PER; ++e) scaled[e] = whole(scale * round_through(whole(act[e] * inv_rms), DT));
+    store_adjacent<PER>(out, at * p.Dk + PER * lane, DT, scaled);
+  };
+#pragma unroll 1
+  for (int s = s0; s < s1; s += 2) {
+    token(s, xr[keep], mask_byte[keep]);
+    if (s + 1 < s1) token(s + 1, ahead, mask_ahead);
   }
 }
 
@@ -340,13 +358,16 @@ extern "C" int dflash_gdn_prepare_rows(const void* qkv, const void* conv_state, 
   // as many tokens per wave as leave 8 waves per SIMD: below that a wave's latency counts, not its instructions
   const long long per = (long long)B * S * heads / 8192;
   p.tokens = per < 1 ? 1 : per > 16 ? 16 : (int)per;
-  // Eight channels per lane once that leaves 4 waves per SIMD: the sums, roots and addresses of a row are then paid for
-  // four heads of 128 at a time, 1024 tokens 23.3 -> 20.3 us.
+  // Eight channels per lane: the sums, roots and addresses of a row are then paid for four heads of 128 at a time.  From 640 such
+  // waves on (16 + 16 + 32 heads of 128, us, a head and several per wave: 32 tokens 4.6 / 4.8, 40 tokens 5.3 / 4.5, 128 tokens
+  // 9.4 / 5.1, 200 tokens 13.2 / 6.9, 1024 tokens 21.2 / 14.8), and as many tokens each as leave the 4 waves per SIMD that fit: a
+  // few more would run by themselves at the end (3072 and 8192 waves / 4096: 512 tokens 10.9 and 14.0 / 9.7, 2048 tokens 24.6
+  // and 26.2 / 23.0).
   const int per_wave = 512 / Dk;  // heads
   const bool wide = dtype != DFLASH_FP32 && Dk == Dv && Dk != 192 && Hk % per_wave == 0 && Hv % per_wave == 0 &&
-                    (long long)B * S * heads / per_wave >= 4096;
+                    (long long)B * S * heads / per_wave >= 640;
   if (wide) {
-    const long long each = (long long)B * S * heads / per_wave / 4096, most = Dk / 8 < 16 ? Dk / 8 : 16;
+    const long long each = ((long long)B * S * heads / per_wave + 4095) / 4096, most = Dk / 8 < 16 ? Dk / 8 : 16;
     p.tokens = (int)(each > most ? most : each);  // (a lane of the head computes a token's gates)
   }
   const long long waves = (long long)B * ((S + p.tokens - 1) / p.tokens) * (wide ? heads / per_wave : heads);

@@ -355,3 +355,12 @@ def test_a_prompt_that_starts_from_nothing(native_lib, T, D, times, normed):
     for a, b in zip(run(None), run(zeros)):
         assert a.dtype == b.dtype and torch.equal(a, b)
     assert run(None, 16) is None and run(zeros, 16) is not None
+
+
+@pytest.mark.parametrize("B,S,Hk,Hv,D,K,masked", [(1, 39, 16, 32, 128, 4, False), (1, 40, 16, 32, 128, 4, True), (1, 257, 16, 32, 128, 4, False),
+                                                  (2, 41, 16, 32, 128, 3, True), (90, 2, 8, 16, 64, 4, True), (1, 515, 2, 4, 256, 2, False)])
+def test_several_heads_per_wave(native_lib, B, S, Hk, Hv, D, K, masked):
+    """Where several heads share a wave (640 waves of them and more), an odd or even number of tokens to each: the bits of one
+    token and head per wave."""
+    for name in ("bf16", "fp16"):
+        test_long_prompts_and_strided_projections(native_lib, name, B, S, Hk, Hv, D, D, K, masked)
