@@ -32,6 +32,7 @@
 #include <mutex>
 
 #include "dflash_common.h"
+#include "qmm_stream_device.h"
 
 namespace dflash {
 namespace {
@@ -429,6 +430,7 @@ int qmm_stream_gather_launch(const void* x, const int32_t* expert_ids, const uin
                              const void* scales, const void* biases, void* y, void* workspace,
                              size_t workspace_bytes, int P, int K, int N, int E, int act_dtype,
                              int sb_dtype, hipStream_t stream);
+int qmm_stream_pick_grid(int units, int row_blocks, int cus);
 bool qmm_stream_packed_eligible(int K, int N, int group_size);
 // qmm_narrow.hip: x and w 16-byte aligned, up to 16 rows
 bool qmm_narrow_covers(const void* scales, const void* biases, int K, int N, int group_size, bool silu_mul);
@@ -462,6 +464,17 @@ namespace {
 int qmm_up_to_16(const void* x, const uint32_t* w_q, const void* scales, const void* biases, void* y, void* workspace,
                  size_t workspace_bytes, int M, int K, int N, int group_size, int act_dtype, int sb_dtype, int variant,
                  int k_parts, int kernel, void* stream);
+
+// Whether the workspace is the one that qmm_stream_launch asks for.  The grid it would take is looked for only where
+// bounds of it do not settle the question (0.45 us of the host's time).
+bool qmm_stream_workspace_given(const void* workspace, size_t bytes, int K, int N) {
+  if (workspace == nullptr) return false;
+  const int stages = (K + stream::kUnitK - 1) / stream::kUnitK, row_blocks = (N + stream::kRows - 1) / stream::kRows;
+  const int units = row_blocks * stages;
+  if (bytes >= qmm_stream_workspace_bytes(N, units)) return true;
+  const int cus = qmm_stream_grid();
+  return bytes >= qmm_stream_workspace_bytes(N, cus) || bytes >= qmm_stream_workspace_bytes(N, qmm_stream_pick_grid(units, row_blocks, cus));
+}
 }  // namespace
 }  // namespace dflash
 
@@ -499,7 +512,7 @@ extern "C" int dflash_qmm_few_silu_mul(const void* x, const uint32_t* w_q, const
                  "dflash_qmm_few_silu_mul: the streaming kernel does not cover K=%d N=%d gs=%d", K, N, group_size);
   DFLASH_REQUIRE((((uintptr_t)x | (uintptr_t)w_q) % 16) == 0 && (((uintptr_t)scales | (uintptr_t)biases) % 4) == 0,
                  DFLASH_ERR_ARG, "dflash_qmm_few_silu_mul: x and w_q must be 16-byte aligned, scales and biases 4-byte aligned");
-  if (qmm_narrow_covers(scales, biases, K, N, group_size, true))
+  if (qmm_narrow_covers(scales, biases, K, N, group_size, true) && qmm_stream_workspace_given(workspace, workspace_bytes, K, N))
     return qmm_narrow_launch(x, w_q, scales, biases, y, M, K, N, group_size, dtype, dtype, true, false, (hipStream_t)stream);
   return qmm_stream_launch(x, w_q, scales, biases, y, workspace, workspace_bytes, M, K, N, group_size, dtype, dtype, true,
                            (hipStream_t)stream);
@@ -530,13 +543,17 @@ int qmm_up_to_16(const void* x, const uint32_t* w_q, const void* scales, const v
                  "dflash_qmm_m16: K=%d is not a multiple of 32*k_parts (k_parts=%d)", K, k_parts);
   DFLASH_REQUIRE(((uintptr_t)x % 16) == 0 && ((uintptr_t)w_q % 16) == 0, DFLASH_ERR_ARG,
                  "dflash_qmm_m16: x and w_q must be 16-byte aligned");
-  if (kernel == DFLASH_QMM_KERNEL_AUTO && qmm_narrow_covers(scales, biases, K, N, group_size, false))
+  // (needs no workspace; what a call has to bring does not depend on that)
+  const bool narrow = kernel == DFLASH_QMM_KERNEL_AUTO && qmm_narrow_covers(scales, biases, K, N, group_size, false);
+  auto narrow_launch = [&] {
     return qmm_narrow_launch(x, w_q, scales, biases, y, M, K, N, group_size, act_dtype, sb_dtype, false, false, (hipStream_t)stream);
+  };
   // (the C interface has always taken scales of 2-byte alignment; the ANYK loads need four)
   const bool any = kernel == DFLASH_QMM_KERNEL_AUTO && qmm_stream_any_eligible(K, N, group_size) &&
                    (((uintptr_t)scales | (uintptr_t)biases) % 4) == 0 && workspace != nullptr &&
                    workspace_bytes >= qmm_stream_workspace_bytes(N, qmm_stream_grid());
   if (kernel != DFLASH_QMM_KERNEL_TILE && (qmm_stream_eligible(K, N, group_size) || any)) {
+    if (narrow && qmm_stream_workspace_given(workspace, workspace_bytes, K, N)) return narrow_launch();
     return qmm_stream_launch(x, w_q, scales, biases, y, workspace, workspace_bytes, M, K, N, group_size, act_dtype,
                              sb_dtype, false, (hipStream_t)stream);
   }
@@ -557,6 +574,7 @@ int qmm_up_to_16(const void* x, const uint32_t* w_q, const void* scales, const v
     counters = (uint32_t*)workspace;
     partials = (float*)((char*)workspace + kCounterBytes);
   }
+  if (narrow) return narrow_launch();
   hipStream_t s = (hipStream_t)stream;
   switch (group_size) {
     case 32:
