@@ -731,7 +731,10 @@ extern "C" int dflash_qmm_m16_gather(const void* x, const int32_t* expert_ids, c
   hipStream_t s = (hipStream_t)stream;
   // With a workspace, shapes the streaming kernel covers go through it; everything else,
   // and callers without a workspace, through the one-workgroup-per-(columns, expert) kernel.
-  if (workspace != nullptr && qmm_stream_gather_eligible(P, K, N, E, group_size)) {
+  // (Calls of more than 256 rows have always been served whatever their workspace, and with scales of 2-byte alignment.)
+  const bool streams = P <= 256 || (workspace_bytes >= qmm_stream_workspace_bytes(N, qmm_stream_grid()) &&
+                                      (((uintptr_t)scales | (uintptr_t)biases) % 4) == 0);
+  if (workspace != nullptr && streams && qmm_stream_gather_eligible(P, K, N, E, group_size)) {
     return qmm_stream_gather_launch(x, expert_ids, w_q, scales, biases, y, workspace, workspace_bytes,
                                     P, K, N, E, act_dtype, sb_dtype, s);
   }

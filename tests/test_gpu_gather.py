@@ -194,3 +194,27 @@ def test_more_rows_than_a_workgroup_has_threads(native_lib, P, E, K, N):
         mine = ids == e
         if mine.any():
             _check(y[mine], x[mine], dequantize(w[e], s[e], b[e], 64, 4, torch.float64), K, torch.bfloat16)
+
+
+def test_many_rows_with_a_workspace_that_is_too_small(native_lib):
+    """Calls of more than 256 rows need no workspace: one that is too small, or scales that start on two bytes, leave them to
+    the kernel without one."""
+    gen = torch.Generator("cuda").manual_seed(7)
+    P, E, K, N = 300, 4, 512, 96
+    w = torch.randint(-2 ** 31, 2 ** 31, (E, N, K // 8), generator=gen, device="cuda", dtype=torch.int32)
+    s = (torch.rand((E, N, K // 64), generator=gen, device="cuda") * 0.02 + 1e-4).to(torch.bfloat16)
+    b = (s.float() * -8).to(torch.bfloat16)
+    odd = torch.empty(s.numel() + 1, dtype=s.dtype, device="cuda")[1:].view(s.shape)
+    odd.copy_(s)
+    x = torch.randn((P, K), generator=gen, device="cuda").to(torch.bfloat16)
+    ids = torch.randint(0, E, (P,), generator=gen, device="cuda", dtype=torch.int32)
+    need = native_lib.dflash_qmm_m16_gather_workspace_bytes(P, K, N, E, 64)
+    ws = torch.zeros(need, dtype=torch.uint8, device="cuda")
+    ys = []
+    for scales, workspace, size in ((s, None, 0), (s, ws, need - 1), (odd, ws, need)):
+        y = torch.empty((P, N), dtype=x.dtype, device="cuda")
+        assert native_lib.dflash_qmm_m16_gather(x.data_ptr(), ids.data_ptr(), w.data_ptr(), scales.data_ptr(), b.data_ptr(), y.data_ptr(),
+                                                None if workspace is None else workspace.data_ptr(), size, P, K, N, E, 64, 0, 0,
+                                                torch.cuda.current_stream().cuda_stream) == 0
+        ys.append(y)
+    assert torch.equal(ys[0], ys[1]) and torch.equal(ys[0], ys[2])
