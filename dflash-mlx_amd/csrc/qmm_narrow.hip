@@ -240,9 +240,9 @@ const void* kernel_for(bool a16, bool s16, int GS, bool silu, bool packed) {
 // Tiles of a workgroup, 0: not this kernel's.  One round of workgroups on 256 compute units: 16 rows of W each up to N = 4096; 32 each up to
 // 8192, where a K of 2048 is the last that 16 rows of x do not make slower (2048 x 8192 7.5 -> 7.0 us, 2560 x 6144 7.5 -> 7.8).
 // Beyond K = 3584 x alone takes as long as the partial sums did (4096 x 4096, 16 rows: 7.9 -> 8.3 us, one row 7.6 -> 6.0), except
-// where the streaming kernel cuts few row blocks into many (4736 x 2304 9.4 -> 8.4; 4096 x 2048, 8.6 against 7.9, stays there: products of
-// that K are chained, and a chain gives the streaming kernel's bits).  K below 512 is the tile kernel's (256 x 512: 2.65 us,
-// here 2.66).  M does not enter: a row must not change with the rows beside it.
+// where the streaming kernel cuts few row blocks into many (4736 x 2304 9.4 -> 8.4; 4096 x 2048, 8.6 against 7.9, is still the
+// streaming kernel's).  K below 512 is the tile kernel's (256 x 512: 2.65 us, here 2.66).  M does not enter: a row must not change
+// with the rows beside it.
 int tiles_for(int K, int N, int group_size) {
   if ((group_size != 32 && group_size != 64 && group_size != 128) || K % kChunk != 0 || N % 16 != 0 || K < 512 || N < 16) return 0;
   if (N <= 4096 && (K <= 3584 || (K <= 4864 && K != 4096 && N <= 2304))) return 1;
@@ -252,8 +252,12 @@ int tiles_for(int K, int N, int group_size) {
 }  // namespace narrow
 
 bool qmm_narrow_covers(const void* scales, const void* biases, int K, int N, int group_size, bool silu_mul) {
+  // The gated activation of a verify block is a chained launch where that has the form for it, and the chain's sums are the
+  // streaming kernel's: fewer rows of such a matrix go there too, so that a token decoded alone has the bits it has in a block
+  // (one row, N of both: 1024 x 4096 6.3 us there, 3.5 here; 2048 x 8192 7.4 and 6.8).
+  const bool chained = silu_mul && group_size == 64 && K % 1024 == 0 && N % 128 == 0;
   // a chunk's scales of a row are one load, of 2, 4 or 8 bytes
-  return narrow::tiles_for(K, N, group_size) != 0 && (((uintptr_t)scales | (uintptr_t)biases) % (256 / group_size)) == 0 &&
+  return !chained && narrow::tiles_for(K, N, group_size) != 0 && (((uintptr_t)scales | (uintptr_t)biases) % (256 / group_size)) == 0 &&
          (!silu_mul || N % 32 == 0);
 }
 

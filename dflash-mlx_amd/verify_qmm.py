@@ -241,7 +241,8 @@ class QmmChain:
     of a layer handed over as a list and run back to back by one persistent grid.  No counterpart
     in the reference, which launches its kernel once per projection
     (``dflash_mlx/verify_linear.py:103-143``); every output is bit for bit what ``verify_matmul``
-    gives for the same operands through the streaming kernel.
+    gives for the same operands through the streaming kernel (``DFLASH_QMM_KERNEL=stream``; the automatic choice takes
+    matrices of few weights through another kernel, whose fp32 sums are in another order).
 
     The chain is planned once (argument block, outputs, workspace) and can be launched any number
     of times: ``chain()`` enqueues the launch on the current stream and returns the outputs, which
@@ -447,7 +448,8 @@ def _packed_kernel() -> int:
 
 def verify_matmul_packed(x: torch.Tensor, packed: PackedWeights) -> torch.Tensor:
     """``verify_matmul`` on packed weights: 16 rows of bf16/fp16 device activations; the result is
-    bit for bit ``verify_matmul``'s on the triple the weights were packed from."""
+    bit for bit ``verify_matmul``'s on the triple the weights were packed from (scales on 4 bytes; the tile kernel, which
+    may be asked for by name, has no packed form)."""
     K, N = packed.K, packed.N
     if packed.gate_up:
         raise ValueError("verify_matmul_packed: these images are ordered for the silu-mul epilogue of a chain")

@@ -60,3 +60,47 @@ def test_gated_activation_at_the_edges(native_lib, K, N, group, dtype):
     tiny = 0.0 if dtype == BF else 2.0 ** -24  # (fp16 below its smallest normal number)
     bound = 1.1 * up.abs() * dg + (act.abs() + dg) * du + 4 * eps * (act * up).abs() + tiny * (1 + 2 * up.abs())
     assert ((y.double() - act * up).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("K,inter", [(1024, 512), (1024, 2048), (1024, 4096), (2048, 1536), (2048, 4096), (3072, 2048), (3072, 2112), (4096, 1024),
+                                     (4096, 1152)])
+def test_a_row_of_the_gated_activation_alone_and_in_its_block(verify_env, native_lib, K, inter, packed):
+    """A token's hidden activation has the same bits decoded alone, in a last short block and in a verify block, with no
+    kernel named, at widths that a chained launch serves (K a multiple of 1024, 64 rows) and on either side of this kernel's rule."""
+    from dflash_mlx_amd import verify_linear as VL
+    from dflash_mlx_amd.quantized import QuantizedLinear
+
+    parent = torch.nn.Module()
+    for name, seed in (("gate_proj", K), ("up_proj", K + 1)):
+        c = make_qmm_case(K, inter, seed).to(DEV)
+        setattr(parent, name, QuantizedLinear(c.w, c.scales * 0.05, c.biases * 0.05, group_size=64, bits=4))
+    model = torch.nn.Module()
+    model.mlp = parent
+    assert VL.install_verify_linears(model) == 2 and VL.fuse_shared_input_linears(model) == 1
+    if packed:
+        assert VL.pack_verify_linears(model) == 1
+    x = torch.randn((1, 16, K), generator=torch.Generator(DEV).manual_seed(inter), device=DEV).to(BF)
+    block = VL.silu_gate_up(parent, x)
+    assert parent._dflash_fused[0].silu_mul_ready(x) and block.shape == (1, 16, inter)
+    for lo, hi in ((0, 1), (15, 16), (2, 4), (0, 15)):
+        assert torch.equal(VL.silu_gate_up(parent, x[:, lo:hi].clone()), block[:, lo:hi]), (lo, hi)
+
+
+@pytest.mark.parametrize("dtype", [BF, HF])
+def test_gated_activation_of_two_tiles_in_groups_of_64(native_lib, dtype):
+    """Two tiles of rows per workgroup at a K that no chained launch serves."""
+    test_gated_activation_at_the_edges(native_lib, 1920, 8192, 64, dtype)
+
+
+@pytest.mark.parametrize("K,N", [(1024, 512), (2048, 8192), (3072, 2048), (4096, 2048)])
+def test_a_chain_beside_the_automatic_choice(verify_env, native_lib, K, N):
+    """A chain is the streaming kernel's also where the automatic choice is this one: the same product, the bits of the kernel
+    named."""
+    c = make_qmm_case(K, N, K + 7).to(DEV)
+    y = VQ.QmmChain([VQ.ChainProblem(c.x, c.w, c.scales, c.biases)])()[0]
+    dense = dequantize(c.w, c.scales, c.biases, 64, 4, torch.float64)
+    _check(y, c.x, dense, K, BF)
+    _check(VQ.verify_matmul(c.x, c.w, c.scales, c.biases, group_size=64), c.x, dense, K, BF)
+    verify_env.setenv("DFLASH_QMM_KERNEL", "stream")
+    assert torch.equal(y, VQ.verify_matmul(c.x, c.w, c.scales, c.biases, group_size=64))
