@@ -137,7 +137,7 @@ __global__ __launch_bounds__(256) void attn_gate_kernel(AttnGateArgs p) {
   unpack_adjacent<4>(oraw, p.dt, o);
   unpack_adjacent<4>(graw, p.dt, g);
 #pragma unroll
-  for (int e = 0; e < 4; ++e) o[e] *= round_through(sigmoid_for(g[e], DFLASH_BF16), p.dt);
+  for (int e = 0; e < 4; ++e) o[e] *= round_through(sigmoid_of_half(g[e]), p.dt);
   store_adjacent<4>(p.y, (size_t)i * 4, p.dt, o);
 }
 

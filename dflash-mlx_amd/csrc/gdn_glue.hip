@@ -14,9 +14,9 @@
 // instructions per element (the sigmoid's exponential and division, the roundings): a wave takes several tokens
 // of its head in turn, so that a row of qkv is read and unpacked once and not once per tap, the taps once per wave, and
 // the gates of all its tokens are computed side by side, one token per lane.  1024 tokens of 16 + 16 + 32 heads of
-// 128: 62 us with a wave per token and head, 21.4 us with several tokens and the library's exponential and division, 17.5 us with
-// the hardware's for 16-bit arrays (errors against fp64 the same in six digits), 14.8 us with rows asked for two tokens
-// ahead (4096 tokens 47.5 -> 40.8); the gated norm 15 -> 10.1 -> 8.6 us.  The projections are read where a joint product
+// 128: 62 us with a wave per token and head, 21.4 us with several tokens, 18.6 us with rows asked for two tokens ahead, 16.2 us with
+// the sigmoid of 16-bit numbers in half the instructions (glue_device.h; 4096 tokens 56.0 -> 46.7); the gated norm 15 -> 10.1 ->
+// 8.4 -> 7.3 us.  The projections are read where a joint product
 // left them (rows with a stride), which saves four copies per layer call (25 us of the same prompt, 12 us of a
 // verify block).
 #include "gdn_block_device.h"
@@ -359,10 +359,10 @@ extern "C" int dflash_gdn_prepare_rows(const void* qkv, const void* conv_state, 
   const long long per = (long long)B * S * heads / 8192;
   p.tokens = per < 1 ? 1 : per > 16 ? 16 : (int)per;
   // Eight channels per lane: the sums, roots and addresses of a row are then paid for four heads of 128 at a time.  From 640 such
-  // waves on (16 + 16 + 32 heads of 128, us, a head and several per wave: 32 tokens 4.6 / 4.8, 40 tokens 5.3 / 4.5, 128 tokens
-  // 9.4 / 5.1, 200 tokens 13.2 / 6.9, 1024 tokens 21.2 / 14.8), and as many tokens each as leave the 4 waves per SIMD that fit: a
-  // few more would run by themselves at the end (3072 and 8192 waves / 4096: 512 tokens 10.9 and 14.0 / 9.7, 2048 tokens 24.6
-  // and 26.2 / 23.0).
+  // waves on (16 + 16 + 32 heads of 128, us, a head and several per wave: 32 tokens 4.6 / 4.8, 40 tokens 5.3 / 4.7, 128 tokens
+  // 9.7 / 5.4, 200 tokens 13.8 / 7.2, 1024 tokens 22.3 / 16.3), and as many tokens each as leave the 4 waves per SIMD that fit: a
+  // few more would run by themselves at the end (3072 and 8192 waves / 4096: 512 tokens 11.3 and 13.0 / 11.2, 1024 tokens 17.8 and
+  // 17.1 / 16.3).
   const int per_wave = 512 / Dk;  // heads
   const bool wide = dtype != DFLASH_FP32 && Dk == Dv && Dk != 192 && Hk % per_wave == 0 && Hv % per_wave == 0 &&
                     (long long)B * S * heads / per_wave >= 640;

@@ -13,10 +13,29 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
-// sigmoid(x), for an array of type dt.  16-bit arrays take the hardware's exp2 and reciprocal (each within an ulp of fp32, where
-// half a unit of the result is 2^-9 or 2^-12 of it): 4 instructions for about 30, of what the kernels here spend most on.
+// sigmoid(x) of an x that a 16-bit array holds, with the error of 1 / (1 + expf(-x)) in 14 vector instructions for its 30.
+//  * -x log2(e) is n + f, n its nearest integer (left in the low bits of a sum with 1.5 2^23).  kLog2E has 13 bits, so that with the
+//    at most 11 of x its product is exact, and so is the difference to n: f is rounded once.
+//  * 2^n is made of n's bits, and 1 + 2^f 2^n is one fma, kept times 2^-24: its reciprocal is a normal number for every x,
+//    and what comes out is rounded once more only where it is a subnormal one.  x is bounded where the result is 1 or
+//    less than any number above 0; the bounds let a NaN pass.
+//  * a Newton step takes the hardware's reciprocal from one unit to the nearest number but for rare ties.
+// Over all numbers of a type, against 64 bits, largest and root mean square relative error: bf16 1.18e-7 and 1.51e-8, fp16 1.20e-7 and
+// 3.41e-8, of either form; 1 / (1 + expf(-x)) has 0 below x = -88.7, where this still has the subnormal numbers.  Conv and gates of
+// 1024 tokens of 16 + 16 + 32 heads of 128 18.6 -> 16.2 us, a block of 16 of them with its recurrence 16.9 -> 16.3 us.
+__device__ __forceinline__ float sigmoid_of_half(float x) {
+  constexpr float kLog2E = 5909.f / 4096.f, kRest = 6.8087763963407e-5f, kRound = 0x1.8p23f, kScale = 0x1p-24f;
+  const float u = __builtin_elementwise_maximum(__builtin_elementwise_minimum(-x, 104.f), -30.f);
+  const float m = __builtin_fmaf(u, kLog2E, kRound), n = m - kRound;
+  const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(u, kRest, __builtin_fmaf(u, kLog2E, -n)));
+  const float d = __builtin_fmaf(e, __uint_as_float((__float_as_uint(m) << 23) + __float_as_uint(kScale)), kScale);
+  const float r = __builtin_amdgcn_rcpf(d);
+  return kScale * __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r);
+}
+
+// sigmoid(x), for an array of type dt
 __device__ __forceinline__ float sigmoid_for(float x, int dt) {
-  return dt == DFLASH_FP32 ? 1.0f / (1.0f + expf(-x)) : __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504088896341f * x));
+  return dt == DFLASH_FP32 ? 1.0f / (1.0f + expf(-x)) : sigmoid_of_half(x);
 }
 
 // x * sigmoid(x) with the sigmoid and the product each rounded to the array dtype

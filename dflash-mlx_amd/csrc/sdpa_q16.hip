@@ -28,7 +28,7 @@
 //                 column 16 c + t of four keys.  No transposed copy of V or P is ever stored.
 // Ranges of keys (splits) write partial outputs in the input dtype (kernels.py:556-558) with their
 // fp32 max and sum; a second kernel merges them (the reference's second pass).
-#include "dflash_common.h"
+#include "glue_device.h"
 
 #include <cmath>
 #include <cstdlib>
@@ -364,7 +364,7 @@ __global__ __launch_bounds__(256) void sdpa_q16_merge_kernel(SdpaArgs a, int D) 
       float y[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float sig = 1.0f / (1.0f + expf(-elem_to_f32<FP16>((uint16_t)gw[e])));
+        const float sig = sigmoid_of_half(elem_to_f32<FP16>((uint16_t)gw[e]));  // the bits of attn_gate_kernel
         y[e] = elem_to_f32<FP16>((uint16_t)ow[e]) * elem_to_f32<FP16>((uint16_t)pack2<FP16>(sig, 0.f));
       }
       packed = uint2{pack2<FP16>(y[0], y[1]), pack2<FP16>(y[2], y[3])};

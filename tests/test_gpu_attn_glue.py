@@ -191,3 +191,22 @@ def test_bits_of_the_array_operators_where_the_norms_sum_is_exact(monkeypatch, D
     want = A._project(attn, x, caches[1])
     for a, b in zip(got[:3], want[:3]):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_both_gates_on_every_number(dtype):
+    """The gate where the key ranges meet and the gate of its own, for all 65536 numbers of the type."""
+    from dflash_mlx_amd.kernels import batched_sdpa_2pass_exact
+
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    Hq, D, N = 32, 128, 400
+    every = torch.arange(-2 ** 15, 2 ** 15, dtype=torch.int32).to(torch.int16).view(dtype).cuda().view(16, Hq, D)
+    projected = torch.cat([torch.zeros_like(every), every], dim=-1).view(1, 16, Hq * 2 * D)
+    attn, _ = _layer(1, 16, Hq, 8, D, D, dtype, dtype, gen, False)
+    q = torch.randn((1, Hq, 16, D), generator=gen, device="cuda").to(dtype)
+    k, v = (torch.randn((1, 8, N, D), generator=gen, device="cuda").to(dtype) for _ in range(2))
+    gated = batched_sdpa_2pass_exact(q, k, v, D ** -0.5, q_proj_output=projected)
+    assert gated.shape == (1, 16, Hq * D)
+    want = A._finish(attn, batched_sdpa_2pass_exact(q, k, v, D ** -0.5), projected)
+    nan = torch.isnan(want)
+    assert torch.equal(torch.isnan(gated), nan) and torch.equal(gated[~nan], want[~nan])

@@ -364,3 +364,51 @@ def test_several_heads_per_wave(native_lib, B, S, Hk, Hv, D, K, masked):
     token and head per wave."""
     for name in ("bf16", "fp16"):
         test_long_prompts_and_strided_projections(native_lib, name, B, S, Hk, Hv, D, D, K, masked)
+
+
+@pytest.mark.parametrize("name", ["bf16", "fp16"])
+def test_activations_of_every_16_bit_number(native_lib, name):
+    """The sigmoid behind beta, the conv's and the norm's silu and the attention's gate, for all 65536 numbers of the type.  Its fp32
+    value is within two units of fp32 (one of the exponential, a half each of the sum and the quotient), so what is stored is the
+    exact sigmoid's rounding or, where that is a tie to 2^-23, its other neighbour - down to the type's subnormal numbers."""
+    from dflash_mlx_amd.attention_layer import GatedAttention, _finish
+
+    dt = TORCH[name]
+    every = torch.arange(-2 ** 15, 2 ** 15, dtype=torch.int32).to(torch.int16).view(dt)
+    x64 = every.double()
+    grow = torch.exp(-x64.abs())
+    exact = torch.where(x64 < 0, grow, 1.0) / (1 + grow)
+    slack = 2.0 ** -23 * exact
+    rounded = [(v.clamp_min(0)).float().to(dt) for v in (exact - slack, exact + slack)]
+    number = ~torch.isnan(x64)
+
+    def check(got, low, high, what):
+        got = got.cpu()
+        assert torch.isnan(got[~number]).all(), what
+        g, a, b = got[number].double(), low[number].double(), high[number].double()
+        nan = torch.isnan(a) | torch.isnan(b)
+        assert torch.equal(torch.isnan(g), nan), what
+        wrong = ~nan & ~((g >= torch.minimum(a, b)) & (g <= torch.maximum(a, b)))
+        assert not wrong.any(), (what, every[number][wrong][:8].tolist(), g[wrong][:8].tolist())
+
+    silu = [(every.float() * s.float()).to(dt) for s in rounded]
+    d = every.to(DEV)
+    zeros = lambda *s: torch.zeros(s, dtype=dt, device=DEV)  # noqa: E731
+    params = [zeros(1024), zeros(1024)]
+    # beta: 1024 value heads, 64 tokens in one run; v: 1024 heads of 64, one token (and its conv only the last tap)
+    dims = dict(Hk=1, Hv=1024, Dk=64, Dv=64)
+    C = 128 + 1024 * 64
+    taps = zeros(C, 4)
+    taps[:, 3] = 1
+    beta = G.gdn_prepare(zeros(1, 64, C), None, taps, zeros(1, 64, 1024), d.view(1, 64, 1024), *params, **dims)[5]
+    check(beta.reshape(-1), *rounded, "beta")
+    v = G.gdn_prepare(torch.cat([zeros(128), d]).view(1, 1, C), zeros(1, 3, C), taps, zeros(1, 1, 1024), zeros(1, 1, 1024), *params, **dims)[3]
+    check(v.reshape(-1), *silu, "silu of the conv")
+    # the norm of a row of ones, with eps 0, is the weight: 1
+    normed = G.gated_norm(torch.ones((1024, 64), dtype=dt, device=DEV), d.view(1024, 64), torch.ones(64, dtype=dt, device=DEV), 0.0)
+    check(normed.reshape(-1), *silu, "silu of the norm")
+    # the gate of 64 heads of 128 behind an output of ones
+    attn = GatedAttention(num_attention_heads=64, num_key_value_heads=64, head_dim=128, q_proj=None, k_proj=None, v_proj=None,
+                          o_proj=torch.nn.Identity())
+    gate = torch.cat([zeros(8, 64, 128), d.view(8, 64, 128)], dim=-1).view(1, 8, 64 * 256)
+    check(_finish(attn, torch.ones((1, 64, 8, 128), dtype=dt, device=DEV), gate).reshape(-1), *rounded, "gate of the attention")
