@@ -427,7 +427,7 @@ PyObject* gdn_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
     w_code = dtype_code(w->scalar_type());
     const int64_t step = z->element_size();
     if (w_code == kNoCode || z->scalar_type() != q->scalar_type() || !has_shape(*z, {B, T, hv, dv}) ||
-        z->device() != q->device() || w->device() != q->device() || w->numel() != dv || !w->is_contiguous() ||
+        z->device() != q->device() || w->device() != q->device() || w->numel() != dv || !w->is_contiguous() || !aligned(at_of(*w), 16) ||
         dv % 64 != 0 || dv > 256)
       Py_RETURN_NONE;
     if (z->stride(3) != 1 || z->stride(2) != dv || z->stride(1) == 0 || !aligned(at_of(*z), 16) ||

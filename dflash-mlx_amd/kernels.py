@@ -155,10 +155,12 @@ def gated_delta_kernel_with_tape(q: torch.Tensor, k: torch.Tensor, v: torch.Tens
         if not fused_output_norm_applies(q, v, state, z, weight):
             raise ValueError("output_norm: shapes or dtypes the fused kernel does not take")
         z_c, w_c = z, weight.contiguous()
-        # steps and slots may have a stride (columns of a joint product); heads and columns lie together
+        if w_c.data_ptr() % 16:
+            w_c = w_c.clone()
+        # steps and slots may have a stride (columns of a joint product); heads and columns lie together, on 16 bytes
         if z_c.stride(3) != 1 or z_c.stride(2) != dv or z_c.stride(1) == 0 or z_c.data_ptr() % 16 \
                 or (z_c.stride(0) | z_c.stride(1)) * z_c.element_size() % 16:
-            z_c = z_c.contiguous()
+            z_c = z_c.clone(memory_format=torch.contiguous_format)
     rc = lib.dflash_gdn_forward(
         q_c.data_ptr(), k_c.data_ptr(), v_c.data_ptr(), g_c.data_ptr(), beta_c.data_ptr(),
         state_c.data_ptr(), state_out.data_ptr(), None if z_c is None else z_c.data_ptr(),

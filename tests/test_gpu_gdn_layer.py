@@ -412,3 +412,43 @@ def test_activations_of_every_16_bit_number(native_lib, name):
                           o_proj=torch.nn.Identity())
     gate = torch.cat([zeros(8, 64, 128), d.view(8, 64, 128)], dim=-1).view(1, 8, 64 * 256)
     check(_finish(attn, torch.ones((1, 64, 8, 128), dtype=dt, device=DEV), gate).reshape(-1), *rounded, "gate of the attention")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("S,armed", [(1, False), (5, True), (16, True), (40, True), (40, False)])
+@pytest.mark.parametrize("shifted", ["weight", "gate", "neither"])
+def test_operands_that_start_on_any_element(native_lib, dtype, S, armed, shifted):
+    """The output norm's weight, or its gate, off the 16-byte grid: the same call, with or without a state and a tape.  A block whose
+    one launch declines it is the prepare kernel and the recurrence, whose bits are the same."""
+    gen = torch.Generator(DEV).manual_seed(S)
+    Hk, Hv, D = 2, 4, 128
+    C = 2 * Hk * D + Hv * D
+
+    def r(*shape, std=1.0):
+        return (torch.randn(shape, generator=gen, device=DEV) * std).to(dtype)
+
+    def off(t):
+        return torch.cat([t.reshape(-1)[:1], t.reshape(-1)])[1:].view(t.shape)
+
+    parts = [r(1, S, n) for n in (C, Hv * D, Hv, Hv)]
+    weight, taps, window, s0 = 1 + r(D, std=0.1), r(C, 4, 1, std=0.5), r(1, 3, C), r(1, Hv, D, D, std=0.1)
+
+    def run(shift, state):
+        z = off(parts[1]) if shift == "gate" else parts[1]
+        mixer = G.GatedDeltaNet(8, num_k_heads=Hk, num_v_heads=Hv, head_k_dim=D, head_v_dim=D, in_proj_qkv=_Given(parts[0]),
+                                in_proj_z=_Given(z), in_proj_b=_Given(parts[2]), in_proj_a=_Given(parts[3]),
+                                out_proj=torch.nn.Identity()).to(DEV)
+        mixer.conv1d.weight.data, mixer.norm.weight.data = taps, off(weight) if shift == "weight" else weight
+        assert (mixer.norm.weight.data_ptr() % 16 != 0) == (shift == "weight")
+        cache = RecurrentRollbackCache(size=2, conv_kernel_size=4)
+        if state:
+            cache[0], cache[1] = window, s0
+        if armed:
+            cache.arm_rollback()
+        y = G._gdn_call(mixer, torch.zeros((1, S, 8), device=DEV, dtype=dtype), None, cache, armed)
+        return y, cache[0], cache[1], cache._tape
+
+    for state in (False, True):
+        for a, b in zip(run(shifted, state), run("neither", state)):
+            assert (a is None) == (b is None)
+            assert a is None or (a.shape == b.shape and a.dtype == b.dtype and torch.equal(a, b))
