@@ -462,15 +462,16 @@ PyObject* gdn_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
 
 // gdn_block(qkv, conv_state, conv_w, a, b, A_log, dt_bias, z, weight, state, Hk, Hv, Dk, Dv, eps, norm_eps, record): a block of
 // up to 16 tokens without a mask in one launch, where that has a form for it; z [B, S, Hv Dv] and the norm's weight None, or what
-// the output norm takes.  (y, state, conv_next, tape, k, g, qkv in one piece); the last three None unless recorded, the last
+// the output norm takes; state None: zeros of qkv's type, filled once the call is known to be served.  (y, state, conv_next, tape, k, g, qkv in one piece); the last three None unless recorded, the last
 // one also where qkv is in one piece already.
 PyObject* gdn_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (n != 17) Py_RETURN_NONE;
   const Tensor *qkv = device_tensor(a[0]), *cs = nullptr, *w = device_tensor(a[2]), *ga = device_tensor(a[3]),
                *gb = device_tensor(a[4]), *A = device_tensor(a[5]), *dt = device_tensor(a[6]), *z = nullptr, *weight = nullptr,
-               *state = device_tensor(a[9]);
-  if (!qkv || !w || !ga || !gb || !A || !dt || !state || qkv->dim() != 3) Py_RETURN_NONE;
+               *state = nullptr;
+  if (!qkv || !w || !ga || !gb || !A || !dt || qkv->dim() != 3) Py_RETURN_NONE;
+  if (a[9] != Py_None && !(state = device_tensor(a[9]))) Py_RETURN_NONE;
   if (a[1] != Py_None && !(cs = device_tensor(a[1]))) Py_RETURN_NONE;
   if (a[7] != Py_None && (!(z = device_tensor(a[7])) || !(weight = device_tensor(a[8])))) Py_RETURN_NONE;
   int Hk, Hv, D, Dv;
@@ -481,7 +482,7 @@ PyObject* gdn_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int64_t B = qkv->size(0), S = qkv->size(1), C = qkv->size(2);
   const auto type = at::kBFloat16;
   const auto device = qkv->device();
-  const int param = dtype_code(A->scalar_type()), s_code = dtype_code(state->scalar_type());
+  const int param = dtype_code(A->scalar_type()), s_code = state ? dtype_code(state->scalar_type()) : DFLASH_BF16;
   if (qkv->scalar_type() != type || param == kNoCode || s_code == kNoCode || D != Dv || (D != 64 && D != 128) || B < 1 || S < 1 ||
       S > 16 || Hk < 1 || Hv < 1 || Hk > (1 << 15) || Hv > (1 << 15) || Hv % Hk != 0 || C != 2 * (int64_t)Hk * D + (int64_t)Hv * D ||
       B * S * (2 * Hk + Hv) * D >= (1ll << 31) || dflash_get_option(DFLASH_OPT_GDN_STEP_BY_STEP) != 0)
@@ -489,11 +490,12 @@ PyObject* gdn_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (w->dim() < 2 || w->dim() > 3 || w->size(0) != C || w->size(1) != 4 || (w->dim() == 3 && w->size(2) != 1) ||
       !w->is_contiguous() || w->scalar_type() != type || ga->scalar_type() != type || gb->scalar_type() != type ||
       dt->scalar_type() != A->scalar_type() || !has_shape(*ga, {B, S, Hv}) || !has_shape(*gb, {B, S, Hv}) || !has_shape(*A, {Hv}) ||
-      !has_shape(*dt, {Hv}) || !A->is_contiguous() || !dt->is_contiguous() || !has_shape(*state, {B, Hv, D, D}) ||
-      !state->is_contiguous() || !aligned(at_of(*state), 16))
+      !has_shape(*dt, {Hv}) || !A->is_contiguous() || !dt->is_contiguous())
     Py_RETURN_NONE;
-  for (const Tensor* t : {w, ga, gb, A, dt, state})
+  for (const Tensor* t : {w, ga, gb, A, dt})
     if (t->device() != device) Py_RETURN_NONE;
+  if (state && (!has_shape(*state, {B, Hv, D, D}) || !state->is_contiguous() || !aligned(at_of(*state), 16) || state->device() != device))
+    Py_RETURN_NONE;
   if (cs && (cs->scalar_type() != type || !has_shape(*cs, {B, 3, C}) || cs->device() != device || !cs->is_contiguous() ||
              !aligned(at_of(*cs), 8)))
     Py_RETURN_NONE;
@@ -506,7 +508,7 @@ PyObject* gdn_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Py_RETURN_NONE;
   dflash_gdn_block_args p = {};
   p.qkv = at_of(*qkv), p.conv_state = cs ? at_of(*cs) : nullptr, p.conv_w = at_of(*w), p.a = at_of(*ga), p.b = at_of(*gb);
-  p.A_log = at_of(*A), p.dt_bias = at_of(*dt), p.state_in = at_of(*state);
+  p.A_log = at_of(*A), p.dt_bias = at_of(*dt);
   p.qkv_slot = qkv->stride(0), p.qkv_row = qkv->stride(1), p.a_slot = ga->stride(0), p.a_row = ga->stride(1);
   p.b_slot = gb->stride(0), p.b_row = gb->stride(1);
   if (z) p.z = at_of(*z), p.norm_weight = at_of(*weight), p.z_slot = z->stride(0), p.z_row = z->stride(1);
@@ -514,9 +516,11 @@ PyObject* gdn_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
   p.weight_dtype = z ? dtype_code(weight->scalar_type()) : DFLASH_BF16;
   p.eps = (float)PyFloat_AS_DOUBLE(a[14]), p.norm_eps = (float)PyFloat_AS_DOUBLE(a[15]);
   void* stream = stream_of(*qkv);
-  Tensor y, next, conv, tape, k, g, one;
+  Tensor y, next, conv, tape, k, g, one, zeros;
   const int rc = released([&] {
     const auto options = qkv->options();
+    if (!state) zeros = at::zeros({B, Hv, D, D}, options), state = &zeros;
+    p.state_in = at_of(*state);
     y = at::empty({B, S, Hv, D}, options);
     next = at::empty({B, Hv, D, D}, state->options());
     conv = at::empty({B, 3, C}, options);

@@ -257,12 +257,10 @@ def _gdn_call(self, inputs: torch.Tensor, mask: Optional[torch.Tensor], cache: O
     normed = isinstance(norm, RMSNormGated) and _native.env(b"DFLASH_GDN_FUSED_NORM") != b"0"
     if mask is None and S <= 16 and qkv.is_cuda:
         # a block: conv, gates, recurrence and norm in one launch, where there is one for these sizes and types
-        state = cache[1] if cache is not None else None
-        if state is None:
-            state = torch.zeros((B, self.num_v_heads, self.head_v_dim, self.head_k_dim), dtype=qkv.dtype, device=qkv.device)
         made = _native.host().gdn_block(
             qkv, conv_state, self.conv1d.weight, a, b, self.A_log, self.dt_bias, z if normed else None, norm.weight if normed else None,
-            state, self.num_k_heads, self.num_v_heads, self.head_k_dim, self.head_v_dim, 1e-6, norm.eps if normed else 0.0, bool(record))
+            cache[1] if cache is not None else None, self.num_k_heads, self.num_v_heads, self.head_k_dim, self.head_v_dim, 1e-6,
+            norm.eps if normed else 0.0, bool(record))
         if made is not None:
             out, state, conv_next, tape, k, g, tape_qkv = made
             if cache is not None:

@@ -452,3 +452,20 @@ def test_operands_that_start_on_any_element(native_lib, dtype, S, armed, shifted
         for a, b in zip(run(shifted, state), run("neither", state)):
             assert (a is None) == (b is None)
             assert a is None or (a.shape == b.shape and a.dtype == b.dtype and torch.equal(a, b))
+
+
+def test_a_first_block_makes_its_zeros_once(native_lib, monkeypatch):
+    """A block that starts from nothing has its state of zeros filled once, also where the launch of the whole block declines it."""
+    filled = []
+    real = torch.zeros
+    monkeypatch.setattr(torch, "zeros", lambda *a, **kw: (filled.append(a), real(*a, **kw))[1])
+    for dtype, K in ((torch.float32, 4), (torch.bfloat16, 3), (torch.bfloat16, 4)):
+        parts = [torch.randn((1, 5, n), device=DEV).to(dtype) for n in (512, 256, 2, 2)]
+        mixer = G.GatedDeltaNet(8, num_k_heads=1, num_v_heads=2, head_k_dim=128, head_v_dim=128, in_proj_qkv=_Given(parts[0]),
+                                in_proj_z=_Given(parts[1]), in_proj_b=_Given(parts[2]), in_proj_a=_Given(parts[3]),
+                                out_proj=torch.nn.Identity(), conv_kernel_size=K, dtype=dtype).to(DEV)
+        x = torch.randn((1, 5, 8), device=DEV).to(dtype)
+        cache = RecurrentRollbackCache(size=2, conv_kernel_size=K)
+        del filled[:]
+        mixer(x, cache=cache)
+        assert len(filled) <= 1 and cache[1].dtype == dtype, (dtype, K, filled)
