@@ -28,13 +28,13 @@
 //    Of more tiles than the chip takes at once, only those of the last, incomplete round are cut.
 //
 // Measured (us, group 64; before: 16 x 16 x 32 instructions, loads to registers): 1024 rows of 5120 x 34816 with the
-// activation 398 -> 344 (1.06 PFLOP/s), 17408 x 5120 207 -> 184, 5120 x 12352 164 -> 134; 200 rows of 4096 x 4096 22.6 -> 17.5; 77 rows
-// of 4096 x 24576 with the activation 36.4 -> 30.8, 12288 x 4096 24.9 -> 21.2; 20 rows of 5120 x 12352 21.4 -> 18.4, of 2048 x 2048 7.1 -> 7.4.
+// activation 398 -> 335 (1.09 PFLOP/s), 17408 x 5120 207 -> 184, 5120 x 12352 164 -> 134; 200 rows of 4096 x 4096 22.6 -> 17.5; 77 rows
+// of 4096 x 24576 with the activation 35.7 -> 29.0, 12288 x 4096 24.9 -> 20.9; 20 rows of 5120 x 12352 21.4 -> 18.4, of 2048 x 2048 7.1 -> 7.4.
 // What bounds it at many rows: the matrix pipes are busy for 60 to 66 % of the cycles at 2.0 to 2.1 of 2.4 GHz (power); with no requests
 // to memory at all the same loop is 15 to 20 % faster, with no dequantisation on top 2 to 10 %.  At few rows:
 // 3300 cycles of setup, requests and their latency before the first product, 1500 a stage of (1,1,2,4), where four dependent steps take 1050 and
 // the barrier the rest, and 5000 and more for the slices.
-#include "dflash_common.h"
+#include "glue_device.h"
 
 #include "qmm_stream_device.h"
 #include <algorithm>
@@ -417,7 +417,7 @@ __global__ __launch_bounds__(64 * W * KG, 2) void qmm_rows_kernel(Args a) {
         o[h] = v[0][r >> 2][r & 3];
         if constexpr (SILU_MUL) {
           const float g = round16<FP16>(o[h]), u = round16<FP16>(v[kTiles - 1][r >> 2][r & 3]);
-          const float sg = round16<FP16>(1.0f / (1.0f + expf(-g)));
+          const float sg = round16<FP16>(sigmoid_of_half(g));
           o[h] = round16<FP16>(g * sg) * u;
         }
       }
@@ -575,7 +575,7 @@ Plan make_plan(int M, int K, int N, int cus, bool fp16, bool mixed, bool silu_mu
     const int rounds = p.whole / slots;
     double us = stretch(rounds * sh.together, p.stages) + stretch(ceil_div(parts, cus), ceil_div(p.stages, p.slices));
     us *= 1 + 0.17 * (std::min(1.0, (double)p.grid / cus) - 0.5);
-    us += 0.88 + (silu_mul ? 2.02 : 0.0);
+    us += 0.88 + (silu_mul ? 0.79 : 0.0);
     const int pieces = silu_mul ? sh.mt : sh.mt * sh.nt, at_once = silu_mul && (sh.mt == 1 || sh.mt == 4) ? 2 : 4;
     if (p.slices > 1)
       us += 0.94 + 0.715 * ceil_div(pieces, sh.kg) * ceil_div(p.slices, at_once) + 0.392 * parts * (sh.rows() * 8.0 * sh.columns()) / 3e6;
