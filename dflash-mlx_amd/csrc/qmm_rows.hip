@@ -29,7 +29,9 @@
 //
 // Measured (us, group 64; before: 16 x 16 x 32 instructions, loads to registers): 1024 rows of 5120 x 34816 with the
 // activation 398 -> 335 (1.09 PFLOP/s), 17408 x 5120 207 -> 184, 5120 x 12352 164 -> 134; 200 rows of 4096 x 4096 22.6 -> 17.5; 77 rows
-// of 4096 x 24576 with the activation 35.7 -> 29.0, 12288 x 4096 24.9 -> 20.9; 20 rows of 5120 x 12352 21.4 -> 18.4, of 2048 x 2048 7.1 -> 7.4.
+// of 4096 x 24576 with the activation 35.7 -> 29.0, 12288 x 4096 24.9 -> 20.9; 20 rows of 5120 x 12352 21.4 -> 18.3, of 1024 x 1024 5.9 -> 5.7.
+// Still slower than that form: 17 to 32 rows of squares of 2048 to 5120 4 to 6 %, 17 to 48 rows of 5120 x 34816 with the activation
+// 2 to 9 % (40 rows 40.4 -> 43.9), 77 to 128 rows of 3072 x 1024 6 to 9 %.
 // What bounds it at many rows: the matrix pipes are busy for 60 to 66 % of the cycles at 2.0 to 2.1 of 2.4 GHz (power); with no requests
 // to memory at all the same loop is 15 to 20 % faster, with no dequantisation on top 2 to 10 %.  At few rows:
 // 3300 cycles of setup, requests and their latency before the first product, 1500 a stage of (1,1,2,4), where four dependent steps take 1050 and
@@ -510,13 +512,15 @@ struct Shape {
   int mt, nt, w, kg, lds;
   int together;        // workgroups that a CU has room for
   double alone, busy;  // us per stage: of one workgroup on a CU, and of each where they share it
+  double start;        // us before the first product and behind the last one
+  int most;            // slices
   const void* kernel[2][3];  // [fp16][plain, scales of the other type, silu-mul]; null: there is none
   int rows() const { return 32 * mt; }
   int columns() const { return 32 * nt * w; }
 };
 template <int MT, int NT, int W, int KG, bool MIXED = false>
-Shape shape(int together, double alone, double busy) {
-  Shape s{MT, NT, W, KG, Tile<MT, NT, W, KG>::kLdsBytes, together, alone, busy, {}};
+Shape shape(int together, double alone, double busy, double start = 4.47, int most = 16) {
+  Shape s{MT, NT, W, KG, Tile<MT, NT, W, KG>::kLdsBytes, together, alone, busy, start, most, {}};
   s.kernel[0][0] = (const void*)qmm_rows_kernel<false, false, MT, NT, W, KG, false>;
   s.kernel[1][0] = (const void*)qmm_rows_kernel<true, true, MT, NT, W, KG, false>;
   if constexpr (MIXED) {
@@ -530,15 +534,19 @@ Shape shape(int together, double alone, double busy) {
   return s;
 }
 // (1,1,4,2), (2,1,4,2), (3,1,4,2), (4,1,4,2), (2,2,2,2), (2,2,4,2), (3,2,4,1), (2,2,8,1) and (4,2,8,1) were measured as well:
-// without them the best of the rest is 0.3 % slower on average.
-constexpr int kShapes = 14;
+// without them the best of the rest is 0.3 % slower on average.  The last four, of four waves side by side along K, start and end sooner
+// than eight waves do, which is most of a call of few rows and weights (20 rows, us, without / with them: 1024 x 1024 6.5 / 5.7, 3072 x 1024
+// 8.6 / 7.7, with the activation 1024 x 6144 9.0 / 7.3; 40 rows 9.5 / 8.0 and 10.5 / 7.6).
+constexpr int kShapes = 18;
 const Shape* shapes() {
   static const Shape all[kShapes] = {
       shape<1, 1, 1, 8>(1, 0.600, 0.571),       shape<2, 1, 1, 8>(1, 0.925, 0.454),
       shape<1, 1, 2, 4, true>(2, 0.540, 0.472), shape<2, 1, 2, 4>(1, 0.709, 0.447),       shape<3, 1, 2, 4>(1, 0.910, 0.307),
       shape<1, 2, 2, 4>(1, 0.924, 0.508),       shape<2, 2, 2, 4, true>(1, 1.100, 0.401), shape<3, 2, 2, 4>(1, 1.367, 0.390),
       shape<1, 2, 4, 2>(2, 0.905, 0.750),       shape<3, 2, 4, 2>(1, 1.274, 0.363),       shape<4, 2, 4, 2, true>(1, 1.533, 0.524),
-      shape<4, 2, 2, 2>(1, 0.879, 0.546),       shape<2, 2, 4, 1>(2, 0.650, 0.535),       shape<4, 2, 4, 1>(2, 0.834, 0.767)};
+      shape<4, 2, 2, 2>(1, 0.879, 0.546),       shape<2, 2, 4, 1>(2, 0.650, 0.535),       shape<4, 2, 4, 1>(2, 0.834, 0.767),
+      shape<1, 1, 1, 4>(3, 0.438, 0.310, 3.78, 6), shape<2, 1, 1, 4>(2, 0.591, 0.445, 3.64, 6),
+      shape<1, 2, 1, 4>(2, 0.676, 0.472, 3.89, 6), shape<2, 2, 1, 4>(1, 0.804, 0.626, 4.54, 6)};
   return all;
 }
 
@@ -560,6 +568,9 @@ bool covers(int M, int K, int N, int group_size, bool mixed, int epilogue) {
 // weights, 20 to 1024 rows; the 2053 within 30 % of the best of their call: 5 % rms, and what it picks is within 0.5 % of the best on
 // average, 12 % at worst).  A workgroup takes `alone` for a stage, or `busy` times those that share its CU; a chip that is full runs
 // against its power.  Adding slices up takes trips to memory and traffic at 3 TB/s and more.
+// The four shapes of the last lines were fitted beside the others as they were (42 matrices, 20 to 1024 rows), their constants
+// 7 % up, so that one is taken only where it is the faster: of 420 calls 1 takes longer than without them (1536 x 8448 with the
+// activation, 96 rows, 12.5 -> 13.1 us), the mean of all is 2 % less, of up to 64 rows 3 %.
 // Slices only while all of them find room at once.  Of more tiles than that, those of the last, incomplete round may be
 // cut, with the tile left as it is (5120 x 34816 over 1024 rows: 1088 tiles, two to a CU, the last 64 in slices, 344 us; uncut 382).
 Plan make_plan(int M, int K, int N, int cus, bool fp16, bool mixed, bool silu_mul) {
@@ -570,7 +581,7 @@ Plan make_plan(int M, int K, int N, int cus, bool fp16, bool mixed, bool silu_mu
     const int slots = cus * sh.together, parts = p.grid - p.whole;
     auto stretch = [&](int on_a_cu, int stages) {  // workgroups one after the other and beside each other
       const int rounds = ceil_div(on_a_cu, sh.together);
-      return rounds * 4.47 + stages * std::max(sh.alone * rounds, sh.busy * on_a_cu);
+      return rounds * sh.start + stages * std::max(sh.alone * rounds, sh.busy * on_a_cu);
     };
     const int rounds = p.whole / slots;
     double us = stretch(rounds * sh.together, p.stages) + stretch(ceil_div(parts, cus), ceil_div(p.stages, p.slices));
@@ -593,9 +604,9 @@ Plan make_plan(int M, int K, int N, int cus, bool fp16, bool mixed, bool silu_mu
     if (tiles > 0x7fffffff / 16) continue;
     p.tiles = (int)tiles;
     p.stages = ceil_div(K, kStageK * sh.kg);
-    const int slots = cus * sh.together, most = sh.kg == 1 ? 4 : 16;
+    const int slots = cus * sh.together, most = sh.kg == 1 ? 4 : sh.most;
     const int rest = p.tiles % slots;
-    for (p.slices = 1; p.slices <= 16 && p.slices <= p.stages; ++p.slices) {
+    for (p.slices = 1; p.slices <= sh.most && p.slices <= p.stages; ++p.slices) {
       const bool all = p.tiles < slots;
       if (p.slices > 1 && (all ? p.tiles * p.slices > slots || p.slices > most : rest == 0 || rest * p.slices > 2 * slots)) break;
       p.whole = p.tiles - rest;

@@ -195,3 +195,17 @@ def test_activation_takes_the_bits_of_the_array_operators(native_lib):
         assert torch.equal(torch.cat([gate, up], dim=-1), dequantize(c.w, c.scales, c.biases, 64, 4, dtype=dtype).t())
         h = rows_matmul(x, c.w, c.scales, c.biases, epilogue="silu_mul")
         assert torch.equal(h, (gate * torch.sigmoid(gate)) * up)
+
+
+# the shapes of eight waves at the sizes where those of four do not serve, each whole and sliced where it is taken so
+MORE_SHAPES = [(17, 1440, 16, 32), (33, 6080, 80, 32), (17, 1056, 8368, 32), (17, 4160, 2768, 32), (33, 2464, 4272, 32), (33, 672, 8224, 32),
+               (33, 3168, 4112, 32), (97, 288, 8592, 32), (33, 2880, 8336, 32), (65, 288, 11024, 32), (65, 2880, 2784, 32), (130, 480, 10976, 32),
+               (65, 2880, 8208, 32), (17, 6080, 8224, 32), (17, 2880, 8240, 32), (33, 1632, 432, 32), (17, 3168, 16, 32), (17, 288, 32832, 32)]
+MORE_SHAPES_SILU = [(65, 2464, 8416, 32), (17, 3552, 11488, 32), (65, 288, 11040, 32), (33, 3168, 992, 32), (130, 480, 10912, 32), (65, 3168, 1376, 32),
+                    (17, 2080, 32, 32), (33, 1632, 608, 32), (33, 288, 8224, 32), (17, 288, 32960, 32)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,K,N,group,silu", [(*t, False) for t in MORE_SHAPES] + [(*t, True) for t in MORE_SHAPES_SILU])
+def test_tile_shapes_of_four_and_eight_waves(native_lib, M, K, N, group, silu, dtype):
+    test_every_tile_shape_at_its_edges(native_lib, M, K, N, group, silu, dtype)
