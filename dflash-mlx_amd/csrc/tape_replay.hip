@@ -452,6 +452,9 @@ __global__ __launch_bounds__(kThreads) void replay_rows(ReplayArgs a) {
 // The form of replay_rows for a head size and state type; rows: how many a workgroup computes.  heads: of all slots.  The lines
 // of the fp32 states (16 bf16 steps, us with one / two / four / eight rows of a pass): 128 x 128, 32 heads 4.5 / 4.4 / 5.1 / 7.2,
 // 192 heads 8.9 / 6.9 / 7.3 / 8.6, 256 heads 11.0 / 7.9 / 7.9 / 9.7, 384 heads 14.9 / 11.6 / 9.8 / 11.2, 1536 heads 42.6 / 39.5 / 37.2 / 39.9;
+// eight rows also where they are one round of the chip and four rows a second one (two and three such workgroups fit a compute unit): 416 heads
+// 15.9 / 13.6 / 13.3 / 11.4, 512 heads 17.6 / 15.4 / 14.3 / 12.8, 544 heads 18.6 / 16.2 / 15.7 / 17.1 (fp32 tapes, four and eight rows: 416 heads
+// 13.5 / 12.0, 512 heads 14.6 / 13.7; a head per workgroup on the matrix cores 13.0 and 13.7).
 // 64 x 64, 32 heads 3.5 / 4.0, 96 heads 4.1 / 4.2, 256 heads 5.1 / 4.5, 1536 heads 13.8 / 11.8.  Of the 16-bit ones: a whole head per
 // workgroup from 1024 heads on, where k is staged once for more rows, but at 16 steps fewer waves cover each other's waits (128 x 128, 16 / 6
 // steps, us, split and whole: 512 heads 16.0 / 10.0 and 19.3 / 10.3, 1024 heads 28.6 / 16.8 and 31.9 / 15.4, 1536 heads 41.6 / 25.4
@@ -461,6 +464,8 @@ const void* replay_rows_for(int Dk, int Dv, long long heads, int* rows) {
   constexpr bool kWide = STATE == DFLASH_FP32;
   const bool many = kWide ? heads > (Dk == 128 ? 192 : 96) : heads >= 1024;
   constexpr int kMany = kWide ? 4 : 8;
+  if (kWide && Dk == 128 && Dv % 128 == 0 && heads * (Dv / 64) > 3 * 256 && heads * (Dv / 128) <= 2 * 256)
+    return *rows = 128, (const void*)replay_rows<STATE, 128, 8>;
   if (Dk == 128 && many && Dv % (16 * kMany) == 0) return *rows = 16 * kMany, (const void*)replay_rows<STATE, 128, kMany>;
   if (Dk == 128 && Dv % 32 == 0) return *rows = 32, (const void*)replay_rows<STATE, 128, 2>;
   if (Dk == 64 && many && Dv % 64 == 0) return *rows = 64, (const void*)replay_rows<STATE, 64, 2>;

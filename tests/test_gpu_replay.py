@@ -458,3 +458,20 @@ def test_a_slot_alone_and_among_many(native_lib, D, slots):
         one = torch.empty_like(d.state[s:s + 1])
         replay_launch(d.tape[s:s + 1], d.k[s:s + 1], d.g[s:s + 1], d.state[s:s + 1], one, steps=int(steps[s]), T_alloc=16, slots=1)
         assert torch.equal(one[0], out[s]), s
+
+
+@pytest.mark.parametrize("slots", [12, 13, 16, 17])
+@pytest.mark.parametrize("tape_dt", [torch.float32, torch.bfloat16])
+def test_heads_that_fit_the_chip_in_one_round(native_lib, slots, tape_dt):
+    """fp32 states of 128 x 128: whole heads per workgroup from 385 to 512 heads, the same bits as a slot alone."""
+    case = make_replay_case(slots, Hk=16, Hv=32, Dk=128, Dv=128, steps=16, seed=60 + slots, tape_dtype=tape_dt)
+    steps = torch.tensor([(5 * s) % 17 for s in range(slots)], dtype=torch.int32)
+    out = _launch(case, steps)
+    d = case.to(DEV)
+    for s in range(slots):
+        one = torch.empty_like(d.state[s:s + 1])
+        replay_launch(d.tape[s:s + 1], d.k[s:s + 1], d.g[s:s + 1], d.state[s:s + 1], one, steps=int(steps[s]), T_alloc=16, slots=1)
+        assert torch.equal(one[0], out[s]), s
+    want = _oracle_slots(case, steps.numpy())
+    for s in (0, slots - 1):
+        assert _rel_l2(_np(out).reshape(slots, -1)[s], want.reshape(slots, -1)[s]) <= TOL, s
