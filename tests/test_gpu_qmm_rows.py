@@ -34,7 +34,7 @@ def test_rows_against_fp64(native_lib, M, K, N, group, dtype):
     assert (y.double() - exact).norm() <= eps * exact.norm()
 
 
-# a call for every tile shape there is: K that ends inside a stage, N and M that end inside a tile, whole and sliced
+# (with MORE_SHAPES) a call for every tile shape there is: K that ends inside a stage, N and M that end inside a tile, whole and sliced
 TILE_SHAPES = [(17, 288, 16, 32), (17, 2080, 48, 32), (20, 96, 528, 32), (17, 160, 8208, 32), (17, 96, 6160, 32), (33, 288, 2064, 32),
                (45, 96, 2064, 32), (33, 160, 12432, 32), (65, 160, 3088, 32), (129, 160, 6160, 32), (129, 96, 12432, 32), (65, 96, 1552, 32),
                (400, 160, 8208, 32), (300, 96, 12432, 32), (97, 4416, 2064, 64), (200, 3136, 1552, 64), (1000, 1664, 5136, 128)]
@@ -197,12 +197,14 @@ def test_activation_takes_the_bits_of_the_array_operators(native_lib):
         assert torch.equal(h, (gate * torch.sigmoid(gate)) * up)
 
 
-# the shapes of eight waves at the sizes where those of four do not serve, each whole and sliced where it is taken so
+# the shapes of more than four waves at the sizes where those of four do not serve, and those of four, whole and sliced
 MORE_SHAPES = [(17, 1440, 16, 32), (33, 6080, 80, 32), (17, 1056, 8368, 32), (17, 4160, 2768, 32), (33, 2464, 4272, 32), (33, 672, 8224, 32),
                (33, 3168, 4112, 32), (97, 288, 8592, 32), (33, 2880, 8336, 32), (65, 288, 11024, 32), (65, 2880, 2784, 32), (130, 480, 10976, 32),
-               (65, 2880, 8208, 32), (17, 6080, 8224, 32), (17, 2880, 8240, 32), (33, 1632, 432, 32), (17, 3168, 16, 32), (17, 288, 32832, 32)]
+               (65, 2880, 8208, 32), (17, 6080, 8224, 32), (17, 2880, 8240, 32), (33, 1632, 432, 32), (17, 3168, 16, 32), (17, 288, 32832, 32),
+               (600, 288, 8224, 32), (400, 480, 13232, 32)]
 MORE_SHAPES_SILU = [(65, 2464, 8416, 32), (17, 3552, 11488, 32), (65, 288, 11040, 32), (33, 3168, 992, 32), (130, 480, 10912, 32), (65, 3168, 1376, 32),
-                    (17, 2080, 32, 32), (33, 1632, 608, 32), (33, 288, 8224, 32), (17, 288, 32960, 32)]
+                    (17, 2080, 32, 32), (33, 1632, 608, 32), (33, 288, 8224, 32), (17, 288, 32960, 32),
+                    (400, 480, 13120, 32)]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
