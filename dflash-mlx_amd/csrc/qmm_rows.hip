@@ -514,15 +514,17 @@ struct Shape {
   double alone, busy;  // us per stage: of one workgroup on a CU, and of each where they share it
   double start;        // us before the first product and behind the last one
   int most;            // slices
-  const void* kernel[2][3];  // [fp16][plain, scales of the other type, silu-mul]; null: there is none
+  const void* kernel[2][3];  // [fp16][plain, scales of the other type, silu-mul]; null: there is none, or it was never the one to take
   int rows() const { return 32 * mt; }
   int columns() const { return 32 * nt * w; }
 };
-template <int MT, int NT, int W, int KG, bool MIXED = false>
+template <int MT, int NT, int W, int KG, bool MIXED = false, bool PLAIN = true>
 Shape shape(int together, double alone, double busy, double start = 4.47, int most = 16) {
   Shape s{MT, NT, W, KG, Tile<MT, NT, W, KG>::kLdsBytes, together, alone, busy, start, most, {}};
-  s.kernel[0][0] = (const void*)qmm_rows_kernel<false, false, MT, NT, W, KG, false>;
-  s.kernel[1][0] = (const void*)qmm_rows_kernel<true, true, MT, NT, W, KG, false>;
+  if constexpr (PLAIN) {
+    s.kernel[0][0] = (const void*)qmm_rows_kernel<false, false, MT, NT, W, KG, false>;
+    s.kernel[1][0] = (const void*)qmm_rows_kernel<true, true, MT, NT, W, KG, false>;
+  }
   if constexpr (MIXED) {
     s.kernel[0][1] = (const void*)qmm_rows_kernel<false, true, MT, NT, W, KG, false>;
     s.kernel[1][1] = (const void*)qmm_rows_kernel<true, false, MT, NT, W, KG, false>;
@@ -546,7 +548,7 @@ const Shape* shapes() {
       shape<1, 2, 4, 2>(2, 0.905, 0.750),       shape<3, 2, 4, 2>(1, 1.274, 0.363),       shape<4, 2, 4, 2, true>(1, 1.533, 0.524),
       shape<4, 2, 2, 2>(1, 0.879, 0.546),       shape<2, 2, 4, 1>(2, 0.650, 0.535),       shape<4, 2, 4, 1>(2, 0.834, 0.767),
       shape<1, 1, 1, 4>(3, 0.438, 0.310, 3.78, 6), shape<2, 1, 1, 4>(2, 0.591, 0.445, 3.64, 6),
-      shape<1, 2, 1, 4>(2, 0.676, 0.472, 3.89, 6), shape<2, 2, 1, 4>(1, 0.804, 0.626, 4.54, 6)};
+      shape<1, 2, 1, 4>(2, 0.676, 0.472, 3.89, 6), shape<2, 2, 1, 4, false, false>(1, 0.804, 0.626, 4.54, 6)};
   return all;
 }
 
