@@ -37,8 +37,8 @@ HBM_PEAK = 8.0e12  # bytes/s, MI355X HBM3E
 # for a 1 GiB copy) kept under profiles/, which also states the SHA-256 of the kernel's source
 # files as they were when the counters were taken.  If the sources have changed since, the figure
 # describes another kernel and is not reported.
-TRAFFIC_PROFILES = {"27b": "profiles/qmm_stream_kernel_27b_stack_pmc.txt"}
-KERNEL_SOURCES = ("dflash-mlx_amd/csrc/qmm_m16_stream.hip", "dflash-mlx_amd/csrc/qmm_stream_device.h")
+TRAFFIC_PROFILES = {"27b": "profiles/qmm_resident_kernel_27b_stack_pmc.txt"}
+KERNEL_SOURCES = ("dflash-mlx_amd/csrc/qmm_resident.h", "dflash-mlx_amd/csrc/qmm_resident.hip", "dflash-mlx_amd/csrc/qmm_stream_device.h")
 
 
 def kernel_sources_sha256() -> str:
@@ -1065,7 +1065,7 @@ def main() -> int:
     roofline = dict(bound="hbm", achieved=round(achieved, 1), peak=HBM_PEAK / 1e9, unit="GB/s",
                     frac=round(achieved * 1e9 / HBM_PEAK, 4),
                     traffic=traffic, traffic_source=traffic_source,
-                    kernel="qmm_stream_kernel", bytes_per_launch=round(main_res["bytes_per_launch"]),
+                    kernel="qmm_resident_kernel", bytes_per_launch=round(main_res["bytes_per_launch"]),
                     avg_launch_us=round(main_res["avg_launch_us"], 3))
     cpu = None if args.skip_cpu else bench_cpu_baseline(args.workload)
 

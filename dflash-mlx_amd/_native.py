@@ -18,17 +18,17 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libdflash_mi355.so")
 HOST_PATH = os.path.join(_HERE, "_dflash_host.so")
 
-ABI_VERSION = 23
+ABI_VERSION = 24
 
 BF16, FP16, FP32 = 0, 1, 2
 QMM_MMA2BIG, QMM_MMA2BIG_PIPE = 0, 1
-QMM_KERNEL_AUTO, QMM_KERNEL_TILE, QMM_KERNEL_STREAM = 0, 1, 2
+QMM_KERNEL_AUTO, QMM_KERNEL_TILE, QMM_KERNEL_STREAM, QMM_KERNEL_FASTEST = 0, 1, 2, 3
 QMM_STATIC_SCRATCH_BYTES = 8 << 20  # DFLASH_QMM_STATIC_SCRATCH_BYTES
 QMM_CHAIN_MAX = 16                       # DFLASH_QMM_CHAIN_MAX
 QMM_ERROR_OFFSET = (16384 - 64 + 1) * 4        # DFLASH_QMM_ERROR_OFFSET
 QMM_CHAIN_ERROR_OFFSET = QMM_ERROR_OFFSET      # DFLASH_QMM_CHAIN_ERROR_OFFSET
 QMM_EPILOGUE_NONE, QMM_EPILOGUE_SILU_MUL = 0, 1
-QMM_CHAIN_JOINT_SPLIT = 1                # DFLASH_QMM_CHAIN_JOINT_SPLIT
+QMM_CHAIN_JOINT_SPLIT, QMM_CHAIN_FASTEST = 1, 4  # DFLASH_QMM_CHAIN_*
 QMM_LAYOUT_ROWS, QMM_LAYOUT_PACKED = 0, 1  # DFLASH_QMM_LAYOUT_*
 OPT_GDN_STEP_BY_STEP, OPT_SDPA_SPLITS, OPT_QMM_SPIN_LIMIT = 0, 1, 2  # DFLASH_OPT_*
 
@@ -50,6 +50,7 @@ EXPORTED_SYMBOLS = (
     "dflash_qmm_few",
     "dflash_qmm_few_silu_mul_workspace_bytes",
     "dflash_qmm_few_silu_mul",
+    "dflash_qmm_few_silu_mul_by",
     "dflash_qmm_error",
     "dflash_qmm_m16_static",
     "dflash_qmm_m16_pack_gate_up",
@@ -111,6 +112,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.dflash_qmm_few_silu_mul_workspace_bytes.argtypes = [c.c_int] * 3
     lib.dflash_qmm_few_silu_mul.restype = c.c_int
     lib.dflash_qmm_few_silu_mul.argtypes = [c.c_void_p] * 6 + [c.c_size_t] + [c.c_int] * 5 + [c.c_void_p]
+    lib.dflash_qmm_few_silu_mul_by.restype = c.c_int
+    lib.dflash_qmm_few_silu_mul_by.argtypes = [c.c_void_p] * 6 + [c.c_size_t] + [c.c_int] * 6 + [c.c_void_p]
     lib.dflash_qmm_error.restype = c.c_int
     lib.dflash_qmm_error.argtypes = [c.c_void_p, c.POINTER(c.c_uint32), c.c_void_p]
     lib.dflash_qmm_m16_static.restype = c.c_int

@@ -194,21 +194,22 @@ PyObject* qmm_few(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// qmm_few_silu_mul(x, w, scales, biases, group_size, workspaces): the gated activation of 1 to 16 rows.
+// qmm_few_silu_mul(x, w, scales, biases, group_size, kernel, workspaces): the gated activation of 1 to 16 rows.
 PyObject* qmm_few_silu_mul(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   Product p;
-  if (n != 6 || !product_of(a, &p) || p.rows > 16 || p.act != p.sb) Py_RETURN_NONE;
+  int kernel;
+  if (n != 7 || !product_of(a, &p) || p.rows > 16 || p.act != p.sb || !integer(a[5], &kernel)) Py_RETURN_NONE;
   if (!aligned(at_of(*p.x), 16) || !aligned(at_of(*p.w), 16) || !aligned(at_of(*p.s), 4) || !aligned(at_of(*p.b), 4)) Py_RETURN_NONE;
   const size_t need = dflash_qmm_few_silu_mul_workspace_bytes(p.K, p.N, p.group);
   if (need == 0) Py_RETURN_NONE;
   void* stream = stream_of(*p.x);
-  Tensor y, ws = kept_workspace(a[5], by_index(*p.x, stream), need);
+  Tensor y, ws = kept_workspace(a[6], by_index(*p.x, stream), need);
   if (!ws.defined()) Py_RETURN_NONE;
   const int rc = released([&] {
     y = at::empty(rows_by(*p.x, p.N / 2), p.x->options());
-    return dflash_qmm_few_silu_mul(at_of(*p.x), (const uint32_t*)at_of(*p.w), at_of(*p.s), at_of(*p.b), y.mutable_data_ptr(),
-                                   ws.mutable_data_ptr(), ws.nbytes(), (int)p.rows, p.K, p.N, p.group, p.act, stream);
+    return dflash_qmm_few_silu_mul_by(at_of(*p.x), (const uint32_t*)at_of(*p.w), at_of(*p.s), at_of(*p.b), y.mutable_data_ptr(),
+                                   ws.mutable_data_ptr(), ws.nbytes(), (int)p.rows, p.K, p.N, p.group, p.act, kernel, stream);
   });
   return rc != 0 ? fail(rc, "dflash_qmm_few_silu_mul") : THPVariable_Wrap(std::move(y));
   END_HANDLE_TH_ERRORS

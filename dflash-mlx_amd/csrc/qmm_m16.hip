@@ -436,6 +436,11 @@ bool qmm_stream_packed_eligible(int K, int N, int group_size);
 bool qmm_narrow_covers(const void* scales, const void* biases, int K, int N, int group_size, bool silu_mul);
 int qmm_narrow_launch(const void* x, const void* w, const void* scales, const void* biases, void* y, int M, int K, int N, int group_size,
                       int act_dtype, int sb_dtype, bool silu_mul, bool packed, hipStream_t stream);
+// qmm_resident.hip: x and w 16-byte aligned, up to 16 rows
+bool qmm_resident_covers(const void* scales, const void* biases, size_t workspace_bytes, int K, int N, int group_size, int act_dtype,
+                         int sb_dtype);
+int qmm_resident_launch(const void* x, const void* w, const void* scales, const void* biases, void* y, void* workspace, int M, int K,
+                        int N, int group_size, int dtype, bool silu_mul, bool packed, int spin_limit, hipStream_t stream);
 void qmm_stream_packed_bytes(int K, int N, size_t* w_bytes, size_t* sb_bytes);
 int qmm_stream_pack(const uint32_t* w, const void* scales, const void* biases, void* w_out,
                     void* s_out, void* b_out, int K, int N, hipStream_t stream);
@@ -503,7 +508,16 @@ extern "C" size_t dflash_qmm_few_silu_mul_workspace_bytes(int K, int N, int grou
 extern "C" int dflash_qmm_few_silu_mul(const void* x, const uint32_t* w_q, const void* scales, const void* biases, void* y,
                                        void* workspace, size_t workspace_bytes, int M, int K, int N, int group_size,
                                        int dtype, void* stream) {
+  return dflash_qmm_few_silu_mul_by(x, w_q, scales, biases, y, workspace, workspace_bytes, M, K, N, group_size, dtype,
+                                    DFLASH_QMM_KERNEL_AUTO, stream);
+}
+
+extern "C" int dflash_qmm_few_silu_mul_by(const void* x, const uint32_t* w_q, const void* scales, const void* biases,
+                                          void* y, void* workspace, size_t workspace_bytes, int M, int K, int N,
+                                          int group_size, int dtype, int kernel, void* stream) {
   using namespace dflash;
+  DFLASH_REQUIRE(kernel == DFLASH_QMM_KERNEL_AUTO || kernel == DFLASH_QMM_KERNEL_FASTEST, DFLASH_ERR_ARG,
+                 "dflash_qmm_few_silu_mul: kernel %d has no form with the activation", kernel);
   DFLASH_REQUIRE(x && w_q && scales && biases && y, DFLASH_ERR_ARG, "dflash_qmm_few_silu_mul: null operand");
   DFLASH_REQUIRE(dtype == DFLASH_BF16 || dtype == DFLASH_FP16, DFLASH_ERR_ARG, "dflash_qmm_few_silu_mul: dtype %d is not bf16/fp16",
                  dtype);
@@ -512,6 +526,9 @@ extern "C" int dflash_qmm_few_silu_mul(const void* x, const uint32_t* w_q, const
                  "dflash_qmm_few_silu_mul: the streaming kernel does not cover K=%d N=%d gs=%d", K, N, group_size);
   DFLASH_REQUIRE((((uintptr_t)x | (uintptr_t)w_q) % 16) == 0 && (((uintptr_t)scales | (uintptr_t)biases) % 4) == 0,
                  DFLASH_ERR_ARG, "dflash_qmm_few_silu_mul: x and w_q must be 16-byte aligned, scales and biases 4-byte aligned");
+  if (kernel == DFLASH_QMM_KERNEL_FASTEST && qmm_resident_covers(scales, biases, workspace_bytes, K, N, group_size, dtype, dtype) &&
+      qmm_stream_workspace_given(workspace, workspace_bytes, K, N))
+    return qmm_resident_launch(x, w_q, scales, biases, y, workspace, M, K, N, group_size, dtype, true, false, 0, (hipStream_t)stream);
   if (qmm_narrow_covers(scales, biases, K, N, group_size, true) && qmm_stream_workspace_given(workspace, workspace_bytes, K, N))
     return qmm_narrow_launch(x, w_q, scales, biases, y, M, K, N, group_size, dtype, dtype, true, false, (hipStream_t)stream);
   return qmm_stream_launch(x, w_q, scales, biases, y, workspace, workspace_bytes, M, K, N, group_size, dtype, dtype, true,
@@ -536,7 +553,7 @@ int qmm_up_to_16(const void* x, const uint32_t* w_q, const void* scales, const v
                  "dflash_qmm_m16: need N %% 16 == 0 and K %% group_size == 0 (K=%d N=%d gs=%d)", K,
                  N, group_size);
   DFLASH_REQUIRE(kernel == DFLASH_QMM_KERNEL_AUTO || kernel == DFLASH_QMM_KERNEL_TILE ||
-                     kernel == DFLASH_QMM_KERNEL_STREAM,
+                     kernel == DFLASH_QMM_KERNEL_STREAM || kernel == DFLASH_QMM_KERNEL_FASTEST,
                  DFLASH_ERR_ARG, "dflash_qmm_m16: unknown kernel selector %d", kernel);
   if (variant == DFLASH_QMM_MMA2BIG) k_parts = 1;
   DFLASH_REQUIRE(k_parts >= 1 && K % (32 * k_parts) == 0, DFLASH_ERR_SHAPE,
@@ -544,15 +561,19 @@ int qmm_up_to_16(const void* x, const uint32_t* w_q, const void* scales, const v
   DFLASH_REQUIRE(((uintptr_t)x % 16) == 0 && ((uintptr_t)w_q % 16) == 0, DFLASH_ERR_ARG,
                  "dflash_qmm_m16: x and w_q must be 16-byte aligned");
   // (needs no workspace; what a call has to bring does not depend on that)
-  const bool narrow = kernel == DFLASH_QMM_KERNEL_AUTO && qmm_narrow_covers(scales, biases, K, N, group_size, false);
+  const bool automatic = kernel == DFLASH_QMM_KERNEL_AUTO || kernel == DFLASH_QMM_KERNEL_FASTEST;
+  const bool narrow = automatic && qmm_narrow_covers(scales, biases, K, N, group_size, false);
   auto narrow_launch = [&] {
     return qmm_narrow_launch(x, w_q, scales, biases, y, M, K, N, group_size, act_dtype, sb_dtype, false, false, (hipStream_t)stream);
   };
   // (the C interface has always taken scales of 2-byte alignment; the ANYK loads need four)
-  const bool any = kernel == DFLASH_QMM_KERNEL_AUTO && qmm_stream_any_eligible(K, N, group_size) &&
+  const bool any = automatic && qmm_stream_any_eligible(K, N, group_size) &&
                    (((uintptr_t)scales | (uintptr_t)biases) % 4) == 0 && workspace != nullptr &&
                    workspace_bytes >= qmm_stream_workspace_bytes(N, qmm_stream_grid());
   if (kernel != DFLASH_QMM_KERNEL_TILE && (qmm_stream_eligible(K, N, group_size) || any)) {
+    if (kernel == DFLASH_QMM_KERNEL_FASTEST && qmm_resident_covers(scales, biases, workspace_bytes, K, N, group_size, act_dtype, sb_dtype) &&
+        qmm_stream_workspace_given(workspace, workspace_bytes, K, N))
+      return qmm_resident_launch(x, w_q, scales, biases, y, workspace, M, K, N, group_size, act_dtype, false, false, 0, (hipStream_t)stream);
     if (narrow && qmm_stream_workspace_given(workspace, workspace_bytes, K, N)) return narrow_launch();
     return qmm_stream_launch(x, w_q, scales, biases, y, workspace, workspace_bytes, M, K, N, group_size, act_dtype,
                              sb_dtype, false, (hipStream_t)stream);
@@ -679,8 +700,8 @@ extern "C" int dflash_qmm_m16_packed_by(const void* x, const void* codes, const 
                                         void* workspace, size_t workspace_bytes, int K, int N, int group_size, int act_dtype,
                                         int sb_dtype, int kernel, void* stream) {
   using namespace dflash;
-  DFLASH_REQUIRE(kernel == DFLASH_QMM_KERNEL_AUTO || kernel == DFLASH_QMM_KERNEL_STREAM, DFLASH_ERR_ARG,
-                 "dflash_qmm_m16_packed: no packed form of kernel %d", kernel);
+  DFLASH_REQUIRE(kernel == DFLASH_QMM_KERNEL_AUTO || kernel == DFLASH_QMM_KERNEL_STREAM || kernel == DFLASH_QMM_KERNEL_FASTEST,
+                 DFLASH_ERR_ARG, "dflash_qmm_m16_packed: no packed form of kernel %d", kernel);
   DFLASH_REQUIRE(x && codes && scales && biases && y, DFLASH_ERR_ARG, "dflash_qmm_m16_packed: null operand");
   DFLASH_REQUIRE(act_dtype == DFLASH_BF16 || act_dtype == DFLASH_FP16, DFLASH_ERR_ARG,
                  "dflash_qmm_m16_packed: act_dtype %d is not bf16/fp16", act_dtype);
@@ -692,7 +713,10 @@ extern "C" int dflash_qmm_m16_packed_by(const void* x, const void* codes, const 
   DFLASH_REQUIRE(((uintptr_t)x % 16) == 0 && ((uintptr_t)codes % 16) == 0 && ((uintptr_t)scales % 16) == 0 &&
                      ((uintptr_t)biases % 16) == 0,
                  DFLASH_ERR_ARG, "dflash_qmm_m16_packed: operands must be 16-byte aligned");
-  if (kernel == DFLASH_QMM_KERNEL_AUTO && qmm_narrow_covers(scales, biases, K, N, group_size, false))
+  if (kernel == DFLASH_QMM_KERNEL_FASTEST && qmm_resident_covers(scales, biases, workspace_bytes, K, N, group_size, act_dtype, sb_dtype) &&
+      qmm_stream_workspace_given(workspace, workspace_bytes, K, N))
+    return qmm_resident_launch(x, codes, scales, biases, y, workspace, 16, K, N, group_size, act_dtype, false, true, 0, (hipStream_t)stream);
+  if (kernel != DFLASH_QMM_KERNEL_STREAM && qmm_narrow_covers(scales, biases, K, N, group_size, false))
     return qmm_narrow_launch(x, codes, scales, biases, y, 16, K, N, group_size, act_dtype, sb_dtype, false, true, (hipStream_t)stream);
   return qmm_stream_packed_launch(x, codes, scales, biases, y, workspace, workspace_bytes, K, N,
                                   act_dtype, sb_dtype, (hipStream_t)stream);

@@ -1,0 +1,80 @@
+// Host side of qmm_resident.h: which products of up to 16 rows its kernel takes, and how their K range is cut.
+#include "qmm_resident.h"
+
+namespace dflash {
+
+int qmm_stream_grid();
+
+namespace resident {
+namespace {
+struct Plan {
+  int chunks;  // NCH of the kernel, 0: not this kernel's
+  int slices;
+};
+// One row of K <= 1024 against few rows of W is qmm_narrow's, which has no ring to set up (1024 x 512, 1 / 16 rows: 3.1 / 3.7 us there, 3.7 /
+// 3.8 here; 1024 x 8192 5.3 / 5.9 there, 4.8 / 5.0 here); beyond that K a unit of x is dearer there (3072 x 2048 5.2 / 7.0 and 4.7 / 5.0).
+//
+// Slices by a model fitted to 1 .. 4 of them at eight shapes, in 10 ns and less what all have: 75 per chunk for x and the first tile, 30 + 40 per
+// chunk for each further tile of the busiest workgroup (a lane in twenty with one more does not count), 120 for the meeting of slices.
+// us for 16 rows, 1 / 2 / 3 / 4 slices: 4096 x 4096 6.1 / 6.7 / 7.0 / 8.0; 5120 x 5120 9.1 / 8.5 / 8.4 / 9.6; 6144 x 512 7.4 / 5.6 / 5.0 / 5.0;
+// 12288 x 4096 - / 11.7 / 11.1 / 11.0; 17408 x 5120 - / - / 17.4 / 17.8 (K x N).  M does not enter: a row must not change with the rows beside it.
+Plan plan_for(int K, int N, int group_size) {
+  const int step = group_size == 128 ? 2 : 1, most = group_size == 32 ? 5 : 6;  // (groups of 32: six chunks do not fit the registers)
+  if ((group_size != 32 && group_size != 64 && group_size != 128) || K % (kChunk * step) != 0 || N % 16 != 0 || N < 16) return {0, 0};
+  if (K <= 1024 && N <= 4096) return {0, 0};
+  if ((long long)N * K / 2 >= (1ll << 31) - (1 << 24)) return {0, 0};  // 32-bit byte offsets, and kPast behind them
+  const int pieces = K / (kChunk * step), tiles = N / 16, cus = qmm_stream_grid();
+  Plan best = {0, 0};
+  int best_cost = 0;
+  for (int slices = 1; slices <= kMostSlices; ++slices) {
+    const int parts = kWaves * slices;
+    if (pieces < parts || slices > cus) break;
+    int chunks = step * ((pieces + parts - 1) / parts);
+    if (chunks > most) continue;
+    if ((long long)(slices - 1) * N > 65536) break;  // every other slice keeps a KiB per tile in the workspace that the streaming kernel asks for
+    if (chunks < 2) chunks = 2;
+    const int lanes = cus / slices, most_tiles = (20 * tiles + 19 * lanes - 1) / (20 * lanes);
+    const int cost = 75 * chunks + (most_tiles - 1) * (30 + 40 * chunks) + (slices > 1 ? 120 : 0);
+    if (best.chunks == 0 || cost < best_cost) best = {chunks, slices}, best_cost = cost;
+  }
+  return best;
+}
+}  // namespace
+}  // namespace resident
+
+size_t qmm_resident_workspace_bytes(int K, int N, int group_size) {
+  const resident::Plan plan = resident::plan_for(K, N, group_size);
+  return plan.slices < 2 ? 0 : (size_t)64 * 1024 + (size_t)(N / 16) * (plan.slices - 1) * 1024;
+}
+
+bool qmm_resident_covers(const void* scales, const void* biases, size_t workspace_bytes, int K, int N, int group_size, int act_dtype,
+                         int sb_dtype) {
+  // (mixed types: the streaming kernel's; a lane's words of scales are four bytes)
+  return act_dtype == sb_dtype && (((uintptr_t)scales | (uintptr_t)biases) % 4) == 0 && resident::plan_for(K, N, group_size).chunks != 0 &&
+         workspace_bytes >= qmm_resident_workspace_bytes(K, N, group_size);
+}
+
+int qmm_resident_launch(const void* x, const void* w, const void* scales, const void* biases, void* y, void* workspace, int M, int K,
+                        int N, int group_size, int dtype, bool silu_mul, bool packed, int spin_limit, hipStream_t stream) {
+  using namespace resident;
+  const Plan plan = plan_for(K, N, group_size);
+  const bool h16 = dtype == DFLASH_FP16;
+  const Kernel k = h16 ? fp16_kernel(group_size, plan.chunks, silu_mul, packed) : bf16_kernel(group_size, plan.chunks, silu_mul, packed);
+  DFLASH_REQUIRE(k.fn != nullptr, DFLASH_ERR_SHAPE, "dflash_qmm_m16: no kernel for K=%d N=%d gs=%d", K, N, group_size);
+  if (spin_limit <= 0) spin_limit = option(DFLASH_OPT_QMM_SPIN_LIMIT) > 0 ? option(DFLASH_OPT_QMM_SPIN_LIMIT) : stream::kSpinLimit;
+  Args p{(const uint16_t*)x, w, scales, biases, (uint16_t*)y, (float*)((char*)workspace + 64 * 1024), (uint32_t*)workspace,
+         M, K, N, plan.slices, spin_limit};
+  // the attribute belongs to the device's copy of the kernel: once per device and kernel
+  static bool attr_set[kMaxDevices][2][3][8][4] = {};
+  const int slot = current_device_slot();
+  bool& done = attr_set[slot][h16][group_size >> 6][plan.chunks][(silu_mul ? 1 : 0) + (packed ? 2 : 0)];
+  if (!done || slot == kMaxDevices - 1) {
+    DFLASH_HIP_OK(hipFuncSetAttribute(k.fn, hipFuncAttributeMaxDynamicSharedMemorySize, k.lds));
+    done = true;
+  }
+  const int of_slice = qmm_stream_grid() / plan.slices, tiles = N / 16;
+  void* args[] = {&p};
+  DFLASH_HIP_OK(hipLaunchKernel(k.fn, dim3((unsigned)(plan.slices * (tiles < of_slice ? tiles : of_slice))), dim3(64 * kWaves), args, k.lds, stream));
+  return DFLASH_OK;
+}
+}  // namespace dflash

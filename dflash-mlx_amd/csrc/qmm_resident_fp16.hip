@@ -1,0 +1,5 @@
+#include "qmm_resident.h"
+
+dflash::resident::Kernel dflash::resident::fp16_kernel(int group_size, int chunks, bool silu, bool packed) {
+  return kernel_of<true>(group_size, chunks, silu, packed);
+}

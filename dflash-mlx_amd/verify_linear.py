@@ -197,6 +197,7 @@ class FusedProjections:
         rows = self.bounds[0][1]
         chain = self._silu_chain
         if chain is not None:
+            chain._take_fastest()
             out = chain._bind_rows(x, rows)
             if out is not None:
                 chain()
@@ -209,6 +210,7 @@ class FusedProjections:
                 problem = ChainProblem(x.reshape(16, -1), self.weight, self.scales, self.biases,
                                        epilogue="silu_mul", out=out.view(16, rows))
             chain = QmmChain([problem])
+            chain._take_fastest()
             self._silu_chain = chain
         else:
             chain.rebind(0, x=x.reshape(16, -1), out=out.view(16, rows))

@@ -13,7 +13,8 @@ and shape dispatch, with the device work done by the gfx950 kernel behind
 * ``DFLASH_VERIFY_VARIANT`` in {auto, mma2big, mma2big_pipe} and
   ``DFLASH_VERIFY_QMM_KPARTS`` select the variant (:15-22, 292-297).
 * ``DFLASH_QMM_KERNEL`` in {auto, tile, stream} picks the device kernel (no counterpart
-  in the reference; auto takes matrices of few weights through a kernel of their own, csrc/qmm_narrow.hip, and the rest through the
+  in the reference; not set: the kernel that keeps x in registers, csrc/qmm_resident.h, wherever it applies, else as auto,
+  which takes matrices of few weights through a kernel of their own, csrc/qmm_narrow.hip, and the rest through the
   streaming kernel, whose every-K form takes all group sizes and K a multiple of 64, wherever it applies).
 * An eligible call needs device tensors and the built HIP library; there is no
   software fallback for it.
@@ -33,14 +34,16 @@ _DTYPE_CODE = {torch.bfloat16: _native.BF16, torch.float16: _native.FP16}
 _VARIANT_CODE = {"mma2big": _native.QMM_MMA2BIG, "mma2big_pipe": _native.QMM_MMA2BIG_PIPE}
 _KERNEL_CODE = {"auto": _native.QMM_KERNEL_AUTO, "tile": _native.QMM_KERNEL_TILE,
                 "stream": _native.QMM_KERNEL_STREAM}
+_AUTOMATIC = (_native.QMM_KERNEL_AUTO, _native.QMM_KERNEL_FASTEST)  # no kernel is named
 
 
 def _kernel_select() -> int:
     """``DFLASH_QMM_KERNEL`` in {auto, tile, stream}: which device kernel serves eligible
-    calls (auto: the streaming kernel wherever it applies, the tile kernel elsewhere)."""
+    calls (auto: the streaming kernel wherever it applies, the tile kernel elsewhere, so that single
+    calls have the bits of a ``QmmChain``).  Without it also the kernel that keeps x in registers, the fastest."""
     chosen = _native.env(b"DFLASH_QMM_KERNEL")
     if chosen is None:
-        return _native.QMM_KERNEL_AUTO
+        return _native.QMM_KERNEL_FASTEST
     return _KERNEL_CODE.get(os.fsdecode(chosen).strip().lower(), _native.QMM_KERNEL_AUTO)
 
 
@@ -364,6 +367,11 @@ class QmmChain:
             t.y = out.data_ptr()
             self.outputs[index] = out
 
+    def _take_fastest(self) -> None:
+        """For a chain of one gate/up projection whose launches need not have the bits of a longer chain: they take the
+        kernel that single calls take (``DFLASH_QMM_KERNEL``)."""
+        self._flags = _native.QMM_CHAIN_FASTEST if _kernel_select() == _native.QMM_KERNEL_FASTEST else 0
+
     def _bind_rows(self, x: torch.Tensor, columns: int) -> Optional[torch.Tensor]:
         """Points a chain of one projection at the rows of ``x`` and at a new tensor for their ``columns`` results, which is
         returned; None (nothing done) where ``rebind`` has to look at them.  For a caller that binds before every launch: the chain
@@ -443,7 +451,8 @@ def pack_weights(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor, *,
 
 def _packed_kernel() -> int:
     """The kernel that packed weights go through: the tile kernel has no packed form."""
-    return _native.QMM_KERNEL_AUTO if _kernel_select() == _native.QMM_KERNEL_AUTO else _native.QMM_KERNEL_STREAM
+    kernel = _kernel_select()
+    return kernel if kernel in _AUTOMATIC else _native.QMM_KERNEL_STREAM
 
 
 def verify_matmul_packed(x: torch.Tensor, packed: PackedWeights) -> torch.Tensor:
@@ -532,13 +541,14 @@ def small_m_silu_mul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
     """``silu(x @ gate.T) * (x @ up.T)`` for at most 16 rows of device activations in one launch of the streaming
     kernel; ``w`` holds the gate rows of an MLP followed by its up rows.  None for what that kernel does not
     cover or ``small_m_matmul`` leaves to the array operators.  No counterpart in the reference."""
-    if (bits == 4 and x.is_cuda and _kernel_select() == _native.QMM_KERNEL_AUTO and _native.plain(x, w, scales, biases)
+    kernel = _kernel_select()
+    if (bits == 4 and x.is_cuda and kernel in _AUTOMATIC and _native.plain(x, w, scales, biases)
             and _native.is_built()):
-        y = _native.host().qmm_few_silu_mul(x, w, scales, biases, group_size, _WORKSPACES)
+        y = _native.host().qmm_few_silu_mul(x, w, scales, biases, group_size, kernel, _WORKSPACES)
         if y is not None:
             return y
     if (not x.is_cuda or bits != 4 or x.dtype not in _DTYPE_CODE or not (scales.dtype == biases.dtype == x.dtype)
-            or w.ndim != 2 or _kernel_select() != _native.QMM_KERNEL_AUTO):
+            or w.ndim != 2 or kernel not in _AUTOMATIC):
         return None
     K, N = int(x.shape[-1]), int(w.shape[0])
     m = x.numel() // K if K else 0
@@ -563,8 +573,8 @@ def small_m_silu_mul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
     y = torch.empty((m, N // 2), dtype=x.dtype, device=x.device)
     stream = _native.raw_stream(x.device)
     ws = _workspace(x.device, stream, need)
-    rc = lib.dflash_qmm_few_silu_mul(x2.data_ptr(), w.data_ptr(), scales.data_ptr(), biases.data_ptr(), y.data_ptr(), ws.data_ptr(),
-                                     ws.numel(), m, K, N, group_size, _DTYPE_CODE[x.dtype], stream)
+    rc = lib.dflash_qmm_few_silu_mul_by(x2.data_ptr(), w.data_ptr(), scales.data_ptr(), biases.data_ptr(), y.data_ptr(), ws.data_ptr(),
+                                        ws.numel(), m, K, N, group_size, _DTYPE_CODE[x.dtype], kernel, stream)
     _native.check(rc, "dflash_qmm_few_silu_mul")
     return y.reshape(*x.shape[:-1], N // 2)
 

@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define DFLASH_ABI_VERSION 23
+#define DFLASH_ABI_VERSION 24
 
 enum {
   DFLASH_OK = 0,
@@ -48,8 +48,16 @@ enum { DFLASH_QMM_MMA2BIG = 0, DFLASH_QMM_MMA2BIG_PIPE = 1 };
  * group_size 64 and K % 512 == 0, and decides the K split itself (variant and k_parts
  * then only name the caller's dispatch decision).  AUTO: STREAM where it applies, and its
  * form for every group size and K a multiple of 64 where scales and biases start on 4 bytes.
+ * FASTEST: AUTO, and before it the kernel that keeps x in registers (K a multiple of 128 from 1024
+ * on, activations and scales of one type).  Its sums are cut in other places than those of STREAM
+ * and of a chained launch, with which AUTO agrees bit for bit beyond matrices of few weights.
  */
-enum { DFLASH_QMM_KERNEL_AUTO = 0, DFLASH_QMM_KERNEL_TILE = 1, DFLASH_QMM_KERNEL_STREAM = 2 };
+enum {
+  DFLASH_QMM_KERNEL_AUTO = 0,
+  DFLASH_QMM_KERNEL_TILE = 1,
+  DFLASH_QMM_KERNEL_STREAM = 2,
+  DFLASH_QMM_KERNEL_FASTEST = 3
+};
 
 int dflash_abi_version(void);
 const char* dflash_last_error(void);
@@ -139,6 +147,10 @@ size_t dflash_qmm_few_silu_mul_workspace_bytes(int K, int N, int group_size);
 int dflash_qmm_few_silu_mul(const void* x, const uint32_t* w_q, const void* scales, const void* biases, void* y,
                             void* workspace, size_t workspace_bytes, int M, int K, int N, int group_size, int dtype,
                             void* stream);
+/* The same with the kernel named: DFLASH_QMM_KERNEL_AUTO (what dflash_qmm_few_silu_mul takes) or _FASTEST. */
+int dflash_qmm_few_silu_mul_by(const void* x, const uint32_t* w_q, const void* scales, const void* biases, void* y,
+                               void* workspace, size_t workspace_bytes, int M, int K, int N, int group_size, int dtype,
+                               int kernel, void* stream);
 
 /*
  * dflash_qmm_m16 for callers that cannot allocate device memory: code under HIP graph
@@ -198,12 +210,13 @@ int dflash_qmm_m16_static(const void* x, const uint32_t* w_q, const void* scales
  * at the two ends of a workgroup's range go through partial tiles.  A row block's sum is then no
  * longer cut where a launch of its own would cut it: results equal dflash_qmm_m16's to within one
  * rounding of the output type instead of bit for bit, and are the same from run to run.  The
- * workspace size depends on the flag.
+ * workspace size depends on the flag.  DFLASH_QMM_CHAIN_FASTEST, for one
+ * problem only: with the silu-mul epilogue it may take the kernel of DFLASH_QMM_KERNEL_FASTEST.
  */
 #define DFLASH_QMM_CHAIN_MAX 16
 #define DFLASH_QMM_CHAIN_ERROR_OFFSET DFLASH_QMM_ERROR_OFFSET
 enum { DFLASH_QMM_EPILOGUE_NONE = 0, DFLASH_QMM_EPILOGUE_SILU_MUL = 1 };
-enum { DFLASH_QMM_CHAIN_JOINT_SPLIT = 1 };
+enum { DFLASH_QMM_CHAIN_JOINT_SPLIT = 1, DFLASH_QMM_CHAIN_FASTEST = 4 };
 enum { DFLASH_QMM_LAYOUT_ROWS = 0, DFLASH_QMM_LAYOUT_PACKED = 1 };
 
 typedef struct dflash_qmm_problem {

@@ -1,0 +1,87 @@
+"""Up to 16 rows through the kernel that keeps x in registers (csrc/qmm_resident.h): widths that are whole chunks for every wave and
+widths that are not, one to four slices of K, rings that go round and that do not, every group size and type, the packed
+images and the gated activation, against the product of the same operands in fp64."""
+import pytest
+import torch
+
+import dflash_mlx_amd._native as nat
+from dflash_mlx_amd import verify_qmm as VQ
+from dflash_mlx_amd.quantized import dequantize, stock_matmul
+from dflash_mlx_amd.workloads import make_qmm_case
+from test_gpu_qmm_any_k import _check
+from test_gpu_qmm_narrow import test_gated_activation_at_the_edges as check_gated_activation
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+BF, HF = torch.bfloat16, torch.float16
+# chunks of 128 k over 8 waves: 1, 1 and 2, 2, .., 6 each, then slices; one tile, a tile per compute unit and one more, nine tiles of some (two
+# meetings and a last odd tile)
+SHAPES = [(1024, 4112, 64), (1152, 16, 64), (1920, 48, 32), (2048, 4112, 128), (2176, 32, 64), (2304, 36880, 64), (3072, 4096, 64), (3584, 80, 128),
+          (4096, 4096, 64), (4096, 1040, 32), (4736, 2320, 64), (5120, 4128, 32), (5120, 12352, 64), (5376, 64, 128), (6144, 512, 64),
+          (6144, 8224, 64), (6272, 112, 64), (8192, 4112, 64), (10240, 48, 32), (12288, 4096, 128), (12288, 1024, 64), (17408, 1040, 64),
+          (17408, 5120, 64), (24576, 32, 64), (24704, 32, 64)]
+
+
+def _clean(native_lib):
+    VQ.raise_on_device_errors(torch.device(DEV))
+    ws = VQ._workspace(torch.device(DEV), nat.raw_stream(torch.device(DEV)), 1)
+    return int((ws != 0).sum()) == 0
+
+
+@pytest.mark.parametrize("K,N,group", SHAPES)
+@pytest.mark.parametrize("dtype", [BF, HF])
+def test_products(verify_env, native_lib, K, N, group, dtype):
+    c = make_qmm_case(K, N, K + N, group_size=group, dtype=dtype).to(DEV)
+    y = stock_matmul(c.x, c.w, c.scales, c.biases, group_size=group)
+    _check(y, c.x, dequantize(c.w, c.scales, c.biases, group, 4, torch.float64), K, dtype)
+    for rows in (1, 2, 5, 15):  # a row's bits do not depend on the rows beside it
+        assert torch.equal(stock_matmul(c.x[:rows].clone(), c.w, c.scales, c.biases, group_size=group), y[:rows])
+    if N % 32 == 0 and K % 256 == 0:
+        assert torch.equal(VQ.verify_matmul(c.x, c.w, c.scales, c.biases, group_size=group), y)
+    if group == 64 and K % 1024 == 0 and N % 32 == 0:
+        assert torch.equal(VQ.verify_matmul_packed(c.x, VQ.pack_weights(c.w, c.scales, c.biases)), y)
+    assert _clean(native_lib)  # (slices leave their tiles at zero)
+
+
+@pytest.mark.parametrize("K,N,group", [(1024, 4128, 64), (1152, 32, 32), (3072, 2112, 64), (4096, 8224, 32), (5120, 4224, 64), (6144, 96, 128), (8192, 1056, 64),
+                                       (12288, 2048, 64)])
+@pytest.mark.parametrize("dtype", [BF, HF])
+def test_gated_activation(native_lib, K, N, group, dtype):
+    check_gated_activation(native_lib, K, N, group, dtype)
+    assert _clean(native_lib)
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+def test_what_is_not_a_number_stays_in_its_row(verify_env, native_lib, value):
+    """Rows are loaded together and padded chunks are multiplied with zeros: neither lets one row's values into another."""
+    c = make_qmm_case(5248, 160, 3).to(DEV)  # (41 chunks over 8 waves)
+    want = stock_matmul(c.x, c.w, c.scales, c.biases)
+    x = c.x.clone()
+    x[3, 5000] = value
+    y = stock_matmul(x, c.w, c.scales, c.biases)
+    assert not torch.isfinite(y[3]).any()
+    keep = [r for r in range(16) if r != 3]
+    assert torch.equal(y[keep], want[keep])
+    scales = c.scales.clone()
+    scales[17, 80] = value  # one row of W: one column of y
+    y = stock_matmul(c.x, c.w, scales, c.biases)
+    assert not torch.isfinite(y[:, 17]).any()
+    cols = [n for n in range(160) if n != 17]
+    assert torch.equal(y[:, cols], want[:, cols])
+
+
+def test_a_slice_that_gives_up_says_so_and_the_launch_ends(verify_env, native_lib):
+    """The wait for the other slices' tiles cut to one poll: as for the streaming kernel's adding workgroups."""
+    c = make_qmm_case(17408, 5120, 41).to(DEV)
+    good = VQ.verify_matmul(c.x, c.w, c.scales, c.biases)
+    VQ.raise_on_device_errors(torch.device(DEV))
+    assert native_lib.dflash_set_option(nat.OPT_QMM_SPIN_LIMIT, 1) == 0
+    try:
+        for _ in range(8):  # (320 tiles of workgroups that finish at different times)
+            VQ.verify_matmul(c.x, c.w, c.scales, c.biases)
+        torch.cuda.synchronize()
+    finally:
+        assert native_lib.dflash_set_option(nat.OPT_QMM_SPIN_LIMIT, 0) == 0
+    with pytest.raises(nat.NativeLibraryError, match="partial tiles of row block"):
+        VQ.raise_on_device_errors(torch.device(DEV))
+    assert torch.equal(VQ.verify_matmul(c.x, c.w, c.scales, c.biases), good) and _clean(native_lib)
