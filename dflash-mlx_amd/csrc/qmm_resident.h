@@ -32,7 +32,6 @@ using stream::u32x2_t;
 constexpr int kWaves = 8;
 constexpr int kChunk = 128;  // k of a piece of 64 bytes of codes
 constexpr int kDepth = 2;    // tiles of a wave's ring
-constexpr int kSlots = 4;    // tiles between two meetings of the waves
 constexpr int kMostSlices = 4;
 constexpr uint32_t kPast = 0x80000000u;  // an offset behind every array: reads zeros
 
@@ -42,13 +41,14 @@ struct Args {
   const void* scales;
   const void* biases;
   uint16_t* y;  // [M, N], SILU: [M, N / 2]
-  float* partials;  // slices > 1: [N / 16][slices - 1] tiles, zero between calls
-  uint32_t* status;
+  float* partials;  // slices > 1: MT = 1: [N / 16][slices - 1] tiles, zero between calls; else [N / 16][MT][slices] tiles
+  uint32_t* status;  // MT = 1: its error word; else a counter per N / 16 and MT, zero between calls
   int M, K, N, slices, spin_limit;
 };
 
-template <int GS, int NCH>
+template <int GS, int NCH, int MT>
 struct Geometry {
+  static constexpr int kSlots = MT == 1 ? 4 : 2;      // tiles between two meetings of the waves
   static constexpr int G = kChunk / GS, WPG = 4 / G;  // groups of a chunk, words of a lane per group
   static constexpr int SD = (NCH * G + 1) / 2;        // words of a row's scales, two groups each
   static constexpr int NS = (SD + 3) / 4;             // loads for them
@@ -56,7 +56,8 @@ struct Geometry {
   static constexpr int kStage = NCH * 1024 + 2 * NS * 256;
   static constexpr int kLoads = NCH + 2 * NS;
   static constexpr int kSums = kWaves * kDepth * kStage;
-  static constexpr int kLds = kSums + kSlots * kWaves * 1024;
+  static constexpr int kSumsOfWave = kSlots * MT * 1024;
+  static constexpr int kLds = kSums + kWaves * kSumsOfWave;
   static_assert(kLds <= 160 * 1024, "LDS of a compute unit");
 };
 
@@ -109,6 +110,19 @@ struct Codes {
   }
 };
 
+// Weights of 17 rows and more are rounded to the activation type, as in the any-rows product (qmm_rows.hip says how the codes become numbers)
+template <bool H16>
+__device__ __forceinline__ uint32_t dequant2(uint32_t w, int p, float s24, float s20, float b, uint32_t mask0, uint32_t mask4) {
+  const uint32_t v = p & 1 ? w >> 8 : w;
+  const f16x2_t lo = __builtin_bit_cast(f16x2_t, v & mask0), hi = __builtin_bit_cast(f16x2_t, v & mask4);
+  return pack_pair<H16 ? DFLASH_FP16 : DFLASH_BF16>(__builtin_fmaf((float)lo[p >> 1], s24, b), __builtin_fmaf((float)hi[p >> 1], s20, b));
+}
+template <bool H16>
+__device__ __forceinline__ uint4 dequant8(uint32_t w, float s24, float s20, float b, uint32_t mask0, uint32_t mask4) {
+  return make_uint4(dequant2<H16>(w, 0, s24, s20, b, mask0, mask4), dequant2<H16>(w, 1, s24, s20, b, mask0, mask4),
+                    dequant2<H16>(w, 2, s24, s20, b, mask0, mask4), dequant2<H16>(w, 3, s24, s20, b, mask0, mask4));
+}
+
 template <int WPG>
 struct Words {
   typedef u32x4_t T;
@@ -140,11 +154,12 @@ __device__ __forceinline__ void load_partials3(const float* const (&p)[3], f32x4
 // H16: activations and scales are fp16, else bf16.  GS: group size.  SILU: W holds the gate rows of an MLP and, behind them, its up rows;
 // the rows of a tile are 8 gate rows and the up rows of the same columns, so that lane li + 8 of a finished tile holds what lane li
 // multiplies with.
-template <bool H16, int GS, int NCH, bool SILU, bool PACKED>
+template <bool H16, int GS, int NCH, int MT, bool SILU, bool PACKED>
 __device__ __forceinline__ void product(const Args& p) {
   using A = Act<H16>;
   using C4 = Codes<H16>;
-  using L = Geometry<GS, NCH>;
+  using L = Geometry<GS, NCH, MT>;
+  constexpr int kSlots = L::kSlots;
   constexpr int G = L::G, WPG = L::WPG, NS = L::NS, NB = L::NB;
   extern __shared__ __align__(16) char lds[];  // every wave's ring; then the waves' sums
   const int lane = threadIdx.x & 63, li = lane & 15, q = lane >> 4;
@@ -166,14 +181,16 @@ __device__ __forceinline__ void product(const Args& p) {
   const auto x_buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.x), 0, (uint32_t)p.M * (uint32_t)K * 2u, 0x00027000);
 
   // x first (from the weights on, a request waits for theirs): 256 bytes of four rows a load; rows past M and chunks past `mine` are zeros
-  u32x4_t xr[NCH][4];
+  u32x4_t xr[MT][NCH][4];
 #pragma unroll
-  for (int c = 0; c < NCH; ++c)
+  for (int m = 0; m < MT; ++m)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint32_t at = (uint32_t)(4 * j + q) * (uint32_t)K * 2u + 256u * (uint32_t)(first + c) + 16u * li;
-      xr[c][j] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(x_buf, c < mine ? at : kPast, 0, 0));
-    }
+    for (int c = 0; c < NCH; ++c)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t at = (uint32_t)(16 * m + 4 * j + q) * (uint32_t)K * 2u + 256u * (uint32_t)(first + c) + 16u * li;
+        xr[m][c][j] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(x_buf, c < mine ? at : kPast, 0, 0));
+      }
   __builtin_amdgcn_sched_barrier(0);
 
   // Where the lanes of a load read.  Load j of a tile fills the wave's granules (16 bytes) 64 j .. 64 j + 63; granule (row, pos) holds piece
@@ -229,40 +246,42 @@ __device__ __forceinline__ void product(const Args& p) {
   // x to the order of the products, a chunk at a time through the wave's 4 KiB of sums: lane (li, q) has row li, of group g the k
   // from GS / 4 * q on, like the codes it reads
   const uint32_t lds0 = stream::lds_address(lds);
-  const uint32_t sums_at = lds0 + L::kSums + wave * (kSlots * 1024);
-  uint4 x[NCH][4];
+  const uint32_t sums_at = lds0 + L::kSums + wave * L::kSumsOfWave;
+  uint4 x[MT][NCH][4];
 #pragma unroll
-  for (int c = 0; c < NCH; ++c) {
+  for (int m = 0; m < MT; ++m)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) lds_write16(sums_at + 1024u * j + 256u * q + 16u * (li ^ (4 * j + q)), xr[c][j]);
-    u32x4_t t[4];
+    for (int c = 0; c < NCH; ++c) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t piece = (uint32_t)((GS / 8) * (i / WPG) + (GS / 32) * q + i % WPG);
-      lds_read<0>(sums_at + 256u * li + 16u * (piece ^ li), t[i]);
+      for (int j = 0; j < 4; ++j) lds_write16(sums_at + 1024u * j + 256u * q + 16u * (li ^ (4 * j + q)), xr[m][c][j]);
+      u32x4_t t[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t piece = (uint32_t)((GS / 8) * (i / WPG) + (GS / 32) * q + i % WPG);
+        lds_read<0>(sums_at + 256u * li + 16u * (piece ^ li), t[i]);
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(t[0]), "+v"(t[1]), "+v"(t[2]), "+v"(t[3])::"memory");
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x[m][c][i] = stream::as_uint4(MT == 1 ? stream::permute_x(t[i]) : t[i]);
     }
-    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(t[0]), "+v"(t[1]), "+v"(t[2]), "+v"(t[3])::"memory");
-#pragma unroll
-    for (int i = 0; i < 4; ++i) x[c][i] = stream::as_uint4(stream::permute_x(t[i]));
-  }
   // xs[i]: sum of x over group 4 i + q of row li, in fp32
   const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
   const uint4 ones = make_uint4(A::kOnes, A::kOnes, A::kOnes, A::kOnes);
   float xs[NB];
 #pragma unroll
-  for (int c = 0; c < NCH; ++c)
+  for (int c = 0; c < (MT == 1 ? NCH : 0); ++c)
 #pragma unroll
     for (int g = 0; g < G; ++g) {
       f32x4_t d = zero;
 #pragma unroll
-      for (int i = 0; i < WPG; ++i) d = A::mfma(ones, x[c][g * WPG + i], d);
+      for (int i = 0; i < WPG; ++i) d = A::mfma(ones, x[0][c][g * WPG + i], d);
       const int gi = c * G + g;
       xs[gi >> 2] = q == (gi & 3) ? d[0] : (gi & 3) == 0 ? 0.f : xs[gi >> 2];
     }
 
   // in registers the compiler cannot see through: one v_and_or_b32 per pair of codes, selections without branches
-  uint32_t mask = C4::kMask, magic = C4::kMagic, upper = q & 2 ? ~0u : 0u;
-  asm("" : "+s"(mask), "+v"(magic), "+v"(upper));
+  uint32_t mask = MT == 1 ? C4::kMask : 0x000F000Fu, mask4 = 0x00F000F0u, magic = C4::kMagic, upper = q & 2 ? ~0u : 0u;
+  asm("" : "+s"(mask), "+s"(mask4), "+v"(magic), "+v"(upper));
   const uint32_t half = q & 1 ? 0u : 16u;
   auto low = [](uint32_t v) { return H16 ? f16_bits_to_f32(v & 0xFFFFu) : __uint_as_float(v << 16); };
   auto high = [](uint32_t v) { return H16 ? f16_bits_to_f32(v >> 16) : __uint_as_float(v & 0xFFFF0000u); };
@@ -307,41 +326,79 @@ __device__ __forceinline__ void product(const Args& p) {
       for (int g = 0; g < G; ++g) asm volatile("" : "+v"(w[c][g]));
     if (left > kDepth) load(tile + kDepth * lanes_of_slice, D, 0u);
     __builtin_amdgcn_sched_barrier(0);
-    f32x4_t acc = zero;
+    if constexpr (MT == 1) {
+      f32x4_t acc = zero;
 #pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      const float sv = of_q(s[i >> 1][2 * (i & 1)], s[i >> 1][2 * (i & 1) + 1]);
-      const float bv = of_q(b[i >> 1][2 * (i & 1)], b[i >> 1][2 * (i & 1) + 1]);
-      acc = mfma4(xs[i], __builtin_fmaf(-C4::kOffset, sv, bv), acc);
-    }
-#pragma unroll
-    for (int c = 0; c < NCH; ++c)
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        f32x4_t d = zero;
-#pragma unroll
-        for (int i = 0; i < WPG; ++i) d = A::mfma(x[c][g * WPG + i], C4::unpack(Words<WPG>::get(w[c][g], i), mask, magic), d);
-        const int gi = c * G + g, word = gi >> 1;
-        const float sv = gi & 1 ? high(s[word >> 2][word & 3]) : low(s[word >> 2][word & 3]);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) acc[r] = __builtin_fmaf(sv, d[r], acc[r]);
+      for (int i = 0; i < NB; ++i) {
+        const float sv = of_q(s[i >> 1][2 * (i & 1)], s[i >> 1][2 * (i & 1) + 1]);
+        const float bv = of_q(b[i >> 1][2 * (i & 1)], b[i >> 1][2 * (i & 1) + 1]);
+        acc = mfma4(xs[i], __builtin_fmaf(-C4::kOffset, sv, bv), acc);
       }
-    lds_write16(sums_at + 1024u * slot + 16u * lane, acc);
+#pragma unroll
+      for (int c = 0; c < NCH; ++c)
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+          f32x4_t d = zero;
+#pragma unroll
+          for (int i = 0; i < WPG; ++i) d = A::mfma(x[0][c][g * WPG + i], C4::unpack(Words<WPG>::get(w[c][g], i), mask, magic), d);
+          const int gi = c * G + g, word = gi >> 1;
+          const float sv = gi & 1 ? high(s[word >> 2][word & 3]) : low(s[word >> 2][word & 3]);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[r] = __builtin_fmaf(sv, d[r], acc[r]);
+        }
+      lds_write16(sums_at + 1024u * slot + 16u * lane, acc);
+    } else {  // weights rounded to the activation type
+      f32x4_t acc[MT];
+#pragma unroll
+      for (int m = 0; m < MT; ++m) acc[m] = zero;
+#pragma unroll
+      for (int c = 0; c < NCH; ++c)
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+          const int gi = c * G + g, word = gi >> 1;
+          const uint32_t sw = s[word >> 2][word & 3], bw = b[word >> 2][word & 3];
+          const float sv = gi & 1 ? high(sw) : low(sw), bv = gi & 1 ? high(bw) : low(bw), s24 = sv * 0x1p24f, s20 = sv * 0x1p20f;
+#pragma unroll
+          for (int i = 0; i < WPG; ++i) {
+            const uint4 v = dequant8<H16>(Words<WPG>::get(w[c][g], i), s24, s20, bv, mask, mask4);
+#pragma unroll
+            for (int m = 0; m < MT; ++m) acc[m] = A::mfma(x[m][c][g * WPG + i], v, acc[m]);
+          }
+        }
+      // the wait states between a matrix instruction and a store of its result: the compiler does not see the stores inside their blocks
+#pragma unroll
+      for (int m = 0; m < MT; ++m) asm volatile("" : "+v"(acc[m]));
+      asm volatile("s_nop 7\n s_nop 7\n s_nop 7" ::: "memory");
+#pragma unroll
+      for (int m = 0; m < MT; ++m) lds_write16(sums_at + 1024u * (slot * MT + m) + 16u * lane, acc[m]);
+    }
   };
 
-  // Wave v adds up tile v of the last `count` ones and stores it
+  // The waves deal out the 16 x 16 pieces of the last `count` tiles, add them up and store them
   const int cols = SILU ? N >> 1 : N;
+  auto emit = [&](int t, int row0, f32x4_t sum, bool mine_to_store) __attribute__((always_inline)) {
+    const int n = (SILU ? 8 : 16) * t + li;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      float v = sum[r];
+      if (SILU) {  // lane li of 16 reads lane li ^ 8 (DPP row_ror:8)
+        const float up = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xF, 0xF, false));
+        v = stream::silu_mul<H16>(v, up);
+      }
+      if (mine_to_store && (!SILU || li < 8) && row0 + 4 * q + r < p.M) p.y[(size_t)(row0 + 4 * q + r) * cols + n] = (uint16_t)A::from_f32(v);
+    }
+  };
   auto finish = [&](int base, int count, bool more) __attribute__((always_inline)) {
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (wave < count) {
-      const int t = base + wave * lanes_of_slice;
+    for (int unit = wave; unit < count * MT; unit += kWaves) {
+      const int t = base + unit / MT * lanes_of_slice, row0 = MT == 1 ? 0 : 16 * (unit % MT);
       f32x4_t sum;
 #pragma unroll
       for (int v0 = 0; v0 < kWaves; v0 += 4) {
         u32x4_t v[4];
         each<4>([&](auto i) __attribute__((always_inline)) {
           constexpr int I = decltype(i)::value;
-          lds_read<I * kSlots * 1024>(lds0 + L::kSums + v0 * (kSlots * 1024) + 1024u * wave + 16u * lane, v[I]);
+          lds_read<I * L::kSumsOfWave>(lds0 + L::kSums + v0 * L::kSumsOfWave + 1024u * unit + 16u * lane, v[I]);
         });
         asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3])::"memory");
 #pragma unroll
@@ -351,7 +408,7 @@ __device__ __forceinline__ void product(const Args& p) {
         }
       }
       bool mine_to_store = true;
-      if (slices > 1) {
+      if (MT == 1 && slices > 1) {
         float* const slot = p.partials + ((size_t)t * (slices - 1) * 64 + lane) * 4;
         if (slice < slices - 1) {
           stream::store_partial(slot + slice * 256, stream::nonzero_words(sum));
@@ -390,16 +447,11 @@ __device__ __forceinline__ void product(const Args& p) {
           sum = total + sum;
         }
       }
-      const int n = (SILU ? 8 : 16) * t + li;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float v = sum[r];
-        if (SILU) {  // lane li of 16 reads lane li ^ 8 (DPP row_ror:8)
-          const float up = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xF, 0xF, false));
-          v = stream::silu_mul<H16>(v, up);
-        }
-        if (mine_to_store && (!SILU || li < 8) && 4 * q + r < p.M) p.y[(size_t)(4 * q + r) * cols + n] = (uint16_t)A::from_f32(v);
+      if (MT > 1 && slices > 1) {
+        stream::store_partial(p.partials + ((size_t)((t * MT + unit % MT) * slices + slice) * 64 + lane) * 4, sum);
+        continue;
       }
+      emit(t, row0, sum, mine_to_store);
     }
     if (more) asm volatile("s_barrier" ::: "memory");
   };
@@ -418,11 +470,42 @@ __device__ __forceinline__ void product(const Args& p) {
   }
   if (left > 0) step(std::integral_constant<int, 0>{}, tile, left, slot++);
   finish(base, slot, false);
+  if (MT > 1 && slices > 1) {
+    // The last slice to come to its tiles adds up what all have stored, in order; nobody waits.  (A slice's stores are acknowledged
+    // before it says so.)
+    const int lane_of_slice = (int)blockIdx.x - slice * lanes_of_slice;
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    uint32_t before = 0;
+    if (lane == 0 && wave == 0) before = atomicInc(&p.status[lane_of_slice], (uint32_t)(slices - 1));
+    if (wave == 0) {
+      const uint32_t told = __builtin_amdgcn_readfirstlane(before);
+      asm volatile("ds_write_b32 %0, %1\n s_waitcnt lgkmcnt(0)" ::"v"(lds0), "v"(told) : "memory");
+    }
+    asm volatile("s_barrier" ::: "memory");
+    if ((int)stream::lds_read_u32(lds0) != slices - 1) return;
+    const int count = (tiles - lane_of_slice + lanes_of_slice - 1) / lanes_of_slice;
+    for (int unit = wave; unit < count * MT; unit += kWaves) {
+      const int t = lane_of_slice + unit / MT * lanes_of_slice, m = unit % MT;
+      float* const slot_of = p.partials + ((size_t)((t * MT + m) * slices) * 64 + lane) * 4;
+      f32x4_t total = zero;
+      for (int s0 = 0; s0 < slices; s0 += 3) {
+        const float* src[3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) src[i] = slot_of + (s0 + i < slices ? s0 + i : slices - 1) * 256;
+        f32x4_t v[3];
+        load_partials3(src, v);
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+          if (s0 + i < slices) total += v[i];
+      }
+      emit(t, 16 * m, total, true);
+    }
+  }
 }
 
-template <bool H16, int GS, int NCH, bool SILU, bool PACKED>
+template <bool H16, int GS, int NCH, int MT, bool SILU, bool PACKED>
 __global__ __launch_bounds__(64 * kWaves, 2) void qmm_resident_kernel(Args p) {
-  product<H16, GS, NCH, SILU, PACKED>(p);
+  product<H16, GS, NCH, MT, SILU, PACKED>(p);
 }
 
 // The instance for a shape and its LDS; null where there is none.
@@ -430,34 +513,58 @@ struct Kernel {
   const void* fn;
   int lds;
 };
-template <bool H16, int GS, int NCH, bool PACKED>
+template <bool H16, int GS, int NCH, int MT, bool PACKED>
 Kernel kernel_of(bool silu) {
-  const void* fn = silu ? (const void*)qmm_resident_kernel<H16, GS, NCH, true, PACKED> : (const void*)qmm_resident_kernel<H16, GS, NCH, false, PACKED>;
-  return {fn, Geometry<GS, NCH>::kLds};
+  const void* fn = silu ? (const void*)qmm_resident_kernel<H16, GS, NCH, MT, true, PACKED> : (const void*)qmm_resident_kernel<H16, GS, NCH, MT, false, PACKED>;
+  return {fn, Geometry<GS, NCH, MT>::kLds};
 }
-template <bool H16, int GS, bool PACKED>
+// Most chunks that the registers hold: x takes 16 per chunk and 16 rows.
+constexpr int most_chunks(int group_size, int row_tiles) {
+  return row_tiles == 1 ? (group_size == 32 ? 5 : 6) : row_tiles == 2 ? (group_size == 128 ? 4 : 5) : row_tiles == 3 ? (group_size == 128 ? 2 : 3) : 2;
+}
+template <bool H16, int GS, int MT, bool PACKED>
 Kernel kernel_of(int chunks, bool silu) {
-  switch (chunks) {
-    case 2: return kernel_of<H16, GS, 2, PACKED>(silu);
-    case 4: return kernel_of<H16, GS, 4, PACKED>(silu);
-    case 6: if constexpr (GS != 32) return kernel_of<H16, GS, 6, PACKED>(silu); else return {nullptr, 0};
-    default: break;
+  constexpr int most = most_chunks(GS, MT);
+  if (chunks == 2) return kernel_of<H16, GS, 2, MT, PACKED>(silu);
+  if constexpr (most >= 4) {
+    if (chunks == 4) return kernel_of<H16, GS, 4, MT, PACKED>(silu);
   }
-  if constexpr (GS != 128) {
-    if (chunks == 3) return kernel_of<H16, GS, 3, PACKED>(silu);
-    if (chunks == 5) return kernel_of<H16, GS, 5, PACKED>(silu);
+  if constexpr (most >= 6) {
+    if (chunks == 6) return kernel_of<H16, GS, 6, MT, PACKED>(silu);
+  }
+  if constexpr (GS != 128 && most >= 3) {
+    if (chunks == 3) return kernel_of<H16, GS, 3, MT, PACKED>(silu);
+  }
+  if constexpr (GS != 128 && most >= 5) {
+    if (chunks == 5) return kernel_of<H16, GS, 5, MT, PACKED>(silu);
   }
   return {nullptr, 0};
 }
-template <bool H16>
-Kernel kernel_of(int group_size, int chunks, bool silu, bool packed) {
-  if (packed) return kernel_of<H16, 64, true>(chunks, silu);
-  return group_size == 32 ? kernel_of<H16, 32, false>(chunks, silu)
-         : group_size == 64 ? kernel_of<H16, 64, false>(chunks, silu)
-                            : kernel_of<H16, 128, false>(chunks, silu);
+template <bool H16, int MT>
+Kernel kernel_of(int group_size, int chunks, bool silu) {
+  return group_size == 32 ? kernel_of<H16, 32, MT, false>(chunks, silu)
+         : group_size == 64 ? kernel_of<H16, 64, MT, false>(chunks, silu)
+                            : kernel_of<H16, 128, MT, false>(chunks, silu);
 }
+template <bool H16>
+Kernel few_kernel(int group_size, int chunks, bool silu, bool packed) {
+  return packed ? kernel_of<H16, 64, 1, true>(chunks, silu) : kernel_of<H16, 1>(group_size, chunks, silu);
+}
+template <bool H16>
+Kernel rows_kernel(int row_tiles, int group_size, int chunks, bool silu) {
+  switch (row_tiles) {
+    case 2: return kernel_of<H16, 2>(group_size, chunks, silu);
+    case 3: return kernel_of<H16, 3>(group_size, chunks, silu);
+    case 4: return kernel_of<H16, 4>(group_size, chunks, silu);
+    case 5: return kernel_of<H16, 5>(group_size, chunks, silu);
+    default: return {nullptr, 0};
+  }
+}
+constexpr int kMostRowTiles = 5;
 Kernel bf16_kernel(int group_size, int chunks, bool silu, bool packed);
 Kernel fp16_kernel(int group_size, int chunks, bool silu, bool packed);
+Kernel bf16_rows_kernel(int row_tiles, int group_size, int chunks, bool silu);  // 16 * row_tiles rows
+Kernel fp16_rows_kernel(int row_tiles, int group_size, int chunks, bool silu);
 
 }  // namespace resident
 }  // namespace dflash

@@ -7,9 +7,14 @@ int qmm_stream_grid();
 
 namespace resident {
 namespace {
+constexpr int kRowCounters = 16384;  // the any-rows product's workspace: 64 KiB of counters (here: one per workgroup of a slice), then tiles
+constexpr int kMostRowSlices = 8;
+
 struct Plan {
   int chunks;  // NCH of the kernel, 0: not this kernel's
   int slices;
+  int cus;
+  size_t workspace;
 };
 // One row of K <= 1024 against few rows of W is qmm_narrow's, which has no ring to set up (1024 x 512, 1 / 16 rows: 3.1 / 3.7 us there, 3.7 /
 // 3.8 here; 1024 x 8192 5.3 / 5.9 there, 4.8 / 5.0 here); beyond that K a unit of x is dearer there (3072 x 2048 5.2 / 7.0 and 4.7 / 5.0).
@@ -18,13 +23,13 @@ struct Plan {
 // chunk for each further tile of the busiest workgroup (a lane in twenty with one more does not count), 120 for the meeting of slices.
 // us for 16 rows, 1 / 2 / 3 / 4 slices: 4096 x 4096 6.1 / 6.7 / 7.0 / 8.0; 5120 x 5120 9.1 / 8.5 / 8.4 / 9.6; 6144 x 512 7.4 / 5.6 / 5.0 / 5.0;
 // 12288 x 4096 - / 11.7 / 11.1 / 11.0; 17408 x 5120 - / - / 17.4 / 17.8 (K x N).  M does not enter: a row must not change with the rows beside it.
-Plan plan_for(int K, int N, int group_size) {
-  const int step = group_size == 128 ? 2 : 1, most = group_size == 32 ? 5 : 6;  // (groups of 32: six chunks do not fit the registers)
-  if ((group_size != 32 && group_size != 64 && group_size != 128) || K % (kChunk * step) != 0 || N % 16 != 0 || N < 16) return {0, 0};
-  if (K <= 1024 && N <= 4096) return {0, 0};
-  if ((long long)N * K / 2 >= (1ll << 31) - (1 << 24)) return {0, 0};  // 32-bit byte offsets, and kPast behind them
-  const int pieces = K / (kChunk * step), tiles = N / 16, cus = qmm_stream_grid();
-  Plan best = {0, 0};
+Plan make_plan(int K, int N, int group_size, int cus) {
+  const int step = group_size == 128 ? 2 : 1, most = most_chunks(group_size, 1);
+  if ((group_size != 32 && group_size != 64 && group_size != 128) || K % (kChunk * step) != 0 || N % 16 != 0 || N < 16) return {0, 0, cus, 0};
+  if (K <= 1024 && N <= 4096) return {0, 0, cus, 0};
+  if ((long long)N * K / 2 >= (1ll << 31) - (1 << 24)) return {0, 0, cus, 0};  // 32-bit byte offsets, and kPast behind them
+  const int pieces = K / (kChunk * step), tiles = N / 16;
+  Plan best = {0, 0, cus, 0};
   int best_cost = 0;
   for (int slices = 1; slices <= kMostSlices; ++slices) {
     const int parts = kWaves * slices;
@@ -35,29 +40,40 @@ Plan plan_for(int K, int N, int group_size) {
     if (chunks < 2) chunks = 2;
     const int lanes = cus / slices, most_tiles = (20 * tiles + 19 * lanes - 1) / (20 * lanes);
     const int cost = 75 * chunks + (most_tiles - 1) * (30 + 40 * chunks) + (slices > 1 ? 120 : 0);
-    if (best.chunks == 0 || cost < best_cost) best = {chunks, slices}, best_cost = cost;
+    if (best.chunks == 0 || cost < best_cost) best.chunks = chunks, best.slices = slices, best_cost = cost;
   }
+  best.cus = cus;
+  best.workspace = best.slices < 2 ? 0 : (size_t)64 * 1024 + (size_t)tiles * (best.slices - 1) * 1024;
   return best;
+}
+
+// The last few plans of this thread: a model asks for the same ones over and over (0.15 us each).
+const Plan& plan_for(int K, int N, int group_size) {
+  struct Entry {
+    int K, N, group_size;
+    Plan p;
+  };
+  static thread_local Entry cache[64] = {};
+  const int cus = qmm_stream_grid();
+  Entry& e = cache[((unsigned)K * 2654435761u + (unsigned)N * 40503u * 65537u + (unsigned)group_size) >> 26];
+  if (e.K != K || e.N != N || e.group_size != group_size || e.p.cus != cus) e = Entry{K, N, group_size, make_plan(K, N, group_size, cus)};
+  return e.p;
 }
 }  // namespace
 }  // namespace resident
 
-size_t qmm_resident_workspace_bytes(int K, int N, int group_size) {
-  const resident::Plan plan = resident::plan_for(K, N, group_size);
-  return plan.slices < 2 ? 0 : (size_t)64 * 1024 + (size_t)(N / 16) * (plan.slices - 1) * 1024;
-}
-
 bool qmm_resident_covers(const void* scales, const void* biases, size_t workspace_bytes, int K, int N, int group_size, int act_dtype,
                          int sb_dtype) {
   // (mixed types: the streaming kernel's; a lane's words of scales are four bytes)
-  return act_dtype == sb_dtype && (((uintptr_t)scales | (uintptr_t)biases) % 4) == 0 && resident::plan_for(K, N, group_size).chunks != 0 &&
-         workspace_bytes >= qmm_resident_workspace_bytes(K, N, group_size);
+  if (act_dtype != sb_dtype || (((uintptr_t)scales | (uintptr_t)biases) % 4) != 0) return false;
+  const resident::Plan& plan = resident::plan_for(K, N, group_size);
+  return plan.chunks != 0 && workspace_bytes >= plan.workspace;
 }
 
 int qmm_resident_launch(const void* x, const void* w, const void* scales, const void* biases, void* y, void* workspace, int M, int K,
                         int N, int group_size, int dtype, bool silu_mul, bool packed, int spin_limit, hipStream_t stream) {
   using namespace resident;
-  const Plan plan = plan_for(K, N, group_size);
+  const Plan& plan = plan_for(K, N, group_size);
   const bool h16 = dtype == DFLASH_FP16;
   const Kernel k = h16 ? fp16_kernel(group_size, plan.chunks, silu_mul, packed) : bf16_kernel(group_size, plan.chunks, silu_mul, packed);
   DFLASH_REQUIRE(k.fn != nullptr, DFLASH_ERR_SHAPE, "dflash_qmm_m16: no kernel for K=%d N=%d gs=%d", K, N, group_size);
@@ -72,9 +88,57 @@ int qmm_resident_launch(const void* x, const void* w, const void* scales, const 
     DFLASH_HIP_OK(hipFuncSetAttribute(k.fn, hipFuncAttributeMaxDynamicSharedMemorySize, k.lds));
     done = true;
   }
-  const int of_slice = qmm_stream_grid() / plan.slices, tiles = N / 16;
+  const int of_slice = plan.cus / plan.slices, tiles = N / 16;
   void* args[] = {&p};
   DFLASH_HIP_OK(hipLaunchKernel(k.fn, dim3((unsigned)(plan.slices * (tiles < of_slice ? tiles : of_slice))), dim3(64 * kWaves), args, k.lds, stream));
+  return DFLASH_OK;
+}
+
+// 17 to 80 rows: the slices of K that take the least time by a model fitted to 328 combinations of 25 matrices, 32 to 80 rows and 1 to 6
+// slices (4.7 % rms, what it picks is within 3 % of the best of its call).  The caller takes this kernel where that is less than what the any-rows
+// product is expected to take: 17 - 32 rows of K >= 2048 nearly always (4096 x 4096 10.7 -> 8.2 us, 5120 x 34816 with the activation 45.9 -> 38.6),
+// 33 - 48 mostly (4096 x 6144 15.1 -> 11.6), up to 80 where the matrix is not wide (80 rows of 4096 x 6144 17.3 -> 14.4; of 4096 x 24576 with the
+// activation 32.5 there, 34.7 here: sums of eight waves for every 16 x 16 piece, and x of 80 rows leaves room for two chunks a wave only).
+bool qmm_resident_rows_plan(int M, int K, int N, int group_size, bool silu_mul, int* chunks_out, int* slices_out, double* us_out, size_t* workspace) {
+  using namespace resident;
+  const int row_tiles = (M + 15) / 16, step = group_size == 128 ? 2 : 1;
+  if (row_tiles < 2 || row_tiles > kMostRowTiles || K % (kChunk * step) != 0 || N % 16 != 0 || (long long)N * K / 2 >= (1ll << 31) - (1 << 24))
+    return false;
+  const int pieces = K / (kChunk * step), tiles = N / 16, cus = qmm_stream_grid(), most = most_chunks(group_size, row_tiles);
+  if (cus > kRowCounters) return false;
+  bool found = false;
+  for (int slices = 1; slices <= kMostRowSlices && slices <= cus && pieces >= kWaves * slices; ++slices) {
+    const int parts = kWaves * slices, fewest = step * ((pieces + parts - 1) / parts), chunks = fewest < 2 ? 2 : fewest;
+    if (chunks > most) continue;
+    const int lanes = cus / slices, more_tiles = (20 * tiles + 19 * lanes - 1) / (20 * lanes) - 1;  // (of the busiest workgroup, but for a lane in 20)
+    double us = 3.1 + 0.536 * row_tiles * chunks + more_tiles * (0.847 * chunks - 0.7 + (0.353 - 0.051 * chunks) * row_tiles) + (silu_mul ? 0.19 : 0.0);
+    if (slices > 1) us += 0.84 + 0.25 * slices - 0.3 * row_tiles * (more_tiles + 1) + 1.12e-3 * tiles * row_tiles * slices;
+    if (!found || us < *us_out) *chunks_out = chunks, *slices_out = slices, *us_out = us, found = true;
+  }
+  if (found) *workspace = *slices_out < 2 ? 0 : (size_t)4 * kRowCounters + (size_t)tiles * row_tiles * *slices_out * 1024;
+  return found;
+}
+
+// scales and biases on 4 bytes, of the activations' type
+int qmm_resident_rows_launch(const void* x, const void* w, const void* scales, const void* biases, void* y, void* workspace, int M, int K,
+                             int N, int group_size, int dtype, bool silu_mul, int chunks, int slices, hipStream_t stream) {
+  using namespace resident;
+  const int row_tiles = (M + 15) / 16;
+  const bool h16 = dtype == DFLASH_FP16;
+  const Kernel k = h16 ? fp16_rows_kernel(row_tiles, group_size, chunks, silu_mul) : bf16_rows_kernel(row_tiles, group_size, chunks, silu_mul);
+  DFLASH_REQUIRE(k.fn != nullptr, DFLASH_ERR_SHAPE, "dflash_qmm_rows: no kernel for M=%d K=%d N=%d gs=%d", M, K, N, group_size);
+  Args p{(const uint16_t*)x, w, scales, biases, (uint16_t*)y, workspace ? (float*)((char*)workspace + 4 * kRowCounters) : nullptr,
+         (uint32_t*)workspace, M, K, N, slices, 0};
+  static bool attr_set[kMaxDevices][2][3][8][kMostRowTiles + 1][2] = {};
+  const int slot = current_device_slot();
+  bool& done = attr_set[slot][h16][group_size >> 6][chunks][row_tiles][silu_mul];
+  if (!done || slot == kMaxDevices - 1) {
+    DFLASH_HIP_OK(hipFuncSetAttribute(k.fn, hipFuncAttributeMaxDynamicSharedMemorySize, k.lds));
+    done = true;
+  }
+  const int of_slice = qmm_stream_grid() / slices, tiles = N / 16;
+  void* args[] = {&p};
+  DFLASH_HIP_OK(hipLaunchKernel(k.fn, dim3((unsigned)(slices * (tiles < of_slice ? tiles : of_slice))), dim3(64 * kWaves), args, k.lds, stream));
   return DFLASH_OK;
 }
 }  // namespace dflash

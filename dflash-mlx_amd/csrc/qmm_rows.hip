@@ -42,6 +42,12 @@
 #include <algorithm>
 
 namespace dflash {
+int qmm_stream_grid();
+// qmm_resident.hip: 17 to 80 rows
+bool qmm_resident_rows_plan(int M, int K, int N, int group_size, bool silu_mul, int* chunks, int* slices, double* us, size_t* workspace);
+int qmm_resident_rows_launch(const void* x, const void* w, const void* scales, const void* biases, void* y, void* workspace, int M, int K,
+                             int N, int group_size, int dtype, bool silu_mul, int chunks, int slices, hipStream_t stream);
+
 namespace rows {
 
 constexpr int kStageK = 64;  // k per stage and set of waves
@@ -556,6 +562,9 @@ struct Plan {
   const Shape* shape;
   int whole, slices, tiles_m, tiles, stages, grid;
   size_t workspace;
+  // qmm_resident's, where it is expected to take less time: chunks of a wave (0: not taken), slices, workspace
+  int resident_chunks, resident_slices;
+  size_t resident_workspace;
 };
 
 constexpr size_t kCounterBytes = 64 * 1024;
@@ -575,7 +584,7 @@ bool covers(int M, int K, int N, int group_size, bool mixed, int epilogue) {
 // activation, 96 rows, 12.5 -> 13.1 us), the mean of all is 2 % less, of up to 64 rows 3 %.
 // Slices only while all of them find room at once.  Of more tiles than that, those of the last, incomplete round may be
 // cut, with the tile left as it is (5120 x 34816 over 1024 rows: 1088 tiles, two to a CU, the last 64 in slices, 344 us; uncut 382).
-Plan make_plan(int M, int K, int N, int cus, bool fp16, bool mixed, bool silu_mul) {
+Plan make_plan(int M, int K, int N, int group_size, int cus, bool fp16, bool mixed, bool silu_mul) {
   const int form = silu_mul ? 2 : mixed ? 1 : 0;
   auto ceil_div = [](long long a, long long b) { return (int)((a + b - 1) / b); };
   auto microseconds = [&](const Plan& p) {
@@ -618,32 +627,38 @@ Plan make_plan(int M, int K, int N, int cus, bool fp16, bool mixed, bool silu_mu
     }
   }
   best.workspace = best.slices > 1 ? kCounterBytes + (size_t)(best.grid - best.whole) * best.shape->rows() * best.shape->columns() * sizeof(float) : 0;
+  double us = 0.;
+  int chunks = 0, slices = 0;
+  size_t workspace = 0;
+  if (!mixed && qmm_resident_rows_plan(M, K, N, group_size, silu_mul, &chunks, &slices, &us, &workspace) && us < 0.98 * best_us)
+    best.resident_chunks = chunks, best.resident_slices = slices, best.resident_workspace = workspace;
   return best;
 }
 
 // The last few plans of this thread: a model asks for the same ones over and over.
-const Plan& plan(int M, int K, int N, int cus, bool fp16, bool mixed, bool silu_mul) {
+const Plan& plan(int M, int K, int N, int group_size, int cus, bool fp16, bool mixed, bool silu_mul) {
   struct Entry {
     int M, K, N, cus, flags;
     Plan p;
   };
   static thread_local Entry cache[64] = {};
-  const int flags = (fp16 ? 4 : 0) | (mixed ? 2 : 0) | (silu_mul ? 1 : 0);
+  const int flags = (group_size << 3) | (fp16 ? 4 : 0) | (mixed ? 2 : 0) | (silu_mul ? 1 : 0);
   Entry& e = cache[((unsigned)M * 2654435761u + (unsigned)K * 40503u + (unsigned)N * 69069u + (unsigned)flags) >> 26];
   if (e.M != M || e.K != K || e.N != N || e.cus != cus || e.flags != flags)
-    e = Entry{M, K, N, cus, flags, make_plan(M, K, N, cus, fp16, mixed, silu_mul)};
+    e = Entry{M, K, N, cus, flags, make_plan(M, K, N, group_size, cus, fp16, mixed, silu_mul)};
   return e.p;
 }
 
 }  // namespace rows
 
-int qmm_stream_grid();
 }  // namespace dflash
 
 extern "C" size_t dflash_qmm_rows_workspace_bytes(int M, int K, int N, int group_size, int act_dtype, int sb_dtype, int epilogue) {
   using namespace dflash;
   if (!rows::covers(M, K, N, group_size, act_dtype != sb_dtype, epilogue)) return 0;
-  return rows::plan(M, K, N, qmm_stream_grid(), act_dtype == DFLASH_FP16, act_dtype != sb_dtype, epilogue != DFLASH_QMM_EPILOGUE_NONE).workspace;
+  const rows::Plan& p = rows::plan(M, K, N, group_size, qmm_stream_grid(), act_dtype == DFLASH_FP16, act_dtype != sb_dtype,
+                                   epilogue != DFLASH_QMM_EPILOGUE_NONE);
+  return std::max(p.workspace, p.resident_workspace);  // (which of the two kernels it is also depends on where the scales start)
 }
 
 extern "C" int dflash_qmm_rows(const void* x, const uint32_t* w_q, const void* scales, const void* biases, void* y,
@@ -659,9 +674,13 @@ extern "C" int dflash_qmm_rows(const void* x, const uint32_t* w_q, const void* s
                  "with the silu-mul epilogue) (M=%d K=%d N=%d gs=%d)", M, K, N, group_size);
   DFLASH_REQUIRE(((uintptr_t)x % 16) == 0 && ((uintptr_t)w_q % 16) == 0 && ((uintptr_t)y % 8) == 0, DFLASH_ERR_ARG,
                  "dflash_qmm_rows: x and w_q must be 16-byte aligned");
-  const rows::Plan& p = rows::plan(M, K, N, qmm_stream_grid(), act_dtype == DFLASH_FP16, mixed, silu_mul);
-  DFLASH_REQUIRE(p.workspace == 0 || (workspace && workspace_bytes >= p.workspace), DFLASH_ERR_WORKSPACE,
-                 "dflash_qmm_rows: workspace of %zu bytes needed, %zu given", p.workspace, workspace ? workspace_bytes : (size_t)0);
+  const rows::Plan& p = rows::plan(M, K, N, group_size, qmm_stream_grid(), act_dtype == DFLASH_FP16, mixed, silu_mul);
+  const size_t given = workspace ? workspace_bytes : 0;
+  if (p.resident_chunks != 0 && given >= p.resident_workspace && (((uintptr_t)scales | (uintptr_t)biases) % 4) == 0)
+    return qmm_resident_rows_launch(x, w_q, scales, biases, y, workspace, M, K, N, group_size, act_dtype, silu_mul, p.resident_chunks,
+                                    p.resident_slices, (hipStream_t)stream);
+  DFLASH_REQUIRE(given >= p.workspace, DFLASH_ERR_WORKSPACE,
+                 "dflash_qmm_rows: workspace of %zu bytes needed, %zu given", p.workspace, given);
   rows::Args a;
   a.x = (const uint16_t*)x; a.w = w_q; a.scales = (const uint16_t*)scales; a.biases = (const uint16_t*)biases;
   a.y = (uint16_t*)y;

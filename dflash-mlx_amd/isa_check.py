@@ -33,6 +33,8 @@ KERNELS = (
     ("qmm_m16_chain.hip", "_ZN6dflash6stream16qmm_chain_kernel", 8, 40),     # activation x scale dtype x weight layout
     ("qmm_resident_bf16.hip", "_ZN6dflash8resident19qmm_resident_kernel", 34, 20),  # group size x chunks x silu-mul, weight layout
     ("qmm_resident_fp16.hip", "_ZN6dflash8resident19qmm_resident_kernel", 34, 20),
+    ("qmm_resident_rows_bf16.hip", "_ZN6dflash8resident19qmm_resident_kernel", 42, 20),  # rows, group size x chunks x silu-mul
+    ("qmm_resident_rows_fp16.hip", "_ZN6dflash8resident19qmm_resident_kernel", 42, 20),
 )
 # source, number of counter bumps (arrival counters; the chained kernel's per-problem and exit counters too)
 ARRIVALS = (("qmm_m16.hip", 24), ("qmm_m16_stream.hip", 0), ("qmm_m16_chain.hip", 64))
@@ -157,12 +159,13 @@ def check_all() -> None:
     from concurrent.futures import ThreadPoolExecutor
 
     sources = sorted({s for s, *_ in KERNELS} | {s for s, _ in ARRIVALS})
-    with ThreadPoolExecutor(max_workers=3) as pool:
+    with ThreadPoolExecutor(max_workers=7) as pool:
         isa = dict(zip(sources, pool.map(compile_to_isa, sources)))
     for source, prefix, count, min_reads in KERNELS:
         check_kernels(isa[source], prefix, count, min_reads)
     for source, arrivals in ARRIVALS:
         check_arrivals(isa[source], source, arrivals)
-    for source in ("qmm_m16_stream.hip", "qmm_m16_chain.hip", "qmm_resident_bf16.hip", "qmm_resident_fp16.hip"):
+    for source in ("qmm_m16_stream.hip", "qmm_m16_chain.hip", "qmm_resident_bf16.hip", "qmm_resident_fp16.hip",
+                   "qmm_resident_rows_bf16.hip", "qmm_resident_rows_fp16.hip"):
         if check_wide_stores(isa[source], source) == 0:
             raise AssertionError(f"{source}: no partial-tile store found")

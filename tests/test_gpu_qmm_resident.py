@@ -10,6 +10,8 @@ from dflash_mlx_amd.quantized import dequantize, stock_matmul
 from dflash_mlx_amd.workloads import make_qmm_case
 from test_gpu_qmm_any_k import _check
 from test_gpu_qmm_narrow import test_gated_activation_at_the_edges as check_gated_activation
+from test_gpu_qmm_rows import test_every_tile_shape_at_its_edges as check_rows_silu
+from test_gpu_qmm_rows import test_rows_against_fp64 as check_rows
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -85,3 +87,23 @@ def test_a_slice_that_gives_up_says_so_and_the_launch_ends(verify_env, native_li
     with pytest.raises(nat.NativeLibraryError, match="partial tiles of row block"):
         VQ.raise_on_device_errors(torch.device(DEV))
     assert torch.equal(VQ.verify_matmul(c.x, c.w, c.scales, c.biases), good) and _clean(native_lib)
+
+
+# two to five tiles of 16 rows, full and not; one slice and more, whole and uneven chunks; fewer tiles than workgroups, one more, an odd number each
+ROWS = [(17, 2048, 16, 64), (32, 4096, 4096, 64), (33, 2304, 4112, 64), (31, 5120, 12352, 64), (40, 3072, 3072, 32), (48, 4096, 6144, 64), (47, 6144, 2048, 128),
+        (49, 3328, 4608, 64), (64, 4096, 6144, 32), (65, 4096, 6144, 64), (77, 8192, 5120, 64), (79, 3328, 4624, 64), (80, 12288, 4096, 64), (80, 4096, 6144, 128),
+        (17, 17408, 2064, 64), (18, 2176, 8224, 64)]
+
+
+@pytest.mark.parametrize("M,K,N,group", ROWS)
+@pytest.mark.parametrize("dtype", [BF, HF])
+def test_rows_of_short_prompts(native_lib, M, K, N, group, dtype):
+    """Weights rounded to the activation type; the counters of the slices at zero again (the result is the same every time)."""
+    check_rows(native_lib, M, K, N, group, dtype)
+
+
+@pytest.mark.parametrize("M,K,N,group", [(17, 2048, 4128, 64), (32, 4096, 24576, 64), (45, 2304, 6912, 32), (64, 3072, 4096, 64), (77, 4096, 6176, 128),
+                                         (80, 5120, 2080, 64)])
+@pytest.mark.parametrize("dtype", [BF, HF])
+def test_gated_activation_of_short_prompts(native_lib, M, K, N, group, dtype):
+    check_rows_silu(native_lib, M, K, N, group, True, dtype)
