@@ -17,7 +17,7 @@ CSRC_INCLUDE = os.path.join(ROOT, "include")
 LIB_PATH = os.path.join(HERE, "libdflash_mi355.so")
 HOST_PATH = os.path.join(HERE, "_dflash_host.so")
 
-SOURCES = ["api.hip", "qmm_m16.hip", "qmm_m16_stream.hip", "qmm_m16_chain.hip", "qmm_narrow.hip", "qmm_resident.hip", "qmm_resident_bf16.hip", "qmm_resident_fp16.hip", "qmm_resident_rows_bf16.hip", "qmm_resident_rows_fp16.hip", "qmm_rows.hip", "tape_replay.hip", "gdn_forward.hip", "gdn_prompt.hip", "gdn_glue.hip", "attn_glue.hip", "sdpa_q16.hip",
+SOURCES = ["api.hip", "qmm_m16.hip", "qmm_m16_stream.hip", "qmm_m16_chain.hip", "qmm_narrow.hip", "qmm_resident.hip", "qmm_resident_bf16.hip", "qmm_resident_fp16.hip", "qmm_resident_rows_bf16.hip", "qmm_resident_rows_fp16.hip", "qmm_resident_gather.hip", "qmm_rows.hip", "tape_replay.hip", "gdn_forward.hip", "gdn_prompt.hip", "gdn_glue.hip", "attn_glue.hip", "sdpa_q16.hip",
            "conv_state.hip"]
 
 HIPCC_FLAGS = [

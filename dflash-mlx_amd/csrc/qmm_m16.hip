@@ -441,6 +441,10 @@ bool qmm_resident_covers(const void* scales, const void* biases, size_t workspac
                          int sb_dtype);
 int qmm_resident_launch(const void* x, const void* w, const void* scales, const void* biases, void* y, void* workspace, int M, int K,
                         int N, int group_size, int dtype, bool silu_mul, bool packed, int spin_limit, hipStream_t stream);
+// qmm_resident_gather.hip: x and w 16-byte aligned, P within the tables' limits
+bool qmm_resident_gather_covers(const void* scales, const void* biases, int P, int K, int N, int E, int group_size, int act_dtype, int sb_dtype);
+int qmm_resident_gather_launch(const void* x, const int32_t* expert_ids, const void* w, const void* scales, const void* biases, void* y, int P,
+                               int K, int N, int E, int dtype, hipStream_t stream);
 void qmm_stream_packed_bytes(int K, int N, size_t* w_bytes, size_t* sb_bytes);
 int qmm_stream_pack(const uint32_t* w, const void* scales, const void* biases, void* w_out,
                     void* s_out, void* b_out, int K, int N, hipStream_t stream);
@@ -759,6 +763,8 @@ extern "C" int dflash_qmm_m16_gather(const void* x, const int32_t* expert_ids, c
   const bool streams = P <= 256 || (workspace_bytes >= qmm_stream_workspace_bytes(N, qmm_stream_grid()) &&
                                       (((uintptr_t)scales | (uintptr_t)biases) % 4) == 0);
   if (workspace != nullptr && streams && qmm_stream_gather_eligible(P, K, N, E, group_size)) {
+    if (qmm_resident_gather_covers(scales, biases, P, K, N, E, group_size, act_dtype, sb_dtype))
+      return qmm_resident_gather_launch(x, expert_ids, w_q, scales, biases, y, P, K, N, E, act_dtype, s);
     return qmm_stream_gather_launch(x, expert_ids, w_q, scales, biases, y, workspace, workspace_bytes,
                                     P, K, N, E, act_dtype, sb_dtype, s);
   }

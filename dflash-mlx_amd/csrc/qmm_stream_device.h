@@ -419,6 +419,106 @@ __device__ __forceinline__ u32x2_t lds_read_u64(uint32_t addr) {
   return v;
 }
 
+// The tables of the gathered forms, built by all THREADS threads of a workgroup; returns the number of entries.  Rows of y whose expert id is
+// outside [0, E) are set to zero by the first workgroup.
+template <int THREADS>
+__device__ __forceinline__ int build_tables(char* tables, const Tables& tab, const int32_t* expert_ids, int P, int E, uint16_t* y, int N) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  uint32_t* t_count = reinterpret_cast<uint32_t*>(tables);
+  uint32_t* t_entry = reinterpret_cast<uint32_t*>(tables + tab.entry);
+  uint16_t* t_rows = reinterpret_cast<uint16_t*>(tables + tab.rows);
+  uint32_t* t_total = reinterpret_cast<uint32_t*>(tables + tab.total);
+  // a thread's rows: tid, tid + THREADS, ..
+  constexpr int kRounds = (kMaxGatherRows + THREADS - 1) / THREADS, kAllWaves = THREADS / 64;
+  // Every workgroup builds the same tables: a row's place among the rows of its expert is
+  // its rank by row index, not the order in which threads happen to get there (partial
+  // tiles of one row block come from several workgroups and must agree on the rows).
+  for (int e = tid; e < E; e += THREADS) t_count[e] = 0;
+  int my_e[kRounds];
+#pragma unroll
+  for (int r = 0; r < kRounds; ++r) {
+    my_e[r] = -1;
+    if (r * THREADS < P && r * THREADS + tid < P) {
+      const int e = expert_ids[r * THREADS + tid];
+      if (e >= 0 && e < E) my_e[r] = e;
+    }
+  }
+  __syncthreads();
+  // Rank among the rows of the same expert: inside a wave by a match of the ids, a ballot per bit; the waves
+  // that hold rows add their numbers up one after the other.  The scan below runs on DPP.  (Counting
+  // the earlier equal ids one by one and scanning through LDS permutes were 2 us of a launch: 128 rows on 103 of 256 experts of
+  // 512 x 32, where little else happens, 9.4 -> 7.1 us; 2048 x 1024 33.8 -> 32.9, 512 x 2048 24.1 -> 21.7 us; 256 rows on 62 of 64
+  // experts 26.4 -> 23.1 and 20.4 -> 16.6 us.)
+  int my_pos[kRounds] = {}, same_expert[kRounds] = {};
+#pragma unroll
+  for (int r = 0; r < kRounds; ++r) {
+    if (r * THREADS + wave * 64 >= P) continue;
+    unsigned long long same = __builtin_amdgcn_ballot_w64(my_e[r] >= 0);
+    for (int bit = 0; (1 << bit) < E; ++bit) {
+      const bool one = (my_e[r] >> bit) & 1;
+      const unsigned long long ones = __builtin_amdgcn_ballot_w64(one);
+      same &= one ? ones : ~ones;
+    }
+    my_pos[r] = __builtin_popcountll(same & ((1ull << lane) - 1ull));
+    same_expert[r] = __builtin_popcountll(same);
+  }
+#pragma unroll
+  for (int r = 0; r < kRounds; ++r) {
+    for (int w = 0; w < kAllWaves && (r * kAllWaves + w) * 64 < P; ++w) {
+      if (wave == w && my_e[r] >= 0) {
+        const uint32_t before = t_count[my_e[r]];  // (read by all lanes of the wave before the first of each expert adds)
+        if (my_pos[r] == 0) t_count[my_e[r]] = before + (uint32_t)same_expert[r];
+        my_pos[r] += (int)before;
+      }
+      __syncthreads();
+    }
+  }
+  if (wave == 0) {
+    // exclusive scan of ceil(rows / 16) over the experts: first entry of each expert
+    int carry = 0;
+    for (int base = 0; base < E; base += 64) {
+      const int e = base + lane;
+      const int rows = e < E ? (int)t_count[e] : 0;
+      const int n = (rows + 15) >> 4;
+      int incl = n;
+      incl += __builtin_amdgcn_update_dpp(0, incl, 0x111, 0xF, 0xF, true);   // row_shr:1, 2, 4, 8
+      incl += __builtin_amdgcn_update_dpp(0, incl, 0x112, 0xF, 0xF, true);
+      incl += __builtin_amdgcn_update_dpp(0, incl, 0x114, 0xF, 0xF, true);
+      incl += __builtin_amdgcn_update_dpp(0, incl, 0x118, 0xF, 0xF, true);
+      incl += __builtin_amdgcn_update_dpp(0, incl, 0x142, 0xA, 0xF, false);  // last lane of rows 0, 2 to rows 1, 3
+      incl += __builtin_amdgcn_update_dpp(0, incl, 0x143, 0xC, 0xF, false);  // lane 31 to rows 2, 3
+      if (e < E) t_count[e] = ((uint32_t)rows << 16) | (uint32_t)(carry + incl - n);
+      carry += __builtin_amdgcn_readlane(incl, 63);
+    }
+    if (lane == 0) *t_total = (uint32_t)carry;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kRounds; ++r) {
+    if (r * THREADS >= P || my_e[r] < 0) continue;
+    const uint32_t c = t_count[my_e[r]];
+    const int rows = (int)(c >> 16), first = (int)(c & 0xFFFFu);
+    const int ent = first + (my_pos[r] >> 4), m = my_pos[r] & 15;
+    t_rows[ent * 16 + m] = (uint16_t)(r * THREADS + tid);
+    if (m == 0) {
+      const int left_rows = rows - (my_pos[r] & ~15);
+      t_entry[ent] = ((uint32_t)(left_rows < 16 ? left_rows : 16) << 16) | (uint32_t)my_e[r];
+    }
+  }
+  __syncthreads();
+  // A row whose expert id is outside [0, E) belongs to no entry: its output is zero (written
+  // here, by the first workgroup, so that no row of y is left as it was found).
+  if (blockIdx.x == 0) {
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+      const int row = r * THREADS + tid;
+      if (r * THREADS >= P || row >= P || my_e[r] >= 0) continue;
+      for (int n = 0; n < N; ++n) y[(size_t)row * N + n] = 0;
+    }
+  }
+  return (int)*t_total;
+}
+
 template <bool FP16>
 __device__ __forceinline__ float silu_mul(float g, float u) {
   using A = Act<FP16>;

@@ -33,6 +33,7 @@ KERNELS = (
     ("qmm_m16_chain.hip", "_ZN6dflash6stream16qmm_chain_kernel", 8, 40),     # activation x scale dtype x weight layout
     ("qmm_resident_bf16.hip", "_ZN6dflash8resident19qmm_resident_kernel", 34, 20),  # group size x chunks x silu-mul, weight layout
     ("qmm_resident_fp16.hip", "_ZN6dflash8resident19qmm_resident_kernel", 34, 20),
+    ("qmm_resident_gather.hip", "_ZN6dflash8resident12_GLOBAL__N_126qmm_resident_gather_kernel", 8, 20),
     ("qmm_resident_rows_bf16.hip", "_ZN6dflash8resident19qmm_resident_kernel", 42, 20),  # rows, group size x chunks x silu-mul
     ("qmm_resident_rows_fp16.hip", "_ZN6dflash8resident19qmm_resident_kernel", 42, 20),
 )

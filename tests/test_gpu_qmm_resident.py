@@ -107,3 +107,26 @@ def test_rows_of_short_prompts(native_lib, M, K, N, group, dtype):
 @pytest.mark.parametrize("dtype", [BF, HF])
 def test_gated_activation_of_short_prompts(native_lib, M, K, N, group, dtype):
     check_rows_silu(native_lib, M, K, N, group, True, dtype)
+
+
+# one, two, four and eight waves to a tile, even and uneven chunks; one tile of W, sets with one unit, with none; entries of one and of sixteen rows
+@pytest.mark.parametrize("K,N,E,P", [(128, 16, 3, 7), (512, 2048, 256, 128), (640, 48, 5, 90), (768, 16, 300, 200), (1152, 80, 7, 33), (1280, 4112, 2, 16),
+                                     (1408, 272, 9, 64), (2048, 1024, 64, 256), (2688, 96, 4, 40), (5120, 144, 3, 50), (1024, 16, 1, 1), (2560, 528, 600, 64)])
+@pytest.mark.parametrize("dtype", [BF, HF])
+def test_routed_experts(native_lib, monkeypatch, K, N, E, P, dtype):
+    monkeypatch.delenv("DFLASH_QMM_KERNEL", raising=False)
+    gen = torch.Generator("cuda").manual_seed(K + P)
+    w = torch.randint(-2 ** 31, 2 ** 31, (E, N, K // 8), generator=gen, device="cuda", dtype=torch.int32)
+    s = (torch.rand((E, N, K // 64), generator=gen, device="cuda") * 0.02 + 1e-4).to(dtype)
+    b = (s.float() * -8).to(dtype)
+    x = torch.randn((P, K), generator=gen, device="cuda").to(dtype)
+    ids = torch.randint(-1 if E > 1 else 0, E + (E > 1), (P,), generator=gen, device="cuda", dtype=torch.int32)
+    y = VQ.gather_qmm(x, w, s, b, ids)
+    assert (y[(ids < 0) | (ids >= E)] == 0).all()
+    for e in range(E):
+        mine = ids == e
+        if mine.any():
+            _check(y[mine], x[mine], dequantize(w[e], s[e], b[e], 64, 4, torch.float64), K, dtype)
+    assert torch.equal(y, VQ.gather_qmm(x, w, s, b, ids))
+    keep = torch.randperm(P, generator=gen, device="cuda")[:P // 2 + 1]  # a row's bits do not depend on the rows beside it
+    assert torch.equal(VQ.gather_qmm(x[keep].contiguous(), w, s, b, ids[keep].contiguous()), y[keep])
