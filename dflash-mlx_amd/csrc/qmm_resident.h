@@ -44,7 +44,16 @@ struct Args {
   float* partials;  // slices > 1: MT = 1: [N / 16][slices - 1] tiles, zero between calls; else [N / 16][MT][slices] tiles
   uint32_t* status;  // MT = 1: its error word; else a counter per N / 16 and MT, zero between calls
   int M, K, N, slices, spin_limit;
+  // what the kernel would otherwise divide for before its first request (0.3 us): workgroups of a slice, tiles of each and how many have one more, and the
+  // same for steps of K and waves (a step: 128 k, in groups of 128 twice that, whose scales are a word)
+  int lanes, tiles_each, tiles_more, steps_each, steps_more;
 };
+inline void set_partition(Args& p, int group_size, int cus) {
+  const int tiles = p.N / 16, of_slice = cus / p.slices, steps = p.K / (group_size == 128 ? 256 : 128), parts = p.slices * kWaves;
+  p.lanes = tiles < of_slice ? tiles : of_slice;
+  p.tiles_each = tiles / p.lanes, p.tiles_more = tiles % p.lanes;
+  p.steps_each = steps / parts, p.steps_more = steps % parts;
+}
 
 template <int GS, int NCH, int MT>
 struct Geometry {
@@ -164,13 +173,14 @@ __device__ __forceinline__ void product(const Args& p) {
   extern __shared__ __align__(16) char lds[];  // every wave's ring; then the waves' sums
   const int lane = threadIdx.x & 63, li = lane & 15, q = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int K = p.K, N = p.N, tiles = N / 16, slices = p.slices;
-  const int lanes_of_slice = (int)gridDim.x / slices;  // workgroups of a slice
-  const int slice = (int)blockIdx.x / lanes_of_slice;
-  // the wave's chunks (groups of 128: pairs of them, whose scales are a word)
+  const int K = p.K, N = p.N, slices = p.slices, lanes_of_slice = p.lanes;
+  int slice = 0, tile = (int)blockIdx.x;
+  while (tile >= lanes_of_slice) tile -= lanes_of_slice, ++slice;
+  const int first_tile = tile, mine_of_tiles = p.tiles_each + (tile < p.tiles_more ? 1 : 0);
+  // the wave's chunks
   constexpr int STEP = GS == 128 ? 2 : 1;
-  const int pieces = K / (kChunk * STEP), parts = slices * kWaves, part = slice * kWaves + wave;
-  const int first = STEP * (part * pieces / parts), mine = STEP * ((part + 1) * pieces / parts) - first;
+  const int part = slice * kWaves + wave;
+  const int first = STEP * (part * p.steps_each + (part < p.steps_more ? part : p.steps_more)), mine = STEP * (p.steps_each + (part < p.steps_more ? 1 : 0));
 
   const int RB = (N + 127) / 128;
   const uint32_t w_bytes = PACKED ? (uint32_t)RB * (uint32_t)(K / 256) * 16384u : (uint32_t)N * (uint32_t)(K / 2);
@@ -237,8 +247,7 @@ __device__ __forceinline__ void product(const Args& p) {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(b_buf, (lds_void_t*)(at + 1024 * NCH + 512 * j + 256), 4, s_at[j] | past, s_tile, 0, 0);
     }
   };
-  int tile = (int)blockIdx.x - slice * lanes_of_slice;
-  int left = (tiles - tile + lanes_of_slice - 1) / lanes_of_slice;
+  int left = mine_of_tiles;
 #pragma unroll
   for (int d = 0; d < kDepth; ++d) load(d < left ? tile + d * lanes_of_slice : 0, d, d < left ? 0u : kPast);
   __builtin_amdgcn_sched_barrier(0);
@@ -473,19 +482,17 @@ __device__ __forceinline__ void product(const Args& p) {
   if (MT > 1 && slices > 1) {
     // The last slice to come to its tiles adds up what all have stored, in order; nobody waits.  (A slice's stores are acknowledged
     // before it says so.)
-    const int lane_of_slice = (int)blockIdx.x - slice * lanes_of_slice;
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
     uint32_t before = 0;
-    if (lane == 0 && wave == 0) before = atomicInc(&p.status[lane_of_slice], (uint32_t)(slices - 1));
+    if (lane == 0 && wave == 0) before = atomicInc(&p.status[first_tile], (uint32_t)(slices - 1));
     if (wave == 0) {
       const uint32_t told = __builtin_amdgcn_readfirstlane(before);
       asm volatile("ds_write_b32 %0, %1\n s_waitcnt lgkmcnt(0)" ::"v"(lds0), "v"(told) : "memory");
     }
     asm volatile("s_barrier" ::: "memory");
     if ((int)stream::lds_read_u32(lds0) != slices - 1) return;
-    const int count = (tiles - lane_of_slice + lanes_of_slice - 1) / lanes_of_slice;
-    for (int unit = wave; unit < count * MT; unit += kWaves) {
-      const int t = lane_of_slice + unit / MT * lanes_of_slice, m = unit % MT;
+    for (int unit = wave; unit < mine_of_tiles * MT; unit += kWaves) {
+      const int t = first_tile + unit / MT * lanes_of_slice, m = unit % MT;
       float* const slot_of = p.partials + ((size_t)((t * MT + m) * slices) * 64 + lane) * 4;
       f32x4_t total = zero;
       for (int s0 = 0; s0 < slices; s0 += 3) {

@@ -79,7 +79,8 @@ int qmm_resident_launch(const void* x, const void* w, const void* scales, const 
   DFLASH_REQUIRE(k.fn != nullptr, DFLASH_ERR_SHAPE, "dflash_qmm_m16: no kernel for K=%d N=%d gs=%d", K, N, group_size);
   if (spin_limit <= 0) spin_limit = option(DFLASH_OPT_QMM_SPIN_LIMIT) > 0 ? option(DFLASH_OPT_QMM_SPIN_LIMIT) : stream::kSpinLimit;
   Args p{(const uint16_t*)x, w, scales, biases, (uint16_t*)y, (float*)((char*)workspace + 64 * 1024), (uint32_t*)workspace,
-         M, K, N, plan.slices, spin_limit};
+         M, K, N, plan.slices, spin_limit, 0, 0, 0, 0, 0};
+  set_partition(p, group_size, plan.cus);
   // the attribute belongs to the device's copy of the kernel: once per device and kernel
   static bool attr_set[kMaxDevices][2][3][8][4] = {};
   const int slot = current_device_slot();
@@ -88,9 +89,8 @@ int qmm_resident_launch(const void* x, const void* w, const void* scales, const 
     DFLASH_HIP_OK(hipFuncSetAttribute(k.fn, hipFuncAttributeMaxDynamicSharedMemorySize, k.lds));
     done = true;
   }
-  const int of_slice = plan.cus / plan.slices, tiles = N / 16;
   void* args[] = {&p};
-  DFLASH_HIP_OK(hipLaunchKernel(k.fn, dim3((unsigned)(plan.slices * (tiles < of_slice ? tiles : of_slice))), dim3(64 * kWaves), args, k.lds, stream));
+  DFLASH_HIP_OK(hipLaunchKernel(k.fn, dim3((unsigned)(p.slices * p.lanes)), dim3(64 * kWaves), args, k.lds, stream));
   return DFLASH_OK;
 }
 
@@ -128,7 +128,8 @@ int qmm_resident_rows_launch(const void* x, const void* w, const void* scales, c
   const Kernel k = h16 ? fp16_rows_kernel(row_tiles, group_size, chunks, silu_mul) : bf16_rows_kernel(row_tiles, group_size, chunks, silu_mul);
   DFLASH_REQUIRE(k.fn != nullptr, DFLASH_ERR_SHAPE, "dflash_qmm_rows: no kernel for M=%d K=%d N=%d gs=%d", M, K, N, group_size);
   Args p{(const uint16_t*)x, w, scales, biases, (uint16_t*)y, workspace ? (float*)((char*)workspace + 4 * kRowCounters) : nullptr,
-         (uint32_t*)workspace, M, K, N, slices, 0};
+         (uint32_t*)workspace, M, K, N, slices, 0, 0, 0, 0, 0, 0};
+  set_partition(p, group_size, qmm_stream_grid());
   static bool attr_set[kMaxDevices][2][3][8][kMostRowTiles + 1][2] = {};
   const int slot = current_device_slot();
   bool& done = attr_set[slot][h16][group_size >> 6][chunks][row_tiles][silu_mul];
@@ -136,9 +137,8 @@ int qmm_resident_rows_launch(const void* x, const void* w, const void* scales, c
     DFLASH_HIP_OK(hipFuncSetAttribute(k.fn, hipFuncAttributeMaxDynamicSharedMemorySize, k.lds));
     done = true;
   }
-  const int of_slice = qmm_stream_grid() / slices, tiles = N / 16;
   void* args[] = {&p};
-  DFLASH_HIP_OK(hipLaunchKernel(k.fn, dim3((unsigned)(slices * (tiles < of_slice ? tiles : of_slice))), dim3(64 * kWaves), args, k.lds, stream));
+  DFLASH_HIP_OK(hipLaunchKernel(k.fn, dim3((unsigned)(p.slices * p.lanes)), dim3(64 * kWaves), args, k.lds, stream));
   return DFLASH_OK;
 }
 }  // namespace dflash

@@ -49,8 +49,8 @@ __device__ __forceinline__ void gathered_product(const GatherArgs& p) {
   const int chunks = K / kChunk, first = part * chunks / kw, mine = (part + 1) * chunks / kw - first;
   // the set's part of the units; all sets of the workgroup make the steps of the longest
   const int all_sets = sets * (int)gridDim.x, of = set * (int)gridDim.x + (int)blockIdx.x;
-  const int u0 = (int)((long long)units * of / all_sets), own = (int)((long long)units * (of + 1) / all_sets) - u0;
-  const int steps = (units + all_sets - 1) / all_sets;
+  const int each_set = units / all_sets, more = units - each_set * all_sets;
+  const int u0 = of * each_set + (of < more ? of : more), own = each_set + (of < more ? 1 : 0), steps = each_set + (more > 0 ? 1 : 0);
   if (steps == 0) return;
 
   const uint32_t w_bytes = (uint32_t)N * (uint32_t)(K / 2), s_bytes = (uint32_t)N * (uint32_t)(K / 64) * 2u;
