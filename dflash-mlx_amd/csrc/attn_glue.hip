@@ -30,6 +30,7 @@ struct AttnPrepareArgs {
   long long ko_batch, ko_head, ko_row, vo_batch, vo_head, vo_row;
   int B, L, Hq, Hk, half, offset, dt, q_weight_dt, k_weight_dt;
   int waves;  // per token; each takes every waves-th head
+  Divisor groups, tokens;  // by the workgroups of a token, by L
   float q_eps, k_eps, base, inv_half;
 };
 
@@ -41,9 +42,9 @@ __global__ __launch_bounds__(kWavesPerGroup * 64) void attn_prepare_kernel(AttnP
 #pragma clang fp contract(off)
   constexpr int D = 64 * PER;
   __shared__ float2 turn[D / 2];  // cosine and sine
-  const int rotated = p.Hq + p.Hk, heads = rotated + p.Hk, groups = (p.waves + kWavesPerGroup - 1) / kWavesPerGroup;
-  const int token = (int)(blockIdx.x / (unsigned)groups), b = token / p.L, l = token - b * p.L;
-  const int first = (int)(blockIdx.x - (unsigned)token * (unsigned)groups) * kWavesPerGroup + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int rotated = p.Hq + p.Hk, heads = rotated + p.Hk;
+  const int token = p.groups.quotient((int)blockIdx.x), b = p.tokens.quotient(token), l = token - b * p.L;
+  const int first = ((int)blockIdx.x - token * (int)p.groups.by) * kWavesPerGroup + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, c = PER * lane;
   const bool rotates = c < 2 * p.half, upper = c >= p.half;
   const int other = rotates ? (upper ? lane - p.half / PER : lane + p.half / PER) : lane;
@@ -183,7 +184,9 @@ extern "C" int dflash_attn_prepare(const void* q, const void* k, const void* v, 
   // One wave per head while that leaves the chip with fewer than 8 waves per SIMD, beyond that several heads per wave.
   const long long tokens = (long long)B * L, want = (8192 + tokens - 1) / tokens;
   p.waves = want < Hq + 2 * Hk ? (int)want : Hq + 2 * Hk;
-  const long long groups = tokens * ((p.waves + kWavesPerGroup - 1) / kWavesPerGroup);
+  p.groups = Divisor::of((p.waves + kWavesPerGroup - 1) / kWavesPerGroup);
+  p.tokens = Divisor::of(L);
+  const long long groups = tokens * p.groups.by;
   DFLASH_REQUIRE(groups * kWavesPerGroup < (1ll << 31), DFLASH_ERR_SHAPE, "dflash_attn_prepare: too many rows");
   const dim3 grid((unsigned)groups), block(kWavesPerGroup * 64);
   switch (per) {

@@ -50,6 +50,7 @@ struct GdnArgs {
   float* tape;
   const uint8_t* mask;
   int T, Hk, Hv, Dk, Dv;
+  Divisor heads, group, row_parts;  // by Hv, by Hv / Hk, by the workgroups of a head (gdn_forward_rows)
   int in_dtype, g_dtype, beta_dtype, state_dtype, g_per_dk;
   int staged;  // step-by-step kernel: steps staged in LDS at a time
   // gated output norm fused behind the recurrence (block kernel only): y is then
@@ -293,8 +294,8 @@ __global__ __launch_bounds__(kThreads) void gdn_forward_rows(GdnArgs a) {
   __shared__ __align__(16) float sV[16 * kRows];  // v, then (row by row, once it has been read) the tape
   __shared__ __align__(16) float sY[16 * kRows];
   __shared__ __align__(16) float sS[16 * 4];      // gate, beta, k . q of a step
-  const int per = a.Dv / kRows, head = (int)blockIdx.x / per, row0 = ((int)blockIdx.x - head * per) * kRows;
-  const int slot = head / a.Hv, hv = head % a.Hv, hk = hv / (a.Hv / a.Hk);
+  const int head = a.row_parts.quotient((int)blockIdx.x), row0 = ((int)blockIdx.x - head * (int)a.row_parts.by) * kRows;
+  const int slot = a.heads.quotient(head), hv = head - slot * a.Hv, hk = a.group.quotient(hv);
   const int tid = threadIdx.x, t16 = tid >> 4, seg = tid & 15;
   const int rr = tid / kLanes, c8 = tid % kLanes;
   const bool wide = a.in_dtype == DFLASH_FP32;
@@ -348,7 +349,7 @@ __global__ __launch_bounds__(kThreads) void gdn_forward_rows(GdnArgs a) {
     if constexpr (BLOCK) {
       asm volatile("" ::: "memory");  // every request above is out before the first value is interpreted
       // rows of v are one workgroup's, a key head is kept by the first of its value heads and of its first rows
-      const bool keeps = row0 == 0 && hv % (a.Hv / a.Hk) == 0;
+      const bool keeps = row0 == 0 && hv == hk * (int)a.group.by;
       if (mine(0)) {
         float x[kK];
         convolve(a.block, slot, t_b, T, C, c_q, keeps, b_q, x);
@@ -614,7 +615,7 @@ __device__ __forceinline__ int block_channel(const GdnArgs& a, int which, int hv
 template <bool WIDE, bool NORM, bool BLOCK>
 __device__ __forceinline__ void issue_item_loads(const GdnArgs& a, int item, int tid, Incoming<WIDE>& in, BlockIncoming& block) {
   const int T = a.T;
-  const int slot = item / a.Hv, hv = item % a.Hv, hk = hv / (a.Hv / a.Hk);
+  const int slot = a.heads.quotient(item), hv = item - slot * a.Hv, hk = a.group.quotient(hv);
   const size_t slotT = (size_t)slot * T;
   const int lane = tid & 63, wave = BLOCK ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6, li = lane & 15, kq = lane >> 4;
   // the block's operands first, the state behind them: loads complete in order
@@ -717,14 +718,14 @@ void gdn_forward_chunk_128(GdnArgs a) {
   const int item = blockIdx.x;
   BlockIncoming block;
   issue_item_loads<WIDE, NORM, BLOCK>(a, item, tid, cur, block);
-  const int slot = item / a.Hv, hv = item % a.Hv;
+  const int slot = a.heads.quotient(item), hv = item - slot * a.Hv;
   const size_t slotT = (size_t)slot * T;
   const size_t sbase = (size_t)item * 128 * 128;
   f32x4_t (&st)[2][8] = cur.st;
   uint2 (&z2)[2] = cur.z2, (&w2)[2] = cur.w2;
   f32x4_t (&z4)[2] = cur.z4, (&w4)[2] = cur.w4;
   if constexpr (BLOCK) {
-    const int seg = tid & 15, per = a.Hv / a.Hk, hk = hv / per, C = (2 * a.Hk + a.Hv) * 128;
+    const int seg = tid & 15, hk = a.group.quotient(hv), C = (2 * a.Hk + a.Hv) * 128;
     // every wave its four steps of q, k and v, of up to four steps in all one of the three
     const bool few = T <= 4;
     const int t = few ? lane >> 4 : tid >> 4;
@@ -734,7 +735,7 @@ void gdn_forward_chunk_128(GdnArgs a) {
       const int pitch = j == 2 ? 128 : kKPad;
       float x[8] = {};
       if (few ? wave == j : 4 * wave < T) {
-        const bool keeps = j == 2 || hv % per == 0;  // a key head's: by the first of its value heads
+        const bool keeps = j == 2 || hv == hk * (int)a.group.by;  // a key head's: by the first of its value heads
         convolve(a.block, slot, t, T, C, block_channel(a, j, hv, hk, seg), keeps, block.rows[j], x);
         if (j < 2) normalise<8, 16>(x, j == 1 ? a.block.scale_k : a.block.scale_q, a.block.eps);
         if (j == 1 && keeps && t < T && a.block.k_out != nullptr)
@@ -1139,6 +1140,7 @@ int gdn_forward_launch(const char* who, const void* q, const void* k, const void
   a.q = q; a.k = k; a.v = v; a.g = g; a.beta = beta; a.state_in = state_in; a.state_out = state_out;
   a.y = y; a.tape = tape; a.mask = mask;
   a.T = T; a.Hk = Hk; a.Hv = Hv; a.Dk = Dk; a.Dv = Dv;
+  a.heads = Divisor::of(Hv); a.group = Divisor::of(Hv / Hk); a.row_parts = Divisor::of(1);
   a.in_dtype = in_dtype; a.g_dtype = g_dtype; a.beta_dtype = beta_dtype; a.state_dtype = state_dtype;
   a.g_per_dk = g_per_dk ? 1 : 0;
   a.z = z; a.z_batch = z_batch; a.z_row = z_row; a.norm_weight = norm_weight; a.weight_dtype = weight_dtype; a.eps = eps;
@@ -1181,6 +1183,7 @@ int gdn_forward_launch(const char* who, const void* q, const void* k, const void
       else hipLaunchKernelGGL((gdn_forward_chunk_128<false, false, false, false>), grid, block, lds, s, a);
     }
   } else if (by_rows != nullptr) {
+    a.row_parts = Divisor::of(Dv / rows);
     void* args[] = {&a};
     DFLASH_HIP_OK(hipLaunchKernel(by_rows, dim3((unsigned)(slots * Hv * (Dv / rows))), block, args, 0, s));
   } else if (fast) {
@@ -1247,6 +1250,7 @@ extern "C" int dflash_gdn_block(const dflash_gdn_block_args* p, void* stream) {
   GdnArgs a = {};
   a.state_in = p->state_in; a.state_out = p->state_out; a.y = p->y; a.tape = p->tape;
   a.T = T; a.Hk = Hk; a.Hv = Hv; a.Dk = a.Dv = D;
+  a.heads = Divisor::of(Hv); a.group = Divisor::of(Hv / Hk); a.row_parts = Divisor::of(1);
   a.in_dtype = a.g_dtype = a.beta_dtype = DFLASH_BF16; a.state_dtype = p->state_dtype;
   a.z = p->z; a.z_batch = p->z_slot; a.z_row = p->z_row; a.norm_weight = p->norm_weight; a.weight_dtype = p->weight_dtype;
   a.eps = p->norm_eps;
@@ -1269,6 +1273,7 @@ extern "C" int dflash_gdn_block(const dflash_gdn_block_args* p, void* stream) {
   }
   int rows = D;
   const void* fn = forward_rows_for<true>(p->state_dtype, slots, Hv, D, D, &rows);
+  a.row_parts = Divisor::of(D / rows);
   DFLASH_HIP_OK(hipLaunchKernel(fn, dim3((unsigned)(slots * Hv * (D / rows))), dim3(kThreads), args, 0, s));
   return p->z ? gdn_gated_norm_launch(p->y, p->z, p->norm_weight, p->y, slots, T, Hv, D, p->z_slot, p->z_row, DFLASH_BF16, p->weight_dtype,
                                       p->norm_eps, s)

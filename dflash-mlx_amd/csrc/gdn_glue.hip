@@ -47,6 +47,7 @@ struct PrepareArgs {
   void* qkv_out;           // [B, S, C]: qkv with masked rows zeroed, or null
   long long qkv_batch, qkv_row, a_batch, a_row, b_batch, b_row;  // strides, elements
   int tokens;              // per wave
+  Divisor heads, runs;     // by the waves of a run of tokens, by the runs of a batch element
   int B, S, Hk, Hv, Dk, Dv, param_dt;
   float eps, scale_q, scale_k;  // scales already rounded to the array dtype
 };
@@ -183,11 +184,11 @@ __device__ __forceinline__ void prepare_head(const PrepareArgs& p, int b, int s0
 template <int DT, int K>
 __global__ __launch_bounds__(kWavesPerGroup * 64) void gdn_prepare_kernel(PrepareArgs p) {
   const int lane = threadIdx.x & 63;
-  const int heads = 2 * p.Hk + p.Hv, runs = (p.S + p.tokens - 1) / p.tokens;
+  const int heads = (int)p.heads.by, runs = (int)p.runs.by;
   const int w = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * kWavesPerGroup + (threadIdx.x >> 6)));
   if (w >= p.B * runs * heads) return;
-  const int h = w % heads, run = w / heads;
-  const int b = run / runs, s0 = (run - b * runs) * p.tokens;
+  const int run = p.heads.quotient(w), h = w - run * heads;
+  const int b = p.runs.quotient(run), s0 = (run - b * runs) * p.tokens;
   const int s1 = s0 + p.tokens < p.S ? s0 + p.tokens : p.S;
   const bool is_v = h >= 2 * p.Hk;
   switch ((is_v ? p.Dv : p.Dk) / 64) {
@@ -203,11 +204,11 @@ template <int DT, int K, int LANES>
 __global__ __launch_bounds__(kWavesPerGroup * 64) void gdn_prepare_wide_kernel(PrepareArgs p) {
   constexpr int kHeads = 64 / LANES;
   const int lane = threadIdx.x & 63;
-  const int groups = (2 * p.Hk + p.Hv) / kHeads, runs = (p.S + p.tokens - 1) / p.tokens;
+  const int groups = (int)p.heads.by, runs = (int)p.runs.by;
   const int w = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * kWavesPerGroup + (threadIdx.x >> 6)));
   if (w >= p.B * runs * groups) return;
-  const int h0 = w % groups * kHeads, run = w / groups;
-  const int b = run / runs, s0 = (run - b * runs) * p.tokens;
+  const int run = p.heads.quotient(w), h0 = (w - run * groups) * kHeads;
+  const int b = p.runs.quotient(run), s0 = (run - b * runs) * p.tokens;
   const int s1 = s0 + p.tokens < p.S ? s0 + p.tokens : p.S;
   prepare_head<DT, 8, K, LANES>(p, b, s0, s1, h0 >= 2 * p.Hk, h0 + lane / LANES, lane % LANES);
 }
@@ -235,6 +236,7 @@ struct NormArgs {
   void* y;             // like x
   long long z_batch, z_row;
   int rows, T, H;      // rows = B T H
+  Divisor heads, tokens;  // by H, by T
   int per_wave;        // rows of a wave
   int D, weight_dt;
   float eps;
@@ -246,7 +248,7 @@ __device__ __forceinline__ void gated_norm_rows(const NormArgs& p, int row, int 
   constexpr bool wide = DT == DFLASH_FP32;
   uint32_t xr[PER], zr[PER], wr[PER];
   auto load = [&](int r) __attribute__((always_inline)) {
-    const int token = r / p.H, h = r - token * p.H, b = token / p.T, t = token - b * p.T;
+    const int token = p.heads.quotient(r), h = r - token * p.H, b = p.tokens.quotient(token), t = token - b * p.T;
     load_adjacent_raw<PER>(p.x, (size_t)r * p.D + PER * lane, wide, xr);
     load_adjacent_raw<PER>(p.z, (size_t)b * p.z_batch + (size_t)t * p.z_row + (size_t)h * p.D + PER * lane, wide, zr);
   };
@@ -370,7 +372,9 @@ extern "C" int dflash_gdn_prepare_rows(const void* qkv, const void* conv_state, 
     const long long each = ((long long)B * S * heads / per_wave + 4095) / 4096, most = Dk / 8 < 16 ? Dk / 8 : 16;
     p.tokens = (int)(each > most ? most : each);  // (a lane of the head computes a token's gates)
   }
-  const long long waves = (long long)B * ((S + p.tokens - 1) / p.tokens) * (wide ? heads / per_wave : heads);
+  p.runs = Divisor::of((S + p.tokens - 1) / p.tokens);
+  p.heads = Divisor::of(wide ? heads / per_wave : heads);
+  const long long waves = (long long)B * p.runs.by * p.heads.by;
   const unsigned groups = (unsigned)((waves + kWavesPerGroup - 1) / kWavesPerGroup);
   const void* fn = wide ? (dtype == DFLASH_BF16 ? wide_kernel_for<DFLASH_BF16>(Dk, conv_kernel)
                                                 : wide_kernel_for<DFLASH_FP16>(Dk, conv_kernel))
@@ -401,6 +405,7 @@ int gdn_gated_norm_launch(const void* x, const void* z, const void* weight, void
   p.x = x; p.z = z; p.weight = weight; p.y = y;
   p.z_batch = z_batch; p.z_row = z_row;
   p.rows = B * T * H; p.T = T; p.H = H; p.D = D;
+  p.heads = Divisor::of(H); p.tokens = Divisor::of(T);
   p.weight_dt = weight_dtype; p.eps = eps;
   p.per_wave = p.rows / 8192 < 1 ? 1 : p.rows / 8192 > 16 ? 16 : p.rows / 8192;
   // eight elements per lane and several rows per wave where that leaves 4 waves per SIMD: 12.3 -> 10.1 us (32 768 rows of 128)

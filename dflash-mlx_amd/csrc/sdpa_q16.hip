@@ -62,6 +62,7 @@ struct SdpaArgs {
   long long k_batch_stride, k_head_stride, k_seq_stride;
   long long v_batch_stride, v_head_stride, v_seq_stride;
   int B, Hq, Hk, N, G, splits, keys_per_split;
+  Divisor ranges, key_heads, heads;  // by splits, Hk, Hq
   float scale, lowest;   // lowest finite value of the input dtype
 };
 
@@ -103,15 +104,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int split = blockIdx.x % a.splits;
-  const int bh = blockIdx.x / a.splits;
-  const int b = bh / a.Hk, hk = bh % a.Hk;
+  const int bh = a.ranges.quotient((int)blockIdx.x), split = (int)blockIdx.x - bh * a.splits;
+  const int b = a.key_heads.quotient(bh), hk = bh - b * a.Hk;
   const int n_begin = split * a.keys_per_split;
   const int n_end = n_begin + a.keys_per_split < a.N ? n_begin + a.keys_per_split : a.N;
   const int j = lane & 15, kb = lane >> 4;
   const bool computes = wave < a.G * CS;  // the other waves only move tiles
-  const int slice = computes ? wave / a.G : 0;
-  const int hq = hk * a.G + (computes ? wave % a.G : 0);
+  int slice = 0, of_group = computes ? wave : 0;  // wave / G, wave % G
+  while (of_group >= a.G) of_group -= a.G, ++slice;
+  const int hq = hk * a.G + of_group;
   const size_t qrow = ((size_t)b * a.Hq + hq) * 16 + j;  // this lane's query
 
   const uint16_t* kbase = a.k + (size_t)b * a.k_batch_stride + (size_t)hk * a.k_head_stride;
@@ -305,7 +306,7 @@ __global__ __launch_bounds__(256) void sdpa_q16_merge_kernel(SdpaArgs a, int D) 
   };
   issue_round(g);
   // (b, hq, i) of the row; the gate is asked for with the partial results
-  const int i = (int)(row % 16), hq = (int)(row / 16 % a.Hq), b = (int)(row / (16 * (size_t)a.Hq));
+  const int i = (int)blockIdx.x % 16, head = (int)blockIdx.x / 16, b = a.heads.quotient(head), hq = head - b * a.Hq;
   uint2 gate = uint2{0u, 0u};
   if (a.gate != nullptr && g == 0 && col)
     gate = *reinterpret_cast<const uint2*>(a.gate + b * a.gate_batch_stride + i * a.gate_row_stride + (size_t)hq * 2 * D + D + 4 * c4);
@@ -432,6 +433,7 @@ int sdpa_launch(const void* q, const void* k, const void* v, const void* mask, c
   a.v_batch_stride = v_batch_stride; a.v_head_stride = v_head_stride; a.v_seq_stride = v_seq_stride;
   a.B = B; a.Hq = Hq; a.Hk = Hk; a.N = N; a.G = Hq / Hk;
   a.splits = pick_splits(B, Hk, N, &a.keys_per_split);
+  a.ranges = Divisor::of(a.splits); a.key_heads = Divisor::of(Hk); a.heads = Divisor::of(Hq);
   a.scale = scale;
   a.lowest = dtype == DFLASH_FP16 ? -65504.0f : -3.3895313892515355e38f;
   a.gate = (const uint16_t*)gate;

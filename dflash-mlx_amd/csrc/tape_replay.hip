@@ -36,6 +36,7 @@ struct ReplayArgs {
   const uint8_t* mask;
   int steps_host;
   int T, Hk, Hv, Dk, Dv;
+  Divisor heads, group, row_parts;  // by Hv, by Hv / Hk, by the workgroups of a head (replay_rows)
   int state_dtype, tape_dtype, k_dtype, g_dtype, g_per_dk;
   // the conv window of the same layer, rebuilt by workgroups behind the replay's (none: conv_keep 0)
   const char* conv_prev;
@@ -178,7 +179,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3, 3))
   float* sG = sD + 16 * kPad;
   float* sGt = sG + 16 * 128;
   if (conv_window_workgroup(a)) return;
-  const int slot = blockIdx.x / a.Hv, hv = blockIdx.x % a.Hv;
+  const int slot = a.heads.quotient((int)blockIdx.x), hv = (int)blockIdx.x - slot * a.Hv;
   const int n = slot_steps(a, slot);
   const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, kq = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -201,7 +202,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3, 3))
   u32x4_t rd0 = {0u, 0u, 0u, 0u}, rd1 = rd0, rk0 = rd0, rk1 = rd0, rg0 = rd0, rg1 = rd0;
   uint32_t mask_t = 1u;
   {
-    const int hk = hv / (a.Hv / a.Hk);
+    const int hk = a.group.quotient(hv);
     const size_t slotT = (size_t)slot * a.T;
     if (row) {
       const size_t d_at = ((slotT + t) * a.Hv + hv) * 128 + 8 * seg;
@@ -327,8 +328,8 @@ __global__ __launch_bounds__(kThreads) void replay_rows(ReplayArgs a) {
   __shared__ __align__(16) float sD[16 * kRows];
   __shared__ float sG[16];
   if (conv_window_workgroup(a)) return;
-  const int per = a.Dv / kRows, head = (int)blockIdx.x / per, row0 = ((int)blockIdx.x - head * per) * kRows;
-  const int slot = head / a.Hv, hv = head % a.Hv, hk = hv / (a.Hv / a.Hk);
+  const int head = a.row_parts.quotient((int)blockIdx.x), row0 = ((int)blockIdx.x - head * (int)a.row_parts.by) * kRows;
+  const int slot = a.heads.quotient(head), hv = head - slot * a.Hv, hk = a.group.quotient(hv);
   const int n = slot_steps(a, slot);
   const int tid = threadIdx.x, t = tid >> 4, seg = tid & 15;
   const size_t slotT = (size_t)slot * a.T;
@@ -600,6 +601,7 @@ int replay_launch(const void* tape, const void* k, const void* g, const void* st
   a.tape = tape; a.k = k; a.g = g; a.state_in = state_in; a.state_out = state_out;
   a.steps_dev = steps_dev; a.mask = mask; a.steps_host = steps_host;
   a.T = T; a.Hk = Hk; a.Hv = Hv; a.Dk = Dk; a.Dv = Dv;
+  a.heads = Divisor::of(Hv); a.group = Divisor::of(Hv / Hk); a.row_parts = Divisor::of(by_rows ? Dv / rows : 1);
   a.state_dtype = state_dtype; a.tape_dtype = tape_dtype; a.k_dtype = k_dtype;
   a.g_dtype = g_dtype; a.g_per_dk = g_per_dk ? 1 : 0;
   const long long blocks = (long long)slots * Hv * (by_rows ? Dv / rows : 1);
