@@ -192,14 +192,18 @@ __device__ __forceinline__ void product(const Args& p) {
 
   // x first (from the weights on, a request waits for theirs): 256 bytes of four rows a load; rows past M and chunks past `mine` are zeros
   u32x4_t xr[MT][NCH][4];
+  // (MT = 1: loads of rows that are all absent are left out; the last rows go first, so that what follows a load that may be left out are loads
+  // that are not, and a wait for any of them counts those only)  (A token through 5120 x 34816 with silu 25.0 -> 23.7 us,
+  // 17408 x 5120 16.3 -> 15.7, 4096 x 24576 with silu 15.0 -> 14.6; 16 rows as before.)
 #pragma unroll
-  for (int m = 0; m < MT; ++m)
+  for (int j = 3; j >= 0; --j)
 #pragma unroll
-    for (int c = 0; c < NCH; ++c)
+    for (int m = 0; m < MT; ++m)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int c = 0; c < NCH; ++c) {
         const uint32_t at = (uint32_t)(16 * m + 4 * j + q) * (uint32_t)K * 2u + 256u * (uint32_t)(first + c) + 16u * li;
-        xr[m][c][j] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(x_buf, c < mine ? at : kPast, 0, 0));
+        if (MT == 1 && j > 0 && p.M <= 4 * j) xr[m][c][j] = u32x4_t{0u, 0u, 0u, 0u};
+        else xr[m][c][j] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(x_buf, c < mine ? at : kPast, 0, 0));
       }
   __builtin_amdgcn_sched_barrier(0);
 
