@@ -559,8 +559,9 @@ constexpr int kOffC = kOffM + 256;
 constexpr int kOffBeta = kOffC + 16;   // 0 for masked and missing steps
 constexpr int kOffGate = kOffBeta + 16;  // 1 for masked and missing steps
 constexpr int kOffOn = kOffGate + 16;    // 1 for steps that count, 0 for masked and missing ones
-constexpr int kOffSS = kOffOn + 16;      // [wave][step]: a wave's share of a step's sum of squares
-constexpr int kChunkLdsFloats = kOffSS + 64;
+constexpr int kOffSS = kOffOn + 16;      // [tile of 16 rows][step]: its share of a step's sum of squares
+constexpr int kChunkLdsFloats = kOffSS + 128;
+constexpr int kBlockThreads = 9 * 64;  // BLOCK: eight waves with a tile of 16 rows of S each, one for what a head has once
 
 // Four consecutive elements at element i (a multiple of 4) of a 16-byte aligned array.
 __device__ __forceinline__ void store4_from_f32(void* p, size_t i, f32x4_t v, int dt) {
@@ -595,25 +596,26 @@ __device__ __forceinline__ f32x4_t mfma16_bf16(const uint32_t (&a)[2], const uin
 }
 
 // What one (slot, head) item brings in from memory, as it sits in registers while in flight.
-template <bool WIDE>
+template <bool WIDE, int TILES>
 struct Incoming {
   Raw8<WIDE> k, q, v;
   uint32_t gate_bits, beta_bits, mask_byte;  // of step tid (threads below 16), as loaded
   // fused output norm: this lane's four columns of z (step li) and of the norm weight per row tile
-  uint2 z2[2], w2[2];    // 16-bit elements
-  f32x4_t z4[2], w4[2];  // fp32 elements
-  f32x4_t st[2][8];
+  uint2 z2[TILES], w2[TILES];    // 16-bit elements
+  f32x4_t z4[TILES], w4[TILES];  // fp32 elements
+  f32x4_t st[TILES][8];
 };
 struct BlockIncoming {
-  ConvRows<8> rows[3];  // q, k, v
-  GateBits gates;
+  ConvRows<4> rows[3];  // q, k, v
 };
 // Channel of lane group `seg` in q (0), k (1) or v (2).
 __device__ __forceinline__ int block_channel(const GdnArgs& a, int which, int hv, int hk, int seg) {
-  return (which == 0 ? hk : which == 1 ? a.Hk + hk : 2 * a.Hk + hv) * 128 + 8 * seg;
+  return (which == 0 ? hk : which == 1 ? a.Hk + hk : 2 * a.Hk + hv) * 128 + 4 * seg;
 }
-template <bool WIDE, bool NORM, bool BLOCK>
-__device__ __forceinline__ void issue_item_loads(const GdnArgs& a, int item, int tid, Incoming<WIDE>& in, BlockIncoming& block) {
+// Step of a block's lane: two steps a wave; of up to four steps in all the first two waves have q, the next two k, the next two v.
+__device__ __forceinline__ int block_step(bool few, int wave, int lane) { return 2 * (few ? wave & 1 : wave) + (lane >> 5); }
+template <bool WIDE, bool NORM, bool BLOCK, int TILES>
+__device__ __forceinline__ void issue_item_loads(const GdnArgs& a, int item, int tid, Incoming<WIDE, TILES>& in, BlockIncoming& block) {
   const int T = a.T;
   const int slot = a.heads.quotient(item), hv = item - slot * a.Hv, hk = a.group.quotient(hv);
   const size_t slotT = (size_t)slot * T;
@@ -625,8 +627,7 @@ __device__ __forceinline__ void issue_item_loads(const GdnArgs& a, int item, int
   if constexpr (BLOCK) {
 #pragma unroll
     for (int j = 0; j < 3; ++j)
-      request_rows(a.block, slot, T <= 4 ? lane >> 4 : t, T, (2 * a.Hk + a.Hv) * 128, block_channel(a, j, hv, hk, seg), block.rows[j]);
-    block.gates = request_gates(a.block, slot, lane < T ? lane : T - 1, hv);
+      request_rows(a.block, slot, block_step(T <= 4, wave, lane), T, (2 * a.Hk + a.Hv) * 128, block_channel(a, j, hv, hk, lane & 31), block.rows[j]);
   } else if (t < T) {
     const size_t kq_at = ((slotT + t) * a.Hk + hk) * 128 + 8 * seg;
     const size_t v_at = ((slotT + t) * a.Hv + hv) * 128 + 8 * seg;
@@ -659,8 +660,8 @@ __device__ __forceinline__ void issue_item_loads(const GdnArgs& a, int item, int
     const size_t zb = (size_t)slot * a.z_batch + (size_t)tz * a.z_row + (size_t)hv * 128;
     const bool wwide = a.weight_dtype == DFLASH_FP32;
 #pragma unroll
-    for (int t2 = 0; t2 < 2; ++t2) {
-      const int col = 32 * wave + 16 * t2 + 4 * kq;
+    for (int t2 = 0; t2 < TILES; ++t2) {
+      const int col = 16 * (TILES * wave + t2) + 4 * kq;
       if (WIDE) {
         in.z4[t2] = *reinterpret_cast<const f32x4_t*>((const float*)a.z + zb + col);
       } else {
@@ -675,25 +676,109 @@ __device__ __forceinline__ void issue_item_loads(const GdnArgs& a, int item, int
   }
   const f32x4_t* src = reinterpret_cast<const f32x4_t*>((const float*)a.state_in + (size_t)item * 128 * 128);
 #pragma unroll
-  for (int t2 = 0; t2 < 2; ++t2)
+  for (int t2 = 0; t2 < TILES; ++t2)
 #pragma unroll
     for (int c = 0; c < 8; ++c)
-      in.st[t2][c] = __builtin_nontemporal_load(&src[memory_index(wave, li, kq, t2, c)]);
+      in.st[t2][c] = __builtin_nontemporal_load(&src[memory_index((TILES * wave + t2) >> 1, li, kq, (TILES * wave + t2) & 1, c)]);
   // Fence: everything above is on its way before the first of these values is looked at.
   asm volatile("" : "+v"(in.gate_bits), "+v"(in.beta_bits), "+v"(in.mask_byte)::"memory");
+}
+// Element j = 4h + e (h = 0, 1) of a lane's operand is column 16 (2C + h) + 4kq + e: the 32
+// columns 32C .. 32C + 31 over the four lane groups, the same on both sides of a product.
+__device__ __forceinline__ void block_operands(const float* sK, const float* sQ, int li, int kq, int C, uint32_t (&kb)[4], uint32_t (&qb)[4]) {
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const float4 kf4 = *reinterpret_cast<const float4*>(sK + li * kKPad + 16 * (2 * C + h) + 4 * kq);
+    const float4 qf4 = *reinterpret_cast<const float4*>(sQ + li * kKPad + 16 * (2 * C + h) + 4 * kq);
+    kb[2 * h] = upper_halves(kf4.x, kf4.y), kb[2 * h + 1] = upper_halves(kf4.z, kf4.w);
+    qb[2 * h] = upper_halves(qf4.x, qf4.y), qb[2 * h + 1] = upper_halves(qf4.z, qf4.w);
+  }
+}
+// A barrier that does not wait for memory: __syncthreads() would, for the state on its way in and every store on its way out.
+__device__ __forceinline__ void bare_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n s_barrier" ::: "memory"); }
+// c_t / c_s = prod_{s < u <= t} g_u for s <= t at 16 t + s, and c_t itself
+__device__ __forceinline__ void gate_ratios(const float* sGate, float* sRat, float* sC, int at) {
+  const int t = at >> 4, sx = at & 15;
+  float gates[16];
+#pragma unroll
+  for (int u = 0; u < 16; u += 4) {
+    const float4 g4 = *reinterpret_cast<const float4*>(sGate + u);
+    gates[u] = g4.x, gates[u + 1] = g4.y, gates[u + 2] = g4.z, gates[u + 3] = g4.w;
+  }
+  float r = sx <= t ? 1.f : 0.f;
+#pragma unroll
+  for (int u = 1; u < 16; ++u) r *= (u > sx && u <= t) ? gates[u] : 1.f;
+  sRat[at] = r;
+  if (sx == 0) sC[t] = r * gates[0];
+}
+// M = (I + L)^-1 by forward substitution, column li per lane.  L[t][s] sits in lane 16 (s / 4) + t, register s % 4 of this wave and
+// reaches the others through v_readlane.
+__device__ __forceinline__ void unit_inverse(const float (&Lr)[4], float* sM, int li, int kq) {
+  float x[16];
+#pragma unroll
+  for (int tt = 0; tt < 16; ++tt) {
+    float acc = tt == li ? 1.f : 0.f;
+#pragma unroll
+    for (int sx = 0; sx < tt; ++sx) {
+      const float l = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(Lr[sx & 3]), 16 * (sx >> 2) + tt));
+      acc -= l * x[sx];
+    }
+    x[tt] = acc;
+    if (kq == 0) sM[tt * 16 + li] = acc;
+  }
+}
+// BLOCK: the wave without rows of S.  Gates, beta and their ratios while the others have the conv, Lq and M while they have the products
+// with S0; two barriers, which the others meet it at.
+__device__ __forceinline__ void block_gates(const GdnArgs& a, int slot, int hv, int lane, float* smem) {
+  const int T = a.T, li = lane & 15, kq = lane >> 4;
+  float* const sK = smem + kOffK;
+  float* const sQ = smem + kOffQ;
+  float* const sRat = smem + kOffRat;
+  float* const sGate = smem + kOffGate;
+  const GateBits bits = request_gates(a.block, slot, lane < T ? lane : T - 1, hv);
+  if (lane < 16) {
+    const float g = lane < T ? gate_of(a.block, bits) : 1.f;
+    if (lane < T && a.block.g_out != nullptr) a.block.g_out[((size_t)slot * T + lane) * a.Hv + hv] = g;
+    sGate[lane] = g;
+    smem[kOffBeta + lane] = lane < T ? beta_of(bits) : 0.f;
+    smem[kOffOn + lane] = lane < T ? 1.f : 0.f;
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < 4; ++i) gate_ratios(sGate, sRat, smem + kOffC, 64 * i + lane);
+  bare_barrier();
+  f32x4_t kk = {0.f, 0.f, 0.f, 0.f}, kq_sum = {0.f, 0.f, 0.f, 0.f};  // [s][t] = k_s . k_t and k_s . q_t
+#pragma unroll
+  for (int C = 0; C < 4; ++C) {
+    uint32_t kb[4], qb[4];
+    block_operands(sK, sQ, li, kq, C, kb, qb);
+    kk = mfma32_bf16(kb, kb, kk);
+    kq_sum = mfma32_bf16(kb, qb, kq_sum);
+  }
+  const float bt = smem[kOffBeta + li];
+  float Lr[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int sx = 4 * kq + r;
+    const float rat = sRat[li * 16 + sx];  // 0 for s > t
+    Lr[r] = sx < li ? bt * rat * kk[r] : 0.f;
+    smem[kOffLq + li * 16 + sx] = rat * kq_sum[r];
+  }
+  unit_inverse(Lr, smem + kOffM, li, kq);
+  bare_barrier();
 }
 // One workgroup per (slot, head); the register cap keeps at least three on a compute unit.
 // SPLIT: q and k are bf16 arrays; the products with S0 and the state update run on the bf16
 // matrix cores with the fp32 factor in three exact pieces (see split_bf16).
 // BLOCK: q, k, v, the gates and beta are made here, from the block's projections (gdn_block_device.h), while the state is on its
-// way.  A launch of the prepare kernel before this one took 5.4 us for what is 0.4 MB, and a microsecond to the next; here it is
-// 3.3 us of vector instructions (32 of 256 compute units have a head to work on): 16 tokens of 32 heads 13.3 + 5.4 -> 16.6 us, the
-// layer's verify block with its rollback 49.2 -> 47.1 us of device time, one token through a layer of 16-bit states (gdn_forward_rows)
-// 30.0 -> 25.1.  256 registers instead of 168: the rows, the taps and the state are all in flight at once, and a launch
-// this small has no second workgroup for a compute unit.
+// way.  A launch of the prepare kernel before this one took 5.4 us for what is 0.4 MB, and a microsecond to the next.  32 of 256 compute units
+// have a head to work on and nothing beside it, so what counts is the longest chain of a head: eight waves with a tile of rows each, two to a
+// SIMD, fill each other's waits, and a ninth has what a head has once, gates, ratios and (I + L)^-1, beside the conv and the products with S0.
+// 16 tokens of 32 heads 16.9 -> 13.8 us (four waves of two tiles, the second of them with the inverse).
 template <bool WIDE, bool NORM, bool SPLIT, bool BLOCK>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(BLOCK ? 2 : 3, BLOCK ? 2 : 3)))
+__global__ __launch_bounds__(BLOCK ? kBlockThreads : kThreads) __attribute__((amdgpu_waves_per_eu(3, 3)))
 void gdn_forward_chunk_128(GdnArgs a) {
+  constexpr int TILES = BLOCK ? 1 : 2;  // of 16 rows of S to a wave
   extern __shared__ __align__(16) float smem[];
   float* sK = smem + kOffK;
   float* sQ = smem + kOffQ;
@@ -714,52 +799,48 @@ void gdn_forward_chunk_128(GdnArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // scalar: branches on it are real branches
   const int li = lane & 15, kq = lane >> 4;
 
-  Incoming<WIDE> cur;
   const int item = blockIdx.x;
-  BlockIncoming block;
-  issue_item_loads<WIDE, NORM, BLOCK>(a, item, tid, cur, block);
   const int slot = a.heads.quotient(item), hv = item - slot * a.Hv;
   const size_t slotT = (size_t)slot * T;
-  const size_t sbase = (size_t)item * 128 * 128;
-  f32x4_t (&st)[2][8] = cur.st;
-  uint2 (&z2)[2] = cur.z2, (&w2)[2] = cur.w2;
-  f32x4_t (&z4)[2] = cur.z4, (&w4)[2] = cur.w4;
   if constexpr (BLOCK) {
-    const int seg = tid & 15, hk = a.group.quotient(hv), C = (2 * a.Hk + a.Hv) * 128;
-    // every wave its four steps of q, k and v, of up to four steps in all one of the three
+    if (wave == kBlockThreads / 64 - 1) {
+      block_gates(a, slot, hv, lane, smem);
+      return;
+    }
+  }
+  Incoming<WIDE, TILES> cur;
+  BlockIncoming block;
+  issue_item_loads<WIDE, NORM, BLOCK, TILES>(a, item, tid, cur, block);
+  const size_t sbase = (size_t)item * 128 * 128;
+  f32x4_t (&st)[TILES][8] = cur.st;
+  uint2 (&z2)[TILES] = cur.z2, (&w2)[TILES] = cur.w2;
+  f32x4_t (&z4)[TILES] = cur.z4, (&w4)[TILES] = cur.w4;
+  if constexpr (BLOCK) {
+    const int seg = lane & 31, hk = a.group.quotient(hv), C = (2 * a.Hk + a.Hv) * 128;
+    // every wave its two steps of q, k and v, of up to four steps in all one of the three
     const bool few = T <= 4;
-    const int t = few ? lane >> 4 : tid >> 4;
+    const int t = block_step(few, wave, lane);
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
       float* const dst = j == 0 ? sQ : j == 1 ? sK : sV;
       const int pitch = j == 2 ? 128 : kKPad;
-      float x[8] = {};
-      if (few ? wave == j : 4 * wave < T) {
+      float x[4] = {};
+      if (few ? wave >> 1 == j : 2 * wave < T) {
         const bool keeps = j == 2 || hv == hk * (int)a.group.by;  // a key head's: by the first of its value heads
         convolve(a.block, slot, t, T, C, block_channel(a, j, hv, hk, seg), keeps, block.rows[j], x);
-        if (j < 2) normalise<8, 16>(x, j == 1 ? a.block.scale_k : a.block.scale_q, a.block.eps);
+        if (j < 2) normalise<4, 32>(x, j == 1 ? a.block.scale_k : a.block.scale_q, a.block.eps);
         if (j == 1 && keeps && t < T && a.block.k_out != nullptr)
-          store_exact<8>(a.block.k_out + ((slotT + t) * a.Hk + hk) * 128 + 8 * seg, x);
+          store_exact<4>(a.block.k_out + ((slotT + t) * a.Hk + hk) * 128 + 4 * seg, x);
       }
       const auto put = [&](int step, bool on) __attribute__((always_inline)) {
-#pragma unroll
-        for (int e = 0; e < 8; e += 4)
-          *reinterpret_cast<f32x4_t*>(dst + step * pitch + 8 * seg + e) =
-              on ? f32x4_t{x[e], x[e + 1], x[e + 2], x[e + 3]} : f32x4_t{0.f, 0.f, 0.f, 0.f};
+        *reinterpret_cast<f32x4_t*>(dst + step * pitch + 4 * seg) = on ? f32x4_t{x[0], x[1], x[2], x[3]} : f32x4_t{0.f, 0.f, 0.f, 0.f};
       };
       if (!few) {
         put(t, t < T);
-      } else if (wave == j) {
+      } else if (wave >> 1 == j) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) put(4 * i + t, i == 0 && t < T);
       }
-    }
-    if (wave == 3 && lane < 16) {
-      const float g = lane < T ? gate_of(a.block, block.gates) : 1.f;
-      if (lane < T && a.block.g_out != nullptr) a.block.g_out[(slotT + lane) * a.Hv + hv] = g;
-      sGate[lane] = g;
-      sBeta[lane] = lane < T ? beta_of(block.gates) : 0.f;
-      sOn[lane] = lane < T ? 1.f : 0.f;
     }
   } else {
     const int t = tid >> 4, seg = tid & 15;
@@ -773,46 +854,29 @@ void gdn_forward_chunk_128(GdnArgs a) {
     sBeta[tid] = on ? bits_as_f32(cur.beta_bits, a.beta_dtype) : 0.f;
     sOn[tid] = on ? 1.f : 0.f;
   }
-  __syncthreads();
-  {  // c_t / c_s = prod_{s < u <= t} g_u for s <= t, and c_t itself
-    const int t = tid >> 4, sx = tid & 15;
-    float gates[16];
-#pragma unroll
-    for (int u = 0; u < 16; u += 4) {
-      const float4 g4 = *reinterpret_cast<const float4*>(sGate + u);
-      gates[u] = g4.x, gates[u + 1] = g4.y, gates[u + 2] = g4.z, gates[u + 3] = g4.w;
-    }
-    float r = sx <= t ? 1.f : 0.f;
-#pragma unroll
-    for (int u = 1; u < 16; ++u) r *= (u > sx && u <= t) ? gates[u] : 1.f;
-    sRat[tid] = r;
-    if (sx == 0) sC[t] = r * gates[0];
+  if constexpr (BLOCK) {
+    bare_barrier();  // (nobody waits for the state here)
+  } else {
+    __syncthreads();
+    gate_ratios(sGate, sRat, sC, tid);
+    __syncthreads();
   }
-  __syncthreads();
 
   // ---- U = S0 K^T, W = S0 Q^T (every wave, its 32 rows); K K^T (wave 1), K Q^T (wave 2) -------
 #pragma unroll
-  for (int t2 = 0; t2 < 2; ++t2)
+  for (int t2 = 0; t2 < TILES; ++t2)
 #pragma unroll
     for (int m = 0; m < 4; ++m) swap_row_bit(st[t2][2 * m], st[t2][2 * m + 1]);
-  f32x4_t U[2], W[2], X = {0.f, 0.f, 0.f, 0.f};
+  f32x4_t U[TILES], W[TILES], X = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int t2 = 0; t2 < 2; ++t2) U[t2] = f32x4_t{0.f, 0.f, 0.f, 0.f}, W[t2] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int t2 = 0; t2 < TILES; ++t2) U[t2] = f32x4_t{0.f, 0.f, 0.f, 0.f}, W[t2] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   if constexpr (SPLIT) {
-    // Element j = 4h + e (h = 0, 1) of a lane's operand is column 16 (2C + h) + 4kq + e: the 32
-    // columns 32C .. 32C + 31 over the four lane groups, the same on both sides of a product.
 #pragma unroll
     for (int C = 0; C < 4; ++C) {
       uint32_t kb[4], qb[4];
+      block_operands(sK, sQ, li, kq, C, kb, qb);
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const float4 kf4 = *reinterpret_cast<const float4*>(sK + li * kKPad + 16 * (2 * C + h) + 4 * kq);
-        const float4 qf4 = *reinterpret_cast<const float4*>(sQ + li * kKPad + 16 * (2 * C + h) + 4 * kq);
-        kb[2 * h] = upper_halves(kf4.x, kf4.y), kb[2 * h + 1] = upper_halves(kf4.z, kf4.w);
-        qb[2 * h] = upper_halves(qf4.x, qf4.y), qb[2 * h + 1] = upper_halves(qf4.z, qf4.w);
-      }
-#pragma unroll
-      for (int t2 = 0; t2 < 2; ++t2) {
+      for (int t2 = 0; t2 < TILES; ++t2) {
         const float f[8] = {st[t2][2 * C][0],     st[t2][2 * C][1],     st[t2][2 * C][2],     st[t2][2 * C][3],
                             st[t2][2 * C + 1][0], st[t2][2 * C + 1][1], st[t2][2 * C + 1][2], st[t2][2 * C + 1][3]};
         const Pieces<8> sp = split_bf16(f);
@@ -823,8 +887,8 @@ void gdn_forward_chunk_128(GdnArgs a) {
         U[t2] = mfma32_bf16(sp.hi, kb, U[t2]);
         W[t2] = mfma32_bf16(sp.hi, qb, W[t2]);
       }
-      if (wave == 1) X = mfma32_bf16(kb, kb, X);  // [s][t] = k_s . k_t
-      if (wave == 2) X = mfma32_bf16(kb, qb, X);  // [s][t] = k_s . q_t
+      if (!BLOCK && wave == 1) X = mfma32_bf16(kb, kb, X);  // [s][t] = k_s . k_t
+      if (!BLOCK && wave == 2) X = mfma32_bf16(kb, qb, X);  // [s][t] = k_s . q_t
     }
   } else {
 #pragma unroll
@@ -836,7 +900,7 @@ void gdn_forward_chunk_128(GdnArgs a) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
 #pragma unroll
-        for (int t2 = 0; t2 < 2; ++t2) {
+        for (int t2 = 0; t2 < TILES; ++t2) {
           U[t2] = mfma4(st[t2][c][e], kf[e], U[t2]);
           W[t2] = mfma4(st[t2][c][e], qf[e], W[t2]);
         }
@@ -849,57 +913,48 @@ void gdn_forward_chunk_128(GdnArgs a) {
     const int t = li;
     const float ct = sC[t], bt = sBeta[t];
     float Lr[4];  // wave 1: L[t][4kq + r], wave 2: Lq[t][4kq + r]
+    if constexpr (!BLOCK) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int sx = 4 * kq + r;
-      const float rat = sRat[t * 16 + sx];  // 0 for s > t
-      Lr[r] = wave == 1 ? (sx < t ? bt * rat * X[r] : 0.f) : rat * X[r];
-      if (wave == 2) sLq[t * 16 + sx] = Lr[r];
+      for (int r = 0; r < 4; ++r) {
+        const int sx = 4 * kq + r;
+        const float rat = sRat[t * 16 + sx];  // 0 for s > t
+        Lr[r] = wave == 1 ? (sx < t ? bt * rat * X[r] : 0.f) : rat * X[r];
+        if (wave == 2) sLq[t * 16 + sx] = Lr[r];
+      }
     }
 #pragma unroll
-    for (int t2 = 0; t2 < 2; ++t2) {
-      const int row0 = 32 * wave + 16 * t2 + 4 * kq;
+    for (int t2 = 0; t2 < TILES; ++t2) {
+      const int row0 = 16 * (TILES * wave + t2) + 4 * kq;
       const float4 v4 = *reinterpret_cast<const float4*>(sV + t * 128 + row0);
       sR[(row0 + 0) * kRPad + t] = bt * (v4.x - ct * U[t2][0]);
       sR[(row0 + 1) * kRPad + t] = bt * (v4.y - ct * U[t2][1]);
       sR[(row0 + 2) * kRPad + t] = bt * (v4.z - ct * U[t2][2]);
       sR[(row0 + 3) * kRPad + t] = bt * (v4.w - ct * U[t2][3]);
     }
-    // ---- M = (I + L)^-1 by forward substitution, column li per lane.  L[t][s] sits in lane
-    // 16 (s / 4) + t, register s % 4 of this wave and reaches the others through v_readlane.
-    if (wave == 1) {
-      float x[16];
-#pragma unroll
-      for (int tt = 0; tt < 16; ++tt) {
-        float acc = tt == li ? 1.f : 0.f;
-#pragma unroll
-        for (int sx = 0; sx < tt; ++sx) {
-          const float l = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(Lr[sx & 3]), 16 * (sx >> 2) + tt));
-          acc -= l * x[sx];
-        }
-        x[tt] = acc;
-        if (kq == 0) sM[tt * 16 + li] = acc;
-      }
-    }
+    if (!BLOCK && wave == 1) unit_inverse(Lr, sM, li, kq);
   }
-  __syncthreads();  // Lq, R and M are complete; nobody reads Q any more
+  if constexpr (BLOCK) bare_barrier();
+  else __syncthreads();
+  // Lq, R and M are complete; nobody reads Q any more
 
   // ---- Delta = R M^T: rows of this wave, accumulator (row 4kq + r, column t = li) ---------------
-  f32x4_t D[2];
+  f32x4_t D[TILES];
 #pragma unroll
-  for (int t2 = 0; t2 < 2; ++t2) {
+  for (int t2 = 0; t2 < TILES; ++t2) {
     D[t2] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      D[t2] = mfma4(sR[(32 * wave + 16 * t2 + li) * kRPad + 4 * j + kq], sM[li * 16 + 4 * j + kq], D[t2]);
+      D[t2] = mfma4(sR[(16 * (TILES * wave + t2) + li) * kRPad + 4 * j + kq], sM[li * 16 + 4 * j + kq], D[t2]);
   }
   const size_t obase = ((slotT + li) * a.Hv + hv) * 128;  // step li of this head in y and the tape
 #pragma unroll
-  for (int t2 = 0; t2 < 2; ++t2) {
-    const int row0 = 32 * wave + 16 * t2 + 4 * kq;
+  for (int t2 = 0; t2 < TILES; ++t2) {
+    const int row0 = 16 * (TILES * wave + t2) + 4 * kq;
     *reinterpret_cast<f32x4_t*>(sD + li * 128 + row0) = D[t2];
   }
-  {
+  if constexpr (BLOCK) {
+    if (li < T) *reinterpret_cast<f32x4_t*>(a.tape + obase + 16 * wave + 4 * kq) = D[0];
+  } else {
     // the tape leaves from LDS in full 128-byte lines: lane (t, q) stores this wave's rows
     // 32 wave + 8 q ..+7 of step t (the matrix-core layout would give 64-byte pieces)
     const int t = lane >> 2, dv0 = 32 * wave + 8 * (lane & 3);
@@ -909,41 +964,43 @@ void gdn_forward_chunk_128(GdnArgs a) {
       *reinterpret_cast<f32x4_t*>(dst + 4) = *reinterpret_cast<const f32x4_t*>(sD + t * 128 + dv0 + 4);
     }
   }
-  __syncthreads();
+  // (a wave reads the rows of Delta that it has written)
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 
   // ---- Y = c W + Delta Lq^T -----------------------------------------------------------------------
-  float Yn[2][4];  // fused norm: Y rounded to the array dtype, kept until every wave's sum of squares is in
-  float dA[2][4];  // Delta[row 16 t2 + li][s = 4j + kq]
+  float Yn[TILES][4];  // fused norm: Y rounded to the array dtype, kept until every wave's sum of squares is in
+  float dA[TILES][4];  // Delta[row 16 t2 + li][s = 4j + kq]
 #pragma unroll
-  for (int t2 = 0; t2 < 2; ++t2)
+  for (int t2 = 0; t2 < TILES; ++t2)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) dA[t2][j] = sD[(4 * j + kq) * 128 + 32 * wave + 16 * t2 + li];
+    for (int j = 0; j < 4; ++j) dA[t2][j] = sD[(4 * j + kq) * 128 + 16 * (TILES * wave + t2) + li];
   {
     const float ct = sC[li];
     const bool on = sOn[li] != 0.f;
 #pragma unroll
-    for (int t2 = 0; t2 < 2; ++t2) {
+    for (int t2 = 0; t2 < TILES; ++t2) {
       f32x4_t Y = W[t2] * ct;
 #pragma unroll
       for (int j = 0; j < 4; ++j) Y = mfma4(dA[t2][j], sLq[li * 16 + 4 * j + kq], Y);
       if (!on) Y = f32x4_t{0.f, 0.f, 0.f, 0.f};
       if (!NORM) {
-        if (li < T) store4_from_f32(a.y, obase + 32 * wave + 16 * t2 + 4 * kq, Y, a.in_dtype);
+        if (li < T) store4_from_f32(a.y, obase + 16 * (TILES * wave + t2) + 4 * kq, Y, a.in_dtype);
       } else {
 #pragma unroll
         for (int r = 0; r < 4; ++r) Yn[t2][r] = round_through(Y[r], a.in_dtype);  // the recurrence's output, as an array
       }
     }
     if (NORM) {
-      // this wave's 32 columns of step li: 8 per lane, the four lanes (li, kq) of a step added up
-      float ss = 0.f;
+      // a tile's 16 columns of step li: 4 per lane, the four lanes (li, kq) of a step added up
 #pragma unroll
-      for (int t2 = 0; t2 < 2; ++t2)
+      for (int t2 = 0; t2 < TILES; ++t2) {
+        float ss = 0.f;
 #pragma unroll
         for (int r = 0; r < 4; ++r) ss += Yn[t2][r] * Yn[t2][r];
-      ss += __shfl_xor(ss, 16, 64);
-      ss += __shfl_xor(ss, 32, 64);
-      if (kq == 0) sSS[16 * wave + li] = ss;  // read after the state update, behind its barrier
+        ss += __shfl_xor(ss, 16, 64);
+        ss += __shfl_xor(ss, 32, 64);
+        if (kq == 0) sSS[16 * (TILES * wave + t2) + li] = ss;  // read after the state update, behind its barrier
+      }
     }
   }
 
@@ -953,13 +1010,13 @@ void gdn_forward_chunk_128(GdnArgs a) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const float cf = sRat[(T - 1) * 16 + 4 * j + kq];  // 0 beyond step T - 1
-      dA[0][j] *= cf;
-      dA[1][j] *= cf;
+#pragma unroll
+      for (int t2 = 0; t2 < TILES; ++t2) dA[t2][j] *= cf;
     }
-    Pieces<4> dp[2];  // SPLIT: the scaled Delta in pieces; element j of a lane's operand is step 4j + kq
+    Pieces<4> dp[TILES];  // SPLIT: the scaled Delta in pieces; element j of a lane's operand is step 4j + kq
     if constexpr (SPLIT) {
 #pragma unroll
-      for (int t2 = 0; t2 < 2; ++t2) dp[t2] = split_bf16(dA[t2]);
+      for (int t2 = 0; t2 < TILES; ++t2) dp[t2] = split_bf16(dA[t2]);
     }
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
@@ -968,7 +1025,7 @@ void gdn_forward_chunk_128(GdnArgs a) {
       for (int j = 0; j < 4; ++j) kA[j] = sK[(4 * j + kq) * kKPad + 16 * c + li];
       const uint32_t ka[2] = {upper_halves(kA[0], kA[1]), upper_halves(kA[2], kA[3])};
 #pragma unroll
-      for (int t2 = 0; t2 < 2; ++t2) {
+      for (int t2 = 0; t2 < TILES; ++t2) {
         f32x4_t acc = st[t2][c] * cT;
         if constexpr (SPLIT) {
           acc = mfma16_bf16(ka, dp[t2].lo, acc);
@@ -988,11 +1045,13 @@ void gdn_forward_chunk_128(GdnArgs a) {
     // input dtype; sums and the reciprocal root are fp32.
     // a bare barrier: __syncthreads() would also wait until every store issued so far has been
     // acknowledged, and the stores of the state are about to follow
-    asm volatile("s_waitcnt lgkmcnt(0)\n s_barrier" ::: "memory");
-    const float total = sSS[li] + sSS[16 + li] + sSS[32 + li] + sSS[48 + li];
-    float zf[2][4], wf[2][4];
+    bare_barrier();
+    float total = sSS[li];
 #pragma unroll
-    for (int t2 = 0; t2 < 2; ++t2) {
+    for (int i = 1; i < 8; ++i) total += sSS[16 * i + li];
+    float zf[TILES][4], wf[TILES][4];
+#pragma unroll
+    for (int t2 = 0; t2 < TILES; ++t2) {
       if (WIDE) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) zf[t2][r] = z4[t2][r];
@@ -1016,14 +1075,14 @@ void gdn_forward_chunk_128(GdnArgs a) {
     // 16-bit array) and a rounding written out for the dtype; fp32 arrays keep the library forms.
     auto finish = [&](auto rnd, auto sigmoid, float inv_rms) __attribute__((always_inline)) {
 #pragma unroll
-      for (int t2 = 0; t2 < 2; ++t2) {
+      for (int t2 = 0; t2 < TILES; ++t2) {
         f32x4_t o;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const float normed = rnd(Yn[t2][r] * inv_rms * wf[t2][r]);
           o[r] = rnd(rnd(zf[t2][r] * rnd(sigmoid(zf[t2][r]))) * normed);
         }
-        if (li < T) store4_rounded(a.y, obase + 32 * wave + 16 * t2 + 4 * kq, o, a.in_dtype);
+        if (li < T) store4_rounded(a.y, obase + 16 * (TILES * wave + t2) + 4 * kq, o, a.in_dtype);
       }
     };
     auto fast_sigmoid = [](float x) { return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504088896341f * x)); };
@@ -1040,14 +1099,14 @@ void gdn_forward_chunk_128(GdnArgs a) {
   {
     f32x4_t* out = reinterpret_cast<f32x4_t*>((float*)a.state_out + sbase);
 #pragma unroll
-    for (int t2 = 0; t2 < 2; ++t2)
+    for (int t2 = 0; t2 < TILES; ++t2)
 #pragma unroll
       for (int m = 0; m < 4; ++m) swap_row_bit(st[t2][2 * m], st[t2][2 * m + 1]);
 #pragma unroll
-    for (int t2 = 0; t2 < 2; ++t2)
+    for (int t2 = 0; t2 < TILES; ++t2)
 #pragma unroll
       for (int c = 0; c < 8; ++c)
-        __builtin_nontemporal_store(st[t2][c], &out[memory_index(wave, li, kq, t2, c)]);
+        __builtin_nontemporal_store(st[t2][c], &out[memory_index((TILES * wave + t2) >> 1, li, kq, (TILES * wave + t2) & 1, c)]);
   }
 }
 
@@ -1268,7 +1327,7 @@ extern "C" int dflash_gdn_block(const dflash_gdn_block_args* p, void* stream) {
   void* args[] = {&a};
   if (D == 128 && p->state_dtype == DFLASH_FP32) {  // the closed form, its output norm in the same launch
     const void* fn = p->z ? (const void*)gdn_forward_chunk_128<false, true, true, true> : (const void*)gdn_forward_chunk_128<false, false, true, true>;
-    DFLASH_HIP_OK(hipLaunchKernel(fn, dim3((unsigned)(slots * Hv)), dim3(kThreads), args, kChunkLdsFloats * sizeof(float), s));
+    DFLASH_HIP_OK(hipLaunchKernel(fn, dim3((unsigned)(slots * Hv)), dim3(kBlockThreads), args, kChunkLdsFloats * sizeof(float), s));
     return DFLASH_OK;
   }
   int rows = D;
