@@ -76,21 +76,21 @@ __device__ __forceinline__ void store_exact(uint16_t* dst, const float (&v)[PER]
   store_words<PER>(dst, words);
 }
 
-// PER adjacent channels (from c on) at one step t: rows t .. t + 3 of [conv_state | qkv] and the taps, as loaded.
-template <int PER>
+// PER adjacent channels (from c on) at STEPS steps from t on: rows t .. t + STEPS + 2 of [conv_state | qkv] and the taps, as loaded.
+template <int PER, int STEPS = 1>
 struct ConvRows {
-  uint32_t x[kTaps][PER], w[PER * kTaps];
+  uint32_t x[kKeep + STEPS][PER], w[PER * kTaps];
 };
 // Every load is unconditional: a row that does not count (no conv state, steps past the block) is some readable row.
-template <int PER>
-__device__ __forceinline__ void request_rows(const BlockArgs& p, int slot, int t, int T, int C, int c, ConvRows<PER>& r) {
+template <int PER, int STEPS>
+__device__ __forceinline__ void request_rows(const BlockArgs& p, int slot, int t, int T, int C, int c, ConvRows<PER, STEPS>& r) {
   const uint16_t* const qkv = p.qkv + (size_t)slot * p.qkv_slot;
   const uint16_t* const before = p.conv_state + (size_t)slot * kKeep * C;
   const uint32_t pitch = (uint32_t)p.qkv_row;  // (16 rows of it are within 32 bits: checked where the launch is)
 #pragma unroll
-  for (int j = 0; j < kTaps; ++j) {
+  for (int j = 0; j < kKeep + STEPS; ++j) {
     const int row = t + j, s = row - kKeep < T ? row - kKeep : T - 1;
-    if (j == kKeep) {
+    if (j >= kKeep) {
       load_adjacent_raw<PER>(qkv, (uint32_t)s * pitch + (uint32_t)c, false, r.x[j]);
     } else {
       const bool stored = row < kKeep && p.conv_state != nullptr;
@@ -102,35 +102,41 @@ __device__ __forceinline__ void request_rows(const BlockArgs& p, int slot, int t
 }
 
 // silu(conv), and what the rows leave behind where `keeps`: the next conv state and qkv in one piece.
-template <int PER>
-__device__ __forceinline__ void convolve(const BlockArgs& p, int slot, int t, int T, int C, int c, bool keeps, ConvRows<PER>& r,
-                                         float (&act)[PER]) {
+template <int PER, int STEPS>
+__device__ __forceinline__ void convolve(const BlockArgs& p, int slot, int t, int T, int C, int c, bool keeps, ConvRows<PER, STEPS>& r,
+                                         float (&act)[STEPS][PER]) {
   if (p.conv_state == nullptr) {
 #pragma unroll
     for (int j = 0; j < kKeep; ++j)
 #pragma unroll
       for (int e = 0; e < PER; ++e) r.x[j][e] = t + j >= kKeep ? r.x[j][e] : 0u;
   }
-  float x[kTaps][PER], w[PER * kTaps];
+  float x[kKeep + STEPS][PER], w[PER * kTaps];
 #pragma unroll
-  for (int j = 0; j < kTaps; ++j) unpack_adjacent<PER>(r.x[j], DFLASH_BF16, x[j]);
+  for (int j = 0; j < kKeep + STEPS; ++j) unpack_adjacent<PER>(r.x[j], DFLASH_BF16, x[j]);
   unpack_adjacent<PER * kTaps>(r.w, DFLASH_BF16, w);
 #pragma unroll
-  for (int e = 0; e < PER; ++e) {
-    float acc = 0.f;
+  for (int i = 0; i < STEPS; ++i)
 #pragma unroll
-    for (int j = 0; j < kTaps; ++j) acc += x[j][e] * w[e * kTaps + j];
-    act[e] = silu_rounded(round_through(acc, DFLASH_BF16), DFLASH_BF16);
-  }
-  if (!keeps || t >= T) return;
+    for (int e = 0; e < PER; ++e) {
+      float acc = 0.f;
+#pragma unroll
+      for (int j = 0; j < kTaps; ++j) acc += x[i + j][e] * w[e * kTaps + j];
+      act[i][e] = silu_rounded(round_through(acc, DFLASH_BF16), DFLASH_BF16);
+    }
+  if (!keeps) return;
   uint16_t* const next = p.conv_next + (size_t)slot * kKeep * C + c;
   if (t == 0) {  // blocks shorter than the state: old rows move up
 #pragma unroll
     for (int row = 1; row < kKeep; ++row)
       if (row >= T) store_words<PER>(next + (size_t)(row - T) * C, r.x[row]);
   }
-  if (t + kKeep >= T) store_words<PER>(next + (size_t)(t + kKeep - T) * C, r.x[kKeep]);
-  if (p.qkv_out != nullptr) store_words<PER>(p.qkv_out + ((size_t)slot * T + t) * C + c, r.x[kKeep]);
+#pragma unroll
+  for (int i = 0; i < STEPS; ++i) {
+    if (t + i >= T) return;
+    if (t + i + kKeep >= T) store_words<PER>(next + (size_t)(t + i + kKeep - T) * C, r.x[i + kKeep]);
+    if (p.qkv_out != nullptr) store_words<PER>(p.qkv_out + ((size_t)slot * T + t + i) * C + c, r.x[i + kKeep]);
+  }
 }
 
 // q or k of the head from its activation: scale * rms_norm, rounded as the array it would be stored in.

@@ -351,15 +351,17 @@ __global__ __launch_bounds__(kThreads) void gdn_forward_rows(GdnArgs a) {
       // rows of v are one workgroup's, a key head is kept by the first of its value heads and of its first rows
       const bool keeps = row0 == 0 && hv == hk * (int)a.group.by;
       if (mine(0)) {
-        float x[kK];
-        convolve(a.block, slot, t_b, T, C, c_q, keeps, b_q, x);
+        float all[1][kK];
+        convolve(a.block, slot, t_b, T, C, c_q, keeps, b_q, all);
+        auto& x = all[0];
         normalise<kK, 16>(x, a.block.scale_q, a.block.eps);
 #pragma unroll
         for (int e = 0; e < kK; ++e) sQ[t_b * DK + plane_index<DK>(kK * seg + e)] = x[e];
       }
       if (mine(1)) {
-        float x[kK];
-        convolve(a.block, slot, t_b, T, C, c_k, keeps, b_k, x);
+        float all[1][kK];
+        convolve(a.block, slot, t_b, T, C, c_k, keeps, b_k, all);
+        auto& x = all[0];
         normalise<kK, 16>(x, a.block.scale_k, a.block.eps);
 #pragma unroll
         for (int e = 0; e < kK; ++e) sK[t_b * DK + plane_index<DK>(kK * seg + e)] = x[e];
@@ -367,8 +369,9 @@ __global__ __launch_bounds__(kThreads) void gdn_forward_rows(GdnArgs a) {
           store_exact<kK>(a.block.k_out + ((slotT + t_b) * a.Hk + hk) * DK + kK * seg, x);
       }
       if (mine(2)) {
-        float x[kD];
-        convolve(a.block, slot, t_b, T, C, c_v, true, b_v, x);
+        float all[1][kD];
+        convolve(a.block, slot, t_b, T, C, c_v, true, b_v, all);
+        auto& x = all[0];
 #pragma unroll
         for (int e = 0; e < kD; ++e) sV[t_b * kRows + kD * seg + e] = x[e];
       }
@@ -561,7 +564,10 @@ constexpr int kOffGate = kOffBeta + 16;  // 1 for masked and missing steps
 constexpr int kOffOn = kOffGate + 16;    // 1 for steps that count, 0 for masked and missing ones
 constexpr int kOffSS = kOffOn + 16;      // [tile of 16 rows][step]: its share of a step's sum of squares
 constexpr int kChunkLdsFloats = kOffSS + 128;
-constexpr int kBlockThreads = 9 * 64;  // BLOCK: eight waves with a tile of 16 rows of S each, one for what a head has once
+// BLOCK: twelve waves with four steps of q, k or v each, the first eight of them with a tile of 16 rows of S as well, and one for what a
+// head has once
+constexpr int kBlockConvWaves = 12, kBlockThreads = 64 * (kBlockConvWaves + 1), kBlockSteps = 2;
+typedef ConvRows<4, kBlockSteps> BlockIncoming;
 
 // Four consecutive elements at element i (a multiple of 4) of a 16-byte aligned array.
 __device__ __forceinline__ void store4_from_f32(void* p, size_t i, f32x4_t v, int dt) {
@@ -605,15 +611,12 @@ struct Incoming {
   f32x4_t z4[TILES], w4[TILES];  // fp32 elements
   f32x4_t st[TILES][8];
 };
-struct BlockIncoming {
-  ConvRows<4> rows[3];  // q, k, v
-};
 // Channel of lane group `seg` in q (0), k (1) or v (2).
 __device__ __forceinline__ int block_channel(const GdnArgs& a, int which, int hv, int hk, int seg) {
   return (which == 0 ? hk : which == 1 ? a.Hk + hk : 2 * a.Hk + hv) * 128 + 4 * seg;
 }
-// Step of a block's lane: two steps a wave; of up to four steps in all the first two waves have q, the next two k, the next two v.
-__device__ __forceinline__ int block_step(bool few, int wave, int lane) { return 2 * (few ? wave & 1 : wave) + (lane >> 5); }
+// First step of a block's lane
+__device__ __forceinline__ int block_step(int wave, int lane) { return 4 * (wave & 3) + kBlockSteps * (lane >> 5); }
 template <bool WIDE, bool NORM, bool BLOCK, int TILES>
 __device__ __forceinline__ void issue_item_loads(const GdnArgs& a, int item, int tid, Incoming<WIDE, TILES>& in, BlockIncoming& block) {
   const int T = a.T;
@@ -625,9 +628,8 @@ __device__ __forceinline__ void issue_item_loads(const GdnArgs& a, int item, int
   for (int j = 0; j < (WIDE ? 2 : 1); ++j) in.k.w[j] = in.q.w[j] = in.v.w[j] = uint4{0u, 0u, 0u, 0u};
   const int t = tid >> 4, seg = tid & 15;
   if constexpr (BLOCK) {
-#pragma unroll
-    for (int j = 0; j < 3; ++j)
-      request_rows(a.block, slot, block_step(T <= 4, wave, lane), T, (2 * a.Hk + a.Hv) * 128, block_channel(a, j, hv, hk, lane & 31), block.rows[j]);
+    request_rows(a.block, slot, block_step(wave, lane), T, (2 * a.Hk + a.Hv) * 128, block_channel(a, wave >> 2, hv, hk, lane & 31), block);
+    if (wave >= 8) return;  // (no rows of S)
   } else if (t < T) {
     const size_t kq_at = ((slotT + t) * a.Hk + hk) * 128 + 8 * seg;
     const size_t v_at = ((slotT + t) * a.Hv + hv) * 128 + 8 * seg;
@@ -716,15 +718,13 @@ __device__ __forceinline__ void gate_ratios(const float* sGate, float* sRat, flo
 __device__ __forceinline__ void unit_inverse(const float (&Lr)[4], float* sM, int li, int kq) {
   float x[16];
 #pragma unroll
-  for (int tt = 0; tt < 16; ++tt) {
-    float acc = tt == li ? 1.f : 0.f;
+  for (int t = 0; t < 16; ++t) x[t] = t == li ? 1.f : 0.f;
 #pragma unroll
-    for (int sx = 0; sx < tt; ++sx) {
-      const float l = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(Lr[sx & 3]), 16 * (sx >> 2) + tt));
-      acc -= l * x[sx];
-    }
-    x[tt] = acc;
-    if (kq == 0) sM[tt * 16 + li] = acc;
+  for (int sx = 0; sx < 16; ++sx) {
+    if (kq == 0) sM[sx * 16 + li] = x[sx];
+#pragma unroll
+    for (int t = sx + 1; t < 16; ++t)
+      x[t] -= __int_as_float(__builtin_amdgcn_readlane(__float_as_int(Lr[sx & 3]), 16 * (sx >> 2) + t)) * x[sx];
   }
 }
 // BLOCK: the wave without rows of S.  Gates, beta and their ratios while the others have the conv, Lq and M while they have the products
@@ -735,6 +735,7 @@ __device__ __forceinline__ void block_gates(const GdnArgs& a, int slot, int hv, 
   float* const sQ = smem + kOffQ;
   float* const sRat = smem + kOffRat;
   float* const sGate = smem + kOffGate;
+  __builtin_amdgcn_s_setprio(3);  // the longest chain of the head
   const GateBits bits = request_gates(a.block, slot, lane < T ? lane : T - 1, hv);
   if (lane < 16) {
     const float g = lane < T ? gate_of(a.block, bits) : 1.f;
@@ -776,8 +777,9 @@ __device__ __forceinline__ void block_gates(const GdnArgs& a, int slot, int hv, 
 // SIMD, fill each other's waits, and a ninth has what a head has once, gates, ratios and (I + L)^-1, beside the conv and the products with S0.
 // 16 tokens of 32 heads 16.9 -> 13.8 us (four waves of two tiles, the second of them with the inverse).
 template <bool WIDE, bool NORM, bool SPLIT, bool BLOCK>
-__global__ __launch_bounds__(BLOCK ? kBlockThreads : kThreads) __attribute__((amdgpu_waves_per_eu(3, 3)))
+__global__ __launch_bounds__(BLOCK ? kBlockThreads : kThreads) __attribute__((amdgpu_waves_per_eu(BLOCK ? 4 : 3, BLOCK ? 4 : 3)))
 void gdn_forward_chunk_128(GdnArgs a) {
+  const int in_dtype = BLOCK || SPLIT ? DFLASH_BF16 : a.in_dtype;
   constexpr int TILES = BLOCK ? 1 : 2;  // of 16 rows of S to a wave
   extern __shared__ __align__(16) float smem[];
   float* sK = smem + kOffK;
@@ -803,7 +805,7 @@ void gdn_forward_chunk_128(GdnArgs a) {
   const int slot = a.heads.quotient(item), hv = item - slot * a.Hv;
   const size_t slotT = (size_t)slot * T;
   if constexpr (BLOCK) {
-    if (wave == kBlockThreads / 64 - 1) {
+    if (wave == kBlockConvWaves) {
       block_gates(a, slot, hv, lane, smem);
       return;
     }
@@ -817,36 +819,33 @@ void gdn_forward_chunk_128(GdnArgs a) {
   f32x4_t (&z4)[TILES] = cur.z4, (&w4)[TILES] = cur.w4;
   if constexpr (BLOCK) {
     const int seg = lane & 31, hk = a.group.quotient(hv), C = (2 * a.Hk + a.Hv) * 128;
-    // every wave its two steps of q, k and v, of up to four steps in all one of the three
-    const bool few = T <= 4;
-    const int t = block_step(few, wave, lane);
+    const int which = wave >> 2, t = block_step(wave, lane);
+    float* const dst = which == 0 ? sQ : which == 1 ? sK : sV;
+    const int pitch = which == 2 ? 128 : kKPad;
+    float x[kBlockSteps][4] = {};
+    if (4 * (wave & 3) < T) {
+      const bool keeps = which == 2 || hv == hk * (int)a.group.by;  // a key head's: by the first of its value heads
+      convolve(a.block, slot, t, T, C, block_channel(a, which, hv, hk, seg), keeps, block, x);
+      if (which < 2) {
+        const float scale = which == 1 ? a.block.scale_k : a.block.scale_q;
 #pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      float* const dst = j == 0 ? sQ : j == 1 ? sK : sV;
-      const int pitch = j == 2 ? 128 : kKPad;
-      float x[4] = {};
-      if (few ? wave >> 1 == j : 2 * wave < T) {
-        const bool keeps = j == 2 || hv == hk * (int)a.group.by;  // a key head's: by the first of its value heads
-        convolve(a.block, slot, t, T, C, block_channel(a, j, hv, hk, seg), keeps, block.rows[j], x);
-        if (j < 2) normalise<4, 32>(x, j == 1 ? a.block.scale_k : a.block.scale_q, a.block.eps);
-        if (j == 1 && keeps && t < T && a.block.k_out != nullptr)
-          store_exact<4>(a.block.k_out + ((slotT + t) * a.Hk + hk) * 128 + 4 * seg, x);
+        for (int i = 0; i < kBlockSteps; ++i) normalise<4, 32>(x[i], scale, a.block.eps);
       }
-      const auto put = [&](int step, bool on) __attribute__((always_inline)) {
-        *reinterpret_cast<f32x4_t*>(dst + step * pitch + 4 * seg) = on ? f32x4_t{x[0], x[1], x[2], x[3]} : f32x4_t{0.f, 0.f, 0.f, 0.f};
-      };
-      if (!few) {
-        put(t, t < T);
-      } else if (wave >> 1 == j) {
+      if (which == 1 && keeps && a.block.k_out != nullptr) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) put(4 * i + t, i == 0 && t < T);
+        for (int i = 0; i < kBlockSteps; ++i)
+          if (t + i < T) store_exact<4>(a.block.k_out + ((slotT + t + i) * a.Hk + hk) * 128 + 4 * seg, x[i]);
       }
     }
+#pragma unroll
+    for (int i = 0; i < kBlockSteps; ++i)
+      *reinterpret_cast<f32x4_t*>(dst + (t + i) * pitch + 4 * seg) =
+          t + i < T ? f32x4_t{x[i][0], x[i][1], x[i][2], x[i][3]} : f32x4_t{0.f, 0.f, 0.f, 0.f};
   } else {
     const int t = tid >> 4, seg = tid & 15;
-    raw8_to_lds(cur.k, a.in_dtype, sK + t * kKPad + 8 * seg);
-    raw8_to_lds(cur.q, a.in_dtype, sQ + t * kKPad + 8 * seg);
-    raw8_to_lds(cur.v, a.in_dtype, sV + t * 128 + 8 * seg);
+    raw8_to_lds(cur.k, in_dtype, sK + t * kKPad + 8 * seg);
+    raw8_to_lds(cur.q, in_dtype, sQ + t * kKPad + 8 * seg);
+    raw8_to_lds(cur.v, in_dtype, sV + t * 128 + 8 * seg);
   }
   if (!BLOCK && tid < 16) {
     const bool on = tid < T && cur.mask_byte != 0;  // masked and missing steps: gate 1, beta 0
@@ -856,6 +855,7 @@ void gdn_forward_chunk_128(GdnArgs a) {
   }
   if constexpr (BLOCK) {
     bare_barrier();  // (nobody waits for the state here)
+    if (wave >= 8) return;
   } else {
     __syncthreads();
     gate_ratios(sGate, sRat, sC, tid);
@@ -984,10 +984,10 @@ void gdn_forward_chunk_128(GdnArgs a) {
       for (int j = 0; j < 4; ++j) Y = mfma4(dA[t2][j], sLq[li * 16 + 4 * j + kq], Y);
       if (!on) Y = f32x4_t{0.f, 0.f, 0.f, 0.f};
       if (!NORM) {
-        if (li < T) store4_from_f32(a.y, obase + 16 * (TILES * wave + t2) + 4 * kq, Y, a.in_dtype);
+        if (li < T) store4_from_f32(a.y, obase + 16 * (TILES * wave + t2) + 4 * kq, Y, in_dtype);
       } else {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) Yn[t2][r] = round_through(Y[r], a.in_dtype);  // the recurrence's output, as an array
+        for (int r = 0; r < 4; ++r) Yn[t2][r] = round_through(Y[r], in_dtype);  // the recurrence's output, as an array
       }
     }
     if (NORM) {
@@ -1058,7 +1058,7 @@ void gdn_forward_chunk_128(GdnArgs a) {
       } else {
         const uint32_t h[4] = {z2[t2].x & 0xFFFFu, z2[t2].x >> 16, z2[t2].y & 0xFFFFu, z2[t2].y >> 16};
 #pragma unroll
-        for (int r = 0; r < 4; ++r) zf[t2][r] = bits_as_f32(h[r], a.in_dtype);
+        for (int r = 0; r < 4; ++r) zf[t2][r] = bits_as_f32(h[r], in_dtype);
       }
       if (a.weight_dtype == DFLASH_FP32) {
 #pragma unroll
@@ -1082,14 +1082,14 @@ void gdn_forward_chunk_128(GdnArgs a) {
           const float normed = rnd(Yn[t2][r] * inv_rms * wf[t2][r]);
           o[r] = rnd(rnd(zf[t2][r] * rnd(sigmoid(zf[t2][r]))) * normed);
         }
-        if (li < T) store4_rounded(a.y, obase + 16 * (TILES * wave + t2) + 4 * kq, o, a.in_dtype);
+        if (li < T) store4_rounded(a.y, obase + 16 * (TILES * wave + t2) + 4 * kq, o, in_dtype);
       }
     };
     auto fast_sigmoid = [](float x) { return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504088896341f * x)); };
-    if (a.in_dtype == DFLASH_BF16) {
+    if (in_dtype == DFLASH_BF16) {
       finish([](float v) { uint32_t u = __float_as_uint(v); u += 0x7fffu + ((u >> 16) & 1u); return __uint_as_float(u & 0xffff0000u); },
              fast_sigmoid, __builtin_amdgcn_rsqf(total * (1.0f / 128.0f) + a.eps));
-    } else if (a.in_dtype == DFLASH_FP16) {
+    } else if (in_dtype == DFLASH_FP16) {
       finish([](float v) { return (float)(_Float16)v; }, fast_sigmoid, __builtin_amdgcn_rsqf(total * (1.0f / 128.0f) + a.eps));
     } else {
       finish([](float v) { return v; }, [](float x) { return 1.0f / (1.0f + expf(-x)); },

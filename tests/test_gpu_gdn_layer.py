@@ -337,6 +337,13 @@ def test_a_block_in_one_launch(monkeypatch, state_dtype, B, S, Hk, Hv, D, joint)
     same([False], window, shifted[1:].view(state.shape), True)
 
 
+@pytest.mark.parametrize("S", [3, 4, 6, 7, 8, 9, 13, 15])
+def test_a_block_whose_last_wave_of_steps_is_not_full(monkeypatch, S):
+    """Four steps to a wave, two to a lane: blocks that end at and within either, the kernels for both kinds of state."""
+    for state_dtype in (torch.float32, torch.bfloat16):
+        test_a_block_in_one_launch(monkeypatch, state_dtype, 1, S, 2, 4, 128, True)
+
+
 @pytest.mark.parametrize("T,D,times", [(17, 128, 1), (40, 64, 1), (33, 128, 40)])
 @pytest.mark.parametrize("normed", [True, False])
 def test_a_prompt_that_starts_from_nothing(native_lib, T, D, times, normed):
