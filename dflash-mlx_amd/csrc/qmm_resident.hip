@@ -66,6 +66,7 @@ bool qmm_resident_covers(const void* scales, const void* biases, size_t workspac
                          int sb_dtype) {
   // (mixed types: the streaming kernel's; a lane's words of scales are four bytes)
   if (act_dtype != sb_dtype || (((uintptr_t)scales | (uintptr_t)biases) % 4) != 0) return false;
+  if (K <= 1024 && N <= 4096) return false;  // as in make_plan, without looking the plan up
   const resident::Plan& plan = resident::plan_for(K, N, group_size);
   return plan.chunks != 0 && workspace_bytes >= plan.workspace;
 }

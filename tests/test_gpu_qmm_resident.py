@@ -92,7 +92,7 @@ def test_a_slice_that_gives_up_says_so_and_the_launch_ends(verify_env, native_li
 # two to five tiles of 16 rows, full and not; one slice and more, whole and uneven chunks; fewer tiles than workgroups, one more, an odd number each
 ROWS = [(17, 2048, 16, 64), (32, 4096, 4096, 64), (33, 2304, 4112, 64), (31, 5120, 12352, 64), (40, 3072, 3072, 32), (48, 4096, 6144, 64), (47, 6144, 2048, 128),
         (49, 3328, 4608, 64), (64, 4096, 6144, 32), (65, 4096, 6144, 64), (77, 8192, 5120, 64), (79, 3328, 4624, 64), (80, 12288, 4096, 64), (80, 4096, 6144, 128),
-        (17, 17408, 2064, 64), (18, 2176, 8224, 64)]
+        (17, 17408, 2064, 64), (18, 2176, 8224, 64), (32, 4096, 36880, 64), (48, 3072, 12304, 64), (63, 2048, 12304, 64), (80, 2048, 12304, 64)]
 
 
 @pytest.mark.parametrize("M,K,N,group", ROWS)
@@ -109,9 +109,11 @@ def test_gated_activation_of_short_prompts(native_lib, M, K, N, group, dtype):
     check_rows_silu(native_lib, M, K, N, group, True, dtype)
 
 
-# one, two, four and eight waves to a tile, even and uneven chunks; one tile of W, sets with one unit, with none; entries of one and of sixteen rows
+# one, two, four and eight waves to a tile, even and uneven chunks; one tile of W, sets with one unit, with none, with two meetings and more; entries of one
+# and of sixteen rows
 @pytest.mark.parametrize("K,N,E,P", [(128, 16, 3, 7), (512, 2048, 256, 128), (640, 48, 5, 90), (768, 16, 300, 200), (1152, 80, 7, 33), (1280, 4112, 2, 16),
-                                     (1408, 272, 9, 64), (2048, 1024, 64, 256), (2688, 96, 4, 40), (5120, 144, 3, 50), (1024, 16, 1, 1), (2560, 528, 600, 64)])
+                                     (1408, 272, 9, 64), (2048, 1024, 64, 256), (2688, 96, 4, 40), (5120, 144, 3, 50), (1024, 16, 1, 1), (2560, 528, 600, 64),
+                                     (640, 4112, 60, 150), (1152, 2064, 64, 200), (2304, 2064, 64, 100), (4096, 1040, 40, 70)])
 @pytest.mark.parametrize("dtype", [BF, HF])
 def test_routed_experts(native_lib, monkeypatch, K, N, E, P, dtype):
     monkeypatch.delenv("DFLASH_QMM_KERNEL", raising=False)
