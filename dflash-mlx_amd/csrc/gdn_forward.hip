@@ -774,8 +774,9 @@ __device__ __forceinline__ void block_gates(const GdnArgs& a, int slot, int hv, 
 // BLOCK: q, k, v, the gates and beta are made here, from the block's projections (gdn_block_device.h), while the state is on its
 // way.  A launch of the prepare kernel before this one took 5.4 us for what is 0.4 MB, and a microsecond to the next.  32 of 256 compute units
 // have a head to work on and nothing beside it, so what counts is the longest chain of a head: eight waves with a tile of rows each, two to a
-// SIMD, fill each other's waits, and a ninth has what a head has once, gates, ratios and (I + L)^-1, beside the conv and the products with S0.
-// 16 tokens of 32 heads 16.9 -> 13.8 us (four waves of two tiles, the second of them with the inverse).
+// SIMD, fill each other's waits, four more share the conv with them, and one has what a head has once, gates, ratios and (I + L)^-1, beside the
+// conv and the products with S0.  16 tokens of 32 heads 16.9 (four waves of two tiles, the second of them with the inverse) -> 13.8 -> 13.1 us
+// (a wave loads the rows and taps of one of q, k, v instead of all three).
 template <bool WIDE, bool NORM, bool SPLIT, bool BLOCK>
 __global__ __launch_bounds__(BLOCK ? kBlockThreads : kThreads) __attribute__((amdgpu_waves_per_eu(BLOCK ? 4 : 3, BLOCK ? 4 : 3)))
 void gdn_forward_chunk_128(GdnArgs a) {
