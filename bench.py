@@ -228,7 +228,12 @@ def bench_qmm_chain_stack(stack: str, steps: int, warmup: int, device: str, laye
     def one_pass():
         return [chain() for chain in chains]
 
+    named = os.environ.get("DFLASH_QMM_KERNEL")
+    if named is None:  # separate launches of the kernel whose sums a chain has
+        os.environ["DFLASH_QMM_KERNEL"] = "auto"
     separate = run_pass(calls[:per_chain])
+    if named is None:
+        del os.environ["DFLASH_QMM_KERNEL"]
     got = one_pass()
     torch.cuda.synchronize()
     for a, b in zip(separate, got[0]):
