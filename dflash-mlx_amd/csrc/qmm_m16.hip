@@ -763,7 +763,9 @@ extern "C" int dflash_qmm_m16_gather(const void* x, const int32_t* expert_ids, c
   const bool streams = P <= 256 || (workspace_bytes >= qmm_stream_workspace_bytes(N, qmm_stream_grid()) &&
                                       (((uintptr_t)scales | (uintptr_t)biases) % 4) == 0);
   if (workspace != nullptr && streams && qmm_stream_gather_eligible(P, K, N, E, group_size)) {
-    if (qmm_resident_gather_covers(scales, biases, P, K, N, E, group_size, act_dtype, sb_dtype))
+    // (needs no workspace; what a call has to bring does not depend on that)
+    if (workspace_bytes >= qmm_stream_workspace_bytes(N, qmm_stream_grid()) &&
+        qmm_resident_gather_covers(scales, biases, P, K, N, E, group_size, act_dtype, sb_dtype))
       return qmm_resident_gather_launch(x, expert_ids, w_q, scales, biases, y, P, K, N, E, act_dtype, s);
     return qmm_stream_gather_launch(x, expert_ids, w_q, scales, biases, y, workspace, workspace_bytes,
                                     P, K, N, E, act_dtype, sb_dtype, s);

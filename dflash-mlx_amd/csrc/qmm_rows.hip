@@ -676,11 +676,12 @@ extern "C" int dflash_qmm_rows(const void* x, const uint32_t* w_q, const void* s
                  "dflash_qmm_rows: x and w_q must be 16-byte aligned");
   const rows::Plan& p = rows::plan(M, K, N, group_size, qmm_stream_grid(), act_dtype == DFLASH_FP16, mixed, silu_mul);
   const size_t given = workspace ? workspace_bytes : 0;
+  // (what a call has to bring does not depend on which of the two kernels it is)
+  DFLASH_REQUIRE(given >= p.workspace, DFLASH_ERR_WORKSPACE,
+                 "dflash_qmm_rows: workspace of %zu bytes needed, %zu given", p.workspace, given);
   if (p.resident_chunks != 0 && given >= p.resident_workspace && (((uintptr_t)scales | (uintptr_t)biases) % 4) == 0)
     return qmm_resident_rows_launch(x, w_q, scales, biases, y, workspace, M, K, N, group_size, act_dtype, silu_mul, p.resident_chunks,
                                     p.resident_slices, (hipStream_t)stream);
-  DFLASH_REQUIRE(given >= p.workspace, DFLASH_ERR_WORKSPACE,
-                 "dflash_qmm_rows: workspace of %zu bytes needed, %zu given", p.workspace, given);
   rows::Args a;
   a.x = (const uint16_t*)x; a.w = w_q; a.scales = (const uint16_t*)scales; a.biases = (const uint16_t*)biases;
   a.y = (uint16_t*)y;

@@ -588,3 +588,15 @@ def test_members_whose_scales_are_learnt_leave_the_joint_product(monkeypatch):
         assert not group._holds(m.mlp, x)
         with torch.no_grad():
             assert group._holds(m.mlp, x)
+
+
+@pytest.mark.parametrize("given", [0, 64 * 1024])
+def test_products_refuse_a_small_workspace_whichever_kernel_they_take(native_lib, given):
+    """What a call has to bring is what the kernel with partial sums asks for, also where the call goes to one that has none.
+    (Refused before anything is launched: the operands are numbers.)"""
+    p = 1 << 20
+    assert native_lib.dflash_qmm_rows_workspace_bytes(32, 4096, 4096, 64, 0, 0, 0) > 64 * 1024
+    assert native_lib.dflash_qmm_rows(p, p, p, p, p, p if given else None, given, 32, 4096, 4096, 64, 0, 0, 0, None) == -3
+    assert native_lib.dflash_qmm_m16_gather_workspace_bytes(128, 2048, 1024, 256, 64) > 64 * 1024
+    assert native_lib.dflash_qmm_m16_gather(p, p, p, p, p, p, p, given, 128, 2048, 1024, 256, 64, 0, 0, None) == -3
+    assert native_lib.dflash_qmm_few(p, p, p, p, p, p, given, 16, 4096, 4096, 64, 0, 0, 3, None) == -3
