@@ -9,8 +9,8 @@
 //  * loads follow the rows: a load instruction covers runs of NCH * 64 bytes, whole 128-byte lines.  In matrix-instruction order (16 rows, 64
 //    bytes each) the same loads with nothing else took 24.6 us for 5120 x 34816, in this order 19.6; for x (256-byte runs, turned through
 //    LDS) 2.2 us of a launch.  LDS takes the pieces in an order without bank conflicts; a row's scales are fetched four bytes a lane;
-//  * scales and biases enter in fp32 as before: s * sum x (offset + q) per group on the vector pipe, the sums of x times (bias - offset *
-//    scale) of four groups in one 16 x 16 x 4 fp32 matrix instruction;
+//  * scales and biases enter in fp32 as before: s * sum x q per group on the vector pipe, the sums of x times the biases of four groups in one
+//    16 x 16 x 4 fp32 matrix instruction;
 //  * the eight waves' sums meet in LDS, in their order.  Where a wave's chunks would be more than NCH, the K range is cut into slices of
 //    whole workgroups: all but the last store their tiles (their own arrival flags, see nonzero_words()), the last adds them in order.
 //    It has the highest index of those it waits for, so they are running or done before it starts, and they wait for nobody.
@@ -102,22 +102,67 @@ __device__ __forceinline__ void wait_loads() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// 8 codes of a word as numbers offset + q, in the slot order of stream::unpack_codes.  fp16 has the mantissa for codes four bits further up, where
-// the offset is 64 and not 1024: what the biases take off again is that much smaller than the sums it comes off.
-template <bool H16>
+// 8 codes of a word as numbers offset + q, in the slot order of stream::unpack_codes.  What the offset adds to a sum is taken off again, and the rounding
+// error of a sum is that of the numbers it is made of, so the offset has to be small or gone before the groups are added up:
+//  * it is taken off inside the matrix instructions, which start from -offset * (sum of x over the group) and not from zero (kStart; four registers per
+//    group, a launch takes as long as without, 4 chunks and one tile 0.1 us longer);
+//  * groups of 32 have registers for that up to three chunks (four: spilled, 4096 x 24576 with the activation 16.5 -> 23.1 us).  Beyond that bf16 codes go to
+//    the top of the mantissa, offset 16, for one more shift per word (1 % of a launch);
+//  * fp16: the mantissa has room for codes four bits further up, where the offset is 64 and not 1024.
+// Share of results that are not those of fp64 rounded, streaming kernel and here: bf16 5120 x 7168 0.12 and 0.06 %, 5120 x 4096 in groups of 32 0.09 and
+// 0.07 %; fp16 6.2 and 0.33 %, in groups of 32 5.2 and 1.1 %.  (Offset 128 and those of all groups in one sum in front of the others: bf16 0.25 and 0.32 %.)
+template <bool H16, int GS, int NCH>
 struct Codes {
-  static constexpr uint32_t kMask = H16 ? 0x00F000F0u : 0x000F000Fu, kMagic = H16 ? 0x54005400u : Act<false>::kMagic;
-  static constexpr float kOffset = H16 ? 64.0f : Act<false>::kOffset;
+  static constexpr bool kStart = GS != 32 || NCH <= 3;
+  static constexpr int kUp = H16 ? 4 : kStart ? 0 : 3;  // bits that the codes move up
+  static constexpr uint32_t kMask = 0x000F000Fu << kUp, kMagic = H16 ? 0x54005400u : kStart ? Act<false>::kMagic : 0x41804180u;
+  static constexpr float kOffset = H16 ? 64.0f : kStart ? Act<false>::kOffset : 16.0f;
+  static constexpr uint32_t kMinusOffset = H16 ? 0xD400D400u : 0xC300C300u;  // twice, in the activation type (kStart)
   static __device__ __forceinline__ uint4 unpack(uint32_t w, uint32_t mask, uint32_t magic) {
-    if (!H16) return stream::unpack_codes(w, mask, magic);
-    uint4 r;
-    r.x = ((w << 4) & mask) | magic;
-    r.y = (w & mask) | magic;
-    r.z = ((w >> 4) & mask) | magic;
-    r.w = ((w >> 8) & mask) | magic;
-    return r;
+    auto at = [&](int bit) { return ((bit > kUp ? w >> (bit - kUp) : w << (kUp - bit)) & mask) | magic; };
+    return make_uint4(at(0), at(4), at(8), at(12));
   }
 };
+
+// Sums of x over groups: xs[i] for the biases, lane (li, q) group 4 i + q of row li; from[c][g], the products' accumulators of that group: -offset times
+// those of rows 4 q + r.  One set of matrix instructions for both: its sums are the same in all sixteen lanes of a q, so each picks the group and row of a lane
+// that fetches it from there.
+template <bool H16, int GS, int NCH>
+__device__ __forceinline__ void sums_of_groups(const uint4 (&x)[NCH][4], int li, int q, float (&xs)[Geometry<GS, NCH, 1>::NB],
+                                               f32x4_t (&from)[NCH][Geometry<GS, NCH, 1>::G]) {
+  using A = Act<H16>;
+  using C4 = Codes<H16, GS, NCH>;
+  using L = Geometry<GS, NCH, 1>;
+  constexpr uint32_t kBy = C4::kStart ? C4::kMinusOffset : A::kOnes;
+  const uint4 by = make_uint4(kBy, kBy, kBy, kBy);
+#pragma unroll
+  for (int c = 0; c < NCH; ++c)
+#pragma unroll
+    for (int g = 0; g < L::G; ++g) {
+      f32x4_t d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < L::WPG; ++i) d = C4::kStart ? A::mfma(x[c][g * L::WPG + i], by, d) : A::mfma(by, x[c][g * L::WPG + i], d);
+      const int gi = c * L::G + g;
+      if constexpr (C4::kStart) {
+        from[c][g] = d;
+        const float sum = li & 2 ? (li & 1 ? d[3] : d[2]) : (li & 1 ? d[1] : d[0]);
+        xs[gi >> 2] = (li >> 2) == (gi & 3) ? sum : (gi & 3) == 0 ? 0.f : xs[gi >> 2];
+      } else {
+        from[c][g] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        xs[gi >> 2] = q == (gi & 3) ? d[0] : (gi & 3) == 0 ? 0.f : xs[gi >> 2];
+      }
+    }
+  if constexpr (C4::kStart) {
+    const int lane = 16 * (li >> 2) + 4 * q + (li & 3);
+#pragma unroll
+    for (int i = 0; i < L::NB; ++i) xs[i] = __int_as_float(__builtin_amdgcn_ds_bpermute(4 * lane, __float_as_int(xs[i]))) * (-1.0f / C4::kOffset);
+  }
+}
+// What a row's scale s and bias b multiply its sums of x with
+template <class C4>
+__device__ __forceinline__ float bias_of(float s, float b) {
+  return C4::kStart ? b : __builtin_fmaf(-C4::kOffset, s, b);
+}
 
 // Weights of 17 rows and more are rounded to the activation type, as in the any-rows product (qmm_rows.hip says how the codes become numbers)
 template <bool H16>
@@ -166,7 +211,7 @@ __device__ __forceinline__ void load_partials3(const float* const (&p)[3], f32x4
 template <bool H16, int GS, int NCH, int MT, bool SILU, bool PACKED>
 __device__ __forceinline__ void product(const Args& p) {
   using A = Act<H16>;
-  using C4 = Codes<H16>;
+  using C4 = Codes<H16, GS, NCH>;
   using L = Geometry<GS, NCH, MT>;
   constexpr int kSlots = L::kSlots;
   constexpr int G = L::G, WPG = L::WPG, NS = L::NS, NB = L::NB;
@@ -277,20 +322,10 @@ __device__ __forceinline__ void product(const Args& p) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) x[m][c][i] = stream::as_uint4(MT == 1 ? stream::permute_x(t[i]) : t[i]);
     }
-  // xs[i]: sum of x over group 4 i + q of row li, in fp32
   const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
-  const uint4 ones = make_uint4(A::kOnes, A::kOnes, A::kOnes, A::kOnes);
   float xs[NB];
-#pragma unroll
-  for (int c = 0; c < (MT == 1 ? NCH : 0); ++c)
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      f32x4_t d = zero;
-#pragma unroll
-      for (int i = 0; i < WPG; ++i) d = A::mfma(ones, x[0][c][g * WPG + i], d);
-      const int gi = c * G + g;
-      xs[gi >> 2] = q == (gi & 3) ? d[0] : (gi & 3) == 0 ? 0.f : xs[gi >> 2];
-    }
+  f32x4_t from[NCH][G];
+  if constexpr (MT == 1) sums_of_groups<H16, GS, NCH>(x[0], li, q, xs, from);
 
   // in registers the compiler cannot see through: one v_and_or_b32 per pair of codes, selections without branches
   uint32_t mask = MT == 1 ? C4::kMask : 0x000F000Fu, mask4 = 0x00F000F0u, magic = C4::kMagic, upper = q & 2 ? ~0u : 0u;
@@ -345,13 +380,13 @@ __device__ __forceinline__ void product(const Args& p) {
       for (int i = 0; i < NB; ++i) {
         const float sv = of_q(s[i >> 1][2 * (i & 1)], s[i >> 1][2 * (i & 1) + 1]);
         const float bv = of_q(b[i >> 1][2 * (i & 1)], b[i >> 1][2 * (i & 1) + 1]);
-        acc = mfma4(xs[i], __builtin_fmaf(-C4::kOffset, sv, bv), acc);
+        acc = mfma4(xs[i], bias_of<C4>(sv, bv), acc);
       }
 #pragma unroll
       for (int c = 0; c < NCH; ++c)
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-          f32x4_t d = zero;
+          f32x4_t d = from[c][g];
 #pragma unroll
           for (int i = 0; i < WPG; ++i) d = A::mfma(x[0][c][g * WPG + i], C4::unpack(Words<WPG>::get(w[c][g], i), mask, magic), d);
           const int gi = c * G + g, word = gi >> 1;

@@ -37,7 +37,7 @@ struct GatherGeometry : Geometry<64, NCH, 1> {
 template <bool H16, int NCH>
 __device__ __forceinline__ void gathered_product(const GatherArgs& p) {
   using A = Act<H16>;
-  using C4 = Codes<H16>;
+  using C4 = Codes<H16, 64, NCH>;
   using L = GatherGeometry<NCH>;
   constexpr int G = 2, NS = L::NS, NB = L::NB, kSlots = L::kSlots;
   extern __shared__ __align__(16) char lds[];  // every wave's ring; the waves' sums; the tables
@@ -103,9 +103,9 @@ __device__ __forceinline__ void gathered_product(const GatherArgs& p) {
   };
 
   const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
-  const uint4 ones = make_uint4(A::kOnes, A::kOnes, A::kOnes, A::kOnes);
   uint4 x[NCH][4];
   float xs[NB];
+  f32x4_t from[NCH][G];
   // x of an entry, in the order of the products (rows past the entry's and chunks past `mine` are zeros), and its sums: asked for, and taken
   u32x4_t t[NCH][4];
   auto ask = [&](int entry) __attribute__((always_inline)) {
@@ -123,15 +123,7 @@ __device__ __forceinline__ void gathered_product(const GatherArgs& p) {
     for (int c = 0; c < NCH; ++c)
 #pragma unroll
       for (int i = 0; i < 4; ++i) x[c][i] = stream::as_uint4(stream::permute_x(t[c][i]));
-#pragma unroll
-    for (int c = 0; c < NCH; ++c)
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        f32x4_t d = A::mfma(ones, x[c][2 * g], zero);
-        d = A::mfma(ones, x[c][2 * g + 1], d);
-        const int gi = c * G + g;
-        xs[gi >> 2] = q == (gi & 3) ? d[0] : (gi & 3) == 0 ? 0.f : xs[gi >> 2];
-      }
+    sums_of_groups<H16, 64, NCH>(x, li, q, xs, from);
   };
 
   uint32_t mask = C4::kMask, magic = C4::kMagic, upper = q & 2 ? ~0u : 0u;
@@ -203,13 +195,13 @@ __device__ __forceinline__ void gathered_product(const GatherArgs& p) {
     for (int n = 0; n < NB; ++n) {
       const float sv = of_q(s[n >> 1][2 * (n & 1)], s[n >> 1][2 * (n & 1) + 1]);
       const float bv = of_q(b[n >> 1][2 * (n & 1)], b[n >> 1][2 * (n & 1) + 1]);
-      acc = mfma4(xs[n], __builtin_fmaf(-C4::kOffset, sv, bv), acc);
+      acc = mfma4(xs[n], bias_of<C4>(sv, bv), acc);
     }
 #pragma unroll
     for (int c = 0; c < NCH; ++c)
 #pragma unroll
       for (int g = 0; g < G; ++g) {
-        f32x4_t d = A::mfma(x[c][2 * g], C4::unpack(w[c][g][0], mask, magic), zero);
+        f32x4_t d = A::mfma(x[c][2 * g], C4::unpack(w[c][g][0], mask, magic), from[c][g]);
         d = A::mfma(x[c][2 * g + 1], C4::unpack(w[c][g][1], mask, magic), d);
         const float sv = g ? high(s[c >> 2][c & 3]) : low(s[c >> 2][c & 3]);
 #pragma unroll

@@ -53,6 +53,28 @@ def test_gated_activation(native_lib, K, N, group, dtype):
     assert _clean(native_lib)
 
 
+@pytest.mark.parametrize("K,N,group", [(1024, 8192, 64), (4096, 4096, 64), (5120, 7168, 64), (4096, 6144, 32), (5120, 4096, 32), (3072, 8192, 32),
+                                       (12288, 4096, 64), (17408, 4096, 64), (5120, 5120, 128)])
+@pytest.mark.parametrize("dtype", [BF, HF])
+def test_no_further_from_64_bits_than_the_streaming_kernel(verify_env, native_lib, K, N, group, dtype):
+    """Results that are not the rounded ones of fp64: what fp32 sums leave in the last place.  A thousandth to a twentieth of all there; fewer here."""
+    c = make_qmm_case(K, N, K + N, group_size=group, dtype=dtype).to(DEV)
+    w = dequantize(c.w, c.scales, c.biases, group, 4, torch.float64)
+    exact = (c.x.double() @ w.T).to(torch.float32).to(dtype)
+    y = {}
+    for kernel in (nat.QMM_KERNEL_AUTO, nat.QMM_KERNEL_FASTEST):
+        y[kernel] = torch.empty((16, N), dtype=dtype, device=DEV)
+        ws = VQ._workspace(torch.device(DEV), nat.raw_stream(torch.device(DEV)), 1)
+        code = VQ._DTYPE_CODE[dtype]
+        nat.check(native_lib.dflash_qmm_few(c.x.data_ptr(), c.w.data_ptr(), c.scales.data_ptr(), c.biases.data_ptr(), y[kernel].data_ptr(), ws.data_ptr(),
+                                            ws.numel(), 16, K, N, group, code, code, kernel, nat.raw_stream(torch.device(DEV))), "dflash_qmm_few")
+    off = {k: int((v != exact).sum()) for k, v in y.items()}
+    assert off[nat.QMM_KERNEL_FASTEST] <= off[nat.QMM_KERNEL_AUTO], off
+    if group == 64 and K <= 5120:  # the gathered form
+        routed = VQ.gather_qmm(c.x, c.w[None], c.scales[None], c.biases[None], torch.zeros(16, dtype=torch.int32, device=DEV))
+        assert int((routed != exact).sum()) <= off[nat.QMM_KERNEL_AUTO], off
+
+
 @pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
 def test_what_is_not_a_number_stays_in_its_row(verify_env, native_lib, value):
     """Rows are loaded together and padded chunks are multiplied with zeros: neither lets one row's values into another."""
