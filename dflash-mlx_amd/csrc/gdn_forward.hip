@@ -34,6 +34,7 @@
 #include <cstdlib>
 
 namespace dflash {
+int qmm_stream_grid();  // compute units
 namespace {
 
 constexpr int kThreads = 256;
@@ -564,10 +565,17 @@ constexpr int kOffGate = kOffBeta + 16;  // 1 for masked and missing steps
 constexpr int kOffOn = kOffGate + 16;    // 1 for steps that count, 0 for masked and missing ones
 constexpr int kOffSS = kOffOn + 16;      // [tile of 16 rows][step]: its share of a step's sum of squares
 constexpr int kChunkLdsFloats = kOffSS + 128;
-// BLOCK: twelve waves with four steps of q, k or v each, the first eight of them with a tile of 16 rows of S as well, and one for what a
-// head has once
+// Where q, k and v come from: arrays, or the block's projections (gdn_block_device.h).  kThirteenWaves: twelve waves with four steps of q, k or v each, the
+// first eight of them with a tile of 16 rows of S as well, and one for what a head has once.  kFourWaves: the four waves of the array form.
+enum Source { kFromArrays = 0, kFourWaves, kThirteenWaves };
 constexpr int kBlockConvWaves = 12, kBlockThreads = 64 * (kBlockConvWaves + 1), kBlockSteps = 2;
-typedef ConvRows<4, kBlockSteps> BlockIncoming;
+template <Source FROM>
+struct BlockIncoming : ConvRows<4, kBlockSteps> {};
+template <>
+struct BlockIncoming<kFourWaves> {
+  ConvRows<8> rows[3];  // q, k, v
+  GateBits gates;
+};
 
 // Four consecutive elements at element i (a multiple of 4) of a 16-byte aligned array.
 __device__ __forceinline__ void store4_from_f32(void* p, size_t i, f32x4_t v, int dt) {
@@ -611,25 +619,30 @@ struct Incoming {
   f32x4_t z4[TILES], w4[TILES];  // fp32 elements
   f32x4_t st[TILES][8];
 };
-// Channel of lane group `seg` in q (0), k (1) or v (2).
-__device__ __forceinline__ int block_channel(const GdnArgs& a, int which, int hv, int hk, int seg) {
-  return (which == 0 ? hk : which == 1 ? a.Hk + hk : 2 * a.Hk + hv) * 128 + 4 * seg;
+// Channel `at` of the head in q (0), k (1) or v (2).
+__device__ __forceinline__ int block_channel(const GdnArgs& a, int which, int hv, int hk, int at) {
+  return (which == 0 ? hk : which == 1 ? a.Hk + hk : 2 * a.Hk + hv) * 128 + at;
 }
-// First step of a block's lane
+// First step of a lane of the wide form
 __device__ __forceinline__ int block_step(int wave, int lane) { return 4 * (wave & 3) + kBlockSteps * (lane >> 5); }
-template <bool WIDE, bool NORM, bool BLOCK, int TILES>
-__device__ __forceinline__ void issue_item_loads(const GdnArgs& a, int item, int tid, Incoming<WIDE, TILES>& in, BlockIncoming& block) {
+template <bool WIDE, bool NORM, Source FROM, int TILES>
+__device__ __forceinline__ void issue_item_loads(const GdnArgs& a, int item, int tid, Incoming<WIDE, TILES>& in, BlockIncoming<FROM>& block) {
   const int T = a.T;
   const int slot = a.heads.quotient(item), hv = item - slot * a.Hv, hk = a.group.quotient(hv);
   const size_t slotT = (size_t)slot * T;
-  const int lane = tid & 63, wave = BLOCK ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6, li = lane & 15, kq = lane >> 4;
+  const int lane = tid & 63, wave = FROM != kFromArrays ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6, li = lane & 15, kq = lane >> 4;
   // the block's operands first, the state behind them: loads complete in order
 #pragma unroll
   for (int j = 0; j < (WIDE ? 2 : 1); ++j) in.k.w[j] = in.q.w[j] = in.v.w[j] = uint4{0u, 0u, 0u, 0u};
   const int t = tid >> 4, seg = tid & 15;
-  if constexpr (BLOCK) {
-    request_rows(a.block, slot, block_step(wave, lane), T, (2 * a.Hk + a.Hv) * 128, block_channel(a, wave >> 2, hv, hk, lane & 31), block);
+  if constexpr (FROM == kThirteenWaves) {
+    request_rows(a.block, slot, block_step(wave, lane), T, (2 * a.Hk + a.Hv) * 128, block_channel(a, wave >> 2, hv, hk, 4 * (lane & 31)), block);
     if (wave >= 8) return;  // (no rows of S)
+  } else if constexpr (FROM == kFourWaves) {
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+      request_rows(a.block, slot, T <= 4 ? lane >> 4 : t, T, (2 * a.Hk + a.Hv) * 128, block_channel(a, j, hv, hk, 8 * seg), block.rows[j]);
+    block.gates = request_gates(a.block, slot, lane < T ? lane : T - 1, hv);
   } else if (t < T) {
     const size_t kq_at = ((slotT + t) * a.Hk + hk) * 128 + 8 * seg;
     const size_t v_at = ((slotT + t) * a.Hv + hv) * 128 + 8 * seg;
@@ -641,7 +654,7 @@ __device__ __forceinline__ void issue_item_loads(const GdnArgs& a, int item, int
   // state has been asked for, so that no request waits for another one's answer
   in.gate_bits = in.beta_bits = 0u;
   in.mask_byte = 1u;
-  if (!BLOCK && tid < T && tid < 16) {
+  if (FROM == kFromArrays && tid < T && tid < 16) {
     const size_t at = (slotT + tid) * a.Hv + hv;
     if (a.g_dtype == DFLASH_FP32) {
       in.gate_bits = ((const uint32_t*)a.g)[at];
@@ -727,7 +740,7 @@ __device__ __forceinline__ void unit_inverse(const float (&Lr)[4], float* sM, in
       x[t] -= __int_as_float(__builtin_amdgcn_readlane(__float_as_int(Lr[sx & 3]), 16 * (sx >> 2) + t)) * x[sx];
   }
 }
-// BLOCK: the wave without rows of S.  Gates, beta and their ratios while the others have the conv, Lq and M while they have the products
+// kThirteenWaves: the wave without rows of S.  Gates, beta and their ratios while the others have the conv, Lq and M while they have the products
 // with S0; two barriers, which the others meet it at.
 __device__ __forceinline__ void block_gates(const GdnArgs& a, int slot, int hv, int lane, float* smem) {
   const int T = a.T, li = lane & 15, kq = lane >> 4;
@@ -768,20 +781,22 @@ __device__ __forceinline__ void block_gates(const GdnArgs& a, int slot, int hv, 
   unit_inverse(Lr, smem + kOffM, li, kq);
   bare_barrier();
 }
-// One workgroup per (slot, head); the register cap keeps at least three on a compute unit.
+// One workgroup per (slot, head); the register cap keeps at least three on a compute unit, two (kFourWaves) or one (kThirteenWaves).
 // SPLIT: q and k are bf16 arrays; the products with S0 and the state update run on the bf16
 // matrix cores with the fp32 factor in three exact pieces (see split_bf16).
-// BLOCK: q, k, v, the gates and beta are made here, from the block's projections (gdn_block_device.h), while the state is on its
-// way.  A launch of the prepare kernel before this one took 5.4 us for what is 0.4 MB, and a microsecond to the next.  32 of 256 compute units
-// have a head to work on and nothing beside it, so what counts is the longest chain of a head: eight waves with a tile of rows each, two to a
+// kFourWaves, kThirteenWaves: q, k, v, the gates and beta are made here, from the block's projections (gdn_block_device.h), while the state is on its
+// way.  A launch of the prepare kernel before this one took 5.4 us for what is 0.4 MB, and a microsecond to the next.  In an ordinary block 32 of
+// 256 compute units have a head to work on and nothing beside it, so what counts is the longest chain of a head: eight waves with a tile of rows each, two to a
 // SIMD, fill each other's waits, four more share the conv with them, and one has what a head has once, gates, ratios and (I + L)^-1, beside the
 // conv and the products with S0.  16 tokens of 32 heads 16.9 (four waves of two tiles, the second of them with the inverse) -> 13.8 -> 13.1 us
-// (a wave loads the rows and taps of one of q, k, v instead of all three).
-template <bool WIDE, bool NORM, bool SPLIT, bool BLOCK>
-__global__ __launch_bounds__(BLOCK ? kBlockThreads : kThreads) __attribute__((amdgpu_waves_per_eu(BLOCK ? 4 : 3, BLOCK ? 4 : 3)))
+// (a wave loads the rows and taps of one of q, k, v instead of all three).  Thirteen waves leave no room for a second head on the compute unit;
+// where there are more heads than compute units the four waves of kFourWaves, two heads at a time, are faster (dflash_gdn_block says from where on).
+template <bool WIDE, bool NORM, bool SPLIT, Source FROM>
+__global__ __launch_bounds__(FROM == kThirteenWaves ? kBlockThreads : kThreads)
+__attribute__((amdgpu_waves_per_eu(FROM == kThirteenWaves ? 4 : FROM == kFourWaves ? 2 : 3, FROM == kThirteenWaves ? 4 : FROM == kFourWaves ? 2 : 3)))
 void gdn_forward_chunk_128(GdnArgs a) {
-  const int in_dtype = BLOCK || SPLIT ? DFLASH_BF16 : a.in_dtype;
-  constexpr int TILES = BLOCK ? 1 : 2;  // of 16 rows of S to a wave
+  const int in_dtype = FROM != kFromArrays || SPLIT ? DFLASH_BF16 : a.in_dtype;
+  constexpr int TILES = FROM == kThirteenWaves ? 1 : 2;  // of 16 rows of S to a wave
   extern __shared__ __align__(16) float smem[];
   float* sK = smem + kOffK;
   float* sQ = smem + kOffQ;
@@ -805,20 +820,20 @@ void gdn_forward_chunk_128(GdnArgs a) {
   const int item = blockIdx.x;
   const int slot = a.heads.quotient(item), hv = item - slot * a.Hv;
   const size_t slotT = (size_t)slot * T;
-  if constexpr (BLOCK) {
+  if constexpr (FROM == kThirteenWaves) {
     if (wave == kBlockConvWaves) {
       block_gates(a, slot, hv, lane, smem);
       return;
     }
   }
   Incoming<WIDE, TILES> cur;
-  BlockIncoming block;
-  issue_item_loads<WIDE, NORM, BLOCK, TILES>(a, item, tid, cur, block);
+  BlockIncoming<FROM> block;
+  issue_item_loads<WIDE, NORM, FROM, TILES>(a, item, tid, cur, block);
   const size_t sbase = (size_t)item * 128 * 128;
   f32x4_t (&st)[TILES][8] = cur.st;
   uint2 (&z2)[TILES] = cur.z2, (&w2)[TILES] = cur.w2;
   f32x4_t (&z4)[TILES] = cur.z4, (&w4)[TILES] = cur.w4;
-  if constexpr (BLOCK) {
+  if constexpr (FROM == kThirteenWaves) {
     const int seg = lane & 31, hk = a.group.quotient(hv), C = (2 * a.Hk + a.Hv) * 128;
     const int which = wave >> 2, t = block_step(wave, lane);
     float* const dst = which == 0 ? sQ : which == 1 ? sK : sV;
@@ -826,7 +841,7 @@ void gdn_forward_chunk_128(GdnArgs a) {
     float x[kBlockSteps][4] = {};
     if (4 * (wave & 3) < T) {
       const bool keeps = which == 2 || hv == hk * (int)a.group.by;  // a key head's: by the first of its value heads
-      convolve(a.block, slot, t, T, C, block_channel(a, which, hv, hk, seg), keeps, block, x);
+      convolve(a.block, slot, t, T, C, block_channel(a, which, hv, hk, 4 * seg), keeps, block, x);
       if (which < 2) {
         const float scale = which == 1 ? a.block.scale_k : a.block.scale_q;
 #pragma unroll
@@ -842,19 +857,57 @@ void gdn_forward_chunk_128(GdnArgs a) {
     for (int i = 0; i < kBlockSteps; ++i)
       *reinterpret_cast<f32x4_t*>(dst + (t + i) * pitch + 4 * seg) =
           t + i < T ? f32x4_t{x[i][0], x[i][1], x[i][2], x[i][3]} : f32x4_t{0.f, 0.f, 0.f, 0.f};
+  } else if constexpr (FROM == kFourWaves) {
+    const int seg = tid & 15, hk = a.group.quotient(hv), C = (2 * a.Hk + a.Hv) * 128;
+    // every wave its four steps of q, k and v, of up to four steps in all one of the three
+    const bool few = T <= 4;
+    const int t = few ? lane >> 4 : tid >> 4;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      float* const dst = j == 0 ? sQ : j == 1 ? sK : sV;
+      const int pitch = j == 2 ? 128 : kKPad;
+      float all[1][8] = {};
+      auto& x = all[0];
+      if (few ? wave == j : 4 * wave < T) {
+        const bool keeps = j == 2 || hv == hk * (int)a.group.by;  // a key head's: by the first of its value heads
+        convolve(a.block, slot, t, T, C, block_channel(a, j, hv, hk, 8 * seg), keeps, block.rows[j], all);
+        if (j < 2) normalise<8, 16>(x, j == 1 ? a.block.scale_k : a.block.scale_q, a.block.eps);
+        if (j == 1 && keeps && t < T && a.block.k_out != nullptr)
+          store_exact<8>(a.block.k_out + ((slotT + t) * a.Hk + hk) * 128 + 8 * seg, x);
+      }
+      const auto put = [&](int step, bool on) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 8; e += 4)
+          *reinterpret_cast<f32x4_t*>(dst + step * pitch + 8 * seg + e) =
+              on ? f32x4_t{x[e], x[e + 1], x[e + 2], x[e + 3]} : f32x4_t{0.f, 0.f, 0.f, 0.f};
+      };
+      if (!few) {
+        put(t, t < T);
+      } else if (wave == j) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) put(4 * i + t, i == 0 && t < T);
+      }
+    }
+    if (wave == 3 && lane < 16) {
+      const float g = lane < T ? gate_of(a.block, block.gates) : 1.f;
+      if (lane < T && a.block.g_out != nullptr) a.block.g_out[(slotT + lane) * a.Hv + hv] = g;
+      sGate[lane] = g;
+      sBeta[lane] = lane < T ? beta_of(block.gates) : 0.f;
+      sOn[lane] = lane < T ? 1.f : 0.f;
+    }
   } else {
     const int t = tid >> 4, seg = tid & 15;
     raw8_to_lds(cur.k, in_dtype, sK + t * kKPad + 8 * seg);
     raw8_to_lds(cur.q, in_dtype, sQ + t * kKPad + 8 * seg);
     raw8_to_lds(cur.v, in_dtype, sV + t * 128 + 8 * seg);
   }
-  if (!BLOCK && tid < 16) {
+  if (FROM == kFromArrays && tid < 16) {
     const bool on = tid < T && cur.mask_byte != 0;  // masked and missing steps: gate 1, beta 0
     sGate[tid] = on ? bits_as_f32(cur.gate_bits, a.g_dtype) : 1.f;
     sBeta[tid] = on ? bits_as_f32(cur.beta_bits, a.beta_dtype) : 0.f;
     sOn[tid] = on ? 1.f : 0.f;
   }
-  if constexpr (BLOCK) {
+  if constexpr (FROM == kThirteenWaves) {
     bare_barrier();  // (nobody waits for the state here)
     if (wave >= 8) return;
   } else {
@@ -888,8 +941,8 @@ void gdn_forward_chunk_128(GdnArgs a) {
         U[t2] = mfma32_bf16(sp.hi, kb, U[t2]);
         W[t2] = mfma32_bf16(sp.hi, qb, W[t2]);
       }
-      if (!BLOCK && wave == 1) X = mfma32_bf16(kb, kb, X);  // [s][t] = k_s . k_t
-      if (!BLOCK && wave == 2) X = mfma32_bf16(kb, qb, X);  // [s][t] = k_s . q_t
+      if (FROM != kThirteenWaves && wave == 1) X = mfma32_bf16(kb, kb, X);  // [s][t] = k_s . k_t
+      if (FROM != kThirteenWaves && wave == 2) X = mfma32_bf16(kb, qb, X);  // [s][t] = k_s . q_t
     }
   } else {
 #pragma unroll
@@ -914,7 +967,7 @@ void gdn_forward_chunk_128(GdnArgs a) {
     const int t = li;
     const float ct = sC[t], bt = sBeta[t];
     float Lr[4];  // wave 1: L[t][4kq + r], wave 2: Lq[t][4kq + r]
-    if constexpr (!BLOCK) {
+    if constexpr (FROM != kThirteenWaves) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int sx = 4 * kq + r;
@@ -932,9 +985,9 @@ void gdn_forward_chunk_128(GdnArgs a) {
       sR[(row0 + 2) * kRPad + t] = bt * (v4.z - ct * U[t2][2]);
       sR[(row0 + 3) * kRPad + t] = bt * (v4.w - ct * U[t2][3]);
     }
-    if (!BLOCK && wave == 1) unit_inverse(Lr, sM, li, kq);
+    if (FROM != kThirteenWaves && wave == 1) unit_inverse(Lr, sM, li, kq);
   }
-  if constexpr (BLOCK) bare_barrier();
+  if constexpr (FROM == kThirteenWaves) bare_barrier();
   else __syncthreads();
   // Lq, R and M are complete; nobody reads Q any more
 
@@ -953,7 +1006,7 @@ void gdn_forward_chunk_128(GdnArgs a) {
     const int row0 = 16 * (TILES * wave + t2) + 4 * kq;
     *reinterpret_cast<f32x4_t*>(sD + li * 128 + row0) = D[t2];
   }
-  if constexpr (BLOCK) {
+  if constexpr (FROM == kThirteenWaves) {
     if (li < T) *reinterpret_cast<f32x4_t*>(a.tape + obase + 16 * wave + 4 * kq) = D[0];
   } else {
     // the tape leaves from LDS in full 128-byte lines: lane (t, q) stores this wave's rows
@@ -1233,14 +1286,14 @@ int gdn_forward_launch(const char* who, const void* q, const void* k, const void
     const bool wide = in_dtype == DFLASH_FP32;
     const bool split = in_dtype == DFLASH_BF16;  // q and k are bf16 numbers: exact products on the bf16 matrix cores
     if (z) {
-      if (wide) hipLaunchKernelGGL((gdn_forward_chunk_128<true, true, false, false>), grid, block, lds, s, a);
-      else if (split) hipLaunchKernelGGL((gdn_forward_chunk_128<false, true, true, false>), grid, block, lds, s, a);
-      else hipLaunchKernelGGL((gdn_forward_chunk_128<false, true, false, false>), grid, block, lds, s, a);
+      if (wide) hipLaunchKernelGGL((gdn_forward_chunk_128<true, true, false, kFromArrays>), grid, block, lds, s, a);
+      else if (split) hipLaunchKernelGGL((gdn_forward_chunk_128<false, true, true, kFromArrays>), grid, block, lds, s, a);
+      else hipLaunchKernelGGL((gdn_forward_chunk_128<false, true, false, kFromArrays>), grid, block, lds, s, a);
       norm_done = true;
     } else {
-      if (wide) hipLaunchKernelGGL((gdn_forward_chunk_128<true, false, false, false>), grid, block, lds, s, a);
-      else if (split) hipLaunchKernelGGL((gdn_forward_chunk_128<false, false, true, false>), grid, block, lds, s, a);
-      else hipLaunchKernelGGL((gdn_forward_chunk_128<false, false, false, false>), grid, block, lds, s, a);
+      if (wide) hipLaunchKernelGGL((gdn_forward_chunk_128<true, false, false, kFromArrays>), grid, block, lds, s, a);
+      else if (split) hipLaunchKernelGGL((gdn_forward_chunk_128<false, false, true, kFromArrays>), grid, block, lds, s, a);
+      else hipLaunchKernelGGL((gdn_forward_chunk_128<false, false, false, kFromArrays>), grid, block, lds, s, a);
     }
   } else if (by_rows != nullptr) {
     a.row_parts = Divisor::of(Dv / rows);
@@ -1327,8 +1380,115 @@ extern "C" int dflash_gdn_block(const dflash_gdn_block_args* p, void* stream) {
   hipStream_t s = (hipStream_t)stream;
   void* args[] = {&a};
   if (D == 128 && p->state_dtype == DFLASH_FP32) {  // the closed form, its output norm in the same launch
-    const void* fn = p->z ? (const void*)gdn_forward_chunk_128<false, true, true, true> : (const void*)gdn_forward_chunk_128<false, false, true, true>;
-    DFLASH_HIP_OK(hipLaunchKernel(fn, dim3((unsigned)(slots * Hv)), dim3(kBlockThreads), args, kChunkLdsFloats * sizeof(float), s));
+    // A compute unit holds one workgroup of thirteen waves or two of four.  us for 16 tokens (one token), thirteen waves and four: 256 heads
+    // 13.7 (13.3) and about 17 (15), 288 heads 24.3 (23.5) and 21.5 (19.7), 512 heads 25.7 (25.3) and 22.5 (19.7), 768 heads 38.0 (36.0) and
+    // 35.8 (30.3), 1024 heads 50.1 (47.3) and 42.7 (35.8).
+    const bool wide = in_dtype == DFLASH_FP32;
+    const bool split = in_dtype == DFLASH_BF16;  // q and k are bf16 numbers: exact products on the bf16 matrix cores
+    if (z) {
+      if (wide) hipLaunchKernelGGL((gdn_forward_chunk_128<true, true, false, kFromArrays>), grid, block, lds, s, a);
+      else if (split) hipLaunchKernelGGL((gdn_forward_chunk_128<false, true, true, kFromArrays>), grid, block, lds, s, a);
+      else hipLaunchKernelGGL((gdn_forward_chunk_128<false, true, false, kFromArrays>), grid, block, lds, s, a);
+      norm_done = true;
+    } else {
+      if (wide) hipLaunchKernelGGL((gdn_forward_chunk_128<true, false, false, kFromArrays>), grid, block, lds, s, a);
+      else if (split) hipLaunchKernelGGL((gdn_forward_chunk_128<false, false, true, kFromArrays>), grid, block, lds, s, a);
+      else hipLaunchKernelGGL((gdn_forward_chunk_128<false, false, false, kFromArrays>), grid, block, lds, s, a);
+    }
+  } else if (by_rows != nullptr) {
+    a.row_parts = Divisor::of(Dv / rows);
+    void* args[] = {&a};
+    DFLASH_HIP_OK(hipLaunchKernel(by_rows, dim3((unsigned)(slots * Hv * (Dv / rows))), block, args, 0, s));
+  } else if (fast) {
+    if (g_per_dk) {
+      hipLaunchKernelGGL((gdn_forward_128<true, false>), grid, block, smem, s, a);
+    } else if (state_dtype == DFLASH_FP32) {
+      hipLaunchKernelGGL((gdn_forward_128<false, true>), grid, block, smem, s, a);
+    } else {
+      hipLaunchKernelGGL((gdn_forward_128<false, false>), grid, block, smem, s, a);
+    }
+  } else {
+    hipLaunchKernelGGL(gdn_forward_generic, grid, block, 0, s, a);
+  }
+  DFLASH_HIP_OK(hipGetLastError());
+  if (z && !norm_done)  // the other kernels leave the recurrence's output in y: normalise it in place
+    return T == 0 ? DFLASH_OK : gdn_gated_norm_launch(y, z, norm_weight, y, slots, T, Hv, Dv, z_batch, z_row, in_dtype, weight_dtype,
+                                                      eps, s);
+  return DFLASH_OK;
+}
+
+// The value a Python float takes when it meets a bf16 array.
+float as_bf16_scalar(double v) {
+  const float f = (float)v;
+  uint32_t u;
+  __builtin_memcpy(&u, &f, 4);
+  u += 0x7fffu + ((u >> 16) & 1u);
+  u &= 0xffff0000u;
+  float r;
+  __builtin_memcpy(&r, &u, 4);
+  return r;
+}
+
+}  // namespace
+}  // namespace dflash
+
+extern "C" int dflash_gdn_block(const dflash_gdn_block_args* p, void* stream) {
+  using namespace dflash;
+  const char* who = "dflash_gdn_block";
+  DFLASH_REQUIRE(p && p->qkv && p->conv_w && p->a && p->b && p->A_log && p->dt_bias && p->conv_next && p->state_in && p->state_out &&
+                     p->y && p->tape && (!p->z || p->norm_weight),
+                 DFLASH_ERR_ARG, "%s: null operand", who);
+  DFLASH_REQUIRE(p->state_in != p->state_out, DFLASH_ERR_ARG, "%s: state_out must not alias state_in", who);
+  auto ok = [](int dt) { return dt == DFLASH_BF16 || dt == DFLASH_FP16 || dt == DFLASH_FP32; };
+  DFLASH_REQUIRE(ok(p->param_dtype) && ok(p->state_dtype) && (!p->z || ok(p->weight_dtype)), DFLASH_ERR_ARG, "%s: unknown dtype code", who);
+  const int slots = p->slots, T = p->T, Hk = p->Hk, Hv = p->Hv, D = p->D;
+  DFLASH_REQUIRE(slots >= 0 && T >= 1 && T <= 16 && Hk > 0 && Hv > 0 && Hv % Hk == 0 && (D == 64 || D == 128), DFLASH_ERR_SHAPE,
+                 "%s: 1 to 16 steps of heads of 64 or 128, whole groups of value heads; got %d steps, %d and %d heads of %d", who, T, Hk,
+                 Hv, D);
+  DFLASH_REQUIRE(p->qkv_row < (1ll << 26), DFLASH_ERR_SHAPE, "%s: rows of %lld elements", who, p->qkv_row);
+  DFLASH_REQUIRE((long long)slots * Hv * 8 < (1ll << 31) && (long long)slots * T * (2ll * Hk + Hv) * D < (1ll << 31), DFLASH_ERR_SHAPE,
+                 "%s: too many (slot, head) pairs", who);
+  uintptr_t strides = 0;
+  for (long long v : {p->qkv_slot, p->qkv_row, p->a_slot, p->a_row, p->b_slot, p->b_row, p->z_slot, p->z_row})
+    DFLASH_REQUIRE(v >= 0, DFLASH_ERR_SHAPE, "%s: negative stride", who);
+  strides = (uintptr_t)(p->qkv_slot | p->qkv_row) * 2;
+  DFLASH_REQUIRE((((uintptr_t)p->qkv | (uintptr_t)p->conv_state | (uintptr_t)p->conv_w | (uintptr_t)p->conv_next | (uintptr_t)p->k |
+                   (uintptr_t)p->qkv_out | strides) % 8) == 0,
+                 DFLASH_ERR_ARG, "%s: projections, conv arrays and k must be 8-byte aligned", who);
+  DFLASH_REQUIRE((((uintptr_t)p->state_in | (uintptr_t)p->state_out | (uintptr_t)p->y | (uintptr_t)p->tape | (uintptr_t)p->z |
+                   (uintptr_t)p->norm_weight | (p->z ? (uintptr_t)(p->z_slot | p->z_row) * 2 : 0)) % 16) == 0,
+                 DFLASH_ERR_ARG, "%s: states, y, tape, z and the norm weight must be 16-byte aligned", who);
+  if (slots == 0) return DFLASH_OK;
+
+  GdnArgs a = {};
+  a.state_in = p->state_in; a.state_out = p->state_out; a.y = p->y; a.tape = p->tape;
+  a.T = T; a.Hk = Hk; a.Hv = Hv; a.Dk = a.Dv = D;
+  a.heads = Divisor::of(Hv); a.group = Divisor::of(Hv / Hk); a.row_parts = Divisor::of(1);
+  a.in_dtype = a.g_dtype = a.beta_dtype = DFLASH_BF16; a.state_dtype = p->state_dtype;
+  a.z = p->z; a.z_batch = p->z_slot; a.z_row = p->z_row; a.norm_weight = p->norm_weight; a.weight_dtype = p->weight_dtype;
+  a.eps = p->norm_eps;
+  BlockArgs& b = a.block;
+  b.qkv = (const uint16_t*)p->qkv; b.conv_state = (const uint16_t*)p->conv_state; b.conv_w = (const uint16_t*)p->conv_w;
+  b.a = (const uint16_t*)p->a; b.b = (const uint16_t*)p->b; b.A_log = p->A_log; b.dt_bias = p->dt_bias;
+  b.conv_next = (uint16_t*)p->conv_next; b.k_out = (uint16_t*)p->k; b.qkv_out = (uint16_t*)p->qkv_out; b.g_out = p->g;
+  b.qkv_slot = p->qkv_slot; b.qkv_row = p->qkv_row; b.a_slot = p->a_slot; b.a_row = p->a_row; b.b_slot = p->b_slot; b.b_row = p->b_row;
+  b.param_dt = p->param_dtype; b.eps = p->eps;
+  const double inv_scale = 1.0 / sqrt((double)D);
+  b.scale_q = as_bf16_scalar(inv_scale * inv_scale);
+  b.scale_k = as_bf16_scalar(inv_scale);
+
+  hipStream_t s = (hipStream_t)stream;
+  void* args[] = {&a};
+  if (D == 128 && p->state_dtype == DFLASH_FP32) {  // the closed form, its output norm in the same launch
+    // A compute unit holds one workgroup of thirteen waves or two of four.  us for 16 tokens (one token), thirteen waves and four: 256 heads
+    // 13.8 (13.3) and 17.7 (15.4), 288 heads 24.3 (23.5) and 23.1 (21.4), 512 heads 25.7 (25.3) and 24.0 (21.0), 768 heads 38.0 (36.0) and 38.4 (32.8),
+    // 1024 heads 50.1 (47.3) and 45.1 (37.9).
+    const bool wide = slots * Hv <= qmm_stream_grid();
+    const void* fn = wide ? (p->z ? (const void*)gdn_forward_chunk_128<false, true, true, kThirteenWaves>
+                                : (const void*)gdn_forward_chunk_128<false, false, true, kThirteenWaves>)
+                          : (p->z ? (const void*)gdn_forward_chunk_128<false, true, true, kFourWaves>
+                                : (const void*)gdn_forward_chunk_128<false, false, true, kFourWaves>);
+    DFLASH_HIP_OK(hipLaunchKernel(fn, dim3((unsigned)(slots * Hv)), dim3(wide ? kBlockThreads : kThreads), args, kChunkLdsFloats * sizeof(float), s));
     return DFLASH_OK;
   }
   int rows = D;

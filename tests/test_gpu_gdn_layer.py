@@ -344,6 +344,13 @@ def test_a_block_whose_last_wave_of_steps_is_not_full(monkeypatch, S):
         test_a_block_in_one_launch(monkeypatch, state_dtype, 1, S, 2, 4, 128, True)
 
 
+@pytest.mark.parametrize("S", [1, 3, 4, 5, 13, 16])
+@pytest.mark.parametrize("B,Hk,Hv", [(9, 16, 32), (1, 1, 258)])
+def test_a_block_of_more_heads_than_compute_units(monkeypatch, S, B, Hk, Hv):
+    """From 257 heads of fp32 states on a head is four waves' work, two heads at a time: the bits of the other form's parts."""
+    test_a_block_in_one_launch(monkeypatch, torch.float32, B, S, Hk, Hv, 128, True)
+
+
 @pytest.mark.parametrize("T,D,times", [(17, 128, 1), (40, 64, 1), (33, 128, 40)])
 @pytest.mark.parametrize("normed", [True, False])
 def test_a_prompt_that_starts_from_nothing(native_lib, T, D, times, normed):
