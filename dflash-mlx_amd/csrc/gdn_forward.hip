@@ -1383,106 +1383,6 @@ extern "C" int dflash_gdn_block(const dflash_gdn_block_args* p, void* stream) {
     // A compute unit holds one workgroup of thirteen waves or two of four.  us for 16 tokens (one token), thirteen waves and four: 256 heads
     // 13.7 (13.3) and about 17 (15), 288 heads 24.3 (23.5) and 21.5 (19.7), 512 heads 25.7 (25.3) and 22.5 (19.7), 768 heads 38.0 (36.0) and
     // 35.8 (30.3), 1024 heads 50.1 (47.3) and 42.7 (35.8).
-    const bool wide = in_dtype == DFLASH_FP32;
-    const bool split = in_dtype == DFLASH_BF16;  // q and k are bf16 numbers: exact products on the bf16 matrix cores
-    if (z) {
-      if (wide) hipLaunchKernelGGL((gdn_forward_chunk_128<true, true, false, kFromArrays>), grid, block, lds, s, a);
-      else if (split) hipLaunchKernelGGL((gdn_forward_chunk_128<false, true, true, kFromArrays>), grid, block, lds, s, a);
-      else hipLaunchKernelGGL((gdn_forward_chunk_128<false, true, false, kFromArrays>), grid, block, lds, s, a);
-      norm_done = true;
-    } else {
-      if (wide) hipLaunchKernelGGL((gdn_forward_chunk_128<true, false, false, kFromArrays>), grid, block, lds, s, a);
-      else if (split) hipLaunchKernelGGL((gdn_forward_chunk_128<false, false, true, kFromArrays>), grid, block, lds, s, a);
-      else hipLaunchKernelGGL((gdn_forward_chunk_128<false, false, false, kFromArrays>), grid, block, lds, s, a);
-    }
-  } else if (by_rows != nullptr) {
-    a.row_parts = Divisor::of(Dv / rows);
-    void* args[] = {&a};
-    DFLASH_HIP_OK(hipLaunchKernel(by_rows, dim3((unsigned)(slots * Hv * (Dv / rows))), block, args, 0, s));
-  } else if (fast) {
-    if (g_per_dk) {
-      hipLaunchKernelGGL((gdn_forward_128<true, false>), grid, block, smem, s, a);
-    } else if (state_dtype == DFLASH_FP32) {
-      hipLaunchKernelGGL((gdn_forward_128<false, true>), grid, block, smem, s, a);
-    } else {
-      hipLaunchKernelGGL((gdn_forward_128<false, false>), grid, block, smem, s, a);
-    }
-  } else {
-    hipLaunchKernelGGL(gdn_forward_generic, grid, block, 0, s, a);
-  }
-  DFLASH_HIP_OK(hipGetLastError());
-  if (z && !norm_done)  // the other kernels leave the recurrence's output in y: normalise it in place
-    return T == 0 ? DFLASH_OK : gdn_gated_norm_launch(y, z, norm_weight, y, slots, T, Hv, Dv, z_batch, z_row, in_dtype, weight_dtype,
-                                                      eps, s);
-  return DFLASH_OK;
-}
-
-// The value a Python float takes when it meets a bf16 array.
-float as_bf16_scalar(double v) {
-  const float f = (float)v;
-  uint32_t u;
-  __builtin_memcpy(&u, &f, 4);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  u &= 0xffff0000u;
-  float r;
-  __builtin_memcpy(&r, &u, 4);
-  return r;
-}
-
-}  // namespace
-}  // namespace dflash
-
-extern "C" int dflash_gdn_block(const dflash_gdn_block_args* p, void* stream) {
-  using namespace dflash;
-  const char* who = "dflash_gdn_block";
-  DFLASH_REQUIRE(p && p->qkv && p->conv_w && p->a && p->b && p->A_log && p->dt_bias && p->conv_next && p->state_in && p->state_out &&
-                     p->y && p->tape && (!p->z || p->norm_weight),
-                 DFLASH_ERR_ARG, "%s: null operand", who);
-  DFLASH_REQUIRE(p->state_in != p->state_out, DFLASH_ERR_ARG, "%s: state_out must not alias state_in", who);
-  auto ok = [](int dt) { return dt == DFLASH_BF16 || dt == DFLASH_FP16 || dt == DFLASH_FP32; };
-  DFLASH_REQUIRE(ok(p->param_dtype) && ok(p->state_dtype) && (!p->z || ok(p->weight_dtype)), DFLASH_ERR_ARG, "%s: unknown dtype code", who);
-  const int slots = p->slots, T = p->T, Hk = p->Hk, Hv = p->Hv, D = p->D;
-  DFLASH_REQUIRE(slots >= 0 && T >= 1 && T <= 16 && Hk > 0 && Hv > 0 && Hv % Hk == 0 && (D == 64 || D == 128), DFLASH_ERR_SHAPE,
-                 "%s: 1 to 16 steps of heads of 64 or 128, whole groups of value heads; got %d steps, %d and %d heads of %d", who, T, Hk,
-                 Hv, D);
-  DFLASH_REQUIRE(p->qkv_row < (1ll << 26), DFLASH_ERR_SHAPE, "%s: rows of %lld elements", who, p->qkv_row);
-  DFLASH_REQUIRE((long long)slots * Hv * 8 < (1ll << 31) && (long long)slots * T * (2ll * Hk + Hv) * D < (1ll << 31), DFLASH_ERR_SHAPE,
-                 "%s: too many (slot, head) pairs", who);
-  uintptr_t strides = 0;
-  for (long long v : {p->qkv_slot, p->qkv_row, p->a_slot, p->a_row, p->b_slot, p->b_row, p->z_slot, p->z_row})
-    DFLASH_REQUIRE(v >= 0, DFLASH_ERR_SHAPE, "%s: negative stride", who);
-  strides = (uintptr_t)(p->qkv_slot | p->qkv_row) * 2;
-  DFLASH_REQUIRE((((uintptr_t)p->qkv | (uintptr_t)p->conv_state | (uintptr_t)p->conv_w | (uintptr_t)p->conv_next | (uintptr_t)p->k |
-                   (uintptr_t)p->qkv_out | strides) % 8) == 0,
-                 DFLASH_ERR_ARG, "%s: projections, conv arrays and k must be 8-byte aligned", who);
-  DFLASH_REQUIRE((((uintptr_t)p->state_in | (uintptr_t)p->state_out | (uintptr_t)p->y | (uintptr_t)p->tape | (uintptr_t)p->z |
-                   (uintptr_t)p->norm_weight | (p->z ? (uintptr_t)(p->z_slot | p->z_row) * 2 : 0)) % 16) == 0,
-                 DFLASH_ERR_ARG, "%s: states, y, tape, z and the norm weight must be 16-byte aligned", who);
-  if (slots == 0) return DFLASH_OK;
-
-  GdnArgs a = {};
-  a.state_in = p->state_in; a.state_out = p->state_out; a.y = p->y; a.tape = p->tape;
-  a.T = T; a.Hk = Hk; a.Hv = Hv; a.Dk = a.Dv = D;
-  a.heads = Divisor::of(Hv); a.group = Divisor::of(Hv / Hk); a.row_parts = Divisor::of(1);
-  a.in_dtype = a.g_dtype = a.beta_dtype = DFLASH_BF16; a.state_dtype = p->state_dtype;
-  a.z = p->z; a.z_batch = p->z_slot; a.z_row = p->z_row; a.norm_weight = p->norm_weight; a.weight_dtype = p->weight_dtype;
-  a.eps = p->norm_eps;
-  BlockArgs& b = a.block;
-  b.qkv = (const uint16_t*)p->qkv; b.conv_state = (const uint16_t*)p->conv_state; b.conv_w = (const uint16_t*)p->conv_w;
-  b.a = (const uint16_t*)p->a; b.b = (const uint16_t*)p->b; b.A_log = p->A_log; b.dt_bias = p->dt_bias;
-  b.conv_next = (uint16_t*)p->conv_next; b.k_out = (uint16_t*)p->k; b.qkv_out = (uint16_t*)p->qkv_out; b.g_out = p->g;
-  b.qkv_slot = p->qkv_slot; b.qkv_row = p->qkv_row; b.a_slot = p->a_slot; b.a_row = p->a_row; b.b_slot = p->b_slot; b.b_row = p->b_row;
-  b.param_dt = p->param_dtype; b.eps = p->eps;
-  const double inv_scale = 1.0 / sqrt((double)D);
-  b.scale_q = as_bf16_scalar(inv_scale * inv_scale);
-  b.scale_k = as_bf16_scalar(inv_scale);
-
-  hipStream_t s = (hipStream_t)stream;
-  void* args[] = {&a};
-  if (D == 128 && p->state_dtype == DFLASH_FP32) {  // the closed form, its output norm in the same launch
-    // A compute unit holds one workgroup of thirteen waves or two of four.  us for 16 tokens (one token), thirteen waves and four: 256 heads
-    // 13.8 (13.3) and 17.7 (15.4), 288 heads 24.3 (23.5) and 23.1 (21.4), 512 heads 25.7 (25.3) and 24.0 (21.0), 768 heads 38.0 (36.0) and 38.4 (32.8),
-    // 1024 heads 50.1 (47.3) and 45.1 (37.9).
     const bool wide = slots * Hv <= qmm_stream_grid();
     const void* fn = wide ? (p->z ? (const void*)gdn_forward_chunk_128<false, true, true, kThirteenWaves>
                                 : (const void*)gdn_forward_chunk_128<false, false, true, kThirteenWaves>)
