@@ -19,18 +19,27 @@ struct Plan {
 // One row of K <= 1024 against few rows of W is qmm_narrow's, which has no ring to set up (1024 x 512, 1 / 16 rows: 3.1 / 3.7 us there, 3.7 /
 // 3.8 here; 1024 x 8192 5.3 / 5.9 there, 4.8 / 5.0 here); beyond that K a unit of x is dearer there (3072 x 2048 5.2 / 7.0 and 4.7 / 5.0).
 //
-// Slices by a model fitted to 1 .. 4 of them at eight shapes, in 10 ns and less what all have: 75 per chunk for x and the first tile, 30 + 40 per
-// chunk for each further tile of the busiest workgroup (a lane in twenty with one more does not count), 120 for the meeting of slices.
-// us for 16 rows, 1 / 2 / 3 / 4 slices: 4096 x 4096 6.1 / 6.7 / 7.0 / 8.0; 5120 x 5120 9.1 / 8.5 / 8.4 / 9.6; 6144 x 512 7.4 / 5.6 / 5.0 / 5.0;
-// 12288 x 4096 - / 11.7 / 11.1 / 11.0; 17408 x 5120 - / - / 17.4 / 17.8 (K x N).  M does not enter: a row must not change with the rows beside it.
+// Slices by a model fitted to 1000 calls of 1 and 16 rows with every number of them (K from 2048 to 24576, N from 1024 to 32768, all group sizes,
+// weights from memory and from the cache): in 10 ns and less what all have, 80 per chunk for x and the first tile, 35 + 9 per chunk for each further tile
+// of the busiest workgroup (groups of 32: 96 and 4) and 8 per chunk for each of the mean one, 110 for the meeting of slices and, for an odd number of chunks, whose runs of 64
+// bytes share their lines with other waves, 1 per MB.  What it picks is within 0.3 % of the best in the mean and 6 % at most.  us for 16 rows, 1 / 2 / 3 / 4
+// slices: 4096 x 5120 7.3 / 6.8 / 7.1 / 8.9; 5120 x 4096 7.6 / 7.4 / 6.8 / 7.6; 6144 x 4096 8.3 / 7.7 / 6.9 / 7.8; 12288 x 4096 - / 11.7 / 10.8 / 10.5; 14336 x 8192
+// - / - / 19.9 / 18.0; 17408 x 5120 - / - / 15.9 / 16.6 (K x N).  M does not enter: a row must not change with the rows beside it.  (The tile that a few
+// workgroups have more than the others counts in full: 14336 x 4096 in three slices has 256 tiles for 85 workgroups, 13.3, in four slices 11.7; the
+// streaming kernel 13.0.)
+//
+// Where N / 128 divides the compute units, the streaming kernel (groups of 64) has equal parts without a remainder and is at its best: there the call is
+// its own if a model of either says so (2.5 % rms over 71 such shapes).  us there and here: 9216 x 16384 21.2 / 22.3, 12800 x 16384 27.5 / 29.4,
+// 6400 x 32768 27.4 / 28.9, 17408 x 8192 21.4 / 22.5; 16384 x 8192 19.7 / 18.3.
 Plan make_plan(int K, int N, int group_size, int cus) {
   const int step = group_size == 128 ? 2 : 1, most = most_chunks(group_size, 1);
   if ((group_size != 32 && group_size != 64 && group_size != 128) || K % (kChunk * step) != 0 || N % 16 != 0 || N < 16) return {0, 0, cus, 0};
   if (K <= 1024 && N <= 4096) return {0, 0, cus, 0};
   if ((long long)N * K / 2 >= (1ll << 31) - (1 << 24)) return {0, 0, cus, 0};  // 32-bit byte offsets, and kPast behind them
   const int pieces = K / (kChunk * step), tiles = N / 16;
+  const double megabytes = 1e-6 * N * K * (0.5 + 4.0 / group_size), first = group_size == 32 ? 96.0 : 80.0, further = group_size == 32 ? 4.0 : 9.0;
   Plan best = {0, 0, cus, 0};
-  int best_cost = 0;
+  double best_cost = 0.0;
   for (int slices = 1; slices <= kMostSlices; ++slices) {
     const int parts = kWaves * slices;
     if (pieces < parts || slices > cus) break;
@@ -38,9 +47,15 @@ Plan make_plan(int K, int N, int group_size, int cus) {
     if (chunks > most) continue;
     if ((long long)(slices - 1) * N > 65536) break;  // every other slice keeps a KiB per tile in the workspace that the streaming kernel asks for
     if (chunks < 2) chunks = 2;
-    const int lanes = cus / slices, most_tiles = (20 * tiles + 19 * lanes - 1) / (20 * lanes);
-    const int cost = 75 * chunks + (most_tiles - 1) * (30 + 40 * chunks) + (slices > 1 ? 120 : 0);
+    const int lanes = tiles < cus / slices ? tiles : cus / slices, more = (tiles + lanes - 1) / lanes - 1;
+    double cost = first * chunks + more * (35.0 + further * chunks) + 8.0 * chunks * ((double)tiles / lanes - 1.0);
+    if (slices > 1) cost += 110.0;
+    if (chunks % 2 != 0) cost += megabytes;
     if (best.chunks == 0 || cost < best_cost) best.chunks = chunks, best.slices = slices, best_cost = cost;
+  }
+  if (best.slices > 1 && group_size == 64 && N % 128 == 0 && N >= 4096 && cus % (N / 128) == 0) {
+    const double us = 1.83 + 0.0109 * best_cost + 0.058 * megabytes, streaming_us = 7.2 + (K % 512 == 0 ? 0.171 : 0.186) * megabytes;
+    if (us > streaming_us) return {0, 0, cus, 0};
   }
   best.cus = cus;
   best.workspace = best.slices < 2 ? 0 : (size_t)64 * 1024 + (size_t)tiles * (best.slices - 1) * 1024;
