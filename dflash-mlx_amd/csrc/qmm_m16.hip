@@ -436,9 +436,9 @@ bool qmm_stream_packed_eligible(int K, int N, int group_size);
 bool qmm_narrow_covers(const void* scales, const void* biases, int K, int N, int group_size, bool silu_mul);
 int qmm_narrow_launch(const void* x, const void* w, const void* scales, const void* biases, void* y, int M, int K, int N, int group_size,
                       int act_dtype, int sb_dtype, bool silu_mul, bool packed, hipStream_t stream);
-// qmm_resident.hip: x and w 16-byte aligned, up to 16 rows
+// qmm_resident.hip: x and w 16-byte aligned, up to 16 rows; narrow: qmm_narrow_covers the call
 bool qmm_resident_covers(const void* scales, const void* biases, size_t workspace_bytes, int K, int N, int group_size, int act_dtype,
-                         int sb_dtype);
+                         int sb_dtype, bool narrow);
 int qmm_resident_launch(const void* x, const void* w, const void* scales, const void* biases, void* y, void* workspace, int M, int K,
                         int N, int group_size, int dtype, bool silu_mul, bool packed, int spin_limit, hipStream_t stream);
 // qmm_resident_gather.hip: x and w 16-byte aligned, P within the tables' limits
@@ -530,10 +530,11 @@ extern "C" int dflash_qmm_few_silu_mul_by(const void* x, const uint32_t* w_q, co
                  "dflash_qmm_few_silu_mul: the streaming kernel does not cover K=%d N=%d gs=%d", K, N, group_size);
   DFLASH_REQUIRE((((uintptr_t)x | (uintptr_t)w_q) % 16) == 0 && (((uintptr_t)scales | (uintptr_t)biases) % 4) == 0,
                  DFLASH_ERR_ARG, "dflash_qmm_few_silu_mul: x and w_q must be 16-byte aligned, scales and biases 4-byte aligned");
-  if (kernel == DFLASH_QMM_KERNEL_FASTEST && qmm_resident_covers(scales, biases, workspace_bytes, K, N, group_size, dtype, dtype) &&
+  const bool narrow = qmm_narrow_covers(scales, biases, K, N, group_size, true);
+  if (kernel == DFLASH_QMM_KERNEL_FASTEST && qmm_resident_covers(scales, biases, workspace_bytes, K, N, group_size, dtype, dtype, narrow) &&
       qmm_stream_workspace_given(workspace, workspace_bytes, K, N))
     return qmm_resident_launch(x, w_q, scales, biases, y, workspace, M, K, N, group_size, dtype, true, false, 0, (hipStream_t)stream);
-  if (qmm_narrow_covers(scales, biases, K, N, group_size, true) && qmm_stream_workspace_given(workspace, workspace_bytes, K, N))
+  if (narrow && qmm_stream_workspace_given(workspace, workspace_bytes, K, N))
     return qmm_narrow_launch(x, w_q, scales, biases, y, M, K, N, group_size, dtype, dtype, true, false, (hipStream_t)stream);
   return qmm_stream_launch(x, w_q, scales, biases, y, workspace, workspace_bytes, M, K, N, group_size, dtype, dtype, true,
                            (hipStream_t)stream);
@@ -575,7 +576,8 @@ int qmm_up_to_16(const void* x, const uint32_t* w_q, const void* scales, const v
                    (((uintptr_t)scales | (uintptr_t)biases) % 4) == 0 && workspace != nullptr &&
                    workspace_bytes >= qmm_stream_workspace_bytes(N, qmm_stream_grid());
   if (kernel != DFLASH_QMM_KERNEL_TILE && (qmm_stream_eligible(K, N, group_size) || any)) {
-    if (kernel == DFLASH_QMM_KERNEL_FASTEST && qmm_resident_covers(scales, biases, workspace_bytes, K, N, group_size, act_dtype, sb_dtype) &&
+    if (kernel == DFLASH_QMM_KERNEL_FASTEST &&
+        qmm_resident_covers(scales, biases, workspace_bytes, K, N, group_size, act_dtype, sb_dtype, narrow) &&
         qmm_stream_workspace_given(workspace, workspace_bytes, K, N))
       return qmm_resident_launch(x, w_q, scales, biases, y, workspace, M, K, N, group_size, act_dtype, false, false, 0, (hipStream_t)stream);
     if (narrow && qmm_stream_workspace_given(workspace, workspace_bytes, K, N)) return narrow_launch();
@@ -717,10 +719,12 @@ extern "C" int dflash_qmm_m16_packed_by(const void* x, const void* codes, const 
   DFLASH_REQUIRE(((uintptr_t)x % 16) == 0 && ((uintptr_t)codes % 16) == 0 && ((uintptr_t)scales % 16) == 0 &&
                      ((uintptr_t)biases % 16) == 0,
                  DFLASH_ERR_ARG, "dflash_qmm_m16_packed: operands must be 16-byte aligned");
-  if (kernel == DFLASH_QMM_KERNEL_FASTEST && qmm_resident_covers(scales, biases, workspace_bytes, K, N, group_size, act_dtype, sb_dtype) &&
+  const bool narrow = kernel != DFLASH_QMM_KERNEL_STREAM && qmm_narrow_covers(scales, biases, K, N, group_size, false);
+  if (kernel == DFLASH_QMM_KERNEL_FASTEST &&
+      qmm_resident_covers(scales, biases, workspace_bytes, K, N, group_size, act_dtype, sb_dtype, narrow) &&
       qmm_stream_workspace_given(workspace, workspace_bytes, K, N))
     return qmm_resident_launch(x, codes, scales, biases, y, workspace, 16, K, N, group_size, act_dtype, false, true, 0, (hipStream_t)stream);
-  if (kernel != DFLASH_QMM_KERNEL_STREAM && qmm_narrow_covers(scales, biases, K, N, group_size, false))
+  if (narrow)
     return qmm_narrow_launch(x, codes, scales, biases, y, 16, K, N, group_size, act_dtype, sb_dtype, false, true, (hipStream_t)stream);
   return qmm_stream_packed_launch(x, codes, scales, biases, y, workspace, workspace_bytes, K, N,
                                   act_dtype, sb_dtype, (hipStream_t)stream);

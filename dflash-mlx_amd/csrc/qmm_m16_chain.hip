@@ -984,7 +984,7 @@ int qmm_stream_grid();
 int qmm_stream_pick_grid(int units, int row_blocks, int cus);
 bool qmm_stream_eligible(int K, int N, int group_size);
 bool qmm_resident_covers(const void* scales, const void* biases, size_t workspace_bytes, int K, int N, int group_size, int act_dtype,
-                         int sb_dtype);
+                         int sb_dtype, bool narrow);
 int qmm_resident_launch(const void* x, const void* w, const void* scales, const void* biases, void* y, void* workspace, int M, int K,
                         int N, int group_size, int dtype, bool silu_mul, bool packed, int spin_limit, hipStream_t stream);
 int qmm_stream_gate_up_launch(const void* x, const uint32_t* w, const void* scales, const void* biases, void* y,
@@ -1085,7 +1085,7 @@ int qmm_chain_launch(const dflash_qmm_problem* problems, int count, void* worksp
   // 4096 x 24576 22.8 -> 19.3 us, packed 21.1 -> 18.0.  (Its kernels are built for one type only.)
   if (count == 1 && problems[0].epilogue == DFLASH_QMM_EPILOGUE_SILU_MUL && act_dtype == sb_dtype) {
     const dflash_qmm_problem& q = problems[0];
-    if ((flags & DFLASH_QMM_CHAIN_FASTEST) != 0 && qmm_resident_covers(q.scales, q.biases, workspace_bytes, q.K, q.N, 64, act_dtype, sb_dtype))
+    if ((flags & DFLASH_QMM_CHAIN_FASTEST) != 0 && qmm_resident_covers(q.scales, q.biases, workspace_bytes, q.K, q.N, 64, act_dtype, sb_dtype, false))
       return qmm_resident_launch(q.x, q.w_q, q.scales, q.biases, q.y, workspace, 16, q.K, q.N, 64, act_dtype, true,
                                  q.layout == DFLASH_QMM_LAYOUT_PACKED, spin_limit, stream);
     return qmm_stream_gate_up_launch(q.x, q.w_q, q.scales, q.biases, q.y, workspace, workspace_bytes, q.K, q.N, act_dtype,

@@ -15,9 +15,13 @@ struct Plan {
   int slices;
   int cus;
   size_t workspace;
+  bool padded;  // qmm_narrow's where that has the shape
 };
 // One row of K <= 1024 against few rows of W is qmm_narrow's, which has no ring to set up (1024 x 512, 1 / 16 rows: 3.1 / 3.7 us there, 3.7 /
-// 3.8 here; 1024 x 8192 5.3 / 5.9 there, 4.8 / 5.0 here); beyond that K a unit of x is dearer there (3072 x 2048 5.2 / 7.0 and 4.7 / 5.0).
+// 3.8 here; 1024 x 8192 5.3 / 5.9 there, 4.8 / 5.0 here), and so is a K that leaves more than a third of the waves' chunks empty: 1152 x 2048 3.5 / 4.4 there and
+// 4.0 / 4.2 here, 2304 x 1024 in groups of 128 3.9 / 6.0 and 5.2 / 5.6.  With fuller waves a verify block gains what one row loses, or more (1536 x 2048
+// 3.8 / 4.7 and 4.0 / 4.2, 2560 x 2048 4.5 / 6.5 and 4.6 / 4.9, 3072 x 2048 in groups of 128 4.5 / 6.8 and 5.3 / 5.6; 3072 x 2048 5.2 / 7.3 and 4.6 / 5.1).
+// A row's bits must not depend on the rows beside it, so there is one kernel for both.
 //
 // Slices by a model fitted to 1000 calls of 1 and 16 rows with every number of them (K from 2048 to 24576, N from 1024 to 32768, all group sizes,
 // weights from memory and from the cache): in 10 ns and less what all have, 80 per chunk for x and the first tile, 35 + 9 per chunk for each further tile
@@ -33,12 +37,12 @@ struct Plan {
 // 6400 x 32768 27.4 / 28.9, 17408 x 8192 21.4 / 22.5; 16384 x 8192 19.7 / 18.3.
 Plan make_plan(int K, int N, int group_size, int cus) {
   const int step = group_size == 128 ? 2 : 1, most = most_chunks(group_size, 1);
-  if ((group_size != 32 && group_size != 64 && group_size != 128) || K % (kChunk * step) != 0 || N % 16 != 0 || N < 16) return {0, 0, cus, 0};
-  if (K <= 1024 && N <= 4096) return {0, 0, cus, 0};
-  if ((long long)N * K / 2 >= (1ll << 31) - (1 << 24)) return {0, 0, cus, 0};  // 32-bit byte offsets, and kPast behind them
+  if ((group_size != 32 && group_size != 64 && group_size != 128) || K % (kChunk * step) != 0 || N % 16 != 0 || N < 16) return {0, 0, cus, 0, false};
+  if (K <= 1024 && N <= 4096) return {0, 0, cus, 0, false};
+  if ((long long)N * K / 2 >= (1ll << 31) - (1 << 24)) return {0, 0, cus, 0, false};  // 32-bit byte offsets, and kPast behind them
   const int pieces = K / (kChunk * step), tiles = N / 16;
   const double megabytes = 1e-6 * N * K * (0.5 + 4.0 / group_size), first = group_size == 32 ? 96.0 : 80.0, further = group_size == 32 ? 4.0 : 9.0;
-  Plan best = {0, 0, cus, 0};
+  Plan best = {0, 0, cus, 0, false};
   double best_cost = 0.0;
   for (int slices = 1; slices <= kMostSlices; ++slices) {
     const int parts = kWaves * slices;
@@ -55,9 +59,9 @@ Plan make_plan(int K, int N, int group_size, int cus) {
   }
   if (best.slices > 1 && group_size == 64 && N % 128 == 0 && N >= 4096 && cus % (N / 128) == 0) {
     const double us = 1.83 + 0.0109 * best_cost + 0.058 * megabytes, streaming_us = 7.2 + (K % 512 == 0 ? 0.171 : 0.186) * megabytes;
-    if (us > streaming_us) return {0, 0, cus, 0};
+    if (us > streaming_us) return {0, 0, cus, 0, false};
   }
-  best.cus = cus;
+  best.padded = N <= 4096 && 3 * pieces * step < 2 * kWaves * best.slices * best.chunks;
   best.workspace = best.slices < 2 ? 0 : (size_t)64 * 1024 + (size_t)tiles * (best.slices - 1) * 1024;
   return best;
 }
@@ -78,12 +82,12 @@ const Plan& plan_for(int K, int N, int group_size) {
 }  // namespace resident
 
 bool qmm_resident_covers(const void* scales, const void* biases, size_t workspace_bytes, int K, int N, int group_size, int act_dtype,
-                         int sb_dtype) {
+                         int sb_dtype, bool narrow) {
   // (mixed types: the streaming kernel's; a lane's words of scales are four bytes)
   if (act_dtype != sb_dtype || (((uintptr_t)scales | (uintptr_t)biases) % 4) != 0) return false;
   if (K <= 1024 && N <= 4096) return false;  // as in make_plan, without looking the plan up
   const resident::Plan& plan = resident::plan_for(K, N, group_size);
-  return plan.chunks != 0 && workspace_bytes >= plan.workspace;
+  return plan.chunks != 0 && !(narrow && plan.padded) && workspace_bytes >= plan.workspace;
 }
 
 int qmm_resident_launch(const void* x, const void* w, const void* scales, const void* biases, void* y, void* workspace, int M, int K,
