@@ -40,11 +40,12 @@ _AUTOMATIC = (_native.QMM_KERNEL_AUTO, _native.QMM_KERNEL_FASTEST)  # no kernel 
 def _kernel_select() -> int:
     """``DFLASH_QMM_KERNEL`` in {auto, tile, stream}: which device kernel serves eligible
     calls (auto: the streaming kernel wherever it applies, the tile kernel elsewhere, so that single
-    calls have the bits of a ``QmmChain``).  Without it also the kernel that keeps x in registers, the fastest."""
+    calls have the bits of a ``QmmChain``).  Without it, or with another name in it, also the kernel that keeps x in
+    registers, which is faster."""
     chosen = _native.env(b"DFLASH_QMM_KERNEL")
     if chosen is None:
         return _native.QMM_KERNEL_FASTEST
-    return _KERNEL_CODE.get(os.fsdecode(chosen).strip().lower(), _native.QMM_KERNEL_AUTO)
+    return _KERNEL_CODE.get(os.fsdecode(chosen).strip().lower(), _native.QMM_KERNEL_FASTEST)
 
 
 def is_enabled() -> bool:

@@ -590,6 +590,18 @@ def test_members_whose_scales_are_learnt_leave_the_joint_product(monkeypatch):
             assert group._holds(m.mlp, x)
 
 
+@pytest.mark.parametrize("name,kernel", [(None, "FASTEST"), ("", "FASTEST"), ("streem", "FASTEST"), ("auto", "AUTO"), (" Tile ", "TILE"),
+                                         ("STREAM", "STREAM")])
+def test_a_kernel_that_does_not_exist_is_none_named(monkeypatch, name, kernel):
+    import dflash_mlx_amd._native as nat
+    from dflash_mlx_amd import verify_qmm as VQ
+
+    monkeypatch.delenv("DFLASH_QMM_KERNEL", raising=False)
+    if name is not None:
+        monkeypatch.setenv("DFLASH_QMM_KERNEL", name)
+    assert VQ._kernel_select() == getattr(nat, "QMM_KERNEL_" + kernel)
+
+
 @pytest.mark.parametrize("given", [0, 64 * 1024])
 def test_products_refuse_a_small_workspace_whichever_kernel_they_take(native_lib, given):
     """What a call has to bring is what the kernel with partial sums asks for, also where the call goes to one that has none.
