@@ -18,7 +18,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libdflash_mi355.so")
 HOST_PATH = os.path.join(_HERE, "_dflash_host.so")
 
-ABI_VERSION = 24
+ABI_VERSION = 25
 
 BF16, FP16, FP32 = 0, 1, 2
 QMM_MMA2BIG, QMM_MMA2BIG_PIPE = 0, 1
@@ -64,6 +64,7 @@ EXPORTED_SYMBOLS = (
     "dflash_qmm_rows",
     "dflash_qmm_m16_gather_workspace_bytes",
     "dflash_qmm_m16_gather",
+    "dflash_qmm_m16_gather_by",
     "dflash_tape_replay",
     "dflash_gdn_forward_tape",
     "dflash_gdn_forward_tape_norm",
@@ -142,6 +143,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.dflash_qmm_m16_gather.argtypes = (
         [c.c_void_p] * 7 + [c.c_size_t] + [c.c_int] * 7 + [c.c_void_p]
     )
+    lib.dflash_qmm_m16_gather_by.restype = c.c_int
+    lib.dflash_qmm_m16_gather_by.argtypes = [c.c_void_p] * 7 + [c.c_size_t] + [c.c_int] * 8 + [c.c_void_p]
     lib.dflash_gdn_forward_tape.restype = c.c_int
     lib.dflash_gdn_forward_tape.argtypes = [c.c_void_p] * 10 + [c.c_int] * 11 + [c.c_void_p]
     lib.dflash_gdn_forward_tape_norm.restype = c.c_int

@@ -242,14 +242,15 @@ PyObject* qmm_rows(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// gather(x, w, scales, biases, ids, group_size, streaming, workspaces): a row of x with the expert ids names, w [E, N, K/8].
+// gather(x, w, scales, biases, ids, group_size, kernel, workspaces): a row of x with the expert ids names, w [E, N, K/8].
 PyObject* gather(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (n != 8) Py_RETURN_NONE;
   const Tensor *x = device_tensor(a[0]), *w = device_tensor(a[1]), *s = device_tensor(a[2]), *b = device_tensor(a[3]),
                *ids = device_tensor(a[4]);
-  int group;
-  if (!x || !w || !s || !b || !ids || !integer(a[5], &group) || group < 1 || x->dim() < 1 || w->dim() != 3) Py_RETURN_NONE;
+  int group, kernel;
+  if (!x || !w || !s || !b || !ids || !integer(a[5], &group) || !integer(a[6], &kernel) || group < 1 || x->dim() < 1 || w->dim() != 3)
+    Py_RETURN_NONE;
   const int64_t K = x->size(-1), E = w->size(0), N = w->size(1);
   if (K < group || K >= (1 << 30) || E < 1 || E >= (1 << 30) || N < 1 || N >= (1 << 30)) Py_RETURN_NONE;
   const int64_t P = x->numel() / K;
@@ -262,14 +263,14 @@ PyObject* gather(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!t->is_contiguous() || t->device() != x->device()) Py_RETURN_NONE;
   void* stream = stream_of(*x);
   const size_t need =
-      a[6] == Py_True ? dflash_qmm_m16_gather_workspace_bytes((int)P, (int)K, (int)N, (int)E, group) : 0;
+      kernel != DFLASH_QMM_KERNEL_TILE ? dflash_qmm_m16_gather_workspace_bytes((int)P, (int)K, (int)N, (int)E, group) : 0;
   Tensor ws, y;
   if (need != 0 && !(ws = kept_workspace(a[7], by_index(*x, stream), need)).defined()) Py_RETURN_NONE;
   const int rc = released([&] {
     y = at::empty(rows_by(*x, N), x->options());
-    return dflash_qmm_m16_gather(at_of(*x), (const int32_t*)at_of(*ids), (const uint32_t*)at_of(*w), at_of(*s), at_of(*b),
-                                 y.mutable_data_ptr(), need ? ws.mutable_data_ptr() : nullptr, need ? ws.nbytes() : 0, (int)P,
-                                 (int)K, (int)N, (int)E, group, act, sb, stream);
+    return dflash_qmm_m16_gather_by(at_of(*x), (const int32_t*)at_of(*ids), (const uint32_t*)at_of(*w), at_of(*s), at_of(*b),
+                                    y.mutable_data_ptr(), need ? ws.mutable_data_ptr() : nullptr, need ? ws.nbytes() : 0, (int)P,
+                                    (int)K, (int)N, (int)E, group, act, sb, kernel, stream);
   });
   return rc != 0 ? fail(rc, "dflash_qmm_m16_gather") : THPVariable_Wrap(std::move(y));
   END_HANDLE_TH_ERRORS

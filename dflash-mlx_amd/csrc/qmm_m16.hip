@@ -741,7 +741,17 @@ extern "C" int dflash_qmm_m16_gather(const void* x, const int32_t* expert_ids, c
                                      void* workspace, size_t workspace_bytes, int P, int K, int N,
                                      int E, int group_size, int act_dtype, int sb_dtype,
                                      void* stream) {
+  return dflash_qmm_m16_gather_by(x, expert_ids, w_q, scales, biases, y, workspace, workspace_bytes, P, K, N, E, group_size, act_dtype,
+                                  sb_dtype, DFLASH_QMM_KERNEL_FASTEST, stream);
+}
+
+extern "C" int dflash_qmm_m16_gather_by(const void* x, const int32_t* expert_ids, const uint32_t* w_q, const void* scales,
+                                        const void* biases, void* y, void* workspace, size_t workspace_bytes, int P, int K, int N,
+                                        int E, int group_size, int act_dtype, int sb_dtype, int kernel, void* stream) {
   using namespace dflash;
+  DFLASH_REQUIRE(kernel == DFLASH_QMM_KERNEL_AUTO || kernel == DFLASH_QMM_KERNEL_TILE || kernel == DFLASH_QMM_KERNEL_STREAM ||
+                     kernel == DFLASH_QMM_KERNEL_FASTEST,
+                 DFLASH_ERR_ARG, "dflash_qmm_m16_gather: unknown kernel selector %d", kernel);
   DFLASH_REQUIRE(x && expert_ids && w_q && scales && biases && y, DFLASH_ERR_ARG,
                  "dflash_qmm_m16_gather: null operand");
   DFLASH_REQUIRE(act_dtype == DFLASH_BF16 || act_dtype == DFLASH_FP16, DFLASH_ERR_ARG,
@@ -761,14 +771,14 @@ extern "C" int dflash_qmm_m16_gather(const void* x, const int32_t* expert_ids, c
                  DFLASH_ERR_ARG, "dflash_qmm_m16_gather: x and w_q must be 16-byte aligned");
   if (P == 0) return DFLASH_OK;
   hipStream_t s = (hipStream_t)stream;
-  // With a workspace, shapes the streaming kernel covers go through it; everything else,
-  // and callers without a workspace, through the one-workgroup-per-(columns, expert) kernel.
+  // With a workspace, shapes the streaming kernel covers go through it or the kernel that keeps x in registers; everything
+  // else, and callers without a workspace, through the one-workgroup-per-(columns, expert) kernel.
   // (Calls of more than 256 rows have always been served whatever their workspace, and with scales of 2-byte alignment.)
   const bool streams = P <= 256 || (workspace_bytes >= qmm_stream_workspace_bytes(N, qmm_stream_grid()) &&
                                       (((uintptr_t)scales | (uintptr_t)biases) % 4) == 0);
-  if (workspace != nullptr && streams && qmm_stream_gather_eligible(P, K, N, E, group_size)) {
+  if (kernel != DFLASH_QMM_KERNEL_TILE && workspace != nullptr && streams && qmm_stream_gather_eligible(P, K, N, E, group_size)) {
     // (needs no workspace; what a call has to bring does not depend on that)
-    if (workspace_bytes >= qmm_stream_workspace_bytes(N, qmm_stream_grid()) &&
+    if (kernel == DFLASH_QMM_KERNEL_FASTEST && workspace_bytes >= qmm_stream_workspace_bytes(N, qmm_stream_grid()) &&
         qmm_resident_gather_covers(scales, biases, P, K, N, E, group_size, act_dtype, sb_dtype))
       return qmm_resident_gather_launch(x, expert_ids, w_q, scales, biases, y, P, K, N, E, act_dtype, s);
     return qmm_stream_gather_launch(x, expert_ids, w_q, scales, biases, y, workspace, workspace_bytes,

@@ -667,8 +667,8 @@ def gather_qmm(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: t
         raise NotImplementedError("only 4-bit codes are implemented")
     if not x.is_cuda:
         raise _native.NativeLibraryError("gather_qmm runs on the GPU only")
-    y = _native.host().gather(x, w, scales, biases, expert_ids, group_size, _kernel_select() != _native.QMM_KERNEL_TILE,
-                              _WORKSPACES)
+    kernel = _kernel_select()
+    y = _native.host().gather(x, w, scales, biases, expert_ids, group_size, kernel, _WORKSPACES)
     if y is not None:
         return y
     lib = _native.lib()
@@ -684,16 +684,16 @@ def gather_qmm(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: t
     _require_operands("gather_qmm", K, N, group_size, w_q, scales, biases, x2.device, lead=(E,))
     y = torch.empty((P, N), dtype=x2.dtype, device=x2.device)
     stream = _native.raw_stream(x2.device)
-    # DFLASH_QMM_KERNEL=tile keeps the streaming kernel out of the gathered form as well
-    need = 0 if _kernel_select() == _native.QMM_KERNEL_TILE else \
+    # DFLASH_QMM_KERNEL names the kernel of the gathered form as well
+    need = 0 if kernel == _native.QMM_KERNEL_TILE else \
         lib.dflash_qmm_m16_gather_workspace_bytes(P, K, N, E, group_size)
     ws_ptr, ws_bytes = None, 0
     if need:
         ws = _workspace(x2.device, stream, need)
         ws_ptr, ws_bytes = ws.data_ptr(), ws.numel() * ws.element_size()
-    rc = lib.dflash_qmm_m16_gather(x2.data_ptr(), ids.data_ptr(), w_q.data_ptr(), scales.data_ptr(),
-                                   biases.data_ptr(), y.data_ptr(), ws_ptr, ws_bytes, P, K, N, E,
-                                   group_size, _DTYPE_CODE[x2.dtype], _DTYPE_CODE[scales.dtype], stream)
+    rc = lib.dflash_qmm_m16_gather_by(x2.data_ptr(), ids.data_ptr(), w_q.data_ptr(), scales.data_ptr(),
+                                      biases.data_ptr(), y.data_ptr(), ws_ptr, ws_bytes, P, K, N, E,
+                                      group_size, _DTYPE_CODE[x2.dtype], _DTYPE_CODE[scales.dtype], kernel, stream)
     _native.check(rc, "dflash_qmm_m16_gather")
     return y.reshape(*x.shape[:-1], N)
 

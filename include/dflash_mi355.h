@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define DFLASH_ABI_VERSION 24
+#define DFLASH_ABI_VERSION 25
 
 enum {
   DFLASH_OK = 0,
@@ -314,11 +314,15 @@ int dflash_qmm_rows(const void* x, const uint32_t* w_q, const void* scales, cons
  *                           bytes, same rules as the workspace of dflash_qmm_m16 (zero-filled
  *                           once, reusable, shareable with it).  With a workspace, calls with
  *                           group_size 64, E <= 1024 and not too many rows and experts together
- *                           (2048 rows: 280 experts; the size is 0 for others) are served by
- *                           the streaming kernel: the weights of the experts that have rows
- *                           are streamed through LDS by persistent workgroups, as for the
- *                           dense form.  Without one, or for other shapes, one workgroup per
- *                           (32 columns, expert) reads its weights directly.
+ *                           (2048 rows: 280 experts; the size is 0 for others) stream the
+ *                           weights of the experts that have rows through LDS by persistent
+ *                           workgroups: K a multiple of 128 up to 5120 with activations and
+ *                           scales of one type by the kernel that keeps x in registers (a row's
+ *                           bits then do not depend on the rows beside it), others by the
+ *                           streaming kernel (they do, within one rounding of the output type:
+ *                           K is cut by what the whole call has to do).  Without one, or for
+ *                           other shapes, one workgroup per (32 columns, expert) reads its
+ *                           weights directly.
  * Requirements: P <= 2048, group_size in {32,64,128}, N % 16 == 0, K % group_size == 0.
  * Rows whose expert id is outside [0, E) give zeros.  Deterministic.
  */
@@ -328,6 +332,12 @@ int dflash_qmm_m16_gather(const void* x, const int32_t* expert_ids, const uint32
                           const void* scales, const void* biases, void* y, void* workspace,
                           size_t workspace_bytes, int P, int K, int N, int E, int group_size,
                           int act_dtype, int sb_dtype, void* stream);
+/* The same with the kernel named: DFLASH_QMM_KERNEL_FASTEST (what dflash_qmm_m16_gather takes), _AUTO and _STREAM (the streaming
+ * kernel where that has the shape) or _TILE (the kernel without a workspace). */
+int dflash_qmm_m16_gather_by(const void* x, const int32_t* expert_ids, const uint32_t* w_q,
+                             const void* scales, const void* biases, void* y, void* workspace,
+                             size_t workspace_bytes, int P, int K, int N, int E, int group_size,
+                             int act_dtype, int sb_dtype, int kernel, void* stream);
 
 /*
  * GatedDeltaNet tape replay: for every slot s and value head hv apply the first

@@ -14,11 +14,15 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-@pytest.fixture(autouse=True, params=["auto", "tile"])
+@pytest.fixture(autouse=True, params=["auto", "tile", "unset"])
 def kernel_mode(request, monkeypatch):
-    """Every test runs once with the streaming kernel where it applies (auto: group 64,
-    K % 512 == 0, at most 256 rows) and once with the per-(columns, expert) kernel forced."""
-    monkeypatch.setenv("DFLASH_QMM_KERNEL", request.param)
+    """Every test runs once with the streaming kernel where it applies (auto: group 64, K a multiple
+    of 64), once with the per-(columns, expert) kernel forced and once with no kernel named: the one
+    that keeps x in registers where that applies (K a multiple of 128 up to 5120, one type)."""
+    if request.param == "unset":
+        monkeypatch.delenv("DFLASH_QMM_KERNEL", raising=False)
+    else:
+        monkeypatch.setenv("DFLASH_QMM_KERNEL", request.param)
     return request.param
 
 
@@ -141,12 +145,13 @@ def test_rows_with_invalid_expert_ids_give_zeros(native_lib, kernel_mode):
     d = case.to(DEV)
     y = torch.full((P, N), 7.0, dtype=torch.bfloat16, device=DEV)
     need = 0 if kernel_mode == "tile" else L.dflash_qmm_m16_gather_workspace_bytes(P, K, N, E, 64)
-    assert (need > 0) == (kernel_mode == "auto")
+    assert (need > 0) == (kernel_mode != "tile")
     ws = torch.zeros(max(need, 16), dtype=torch.uint8, device=DEV)
     for _ in range(2):  # the workspace is handed back reusable
-        rc = L.dflash_qmm_m16_gather(d.x.data_ptr(), d.expert_ids.data_ptr(), d.w.data_ptr(),
-                                     d.scales.data_ptr(), d.biases.data_ptr(), y.data_ptr(),
-                                     ws.data_ptr() if need else None, need, P, K, N, E, 64, 0, 0, None)
+        rc = L.dflash_qmm_m16_gather_by(d.x.data_ptr(), d.expert_ids.data_ptr(), d.w.data_ptr(),
+                                        d.scales.data_ptr(), d.biases.data_ptr(), y.data_ptr(),
+                                        ws.data_ptr() if need else None, need, P, K, N, E, 64, 0, 0,
+                                        nat.QMM_KERNEL_AUTO if kernel_mode == "auto" else nat.QMM_KERNEL_FASTEST, None)
         assert rc == 0, L.dflash_last_error()
         torch.cuda.synchronize()
     bad = [3, 10, 23]
@@ -176,7 +181,7 @@ def test_argument_checks(native_lib):
 @pytest.mark.parametrize("P,E,K,N", [(257, 8, 512, 96), (768, 256, 512, 32), (769, 64, 1024, 144), (1536, 1, 512, 128), (1537, 5, 1536, 160),
                                      (2048, 3, 640, 272), (2048, 256, 512, 16), (2048, 1000, 512, 16)])
 def test_more_rows_than_a_workgroup_has_threads(native_lib, P, E, K, N):
-    """Up to 2048 rows in one launch of the streaming kernel: rows of a thread's second and third round, experts with many entries and
+    """Up to 2048 rows in one launch of the kernels that stream: rows of a thread's second and third round, experts with many entries and
     with none, ids that belong to no expert, tables that just fit (and, the last case, that do not: the other kernel)."""
     from dflash_mlx_amd.quantized import dequantize
     from test_gpu_qmm_any_k import _check
@@ -218,3 +223,67 @@ def test_many_rows_with_a_workspace_that_is_too_small(native_lib):
                                                 torch.cuda.current_stream().cuda_stream) == 0
         ys.append(y)
     assert torch.equal(ys[0], ys[1]) and torch.equal(ys[0], ys[2])
+
+
+BF, HF = torch.bfloat16, torch.float16
+
+
+def _experts(K, N, E, act, sb, seed):
+    gen = torch.Generator("cuda").manual_seed(seed)
+    w = torch.randint(-2 ** 31, 2 ** 31, (E, N, K // 8), generator=gen, device="cuda", dtype=torch.int32)
+    s = (torch.rand((E, N, K // 64), generator=gen, device="cuda") * 0.02 + 1e-4).to(sb)
+    return gen, w, s, (s.float() * -8).to(sb)
+
+
+@pytest.mark.parametrize("K,N,rows", [
+    (5632, 144, (20, 0, 5, 1)),       # wider than the kernel with x in registers takes, K a multiple of 512; 17 rows and more of an expert
+    (6144, 2064, (37, 1, 16, 3)),     # a multiple of 1024
+    (5248, 272, (3, 0, 18, 2)),       # a multiple of 128 only
+    (704, 48, (9, 33)), (1088, 528, (1, 16, 17, 0, 2)), (6208, 32, (40,)),  # of 64 only
+    (1024, 272, (2, 40, 0, 7)), (640, 1040, (18, 1)), (2560, 96, (5, 5, 5))])
+@pytest.mark.parametrize("act,sb", [(BF, BF), (HF, HF), (BF, HF), (HF, BF)])
+def test_shapes_and_types_that_only_the_streaming_kernel_has(native_lib, K, N, rows, act, sb):
+    """What the kernel that keeps x in registers leaves to the streaming kernel: wide matrices, K that are no multiple of 128, scales of
+    another type; ids that belong to no expert, ranges of workgroups that cut row blocks."""
+    from dflash_mlx_amd.quantized import dequantize
+    from test_gpu_qmm_any_k import _check
+
+    E = len(rows)
+    gen, w, s, b = _experts(K, N, E, act, sb, K + N)
+    ids = torch.cat([torch.full((n,), e, dtype=torch.int32) for e, n in enumerate(rows)] + [torch.tensor([-1, E], dtype=torch.int32)])
+    ids = ids[torch.randperm(ids.numel(), generator=torch.Generator().manual_seed(K))].cuda()
+    x = torch.randn((ids.numel(), K), generator=gen, device="cuda").to(act)
+    y = gather_qmm(x, w, s, b, ids)
+    assert y.dtype == act and (y[(ids < 0) | (ids >= E)] == 0).all()
+    for e in range(E):
+        mine = ids == e
+        if mine.any():
+            _check(y[mine], x[mine], dequantize(w[e], s[e], b[e], 64, 4, torch.float64), K, act)
+    assert torch.equal(y, gather_qmm(x, w, s, b, ids))
+
+
+def test_the_kernel_named_is_the_kernel_taken(native_lib, monkeypatch):
+    """Three kernels for a gathered call, by name and by selector: the same bits either way, and not all of them those of another."""
+    K, N, E, P = 2048, 1024, 8, 40
+    gen, w, s, b = _experts(K, N, E, BF, BF, 3)
+    x = torch.randn((P, K), generator=gen, device="cuda").to(BF)
+    ids = torch.randint(0, E, (P,), generator=gen, device="cuda", dtype=torch.int32)
+    ws = torch.zeros(native_lib.dflash_qmm_m16_gather_workspace_bytes(P, K, N, E, 64), dtype=torch.uint8, device="cuda")
+    found = {}
+    for name, kernel in (("auto", nat.QMM_KERNEL_AUTO), ("stream", nat.QMM_KERNEL_STREAM), ("tile", nat.QMM_KERNEL_TILE),
+                         (None, nat.QMM_KERNEL_FASTEST)):
+        if name is None:
+            monkeypatch.delenv("DFLASH_QMM_KERNEL", raising=False)
+        else:
+            monkeypatch.setenv("DFLASH_QMM_KERNEL", name)
+        y = torch.empty((P, N), dtype=BF, device="cuda")
+        assert native_lib.dflash_qmm_m16_gather_by(x.data_ptr(), ids.data_ptr(), w.data_ptr(), s.data_ptr(), b.data_ptr(), y.data_ptr(),
+                                                   ws.data_ptr(), ws.numel(), P, K, N, E, 64, 0, 0, kernel,
+                                                   torch.cuda.current_stream().cuda_stream) == 0
+        found[name] = gather_qmm(x, w, s, b, ids)
+        assert torch.equal(found[name], y)
+    assert torch.equal(found["auto"], found["stream"])
+    for one, other in (("auto", "tile"), ("auto", None), ("tile", None)):
+        assert not torch.equal(found[one], found[other]), (one, other)
+    assert native_lib.dflash_qmm_m16_gather_by(x.data_ptr(), ids.data_ptr(), w.data_ptr(), s.data_ptr(), b.data_ptr(), y.data_ptr(),
+                                               ws.data_ptr(), ws.numel(), P, K, N, E, 64, 0, 0, 9, None) == -1
