@@ -38,7 +38,8 @@ KERNELS = (
     ("qmm_resident_rows_fp16.hip", "_ZN6dflash8resident19qmm_resident_kernel", 42, 20),
 )
 # source, number of counter bumps (arrival counters; the chained kernel's per-problem and exit counters too)
-ARRIVALS = (("qmm_m16.hip", 24), ("qmm_m16_stream.hip", 0), ("qmm_m16_chain.hip", 64))
+ARRIVALS = (("qmm_m16.hip", 24), ("qmm_m16_stream.hip", 0), ("qmm_m16_chain.hip", 64), ("qmm_resident_bf16.hip", 0),
+            ("qmm_resident_fp16.hip", 0), ("qmm_resident_rows_bf16.hip", 42), ("qmm_resident_rows_fp16.hip", 42))
 
 
 def _regs(text: str) -> set:
