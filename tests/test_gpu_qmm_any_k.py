@@ -1,6 +1,7 @@
 """Up to 16 rows through the streaming kernel's variants for every group size and K that is a multiple of 64
-only, against the product of the same operands in fp64: last chunks and last stages that are cut
-short in every way, ragged row blocks, one to sixteen rows, both activation types, gathered experts."""
+only, and through what is taken where no kernel is named, against the product of the same operands in fp64: last
+chunks and last stages that are cut short in every way, ragged row blocks, one to sixteen rows, both activation types,
+gathered experts."""
 import pytest
 import torch
 
@@ -10,6 +11,15 @@ from dflash_mlx_amd.workloads import make_qmm_case
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
+# the streaming kernel, and what calls take where no kernel is named (the one that keeps x in registers, where that has the shape)
+each_kernel = pytest.mark.parametrize("kernel", ["auto", None])
+
+
+def _choose(monkeypatch, kernel):
+    if kernel is None:
+        monkeypatch.delenv("DFLASH_QMM_KERNEL", raising=False)
+    else:
+        monkeypatch.setenv("DFLASH_QMM_KERNEL", kernel)
 
 
 def _check(y, x, dense, K, dtype):
@@ -23,15 +33,16 @@ def _check(y, x, dense, K, dtype):
     assert (y.double() - exact).norm() <= eps * exact.norm()
 
 
+@each_kernel
 @pytest.mark.parametrize("K,N,group,dtype", [
     (512, 16, 32, torch.bfloat16), (576, 48, 32, torch.bfloat16), (640, 128, 64, torch.bfloat16), (768, 144, 64, torch.float16),
     (832, 272, 32, torch.float16), (896, 1040, 64, torch.bfloat16), (1024, 512, 32, torch.bfloat16),
     (1024, 512, 128, torch.bfloat16), (1152, 2064, 64, torch.bfloat16), (1280, 112, 128, torch.float16),
     (2176, 4096, 64, torch.bfloat16), (2816, 528, 128, torch.bfloat16), (4096, 6144, 32, torch.bfloat16),
     (5376, 144, 64, torch.bfloat16), (12288, 4096, 32, torch.bfloat16), (4352, 5120, 128, torch.bfloat16)])
-def test_every_group_size_and_k(native_lib, monkeypatch, K, N, group, dtype):
+def test_every_group_size_and_k(native_lib, monkeypatch, K, N, group, dtype, kernel):
     monkeypatch.setenv("DFLASH_VERIFY_QMM", "1")
-    monkeypatch.delenv("DFLASH_QMM_KERNEL", raising=False)
+    _choose(monkeypatch, kernel)
     c = make_qmm_case(K, N, 300 + K, group_size=group, dtype=dtype).to(DEV)
     dense = dequantize(c.w, c.scales, c.biases, group, 4, dtype=torch.float64)
     y = VQ._launch(c.x, c.w, c.scales, c.biases, K, N, group, "mma2big", 1)
@@ -44,8 +55,10 @@ def test_every_group_size_and_k(native_lib, monkeypatch, K, N, group, dtype):
     assert int((ws != 0).sum()) == 0
 
 
+@each_kernel
 @pytest.mark.parametrize("K,N,E,P", [(640, 144, 4, 37), (768, 256, 3, 16), (896, 2048, 8, 128), (1152, 272, 2, 250)])
-def test_gathered_experts_of_any_k(native_lib, K, N, E, P):
+def test_gathered_experts_of_any_k(native_lib, monkeypatch, K, N, E, P, kernel):
+    _choose(monkeypatch, kernel)
     cases = [make_qmm_case(K, N, 500 + e).to(DEV) for e in range(E)]
     w, s, b = (torch.stack([getattr(c, n) for c in cases]) for n in ("w", "scales", "biases"))
     gen = torch.Generator().manual_seed(K)
@@ -60,15 +73,16 @@ def test_gathered_experts_of_any_k(native_lib, K, N, E, P):
     assert torch.equal(y, VQ.gather_qmm(x, w, s, b, ids))
 
 
+@each_kernel
 @pytest.mark.parametrize("K,N,group,dtype", [
     (512, 32, 64, torch.bfloat16), (512, 16, 32, torch.bfloat16), (576, 48, 32, torch.float16), (896, 272, 64, torch.bfloat16),
     (1024, 1040, 64, torch.bfloat16), (1280, 112, 128, torch.float16), (1536, 4128, 64, torch.float16),
     (4096, 24576, 32, torch.bfloat16), (5120, 34816, 64, torch.bfloat16)])
-def test_gated_activation_of_few_rows(native_lib, monkeypatch, K, N, group, dtype):
+def test_gated_activation_of_few_rows(native_lib, monkeypatch, K, N, group, dtype, kernel):
     """The silu-mul form (8 gate rows and their 8 up rows to a tile) against the joint product of the same matrix and the array
     operators, and both against float64."""
     monkeypatch.setenv("DFLASH_VERIFY_QMM", "1")
-    monkeypatch.delenv("DFLASH_QMM_KERNEL", raising=False)
+    _choose(monkeypatch, kernel)
     c = make_qmm_case(K, N, 700 + K, group_size=group, dtype=dtype).to(DEV)
     x = (c.x / (K ** 0.5 * c.scales.float().abs().mean() * 4)).to(dtype)  # gates of a few units
     assert VQ.small_m_silu_mul(x[:, :K - 64], c.w, c.scales, c.biases, group_size=group) is None
@@ -98,7 +112,8 @@ def test_gated_activation_of_few_rows(native_lib, monkeypatch, K, N, group, dtyp
     assert int((ws != 0).sum()) == 0
 
 
-def test_few_rows_take_the_joint_launch(native_lib, monkeypatch):
+@each_kernel
+def test_few_rows_take_the_joint_launch(native_lib, monkeypatch, kernel):
     """One token and a short block through joined projections: the rows a block of 16 gets, also for members
     behind a wrapper that pads, and the members' own launches with DFLASH_STOCK_KERNEL=0 or once a member has left."""
     from dflash_mlx_amd import verify_linear as VL
@@ -106,7 +121,7 @@ def test_few_rows_take_the_joint_launch(native_lib, monkeypatch):
     from dflash_mlx_amd.quantized import QuantizedLinear
 
     monkeypatch.setenv("DFLASH_VERIFY_QMM", "1")
-    monkeypatch.delenv("DFLASH_QMM_KERNEL", raising=False)
+    _choose(monkeypatch, kernel)
     parent = torch.nn.Module()
     widths = dict(in_proj_qkv=256, in_proj_z=128, in_proj_b=48, in_proj_a=48)
     for i, (name, n) in enumerate(widths.items()):
@@ -130,10 +145,11 @@ def test_few_rows_take_the_joint_launch(native_lib, monkeypatch):
     assert not group.serves_few(parent, x[:, :1])
 
 
+@each_kernel
 @pytest.mark.parametrize("rows", [1, 3, 15])
-def test_few_rows_that_start_anywhere(native_lib, monkeypatch, rows):
+def test_few_rows_that_start_anywhere(native_lib, monkeypatch, rows, kernel):
     """The kernel loads x in pieces of 16 bytes; fewer rows than a block may start on any element all the same."""
-    monkeypatch.delenv("DFLASH_QMM_KERNEL", raising=False)
+    _choose(monkeypatch, kernel)
     for group, K, N in ((64, 1024, 256), (32, 576, 48), (128, 128, 16)):
         c = make_qmm_case(K, N, 960 + rows, group_size=group, M=rows).to(DEV)
         want = stock_matmul(c.x, c.w, c.scales, c.biases, group_size=group)

@@ -112,6 +112,29 @@ def test_a_slice_that_gives_up_says_so_and_the_launch_ends(verify_env, native_li
     assert torch.equal(VQ.verify_matmul(c.x, c.w, c.scales, c.biases), good) and _clean(native_lib)
 
 
+def test_sliced_launches_of_two_streams_beside_each_other(verify_env, native_lib):
+    """The last slice of a product waits inside the launch for the others.  Two streams, each with such products of its own in flight:
+    a workgroup waits for workgroups before it only, which wait for nobody, so neither stream can keep the other's from finishing."""
+    cases = [make_qmm_case(17408, 5120, 51).to(DEV), make_qmm_case(14336, 4096, 52).to(DEV)]  # three slices, four slices
+    alone = [VQ.verify_matmul(c.x, c.w, c.scales, c.biases) for c in cases]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    for s in streams:
+        s.wait_stream(torch.cuda.current_stream())
+    got = [[], []]
+    for i in range(20):
+        for k, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                c = cases[(i + k) % 2]
+                got[k].append(VQ.verify_matmul(c.x, c.w, c.scales, c.biases))
+    torch.cuda.synchronize()
+    VQ.raise_on_device_errors(torch.device(DEV))
+    for k in range(2):
+        for i, y in enumerate(got[k]):
+            assert torch.equal(y, alone[(i + k) % 2]), (k, i)
+    for s in streams:
+        assert int((VQ._workspace(torch.device(DEV), s.cuda_stream, 1) != 0).sum()) == 0
+
+
 # two to five tiles of 16 rows, full and not; one slice and more, whole and uneven chunks; fewer tiles than workgroups, one more, an odd number each
 ROWS = [(17, 2048, 16, 64), (32, 4096, 4096, 64), (33, 2304, 4112, 64), (31, 5120, 12352, 64), (40, 3072, 3072, 32), (48, 4096, 6144, 64), (47, 6144, 2048, 128),
         (49, 3328, 4608, 64), (64, 4096, 6144, 32), (65, 4096, 6144, 64), (77, 8192, 5120, 64), (79, 3328, 4624, 64), (80, 12288, 4096, 64), (80, 4096, 6144, 128),
