@@ -34,7 +34,10 @@ struct Plan {
 //
 // Where N / 128 divides the compute units, the streaming kernel (groups of 64) has equal parts without a remainder and is at its best: there the call is
 // its own if a model of either says so (2.5 % rms over 71 such shapes).  us there and here: 9216 x 16384 21.2 / 22.3, 12800 x 16384 27.5 / 29.4,
-// 6400 x 32768 27.4 / 28.9, 17408 x 8192 21.4 / 22.5; 16384 x 8192 19.7 / 18.3.
+// 6400 x 32768 27.4 / 28.9, 17408 x 8192 21.4 / 22.5; 16384 x 8192 19.7 / 18.3.  Waves that are a third empty and more also lose to it on wide matrices
+// whose N / 128 is a multiple of the compute units (1280 x 65536 13.5 / 14.6, 1024 x 65536 in groups of 32 13.2 / 15.6, 2304 x 32768 in groups of 128
+// 12.0 / 12.9), half empty ones on any but those between 32768 and 65536, where its parts are uneven (1024 x 28672 7.3 / 8.4, 1024 x 151936 25.7 / 28.8;
+// 1024 x 40960 10.8 / 10.5).
 Plan make_plan(int K, int N, int group_size, int cus) {
   const int step = group_size == 128 ? 2 : 1, most = most_chunks(group_size, 1);
   if ((group_size != 32 && group_size != 64 && group_size != 128) || K % (kChunk * step) != 0 || N % 16 != 0 || N < 16) return {0, 0, cus, 0, false};
@@ -61,7 +64,10 @@ Plan make_plan(int K, int N, int group_size, int cus) {
     const double us = 1.83 + 0.0109 * best_cost + 0.058 * megabytes, streaming_us = 7.2 + (K % 512 == 0 ? 0.171 : 0.186) * megabytes;
     if (us > streaming_us) return {0, 0, cus, 0, false};
   }
-  best.padded = N <= 4096 && 3 * pieces * step < 2 * kWaves * best.slices * best.chunks;
+  const bool padded = 3 * pieces * step < 2 * kWaves * best.slices * best.chunks;
+  if (padded && best.slices == 1 && N > 20480 &&
+      ((N % 128 == 0 && N / 128 % cus == 0) || (K <= 1024 && group_size == 64 && (N <= 32768 || N >= 65536)))) return {0, 0, cus, 0, false};
+  best.padded = padded && N <= 4096;
   best.workspace = best.slices < 2 ? 0 : (size_t)64 * 1024 + (size_t)tiles * (best.slices - 1) * 1024;
   return best;
 }

@@ -18,11 +18,11 @@ DEV = "cuda:0"
 BF, HF = torch.bfloat16, torch.float16
 # chunks of 128 k over 8 waves: 1, 1 and 2, 2, .., 6 each, then slices; one tile, a tile per compute unit and one more, nine tiles of some (two
 # meetings and a last odd tile); three slices of two chunks, four with one round less than three have, a matrix left to the streaming kernel; narrow
-# ones whose waves would be half empty
+# and wide ones whose waves would be half empty
 SHAPES = [(1024, 4112, 64), (1152, 16, 64), (1920, 48, 32), (2048, 4112, 128), (2176, 32, 64), (2304, 36880, 64), (3072, 4096, 64), (3584, 80, 128),
           (4096, 4096, 64), (4096, 1040, 32), (4736, 2320, 64), (5120, 4128, 32), (5120, 12352, 64), (5376, 64, 128), (6144, 512, 64),
           (6144, 8224, 64), (6272, 112, 64), (8192, 4112, 64), (10240, 48, 32), (12288, 4096, 128), (12288, 1024, 64), (17408, 1040, 64),
-          (1280, 2048, 64), (2560, 1040, 128), (17408, 5120, 64), (24576, 32, 64), (24704, 32, 64), (6144, 4096, 128), (14336, 4096, 64), (12800, 16384, 64)]
+          (1280, 2048, 64), (2560, 1040, 128), (1024, 24576, 64), (1280, 32768, 32), (17408, 5120, 64), (24576, 32, 64), (24704, 32, 64), (6144, 4096, 128), (14336, 4096, 64), (12800, 16384, 64)]
 
 
 def _clean(native_lib):
