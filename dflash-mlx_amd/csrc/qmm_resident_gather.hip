@@ -276,10 +276,15 @@ int chunks_of_wave(int K, int kw) {
 }  // namespace
 }  // namespace resident
 
-// expert_ids on the device; P rows, E experts within the tables' limits (the caller has asked the streaming kernel's rule)
+// expert_ids on the device; P rows, E experts within the tables' limits (the caller has asked the streaming kernel's rule).  Beyond K = 4096 every wave
+// has four and a half to five chunks of each tile, and where experts have four rows and more the streaming kernel is as fast or faster (us there and here:
+// 32 rows on 8 experts of 5120 x 4096 20.6 / 22.8, 128 rows 31.9 / 34.3; 128 rows on 8 of 5120 x 2048 20.2 / 23.8, on 16 of 4608 x 2048 20.4 / 23.6, 256 on 32
+// of 4608 x 1024 20.8 / 23.9; with fewer 8 rows on 8 of 5120 x 4096 18.9 / 18.7, 2 rows 11.3 / 9.4, 32 on 256 of 4608 x 1024 as fast).  Up to there it is
+// slower only where 128 - 256 rows meet on 1000 - 1600 tiles (128 on 8 of 2560 x 2048 14.0 / 15.8, of 3584 x 2048 16.4 / 18.0), else 5 - 30 % faster.
 bool qmm_resident_gather_covers(const void* scales, const void* biases, int P, int K, int N, int E, int group_size, int act_dtype, int sb_dtype) {
   using namespace resident;
   if (group_size != 64 || act_dtype != sb_dtype || K % kChunk != 0 || N % 16 != 0 || (((uintptr_t)scales | (uintptr_t)biases) % 4) != 0) return false;
+  if (K > 4096 && N > 512 && P >= 4 * E) return false;
   const int kw = waves_of_tile(K);
   if (kw == 0 || (long long)N * K / 2 >= (1ll << 31) || (long long)P * K * 2 >= (1ll << 31)) return false;
   const int most = stream::most_entries(P, E);

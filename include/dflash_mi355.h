@@ -318,11 +318,11 @@ int dflash_qmm_rows(const void* x, const uint32_t* w_q, const void* scales, cons
  *                           weights of the experts that have rows through LDS by persistent
  *                           workgroups: K a multiple of 128 up to 5120 with activations and
  *                           scales of one type by the kernel that keeps x in registers (a row's
- *                           bits then do not depend on the rows beside it), others by the
- *                           streaming kernel (they do, within one rounding of the output type:
- *                           K is cut by what the whole call has to do).  Without one, or for
- *                           other shapes, one workgroup per (32 columns, expert) reads its
- *                           weights directly.
+ *                           bits then do not depend on the rows beside it), others, and K from
+ *                           4097 on where P >= 4 E and N > 512, by the streaming kernel (they
+ *                           do, within one rounding of the output type: K is cut by what the
+ *                           whole call has to do).  Without one, or for other shapes, one
+ *                           workgroup per (32 columns, expert) reads its weights directly.
  * Requirements: P <= 2048, group_size in {32,64,128}, N % 16 == 0, K % group_size == 0.
  * Rows whose expert id is outside [0, E) give zeros.  Deterministic.
  */

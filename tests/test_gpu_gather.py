@@ -239,6 +239,7 @@ def _experts(K, N, E, act, sb, seed):
     (5632, 144, (20, 0, 5, 1)),       # wider than the kernel with x in registers takes, K a multiple of 512; 17 rows and more of an expert
     (6144, 2064, (37, 1, 16, 3)),     # a multiple of 1024
     (5248, 272, (3, 0, 18, 2)),       # a multiple of 128 only
+    (5120, 528, (17, 1)), (4608, 1040, (16, 16, 3)),  # many rows of a wide expert
     (704, 48, (9, 33)), (1088, 528, (1, 16, 17, 0, 2)), (6208, 32, (40,)),  # of 64 only
     (1024, 272, (2, 40, 0, 7)), (640, 1040, (18, 1)), (2560, 96, (5, 5, 5))])
 @pytest.mark.parametrize("act,sb", [(BF, BF), (HF, HF), (BF, HF), (HF, BF)])
