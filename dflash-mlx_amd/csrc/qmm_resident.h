@@ -6,17 +6,18 @@
 //  * a wave owns NCH chunks of 128 k, of all rows.  Its part of x stays in registers, read once (a compute unit has 512 KiB of them,
 //    x of 16 rows and K = 6144 is 192), and its part of 16 rows of W at a time comes through a ring of LDS that no other wave sees:
 //    direct loads, two tiles ahead, no registers and no barriers for them;
-//  * loads follow the rows: a load instruction covers runs of NCH * 64 bytes, whole 128-byte lines.  In matrix-instruction order (16 rows, 64
-//    bytes each) the same loads with nothing else took 24.6 us for 5120 x 34816, in this order 19.6; for x (256-byte runs, turned through
-//    LDS) 2.2 us of a launch.  LDS takes the pieces in an order without bank conflicts; a row's scales are fetched four bytes a lane;
+//  * loads follow the rows: a load instruction covers runs of NCH * 64 bytes, whole 128-byte lines where NCH and the wave's first chunk are even;
+//    else the ends of a run share their lines with the waves beside it.  In matrix-instruction order (16 rows, 64 bytes each) the same loads with
+//    nothing else took 24.6 us for 5120 x 34816, in this order 17 - 20; for x (256-byte runs, turned through LDS) 2.2 us of a launch.  LDS takes the pieces in an order without bank conflicts; a row's scales are fetched four bytes a lane;
 //  * scales and biases enter in fp32 as before: s * sum x q per group on the vector pipe, the sums of x times the biases of four groups in one
 //    16 x 16 x 4 fp32 matrix instruction;
 //  * the eight waves' sums meet in LDS, in their order.  Where a wave's chunks would be more than NCH, the K range is cut into slices of
 //    whole workgroups: all but the last store their tiles (their own arrival flags, see nonzero_words()), the last adds them in order.
-//    It has the highest index of those it waits for, so they are running or done before it starts, and they wait for nobody.
-// us, streaming kernel -> here (16 rows): 4096 x 4096 8.3 -> 5.9, 4096 x 6144 9.6 -> 7.3, 5120 x 5120 10.1 -> 9.1, 5120 x 7168 11.5 -> 9.5,
-// 5120 x 17408 18.6 -> 16.3, 5120 x 34816 with the activation 30 -> 26, 4096 x 49152 30.5 -> 23.9 (4.75 TB/s).  Eight waves: with
-// twelve or sixteen (fewer chunks each) 5 - 13 % slower; three tiles ahead 7 % slower; arithmetic alone takes 20 of the 26 us, loads alone 22.
+//    Those it waits for wait for nobody and have lower indexes, but workgroups start in order on each XCD only, and another stream's kernel can hold one
+//    of them back there: the wait ends once they have had their turn, and spin_limit bounds it.
+// us, streaming kernel -> here (16 rows, weights from memory): 4096 x 4096 8.0 -> 6.1, 4096 x 7168 9.5 -> 7.7, 5120 x 5120 9.5 -> 7.4, 5120 x 7168 10.8 -> 9.4,
+// 12288 x 4096 12.3 -> 10.6, 17408 x 5120 16.3 -> 16.0, 5120 x 34816 with the activation 26.7 -> 24.7, 4096 x 49152 27.0 -> 23.3 (4.85 TB/s).  Eight waves: with
+// twelve or sixteen (fewer chunks each) 5 - 13 % slower; three tiles ahead 7 % slower; arithmetic alone takes 20 of the 25 us.
 #pragma once
 #include <utility>
 

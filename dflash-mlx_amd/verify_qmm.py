@@ -13,8 +13,8 @@ and shape dispatch, with the device work done by the gfx950 kernel behind
 * ``DFLASH_VERIFY_VARIANT`` in {auto, mma2big, mma2big_pipe} and
   ``DFLASH_VERIFY_QMM_KPARTS`` select the variant (:15-22, 292-297).
 * ``DFLASH_QMM_KERNEL`` in {auto, tile, stream} picks the device kernel (no counterpart
-  in the reference; not set: the kernel that keeps x in registers, csrc/qmm_resident.h, wherever it applies, else as auto,
-  which takes matrices of few weights through a kernel of their own, csrc/qmm_narrow.hip, and the rest through the
+  in the reference; not set: the kernel that keeps x in registers, csrc/qmm_resident.h, for the sizes where it takes less
+  time, else as auto, which takes matrices of few weights through a kernel of their own, csrc/qmm_narrow.hip, and the rest through the
   streaming kernel, whose every-K form takes all group sizes and K a multiple of 64, wherever it applies).
 * An eligible call needs device tensors and the built HIP library; there is no
   software fallback for it.
@@ -99,8 +99,8 @@ def _workspace(device: torch.device, stream: int, nbytes: int) -> torch.Tensor:
 def raise_on_device_errors(device: Optional[torch.device] = None) -> None:
     """Call where the host synchronises with the device anyway (the read-back of the acceptance
     length in a speculative cycle): a bounded wait inside a qmm kernel that gave up - a chained
-    projection waiting for its input, the streaming kernel's adding workgroup waiting for partial
-    tiles - leaves a word in the workspace and wrong outputs behind, and nothing else tells the
+    projection waiting for its input, the streaming kernel's adding workgroup or the last slice of a
+    product of few rows waiting for partial tiles - leaves a word in the workspace and wrong outputs behind, and nothing else tells the
     caller.  Reads that word of every workspace of ``device`` (all devices if None; each read waits
     for the device); on a non-zero word the workspace is zero-filled again, as its contract asks,
     and ``NativeLibraryError`` raised."""
@@ -112,7 +112,7 @@ def raise_on_device_errors(device: Optional[torch.device] = None) -> None:
             continue
         ws.zero_()
         if word & 0x80000000:
-            what = f"the streaming kernel gave up waiting for the partial tiles of row block {word & 0x3FFFFFFF}"
+            what = f"a product of few rows gave up waiting for the partial tiles of row block {word & 0x3FFFFFFF}"
         else:
             what = f"projection {word - 1} of a chained launch gave up waiting for its input"
         raise _native.NativeLibraryError(
@@ -539,8 +539,8 @@ def small_m_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biase
 
 def small_m_silu_mul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
                      *, group_size: int = 64, bits: int = 4) -> "torch.Tensor | None":
-    """``silu(x @ gate.T) * (x @ up.T)`` for at most 16 rows of device activations in one launch of the streaming
-    kernel; ``w`` holds the gate rows of an MLP followed by its up rows.  None for what that kernel does not
+    """``silu(x @ gate.T) * (x @ up.T)`` for at most 16 rows of device activations in one launch; ``w`` holds the
+    gate rows of an MLP followed by its up rows.  None for what the streaming kernel does not
     cover or ``small_m_matmul`` leaves to the array operators.  No counterpart in the reference."""
     kernel = _kernel_select()
     if (bits == 4 and x.is_cuda and kernel in _AUTOMATIC and _native.plain(x, w, scales, biases)

@@ -48,8 +48,8 @@ enum { DFLASH_QMM_MMA2BIG = 0, DFLASH_QMM_MMA2BIG_PIPE = 1 };
  * group_size 64 and K % 512 == 0, and decides the K split itself (variant and k_parts
  * then only name the caller's dispatch decision).  AUTO: STREAM where it applies, and its
  * form for every group size and K a multiple of 64 where scales and biases start on 4 bytes.
- * FASTEST: AUTO, and before it the kernel that keeps x in registers (K a multiple of 128 from 1024
- * on, activations and scales of one type).  Its sums are cut in other places than those of STREAM
+ * FASTEST: AUTO, and before it the kernel that keeps x in registers, for the sizes where it takes
+ * less time (K a multiple of 128 from 1024 on, activations and scales of one type).  Its sums are cut in other places than those of STREAM
  * and of a chained launch, with which AUTO agrees bit for bit beyond matrices of few weights.
  */
 enum {
@@ -266,7 +266,7 @@ int dflash_qmm_m16_chain(const dflash_qmm_problem* problems, int count, void* wo
  * Requirements: group_size 64, K % 1024 == 0, N % 16 == 0; all pointers 16-byte aligned; the
  * workspace of dflash_qmm_m16 (kernel = DFLASH_QMM_KERNEL_STREAM) with the same rules.
  * dflash_qmm_m16_packed returns bit for bit what dflash_qmm_m16 returns through the streaming
- * kernel for the unpacked operands, dflash_qmm_m16_packed_by what it returns for `kernel` (AUTO or STREAM).
+ * kernel for the unpacked operands, dflash_qmm_m16_packed_by what it returns for `kernel` (AUTO, STREAM or FASTEST).
  */
 int dflash_qmm_m16_packed_bytes(int K, int N, int group_size, size_t* codes_bytes,
                                 size_t* scales_bytes /* = biases bytes */);
