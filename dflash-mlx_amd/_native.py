@@ -81,6 +81,7 @@ EXPORTED_SYMBOLS = (
     "dflash_sdpa_q16_gated",
     "dflash_conv_state_rebuild",
     "dflash_rollback_layer",
+    "dflash_rollback_layers",
 )
 
 
@@ -185,6 +186,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.dflash_conv_state_rebuild.argtypes = [c.c_void_p] * 4 + [c.c_int] * 6 + [c.c_void_p]
     lib.dflash_rollback_layer.restype = c.c_int
     lib.dflash_rollback_layer.argtypes = [c.c_void_p] * 9 + [c.c_int] * 16 + [c.c_void_p]
+    lib.dflash_rollback_layers.restype = c.c_int
+    lib.dflash_rollback_layers.argtypes = [c.c_void_p] + [c.c_int] * 16 + [c.c_void_p]
 
 
 def lib() -> ctypes.CDLL:

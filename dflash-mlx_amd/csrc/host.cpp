@@ -550,44 +550,110 @@ PyObject* gdn_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// What a rollback of one cache takes: device tensors as record_tape() keeps them, of extents that the kernel can index.
+struct Rollback {
+  const Tensor *tape, *k, *g, *qkv, *state, *prev;
+  int64_t B, T, hv, dv, hk, dk, C;
+  int t_code, k_code, g_code, s_code;
+};
+bool rollback_of(PyObject* const (&a)[6], int steps, int keep, Rollback* r) {
+  r->tape = device_tensor(a[0]), r->k = device_tensor(a[1]), r->g = device_tensor(a[2]), r->qkv = device_tensor(a[3]);
+  r->state = device_tensor(a[4]), r->prev = nullptr;
+  if (!r->tape || !r->k || !r->g || !r->qkv || !r->state) return false;
+  const Tensor &tape = *r->tape, &k = *r->k, &g = *r->g, &qkv = *r->qkv, &state = *r->state;
+  if (tape.dim() != 4 || k.dim() != 4 || g.dim() != 3 || qkv.dim() != 3 || keep < 1) return false;
+  if (a[5] != Py_None && !(r->prev = device_tensor(a[5]))) return false;
+  const int64_t B = r->B = tape.size(0), T = r->T = tape.size(1), hv = r->hv = tape.size(2), dv = r->dv = tape.size(3);
+  const int64_t hk = r->hk = k.size(2), dk = r->dk = k.size(3), C = r->C = qkv.size(2);
+  if (hk < 1 || steps > T || !has_shape(k, {B, T, hk, dk}) || !has_shape(g, {B, T, hv}) || !has_shape(qkv, {B, T, C}) ||
+      !has_shape(state, {B, hv, dv, dk}) || dk < 32 || dk % 32 != 0 || hv % hk != 0 ||
+      T * (dv + 2 * dk + 1) * 4 + dk * 4 > 64 * 1024)
+    return false;
+  for (const Tensor* t : {&tape, &k, &g, &qkv, &state})
+    if (!t->is_contiguous() || t->device() != state.device()) return false;
+  if (r->prev && (r->prev->device() != qkv.device() || !r->prev->is_contiguous() || r->prev->scalar_type() != qkv.scalar_type() ||
+                  !has_shape(*r->prev, {B, keep, C})))
+    return false;
+  r->t_code = dtype_code(tape.scalar_type()), r->k_code = dtype_code(k.scalar_type()), r->g_code = dtype_code(g.scalar_type());
+  r->s_code = dtype_code(state.scalar_type());
+  return r->t_code != kNoCode && r->k_code != kNoCode && r->g_code != kNoCode && r->s_code != kNoCode;
+}
+
 // rollback_layer(tape, k, g, qkv, state, conv_prev, steps, keep, exact): replay and conv window of one cache's tape;
 // (state, conv window).
 PyObject* rollback_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (n != 9) Py_RETURN_NONE;
-  const Tensor *tape = device_tensor(a[0]), *k = device_tensor(a[1]), *g = device_tensor(a[2]), *qkv = device_tensor(a[3]),
-               *state = device_tensor(a[4]), *prev = nullptr;
+  Rollback r = {};
   int steps, keep, exact;
-  if (!tape || !k || !g || !qkv || !state || tape->dim() != 4 || k->dim() != 4 || g->dim() != 3 || qkv->dim() != 3 ||
-      !integer(a[6], &steps) || !integer(a[7], &keep) || !integer(a[8], &exact) || keep < 1)
+  if (!integer(a[6], &steps) || !integer(a[7], &keep) || !integer(a[8], &exact) ||
+      !rollback_of({a[0], a[1], a[2], a[3], a[4], a[5]}, steps, keep, &r))
     Py_RETURN_NONE;
-  if (a[5] != Py_None && !(prev = device_tensor(a[5]))) Py_RETURN_NONE;
-  const int64_t B = tape->size(0), T = tape->size(1), hv = tape->size(2), dv = tape->size(3), hk = k->size(2), dk = k->size(3),
-                C = qkv->size(2);
-  if (hk < 1 || steps > T || !has_shape(*k, {B, T, hk, dk}) || !has_shape(*g, {B, T, hv}) || !has_shape(*qkv, {B, T, C}) ||
-      !has_shape(*state, {B, hv, dv, dk}) || dk < 32 || dk % 32 != 0 || hv % hk != 0 ||
-      T * (dv + 2 * dk + 1) * 4 + dk * 4 > 64 * 1024)
-    Py_RETURN_NONE;
-  for (const Tensor* t : {tape, k, g, qkv, state})
-    if (!t->is_contiguous() || t->device() != state->device()) Py_RETURN_NONE;
-  if (prev && (prev->device() != qkv->device() || !prev->is_contiguous() || prev->scalar_type() != qkv->scalar_type() ||
-               !has_shape(*prev, {B, keep, C})))
-    Py_RETURN_NONE;
-  const int t_code = dtype_code(tape->scalar_type()), k_code = dtype_code(k->scalar_type()), g_code = dtype_code(g->scalar_type()),
-            s_code = dtype_code(state->scalar_type());
-  if (t_code == kNoCode || k_code == kNoCode || g_code == kNoCode || s_code == kNoCode) Py_RETURN_NONE;
-  void* stream = stream_of(*state);
+  void* stream = stream_of(*r.state);
   Tensor next, conv;
   const int rc = released([&] {
-    next = at::empty({B, hv, dv, dk}, state->options());
-    conv = at::empty({B, keep, C}, qkv->options());
-    return dflash_rollback_layer(at_of(*tape), at_of(*k), at_of(*g), at_of(*state), next.mutable_data_ptr(),
-                                 prev ? at_of(*prev) : nullptr, at_of(*qkv), conv.mutable_data_ptr(), nullptr, steps, (int)B,
-                                 (int)T, (int)hk, (int)hv, (int)dk, (int)dv, s_code, t_code, k_code, g_code, 0, exact, keep,
-                                 (int)C, (int)qkv->element_size(), stream);
+    next = at::empty({r.B, r.hv, r.dv, r.dk}, r.state->options());
+    conv = at::empty({r.B, keep, r.C}, r.qkv->options());
+    return dflash_rollback_layer(at_of(*r.tape), at_of(*r.k), at_of(*r.g), at_of(*r.state), next.mutable_data_ptr(),
+                                 r.prev ? at_of(*r.prev) : nullptr, at_of(*r.qkv), conv.mutable_data_ptr(), nullptr, steps, (int)r.B,
+                                 (int)r.T, (int)r.hk, (int)r.hv, (int)r.dk, (int)r.dv, r.s_code, r.t_code, r.k_code, r.g_code, 0,
+                                 exact, keep, (int)r.C, (int)r.qkv->element_size(), stream);
   });
   if (rc != 0) return fail(rc, "dflash_rollback_layer");
   return Py_BuildValue("(NN)", THPVariable_Wrap(std::move(next)), THPVariable_Wrap(std::move(conv)));
+  END_HANDLE_TH_ERRORS
+}
+
+// rollback_layers(operands, steps, keep, exact): the same for several caches whose operands have the same extents, types and
+// device.  operands: a list of the tuples (tape, k, g, qkv, state, conv_prev).  A list of (conv window, state): a cache's entries.
+PyObject* rollback_layers(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  int steps, keep, exact;
+  if (n != 4 || !PyList_CheckExact(a[0]) || !integer(a[1], &steps) || !integer(a[2], &keep) || !integer(a[3], &exact)) Py_RETURN_NONE;
+  const Py_ssize_t count = PyList_GET_SIZE(a[0]);
+  if (count < 2 || count >= (1 << 20)) Py_RETURN_NONE;
+  std::vector<dflash_rollback_operands> at(count);
+  Rollback r = {};
+  for (Py_ssize_t i = 0; i < count; ++i) {
+    PyObject* one = PyList_GET_ITEM(a[0], i);
+    if (!PyTuple_CheckExact(one) || PyTuple_GET_SIZE(one) != 6) Py_RETURN_NONE;
+    Rollback o = {};
+    PyObject* const parts[6] = {PyTuple_GET_ITEM(one, 0), PyTuple_GET_ITEM(one, 1), PyTuple_GET_ITEM(one, 2),
+                                PyTuple_GET_ITEM(one, 3), PyTuple_GET_ITEM(one, 4), PyTuple_GET_ITEM(one, 5)};
+    if (!rollback_of(parts, steps, keep, &o)) Py_RETURN_NONE;
+    if (i == 0) r = o;
+    if (o.B != r.B || o.T != r.T || o.hv != r.hv || o.dv != r.dv || o.hk != r.hk || o.dk != r.dk || o.C != r.C || o.t_code != r.t_code ||
+        o.k_code != r.k_code || o.g_code != r.g_code || o.s_code != r.s_code || o.qkv->scalar_type() != r.qkv->scalar_type() ||
+        o.state->device() != r.state->device())
+      Py_RETURN_NONE;
+    at[i] = {at_of(*o.tape), at_of(*o.k), at_of(*o.g), at_of(*o.state), nullptr, o.prev ? at_of(*o.prev) : nullptr, at_of(*o.qkv), nullptr};
+  }
+  void* stream = stream_of(*r.state);
+  std::vector<Tensor> made(2 * count);
+  const int rc = released([&] {
+    const auto state_options = r.state->options(), conv_options = r.qkv->options();
+    for (Py_ssize_t i = 0; i < count; ++i) {
+      made[2 * i] = at::empty({r.B, keep, r.C}, conv_options);
+      made[2 * i + 1] = at::empty({r.B, r.hv, r.dv, r.dk}, state_options);
+      at[i].conv_out = made[2 * i].mutable_data_ptr(), at[i].state_out = made[2 * i + 1].mutable_data_ptr();
+    }
+    return dflash_rollback_layers(at.data(), (int)count, steps, (int)r.B, (int)r.T, (int)r.hk, (int)r.hv, (int)r.dk, (int)r.dv, r.s_code,
+                                  r.t_code, r.k_code, r.g_code, exact, keep, (int)r.C, (int)r.qkv->element_size(), stream);
+  });
+  if (rc != 0) return fail(rc, "dflash_rollback_layers");
+  THPObjectPtr out(PyList_New(count));
+  if (!out) return nullptr;
+  for (Py_ssize_t i = 0; i < count; ++i) {
+    PyObject* pair = PyList_New(2);
+    if (pair == nullptr) return nullptr;
+    PyList_SET_ITEM(out.get(), i, pair);
+    for (int j = 0; j < 2; ++j) {
+      PyObject* t = THPVariable_Wrap(std::move(made[2 * i + j]));
+      if (t == nullptr) return nullptr;
+      PyList_SET_ITEM(pair, j, t);
+    }
+  }
+  return out.release();
   END_HANDLE_TH_ERRORS
 }
 
@@ -694,7 +760,7 @@ PyObject* bind(PyObject*, PyObject* error) {  // the class that failed launches 
 #define DFLASH_HOST(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
 PyMethodDef kMethods[] = {DFLASH_HOST(qmm_m16), DFLASH_HOST(qmm_packed), DFLASH_HOST(qmm_few), DFLASH_HOST(qmm_few_silu_mul),
                           DFLASH_HOST(qmm_rows), DFLASH_HOST(columns), DFLASH_HOST(gather), DFLASH_HOST(chain_bind), DFLASH_HOST(chain_launch), DFLASH_HOST(gdn_prepare), DFLASH_HOST(gdn_forward), DFLASH_HOST(gdn_block),
-                          DFLASH_HOST(rollback_layer), DFLASH_HOST(attn_prepare), DFLASH_HOST(sdpa_q16), {"bind", bind, METH_O, nullptr},
+                          DFLASH_HOST(rollback_layer), DFLASH_HOST(rollback_layers), DFLASH_HOST(attn_prepare), DFLASH_HOST(sdpa_q16), {"bind", bind, METH_O, nullptr},
                           {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_dflash_host", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
 

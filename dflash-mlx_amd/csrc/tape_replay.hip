@@ -124,9 +124,9 @@ __device__ __forceinline__ int slot_steps(const ReplayArgs& a, int slot) {
 
 // Workgroups beyond the replay's own rebuild the conv window, one output row each.  True if this
 // workgroup was one of them (and is done).
-__device__ __forceinline__ bool conv_window_workgroup(const ReplayArgs& a) {
-  if ((int)blockIdx.x < a.replay_blocks) return false;
-  const int b = (int)blockIdx.x - a.replay_blocks;
+__device__ __forceinline__ bool conv_window_workgroup(const ReplayArgs& a, int block) {
+  if (block < a.replay_blocks) return false;
+  const int b = block - a.replay_blocks;
   const int slot = b / a.conv_keep, j = b % a.conv_keep;
   const int steps = a.steps_dev ? a.steps_dev[slot] : a.steps_host;
   if (a.conv_vec16) conv_rebuild_row<uint4>(a.conv_prev, a.conv_qkv, a.conv_out, steps, a.T, a.conv_keep, a.conv_row_bytes, slot, j);
@@ -178,7 +178,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3, 3))
   float* sD = sK + 16 * kPad;
   float* sG = sD + 16 * kPad;
   float* sGt = sG + 16 * 128;
-  if (conv_window_workgroup(a)) return;
+  if (conv_window_workgroup(a, (int)blockIdx.x)) return;
   const int slot = a.heads.quotient((int)blockIdx.x), hv = (int)blockIdx.x - slot * a.Hv;
   const int n = slot_steps(a, slot);
   const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, kq = lane >> 4;
@@ -320,15 +320,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3, 3))
 // 4.7 / 3.9 -> 3.5 / 3.2, 1536 heads 14.5 / 13.1 -> 11.8 / 11.6.
 // ---------------------------------------------------------------------------
 template <int STATE, int DK, int R>
-__global__ __launch_bounds__(kThreads) void replay_rows(ReplayArgs a) {
+__device__ __forceinline__ void replay_rows_of(const ReplayArgs& a, int block) {
   constexpr bool kWide = STATE == DFLASH_FP32;
   constexpr int kLanes = DK / 8, kPass = kThreads / kLanes, kRows = kPass * R;  // lanes of a row, rows of a pass, of the workgroup
   constexpr int kD = kRows / 16, kK = DK / 16;  // elements of delta and k that a thread brings
   __shared__ __align__(16) float sK[16 * DK];
   __shared__ __align__(16) float sD[16 * kRows];
   __shared__ float sG[16];
-  if (conv_window_workgroup(a)) return;
-  const int head = a.row_parts.quotient((int)blockIdx.x), row0 = ((int)blockIdx.x - head * (int)a.row_parts.by) * kRows;
+  if (conv_window_workgroup(a, block)) return;
+  const int head = a.row_parts.quotient(block), row0 = (block - head * (int)a.row_parts.by) * kRows;
   const int slot = a.heads.quotient(head), hv = head - slot * a.Hv, hk = a.group.quotient(hv);
   const int n = slot_steps(a, slot);
   const int tid = threadIdx.x, t = tid >> 4, seg = tid & 15;
@@ -450,6 +450,42 @@ __global__ __launch_bounds__(kThreads) void replay_rows(ReplayArgs a) {
   }
 }
 
+template <int STATE, int DK, int R>
+__global__ __launch_bounds__(kThreads) void replay_rows(ReplayArgs a) {
+  replay_rows_of<STATE, DK, R>(a, (int)blockIdx.x);
+}
+
+// Layers that hold tensors of their own, of one shape, in one launch: a workgroup finds its layer by its place and the layer's
+// addresses among the arguments.  A launch per layer leaves most of the chip idle for its 5 to 6 us and costs the host 4.  Kernel
+// time, a launch each and together: 20 layers of 2 x 32 heads of 128 x 128, bf16 states, 13 steps 119 -> 36 us; 10 of 64 heads, fp32,
+// 8 steps 50 -> 18; 48 of 32 heads, fp32, 7 steps 228 -> 42 (two launches).  The calls around them 188 -> 106, 89 -> 56 and
+// 430 -> 254 us: what is left is the host's, two allocations a layer and the caches' own steps.
+constexpr int kLayersAtOnce = 32;  // their addresses and the rest of the arguments are 2.3 KB
+struct LayersArgs {
+  ReplayArgs one;  // of a layer, without addresses
+  Divisor per_layer, windows;  // by the workgroups of a layer that replay and that rebuild its conv window
+  int replay_blocks;  // of all layers
+  dflash_rollback_operands at[kLayersAtOnce];
+};
+
+template <int STATE, int DK, int R>
+__global__ __launch_bounds__(kThreads) void replay_rows_layers(LayersArgs p) {
+  ReplayArgs a = p.one;
+  int block = (int)blockIdx.x, layer;
+  if (block < p.replay_blocks) {
+    layer = p.per_layer.quotient(block);
+    block -= layer * a.replay_blocks;
+  } else {
+    block -= p.replay_blocks;
+    layer = p.windows.quotient(block);
+    block += a.replay_blocks - layer * (int)p.windows.by;
+  }
+  const dflash_rollback_operands& at = p.at[layer];
+  a.tape = at.tape, a.k = at.k, a.g = at.g, a.state_in = at.state_in, a.state_out = at.state_out;
+  a.conv_prev = (const char*)at.conv_prev, a.conv_qkv = (const char*)at.qkv, a.conv_out = (char*)at.conv_out;
+  replay_rows_of<STATE, DK, R>(a, block);
+}
+
 // The form of replay_rows for a head size and state type; rows: how many a workgroup computes.  heads: of all slots.  The lines
 // of the fp32 states (16 bf16 steps, us with one / two / four / eight rows of a pass): 128 x 128, 32 heads 4.5 / 4.4 / 5.1 / 7.2,
 // 192 heads 8.9 / 6.9 / 7.3 / 8.6, 256 heads 11.0 / 7.9 / 7.9 / 9.7, 384 heads 14.9 / 11.6 / 9.8 / 11.2, 1536 heads 42.6 / 39.5 / 37.2 / 39.9;
@@ -461,17 +497,24 @@ __global__ __launch_bounds__(kThreads) void replay_rows(ReplayArgs a) {
 // steps, us, split and whole: 512 heads 16.0 / 10.0 and 19.3 / 10.3, 1024 heads 28.6 / 16.8 and 31.9 / 15.4, 1536 heads 41.6 / 25.4
 // and 44.4 / 20.5; 64 x 64 at 1024 heads 10.6 / 7.2 and 9.6 / 6.1).
 template <int STATE>
-const void* replay_rows_for(int Dk, int Dv, long long heads, int* rows) {
+const void* replay_rows_for(int Dk, int Dv, long long heads, bool layers, int* rows) {
+#define DFLASH_REPLAY_ROWS(DK_, R_, ROWS_) \
+  return *rows = ROWS_, layers ? (const void*)replay_rows_layers<STATE, DK_, R_> : (const void*)replay_rows<STATE, DK_, R_>
   constexpr bool kWide = STATE == DFLASH_FP32;
   const bool many = kWide ? heads > (Dk == 128 ? 192 : 96) : heads >= 1024;
   constexpr int kMany = kWide ? 4 : 8;
-  if (kWide && Dk == 128 && Dv % 128 == 0 && heads * (Dv / 64) > 3 * 256 && heads * (Dv / 128) <= 2 * 256)
-    return *rows = 128, (const void*)replay_rows<STATE, 128, 8>;
-  if (Dk == 128 && many && Dv % (16 * kMany) == 0) return *rows = 16 * kMany, (const void*)replay_rows<STATE, 128, kMany>;
-  if (Dk == 128 && Dv % 32 == 0) return *rows = 32, (const void*)replay_rows<STATE, 128, 2>;
-  if (Dk == 64 && many && Dv % 64 == 0) return *rows = 64, (const void*)replay_rows<STATE, 64, 2>;
-  if (Dk == 64 && Dv % 32 == 0) return *rows = 32, (const void*)replay_rows<STATE, 64, 1>;
+  if (kWide && Dk == 128 && Dv % 128 == 0 && heads * (Dv / 64) > 3 * 256 && heads * (Dv / 128) <= 2 * 256) DFLASH_REPLAY_ROWS(128, 8, 128);
+  if (Dk == 128 && many && Dv % (16 * kMany) == 0) DFLASH_REPLAY_ROWS(128, kMany, 16 * kMany);
+  if (Dk == 128 && Dv % 32 == 0) DFLASH_REPLAY_ROWS(128, 2, 32);
+  if (Dk == 64 && many && Dv % 64 == 0) DFLASH_REPLAY_ROWS(64, 2, 64);
+  if (Dk == 64 && Dv % 32 == 0) DFLASH_REPLAY_ROWS(64, 1, 32);
   return nullptr;
+#undef DFLASH_REPLAY_ROWS
+}
+const void* replay_rows_for(int state_dtype, int Dk, int Dv, long long heads, bool layers, int* rows) {
+  return state_dtype == DFLASH_BF16   ? replay_rows_for<DFLASH_BF16>(Dk, Dv, heads, layers, rows)
+         : state_dtype == DFLASH_FP16 ? replay_rows_for<DFLASH_FP16>(Dk, Dv, heads, layers, rows)
+                                      : replay_rows_for<DFLASH_FP32>(Dk, Dv, heads, layers, rows);
 }
 
 // ---------------------------------------------------------------------------
@@ -481,7 +524,7 @@ const void* replay_rows_for(int Dk, int Dv, long long heads, int* rows) {
 template <bool EXACT>
 __global__ __launch_bounds__(kThreads) void replay_generic(ReplayArgs a) {
   extern __shared__ float smem[];
-  if (conv_window_workgroup(a)) return;
+  if (conv_window_workgroup(a, (int)blockIdx.x)) return;
   const Smem s = carve(smem, a, a.T);
   const int slot = blockIdx.x / a.Hv, hv = blockIdx.x % a.Hv;
   const int n = slot_steps(a, slot);
@@ -577,9 +620,7 @@ int replay_launch(const void* tape, const void* k, const void* g, const void* st
   if (!g_per_dk && T >= 1 && T <= 16 && aligned16 && (((uintptr_t)state_in | (uintptr_t)state_out) % 16) == 0 &&
       (!exact || state_dtype != DFLASH_FP32)) {
     const long long heads = (long long)slots * Hv;
-    by_rows = state_dtype == DFLASH_BF16   ? replay_rows_for<DFLASH_BF16>(Dk, Dv, heads, &rows)
-              : state_dtype == DFLASH_FP16 ? replay_rows_for<DFLASH_FP16>(Dk, Dv, heads, &rows)
-                                           : replay_rows_for<DFLASH_FP32>(Dk, Dv, heads, &rows);
+    by_rows = replay_rows_for(state_dtype, Dk, Dv, heads, false, &rows);
   }
   // gates per element of a row: the matrix-core form
   const bool fast = !exact && g_per_dk && Dk == 128 && Dv == 128 && T <= 16 && aligned16;
@@ -670,4 +711,61 @@ extern "C" int dflash_rollback_layer(const void* tape, const void* k, const void
                                Dv, state_dtype, tape_dtype, k_dtype, g_dtype, g_per_dk, exact_order,
                                window ? conv_prev : nullptr, window ? qkv : nullptr, window ? conv_out : nullptr,
                                window ? keep : 0, window ? C : 0, window ? qkv_elem_bytes : 0, stream);
+}
+
+extern "C" int dflash_rollback_layers(const dflash_rollback_operands* layers, int count, int steps, int slots, int T, int Hk, int Hv,
+                                      int Dk, int Dv, int state_dtype, int tape_dtype, int k_dtype, int g_dtype, int exact_order,
+                                      int keep, int C, int qkv_elem_bytes, void* stream) {
+  using namespace dflash;
+  DFLASH_REQUIRE(count == 0 || layers, DFLASH_ERR_ARG, "dflash_rollback_layers: null operands");
+  DFLASH_REQUIRE(count >= 0 && slots >= 0 && T >= 0 && Hk > 0 && Hv > 0 && Dk > 0 && Dv > 0, DFLASH_ERR_SHAPE,
+                 "dflash_rollback_layers: non-positive dimension");
+  DFLASH_REQUIRE(valid_dtype(state_dtype) && valid_dtype(tape_dtype) && valid_dtype(k_dtype) && valid_dtype(g_dtype), DFLASH_ERR_ARG,
+                 "dflash_rollback_layers: unknown dtype code");
+  bool joint = count > 1 && slots > 0 && T >= 1 && T <= 16 && Hv % Hk == 0 && (state_dtype != DFLASH_FP32 || exact_order == 0);
+  const bool window = keep > 0;
+  const size_t row_bytes = window && C > 0 && qkv_elem_bytes > 0 ? (size_t)C * qkv_elem_bytes : 0;
+  joint = joint && (!window || row_bytes != 0);
+  bool vec16 = row_bytes % 16 == 0;
+  for (int i = 0; i < count; ++i) {
+    const dflash_rollback_operands& at = layers[i];
+    const uintptr_t wide = (uintptr_t)at.tape | (uintptr_t)at.k | (uintptr_t)at.state_in | (uintptr_t)at.state_out;
+    joint = joint && at.tape && at.k && at.g && at.state_in && at.state_out && at.state_in != at.state_out && wide % 16 == 0 &&
+            (!window || (at.qkv && at.conv_out && at.conv_out != at.conv_prev));
+    vec16 = vec16 && ((uintptr_t)at.conv_prev | (uintptr_t)at.qkv | (uintptr_t)at.conv_out) % 16 == 0;
+  }
+  for (int first = 0; first < count;) {
+    const int here = count - first < kLayersAtOnce ? count - first : kLayersAtOnce;
+    int rows = 0;
+    const long long heads = (long long)slots * Hv;
+    const void* const fn = joint && here > 1 ? replay_rows_for(state_dtype, Dk, Dv, heads * here, true, &rows) : nullptr;
+    const long long blocks = fn ? heads * (Dv / rows) : 0, windows = window ? (long long)slots * keep : 0;
+    if (fn == nullptr || (blocks + windows) * here >= (1ll << 31)) {
+      // layer by layer, also for whatever that call refuses
+      for (int i = first; i < first + here; ++i) {
+        const dflash_rollback_operands& at = layers[i];
+        const int rc = dflash_rollback_layer(at.tape, at.k, at.g, at.state_in, at.state_out, at.conv_prev, at.qkv, at.conv_out, nullptr,
+                                             steps, slots, T, Hk, Hv, Dk, Dv, state_dtype, tape_dtype, k_dtype, g_dtype, 0, exact_order,
+                                             keep, C, qkv_elem_bytes, stream);
+        if (rc != DFLASH_OK) return rc;
+      }
+      first += here;
+      continue;
+    }
+    LayersArgs p = {};
+    ReplayArgs& a = p.one;
+    a.steps_host = steps;
+    a.T = T; a.Hk = Hk; a.Hv = Hv; a.Dk = Dk; a.Dv = Dv;
+    a.heads = Divisor::of(Hv); a.group = Divisor::of(Hv / Hk); a.row_parts = Divisor::of(Dv / rows);
+    a.state_dtype = state_dtype; a.tape_dtype = tape_dtype; a.k_dtype = k_dtype; a.g_dtype = g_dtype;
+    a.conv_row_bytes = row_bytes; a.conv_keep = window ? keep : 0; a.conv_vec16 = vec16;
+    a.replay_blocks = (int)blocks;
+    p.per_layer = Divisor::of(blocks); p.windows = Divisor::of(windows > 0 ? windows : 1);
+    p.replay_blocks = (int)(blocks * here);
+    for (int i = 0; i < here; ++i) p.at[i] = layers[first + i];
+    void* args[] = {&p};
+    DFLASH_HIP_OK(hipLaunchKernel(fn, dim3((unsigned)((blocks + windows) * here)), dim3(kThreads), args, 0, (hipStream_t)stream));
+    first += here;
+  }
+  return DFLASH_OK;
 }

@@ -5,8 +5,9 @@ device kernels: the load-time decision to swap linears (:714-753), acceptance
 matching (:101-108), arming (:833-846) and the per-layer restore after acceptance
 (:849-907).  Index arithmetic is integer-exact with the reference.
 
-Caches handed out by a ``RollbackArena`` are rolled back with one batched launch
-instead of one launch per layer; everything else follows the per-layer loop.
+Caches handed out by a ``RollbackArena`` are rolled back with one batched launch, caches
+of one shape that hold tensors of their own with one launch for up to 32 of them;
+everything else follows the per-layer loop.
 """
 from __future__ import annotations
 
@@ -17,7 +18,7 @@ from typing import Any, List, Optional, Sequence
 import torch
 
 from .cache import KVCache
-from .recurrent_rollback_cache import RecurrentRollbackCache, RollbackArena
+from .recurrent_rollback_cache import RecurrentRollbackCache, RollbackArena, rollback_together
 
 
 def _verify_enabled_for(config: Any) -> bool:
@@ -152,9 +153,14 @@ def _restore_target_cache_after_acceptance(cache_entries: List[Any], *, target_l
         replay_start_ns = time.perf_counter_ns()
         arena.rollback_all(int(acceptance_length), drafted_tokens=drafted_tokens)
         replay_ns_total += time.perf_counter_ns() - replay_start_ns
+    done = arena is not None
+    if not done and not fully_accepted:
+        replay_start_ns = time.perf_counter_ns()
+        done = rollback_together([c for c in cache_entries if hasattr(c, "rollback")], acceptance_length)
+        replay_ns_total += time.perf_counter_ns() - replay_start_ns if done else 0
     for cache_entry in cache_entries:
         if hasattr(cache_entry, "rollback"):
-            if arena is not None:
+            if done:
                 continue
             if fully_accepted:
                 _clear_rollback_state(cache_entry)

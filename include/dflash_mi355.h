@@ -587,6 +587,23 @@ int dflash_rollback_layer(const void* tape, const void* k, const void* g, const 
                           int g_dtype, int g_per_dk, int exact_order, int keep, int C,
                           int qkv_elem_bytes, void* stream);
 
+/*
+ * The rollback of several layers of one shape that hold tensors of their own (no counterpart in the reference, whose loop
+ * over caches, dflash_mlx/runtime.py:880-900, leaves it to lazy evaluation): results bit for bit those of `count` calls of
+ * dflash_rollback_layer with one gate per head and the host's step count.  Up to 32 layers take one launch where the
+ * tapes have at most 16 rows, Dk is 64 or 128 and pointers are 16-byte aligned; others take a launch each.  No layer's
+ * results may overlap any layer's operands.  keep == 0 leaves the conv windows out.
+ */
+typedef struct dflash_rollback_operands {
+  const void *tape, *k, *g, *state_in;
+  void* state_out;
+  const void *conv_prev, *qkv; /* conv_prev NULL: zeros */
+  void* conv_out;
+} dflash_rollback_operands;
+int dflash_rollback_layers(const dflash_rollback_operands* layers, int count, int steps, int slots, int T, int Hk, int Hv,
+                           int Dk, int Dv, int state_dtype, int tape_dtype, int k_dtype, int g_dtype, int exact_order,
+                           int keep, int C, int qkv_elem_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -283,6 +283,83 @@ def test_rollback_in_one_library_call_equals_the_two_wrappers(native_lib, monkey
         assert state_a.data_ptr() != state_b.data_ptr()
 
 
+@pytest.mark.parametrize("layers,batch,Hk,Hv,D,T,state,odd", [
+    (2, 1, 2, 4, 128, 16, torch.float32, None), (33, 1, 1, 2, 64, 16, torch.bfloat16, None),
+    (32, 2, 2, 4, 128, 1, torch.bfloat16, "no window"), (65, 1, 1, 1, 64, 7, torch.float32, "widths"),
+    (5, 3, 2, 32, 128, 16, torch.float32, "addresses"), (3, 2, 2, 4, 96, 16, torch.float32, None),
+    (4, 1, 2, 4, 128, 17, torch.float32, None), (17, 1, 16, 64, 128, 16, torch.float32, None),
+    (4, 1, 2, 4, 128, 16, torch.float32, "shapes")])
+def test_layers_rolled_back_together_have_the_bits_of_each_by_itself(native_lib, layers, batch, Hk, Hv, D, T, state, odd):
+    """One launch for caches with tensors of their own: remainders of 32 layers, every form of the kernel and what has none,
+    conv windows that are missing, of odd width or at odd addresses, a layer of another shape among the rest."""
+    from dflash_mlx_amd.engine import HybridGDNEngine
+
+    gen = torch.Generator(device=DEV).manual_seed(97)
+    normal = lambda *shape, dtype=torch.float32: torch.randn(shape, generator=gen, device=DEV).to(dtype)
+
+    def at_odd_address(t):
+        flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=DEV)
+        return flat[1:].view(t.shape).copy_(t)
+
+    made = []
+    for i in range(layers):
+        hv = 2 * Hv if odd == "shapes" and i == 2 else Hv
+        C = 2 * Hk * D + Hv * D + (1 if odd == "widths" else 0)
+        window = None if odd == "no window" and i % 2 else normal(batch, 3, C, dtype=torch.bfloat16)
+        tape = dict(tape=normal(batch, T, hv, D), k=normal(batch, T, Hk, D, dtype=torch.bfloat16), g=torch.sigmoid(normal(batch, T, hv)),
+                    qkv=normal(batch, T, C, dtype=torch.bfloat16))
+        if odd == "addresses" and i == 3:
+            tape["qkv"], window = at_odd_address(tape["qkv"]), at_odd_address(window)
+        made.append((window, normal(batch, hv, D, D, dtype=state), tape))
+
+    def run(accepted, together):
+        caches = [RecurrentRollbackCache(size=2, conv_kernel_size=4) for _ in range(layers)]
+        for c, (window, s, tape) in zip(caches, made):
+            c[0], c[1] = window, s
+            c.arm_rollback()
+            c.record_tape(**tape)
+        if together:
+            HybridGDNEngine().rollback(caches, target_len=0, acceptance_len=accepted, drafted_tokens=T + 1)
+        else:
+            for c in caches:
+                c.rollback(accepted)
+        torch.cuda.synchronize()
+        assert all(c._snapshot is None and c._tape is None and not c._armed for c in caches)
+        return [t for c in caches for t in c.cache]
+
+    for accepted in sorted({0, T // 2, T - 1}):
+        for a, b in zip(run(accepted, True), run(accepted, False)):
+            assert a.dtype == b.dtype and a.shape == b.shape and torch.equal(a, b)
+
+
+def test_caches_that_are_not_all_alike_are_rolled_back_one_by_one(native_lib):
+    """An unarmed cache, one of a subclass, one with a rollback of its own: nothing is done for the rest in their place."""
+    from dflash_mlx_amd.recurrent_rollback_cache import rollback_together
+
+    case, qkv, conv0 = _gdn_cycle_inputs(98, L=1, B=1)
+
+    class Other(RecurrentRollbackCache):
+        pass
+
+    def armed(cls=RecurrentRollbackCache):
+        c = cls(size=2, conv_kernel_size=4)
+        c[0], c[1] = conv0[0].to(DEV), case.state[0].to(DEV)
+        c.arm_rollback()
+        c.record_tape(tape=case.tape[0].to(DEV), k=case.k[0].to(DEV), g=case.g[0].to(DEV), qkv=qkv[0].to(DEV))
+        return c
+
+    patched = armed()
+    patched.rollback = lambda n: None
+    untaped = armed()
+    untaped._tape = None
+    for other in (RecurrentRollbackCache(size=2, conv_kernel_size=4), armed(Other), patched, untaped):
+        first = armed()
+        before = list(first.cache)
+        assert not rollback_together([first, other], 3)
+        assert first._snapshot is not None and all(a is b for a, b in zip(first.cache, before))
+    assert not rollback_together([armed()], 3) and rollback_together([armed(), armed()], 3)
+
+
 def test_rollback_outside_the_one_call_case_takes_the_wrappers(native_lib):
     """Per-element gates are not what the one-call path takes: it declines, and the result is
     the oracle model's all the same."""
