@@ -79,6 +79,8 @@ EXPORTED_SYMBOLS = (
     "dflash_sdpa_q16_workspace_bytes",
     "dflash_sdpa_q16",
     "dflash_sdpa_q16_gated",
+    "dflash_attn_block_workspace_bytes",
+    "dflash_attn_block",
     "dflash_conv_state_rebuild",
     "dflash_rollback_layer",
     "dflash_rollback_layers",
@@ -176,6 +178,10 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.dflash_sdpa_q16_gated.restype = c.c_int
     lib.dflash_sdpa_q16_gated.argtypes = ([c.c_void_p] * 7 + [c.c_size_t] + [c.c_int] * 5 + [c.c_longlong] * 8 +
                                           [c.c_float, c.c_int, c.c_void_p])
+    lib.dflash_attn_block_workspace_bytes.restype = c.c_size_t
+    lib.dflash_attn_block_workspace_bytes.argtypes = [c.c_int] * 5
+    lib.dflash_attn_block.restype = c.c_int
+    lib.dflash_attn_block.argtypes = [c.c_void_p] * 2
     lib.dflash_tape_replay.restype = c.c_int
     lib.dflash_tape_replay.argtypes = (
         [c.c_void_p] * 6 + [c.c_int] + [c.c_void_p] + [c.c_int] * 12 + [c.c_void_p]

@@ -142,11 +142,15 @@ class GatedAttention(nn.Module):
 
 def _project(self, x: torch.Tensor, cache: Optional[Any]):
     """dflash_mlx/runtime.py:527-556: projections, head norms, rope, cache update."""
+    # one launch for the three where fuse_shared_input_linears joined them
+    return _behind_projections(self, x, cache, *shared_input_outputs(self, ("q_proj", "k_proj", "v_proj"), x, columns=True))
+
+
+def _behind_projections(self, x: torch.Tensor, cache: Optional[Any], q_proj_output: torch.Tensor, keys: torch.Tensor,
+                        values: torch.Tensor):
     B, L, _ = x.shape
     num_attention_heads = _attention_num_heads(self)
     num_key_value_heads = _attention_num_kv_heads(self)
-    # one launch for the three where fuse_shared_input_linears joined them
-    q_proj_output, keys, values = shared_input_outputs(self, ("q_proj", "k_proj", "v_proj"), x, columns=True)
     on_device = _project_on_device(self, q_proj_output, keys, values, cache)
     if on_device is not None:
         return on_device
@@ -239,6 +243,31 @@ def _project_on_device(self, q_proj_output: torch.Tensor, keys: torch.Tensor, va
     return queries, ko[:, :, :end], vo[:, :, :end], q_proj_output, prev
 
 
+def _attend_in_one(self, q_proj_output: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, cache: Any) -> Optional[torch.Tensor]:
+    """A verify block from its projections to its gated attention, in the attention's own launches (``dflash_attn_block``): the
+    cache has room for the block and holds what comes before it.  None, and nothing done, where ``_project_on_device`` would not
+    take the block or that launch has no form for it."""
+    q_norm, k_norm, rope = self.q_norm, self.k_norm, self.rope
+    if type(cache) is not KVCache or type(q_norm) is not HeadRMSNorm or type(k_norm) is not HeadRMSNorm \
+            or type(rope) is not RotaryEmbedding or not unhooked(q_norm, k_norm, rope):
+        return None
+    cache_keys, cache_values, qw, kw = cache.keys, cache.values, q_norm.weight, k_norm.weight
+    if (cache_keys is None or not q_proj_output.is_cuda
+            or not _native.plain(q_proj_output, keys, values, qw, kw, cache_keys, cache_values)
+            or q_proj_output.shape[-1] != 2 * _attention_num_heads(self) * cache_keys.shape[-1]
+            or cache_keys.shape[1] != _attention_num_kv_heads(self)):
+        return None
+    end = cache.offset + 16
+    rows = _native.host().first_rows(cache_keys, cache_values, end)
+    if rows is None:
+        return None
+    gated = batched_sdpa_2pass_exact(queries=None, keys=rows[0], values=rows[1], scale=self.scale, q_proj_output=q_proj_output,
+                                     unprepared=(keys, values, qw, kw, rope.dims, q_norm.eps, k_norm.eps, float(rope.base)))
+    if gated is not None:
+        cache.offset = end  # the rows are on their way: not before
+    return gated
+
+
 def _finish(self, output: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
     """Gate and output projection.  ``gate`` [B, L, Hq * D], or the whole output of q_proj, [B, L, Hq * 2 D], as ``_project_on_device`` leaves it."""
     B, H, L, D = output.shape
@@ -269,9 +298,15 @@ def _install_split_full_attention_hook(attn: Any) -> None:
             return original_call(self, x, mask=mask, cache=cache)
         if not _attention_has_gated_q_proj(self):
             return original_call(self, x, mask=mask, cache=cache)
-        queries, keys, values, gate, cached_prefix_len = _project(self, x, cache)
         exact_prefix_threshold = int(getattr(self, "_dflash_split_sdpa_exact_kv_threshold",
                                              _HYBRID_SDPA_EXACT_KV_THRESHOLD))
+        projected = shared_input_outputs(self, ("q_proj", "k_proj", "v_proj"), x, columns=True)
+        if x.shape[1] == 16 and (mask is None or (isinstance(mask, str) and mask == "causal")) \
+                and type(cache) is KVCache and 0 < cache.offset >= exact_prefix_threshold:
+            gated = _attend_in_one(self, *projected, cache)
+            if gated is not None:
+                return self.o_proj(gated)
+        queries, keys, values, gate, cached_prefix_len = _behind_projections(self, x, cache, *projected)
         is_array = isinstance(mask, torch.Tensor)
         should_split = (cache is not None and cached_prefix_len >= exact_prefix_threshold and
                         (mask is None or is_array or mask == "causal"))

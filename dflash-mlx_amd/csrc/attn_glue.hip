@@ -76,36 +76,17 @@ __global__ __launch_bounds__(kWavesPerGroup * 64) void attn_prepare_kernel(AttnP
   for (int h = first; h < heads; h += p.waves) {
     if (h >= rotated) {
       uint16_t* const dst = p.v_out + b * p.vo_batch + (h - rotated) * p.vo_head + l * p.vo_row + c;
-      if constexpr (PER == 4) {
-        *reinterpret_cast<uint2*>(dst) = make_uint2(raw[0], raw[1]);
-      } else if constexpr (PER == 2) {
-        *reinterpret_cast<uint32_t*>(dst) = raw[0];
-      } else {
-#pragma unroll
-        for (int e = 0; e < PER; ++e) dst[e] = (uint16_t)raw[e];
-      }
+      store_raw<PER>(dst, raw);
       if (h + p.waves < heads) request(h + p.waves);
       continue;
     }
     const bool is_q = h < p.Hq;
     const int hk = h - p.Hq;
-    float x[PER], w[PER], ss = 0.f;
+    float x[PER], w[PER];
     unpack_adjacent<PER>(raw, p.dt, x);
     unpack_adjacent<PER>(wraw, is_q ? p.q_weight_dt : p.k_weight_dt, w);
     if (h + p.waves < heads) request(h + p.waves);
-#pragma unroll
-    for (int e = 0; e < PER; ++e) ss += x[e] * x[e];
-    // (the array operators divide by a number by multiplying with its reciprocal: the mean here, the exponents above)
-    const float inv_rms = 1.0f / sqrtf(wave_sum(ss) * (1.0f / (float)D) + (is_q ? p.q_eps : p.k_eps));
-#pragma unroll
-    for (int e = 0; e < PER; ++e) {
-      x[e] = round_through(x[e] * inv_rms * w[e], p.dt);
-      const float y = __shfl(x[e], other, 64);  // the other half's feature of the pair
-      if (rotates) {
-        const float a = x[e] * cs[e], d = y * sn[e];
-        x[e] = upper ? d + a : a - d;
-      }
-    }
+    norm_and_turn<PER>(x, w, is_q ? p.q_eps : p.k_eps, cs, sn, rotates, upper, other, p.dt);
     if (is_q) {
       store_adjacent<PER>(p.q_out, (((size_t)b * p.Hq + h) * p.L + l) * D + c, p.dt, x);
     } else {

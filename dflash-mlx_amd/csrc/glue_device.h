@@ -119,5 +119,40 @@ __device__ __forceinline__ void store_adjacent(void* p, size_t i, int dt, const 
   }
 }
 
+// PER adjacent 16-bit elements stored as load_adjacent_raw() left them.
+template <int PER>
+__device__ __forceinline__ void store_raw(uint16_t* dst, const uint32_t (&raw)[PER]) {
+  if constexpr (PER == 4) {
+    *reinterpret_cast<uint2*>(dst) = make_uint2(raw[0], raw[1]);
+  } else if constexpr (PER == 2) {
+    *reinterpret_cast<uint32_t*>(dst) = raw[0];
+  } else {
+#pragma unroll
+    for (int e = 0; e < PER; ++e) dst[e] = (uint16_t)raw[e];
+  }
+}
+
+// Norm and rotation of one head by a wave, a lane on PER adjacent features: x <- turned(round(x rsqrt(mean x^2 + eps) w)), the
+// products and sums of the rotation rounded one by one, as the array operators do it.  other: the lane of the pair's other half.
+template <int PER>
+__device__ __forceinline__ void norm_and_turn(float (&x)[PER], const float (&w)[PER], float eps, const float (&cs)[PER],
+                                              const float (&sn)[PER], bool rotates, bool upper, int other, int dt) {
+#pragma clang fp contract(off)
+  float ss = 0.f;
+#pragma unroll
+  for (int e = 0; e < PER; ++e) ss += x[e] * x[e];
+  // (the array operators divide by a number by multiplying with its reciprocal)
+  const float inv_rms = 1.0f / sqrtf(wave_sum(ss) * (1.0f / (float)(64 * PER)) + eps);
+#pragma unroll
+  for (int e = 0; e < PER; ++e) {
+    x[e] = round_through(x[e] * inv_rms * w[e], dt);
+    const float y = __shfl(x[e], other, 64);  // the other half's feature of the pair
+    if (rotates) {
+      const float a = x[e] * cs[e], d = y * sn[e];
+      x[e] = upper ? d + a : a - d;
+    }
+  }
+}
+
 }  // namespace
 }  // namespace dflash

@@ -749,6 +749,71 @@ PyObject* sdpa_q16(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// first_rows(keys, values, rows): a cache's buffers [B, H, capacity, D] up to a row.
+PyObject* first_rows(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 3) Py_RETURN_NONE;
+  const Tensor *k = device_tensor(a[0]), *v = device_tensor(a[1]);
+  int rows;
+  if (!k || !v || !integer(a[2], &rows) || k->dim() != 4 || v->dim() != 4 || rows > k->size(2) || rows > v->size(2)) Py_RETURN_NONE;
+  return Py_BuildValue("(NN)", THPVariable_Wrap(k->narrow(2, 0, rows)), THPVariable_Wrap(v->narrow(2, 0, rows)));
+  END_HANDLE_TH_ERRORS
+}
+
+// attn_block(q_proj_output, keys, values, q_weight, k_weight, cache_keys, cache_values, rope_dims, q_eps, k_eps, base, scale, workspaces):
+// a block of 16 tokens from its projections to its gated attention; cache_keys and cache_values [B, Hk, N, D] hold the block's rows
+// last, which are written here.
+PyObject* attn_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 13) Py_RETURN_NONE;
+  const Tensor* t[7];
+  for (int i = 0; i < 7; ++i)
+    if (!(t[i] = device_tensor(a[i]))) Py_RETURN_NONE;
+  const Tensor &q = *t[0], &k = *t[1], &v = *t[2], &qw = *t[3], &kw = *t[4], &ck = *t[5], &cv = *t[6];
+  int rope;
+  if (!integer(a[7], &rope) || q.dim() != 3 || ck.dim() != 4) Py_RETURN_NONE;
+  for (int i = 8; i < 12; ++i)
+    if (!PyFloat_CheckExact(a[i])) Py_RETURN_NONE;
+  const int64_t B = q.size(0), Hk = ck.size(1), N = ck.size(2), D = ck.size(3);
+  const int code = half_code(q.scalar_type());
+  if (code == kNoCode || B < 1 || Hk < 1 || (D != 128 && D != 256) || N <= 16 || N >= (1 << 30) || q.size(1) != 16 ||
+      q.size(2) % (2 * D) != 0 || (rope != 64 && rope != 128 && (rope != 256 || D != 256)))
+    Py_RETURN_NONE;
+  const int64_t Hq = q.size(2) / (2 * D);
+  if (Hq < 1 || Hq % Hk != 0 || Hq / Hk > 8 || B * Hq >= (1 << 26) || !has_shape(k, {B, 16, Hk * D}) || !has_shape(v, {B, 16, Hk * D}) ||
+      !has_shape(qw, {D}) || !has_shape(kw, {D}) || !qw.is_contiguous() || !kw.is_contiguous() || !has_shape(ck, {B, Hk, N, D}) ||
+      !has_shape(cv, {B, Hk, N, D}))
+    Py_RETURN_NONE;
+  for (const Tensor* x : t)
+    if (x->scalar_type() != q.scalar_type() || x->device() != q.device() || !aligned(at_of(*x), 16)) Py_RETURN_NONE;
+  for (const Tensor* x : {&q, &k, &v})
+    if (x->stride(2) != 1 || (x->stride(0) | x->stride(1)) % 8 != 0) Py_RETURN_NONE;
+  for (const Tensor* x : {&ck, &cv})
+    if (x->stride(3) != 1 || (x->stride(0) | x->stride(1) | x->stride(2)) % 8 != 0 || x->stride(2) < D) Py_RETURN_NONE;
+  const size_t need = dflash_attn_block_workspace_bytes((int)B, (int)Hq, (int)Hk, (int)N, (int)D);
+  if (need == 0) Py_RETURN_NONE;
+  void* stream = stream_of(q);
+  Tensor out, ws = kept_workspace(a[12], Py_BuildValue("(NK)", THPDevice_New(q.device()), (unsigned long long)(uintptr_t)stream), need);
+  if (!ws.defined()) Py_RETURN_NONE;
+  dflash_attn_block_args p = {};
+  p.q = at_of(q), p.k = at_of(k), p.v = at_of(v), p.q_weight = at_of(qw), p.k_weight = at_of(kw);
+  p.k_cache = ck.mutable_data_ptr(), p.v_cache = cv.mutable_data_ptr(), p.workspace = ws.mutable_data_ptr(), p.workspace_bytes = ws.nbytes();
+  p.q_batch = q.stride(0), p.q_row = q.stride(1), p.k_batch = k.stride(0), p.k_row = k.stride(1);
+  p.v_batch = v.stride(0), p.v_row = v.stride(1);
+  p.k_cache_batch = ck.stride(0), p.k_cache_head = ck.stride(1), p.k_cache_row = ck.stride(2);
+  p.v_cache_batch = cv.stride(0), p.v_cache_head = cv.stride(1), p.v_cache_row = cv.stride(2);
+  p.B = (int)B, p.Hq = (int)Hq, p.Hk = (int)Hk, p.N = (int)N, p.D = (int)D, p.rope_dims = rope, p.dtype = code;
+  p.q_eps = (float)PyFloat_AS_DOUBLE(a[8]), p.k_eps = (float)PyFloat_AS_DOUBLE(a[9]);
+  p.rope_base = (float)PyFloat_AS_DOUBLE(a[10]), p.scale = (float)PyFloat_AS_DOUBLE(a[11]);
+  const int rc = released([&] {
+    out = at::empty({B, 16, Hq * D}, q.options());
+    p.out = out.mutable_data_ptr();
+    return dflash_attn_block(&p, stream);
+  });
+  return rc != 0 ? fail(rc, "dflash_attn_block") : THPVariable_Wrap(std::move(out));
+  END_HANDLE_TH_ERRORS
+}
+
 // ---- module -----------------------------------------------------------------------------------------------------------
 PyObject* bind(PyObject*, PyObject* error) {  // the class that failed launches raise
   Py_INCREF(error);
@@ -760,7 +825,7 @@ PyObject* bind(PyObject*, PyObject* error) {  // the class that failed launches 
 #define DFLASH_HOST(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
 PyMethodDef kMethods[] = {DFLASH_HOST(qmm_m16), DFLASH_HOST(qmm_packed), DFLASH_HOST(qmm_few), DFLASH_HOST(qmm_few_silu_mul),
                           DFLASH_HOST(qmm_rows), DFLASH_HOST(columns), DFLASH_HOST(gather), DFLASH_HOST(chain_bind), DFLASH_HOST(chain_launch), DFLASH_HOST(gdn_prepare), DFLASH_HOST(gdn_forward), DFLASH_HOST(gdn_block),
-                          DFLASH_HOST(rollback_layer), DFLASH_HOST(rollback_layers), DFLASH_HOST(attn_prepare), DFLASH_HOST(sdpa_q16), {"bind", bind, METH_O, nullptr},
+                          DFLASH_HOST(rollback_layer), DFLASH_HOST(rollback_layers), DFLASH_HOST(attn_prepare), DFLASH_HOST(sdpa_q16), DFLASH_HOST(first_rows), DFLASH_HOST(attn_block), {"bind", bind, METH_O, nullptr},
                           {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_dflash_host", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
 

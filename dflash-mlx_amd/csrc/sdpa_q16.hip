@@ -66,6 +66,25 @@ struct SdpaArgs {
   float scale, lowest;   // lowest finite value of the input dtype
 };
 
+// What stands between the projections and the attention of a block, where the attention's launch does it (BLOCK): queries and
+// keys of the block as the projections gave them, and the cache's rows N - 16 .. N - 1, which are written here.
+struct BlockArgs {
+  const uint16_t *q, *k, *v;  // [B, 16, Hq, 2 D] (queries, gate), [B, 16, Hk, D] twice, through strides (elements)
+  long long q_batch, q_row, k_batch, k_row, v_batch, v_row;
+  const uint16_t *q_weight, *k_weight;  // [D], of the input dtype
+  uint16_t *k_cache, *v_cache;          // where k and v of SdpaArgs begin
+  int half;                             // rotated features / 2: 32, 64 or 128
+  float q_eps, k_eps, base, inv_half;
+};
+template <bool BLOCK>
+struct KernelArgs : SdpaArgs {};
+template <>
+struct KernelArgs<true> : SdpaArgs {
+  BlockArgs block;
+};
+constexpr int kTurnPad = 2;  // pairs between the rows of the table of angles: its rows start 16 bytes apart modulo 128
+constexpr size_t turn_bytes(int half) { return 16 * (size_t)(half + kTurnPad) * sizeof(float2) + half * sizeof(float); }
+
 template <bool FP16>
 __device__ __forceinline__ f32x4_t mfma32(uint4 a, uint4 b, f32x4_t c) {
   if (FP16) {
@@ -93,8 +112,8 @@ __device__ __forceinline__ float elem_to_f32(uint16_t h) {
 // heads per key/value head the output columns are split over CS waves (each repeats the cheap
 // K Q^T) so that a SIMD has more than one wave to switch between.  Every launch has kThreads
 // threads: waves beyond G * CS move tiles only.
-template <int D, bool FP16, int CS, bool MASK>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void sdpa_q16_kernel(SdpaArgs a) {
+template <int D, bool FP16, int CS, bool MASK, bool BLOCK>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void sdpa_q16_kernel(KernelArgs<BLOCK> a) {
   constexpr int kCols = D / 16 / CS;          // 16-column chunks of the output per wave
   constexpr int P = D + kPadElems;            // row pitch of a tile in LDS, elements
   constexpr int kTileElems = kTileKeys * P;   // one K or V tile
@@ -107,7 +126,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
   const int bh = a.ranges.quotient((int)blockIdx.x), split = (int)blockIdx.x - bh * a.splits;
   const int b = a.key_heads.quotient(bh), hk = bh - b * a.Hk;
   const int n_begin = split * a.keys_per_split;
-  const int n_end = n_begin + a.keys_per_split < a.N ? n_begin + a.keys_per_split : a.N;
+  const int cached = BLOCK ? a.N - 16 : a.N;  // (a last range may have none of them)
+  const int n_end = n_begin + a.keys_per_split < cached ? n_begin + a.keys_per_split : cached;
   const int j = lane & 15, kb = lane >> 4;
   const bool computes = wave < a.G * CS;  // the other waves only move tiles
   int slice = 0, of_group = computes ? wave : 0;  // wave / G, wave % G
@@ -154,21 +174,186 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
   // ---- this wave's queries, as the B operand of K Q^T -----------------------------------------
   uint4 qreg[D / 32];
 #pragma unroll
-  for (int s = 0; s < D / 32; ++s)
-    qreg[s] = computes ? *reinterpret_cast<const uint4*>(a.q + qrow * D + 32 * s + 8 * kb) : uint4{0u, 0u, 0u, 0u};
+  for (int s = 0; s < D / 32; ++s) {
+    const uint16_t* from = a.q + qrow * D;
+    if constexpr (BLOCK) from = a.block.q + b * a.block.q_batch + j * a.block.q_row + (size_t)hq * (2 * D);
+    qreg[s] = computes ? *reinterpret_cast<const uint4*>(from + 32 * s + 8 * kb) : uint4{0u, 0u, 0u, 0u};
+  }
   // (asked for ahead of the tiles: loads return in order, and the first product needs these)
+  [[maybe_unused]] uint4 qw[BLOCK ? D / 32 : 1];
+  if constexpr (BLOCK) {
+#pragma unroll
+    for (int s = 0; s < D / 32; ++s) qw[s] = *reinterpret_cast<const uint4*>(a.block.q_weight + 32 * s + 8 * kb);
+  }
 
   fetch(stage0, n_begin);
   fetch(stage1, n_begin + kTileKeys);
+
+  [[maybe_unused]] const bool has_block = BLOCK && split == a.splits - 1;
+  [[maybe_unused]] uint16_t* const block_k = lds + 4 * kTileElems;  // the block's own tile, its upper half zeros
+  [[maybe_unused]] uint16_t* const block_v = block_k + kTileElems;
+  if constexpr (BLOCK) {
+    // Norm and rotation of the queries by the waves that multiply with them, of the block's keys by the last range, which also
+    // writes them to the cache; all while the first tiles are on their way.  A launch of its own for it (attn_prepare_kernel,
+    // whose bits these are) took 4 to 5 us and its place in the queue.  Here every range does it again, bound by its vector
+    // instructions: 1.5 us of a launch with heads of 128, 3.2 of 256 (4.7 with one wave for all of a head's queries and the
+    // powers computed by every thread).  Layer calls, us, before and with it: 4 112 keys of 8 x 256 48.1 -> 46.4, 32 716 89.5 ->
+    // 88.7; of calls that the host bounds (five launches, now four) 8 299 keys of 8 x 128 43.4 -> 36.0, 2 016 of 2 x 256 43.2 -> 35.8.
+    constexpr int PER = D / 64, kRowsPerWave = 16 / (kThreads / 64);
+    const BlockArgs& p = a.block;
+    const int half = p.half, pitch = half + kTurnPad;
+    float2* const turn = reinterpret_cast<float2*>(lds + 6 * kTileElems);  // cosine and sine, [token][pair]
+    float* const frequency = reinterpret_cast<float*>(turn + 16 * pitch);
+    uint32_t k_raw[kRowsPerWave][PER], v_raw[kRowsPerWave][PER], kw_raw[PER];
+    if (has_block) {
+      load_adjacent_raw<PER>(p.k_weight, PER * lane, false, kw_raw);
+#pragma unroll
+      for (int u = 0; u < kRowsPerWave; ++u) {
+        const int row = kRowsPerWave * wave + u;
+        load_adjacent_raw<PER>(p.k + b * p.k_batch + row * p.k_row + (size_t)hk * D, PER * lane, false, k_raw[u]);
+        load_adjacent_raw<PER>(p.v + b * p.v_batch + row * p.v_row + (size_t)hk * D, PER * lane, false, v_raw[u]);
+      }
+    }
+    asm volatile("" ::: "memory");  // on their way before the angles
+    if (tid < half) frequency[tid] = powf(p.base, -(float)tid * p.inv_half);
+    __syncthreads();
+    {
+      const int shift = 31 - __builtin_clz(half), pair = tid & (half - 1);
+      const float f = frequency[pair];
+      for (int row = tid >> shift; row < 16; row += kThreads >> shift) {
+        float2 t;
+        sincosf((float)(a.N - 16 + row) * f, &t.y, &t.x);
+        turn[row * pitch + pair] = t;
+      }
+    }
+    __syncthreads();
+    if (computes) {
+#pragma clang fp contract(off)
+      constexpr int S = D / 32, H = 8 / PER;
+      auto element = [](const uint4& v, int e) __attribute__((always_inline)) {
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+        return elem_to_f32<FP16>((uint16_t)(e & 1 ? w[e >> 1] >> 16 : w[e >> 1]));
+      };
+      // the squares in the order in which a wave that has PER adjacent features a lane adds them up
+      float part[S][H];
+#pragma unroll
+      for (int s = 0; s < S; ++s)
+#pragma unroll
+        for (int h = 0; h < H; ++h) {
+          part[s][h] = 0.f;
+#pragma unroll
+          for (int e = 0; e < PER; ++e) {
+            const float x = element(qreg[s], PER * h + e);
+            part[s][h] += x * x;
+          }
+        }
+#pragma unroll
+      for (int step = S / 2; step >= 1; step /= 2)
+#pragma unroll
+        for (int s = 0; s < step; ++s)
+#pragma unroll
+          for (int h = 0; h < H; ++h) part[s][h] += part[s + step][h];
+#pragma unroll
+      for (int h = 0; h < H; ++h) part[0][h] += __shfl_xor(part[0][h], 32, 64);
+#pragma unroll
+      for (int h = 0; h < H; ++h) part[0][h] += __shfl_xor(part[0][h], 16, 64);
+#pragma unroll
+      for (int step = H / 2; step >= 1; step /= 2)
+#pragma unroll
+        for (int h = 0; h < step; ++h) part[0][h] += part[0][h + step];
+      const float inv_rms = 1.0f / sqrtf(part[0][0] * (1.0f / (float)D) + p.q_eps);
+      // The waves that share a head each take kWords of the four words of every piece, and meet in the second tile's place.
+      constexpr int kWords = 4 / CS;
+      uint32_t mine[S][kWords];
+      auto word = [](const uint4& v, int w) __attribute__((always_inline)) { return w == 0 ? v.x : w == 1 ? v.y : w == 2 ? v.z : v.w; };
+      auto low = [](uint32_t w) __attribute__((always_inline)) { return elem_to_f32<FP16>((uint16_t)w); };
+      auto high = [](uint32_t w) __attribute__((always_inline)) { return elem_to_f32<FP16>((uint16_t)(w >> 16)); };
+#pragma unroll
+      for (int s = 0; s < S; ++s)
+#pragma unroll
+        for (int i = 0; i < kWords; ++i) {
+          uint32_t x = word(qreg[s], i), w = word(qw[s], i);
+#pragma unroll
+          for (int c = 1; c < CS; ++c) {
+            uint32_t other_x = word(qreg[s], kWords * c + i), other_w = word(qw[s], kWords * c + i);
+            asm("" : "+v"(other_x), "+v"(other_w));  // (a choice of values: of addresses, the pieces would go to memory)
+            x = slice == c ? other_x : x, w = slice == c ? other_w : w;
+          }
+          mine[s][i] = pack2<FP16>(low(x) * inv_rms * low(w), high(x) * inv_rms * high(w));
+        }
+      // features i and i + half, in pieces s and s + half / 32 of one lane
+      auto rotate = [&](auto apart) __attribute__((always_inline)) {
+        constexpr int A = decltype(apart)::value;
+        if constexpr (2 * A <= S) {
+#pragma unroll
+          for (int s = 0; s < A; ++s)
+#pragma unroll
+            for (int i = 0; i < kWords; ++i) {
+              // cosine and sine of two pairs
+              const f32x4_t t = *reinterpret_cast<const f32x4_t*>(turn + j * pitch + 32 * s + 8 * kb + 2 * (kWords * slice + i));
+              const uint32_t xw = mine[s][i], yw = mine[s + A][i];
+              const float x0 = low(xw), x1 = high(xw), y0 = low(yw), y1 = high(yw);
+              mine[s][i] = pack2<FP16>(x0 * t[0] - y0 * t[1], x1 * t[2] - y1 * t[3]);
+              mine[s + A][i] = pack2<FP16>(x0 * t[1] + y0 * t[0], x1 * t[3] + y1 * t[2]);
+            }
+        }
+      };
+      if (half == 32) rotate(std::integral_constant<int, 1>{});
+      else if (half == 64) rotate(std::integral_constant<int, 2>{});
+      else rotate(std::integral_constant<int, 4>{});
+      uint32_t* const shared = reinterpret_cast<uint32_t*>(lds + 2 * kTileElems) + (of_group * S * 64 + lane) * 4;
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        if constexpr (CS == 1) qreg[s] = uint4{mine[s][0], mine[s][1 % kWords], mine[s][2 % kWords], mine[s][3 % kWords]};
+        else if constexpr (CS == 2) *reinterpret_cast<uint2*>(shared + 256 * s + 2 * slice) = uint2{mine[s][0], mine[s][1 % kWords]};
+        else shared[256 * s + slice] = mine[s][0];
+      }
+    }
+    if constexpr (CS > 1) {
+      __syncthreads();
+      if (computes) {
+#pragma unroll
+        for (int s = 0; s < D / 32; ++s) qreg[s] = reinterpret_cast<const uint4*>(lds + 2 * kTileElems)[(of_group * (D / 32) + s) * 64 + lane];
+      }
+    }
+    if (has_block) {
+      constexpr int dt = FP16 ? DFLASH_FP16 : DFLASH_BF16;
+      const int c = PER * lane;
+      const bool rotates = c < 2 * half, upper = c >= half;
+      const int other = rotates ? (upper ? lane - half / PER : lane + half / PER) : lane;
+      float w[PER];
+      unpack_adjacent<PER>(kw_raw, dt, w);
+#pragma unroll
+      for (int u = 0; u < kRowsPerWave; ++u) {
+        const int row = kRowsPerWave * wave + u;
+        float x[PER], cs[PER], sn[PER];
+#pragma unroll
+        for (int e = 0; e < PER; ++e) {
+          const float2 t = turn[row * pitch + (rotates ? (upper ? c - half : c) + e : 0)];
+          cs[e] = t.x, sn[e] = t.y;
+        }
+        unpack_adjacent<PER>(k_raw[u], dt, x);
+        norm_and_turn<PER>(x, w, p.k_eps, cs, sn, rotates, upper, other, dt);
+        const long long at = b * a.k_batch_stride + hk * a.k_head_stride + (a.N - 16 + row) * a.k_seq_stride + c;
+        const long long vat = b * a.v_batch_stride + hk * a.v_head_stride + (a.N - 16 + row) * a.v_seq_stride + c;
+        store_adjacent<PER>(p.k_cache, (size_t)at, dt, x);
+        store_adjacent<PER>(block_k, (size_t)(row * P + c), dt, x);
+        store_raw<PER>(p.v_cache + vat, v_raw[u]);
+        store_raw<PER>(block_v + row * P + c, v_raw[u]);
+        const uint32_t zero[PER] = {};
+        store_raw<PER>(block_k + (16 + row) * P + c, zero);
+        store_raw<PER>(block_v + (16 + row) * P + c, zero);
+      }
+    }
+  }
 
   f32x4_t O[kCols];
 #pragma unroll
   for (int c = 0; c < kCols; ++c) O[c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   float m_run = kMasked, l_run = 0.f;  // l_run: this lane's keys only, merged at the end
 
-  auto compute_tile = [&](int buf, int n0) __attribute__((always_inline)) {
+  auto compute_tile = [&](const uint16_t* sk, int n0, int n_end) __attribute__((always_inline)) {
     if (computes) {
-      const uint16_t* sk = lds + buf * 2 * kTileElems;
       const uint16_t* sv = sk + kTileElems;
       // S^T = K Q^T for the two 16-key halves of the tile
       // (all reads of the tile are issued before the first product: one LDS latency, not sixteen)
@@ -245,15 +430,21 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
   for (int n0 = n_begin; n0 < n_end; n0 += 2 * kTileKeys) {
     // even tile in buffer 0; stage 1 holds the next tile, stage 0 is free
     fetch(stage0, n0 + 2 * kTileKeys);
-    compute_tile(0, n0);
+    compute_tile(lds, n0, n_end);
     stash(stage1, 1);
     __syncthreads();
     if (n0 + kTileKeys >= n_end) break;
     // odd tile in buffer 1; stage 0 holds the next tile, stage 1 is free
     fetch(stage1, n0 + 3 * kTileKeys);
-    compute_tile(1, n0 + kTileKeys);
+    compute_tile(lds + 2 * kTileElems, n0 + kTileKeys, n_end);
     stash(stage0, 0);
     __syncthreads();
+  }
+  if constexpr (BLOCK) {
+    if (has_block) {
+      __syncthreads();  // (a range without cached keys has met nowhere since the block's tile was written)
+      compute_tile(block_k, a.N - 16, a.N);
+    }
   }
 
   if (!computes) return;
@@ -375,6 +566,7 @@ __global__ __launch_bounds__(256) void sdpa_q16_merge_kernel(SdpaArgs a, int D) 
   }
 }
 
+// keys: that the ranges are to share.
 int pick_splits(int B, int Hk, int N, int* keys_per_split) {
   // About one workgroup per compute unit, and never less than 128 keys per split: every split
   // adds B * Hq * 16 * (2 D + 8) bytes of partial results, written once and read once.
@@ -391,6 +583,14 @@ int pick_splits(int B, int Hk, int N, int* keys_per_split) {
   return (N + per - 1) / per;  // no empty split
 }
 
+// A block that its launch prepares: the last range has these keys fewer than the others, for the block's own tile and for
+// what stands before it.
+constexpr int kBlockKeys = 48;
+
+size_t partial_bytes(int splits, int B, int Hq, int D) {
+  return splits == 1 ? 0 : (size_t)splits * B * Hq * 16 * (D * sizeof(uint16_t) + 2 * sizeof(float));
+}
+
 }  // namespace
 }  // namespace dflash
 
@@ -398,9 +598,14 @@ extern "C" size_t dflash_sdpa_q16_workspace_bytes(int B, int Hq, int Hk, int N, 
   using namespace dflash;
   if (B <= 0 || Hq <= 0 || Hk <= 0 || N <= 0 || D <= 0) return 0;
   int per = 0;
-  const int splits = pick_splits(B, Hk, N, &per);
-  if (splits == 1) return 0;
-  return (size_t)splits * B * Hq * 16 * (D * sizeof(uint16_t) + 2 * sizeof(float));
+  return partial_bytes(pick_splits(B, Hk, N, &per), B, Hq, D);
+}
+
+extern "C" size_t dflash_attn_block_workspace_bytes(int B, int Hq, int Hk, int N, int D) {
+  using namespace dflash;
+  if (B <= 0 || Hq <= 0 || Hk <= 0 || N <= 16 || D <= 0) return 0;
+  int per = 0;
+  return partial_bytes(pick_splits(B, Hk, N - 16 + kBlockKeys, &per), B, Hq, D);
 }
 
 namespace dflash {
@@ -409,7 +614,8 @@ int sdpa_launch(const void* q, const void* k, const void* v, const void* mask, c
                 void* workspace, size_t workspace_bytes, int B, int Hq, int Hk, int N, int D,
                 long long k_batch_stride, long long k_head_stride, long long k_seq_stride,
                 long long v_batch_stride, long long v_head_stride, long long v_seq_stride,
-                long long gate_batch_stride, long long gate_row_stride, float scale, int dtype, void* stream) {
+                long long gate_batch_stride, long long gate_row_stride, float scale, int dtype, void* stream,
+                const BlockArgs* block = nullptr) {
   DFLASH_REQUIRE(q && k && v && out, DFLASH_ERR_ARG, "dflash_sdpa_q16: null operand");
   DFLASH_REQUIRE(dtype == DFLASH_BF16 || dtype == DFLASH_FP16, DFLASH_ERR_ARG,
                  "dflash_sdpa_q16: bf16 or fp16 only");
@@ -426,13 +632,14 @@ int sdpa_launch(const void* q, const void* k, const void* v, const void* mask, c
   DFLASH_REQUIRE((long long)B * Hq * 16 < (1ll << 31) && (long long)B * Hk * ((N + 127) / 128) < (1ll << 31),
                  DFLASH_ERR_SHAPE, "dflash_sdpa_q16: too many rows");
 
-  SdpaArgs a;
+  KernelArgs<true> a;
   a.q = (const uint16_t*)q; a.k = (const uint16_t*)k; a.v = (const uint16_t*)v; a.mask = (const uint16_t*)mask;
   a.out = (uint16_t*)out;
   a.k_batch_stride = k_batch_stride; a.k_head_stride = k_head_stride; a.k_seq_stride = k_seq_stride;
   a.v_batch_stride = v_batch_stride; a.v_head_stride = v_head_stride; a.v_seq_stride = v_seq_stride;
   a.B = B; a.Hq = Hq; a.Hk = Hk; a.N = N; a.G = Hq / Hk;
-  a.splits = pick_splits(B, Hk, N, &a.keys_per_split);
+  a.splits = pick_splits(B, Hk, block ? N - 16 + kBlockKeys : N, &a.keys_per_split);
+  if (block) a.block = *block;
   a.ranges = Divisor::of(a.splits); a.key_heads = Divisor::of(Hk); a.heads = Divisor::of(Hq);
   a.scale = scale;
   a.lowest = dtype == DFLASH_FP16 ? -65504.0f : -3.3895313892515355e38f;
@@ -442,7 +649,7 @@ int sdpa_launch(const void* q, const void* k, const void* v, const void* mask, c
   a.part_o = nullptr;
   a.part_ml = nullptr;
   if (a.splits > 1) {
-    const size_t need = (size_t)a.splits * B * Hq * 16 * (D * sizeof(uint16_t) + 2 * sizeof(float));
+    const size_t need = partial_bytes(a.splits, B, Hq, D);
     DFLASH_REQUIRE(workspace && workspace_bytes >= need && ((uintptr_t)workspace % 16) == 0, DFLASH_ERR_WORKSPACE,
                    "dflash_sdpa_q16: workspace of %zu bytes needed, %zu given", need,
                    workspace ? workspace_bytes : (size_t)0);
@@ -453,37 +660,40 @@ int sdpa_launch(const void* q, const void* k, const void* v, const void* mask, c
   hipStream_t s = (hipStream_t)stream;
   // column split: as many waves as fit eight, in powers of two
   const int cs = a.G <= 2 ? 4 : a.G <= 4 ? 2 : 1;
-  const size_t lds_bytes = (size_t)2 * 2 * kTileKeys * (D + kPadElems) * sizeof(uint16_t);
+  const int tiles = block ? 6 : 4;
+  const size_t lds_bytes = (size_t)tiles * kTileKeys * (D + kPadElems) * sizeof(uint16_t) +
+                           (block ? turn_bytes(block->half) : 0);
+  const size_t lds_most = (size_t)tiles * kTileKeys * (D + kPadElems) * sizeof(uint16_t) +
+                          (block ? turn_bytes(D / 2) : 0);
   const bool f16 = dtype == DFLASH_FP16;
-#define DFLASH_SDPA_ROW(D_, F_, M_)                                                                      \
-  {(const void*)sdpa_q16_kernel<D_, F_, 1, M_>, (const void*)sdpa_q16_kernel<D_, F_, 2, M_>, \
-   (const void*)sdpa_q16_kernel<D_, F_, 4, M_>}
-  const void* table[2][2][2][3] = {
-      {{DFLASH_SDPA_ROW(128, false, false), DFLASH_SDPA_ROW(128, false, true)},
-       {DFLASH_SDPA_ROW(128, true, false), DFLASH_SDPA_ROW(128, true, true)}},
-      {{DFLASH_SDPA_ROW(256, false, false), DFLASH_SDPA_ROW(256, false, true)},
-       {DFLASH_SDPA_ROW(256, true, false), DFLASH_SDPA_ROW(256, true, true)}}};
+#define DFLASH_SDPA_ROW(D_, F_, M_, B_)                                                                        \
+  {(const void*)sdpa_q16_kernel<D_, F_, 1, M_, B_>, (const void*)sdpa_q16_kernel<D_, F_, 2, M_, B_>, \
+   (const void*)sdpa_q16_kernel<D_, F_, 4, M_, B_>}
+#define DFLASH_SDPA_FORMS(D_, F_) {DFLASH_SDPA_ROW(D_, F_, false, false), DFLASH_SDPA_ROW(D_, F_, true, false), DFLASH_SDPA_ROW(D_, F_, false, true)}
+  static const void* const table[2][2][3][3] = {{DFLASH_SDPA_FORMS(128, false), DFLASH_SDPA_FORMS(128, true)},
+                                                {DFLASH_SDPA_FORMS(256, false), DFLASH_SDPA_FORMS(256, true)}};
+#undef DFLASH_SDPA_FORMS
 #undef DFLASH_SDPA_ROW
-  const bool masked = mask != nullptr;
+  const int form = block ? 2 : mask != nullptr ? 1 : 0;
   const int ics = cs == 1 ? 0 : cs == 2 ? 1 : 2;
   void* args[] = {&a};
   const int slot = current_device_slot();
   {
-    const void* fn = table[D == 256][f16][masked][ics];
+    const void* fn = table[D == 256][f16][form][ics];
     // the attribute belongs to the device's copy of the kernel: once per device and kernel
-    static bool attr_set[kMaxDevices][24] = {};
-    const int idx = (((D == 256) * 2 + f16) * 2 + masked) * 3 + ics;
-    if (!attr_set[slot][idx] || slot == kMaxDevices - 1) {
-      DFLASH_HIP_OK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
-      attr_set[slot][idx] = true;
+    static bool attr_set[kMaxDevices][2][2][3][3] = {};
+    bool& set = attr_set[slot][D == 256][f16][form][ics];
+    if (!set || slot == kMaxDevices - 1) {
+      DFLASH_HIP_OK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_most));
+      set = true;
     }
     DFLASH_HIP_OK(hipLaunchKernel(fn, dim3((unsigned)(B * Hk * a.splits)), dim3(kThreads), args, lds_bytes, s));
   }
   if (a.splits > 1) {
     if (dtype == DFLASH_FP16) {
-      hipLaunchKernelGGL(sdpa_q16_merge_kernel<true>, dim3((unsigned)(B * Hq * 16)), dim3(256), 0, s, a, D);
+      hipLaunchKernelGGL(sdpa_q16_merge_kernel<true>, dim3((unsigned)(B * Hq * 16)), dim3(256), 0, s, (const SdpaArgs&)a, D);
     } else {
-      hipLaunchKernelGGL(sdpa_q16_merge_kernel<false>, dim3((unsigned)(B * Hq * 16)), dim3(256), 0, s, a, D);
+      hipLaunchKernelGGL(sdpa_q16_merge_kernel<false>, dim3((unsigned)(B * Hq * 16)), dim3(256), 0, s, (const SdpaArgs&)a, D);
     }
     DFLASH_HIP_OK(hipGetLastError());
   }
@@ -517,4 +727,31 @@ extern "C" int dflash_sdpa_q16_gated(const void* q, const void* k, const void* v
   return sdpa_launch(q, k, v, mask, gate, out, workspace, workspace_bytes, B, Hq, Hk, N, D, k_batch_stride, k_head_stride,
                      k_seq_stride, v_batch_stride, v_head_stride, v_seq_stride, gate_batch_stride, gate_row_stride, scale, dtype,
                      stream);
+}
+
+extern "C" int dflash_attn_block(const dflash_attn_block_args* args, void* stream) {
+  using namespace dflash;
+  DFLASH_REQUIRE(args, DFLASH_ERR_ARG, "dflash_attn_block: null arguments");
+  const dflash_attn_block_args& p = *args;
+  DFLASH_REQUIRE(p.q && p.k && p.v && p.q_weight && p.k_weight && p.k_cache && p.v_cache && p.out, DFLASH_ERR_ARG, "dflash_attn_block: null operand");
+  DFLASH_REQUIRE(p.N > 16, DFLASH_ERR_SHAPE, "dflash_attn_block: no keys before the block (N %d)", p.N);
+  DFLASH_REQUIRE(p.rope_dims == 64 || p.rope_dims == 128 || (p.rope_dims == 256 && p.D == 256), DFLASH_ERR_SHAPE,
+                 "dflash_attn_block: %d rotated features of %d (64, 128 or 256)", p.rope_dims, p.D);
+  const long long rows[] = {p.q_batch, p.q_row, p.k_batch, p.k_row, p.v_batch, p.v_row};
+  uintptr_t bits = (uintptr_t)p.q | (uintptr_t)p.k | (uintptr_t)p.v | (uintptr_t)p.q_weight | (uintptr_t)p.k_weight;
+  for (long long r : rows) {
+    DFLASH_REQUIRE(r >= 0, DFLASH_ERR_SHAPE, "dflash_attn_block: negative stride");
+    bits |= (uintptr_t)r * 2;
+  }
+  DFLASH_REQUIRE(bits % 16 == 0, DFLASH_ERR_ARG, "dflash_attn_block: operands and rows must be 16-byte aligned");
+  BlockArgs b;
+  b.q = (const uint16_t*)p.q; b.k = (const uint16_t*)p.k; b.v = (const uint16_t*)p.v;
+  b.q_batch = p.q_batch; b.q_row = p.q_row; b.k_batch = p.k_batch; b.k_row = p.k_row; b.v_batch = p.v_batch; b.v_row = p.v_row;
+  b.q_weight = (const uint16_t*)p.q_weight; b.k_weight = (const uint16_t*)p.k_weight;
+  b.k_cache = (uint16_t*)p.k_cache; b.v_cache = (uint16_t*)p.v_cache;
+  b.half = p.rope_dims / 2;
+  b.q_eps = p.q_eps; b.k_eps = p.k_eps; b.base = p.rope_base; b.inv_half = 1.0f / (float)b.half;
+  return sdpa_launch(p.q, p.k_cache, p.v_cache, nullptr, p.q, p.out, p.workspace, p.workspace_bytes, p.B, p.Hq, p.Hk, p.N, p.D,
+                     p.k_cache_batch, p.k_cache_head, p.k_cache_row, p.v_cache_batch, p.v_cache_head, p.v_cache_row, p.q_batch,
+                     p.q_row, p.scale, p.dtype, stream, &b);
 }

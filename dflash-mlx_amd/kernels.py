@@ -359,8 +359,8 @@ def _sdpa_workspace(device: torch.device, nbytes: int) -> torch.Tensor:
 
 
 def batched_sdpa_2pass_exact(queries: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, scale: float,
-                             mask: Optional[torch.Tensor] = None, *,
-                             q_proj_output: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+                             mask: Optional[torch.Tensor] = None, *, q_proj_output: Optional[torch.Tensor] = None,
+                             unprepared: Optional[tuple] = None) -> Optional[torch.Tensor]:
     """Exact attention of a 16-token verify block over a long KV cache (mirror of
     dflash_mlx/kernels.py:658-761): queries [B,Hq,16,D], keys / values [B,Hk,N,D] (views of a
     cache are read in place), mask None, bool or additive, broadcastable to [B,Hq,16,N].
@@ -371,7 +371,23 @@ def batched_sdpa_2pass_exact(queries: torch.Tensor, keys: torch.Tensor, values: 
 
     ``q_proj_output`` [B,16,Hq*2D] (no counterpart in the reference, which gates with array operators): the result is
     [B,16,Hq*D], every head times the sigmoid of the second half of its part of q_proj_output, where the same launch can do
-    it; where it cannot (one range of keys), the plain result."""
+    it; where it cannot (one range of keys), the plain result.
+
+    ``unprepared`` (likewise): ``(keys, values, q weight, k weight, rope_dims, q eps, k eps, rope base)`` of a block that is as
+    the projections left it, with ``queries`` None, no mask and ``q_proj_output`` [B,16,Hq*2D]: head norms, rotation and the
+    block's rows, the last 16 of the cache's keys and values, are made by the launch as well.  None, and nothing done,
+    where there is no such launch."""
+    if unprepared is not None:
+        call = (q_proj_output, *unprepared[:4], keys, values, *unprepared[4:], float(scale), _SDPA_WORKSPACE)
+        out = _native.host().attn_block(*call)
+        if out is None and keys.is_cuda and q_proj_output.ndim == 3:
+            bsz, hk, n_kv, d = (int(x) for x in keys.shape)
+            need = int(_native.lib().dflash_attn_block_workspace_bytes(bsz, int(q_proj_output.shape[2]) // (2 * d), hk, n_kv, d))
+            held = _SDPA_WORKSPACE.get((keys.device, _native.raw_stream(keys.device)))
+            if need and (held is None or held.numel() < need):
+                _sdpa_workspace(keys.device, need)
+                out = _native.host().attn_block(*call)
+        return out
     if mask is None and queries.is_cuda:
         out = _native.host().sdpa_q16(queries, keys, values, float(scale), q_proj_output, _SDPA_WORKSPACE)
         if out is not None:

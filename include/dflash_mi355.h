@@ -558,6 +558,26 @@ int dflash_sdpa_q16_gated(const void* q, const void* k, const void* v, const voi
                           long long gate_batch_stride, long long gate_row_stride, float scale, int dtype, void* stream);
 
 /*
+ * dflash_attn_prepare and dflash_sdpa_q16_gated of a block of 16 tokens behind N - 16 cached ones, without a mask, in the
+ * launches of the attention alone: q [B, 16, Hq, 2 D] (a head's queries, then its gate), k, v [B, 16, Hk, D] as the projections
+ * gave them, through strides (elements); k_cache, v_cache [B, Hk, N.., D] through strides, rows N - 16 .. N - 1 of them written
+ * here with the bits that dflash_attn_prepare leaves; out [B, 16, Hq, D].
+ * D 128 or 256, rope_dims 64, 128 or 256; norm weights of the activations' dtype; q, k, v, their rows and the weights 16-byte
+ * aligned; more than one range of keys (a workspace size of 0: there is no form).  workspace as for dflash_sdpa_q16.
+ */
+typedef struct dflash_attn_block_args {
+  const void *q, *k, *v, *q_weight, *k_weight;
+  void *k_cache, *v_cache, *out, *workspace;
+  size_t workspace_bytes;
+  long long q_batch, q_row, k_batch, k_row, v_batch, v_row;
+  long long k_cache_batch, k_cache_head, k_cache_row, v_cache_batch, v_cache_head, v_cache_row;
+  int B, Hq, Hk, N, D, rope_dims, dtype;
+  float q_eps, k_eps, rope_base, scale;
+} dflash_attn_block_args;
+size_t dflash_attn_block_workspace_bytes(int B, int Hq, int Hk, int N, int D);
+int dflash_attn_block(const dflash_attn_block_args* args, void* stream);
+
+/*
  * Conv-window rebuild of a GatedDeltaNet layer after a partial acceptance: output
  * row j of a slot is row steps+j of concat([conv_prev, qkv], axis=rows).  Replaces the
  * array ops of dflash_mlx/recurrent_rollback_cache.py:129-146 (zeros stand in for a

@@ -210,3 +210,95 @@ def test_both_gates_on_every_number(dtype):
     want = A._finish(attn, batched_sdpa_2pass_exact(q, k, v, D ** -0.5), projected)
     nan = torch.isnan(want)
     assert torch.equal(torch.isnan(gated), nan) and torch.equal(gated[~nan], want[~nan])
+
+
+def _block_layer(*args):
+    """A layer whose verify blocks take the exact path behind any prefix."""
+    attn, outs = _layer(*args)
+    attn.q_proj.weight = torch.empty((outs[0].shape[-1], 1), device="cuda")  # (its height says that a gate rides along)
+    A.configure_full_attention_split([type("L", (), {"is_linear": False, "self_attn": attn})()], enabled=True)
+    attn._dflash_split_sdpa_exact_kv_threshold = 1
+    return attn, outs
+
+
+@pytest.mark.parametrize("B,Hq,Hk,D,dims,prefix,dtype,joint", [
+    (1, 32, 8, 256, 256, 4096, torch.bfloat16, True),
+    (1, 16, 2, 128, 128, 1025, torch.float16, True),    # eight heads of a key head, an odd prefix
+    (2, 3, 1, 128, 64, 1039, torch.bfloat16, False),    # three heads, half of the features turned
+    (1, 4, 4, 256, 64, 130, torch.float16, False),      # waves share a head four ways
+    (1, 6, 2, 256, 128, 90, torch.bfloat16, True),      # two ranges, the last one without a cached key
+    (1, 4, 2, 128, 128, 112, torch.bfloat16, True),     # ... with one tile of them
+])
+def test_block_from_its_projections_in_the_launch_of_its_attention(monkeypatch, B, Hq, Hk, D, dims, prefix, dtype, joint):
+    """Against the launch of its own for norms, rotation and cache rows: the same rows in the cache, an attention that is as
+    close to 64 bits as that one's."""
+    gen = torch.Generator(device="cuda").manual_seed(21)
+    attn, outs = _block_layer(B, 16, Hq, Hk, D, dims, dtype, dtype, gen, joint)
+    x = torch.empty((B, 16, 8), device="cuda")
+    before = [torch.randn((B, Hk, prefix, D), generator=gen, device="cuda").to(dtype) for _ in range(2)]
+    fused, real = [], A._native.host().attn_block
+    results = []
+    for in_one in (True, False):
+        if not in_one:
+            monkeypatch.setattr(A, "_attend_in_one", lambda *a: None)
+        else:
+            spy = type("H", (), {"__getattr__": lambda self, n, h=A._native.host(): getattr(h, n),
+                                 "attn_block": lambda self, *a: fused.append(real(*a)) or fused[-1]})()
+            monkeypatch.setattr(A._native, "host", lambda: spy)
+        cache = KVCache()
+        cache.update_and_fetch(*before)
+        if cache.keys.shape[2] < prefix + 16:
+            cache._make_room(B, Hk, 16, D, D, *before)
+        y = attn(x, mask="causal" if in_one else None, cache=cache)
+        assert cache.offset == prefix + 16
+        results.append((y, *cache.state))
+    assert fused and fused[-1] is not None
+    (got, keys, values), (ref, ref_keys, ref_values) = results
+    assert torch.equal(keys, ref_keys) and torch.equal(values, ref_values)
+    q = A.rms_norm_ops(outs[0].reshape(B, 16, Hq, 2 * D)[..., :D], attn.q_norm.weight, attn.q_norm.eps).transpose(1, 2)
+    q = attn.rope(q, offset=prefix).double()
+    k, v = (t.double().repeat_interleave(Hq // Hk, dim=1) for t in (ref_keys, ref_values))
+    scores = torch.matmul(q, k.transpose(2, 3).contiguous()) * attn.scale
+    late = torch.arange(prefix + 16, device="cuda") > prefix + torch.arange(16, device="cuda")[:, None]
+    o = torch.matmul(torch.softmax(scores.masked_fill(late, float("-inf")), dim=-1), v).transpose(1, 2)
+    exact = (o * torch.sigmoid(outs[0].reshape(B, 16, Hq, 2 * D)[..., D:].double())).reshape(B, 16, Hq * D)
+    err = [((t.double() - exact).norm() / exact.norm()).item() for t in (got, ref)]
+    # (partial outputs, the output, the gate and their product are rounded to the type, each by eps / sqrt(48) on average, and other
+    # ranges of keys have other partial outputs)
+    assert err[0] <= max(1.1 * err[1], 4 * torch.finfo(dtype).eps / 48 ** 0.5), err
+
+
+def test_what_the_block_launch_does_not_cover_takes_the_launch_of_its_own(monkeypatch):
+    """One range of keys, a rotation of 96 features, weights of another type, rows at odd addresses, a mask, no room."""
+    for change in ("short", "rotation", "weights", "address", "mask", "room", "none"):
+        gen = torch.Generator(device="cuda").manual_seed(22)
+        prefix = 50 if change == "short" else 240 if change != "room" else 250
+        attn, outs = _block_layer(1, 16, 4, 2, 128, 96 if change == "rotation" else 128, torch.bfloat16,
+                                  torch.float32 if change == "weights" else torch.bfloat16, gen, True)
+        if change == "address":
+            attn.k_proj.out = torch.empty(16 * 256 + 4, dtype=torch.bfloat16, device="cuda")[4:].view(1, 16, 256).copy_(outs[1])
+        cache = KVCache()
+        cache.update_and_fetch(*(torch.randn((1, 2, prefix, 128), generator=gen, device="cuda").to(torch.bfloat16) for _ in range(2)))
+        took = []
+        real = A._attend_in_one
+        with monkeypatch.context() as m:
+            m.setattr(A, "_attend_in_one", lambda *a: took.append(real(*a)) or took[-1])
+            mask = torch.zeros((1, 1, 16, prefix + 16), dtype=torch.bfloat16, device="cuda") if change == "mask" else "causal"
+            y = attn(torch.empty((1, 16, 8), device="cuda"), mask=mask, cache=cache)
+        assert y.shape == (1, 16, 4 * 128) and cache.offset == prefix + 16
+        assert (not took or took[-1] is None) == (change != "none"), change
+
+
+def test_a_refused_block_launch_leaves_the_cache_where_it_was(monkeypatch):
+    gen = torch.Generator(device="cuda").manual_seed(23)
+    attn, _ = _block_layer(1, 16, 4, 2, 128, 128, torch.bfloat16, torch.bfloat16, gen, True)
+    cache = KVCache()
+    cache.update_and_fetch(*(torch.zeros((1, 2, 240, 128), dtype=torch.bfloat16, device="cuda") for _ in range(2)))
+
+    def refused(**kw):
+        raise A._native.NativeLibraryError("refused")
+
+    monkeypatch.setattr(A, "batched_sdpa_2pass_exact", refused)
+    with pytest.raises(A._native.NativeLibraryError):
+        attn(torch.empty((1, 16, 8), device="cuda"), mask="causal", cache=cache)
+    assert cache.offset == 240

@@ -250,7 +250,8 @@ def test_host_tensors_and_strangers_are_left_alone(native_lib):
     host, x = nat.host(), torch.zeros(16, 64)
     for name, count in (("qmm_m16", 7), ("qmm_packed", 9), ("qmm_few", 7), ("qmm_few_silu_mul", 7), ("qmm_rows", 7), ("columns", 2),
                         ("gather", 8), ("chain_bind", 4), ("chain_launch", 10), ("gdn_prepare", 13), ("gdn_forward", 10),
-                        ("rollback_layer", 9), ("rollback_layers", 4), ("sdpa_q16", 6), ("attn_prepare", 11)):
+                        ("rollback_layer", 9), ("rollback_layers", 4), ("sdpa_q16", 6), ("attn_prepare", 11), ("first_rows", 3),
+                        ("attn_block", 13)):
         for value in (x, x.to("meta"), None, 1, -1, 2 ** 70, 1.5, "x", {}):
             assert getattr(host, name)(*[value] * count) is None
         assert getattr(host, name)() is None
