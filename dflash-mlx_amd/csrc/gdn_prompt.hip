@@ -9,7 +9,7 @@
 //     S^T   = c_T S0^T + K^T diag(c_T/c_s) Delta,
 // a chunk needs the state only in two products with it and one update of it.
 //
-//  * gdn_chunk_kernel, one wave per (slot, chunk, head), computes what does not depend on the state: M' and
+//  * gdn_chunk_kernel, four waves per (slot, chunk, head), computes what does not depend on the state: M' and
 //    Lq, in the register order the other kernel multiplies them in, and K^T likewise.  All chunks at once.
 //  * gdn_prompt_kernel, one workgroup per (slot, head, 16 rows of the state), walks the chunks.  Rows of S are
 //    independent, so 32 heads of 128 x 128 fill 256 compute units with one workgroup each, and what bounds
@@ -31,7 +31,7 @@
 //    token holds never enters a product: its rows of K and Q are zeros, its element of V - c U as well.
 // A 16-bit state is carried in fp32 and rounded once, at the end.
 //
-// Measured, 1024 tokens, 16 / 32 heads of 128 x 128: 15 + 51 us (64 with one wave per 16 rows), against 123.7 ms with one
+// Measured, 1024 tokens, 16 / 32 heads of 128 x 128: 12.5 + 51 us (64 with one wave per 16 rows), against 123.7 ms with one
 // workgroup per head that kept S in memory (the step-by-step kernel held 41 tokens at most); 678 tokens of 16 heads both kernels
 // 46 us (55).  What the second kernel is bound by is its chain.  One wave: 4560 cycles (2 us) per chunk by its counters, 605
 // vector instructions (53 %), 96 matrix instructions (34 %; 72 of them with S), waits 16 %.  Four: 3500 cycles, 315 vector and
@@ -41,6 +41,8 @@
 // of depth 32 in the update is filled; 64 would need more registers than a wave has.  The look for numbers that are not
 // finite costs 0.3 % of a layer call, a chunk token by token what 32 steps of one wave cost.
 #include "gdn_device.h"
+
+#include <type_traits>
 
 namespace dflash {
 namespace prompt {
@@ -95,26 +97,33 @@ __device__ __forceinline__ size_t chunk_bytes(const Args& a) {
   return (size_t)a.Hv * kHeadBytes + (size_t)a.Hk * (kChunk * DK * 2);
 }
 
+// Four waves on a chunk of a head.  What bounds a call of few chunks is the chain of one: a wave by itself took 12 us, its products, the 32
+// steps of the ratios, 32 of the inverse and K^T out of LDS one after the other.  Here the products of K with K and Q are divided,
+// two waves make the entries of 16 tokens each while the other two turn K, and the inverse is one of two 16 x 16 triangles side by
+// side with the block below them from two products: X21 = -X22 (L21 X11).  One wave and four, us: 100 tokens of 32 heads of 128 12.6
+// and 7.2, 300 of 48 13.6 and 8.4, 1024 of 32 16.2 and 12.5 (33 MB in and out), 900 of 64 20 and 20.
 template <int DK>
-__global__ __launch_bounds__(64, 3) void gdn_chunk_kernel(Args a) {
+__global__ __launch_bounds__(256) void gdn_chunk_kernel(Args a) {
   constexpr int NC = DK / 32;
   constexpr int kKRow = DK + 8;  // 16-bit elements per row of K in LDS
   __shared__ __align__(16) float sA[kChunk * kPitch];  // k_s . k_t, then L, then M'
   __shared__ __align__(16) float sB[kChunk * kPitch];  // k_s . q_t, then Lq
+  __shared__ __align__(16) float sX[kChunk * kPitch];  // the two triangles' inverses
   __shared__ __align__(16) uint16_t sK[kChunk * kKRow];
-  __shared__ float sGate[kChunk], sBeta[kChunk];
+  __shared__ __align__(16) float sGate[kChunk], sBeta[kChunk];
+  __shared__ int sFinite[4];
 
   const int hv = blockIdx.x % a.Hv, rest = blockIdx.x / a.Hv;
   const int chunk = rest % a.chunks, slot = rest / a.chunks;
   const int per = a.Hv / a.Hk, hk = hv / per;
   const bool writes_k = hv % per == 0;
-  const int lane = threadIdx.x, li = lane & 15, kq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, li = lane & 15, kq = lane >> 4;
   const int t0 = chunk * kChunk;
   const size_t slotT = (size_t)slot * a.T;
 
-  uint4 kf[2][NC], qf[2][NC];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
+  // Rows 16 i + li of K or Q; those of masked and missing tokens are zeros.
+  auto load_rows = [&](const uint16_t* from, int i, uint4 (&f)[NC]) __attribute__((always_inline)) {
     int t = t0 + 16 * i + li;
     const bool past = t >= a.T;
     t = past ? a.T - 1 : t;
@@ -122,85 +131,139 @@ __global__ __launch_bounds__(64, 3) void gdn_chunk_kernel(Args a) {
     const bool on = !past && (a.mask == nullptr || a.mask[slotT + t] != 0);
 #pragma unroll
     for (int C = 0; C < NC; ++C) {
-      kf[i][C] = *reinterpret_cast<const uint4*>(a.k + row + 32 * C);
-      qf[i][C] = *reinterpret_cast<const uint4*>(a.q + row + 32 * C);
-      if (!on) kf[i][C] = qf[i][C] = uint4{0u, 0u, 0u, 0u};
+      f[C] = *reinterpret_cast<const uint4*>(from + row + 32 * C);
+      if (!on) f[C] = uint4{0u, 0u, 0u, 0u};
+    }
+  };
+  float finite = 0.f;  // stays zero
+  // rows s = 16 ts + 4 kq + r, column t = 16 tt + li (with the diagonals k . k and k . q among them: nothing that is not finite in K or Q
+  // stays unseen)
+  auto product = [&](const uint4 (&left)[NC], const uint4 (&right)[NC], int ts, int tt, float* to) __attribute__((always_inline)) {
+    f32x4_t x = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int C = 0; C < NC; ++C) x = mfma(left[C], right[C], x);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) finite = fmaf(x[e], 0.f, finite);
+    *reinterpret_cast<f32x4_t*>(to + (16 * tt + li) * kPitch + 16 * ts + 4 * kq) = x;
+  };
+  uint32_t on_bits = 0;
+  {  // (every wave has the bits, the last one the gates)
+    const int t = t0 + (lane & 31);
+    const bool on = t < a.T && (a.mask == nullptr || a.mask[slotT + t] != 0);
+    on_bits = (uint32_t)__ballot(on);
+    if (wave == 3) {
+      const size_t at = (slotT + (t < a.T ? t : a.T - 1)) * a.Hv + hv;
+      float g = load_as_f32(a.g, at, a.g_dtype), beta = load_as_f32(a.beta, at, a.beta_dtype);
+      g = on ? g : 1.f, beta = on ? beta : 0.f;
+      if (lane < kChunk) sGate[lane] = g, sBeta[lane] = beta;
+      finite = fmaf(g, 0.f, beta * 0.f);
     }
   }
-  float finite = 0.f;  // stays zero
-  float on_v = 0.f;
-  if (lane < kChunk) {
-    const int t = t0 + lane;
-    const bool on = t < a.T && (a.mask == nullptr || a.mask[slotT + t] != 0);
-    const size_t at = (slotT + (t < a.T ? t : a.T - 1)) * a.Hv + hv;
-    const float g = on ? load_as_f32(a.g, at, a.g_dtype) : 1.f, beta = on ? load_as_f32(a.beta, at, a.beta_dtype) : 0.f;
-    sGate[lane] = g;
-    sBeta[lane] = beta;
-    finite = fmaf(g, 0.f, beta * 0.f);
-    on_v = on ? 1.f : 0.f;
-  }
-  if (writes_k) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int C = 0; C < NC; ++C) *reinterpret_cast<uint4*>(sK + (16 * i + li) * kKRow + 32 * C + 8 * kq) = kf[i][C];
-  }
-#pragma unroll
-  for (int ts = 0; ts < 2; ++ts)
-#pragma unroll
-    for (int tt = ts; tt < 2; ++tt) {
-      f32x4_t x1 = {0.f, 0.f, 0.f, 0.f}, x2 = x1;  // rows s = 16 ts + 4 kq + r, column t = 16 tt + li
+  {
+    uint4 f0[NC], f1[NC], f2[NC];
+    if (wave == 0) {
+      load_rows(a.k, 0, f0), load_rows(a.k, 1, f1);
+      product(f0, f0, 0, 0, sA), product(f0, f1, 0, 1, sA);
+    } else if (wave == 1) {
+      load_rows(a.k, 1, f0), load_rows(a.q, 1, f1);
+      product(f0, f0, 1, 1, sA), product(f0, f1, 1, 1, sB);
+    } else if (wave == 2) {
+      load_rows(a.k, 0, f0), load_rows(a.q, 0, f1), load_rows(a.q, 1, f2);
+      product(f0, f1, 0, 0, sB), product(f0, f2, 0, 1, sB);
+    } else if (writes_k) {
+      load_rows(a.k, 0, f0), load_rows(a.k, 1, f1);
 #pragma unroll
       for (int C = 0; C < NC; ++C) {
-        x1 = mfma(kf[ts][C], kf[tt][C], x1);
-        x2 = mfma(kf[ts][C], qf[tt][C], x2);
+        *reinterpret_cast<uint4*>(sK + li * kKRow + 32 * C + 8 * kq) = f0[C];
+        *reinterpret_cast<uint4*>(sK + (16 + li) * kKRow + 32 * C + 8 * kq) = f1[C];
       }
-      // (with the diagonals k . k and k . q among them: nothing that is not finite in K or Q stays unseen)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) finite = fmaf(x1[e], 0.f, fmaf(x2[e], 0.f, finite));
-      *reinterpret_cast<f32x4_t*>(sA + (16 * tt + li) * kPitch + 16 * ts + 4 * kq) = x1;
-      *reinterpret_cast<f32x4_t*>(sB + (16 * tt + li) * kPitch + 16 * ts + 4 * kq) = x2;
     }
+  }
   __syncthreads();
-  char* const out = a.work + ((size_t)slot * a.chunks + chunk) * chunk_bytes<DK>(a) + (size_t)hv * kHeadBytes;
+  const size_t here = ((size_t)slot * a.chunks + chunk) * chunk_bytes<DK>(a);
+  char* const out = a.work + here + (size_t)hv * kHeadBytes;
   float* const vec = reinterpret_cast<float*>(out + 2 * kMatBytes);
-  {
-    // one column s per lane: the lower half of the wave L, the upper half Lq
+  if (wave < 2) {
+    // one column s per lane: the lower half of the wave L, the upper half Lq; tokens 16 wave .. + 15
     const int s = lane & 31;
     const bool lower = lane < 32;
-    float* mat = lower ? sA : sB;
-    float r = 0.f, c_mine = 0.f, c = 1.f, on_t[kChunk];
+    float* const mat = (lower ? sA : sB) + s;
+    f32x4_t gate[kChunk / 4], beta[4];
 #pragma unroll
-    for (int t = 0; t < kChunk; ++t) on_t[t] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(on_v), t));
+    for (int t = 0; t < kChunk / 4; ++t) gate[t] = *reinterpret_cast<const f32x4_t*>(sGate + 4 * t);
 #pragma unroll
-    for (int t = 0; t < kChunk; ++t) {
-      const float g = sGate[t];
+    for (int t = 0; t < 4; ++t) beta[t] = *reinterpret_cast<const f32x4_t*>(sBeta + 16 * wave + 4 * t);
+    float x[16];
+#pragma unroll
+    for (int t = 0; t < 16; ++t) x[t] = mat[(16 * wave + t) * kPitch];
+    float r = 0.f, c_mine = 0.f, c = 1.f;
+    auto step = [&](int t) __attribute__((always_inline)) {
+      const float g = gate[t >> 2][t & 3];
       r = t == s ? 1.f : (t > s ? r * g : 0.f);
       c *= g;
       c_mine = t == s ? c : c_mine;
-      const float x = mat[t * kPitch + s];
-      const bool counts = lower ? t > s : t >= s && on_t[t] != 0.f;  // (a masked token's y is zero)
-      const float entry = counts ? (lower ? sBeta[t] * r * x : r * x) : 0.f;
-      mat[t * kPitch + s] = entry;
-      finite = fmaf(entry, 0.f, finite);
+    };
+    auto entries = [&](auto half) __attribute__((always_inline)) {
+      constexpr int H = decltype(half)::value;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int t = 16 * H + i;
+        step(t);
+        const bool counts = lower ? t > s : t >= s && ((on_bits >> t) & 1u) != 0;  // (a masked token's y is zero)
+        const float entry = counts ? (lower ? beta[i >> 2][i & 3] * r * x[i] : r * x[i]) : 0.f;
+        mat[t * kPitch] = entry;
+        finite = fmaf(entry, 0.f, finite);
+      }
+    };
+    if (wave == 0) {
+      entries(std::integral_constant<int, 0>{});
+    } else {
+#pragma unroll
+      for (int t = 0; t < 16; ++t) step(t);
+      entries(std::integral_constant<int, 1>{});
+      finite = fmaf(r, 0.f, fmaf(c, 0.f, finite));
+      if (lower) {
+        vec[s] = ((on_bits >> s) & 1u) != 0 ? c_mine : 0.f;
+        vec[kChunk + s] = r;
+        if (s == 0) vec[kTail] = c, vec[kTail + 2] = __uint_as_float(on_bits);
+      }
     }
-    finite = fmaf(r, 0.f, fmaf(c, 0.f, finite));
-    if (lower) {
-      vec[s] = on_v != 0.f ? c_mine : 0.f;
-      vec[kChunk + s] = r;
-      if (s == 0) vec[kTail] = c;
+  } else if (writes_k) {
+    // K^T: lane (li, kq) takes row dk_of(c, li) of tokens token_of(kq, 0 .. 7), four of them by a transposing read: its lane 4 e + q points
+    // at token 4 kq + e and four dk, lane t receives element t % 4 of lanes t / 4, 4 + t / 4, 8 + t / 4, 12 + t / 4
+    typedef short s16x4_t __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) s16x4_t lds_s16x4;
+    char* const kt = a.work + here + (size_t)a.Hv * kHeadBytes + (size_t)hk * (kChunk * DK * 2);
+    const uint16_t* const from = sK + (4 * kq + (li >> 2)) * kKRow + 8 * (li & 3);
+#pragma unroll
+    for (int i = 0; i < DK / 32; ++i) {
+      const int c = (wave - 2) * (DK / 32) + i, dk = 32 * (c >> 1) + 4 * (c & 1);
+      const uint2 lo = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(from + dk)));
+      const uint2 hi = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(from + 16 * kKRow + dk)));
+      reinterpret_cast<uint4*>(kt)[c * 64 + lane] = uint4{lo.x, lo.y, hi.x, hi.y};
     }
   }
   __syncthreads();
-  {  // column j of (I + L)^-1 by forward substitution, rows of L read by all lanes at once
-    const int j = lane & 31;
-    float x[kChunk];
-    f32x4_t row[2][kChunk / 4];  // the row in use and the next one
+  auto store_pieces = [&](const float* mat, int m, int i) __attribute__((always_inline)) {
+    const f32x4_t lo = *reinterpret_cast<const f32x4_t*>(mat + (16 * i + li) * kPitch + 4 * kq);
+    const f32x4_t hi = *reinterpret_cast<const f32x4_t*>(mat + (16 * i + li) * kPitch + 16 + 4 * kq);
+    const float f[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    const Pieces<8> p = split_bf16(f);
+    uint4* dst = reinterpret_cast<uint4*>(out + m * kMatBytes + i * 3072) + lane;
+    dst[0] = uint4{p.hi[0], p.hi[1], p.hi[2], p.hi[3]};
+    dst[64] = uint4{p.mid[0], p.mid[1], p.mid[2], p.mid[3]};
+    dst[128] = uint4{p.lo[0], p.lo[1], p.lo[2], p.lo[3]};
+  };
+  if (wave == 0) {
+    // column j of the inverse of either triangle by forward substitution, lanes 0 .. 15 the first, 16 .. 31 the second (the rest as these)
+    const int first = lane & 16, j = li;
+    float x[16];
+    f32x4_t row[2][4];  // the row in use and the next one
 #pragma unroll
-    for (int t = 0; t < kChunk; ++t) {
-      if (t + 1 < kChunk) {
+    for (int t = 0; t < 16; ++t) {
+      if (t + 1 < 16) {
 #pragma unroll
-        for (int s4 = 0; s4 < t + 1; s4 += 4) row[(t + 1) & 1][s4 / 4] = *reinterpret_cast<const f32x4_t*>(sA + (t + 1) * kPitch + s4);
+        for (int s4 = 0; s4 < t + 1; s4 += 4) row[(t + 1) & 1][s4 / 4] = *reinterpret_cast<const f32x4_t*>(sA + (first + t + 1) * kPitch + first + s4);
       }
       float acc0 = t == j ? 1.f : 0.f, acc1 = 0.f;
 #pragma unroll
@@ -209,53 +272,48 @@ __global__ __launch_bounds__(64, 3) void gdn_chunk_kernel(Args a) {
         else acc0 -= row[t & 1][s / 4][s & 3] * x[s];
       }
       x[t] = acc0 + acc1;
-      // row by row: all of L at once does not fit the registers
-      asm volatile("" : "+v"(x[t]));
+      asm volatile("" : "+v"(x[t]));  // row by row
       __builtin_amdgcn_sched_barrier(0);
     }
-    __syncthreads();
-    const float beta = sBeta[j];
-#pragma unroll
-    for (int t = 0; t < kChunk; ++t) finite = fmaf(x[t] * beta, 0.f, finite);
     if (lane < 32) {
 #pragma unroll
-      for (int t = 0; t < kChunk; ++t) sA[t * kPitch + j] = x[t] * beta;
+      for (int t = 0; t < 16; ++t) sX[(first + t) * kPitch + first + j] = x[t];
     }
+    asm volatile("" ::: "memory");  // (one wave: what it has written is there for its reads)
+    // k of a product in the order 4 kq + step
+    const f32x4_t l21 = *reinterpret_cast<const f32x4_t*>(sA + (16 + li) * kPitch + 4 * kq);
+    f32x4_t below = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int step = 0; step < 4; ++step) below = mfma4(l21[step], sX[(4 * kq + step) * kPitch + li], below);
+    const f32x4_t x22 = *reinterpret_cast<const f32x4_t*>(sX + (16 + li) * kPitch + 16 + 4 * kq);
+    f32x4_t x21 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int step = 0; step < 4; ++step) x21 = mfma4(x22[step], below[step], x21);
+    const float beta = sBeta[first + j], beta0 = sBeta[li];
+    if (lane < 32) {
+#pragma unroll
+      for (int t = 0; t < 16; ++t) {
+        const float m = x[t] * beta;
+        finite = fmaf(m, 0.f, finite);
+        sA[(first + t) * kPitch + first + j] = m;  // (above the triangles L's zeros stay)
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float m = -x21[e] * beta0;
+      finite = fmaf(m, 0.f, finite);
+      sA[(16 + 4 * kq + e) * kPitch + li] = m;
+    }
+  } else if (wave >= 2) {
+    store_pieces(sB, 1, wave - 2);
   }
   {
     const bool all_finite = __all(finite == 0.f);
-    const uint32_t on_bits = (uint32_t)__ballot(on_v != 0.f);
-    if (lane == 0) vec[kTail + 1] = all_finite ? 0.f : __builtin_nanf(""), vec[kTail + 2] = __uint_as_float(on_bits);
+    if (lane == 0) sFinite[wave] = all_finite;
   }
   __syncthreads();
-#pragma unroll
-  for (int m = 0; m < 2; ++m) {
-    const float* mat = m == 0 ? sA : sB;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const f32x4_t lo = *reinterpret_cast<const f32x4_t*>(mat + (16 * i + li) * kPitch + 4 * kq);
-      const f32x4_t hi = *reinterpret_cast<const f32x4_t*>(mat + (16 * i + li) * kPitch + 16 + 4 * kq);
-      const float f[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-      const Pieces<8> p = split_bf16(f);
-      uint4* dst = reinterpret_cast<uint4*>(out + m * kMatBytes + i * 3072) + lane;
-      dst[0] = uint4{p.hi[0], p.hi[1], p.hi[2], p.hi[3]};
-      dst[64] = uint4{p.mid[0], p.mid[1], p.mid[2], p.mid[3]};
-      dst[128] = uint4{p.lo[0], p.lo[1], p.lo[2], p.lo[3]};
-    }
-  }
-  if (writes_k) {
-    char* const kt = a.work + ((size_t)slot * a.chunks + chunk) * chunk_bytes<DK>(a) + (size_t)a.Hv * kHeadBytes +
-                     (size_t)hk * (kChunk * DK * 2);
-#pragma unroll
-    for (int c = 0; c < DK / 16; ++c) {
-      uint32_t w[4];
-#pragma unroll
-      for (int j = 0; j < 8; j += 2)
-        w[j / 2] = (uint32_t)sK[token_of(kq, j) * kKRow + dk_of(c, li)] |
-                   ((uint32_t)sK[token_of(kq, j + 1) * kKRow + dk_of(c, li)] << 16);
-      reinterpret_cast<uint4*>(kt)[c * 64 + lane] = uint4{w[0], w[1], w[2], w[3]};
-    }
-  }
+  if (wave < 2) store_pieces(sA, 0, wave);
+  if (threadIdx.x == 64) vec[kTail + 1] = sFinite[0] & sFinite[1] & sFinite[2] & sFinite[3] ? 0.f : __builtin_nanf("");
 }
 
 // MASKED: some tokens may not count (those past T read zeros and need no looking after).  WAVES: of a workgroup, which
@@ -586,7 +644,7 @@ void gdn_prompt_kernel(Args a) {
 
 template <int DK>
 int launch(const Args& a, hipStream_t s) {
-  hipLaunchKernelGGL((gdn_chunk_kernel<DK>), dim3((unsigned)(a.slots * a.chunks * a.Hv)), dim3(64), 0, s, a);
+  hipLaunchKernelGGL((gdn_chunk_kernel<DK>), dim3((unsigned)(a.slots * a.chunks * a.Hv)), dim3(256), 0, s, a);
   const int groups = a.slots * a.Hv * (a.Dv / 16);
   const bool spread = groups <= kSpread;
   const void* fn = a.mask != nullptr ? (spread ? (const void*)gdn_prompt_kernel<DK, true, DK / 32> : (const void*)gdn_prompt_kernel<DK, true, 1>)
