@@ -17,8 +17,9 @@
 //    lane holds four consecutive rows of one column) are read as the B operand of the next product with k in the order the
 //    lane happens to have it, and the A operands (M', Lq, K^T) were laid out in that order.
 //  * Where that leaves the chip with one wave per compute unit, a row's elements are divided among as many waves as it has
-//    32ths: each cuts its part of S into pieces, multiplies and updates it, and the parts of U and Q S0^T meet in LDS,
-//    one barrier per chunk.  Delta is computed by all of them, from the same sums in the same order, Y by one each.
+//    32ths (gdn_prompt_spread_kernel): each cuts its part of S into pieces, multiplies and updates it, and the parts of U meet in LDS,
+//    one barrier per chunk.  Delta is computed by all of them, from the same sums in the same order.  Four more waves do what the
+//    chain does not wait for: two the results, two bring the next chunk's operands.
 //  * fp32 factors (S, V - c U, Delta, M', Lq) are cut into three bf16 pieces (24 bits, exact); products with bf16
 //    K and Q take three matrix-core passes, products of two fp32 factors the six of relative size 2^-16 and up.
 //    The result carries fp32 accuracy, as the step-by-step kernel's does.
@@ -31,12 +32,13 @@
 //    token holds never enters a product: its rows of K and Q are zeros, its element of V - c U as well.
 // A 16-bit state is carried in fp32 and rounded once, at the end.
 //
-// Measured, 1024 tokens, 16 / 32 heads of 128 x 128: 12.5 + 51 us (64 with one wave per 16 rows), against 123.7 ms with one
-// workgroup per head that kept S in memory (the step-by-step kernel held 41 tokens at most); 678 tokens of 16 heads both kernels
-// 46 us (55).  What the second kernel is bound by is its chain.  One wave: 4560 cycles (2 us) per chunk by its counters, 605
-// vector instructions (53 %), 96 matrix instructions (34 %; 72 of them with S), waits 16 %.  Four: 3500 cycles, 315 vector and
-// 36 matrix instructions a wave; with no loads in the loop at all it takes 2900, the rest is the hand-over and results that the next
-// instruction waits for.  Chunks of
+// Measured, 1024 tokens of 32 heads of 128 x 128: 12.5 + 42 us, against 123.7 ms with one workgroup per head that kept S in memory (the
+// step-by-step kernel held 41 tokens at most); 600 tokens of 16 heads 7.9 + 23.6.  What the second kernel is bound by is its chain.
+// Four waves that did everything took 2950 cycles a chunk (56 and 32 us): a third of them waited for the path to memory, which
+// took 124 requests a chunk, M' and vectors for every wave and V two bytes at a time.  Now the chain asks for K and K^T, V is one request
+// and a transposing read, the tape's stores are there for those who want it, and a chunk takes 2200 cycles, shared by the
+// path through LDS (1000 of them), 160 vector and 18 matrix instructions a wave, and results that the next instruction waits for.
+// One wave, 900 tokens of 64 heads: 72 -> 64 us with V and the tape's stores so.  Chunks of
 // 32 and not 16: cutting S into pieces (176 vector instructions) is paid per chunk, and a matrix instruction
 // of depth 32 in the update is filled; 64 would need more registers than a wave has.  The look for numbers that are not
 // finite costs 0.3 % of a layer call, a chunk token by token what 32 steps of one wave cost.
@@ -53,8 +55,8 @@ constexpr int kHeadBytes = 2 * kMatBytes + 3 * kChunk * 4;  // M', Lq, then per 
 constexpr int kTail = 2 * kChunk;                      // four words: c_T, 0 or (numbers that are not finite) NaN, one bit per token that counts, -
 constexpr int kPitch = 36;                             // floats per row of the 32 x 32 matrices in LDS
 // Up to as many (head, 16 rows) as there are compute units, the 32ths of a row on a wave each.  With more of them the units
-// are shared, and what the waves of a row do twice (Delta, the pieces of it) costs more than their chain is shorter: us per
-// 1024 tokens with the chunk kernel, one wave and four, 32 heads of 128 x 128 78 and 66, 48 heads 88 and 90, 64 heads 89 and 94.
+// are shared, and what the waves of a row do twice (Delta, the pieces of it) costs more than their chain is shorter: us, one wave and
+// several, 300 tokens of 48 heads of 128 x 128 25.2 and 28.5, 900 tokens of 64 64.4 and 74.5.
 constexpr int kSpread = 256;
 
 struct Args {
@@ -316,149 +318,165 @@ __global__ __launch_bounds__(256) void gdn_chunk_kernel(Args a) {
   if (threadIdx.x == 64) vec[kTail + 1] = sFinite[0] & sFinite[1] & sFinite[2] & sFinite[3] ? 0.f : __builtin_nanf("");
 }
 
-// MASKED: some tokens may not count (those past T read zeros and need no looking after).  WAVES: of a workgroup, which
-// divide the DK elements of a row among themselves, 1 or DK / 32.
-template <int DK, bool MASKED, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(1, WAVES == 1 ? 1 : 2)))
-void gdn_prompt_kernel(Args a) {
-  constexpr int NC = DK / 32 / WAVES, NT = 2 * NC;  // pieces of 32 and of 16 dk that a wave has
-  constexpr int kTiles = WAVES == 1 ? 2 : 1;         // of the tokens whose Y it computes
-  constexpr bool kEarly = WAVES > 1;                 // c and c_T / c_s of the next chunk are asked for at their last use, not last
-  constexpr int kStored = WAVES == 4 ? 2 : 4;        // tokens of a lane's four there whose results it writes
-  // the waves' parts of U (two tiles) and W, those of a chunk while the ones before may still be read
-  __shared__ f32x4_t parts[2][WAVES][4][WAVES == 1 ? 1 : 64];
-  __shared__ float sums[WAVES][16];  // (token by token: their parts of one row each)
-  const int slices = a.Dv / 16;
-  // the slices of a head read the same K, Q, M' and Lq: all of them behind one L2 (blocks go to the XCDs in turn)
-  const int heads = a.slots * a.Hv;
-  int item, slice;
-  if (heads % 8 == 0) {
-    const int b = blockIdx.x / 8;
-    item = (b / slices) * 8 + blockIdx.x % 8;
-    slice = b % slices;
-  } else {
-    item = blockIdx.x / slices;
-    slice = blockIdx.x % slices;
-  }
-  const int slot = item / a.Hv, hv = item % a.Hv, hk = hv / (a.Hv / a.Hk);
-  const int lane = threadIdx.x & 63, li = lane & 15, kq = lane >> 4;
-  const int wave = WAVES == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int tile0 = WAVES == 4 ? wave >> 1 : wave;          // the first (or only) tile of tokens whose Y it computes
-  const int first = WAVES == 4 ? 2 * (wave & 1) : 0;        // of a lane's four tokens there
-  const size_t slotT = (size_t)slot * a.T;
-  const int dv = 16 * slice + li;
+// arithmetic may move across, requests to memory stay where they were written
+#define DFLASH_KEEP_REQUESTS() __builtin_amdgcn_sched_barrier(0xF)
 
-  // S^T tile c of this wave: rows dk_of(NT wave + c, 4 kq + r), column dv = this lane's; two tiles are 8 consecutive dk of a
-  // row of S
-  f32x4_t st[NT];
-  const size_t srow = ((size_t)item * a.Dv + dv) * DK + 32 * NC * wave + 8 * kq;
+// What a workgroup walks: 16 rows of the state of one head, and the addresses of what their chunks read and write.  What a chunk reads
+// and writes by token goes through buffer descriptors of this slot: tokens past T read zeros and are not written, with no branch
+// (a branch around a store leaves the count of requests in flight open, and the next wait for a load becomes a wait for every store).
+template <int DK>
+struct Rows {
+  const Args& a;
+  int item, slice, slot, hv, hk, lane, li, kq, dv;
+  size_t slotT, per_chunk;
+  __amdgpu_buffer_rsrc_t k_buf, q_buf, v_buf, y_buf, tape_buf;
+  uint32_t k_step, v_step;  // bytes per token
+  uint32_t k_at, v_at;      // of row li and 16-byte piece kq of K and Q, of token 4 kq and column dv of V
+  const char *head0, *kt0;
+
+  __device__ __forceinline__ explicit Rows(const Args& args) : a(args) {
+    const int slices = a.Dv / 16;
+    // the slices of a head read the same K, Q, M' and Lq: all of them behind one L2 (blocks go to the XCDs in turn)
+    const int heads = a.slots * a.Hv;
+    if (heads % 8 == 0) {
+      const int b = blockIdx.x / 8;
+      item = (b / slices) * 8 + blockIdx.x % 8;
+      slice = b % slices;
+    } else {
+      item = blockIdx.x / slices;
+      slice = blockIdx.x % slices;
+    }
+    slot = item / a.Hv, hv = item % a.Hv, hk = hv / (a.Hv / a.Hk);
+    lane = threadIdx.x & 63, li = lane & 15, kq = lane >> 4;
+    dv = 16 * slice + li;
+    slotT = (size_t)slot * a.T;
+    const uint32_t k_bytes = (uint32_t)a.T * a.Hk * DK * 2, v_bytes = (uint32_t)a.T * a.Hv * a.Dv * 2;
+    k_buf = buffer_of(a.k + slotT * a.Hk * DK, k_bytes), q_buf = buffer_of(a.q + slotT * a.Hk * DK, k_bytes);
+    v_buf = buffer_of(a.v + slotT * a.Hv * a.Dv, v_bytes), y_buf = buffer_of(a.y + slotT * a.Hv * a.Dv, v_bytes);
+    tape_buf = buffer_of(a.tape + slotT * a.Hv * a.Dv, a.tape != nullptr ? 2 * v_bytes : 0u);
+    k_step = (uint32_t)a.Hk * DK * 2, v_step = (uint32_t)a.Hv * a.Dv * 2;
+    k_at = li * k_step + hk * (DK * 2) + 16 * kq;
+    v_at = 4 * kq * v_step + (hv * a.Dv + dv) * 2;
+    per_chunk = chunk_bytes<DK>(a);
+    head0 = a.work + (size_t)slot * a.chunks * per_chunk + (size_t)hv * kHeadBytes;
+    kt0 = a.work + (size_t)slot * a.chunks * per_chunk + (size_t)a.Hv * kHeadBytes + (size_t)hk * (kChunk * DK * 2);
+  }
+
+  // Element 8 kq of piece `first` (of 32 dk) of row dv of the state.
+  __device__ __forceinline__ size_t state_at(int first) const { return ((size_t)item * a.Dv + dv) * DK + 32 * first + 8 * kq; }
+  // S^T tile c: rows dk_of(2 first + c, 4 kq + r), column dv; two tiles are 8 consecutive dk of a row of S.
+  template <int NT>
+  __device__ __forceinline__ void load_state(int first, f32x4_t (&st)[NT]) const {
+    const size_t srow = state_at(first);
 #pragma unroll
-  for (int C = 0; C < NC; ++C)
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int c = 0; c < NT; ++c) {
+      const size_t at = srow + 32 * (c >> 1) + 4 * (c & 1);
       if (a.state_in == nullptr) {
-        st[2 * C + h] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        st[c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
       } else if (a.state_dtype == DFLASH_FP32) {
-        st[2 * C + h] = *reinterpret_cast<const f32x4_t*>((const float*)a.state_in + srow + 32 * C + 4 * h);
+        st[c] = *reinterpret_cast<const f32x4_t*>((const float*)a.state_in + at);
       } else {
-        const uint2 w = *reinterpret_cast<const uint2*>((const uint16_t*)a.state_in + srow + 32 * C + 4 * h);
+        const uint2 w = *reinterpret_cast<const uint2*>((const uint16_t*)a.state_in + at);
         const uint32_t b[4] = {w.x & 0xffffu, w.x >> 16, w.y & 0xffffu, w.y >> 16};
 #pragma unroll
-        for (int e = 0; e < 4; ++e) st[2 * C + h][e] = a.state_dtype == DFLASH_BF16 ? bf16_bits_to_f32(b[e]) : f16_bits_to_f32(b[e]);
+        for (int e = 0; e < 4; ++e) st[c][e] = a.state_dtype == DFLASH_BF16 ? bf16_bits_to_f32(b[e]) : f16_bits_to_f32(b[e]);
       }
     }
-
-  // What a chunk reads and writes by token goes through buffer descriptors of this slot: tokens past T read
-  // zeros and are not written, with no branch (a branch around a store leaves the count of requests in flight
-  // open, and the next wait for a load becomes a wait for every store).
-  const uint32_t k_bytes = (uint32_t)a.T * a.Hk * DK * 2, v_bytes = (uint32_t)a.T * a.Hv * a.Dv * 2;
-  const auto k_buf = buffer_of(a.k + slotT * a.Hk * DK, k_bytes), q_buf = buffer_of(a.q + slotT * a.Hk * DK, k_bytes);
-  const auto v_buf = buffer_of(a.v + slotT * a.Hv * a.Dv, v_bytes), y_buf = buffer_of(a.y + slotT * a.Hv * a.Dv, v_bytes);
-  const auto tape_buf = buffer_of(a.tape + slotT * a.Hv * a.Dv, a.tape != nullptr ? 2 * v_bytes : 0u);
-  const uint32_t k_step = (uint32_t)a.Hk * DK * 2, v_step = (uint32_t)a.Hv * a.Dv * 2;  // bytes per token
-  const uint32_t k_at = li * k_step + hk * (DK * 2) + 64 * NC * wave + 16 * kq;
-  const uint32_t v_at = 4 * kq * v_step + (hv * a.Dv + dv) * 2;
-
-  uint4 kf[2][NC], qf[2][NC], kt[NT], mf[2][3], lf[kTiles][3];
-  uint32_t vb[8];
-  f32x4_t cv[2], cfv[2];
-  f32x4_t tail_next;  // (asked for with K and Q: the scheduler moves the scaling of S to the front)
-  const size_t per_chunk = chunk_bytes<DK>(a);
-  const char* const head0 = a.work + (size_t)slot * a.chunks * per_chunk + (size_t)hv * kHeadBytes;
-  const char* const kt0 = a.work + (size_t)slot * a.chunks * per_chunk + (size_t)a.Hv * kHeadBytes + (size_t)hk * (kChunk * DK * 2);
-  auto load_kq = [&](int ch) __attribute__((always_inline)) {
-    tail_next = reinterpret_cast<const f32x4_t*>(head0 + ch * per_chunk + 2 * kMatBytes + 4 * kTail)[lane >> 6];
+  }
+  template <int NT>
+  __device__ __forceinline__ void store_state(int first, const f32x4_t (&st)[NT]) const {
+    const size_t srow = state_at(first);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const uint32_t at = k_at + (ch * kChunk + 16 * i) * k_step;
+    for (int c = 0; c < NT; ++c) {
+      const size_t at = srow + 32 * (c >> 1) + 4 * (c & 1);
+      if (a.state_dtype == DFLASH_FP32) {
+        *reinterpret_cast<f32x4_t*>((float*)a.state_out + at) = st[c];
+      } else {
+        uint32_t b[4];
 #pragma unroll
-      for (int C = 0; C < NC; ++C) {
-        kf[i][C] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(k_buf, at + 64 * C, 0, 0));
-        qf[i][C] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(q_buf, at + 64 * C, 0, 0));
+        for (int e = 0; e < 4; ++e) b[e] = a.state_dtype == DFLASH_BF16 ? f32_to_bf16_bits(st[c][e]) : f32_to_f16_bits(st[c][e]);
+        *reinterpret_cast<uint2*>((uint16_t*)a.state_out + at) = uint2{b[0] | (b[1] << 16), b[2] | (b[3] << 16)};
       }
     }
-  };
-  auto load_v = [&](int ch) __attribute__((always_inline)) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-      vb[j] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(v_buf, v_at + (ch * kChunk + 16 * (j >> 2) + (j & 3)) * v_step, 0, 0);
-  };
-  auto load_m = [&](int ch) __attribute__((always_inline)) {
-    const uint4* src = reinterpret_cast<const uint4*>(head0 + ch * per_chunk) + lane;
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int p = 0; p < 3; ++p) mf[i][p] = src[(3 * i + p) * 64];
-  };
-  auto load_l = [&](int ch) __attribute__((always_inline)) {
-    const uint4* src = reinterpret_cast<const uint4*>(head0 + ch * per_chunk + kMatBytes) + 3 * tile0 * 64 + lane;
-#pragma unroll
-    for (int i = 0; i < kTiles; ++i)
-#pragma unroll
-      for (int p = 0; p < 3; ++p) lf[i][p] = src[(3 * i + p) * 64];
-  };
-  auto load_kt = [&](int ch) __attribute__((always_inline)) {
-    const uint4* src = reinterpret_cast<const uint4*>(kt0 + ch * per_chunk) + NT * wave * 64 + lane;
-#pragma unroll
-    for (int c = 0; c < NT; ++c) kt[c] = src[c * 64];
-  };
-  auto load_vec = [&](int ch, int which, f32x4_t (&f)[2]) __attribute__((always_inline)) {
-    const float* vec = reinterpret_cast<const float*>(head0 + ch * per_chunk + 2 * kMatBytes) + which * kChunk;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) f[i] = *reinterpret_cast<const f32x4_t*>(vec + 16 * i + 4 * kq);
-  };
-  // arithmetic may move across, requests to memory stay where they were written
-#define DFLASH_KEEP_REQUESTS() __builtin_amdgcn_sched_barrier(0xF)
-  // a barrier for what the waves hand over through LDS; requests to memory stay in flight
-  auto meet = [&]() __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-  // sum of the six piece products of two fp32 factors that matter; two accumulators, smaller terms first
-  auto product6 = [&](const uint4 (&f)[3], const Pieces<8>& p, f32x4_t big) __attribute__((always_inline)) {
-    f32x4_t small = {0.f, 0.f, 0.f, 0.f};
-    small = mfma(f[0], p.lo, small);
-    big = mfma(f[0], p.mid, big);
-    small = mfma(f[2], p.hi, small);
-    big = mfma(f[1], p.hi, big);
-    small = mfma(f[1], p.mid, small);
-    big = mfma(f[0], p.hi, big);
-    return big + small;
-  };
-  // sum over all waves of what each has for the lane's row of S, in the order of the waves
-  auto over_waves = [&](float x) __attribute__((always_inline)) -> float {
-    x += __shfl_xor(x, 16, 64);
-    x += __shfl_xor(x, 32, 64);
-    if (WAVES == 1) return x;
-    if (kq == 0) sums[wave][li] = x;
-    meet();
-    float sum = sums[0][li];
-#pragma unroll
-    for (int w = 1; w < WAVES; ++w) sum += sums[w][li];
-    meet();
-    return sum;
-  };
+  }
 
-  // The recurrence itself, for a chunk with numbers that are not finite.
-  auto token_by_token = [&](int ch) __attribute__((always_inline)) {
+  template <int NC>  // pieces first .. first + NC - 1 of rows 16 i + li of K or Q
+  __device__ __forceinline__ void load_rows(__amdgpu_buffer_rsrc_t from, int ch, int i, int first, uint4 (&f)[NC]) const {
+    const uint32_t at = k_at + 64 * first + (ch * kChunk + 16 * i) * k_step;
+#pragma unroll
+    for (int C = 0; C < NC; ++C) f[C] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(from, at + 64 * C, 0, 0));
+  }
+  __device__ __forceinline__ void load_matrix(int ch, int which, int i, uint4 (&f)[3]) const {  // tile i of M' (0) or Lq (1)
+    const uint4* src = reinterpret_cast<const uint4*>(head0 + ch * per_chunk + which * kMatBytes) + lane;
+#pragma unroll
+    for (int p = 0; p < 3; ++p) f[p] = src[(3 * i + p) * 64];
+  }
+  template <int NT>
+  __device__ __forceinline__ void load_kt(int ch, int first, uint4 (&f)[NT]) const {
+    const uint4* src = reinterpret_cast<const uint4*>(kt0 + ch * per_chunk) + 2 * first * 64 + lane;
+#pragma unroll
+    for (int c = 0; c < NT; ++c) f[c] = src[c * 64];
+  }
+  __device__ __forceinline__ f32x4_t load_vec(int ch, int which, int i) const {  // of the four tokens of tile i: c (0), c_T / c_s (1)
+    return *reinterpret_cast<const f32x4_t*>(reinterpret_cast<const float*>(head0 + ch * per_chunk + 2 * kMatBytes) + which * kChunk + 16 * i + 4 * kq);
+  }
+  __device__ __forceinline__ f32x4_t load_tail(int ch) const {
+    return reinterpret_cast<const f32x4_t*>(head0 + ch * per_chunk + 2 * kMatBytes + 4 * kTail)[lane >> 6];
+  }
+
+  // Of a chunk, 16 bytes per lane: V of these 16 columns, lane l half l % 2 of token l / 2 (of the last one for those past T, which count for
+  // nothing), or the vectors and the four words behind them.  One load either way.
+  __device__ __forceinline__ uint4 load_columns(int ch, bool vectors) const {
+    constexpr int kLast = (kTail + 4) / 4 - 1;
+    int t = ch * kChunk + (lane >> 1);
+    t = t < a.T ? t : a.T - 1;
+    const size_t of_v = (slotT + t) * v_step + (hv * a.Dv + 16 * slice) * 2 + 16 * (lane & 1);
+    const size_t of_vectors = ch * per_chunk + 2 * kMatBytes + 16 * (lane < kLast ? lane : kLast);
+    return *reinterpret_cast<const uint4*>((vectors ? head0 : (const char*)a.v) + (vectors ? of_vectors : of_v));
+  }
+
+  // Brings a chunk into the L2 that the slices of a head share, a line of 128 bytes per lane of two waves per slice: a chunk's time is about that of
+  // one trip to memory, and the operands are asked for one chunk ahead.  What comes back is looked at by nobody; see keep().
+  __device__ __forceinline__ uint32_t touch(int ch, int wave) const {
+    constexpr int kHeadLines = (kHeadBytes + 127) / 128, kRowLines = DK / 64, kLines = kChunk * kRowLines;
+    ch = ch < a.chunks ? ch : a.chunks - 1;
+    int line = 64 * (2 * slice + wave) + lane;
+    const char* from = head0 + ch * per_chunk + 128 * line;
+    if (line >= kHeadLines) {
+      line -= kHeadLines;
+      const bool turned = line < kLines, of_k = line < 2 * kLines, of_q = line < 3 * kLines;
+      const int in = line - (turned ? 0 : of_k ? kLines : of_q ? 2 * kLines : 3 * kLines);
+      int t = ch * kChunk + in / kRowLines;
+      t = t < a.T ? t : a.T - 1;
+      const char* const row = (const char*)(of_k ? a.k : a.q) + (slotT + t) * k_step + hk * (DK * 2) + 128 * (in % kRowLines);
+      const int v_lines = (a.Dv + 63) / 64;
+      int tv = ch * kChunk + in / v_lines;
+      tv = tv < a.T ? tv : a.T - 1;
+      const char* const v_row = (const char*)a.v + (slotT + tv) * v_step + hv * a.Dv * 2;
+      from = turned ? kt0 + ch * per_chunk + 128 * in : of_q ? row : v_row + (128 * (in % v_lines) < 2 * a.Dv ? 128 * (in % v_lines) : 0);
+    }
+    return *reinterpret_cast<const uint32_t*>(from);
+  }
+  static __device__ __forceinline__ void keep(uint32_t touched) { asm volatile("" ::"v"(touched)); }
+
+  // y and the tape of token `t` (and 4 kq) of a chunk
+  template <bool MASKED, bool TAPE>
+  __device__ __forceinline__ void store_token(int ch, int t, float y_t, float delta, uint32_t on_bits, uint32_t nowhere) const {
+    const uint32_t at = (v_at + (ch * kChunk + t) * v_step) | nowhere;  // (2^31 or more is behind every row)
+    uint16_t y = __builtin_bit_cast(uint16_t, (__bf16)y_t);
+    if (MASKED) y &= (uint16_t)-(int)((on_bits >> (t + 4 * kq)) & 1u);
+    __builtin_amdgcn_raw_buffer_store_b16(y, y_buf, at, 0, 0);
+    if (TAPE) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(delta), tape_buf, 2 * at | nowhere, 0, 0);
+  }
+
+  // The recurrence itself, for a chunk with numbers that are not finite: by one wave, which has all of its rows.
+  __device__ __forceinline__ void token_by_token(int ch, f32x4_t (&st)[DK / 16]) const {
+    constexpr int NC = DK / 32;
     const int end = (ch + 1) * kChunk < a.T ? (ch + 1) * kChunk : a.T;
+    auto over_row = [](float x) __attribute__((always_inline)) {  // the four lanes that hold a row
+      x += __shfl_xor(x, 16, 64);
+      return x + __shfl_xor(x, 32, 64);
+    };
 #pragma unroll 1
     for (int t = ch * kChunk; t < end; ++t) {
       const uint32_t at = (uint32_t)t * v_step + (hv * a.Dv + dv) * 2;
@@ -467,7 +485,7 @@ void gdn_prompt_kernel(Args a) {
         const float g = load_as_f32(a.g, (slotT + t) * a.Hv + hv, a.g_dtype);
         const float beta = load_as_f32(a.beta, (slotT + t) * a.Hv + hv, a.beta_dtype);
         const float v = bf16_bits_to_f32((uint16_t)__builtin_amdgcn_raw_buffer_load_b16(v_buf, at, 0, 0));
-        const size_t row = ((slotT + t) * a.Hk + hk) * DK + 32 * NC * wave + 8 * kq;
+        const size_t row = ((slotT + t) * a.Hk + hk) * DK + 8 * kq;
         auto element = [](uint4 w, int e) __attribute__((always_inline)) {  // 0 .. 7
           const uint32_t half[4] = {w.x, w.y, w.z, w.w};
           return __uint_as_float(e & 1 ? half[e >> 1] & 0xffff0000u : half[e >> 1] << 16);
@@ -478,7 +496,7 @@ void gdn_prompt_kernel(Args a) {
           kw[C] = *reinterpret_cast<const uint4*>(a.k + row + 32 * C);
           qw[C] = *reinterpret_cast<const uint4*>(a.q + row + 32 * C);
         }
-        float known = 0.f;  // S k, summed over the four lanes of every wave that hold a row of S
+        float known = 0.f;  // S k
 #pragma unroll
         for (int C = 0; C < NC; ++C)
 #pragma unroll
@@ -487,7 +505,7 @@ void gdn_prompt_kernel(Args a) {
             entry[e & 3] *= g;
             known = fmaf(entry[e & 3], element(kw[C], e), known);
           }
-        delta = (v - over_waves(known)) * beta;
+        delta = (v - over_row(known)) * beta;
 #pragma unroll
         for (int C = 0; C < NC; ++C)
 #pragma unroll
@@ -496,28 +514,94 @@ void gdn_prompt_kernel(Args a) {
             entry[e & 3] = fmaf(element(kw[C], e), delta, entry[e & 3]);
             y = fmaf(entry[e & 3], element(qw[C], e), y);
           }
-        y = over_waves(y);
+        y = over_row(y);
       }
-      if (kq == 0 && wave == 0) {
+      if (kq == 0) {
         __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(uint16_t, (__bf16)y), y_buf, at, 0, 0);
         __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(delta), tape_buf, 2 * at, 0, 0);
       }
     }
+  }
+};
+
+// V of a lane's eight tokens out of a chunk's 16 columns in LDS: a transposing read gives the lane its column of four (see the chunk
+// kernel).
+typedef uint16_t Columns[kChunk][16];
+struct Values {
+  typedef short s16x4_t __attribute__((ext_vector_type(4)));
+  s16x4_t lo, hi;
+  __device__ __forceinline__ void read(const Columns& from, int li, int kq) {
+    typedef __attribute__((address_space(3))) s16x4_t lds_s16x4;
+    const uint16_t* const at = &from[4 * kq + (li >> 2)][4 * (li & 3)];
+    lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)at);
+    hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(at + 16 * 16));
+  }
+  __device__ __forceinline__ float operator[](int j) const { return bf16_bits_to_f32((uint16_t)(j < 4 ? lo[j & 3] : hi[j & 3])); }
+};
+
+// sum of the six piece products of two fp32 factors that matter; two accumulators, smaller terms first
+__device__ __forceinline__ f32x4_t product6(const uint4 (&f)[3], const Pieces<8>& p, f32x4_t big) {
+  f32x4_t small = {0.f, 0.f, 0.f, 0.f};
+  small = mfma(f[0], p.lo, small);
+  big = mfma(f[0], p.mid, big);
+  small = mfma(f[2], p.hi, small);
+  big = mfma(f[1], p.hi, big);
+  small = mfma(f[1], p.mid, small);
+  big = mfma(f[0], p.hi, big);
+  return big + small;
+}
+__device__ __forceinline__ Pieces<8> split_tiles(f32x4_t x, f32x4_t y) {
+  const float f[8] = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+  return split_bf16(f);
+}
+// V - c U for the eight tokens of a lane, what a masked token holds left out
+template <bool MASKED>
+__device__ __forceinline__ Pieces<8> right_side(const Values& v, const f32x4_t (&cv)[2], const f32x4_t (&U)[2], uint32_t on_bits, int kq) {
+  float rhs[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    rhs[j] = v[j] - cv[j >> 2][j & 3] * U[j >> 2][j & 3];
+    if (MASKED) rhs[j] = __int_as_float(__float_as_int(rhs[j]) & -(int)((on_bits >> token_of(kq, j)) & 1u));
+  }
+  return split_bf16(rhs);
+}
+
+// One wave with all of its 16 rows.  MASKED: some tokens may not count (those past T read zeros and need no looking after).
+template <int DK, bool MASKED, bool TAPE>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void gdn_prompt_kernel(Args a) {
+  constexpr int NC = DK / 32, NT = 2 * NC;  // pieces of 32 and of 16 dk
+  __shared__ __align__(16) Columns values;  // V
+  const Rows<DK> rows(a);
+  f32x4_t st[NT];
+  rows.load_state(0, st);
+  uint4 kf[2][NC], qf[2][NC], kt[NT], mf[2][3], lf[2][3];
+  uint4 columns;
+  f32x4_t cv[2], cfv[2];
+  f32x4_t tail_next;  // (asked for with K and Q: the scheduler moves the scaling of S to the front)
+  auto load_kq = [&](int ch) __attribute__((always_inline)) {
+    tail_next = rows.load_tail(ch);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) rows.load_rows(rows.k_buf, ch, i, 0, kf[i]), rows.load_rows(rows.q_buf, ch, i, 0, qf[i]);
+  };
+  auto load_matrices = [&](int ch, int which, uint4 (&f)[2][3]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) rows.load_matrix(ch, which, i, f[i]);
+  };
+  auto load_vecs = [&](int ch) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) cv[i] = rows.load_vec(ch, 0, i), cfv[i] = rows.load_vec(ch, 1, i);
   };
 
-  // (the way to the token-by-token form leaves the loop: the loop itself stays without a branch around its stores.  Every
-  // wave leaves it at the same chunk: what they look at, Delta, is the same numbers in all of them.)
+  // (the way to the token-by-token form leaves the loop: the loop itself stays without a branch around its stores)
   int ch = 0;
   while (ch < a.chunks) {
     load_kq(ch);
     DFLASH_KEEP_REQUESTS();  // in the order of the loop: what its first wait may leave in flight is the least of both
-    load_v(ch);
-    if (kEarly) load_vec(ch, 0, cv);
-    load_m(ch);
-    if (kEarly) load_vec(ch, 1, cfv);
-    load_kt(ch);
-    load_l(ch);
-    if (!kEarly) load_vec(ch, 0, cv), load_vec(ch, 1, cfv);
+    columns = rows.load_columns(ch, false);
+    load_matrices(ch, 0, mf);
+    rows.load_kt(ch, 0, kt);
+    load_matrices(ch, 1, lf);
+    load_vecs(ch);
     DFLASH_KEEP_REQUESTS();
 #pragma unroll 1
     for (; ch < a.chunks; ++ch) {
@@ -531,9 +615,7 @@ void gdn_prompt_kernel(Args a) {
       for (int i = 0; i < 2; ++i) U[i] = W[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int C = 0; C < NC; ++C) {
-        const float f[8] = {st[2 * C][0],     st[2 * C][1],     st[2 * C][2],     st[2 * C][3],
-                            st[2 * C + 1][0], st[2 * C + 1][1], st[2 * C + 1][2], st[2 * C + 1][3]};
-        const Pieces<8> sp = split_bf16(f);
+        const Pieces<8> sp = split_tiles(st[2 * C], st[2 * C + 1]);
 #pragma unroll
         for (int i = 0; i < 2; ++i) U[i] = mfma(kf[i][C], sp.lo, U[i]), W[i] = mfma(qf[i][C], sp.lo, W[i]);
 #pragma unroll
@@ -541,56 +623,28 @@ void gdn_prompt_kernel(Args a) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) U[i] = mfma(kf[i][C], sp.hi, U[i]), W[i] = mfma(qf[i][C], sp.hi, W[i]);
       }
-      if constexpr (WAVES > 1) {  // the sums over the waves, in their order: the same numbers in every wave
-#pragma unroll
-        for (int i = 0; i < 2; ++i) parts[ch & 1][wave][i][lane] = U[i], parts[ch & 1][wave][2 + i][lane] = W[i];
-      }
       load_kq(next);
       DFLASH_KEEP_REQUESTS();
-      if constexpr (WAVES > 1) {
-        meet();
-        auto total = [&](int part) __attribute__((always_inline)) -> f32x4_t {
-          f32x4_t sum = parts[ch & 1][0][part][lane];
-#pragma unroll
-          for (int w = 1; w < WAVES; ++w) sum += parts[ch & 1][w][part][lane];
-          return sum;
-        };
-        U[0] = total(0), U[1] = total(1), W[0] = total(2 + tile0);
-      }
       // ---- Delta = M' (V - c U) ----------------------------------------------------------------------
-      float rhs[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        rhs[j] = bf16_bits_to_f32(vb[j]) - cv[j >> 2][j & 3] * U[j >> 2][j & 3];
-        if (MASKED) rhs[j] = __int_as_float(__float_as_int(rhs[j]) & -(int)((on_bits >> token_of(kq, j)) & 1u));
-      }
-      if (kEarly) W[0] *= tile0 ? cv[1] : cv[0];
-      load_v(next);
-      if (kEarly) load_vec(next, 0, cv);
+      *reinterpret_cast<uint4*>(&values[rows.lane >> 1][8 * (rows.lane & 1)]) = columns;
+      asm volatile("" ::: "memory");  // (one wave: what it has written is there for its reads)
+      Values v;
+      v.read(values, rows.li, rows.kq);
+      const Pieces<8> rp = right_side<MASKED>(v, cv, U, on_bits, rows.kq);
+      columns = rows.load_columns(next, false);
       DFLASH_KEEP_REQUESTS();
-      const Pieces<8> rp = split_bf16(rhs);
       f32x4_t D[2];
 #pragma unroll
       for (int i = 0; i < 2; ++i) D[i] = product6(mf[i], rp, f32x4_t{0.f, 0.f, 0.f, 0.f});
-      load_m(next);
+      load_matrices(next, 0, mf);
       DFLASH_KEEP_REQUESTS();
       // a number that is not finite in V, U (and so in S) or M' is one in every Delta of its column
 #pragma unroll
       for (int j = 0; j < 8; ++j) finite = fmaf(D[j >> 2][j & 3], 0.f, finite);
       if (!__all(finite == 0.f)) break;
       // ---- S^T = c_T S^T + K^T diag(c_T / c_s) Delta ----------------------------------------------
-      float scaled[8], plain[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        plain[j] = D[j >> 2][j & 3];
-        scaled[j] = plain[j] * cfv[j >> 2][j & 3];
-      }
-      if (kEarly) {
-        load_vec(next, 1, cfv);
-        DFLASH_KEEP_REQUESTS();
-      }
       {
-        const Pieces<8> dp = split_bf16(scaled);
+        const Pieces<8> dp = split_tiles(D[0] * cfv[0], D[1] * cfv[1]);
 #pragma unroll
         for (int c = 0; c < NT; ++c) st[c] *= c_last;
 #pragma unroll
@@ -600,58 +654,251 @@ void gdn_prompt_kernel(Args a) {
 #pragma unroll
         for (int c = 0; c < NT; ++c) st[c] = mfma(kt[c], dp.hi, st[c]);
       }
-      load_kt(next);
+      rows.load_kt(next, 0, kt);
       DFLASH_KEEP_REQUESTS();
-      // ---- Y = c W + Lq Delta, for the tokens of this wave's tiles -------------------------------------
-      const Pieces<8> dq = split_bf16(plain);
+      // ---- Y = c W + Lq Delta ---------------------------------------------------------------------------
+      const Pieces<8> dq = split_tiles(D[0], D[1]);
 #pragma unroll
-      for (int i = 0; i < kTiles; ++i) {
-        const f32x4_t Y = product6(lf[i], dq, kEarly ? W[i] : W[i] * cv[i]), mine = i == 1 || (WAVES > 1 && tile0) ? D[1] : D[0];
+      for (int i = 0; i < 2; ++i) {
+        const f32x4_t Y = product6(lf[i], dq, W[i] * cv[i]);
 #pragma unroll
-        for (int r = 0; r < kStored; ++r) {
-          const float y_r = kStored == 2 && first ? Y[(r + 2) & 3] : Y[r], d_r = kStored == 2 && first ? mine[(r + 2) & 3] : mine[r];
-          const int t = 16 * (tile0 + i) + first + r;  // and 4 kq, which v_at holds
-          const uint32_t at = v_at + (ch * kChunk + t) * v_step;
-          uint16_t y = __builtin_bit_cast(uint16_t, (__bf16)y_r);
-          if (MASKED) y &= (uint16_t)-(int)((on_bits >> (t + 4 * kq)) & 1u);
-          __builtin_amdgcn_raw_buffer_store_b16(y, y_buf, at, 0, 0);
-          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(d_r), tape_buf, 2 * at, 0, 0);
-        }
+        for (int r = 0; r < 4; ++r) rows.template store_token<MASKED, TAPE>(ch, 16 * i + r, Y[r], D[i][r], on_bits, 0);
       }
-      load_l(next);
-      if (!kEarly) load_vec(next, 0, cv), load_vec(next, 1, cfv);
+      load_matrices(next, 1, lf);
+      load_vecs(next);
       DFLASH_KEEP_REQUESTS();
     }
-    if (ch < a.chunks) token_by_token(ch++);
+    if (ch < a.chunks) rows.token_by_token(ch++, st);
   }
-#undef DFLASH_KEEP_REQUESTS
-
-#pragma unroll
-  for (int C = 0; C < NC; ++C)
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const f32x4_t entry = st[2 * C + h];
-      if (a.state_dtype == DFLASH_FP32) {
-        *reinterpret_cast<f32x4_t*>((float*)a.state_out + srow + 32 * C + 4 * h) = entry;
-      } else {
-        uint32_t b[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) b[e] = a.state_dtype == DFLASH_BF16 ? f32_to_bf16_bits(entry[e]) : f32_to_f16_bits(entry[e]);
-        *reinterpret_cast<uint2*>((uint16_t*)a.state_out + srow + 32 * C + 4 * h) = uint2{b[0] | (b[1] << 16), b[2] | (b[3] << 16)};
-      }
-    }
+  rows.store_state(0, st);
 }
+
+// A wave for every 32 elements of the rows.  What bounds it is the chain from a chunk's state to the next one's: S is cut into pieces, the
+// waves' parts of U meet in LDS (the chunk's one barrier), and all of them compute Delta from the same sums in the same order and their
+// part of the next S.  Q S0^T, Lq Delta and the stores are nobody's input: two more waves, a tile of tokens each, find the pieces of S
+// and Delta in LDS and do a chunk's while the next one is under way.  Another two bring what all waves of the chain read, M', V and the
+// vectors, to LDS, and the lines of later chunks to the L2.
+//   barrier of chunk n: its parts of U, pieces of S, M', V and vectors are there, and Delta of chunk n - 1
+// A chunk with numbers that are not finite ends in three more: S is in LDS; one wave has walked the chunk token by token; S is out of LDS again.
+template <int DK, bool MASKED, bool TAPE>
+__global__ __launch_bounds__(64 * (DK / 32 + 4)) __attribute__((amdgpu_waves_per_eu(1, 2))) void gdn_prompt_spread_kernel(Args a) {
+  constexpr int kWaves = DK / 32;
+  constexpr int kPitchS = DK + 4;
+  __shared__ f32x4_t parts[2][kWaves][2][64];
+  __shared__ uint4 pieces[2][kWaves][3][64];
+  __shared__ f32x4_t deltas[2][2][64];
+  __shared__ uint4 matrix[2][2][3][64];              // M'
+  __shared__ __align__(16) Columns values[2];        // V
+  __shared__ f32x4_t vectors[2][(kTail + 4) / 4];
+  __shared__ int walked[2];
+  static_assert(sizeof(pieces[0]) >= 16 * kPitchS * sizeof(float), "a chunk's pieces leave room for S");
+  const Rows<DK> rows(a);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = rows.lane, kq = rows.kq;
+  // what the waves hand over through LDS is there; requests to memory stay in flight
+  auto meet = [&]() __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+
+  // Where a chunk turned out not to be finite: the two barriers of its walk, and that of the chunk behind it (or the last one).
+  auto sit_out = [&](int ch) __attribute__((always_inline)) {
+    if (!__builtin_amdgcn_readfirstlane(walked[ch & 1])) return false;
+    meet();
+    meet();
+    meet();
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): a loop's waits are for the requests of the loop
+    return true;
+  };
+  if (wave >= kWaves + 2) {  // M', V and the vectors, a chunk ahead
+    const int half = wave - kWaves - 2;
+    uint4 m0, m1, m2, other;
+    auto load_shared = [&](int ch) __attribute__((always_inline)) {
+      ch = ch < a.chunks ? ch : a.chunks - 1;
+      uint4 m[3];
+      rows.load_matrix(ch, 0, half, m);
+      m0 = m[0], m1 = m[1], m2 = m[2];  // (as an array across the loop they went to memory)
+      other = rows.load_columns(ch, half != 0);
+    };
+    auto store_shared = [&](int ch) __attribute__((always_inline)) {
+      matrix[ch & 1][half][0][lane] = m0, matrix[ch & 1][half][1][lane] = m1, matrix[ch & 1][half][2][lane] = m2;
+      if (half == 0) *reinterpret_cast<uint4*>(&values[ch & 1][lane >> 1][8 * (lane & 1)]) = other;
+      else if (lane < (kTail + 4) / 4) vectors[ch & 1][lane] = __builtin_bit_cast(f32x4_t, other);
+    };
+    load_shared(0);
+    store_shared(0);
+    load_shared(1);
+    uint32_t touched = rows.touch(2, half);
+    Rows<DK>::keep(rows.touch(3, half));
+    meet();
+    store_shared(1);
+    load_shared(2);
+    __builtin_amdgcn_s_waitcnt(0x0f70);
+    for (int ch = 1;; ++ch) {
+      meet();
+      sit_out(ch - 1);
+      if (ch == a.chunks) return;
+      store_shared(ch + 1);  // (behind the last chunk: the last one, which nobody reads)
+      load_shared(ch + 2);
+      Rows<DK>::keep(touched);
+      touched = rows.touch(ch + 4, half);
+    }
+  }
+  if (wave >= kWaves) {
+    const int tile = wave - kWaves;
+    uint4 qf[kWaves], lf[3];
+    f32x4_t c, W;
+    uint32_t on_bits;
+    // Q S^T: every wave's part as it would add it up, then the waves in their order
+    auto times_state = [&](int ch) __attribute__((always_inline)) {
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) {
+        f32x4_t part = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int p = 2; p >= 0; --p) part = mfma(qf[w], pieces[ch & 1][w][p][lane], part);
+        W = w == 0 ? part : W + part;
+      }
+      c = vectors[ch & 1][4 * tile + kq];
+      on_bits = __float_as_uint(vectors[ch & 1][kTail / 4][2]);
+      rows.load_rows(rows.q_buf, ch + 1 < a.chunks ? ch + 1 : ch, tile, 0, qf);
+    };
+    rows.load_rows(rows.q_buf, 0, tile, 0, qf);
+    rows.load_matrix(0, 1, tile, lf);
+    meet();
+    times_state(0);
+    __builtin_amdgcn_s_waitcnt(0x0f70);
+    for (int ch = 1;; ++ch) {
+      meet();
+      const uint32_t nowhere = sit_out(ch - 1) ? 0x80000000u : 0u;  // (whose results somebody else has stored)
+      const f32x4_t D0 = deltas[(ch - 1) & 1][0][lane], D1 = deltas[(ch - 1) & 1][1][lane], mine = tile ? D1 : D0;
+      const f32x4_t Y = product6(lf, split_tiles(D0, D1), W * c);
+      rows.load_matrix(ch < a.chunks ? ch : ch - 1, 1, tile, lf);
+      DFLASH_KEEP_REQUESTS();
+      // (before the stores: a wait for what was asked for behind them is a wait for them)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) rows.template store_token<MASKED, TAPE>(ch - 1, 16 * tile + r, Y[r], mine[r], on_bits, nowhere);
+      if (ch == a.chunks) return;
+      DFLASH_KEEP_REQUESTS();
+      times_state(ch);
+      DFLASH_KEEP_REQUESTS();
+    }
+  }
+
+  __builtin_amdgcn_s_setprio(2);  // the others have a chunk's time for what they do
+  f32x4_t st[2];
+  rows.load_state(wave, st);
+  uint4 kf[2][1], kt[2];
+  auto load_k = [&](int ch) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) rows.load_rows(rows.k_buf, ch, i, wave, kf[i]);
+  };
+  load_k(0);
+  DFLASH_KEEP_REQUESTS();  // in the order of the loop
+  rows.load_kt(0, wave, kt);
+  DFLASH_KEEP_REQUESTS();
+#pragma unroll 1
+  for (int ch = 0; ch < a.chunks; ++ch) {
+    const int next = ch + 1 < a.chunks ? ch + 1 : ch, now = ch & 1;
+    f32x4_t U[2];
+    {
+      const Pieces<8> sp = split_tiles(st[0], st[1]);
+      uint4* const to = &pieces[now][wave][0][lane];
+      to[0] = uint4{sp.hi[0], sp.hi[1], sp.hi[2], sp.hi[3]};
+      to[64] = uint4{sp.mid[0], sp.mid[1], sp.mid[2], sp.mid[3]};
+      to[128] = uint4{sp.lo[0], sp.lo[1], sp.lo[2], sp.lo[3]};
+#pragma unroll
+      for (int i = 0; i < 2; ++i) U[i] = mfma(kf[i][0], sp.lo, f32x4_t{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+      for (int i = 0; i < 2; ++i) U[i] = mfma(kf[i][0], sp.mid, U[i]);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) U[i] = mfma(kf[i][0], sp.hi, U[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) parts[now][wave][i][lane] = U[i];
+    load_k(next);
+    DFLASH_KEEP_REQUESTS();
+    meet();
+    f32x4_t part[2][kWaves], cv[2], cfv[2];
+    uint4 mf[2][3];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) part[i][w] = parts[now][w][i][lane];
+    Values v;
+    v.read(values[now], rows.li, kq);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) cv[i] = vectors[now][4 * i + kq];
+    const f32x4_t tail = vectors[now][kTail / 4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int p = 0; p < 3; ++p) mf[i][p] = matrix[now][i][p][lane];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) cfv[i] = vectors[now][kChunk / 4 + 4 * i + kq];
+    __builtin_amdgcn_sched_barrier(0);  // all of them asked for before the first is awaited
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {  // the sums over the waves, in their order: the same numbers in every wave
+      U[i] = part[i][0];
+#pragma unroll
+      for (int w = 1; w < kWaves; ++w) U[i] += part[i][w];
+    }
+    const Pieces<8> rp = right_side<MASKED>(v, cv, U, __float_as_uint(tail[2]), kq);
+    f32x4_t D[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) D[i] = product6(mf[i], rp, f32x4_t{0.f, 0.f, 0.f, 0.f});
+    if (wave < 2) deltas[now][wave][lane] = wave ? D[1] : D[0];
+    // a number that is not finite in V, U (and so in S) or M' is one in every Delta of its column; the same in every wave
+    float finite = tail[1];  // stays zero
+#pragma unroll
+    for (int j = 0; j < 8; ++j) finite = fmaf(D[j >> 2][j & 3], 0.f, finite);
+    const bool all_finite = __all(finite == 0.f);
+    if (wave == 0 && lane == 0) walked[now] = !all_finite;
+    if (all_finite) {
+      const Pieces<8> dp = split_tiles(D[0] * cfv[0], D[1] * cfv[1]);
+#pragma unroll
+      for (int c = 0; c < 2; ++c) st[c] = mfma(kt[c], dp.lo, st[c] * tail[0]);
+#pragma unroll
+      for (int c = 0; c < 2; ++c) st[c] = mfma(kt[c], dp.mid, st[c]);
+#pragma unroll
+      for (int c = 0; c < 2; ++c) st[c] = mfma(kt[c], dp.hi, st[c]);
+    } else {
+      // (the pieces of the chunk before are nobody's any more)
+      float* const held = reinterpret_cast<float*>(&pieces[now ^ 1][0][0][0]) + rows.li * kPitchS + 8 * kq;
+#pragma unroll
+      for (int c = 0; c < 2; ++c) *reinterpret_cast<f32x4_t*>(held + 32 * wave + 4 * c) = st[c];
+      meet();
+      if (wave == 0) {
+        f32x4_t all[DK / 16];
+#pragma unroll
+        for (int c = 0; c < DK / 16; ++c) all[c] = *reinterpret_cast<const f32x4_t*>(held + 32 * (c >> 1) + 4 * (c & 1));
+        rows.token_by_token(ch, all);
+#pragma unroll
+        for (int c = 0; c < DK / 16; ++c) *reinterpret_cast<f32x4_t*>(held + 32 * (c >> 1) + 4 * (c & 1)) = all[c];
+      }
+      meet();
+#pragma unroll
+      for (int c = 0; c < 2; ++c) st[c] = *reinterpret_cast<const f32x4_t*>(held + 32 * wave + 4 * c);
+      meet();  // (the next chunk's pieces take its place)
+      __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0), as above
+    }
+    rows.load_kt(next, wave, kt);
+    DFLASH_KEEP_REQUESTS();
+  }
+  meet();  // Delta of the last chunk
+  rows.store_state(wave, st);
+}
+#undef DFLASH_KEEP_REQUESTS
 
 template <int DK>
 int launch(const Args& a, hipStream_t s) {
   hipLaunchKernelGGL((gdn_chunk_kernel<DK>), dim3((unsigned)(a.slots * a.chunks * a.Hv)), dim3(256), 0, s, a);
   const int groups = a.slots * a.Hv * (a.Dv / 16);
   const bool spread = groups <= kSpread;
-  const void* fn = a.mask != nullptr ? (spread ? (const void*)gdn_prompt_kernel<DK, true, DK / 32> : (const void*)gdn_prompt_kernel<DK, true, 1>)
-                                     : (spread ? (const void*)gdn_prompt_kernel<DK, false, DK / 32> : (const void*)gdn_prompt_kernel<DK, false, 1>);
+  const bool masked = a.mask != nullptr, tape = a.tape != nullptr;
+#define DFLASH_PROMPT_FORMS(KERNEL_) \
+  (masked ? (tape ? (const void*)KERNEL_<DK, true, true> : (const void*)KERNEL_<DK, true, false>) \
+          : (tape ? (const void*)KERNEL_<DK, false, true> : (const void*)KERNEL_<DK, false, false>))
+  const void* const fn = spread ? DFLASH_PROMPT_FORMS(gdn_prompt_spread_kernel) : DFLASH_PROMPT_FORMS(gdn_prompt_kernel);
+#undef DFLASH_PROMPT_FORMS
   Args args = a;
   void* argv[] = {&args};
-  DFLASH_HIP_OK(hipLaunchKernel(fn, dim3((unsigned)groups), dim3(spread ? 2 * DK : 64), argv, 0, s));
+  DFLASH_HIP_OK(hipLaunchKernel(fn, dim3((unsigned)groups), dim3(spread ? 64 * (DK / 32 + 4) : 64), argv, 0, s));
   DFLASH_HIP_OK(hipGetLastError());
   return DFLASH_OK;
 }

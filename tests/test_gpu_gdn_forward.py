@@ -459,3 +459,29 @@ def test_prompts_of_few_heads_and_of_many(native_lib, shape, masked, value):
         _same_values(s2, s, 4e-5)
         _same_values(tape2, tape, 4e-5)
         _same_values(y2, y, 2.0 ** -7)
+
+
+@pytest.mark.parametrize("shape", [dict(T=100, B=1), dict(T=33, B=33), dict(T=40, B=2, Hk=1, Hv=1, Dv=16), dict(T=32, B=2, Dk=64, Dv=48)])
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("at", [None, 3, 31])
+def test_a_prompt_without_its_tape_has_the_bits_of_one_with_it(native_lib, shape, masked, at):
+    """Rows of a state on several waves and on one, chunks walked token by token (the first, with others behind it, and the last)."""
+    args = _case(seed=90 + shape["T"], **shape)
+    B, T, Hv, Dv = args[2].shape
+    mask = None
+    if masked:
+        mask = torch.rand((B, T), generator=torch.Generator().manual_seed(T)) > 0.3
+    if at is not None:
+        args[2][0, at, 0, 5] = float("inf")
+        args[1][-1, at, 0, 7] = 1e25  # k . k leaves the range, the recurrence does not
+    on_device = [t.to(DEV) for t in args]
+    m = None if mask is None else mask.to(DEV)
+    y, state, tape = gated_delta_kernel_with_tape(*on_device, m)
+    y2, state2, none = gated_delta_kernel_with_tape(*on_device, m, with_tape=False)
+    assert none is None and tape is not None
+
+    def bits(t):
+        return t.view(torch.int16 if t.element_size() == 2 else torch.int32)
+
+    for a, b in ((y, y2), (state, state2)):  # (a NaN is a NaN)
+        assert torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(bits(torch.nan_to_num(a)), bits(torch.nan_to_num(b)))
