@@ -5,6 +5,8 @@
 // pointer and number converted for ctypes.  Here the same is done on the tensors themselves.  One verify_matmul of
 // 1024 x 512 13.9 -> 6.9 us (its device time: 6.0), a GatedDeltaNet layer's verify block with its rollback 106 -> 51 us (49),
 // the attention layer of one over 4096 keys 81 -> 54 us, one token through the projections of a 9B-shaped layer 61 -> 44 us.
+// Results that skip the dispatcher and a block's operands read from the joint product: the call 5.6 -> 4.8 us, the recurrent
+// layer's block of a 1024-wide model, which waits for its host, 43.6 -> 33.7, one token 34.9 -> 27.6.
 //
 // Each function serves the ordinary form of a call - strided device tensors of the exact extents, in one piece - and
 // returns None for every other form and for whatever it would have to refuse: the Python function that asked then goes on
@@ -15,6 +17,8 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/EmptyTensor.h>
+#include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/Device.h>
@@ -97,6 +101,15 @@ int released(F&& work) {
   return work();
 }
 
+// A new tensor beside `like`: at::empty without the way through the dispatcher, half of its 0.5 us.  A verify block of a recurrent layer
+// with its rollback makes ten.
+Tensor fresh(at::IntArrayRef shape, const Tensor& like, at::ScalarType type) {
+  c10::Allocator* const allocator = like.storage().allocator();
+  if (allocator == nullptr || c10::hip::current_device() != like.device().index()) return at::empty(shape, like.options().dtype(type));
+  return Tensor(at::detail::empty_generic(shape, allocator, c10::DispatchKeySet(c10::DispatchKey::CUDA), type, std::nullopt));
+}
+Tensor fresh(at::IntArrayRef shape, const Tensor& like) { return fresh(shape, like, like.scalar_type()); }
+
 std::vector<int64_t> rows_by(const Tensor& x, int64_t n) {
   std::vector<int64_t> shape(x.sizes().begin(), x.sizes().end());
   shape.back() = n;
@@ -140,7 +153,7 @@ PyObject* qmm_m16(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Tensor ws, y;
   if (need != 0 && !(ws = kept_workspace(a[6], by_index(*p.x, stream), need)).defined()) Py_RETURN_NONE;
   const int rc = released([&] {
-    y = at::empty(rows_by(*p.x, p.N), p.x->options());
+    y = fresh(rows_by(*p.x, p.N), *p.x);
     return dflash_qmm_m16(at_of(*p.x), (const uint32_t*)at_of(*p.w), at_of(*p.s), at_of(*p.b), y.mutable_data_ptr(),
                           need ? ws.mutable_data_ptr() : nullptr, need ? ws.nbytes() : 0, p.K, p.N, p.group, p.act, p.sb,
                           variant, parts, kernel, stream);
@@ -165,7 +178,7 @@ PyObject* qmm_packed(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Tensor y, ws = kept_workspace(a[8], by_index(*x, stream), need);
   if (!ws.defined()) Py_RETURN_NONE;
   const int rc = released([&] {
-    y = at::empty(rows_by(*x, N), x->options());
+    y = fresh(rows_by(*x, N), *x);
     return dflash_qmm_m16_packed_by(at_of(*x), at_of(*w), at_of(*s), at_of(*b), y.mutable_data_ptr(), ws.mutable_data_ptr(),
                                     ws.nbytes(), K, N, group, act, sb, kernel, stream);
   });
@@ -185,7 +198,7 @@ PyObject* qmm_few(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Tensor ws, y;
   if (need != 0 && !(ws = kept_workspace(a[6], by_index(*p.x, stream), need)).defined()) Py_RETURN_NONE;
   const int rc = released([&] {
-    y = at::empty(rows_by(*p.x, p.N), p.x->options());
+    y = fresh(rows_by(*p.x, p.N), *p.x);
     return dflash_qmm_few(at_of(*p.x), (const uint32_t*)at_of(*p.w), at_of(*p.s), at_of(*p.b), y.mutable_data_ptr(),
                           need ? ws.mutable_data_ptr() : nullptr, need ? ws.nbytes() : 0, (int)p.rows, p.K, p.N, p.group,
                           p.act, p.sb, kernel, stream);
@@ -207,7 +220,7 @@ PyObject* qmm_few_silu_mul(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Tensor y, ws = kept_workspace(a[6], by_index(*p.x, stream), need);
   if (!ws.defined()) Py_RETURN_NONE;
   const int rc = released([&] {
-    y = at::empty(rows_by(*p.x, p.N / 2), p.x->options());
+    y = fresh(rows_by(*p.x, p.N / 2), *p.x);
     return dflash_qmm_few_silu_mul_by(at_of(*p.x), (const uint32_t*)at_of(*p.w), at_of(*p.s), at_of(*p.b), y.mutable_data_ptr(),
                                    ws.mutable_data_ptr(), ws.nbytes(), (int)p.rows, p.K, p.N, p.group, p.act, kernel, stream);
   });
@@ -233,7 +246,7 @@ PyObject* qmm_rows(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!(ws = kept_workspace(a[6], by_index(*p.x, stream), need)).defined()) Py_RETURN_NONE;
   }
   const int rc = released([&] {
-    y = at::empty(rows_by(*p.x, silu ? p.N / 2 : p.N), p.x->options());
+    y = fresh(rows_by(*p.x, silu ? p.N / 2 : p.N), *p.x);
     return dflash_qmm_rows(at_of(*p.x), (const uint32_t*)at_of(*p.w), at_of(*p.s), at_of(*p.b), y.mutable_data_ptr(),
                            need ? ws.mutable_data_ptr() : nullptr, need ? ws.nbytes() : 0, (int)p.rows, p.K, p.N, p.group,
                            p.act, p.sb, epilogue, stream);
@@ -267,7 +280,7 @@ PyObject* gather(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Tensor ws, y;
   if (need != 0 && !(ws = kept_workspace(a[7], by_index(*x, stream), need)).defined()) Py_RETURN_NONE;
   const int rc = released([&] {
-    y = at::empty(rows_by(*x, N), x->options());
+    y = fresh(rows_by(*x, N), *x);
     return dflash_qmm_m16_gather_by(at_of(*x), (const int32_t*)at_of(*ids), (const uint32_t*)at_of(*w), at_of(*s), at_of(*b),
                                     y.mutable_data_ptr(), need ? ws.mutable_data_ptr() : nullptr, need ? ws.nbytes() : 0, (int)P,
                                     (int)K, (int)N, (int)E, group, act, sb, kernel, stream);
@@ -288,7 +301,7 @@ PyObject* chain_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (problem == nullptr || problem->wait_for >= 0 || x->dim() < 1 || x->size(-1) != problem->K || x->numel() != 16 * (int64_t)problem->K ||
       !x->is_contiguous() || x->scalar_type() != before->scalar_type() || x->device() != before->device())
     Py_RETURN_NONE;
-  Tensor out = at::empty(rows_by(*x, cols), x->options());
+  Tensor out = fresh(rows_by(*x, cols), *x);
   problem->x = at_of(*x);
   problem->y = out.mutable_data_ptr();
   return THPVariable_Wrap(std::move(out));
@@ -381,13 +394,12 @@ PyObject* gdn_prepare(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const float eps = (float)PyFloat_AS_DOUBLE(a[12]);
   Tensor next, q, k, v, g, beta;
   const int rc = released([&] {
-    const auto options = qkv->options();
-    next = at::empty({B, K - 1, C}, options);
-    q = at::empty({B, S, Hk, Dk}, options);
-    k = at::empty({B, S, Hk, Dk}, options);
-    v = at::empty({B, S, Hv, Dv}, options);
-    g = at::empty({B, S, Hv}, options.dtype(at::kFloat));
-    beta = at::empty({B, S, Hv}, options);
+    next = fresh({B, K - 1, C}, *qkv);
+    q = fresh({B, S, Hk, Dk}, *qkv);
+    k = fresh({B, S, Hk, Dk}, *qkv);
+    v = fresh({B, S, Hv, Dv}, *qkv);
+    g = fresh({B, S, Hv}, *qkv, at::kFloat);
+    beta = fresh({B, S, Hv}, *qkv);
     return dflash_gdn_prepare_rows(at_of(*qkv), cs ? at_of(*cs) : nullptr, at_of(*w), at_of(*ga), at_of(*gb), at_of(*A), at_of(*dt),
                                    nullptr, next.mutable_data_ptr(), q.mutable_data_ptr(), k.mutable_data_ptr(),
                                    v.mutable_data_ptr(), (float*)g.mutable_data_ptr(), beta.mutable_data_ptr(),
@@ -445,11 +457,10 @@ PyObject* gdn_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const float eps = (float)PyFloat_AS_DOUBLE(a[8]);
   Tensor y, next, tape, ws;
   const int rc = released([&] {
-    const auto options = q->options();
-    y = at::empty({B, T, hv, dv}, options);
-    if (need != 0) ws = at::empty({(int64_t)need}, options.dtype(at::kByte));
-    if (with_tape) tape = at::empty({B, T, hv, dv}, options.dtype(at::kFloat));
-    next = at::empty({B, hv, dv, dk}, state ? state->options() : options);
+    y = fresh({B, T, hv, dv}, *q);
+    if (need != 0) ws = fresh({(int64_t)need}, *q, at::kByte);
+    if (with_tape) tape = fresh({B, T, hv, dv}, *q, at::kFloat);
+    next = fresh({B, hv, dv, dk}, state ? *state : *q);
     return dflash_gdn_forward(at_of(*q), at_of(*k), at_of(*v), at_of(*g), at_of(*beta), state ? at_of(*state) : nullptr, next.mutable_data_ptr(),
                               z ? at_of(*z) : nullptr, z ? at_of(*w) : nullptr, y.mutable_data_ptr(),
                               with_tape ? (float*)tape.mutable_data_ptr() : nullptr, nullptr,
@@ -462,79 +473,100 @@ PyObject* gdn_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// gdn_block(qkv, conv_state, conv_w, a, b, A_log, dt_bias, z, weight, state, Hk, Hv, Dk, Dv, eps, norm_eps, record): a block of
-// up to 16 tokens without a mask in one launch, where that has a form for it; z [B, S, Hv Dv] and the norm's weight None, or what
-// the output norm takes; state None: zeros of qkv's type, filled once the call is known to be served.  (y, state, conv_next, tape, k, g, qkv in one piece); the last three None unless recorded, the last
-// one also where qkv is in one piece already.
-PyObject* gdn_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  HANDLE_TH_ERRORS
-  if (n != 17) Py_RETURN_NONE;
-  const Tensor *qkv = device_tensor(a[0]), *cs = nullptr, *w = device_tensor(a[2]), *ga = device_tensor(a[3]),
-               *gb = device_tensor(a[4]), *A = device_tensor(a[5]), *dt = device_tensor(a[6]), *z = nullptr, *weight = nullptr,
+// [B, S, width] of a product of three extents: all of it, or some of its columns.
+struct Columns {
+  const Tensor* of = nullptr;
+  int64_t first = 0, width = 0;
+  const void* at() const { return static_cast<const char*>(at_of(*of)) + first * of->element_size(); }
+  int64_t slot() const { return of->stride(0); }
+  int64_t row() const { return of->stride(1); }
+  bool whole() const { return width == of->size(2) && of->is_contiguous(); }
+  bool is(int64_t B, int64_t S, int64_t n, at::ScalarType type, c10::Device device) const {
+    return of->dim() == 3 && of->size(0) == B && of->size(1) == S && width == n && of->scalar_type() == type && of->device() == device &&
+           of->stride(2) == 1;
+  }
+};
+bool columns_of(PyObject* o, Columns* c) {
+  c->of = device_tensor(o);
+  if (c->of == nullptr || c->of->dim() != 3) return false;
+  c->width = c->of->size(2);
+  return true;
+}
+bool columns_of(const Tensor& product, PyObject* pair, Columns* c) {
+  long lo, hi;
+  if (!PyTuple_CheckExact(pair) || PyTuple_GET_SIZE(pair) != 2 || !integer(PyTuple_GET_ITEM(pair, 0), &lo) ||
+      !integer(PyTuple_GET_ITEM(pair, 1), &hi) || lo > hi || hi > product.size(2))
+    return false;
+  c->of = &product, c->first = lo, c->width = hi - lo;
+  return true;
+}
+
+// The launch behind gdn_block and gdn_block_of: a block of up to 16 tokens without a mask, where that has a form for it; rest: conv_state, conv_w,
+// A_log, dt_bias, weight, state, Hk, Hv, Dk, Dv, eps, norm_eps, record.  z.of null: no output norm.
+PyObject* block_of(const Columns& qkv, const Columns& z, const Columns& b, const Columns& a, PyObject* const (&rest)[13]) {
+  const Tensor *cs = nullptr, *w = device_tensor(rest[1]), *A = device_tensor(rest[2]), *dt = device_tensor(rest[3]), *weight = nullptr,
                *state = nullptr;
-  if (!qkv || !w || !ga || !gb || !A || !dt || qkv->dim() != 3) Py_RETURN_NONE;
-  if (a[9] != Py_None && !(state = device_tensor(a[9]))) Py_RETURN_NONE;
-  if (a[1] != Py_None && !(cs = device_tensor(a[1]))) Py_RETURN_NONE;
-  if (a[7] != Py_None && (!(z = device_tensor(a[7])) || !(weight = device_tensor(a[8])))) Py_RETURN_NONE;
+  if (!w || !A || !dt) Py_RETURN_NONE;
+  if (rest[0] != Py_None && !(cs = device_tensor(rest[0]))) Py_RETURN_NONE;
+  if (z.of && !(weight = device_tensor(rest[4]))) Py_RETURN_NONE;
+  if (rest[5] != Py_None && !(state = device_tensor(rest[5]))) Py_RETURN_NONE;
   int Hk, Hv, D, Dv;
-  if (!integer(a[10], &Hk) || !integer(a[11], &Hv) || !integer(a[12], &D) || !integer(a[13], &Dv) || !PyFloat_CheckExact(a[14]) ||
-      !PyFloat_CheckExact(a[15]))
+  if (!integer(rest[6], &Hk) || !integer(rest[7], &Hv) || !integer(rest[8], &D) || !integer(rest[9], &Dv) || !PyFloat_CheckExact(rest[10]) ||
+      !PyFloat_CheckExact(rest[11]))
     Py_RETURN_NONE;
-  const bool record = a[16] == Py_True;
-  const int64_t B = qkv->size(0), S = qkv->size(1), C = qkv->size(2);
+  const bool record = rest[12] == Py_True;
+  const Tensor& first = *qkv.of;
+  const int64_t B = first.size(0), S = first.size(1), C = qkv.width;
   const auto type = at::kBFloat16;
-  const auto device = qkv->device();
+  const auto device = first.device();
   const int param = dtype_code(A->scalar_type()), s_code = state ? dtype_code(state->scalar_type()) : DFLASH_BF16;
-  if (qkv->scalar_type() != type || param == kNoCode || s_code == kNoCode || D != Dv || (D != 64 && D != 128) || B < 1 || S < 1 ||
-      S > 16 || Hk < 1 || Hv < 1 || Hk > (1 << 15) || Hv > (1 << 15) || Hv % Hk != 0 || C != 2 * (int64_t)Hk * D + (int64_t)Hv * D ||
+  if (param == kNoCode || s_code == kNoCode || D != Dv || (D != 64 && D != 128) || B < 1 || S < 1 ||
+      S > 16 || Hk < 1 || Hv < 1 || Hk > (1 << 15) || Hv > (1 << 15) || Hv % Hk != 0 ||
+      !qkv.is(B, S, 2 * (int64_t)Hk * D + (int64_t)Hv * D, type, device) ||
       B * S * (2 * Hk + Hv) * D >= (1ll << 31) || dflash_get_option(DFLASH_OPT_GDN_STEP_BY_STEP) != 0)
     Py_RETURN_NONE;
   if (w->dim() < 2 || w->dim() > 3 || w->size(0) != C || w->size(1) != 4 || (w->dim() == 3 && w->size(2) != 1) ||
-      !w->is_contiguous() || w->scalar_type() != type || ga->scalar_type() != type || gb->scalar_type() != type ||
-      dt->scalar_type() != A->scalar_type() || !has_shape(*ga, {B, S, Hv}) || !has_shape(*gb, {B, S, Hv}) || !has_shape(*A, {Hv}) ||
-      !has_shape(*dt, {Hv}) || !A->is_contiguous() || !dt->is_contiguous())
+      !w->is_contiguous() || w->scalar_type() != type || !a.is(B, S, Hv, type, device) || !b.is(B, S, Hv, type, device) ||
+      dt->scalar_type() != A->scalar_type() || !has_shape(*A, {Hv}) || !has_shape(*dt, {Hv}) || !A->is_contiguous() || !dt->is_contiguous())
     Py_RETURN_NONE;
-  for (const Tensor* t : {w, ga, gb, A, dt})
+  for (const Tensor* t : {w, A, dt})
     if (t->device() != device) Py_RETURN_NONE;
   if (state && (!has_shape(*state, {B, Hv, D, D}) || !state->is_contiguous() || !aligned(at_of(*state), 16) || state->device() != device))
     Py_RETURN_NONE;
   if (cs && (cs->scalar_type() != type || !has_shape(*cs, {B, 3, C}) || cs->device() != device || !cs->is_contiguous() ||
              !aligned(at_of(*cs), 8)))
     Py_RETURN_NONE;
-  if (qkv->stride(2) != 1 || !aligned(at_of(*qkv), 8) || (qkv->stride(0) | qkv->stride(1)) % 4 != 0 || qkv->stride(1) >= (1 << 26) || !aligned(at_of(*w), 8) ||
-      ga->stride(2) != 1 || gb->stride(2) != 1)
-    Py_RETURN_NONE;
-  if (z && (z->scalar_type() != type || !has_shape(*z, {B, S, (int64_t)Hv * D}) || z->device() != device || z->stride(2) != 1 ||
-            (z->stride(0) | z->stride(1)) % 8 != 0 || !aligned(at_of(*z), 16) || dtype_code(weight->scalar_type()) == kNoCode ||
-            weight->numel() != D || !weight->is_contiguous() || weight->device() != device || !aligned(at_of(*weight), 16)))
+  if (!aligned(qkv.at(), 8) || (qkv.slot() | qkv.row()) % 4 != 0 || qkv.row() >= (1 << 26) || !aligned(at_of(*w), 8)) Py_RETURN_NONE;
+  if (z.of && (!z.is(B, S, (int64_t)Hv * D, type, device) || (z.slot() | z.row()) % 8 != 0 || !aligned(z.at(), 16) ||
+               dtype_code(weight->scalar_type()) == kNoCode || weight->numel() != D || !weight->is_contiguous() ||
+               weight->device() != device || !aligned(at_of(*weight), 16)))
     Py_RETURN_NONE;
   dflash_gdn_block_args p = {};
-  p.qkv = at_of(*qkv), p.conv_state = cs ? at_of(*cs) : nullptr, p.conv_w = at_of(*w), p.a = at_of(*ga), p.b = at_of(*gb);
+  p.qkv = qkv.at(), p.conv_state = cs ? at_of(*cs) : nullptr, p.conv_w = at_of(*w), p.a = a.at(), p.b = b.at();
   p.A_log = at_of(*A), p.dt_bias = at_of(*dt);
-  p.qkv_slot = qkv->stride(0), p.qkv_row = qkv->stride(1), p.a_slot = ga->stride(0), p.a_row = ga->stride(1);
-  p.b_slot = gb->stride(0), p.b_row = gb->stride(1);
-  if (z) p.z = at_of(*z), p.norm_weight = at_of(*weight), p.z_slot = z->stride(0), p.z_row = z->stride(1);
+  p.qkv_slot = qkv.slot(), p.qkv_row = qkv.row(), p.a_slot = a.slot(), p.a_row = a.row();
+  p.b_slot = b.slot(), p.b_row = b.row();
+  if (z.of) p.z = z.at(), p.norm_weight = at_of(*weight), p.z_slot = z.slot(), p.z_row = z.row();
   p.slots = (int)B, p.T = (int)S, p.Hk = Hk, p.Hv = Hv, p.D = D, p.param_dtype = param, p.state_dtype = s_code;
-  p.weight_dtype = z ? dtype_code(weight->scalar_type()) : DFLASH_BF16;
-  p.eps = (float)PyFloat_AS_DOUBLE(a[14]), p.norm_eps = (float)PyFloat_AS_DOUBLE(a[15]);
-  void* stream = stream_of(*qkv);
+  p.weight_dtype = z.of ? dtype_code(weight->scalar_type()) : DFLASH_BF16;
+  p.eps = (float)PyFloat_AS_DOUBLE(rest[10]), p.norm_eps = (float)PyFloat_AS_DOUBLE(rest[11]);
+  void* stream = stream_of(first);
   Tensor y, next, conv, tape, k, g, one, zeros;
   const int rc = released([&] {
-    const auto options = qkv->options();
-    if (!state) zeros = at::zeros({B, Hv, D, D}, options), state = &zeros;
+    if (!state) zeros = at::zeros({B, Hv, D, D}, first.options()), state = &zeros;
     p.state_in = at_of(*state);
-    y = at::empty({B, S, Hv, D}, options);
-    next = at::empty({B, Hv, D, D}, state->options());
-    conv = at::empty({B, 3, C}, options);
-    tape = at::empty({B, S, Hv, D}, options.dtype(at::kFloat));
+    y = fresh({B, S, (int64_t)Hv * D}, first);
+    next = fresh({B, Hv, D, D}, *state);
+    conv = fresh({B, 3, C}, first);
+    tape = fresh({B, S, Hv, D}, first, at::kFloat);
     p.y = y.mutable_data_ptr(), p.state_out = next.mutable_data_ptr(), p.conv_next = conv.mutable_data_ptr();
     p.tape = (float*)tape.mutable_data_ptr();
     if (record) {
-      k = at::empty({B, S, Hk, D}, options);
-      g = at::empty({B, S, Hv}, options.dtype(at::kFloat));
+      k = fresh({B, S, Hk, D}, first);
+      g = fresh({B, S, Hv}, first, at::kFloat);
       p.k = k.mutable_data_ptr(), p.g = (float*)g.mutable_data_ptr();
-      if (!qkv->is_contiguous()) {
-        one = at::empty({B, S, C}, options);
+      if (!qkv.whole()) {
+        one = fresh({B, S, C}, first);
         p.qkv_out = one.mutable_data_ptr();
       }
     }
@@ -547,6 +579,32 @@ PyObject* gdn_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
   };
   return Py_BuildValue("(NNNNNNN)", wrapped(std::move(y)), wrapped(std::move(next)), wrapped(std::move(conv)), wrapped(std::move(tape)),
                        wrapped(std::move(k)), wrapped(std::move(g)), wrapped(std::move(one)));
+}
+
+// gdn_block(qkv, conv_state, conv_w, a, b, A_log, dt_bias, z, weight, state, Hk, Hv, Dk, Dv, eps, norm_eps, record): z [B, S, Hv Dv] and the norm's
+// weight None, or what the output norm takes; state None: zeros of qkv's type, filled once the call is known to be served.
+// (y [B, S, Hv Dv], state, conv_next, tape, k, g, qkv in one piece); the last three None unless recorded, the last one also where
+// qkv is in one piece already.
+PyObject* gdn_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Columns qkv, z, gb, ga;
+  if (n != 17 || !columns_of(a[0], &qkv) || !columns_of(a[3], &ga) || !columns_of(a[4], &gb) || (a[7] != Py_None && !columns_of(a[7], &z)))
+    Py_RETURN_NONE;
+  return block_of(qkv, z, gb, ga, {a[1], a[2], a[5], a[6], a[8], a[9], a[10], a[11], a[12], a[13], a[14], a[15], a[16]});
+  END_HANDLE_TH_ERRORS
+}
+
+// gdn_block_of(product, bounds, conv_state, conv_w, A_log, dt_bias, weight, state, Hk, Hv, Dk, Dv, eps, norm_eps, record): the same from the joint
+// product of the layer's input projections; bounds: the columns of qkv, z, b and a.  weight None: no output norm.
+PyObject* gdn_block_of(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  const Tensor* product = n == 15 ? device_tensor(a[0]) : nullptr;
+  Columns part[4];
+  if (product == nullptr || product->dim() != 3 || !PyList_CheckExact(a[1]) || PyList_GET_SIZE(a[1]) != 4) Py_RETURN_NONE;
+  for (int i = 0; i < 4; ++i)
+    if (!columns_of(*product, PyList_GET_ITEM(a[1], i), &part[i])) Py_RETURN_NONE;
+  if (a[6] == Py_None) part[1].of = nullptr;
+  return block_of(part[0], part[1], part[2], part[3], {a[2], a[3], a[4], a[5], a[6], a[7], a[8], a[9], a[10], a[11], a[12], a[13], a[14]});
   END_HANDLE_TH_ERRORS
 }
 
@@ -592,8 +650,8 @@ PyObject* rollback_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
   void* stream = stream_of(*r.state);
   Tensor next, conv;
   const int rc = released([&] {
-    next = at::empty({r.B, r.hv, r.dv, r.dk}, r.state->options());
-    conv = at::empty({r.B, keep, r.C}, r.qkv->options());
+    next = fresh({r.B, r.hv, r.dv, r.dk}, *r.state);
+    conv = fresh({r.B, keep, r.C}, *r.qkv);
     return dflash_rollback_layer(at_of(*r.tape), at_of(*r.k), at_of(*r.g), at_of(*r.state), next.mutable_data_ptr(),
                                  r.prev ? at_of(*r.prev) : nullptr, at_of(*r.qkv), conv.mutable_data_ptr(), nullptr, steps, (int)r.B,
                                  (int)r.T, (int)r.hk, (int)r.hv, (int)r.dk, (int)r.dv, r.s_code, r.t_code, r.k_code, r.g_code, 0,
@@ -631,10 +689,9 @@ PyObject* rollback_layers(PyObject*, PyObject* const* a, Py_ssize_t n) {
   void* stream = stream_of(*r.state);
   std::vector<Tensor> made(2 * count);
   const int rc = released([&] {
-    const auto state_options = r.state->options(), conv_options = r.qkv->options();
     for (Py_ssize_t i = 0; i < count; ++i) {
-      made[2 * i] = at::empty({r.B, keep, r.C}, conv_options);
-      made[2 * i + 1] = at::empty({r.B, r.hv, r.dv, r.dk}, state_options);
+      made[2 * i] = fresh({r.B, keep, r.C}, *r.qkv);
+      made[2 * i + 1] = fresh({r.B, r.hv, r.dv, r.dk}, *r.state);
       at[i].conv_out = made[2 * i].mutable_data_ptr(), at[i].state_out = made[2 * i + 1].mutable_data_ptr();
     }
     return dflash_rollback_layers(at.data(), (int)count, steps, (int)r.B, (int)r.T, (int)r.hk, (int)r.hv, (int)r.dk, (int)r.dv, r.s_code,
@@ -687,7 +744,7 @@ PyObject* attn_prepare(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (x->stride(2) != 1 || (x->stride(0) | x->stride(1)) % 4 != 0 || !aligned(at_of(*x), 8)) Py_RETURN_NONE;
   for (const Tensor* x : {&ck, &cv})
     if (x->stride(3) != 1 || (x->stride(0) | x->stride(1) | x->stride(2)) % 4 != 0 || !aligned(at_of(*x), 8)) Py_RETURN_NONE;
-  Tensor queries = at::empty({B, Hq, L, D}, q.options());
+  Tensor queries = fresh({B, Hq, L, D}, q);
   const auto address = [](const void* p, int64_t elements) { return (unsigned long long)(uintptr_t)p + 2 * (unsigned long long)elements; };
   PyObject* args = Py_BuildValue("(KKKKKKKKiiiiiii)", address(at_of(q), 0), address(at_of(k), 0), address(at_of(v), 0), address(at_of(qw), 0),
                                  address(at_of(kw), 0), address(queries.mutable_data_ptr(), 0),
@@ -731,16 +788,15 @@ PyObject* sdpa_q16(PyObject*, PyObject* const* a, Py_ssize_t n) {
                      (gate->stride(0) | gate->stride(1)) % 4 == 0 && aligned(at_of(*gate), 8);
   const float scale = (float)PyFloat_AS_DOUBLE(a[3]);
   const int rc = released([&] {
-    const auto options = q->options();
     void* scratch = need ? ws.mutable_data_ptr() : nullptr;
     const size_t bytes = need ? ws.nbytes() : 0;
     if (gated) {
-      out = at::empty({B, 16, hq * d}, options);
+      out = fresh({B, 16, hq * d}, *q);
       return dflash_sdpa_q16_gated(at_of(*q), at_of(*k), at_of(*v), nullptr, at_of(*gate), out.mutable_data_ptr(), scratch, bytes,
                                    (int)B, (int)hq, (int)hk, (int)N, (int)d, k->stride(0), k->stride(1), k->stride(2),
                                    v->stride(0), v->stride(1), v->stride(2), gate->stride(0), gate->stride(1), scale, code, stream);
     }
-    out = at::empty({B, hq, 16, d}, options);
+    out = fresh({B, hq, 16, d}, *q);
     return dflash_sdpa_q16(at_of(*q), at_of(*k), at_of(*v), nullptr, out.mutable_data_ptr(), scratch, bytes, (int)B, (int)hq,
                            (int)hk, (int)N, (int)d, k->stride(0), k->stride(1), k->stride(2), v->stride(0), v->stride(1),
                            v->stride(2), scale, code, stream);
@@ -806,7 +862,7 @@ PyObject* attn_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
   p.q_eps = (float)PyFloat_AS_DOUBLE(a[8]), p.k_eps = (float)PyFloat_AS_DOUBLE(a[9]);
   p.rope_base = (float)PyFloat_AS_DOUBLE(a[10]), p.scale = (float)PyFloat_AS_DOUBLE(a[11]);
   const int rc = released([&] {
-    out = at::empty({B, 16, Hq * D}, q.options());
+    out = fresh({B, 16, Hq * D}, q);
     p.out = out.mutable_data_ptr();
     return dflash_attn_block(&p, stream);
   });
@@ -824,7 +880,7 @@ PyObject* bind(PyObject*, PyObject* error) {  // the class that failed launches 
 
 #define DFLASH_HOST(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
 PyMethodDef kMethods[] = {DFLASH_HOST(qmm_m16), DFLASH_HOST(qmm_packed), DFLASH_HOST(qmm_few), DFLASH_HOST(qmm_few_silu_mul),
-                          DFLASH_HOST(qmm_rows), DFLASH_HOST(columns), DFLASH_HOST(gather), DFLASH_HOST(chain_bind), DFLASH_HOST(chain_launch), DFLASH_HOST(gdn_prepare), DFLASH_HOST(gdn_forward), DFLASH_HOST(gdn_block),
+                          DFLASH_HOST(qmm_rows), DFLASH_HOST(columns), DFLASH_HOST(gather), DFLASH_HOST(chain_bind), DFLASH_HOST(chain_launch), DFLASH_HOST(gdn_prepare), DFLASH_HOST(gdn_forward), DFLASH_HOST(gdn_block), DFLASH_HOST(gdn_block_of),
                           DFLASH_HOST(rollback_layer), DFLASH_HOST(rollback_layers), DFLASH_HOST(attn_prepare), DFLASH_HOST(sdpa_q16), DFLASH_HOST(first_rows), DFLASH_HOST(attn_block), {"bind", bind, METH_O, nullptr},
                           {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_dflash_host", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};

@@ -30,7 +30,7 @@ import torch.nn as nn
 from . import _native
 from .kernels import _DTYPE_CODE, fused_output_norm_applies, gated_delta_kernel_with_tape
 from .recurrent_rollback_cache import RecurrentRollbackCache
-from .verify_linear import shared_input_outputs
+from .verify_linear import joint_product, shared_input_outputs
 
 _EXACT_SMALL_PROJ_PAD_M = 16
 
@@ -246,32 +246,47 @@ class _DepthwiseConv1d(nn.Module):
         self.weight = nn.Parameter(torch.zeros((channels, kernel_size, 1), dtype=dtype), requires_grad=False)
 
 
+_IN_PROJ = ("in_proj_qkv", "in_proj_z", "in_proj_b", "in_proj_a")
+
+
 def _gdn_call(self, inputs: torch.Tensor, mask: Optional[torch.Tensor], cache: Optional[Any],
               record: bool) -> torch.Tensor:
     """The body shared by the plain and the speculative call (dflash_mlx/runtime.py:359-453)."""
     B, S, _ = inputs.shape
-    # one launch for those of the four that fuse_shared_input_linears joined
-    qkv, z, b, a = shared_input_outputs(self, ("in_proj_qkv", "in_proj_z", "in_proj_b", "in_proj_a"), inputs, columns=True)
-    conv_state = cache[0] if cache is not None else None
     norm = self.norm
     normed = isinstance(norm, RMSNormGated) and _native.env(b"DFLASH_GDN_FUSED_NORM") != b"0"
-    if mask is None and S <= 16 and qkv.is_cuda:
-        # a block: conv, gates, recurrence and norm in one launch, where there is one for these sizes and types
+    conv_state, state = (cache[0], cache[1]) if cache is not None else (None, None)
+    made = qkv = None
+    # one launch for those of the four that fuse_shared_input_linears joined
+    if mask is None and S <= 16 and normed and inputs.is_cuda:
+        # a block: conv, gates, recurrence and norm in one launch, where there is one for these sizes and types, which finds all four
+        # in the joint product (four views of it and the result's other shape are 2 us of host time)
+        joint = joint_product(self, _IN_PROJ, inputs)
+        if joint is not None:
+            group, qkv = joint
+            made = _native.host().gdn_block_of(
+                qkv, group.bounds, conv_state, self.conv1d.weight, self.A_log, self.dt_bias, norm.weight, state, self.num_k_heads,
+                self.num_v_heads, self.head_k_dim, self.head_v_dim, 1e-6, norm.eps, bool(record))
+            if made is None:
+                qkv, z, b, a = group._columns(qkv)
+    if qkv is None:
+        qkv, z, b, a = shared_input_outputs(self, _IN_PROJ, inputs, columns=True)
+    if made is None and mask is None and S <= 16 and qkv.is_cuda:
         made = _native.host().gdn_block(
             qkv, conv_state, self.conv1d.weight, a, b, self.A_log, self.dt_bias, z if normed else None, norm.weight if normed else None,
-            cache[1] if cache is not None else None, self.num_k_heads, self.num_v_heads, self.head_k_dim, self.head_v_dim, 1e-6,
-            norm.eps if normed else 0.0, bool(record))
-        if made is not None:
-            out, state, conv_next, tape, k, g, tape_qkv = made
-            if cache is not None:
-                cache[0] = conv_next
-            if record:
-                cache.record_tape(tape=tape, k=k, g=g, qkv=qkv if tape_qkv is None else tape_qkv)
-            if cache is not None:
-                cache[1] = state
-            if not normed:
-                out = norm(out, z.reshape(B, S, self.num_v_heads, self.head_v_dim).contiguous())
-            return self.out_proj(out.view(B, S, -1))
+            state, self.num_k_heads, self.num_v_heads, self.head_k_dim, self.head_v_dim, 1e-6, norm.eps if normed else 0.0, bool(record))
+    if made is not None:
+        out, state, conv_next, tape, k, g, tape_qkv = made
+        if cache is not None:
+            cache[0] = conv_next
+        if record:
+            cache.record_tape(tape=tape, k=k, g=g, qkv=qkv if tape_qkv is None else tape_qkv)
+        if cache is not None:
+            cache[1] = state
+        if not normed:
+            heads = (B, S, self.num_v_heads, self.head_v_dim)
+            out = norm(out.view(heads), z.reshape(heads).contiguous()).view(B, S, -1)
+        return self.out_proj(out)
     z = z.reshape(B, S, self.num_v_heads, self.head_v_dim)
 
     # the rollback wants qkv in one piece, without what the mask hides
@@ -285,7 +300,6 @@ def _gdn_call(self, inputs: torch.Tensor, mask: Optional[torch.Tensor], cache: O
     if cache is not None:
         cache[0] = conv_next
 
-    state = cache[1] if cache is not None else None
     made = None
     if state is None and mask is None and S > 16 and q.is_cuda:  # a prompt that starts from nothing: no zeros to write and read
         fused = normed

@@ -109,9 +109,11 @@ def _arm_target_rollback(cache_entries: List[Any]) -> None:
 
 
 def _arm_target_rollback_with_prefix(cache_entries: List[Any], *, prefix_len: int) -> None:
+    prefix_len = int(prefix_len)
     for cache_entry in cache_entries:
-        if hasattr(cache_entry, "arm_rollback"):
-            cache_entry.arm_rollback(prefix_len=int(prefix_len))
+        arm = getattr(cache_entry, "arm_rollback", None)
+        if arm is not None:
+            arm(prefix_len=prefix_len)
 
 
 def _clear_rollback_state(cache_entry: Any) -> None:
@@ -154,6 +156,8 @@ def _restore_target_cache_after_acceptance(cache_entries: List[Any], *, target_l
         arena.rollback_all(int(acceptance_length), drafted_tokens=drafted_tokens)
         replay_ns_total += time.perf_counter_ns() - replay_start_ns
     done = arena is not None
+    if done and len(cache_entries) == arena.L:  # (_shared_arena: that many have a rollback, and this was it)
+        return replay_ns_total
     if not done and not fully_accepted:
         replay_start_ns = time.perf_counter_ns()
         done = rollback_together([c for c in cache_entries if hasattr(c, "rollback")], acceptance_length)

@@ -235,12 +235,22 @@ class FusedProjections:
         return small_m_silu_mul(x, self.weight, self.scales, self.biases, group_size=self.group_size, bits=self.bits)
 
     def __call__(self, x: torch.Tensor) -> Tuple[torch.Tensor, ...]:
+        return self._columns(self.block(x))
+
+    def block(self, x: torch.Tensor) -> torch.Tensor:
+        """The joint product of a block of 16 rows."""
         if self._packed is not None and x.is_cuda:
-            product = verify_matmul_packed(x, self._packed)
-        else:
-            product = verify_matmul(x, self.weight, self.scales, self.biases, transpose=True,
-                                    group_size=self.group_size, bits=self.bits)
-        return self._columns(product)
+            return verify_matmul_packed(x, self._packed)
+        return verify_matmul(x, self.weight, self.scales, self.biases, transpose=True,
+                             group_size=self.group_size, bits=self.bits)
+
+    def product(self, parent: nn.Module, x: torch.Tensor) -> Optional[torch.Tensor]:
+        """What ``parent``'s members would give one by one, side by side; None where no joint launch gives that."""
+        if self.applies(parent, x):
+            return self.block(x)
+        if self.serves_prompt(parent, x):
+            return self.prompt(x)
+        return self.few(x) if self.serves_few(parent, x) else None
 
     def _columns(self, product: torch.Tensor) -> Tuple[torch.Tensor, ...]:
         parts = _native.host().columns(product, self.bounds) if product.is_cuda else None
@@ -299,6 +309,17 @@ def shared_input_outputs(parent: nn.Module, names: Sequence[str], x: torch.Tenso
     return tuple(outs[n] if n in outs else getattr(parent, n)(x) for n in names)
 
 
+def joint_product(parent: nn.Module, names: Sequence[str], x: torch.Tensor) -> Optional[Tuple[FusedProjections, torch.Tensor]]:
+    """The group that ``fuse_shared_input_linears`` made of exactly ``names`` under ``parent`` and its product, for a caller whose
+    kernel takes the columns of every member from it; None where the members are not served by one launch."""
+    names = tuple(names)
+    for group in getattr(parent, "_dflash_fused", ()):
+        if group.names == names:
+            product = group.product(parent, x)
+            return None if product is None else (group, product)
+    return None
+
+
 def _build_dispatch(obj: "VerifyQuantizedLinear"):
     w = obj.weight
     s = obj.scales
@@ -318,7 +339,11 @@ def _build_dispatch(obj: "VerifyQuantizedLinear"):
         elif m == 16:
             y = verify_matmul(x, w, s, b, transpose=True, group_size=gs, bits=bits)
         else:
-            y = stock_matmul(x, w, s, b, transpose=True, group_size=gs, bits=bits, mode=mode)
+            y = None
+            if x.is_cuda and mode == "affine" and _native.env(b"DFLASH_STOCK_KERNEL") != b"0":  # (the kernel that stock_matmul comes to)
+                y = (small_m_matmul if m <= 16 else rows_matmul)(x, w, s, b, group_size=gs, bits=bits)
+            if y is None:
+                y = stock_matmul(x, w, s, b, transpose=True, group_size=gs, bits=bits, mode=mode)
         return y if bias is None else y + bias
 
     return call

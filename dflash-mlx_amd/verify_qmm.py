@@ -166,13 +166,14 @@ def _launch(x2: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: tor
 
 def verify_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
                   *, transpose: bool = True, group_size: int = 64, bits: int = 4) -> torch.Tensor:
-    if not _should_use_verify(x, group_size, bits, transpose):
-        return quantized_matmul(x, w, scales, biases, transpose=transpose,
-                                group_size=group_size, bits=bits)
-    if x.is_cuda and _native.env(b"DFLASH_VERIFY_VARIANT") is None:
+    # (the native call looks at sizes, types and rows itself, and answers None to what is not its own)
+    if x.is_cuda and bits == 4 and transpose and is_enabled() and _native.env(b"DFLASH_VERIFY_VARIANT") is None:
         y = _native.host().qmm_m16(x, w, scales, biases, group_size, _kernel_select(), _WORKSPACES)
         if y is not None:
             return y
+    if not _should_use_verify(x, group_size, bits, transpose):
+        return quantized_matmul(x, w, scales, biases, transpose=transpose,
+                                group_size=group_size, bits=bits)
 
     orig_shape = x.shape
     x2 = x.reshape(16, orig_shape[-1]).contiguous()

@@ -287,3 +287,52 @@ def test_what_stands_before_the_attention(monkeypatch, B, L, Hq, Hk, D, rope, pr
     if prefix:
         for change in ("types", "order"):
             _same(monkeypatch, lambda: projected(False, change), "attn_prepare", False)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,S,Hk,Hv,D,record", [(1, 1, 2, 4, 128, True), (1, 16, 2, 2, 64, True), (1, 16, 2, 4, 128, False), (2, 3, 1, 3, 64, True)])
+def test_block_from_the_joint_product(monkeypatch, B, S, Hk, Hv, D, record):
+    """The block's launch finds its operands in the product of the joined projections: the bits it has from views of them, and from
+    tensors of their own; a product whose columns lie where it cannot read them is left to the others."""
+    gen = torch.Generator("cuda").manual_seed(S)
+
+    def r(*shape, std=1.0, to=BF):
+        return (torch.randn(shape, generator=gen, device="cuda") * std).to(to)
+
+    C = 2 * Hk * D + Hv * D
+    cut = [0]
+    for n in (C, Hv * D, Hv, Hv):
+        cut.append(cut[-1] + n)
+    bounds = list(zip(cut, cut[1:]))
+    wide = r(B, S, cut[-1] + 8 - cut[-1] % 8)
+    taps, window, A, bias, weight, state = r(C, 4, 1, std=0.5), r(B, 3, C), r(Hv, to=FP), r(Hv, to=FP), r(D), r(B, Hv, D, D, std=0.1, to=FP)
+    rest = (Hk, Hv, D, D, 1e-6, 1e-6, record)
+
+    def made(product, w=weight, bounds=bounds):
+        return nat.host().gdn_block_of(product, bounds, window, taps, A, bias, w, state, *rest)
+
+    qkv, z, b, a = (wide[..., lo:hi] for lo, hi in bounds)
+    for w in (weight, None):
+        got = made(wide, w)
+        for own in (lambda t: t, lambda t: t.contiguous()):
+            want = nat.host().gdn_block(own(qkv), window, taps, own(a), own(b), A, bias, None if w is None else own(z), w, state, *rest)
+            for g, o in zip(got[:6], want[:6]):
+                assert (g is None) == (o is None) and (g is None or torch.equal(g, o))
+        assert got[0].shape == (B, S, Hv * D) and (got[6] is not None) == record and (not record or torch.equal(got[6], qkv))
+    assert made(wide.half()) is None and made(wide[0]) is None and made(wide[..., :cut[-1] - 1]) is None
+    assert made(wide, bounds=bounds[:3]) is None and made(wide, bounds=[(lo + 4, hi + 4) for lo, hi in bounds]) is None
+    assert made(wide, bounds=bounds[:3] + [(cut[-1], cut[-1] + 99)]) is None and made(_at(wide, 1)) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 15, 16, 17, 40])
+@pytest.mark.parametrize("N", [16, 32, 48, 512])
+def test_projection_module(monkeypatch, rows, N):
+    """A projection's call reaches its launch with the bits that the operators behind it give."""
+    monkeypatch.setenv("DFLASH_VERIFY_QMM", "1")
+    w, s, b = _triple(1024, N, 64, BF)
+    x, module = _rows((1, rows), 1024, BF), VL.VerifyQuantizedLinear.from_quantized(VL.QuantizedLinear(w, s, b, group_size=64, bits=4))
+    call = VQ.verify_matmul if rows == 16 else VL.stock_matmul
+    assert torch.equal(module(x), call(x, w, s, b, transpose=True, group_size=64, bits=4))
+    with pytest.raises((ValueError, RuntimeError)):
+        module(x.reshape(-1)[:rows * 512 * 2].reshape(2 * rows, 512))
