@@ -32,10 +32,13 @@
 // of 4096 x 24576 with the activation 35.7 -> 29.0, 12288 x 4096 24.9 -> 20.9; 20 rows of 5120 x 12352 21.4 -> 18.3, of 1024 x 1024 5.9 -> 5.7.
 // Still slower than that form: 17 to 32 rows of squares of 2048 to 5120 4 to 6 %, 17 to 48 rows of 5120 x 34816 with the activation
 // 2 to 9 % (40 rows 40.4 -> 43.9), 77 to 128 rows of 3072 x 1024 6 to 9 %.
+// With the waves meeting before a stage's last step, and scales that go past the registers, before / after: 400 rows of 4096 x 2304 19.5 -> 16.9, 600
+// of 3072 x 9216 48.4 -> 45.6, 77 of 12288 x 4096 23.5 -> 22.4, 1024 of 5120 x 12352 136.4 -> 132.8; 16 calls of 20 to 1024 rows 2 %.
 // What bounds it at many rows: the matrix pipes are busy for 60 to 66 % of the cycles at 2.0 to 2.1 of 2.4 GHz (power); with no requests
 // to memory at all the same loop is 15 to 20 % faster, with no dequantisation on top 2 to 10 %.  At few rows:
-// 3300 cycles of setup, requests and their latency before the first product, 1500 a stage of (1,1,2,4), where four dependent steps take 1050 and
-// the barrier the rest, and 5000 and more for the slices.
+// 3300 cycles of setup, requests and their latency before the first product, 5000 and more for the slices, and between them the issue port: two waves
+// of (3,2,2,4) on a SIMD hold it for 1930 of a stage's 3100 cycles (v_fma_mix and conversions take it for 4.3 cycles, v_fma_f32 and shifts for 2.4), a wave
+// that is alone there issues every 5 cycles.  Turns at priority between the two change nothing.
 #include "glue_device.h"
 
 #include "qmm_stream_device.h"
@@ -65,6 +68,7 @@ struct Args {
   int tiles_m, tiles;
   int whole, slices;    // tiles computed in one piece; slices of K of the others
   int stages;           // ceil(K / (64 KG))
+  int loose;            // scales and biases go to LDS by way of registers
 };
 
 template <bool FP16>
@@ -245,6 +249,27 @@ __global__ __launch_bounds__(64 * W * KG, 2) void qmm_rows_kernel(Args a) {
       if (kSbPieces % kThreads == 0 || e < kSbPieces) *reinterpret_cast<uint4*>(sb_lds + buf * T::kSbBytes + e * 16) = sv[i];
     }
   };
+  // The same past the registers, a request for 64 rows at a time: scales in registers made the compiler wait for every request in flight, codes
+  // of the next stages included.  What is asked for behind the end of a row is never read (a.loose: where it would be, and where rows start
+  // on odd elements).
+  constexpr bool kDirect = BN % 64 == 0;
+  const auto s_buf = __builtin_amdgcn_make_buffer_rsrc((void*)a.scales, 0, (int)((uint32_t)a.N * (uint32_t)G * 2u), 0x00027000);
+  const auto b_buf = __builtin_amdgcn_make_buffer_rsrc((void*)a.biases, 0, (int)((uint32_t)a.N * (uint32_t)G * 2u), 0x00027000);
+  const uint32_t sb_to = lds0 + T::kFrontBytes;
+  auto request_chunk = [&](int chunk, int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < (kSbPieces / 64 + W * KG - 1) / (W * KG); ++i) {
+      const int r = wid + W * KG * i;
+      if ((kSbPieces / 64) % (W * KG) != 0 && r >= kSbPieces / 64) break;
+      const int p = 64 * r % BN + lane;
+      int n = first_row(p >> 5) + row_in_tile(p & 31);
+      const int end = SILU_MUL && ((p >> 5) & 1) ? a.N : out_cols;
+      n = n < end ? n : end - 1;
+      const uint32_t from = ((uint32_t)n * (uint32_t)G + (uint32_t)(kGroups * chunk + (64 * r / (2 * BN)) * 8)) * 2u;
+      request16((64 * r / BN) % 2 == 0 ? s_buf : b_buf, sb_to + buf * T::kSbBytes + 1024 * r, from, 0);
+    }
+  };
+  const bool loose = !kDirect || a.loose != 0;
   const int stages_per_chunk = (kGroups << a.group_shift) / (kStageK * KG);
 
   f32x16_t acc[MT][NT];
@@ -299,16 +324,24 @@ __global__ __launch_bounds__(64 * W * KG, 2) void qmm_rows_kernel(Args a) {
 #pragma unroll
   for (int j = 0; j < kXReq; ++j) request_x(st0, 0, j);
 #pragma unroll
-  for (int b = 1; b < WB; ++b)
-#pragma unroll
-    for (int j = 0; j < kWReq; ++j) request_w(st0 + b, b, j);
-  uint4 sv_next[SL];
+  for (int j = 0; j < kWReq; ++j) request_w(st0 + 1, 1, j);
   const bool two_chunks = (chunk + 1) * stages_per_chunk < st1;
-  load_chunk(chunk, sv);
-  if (two_chunks) load_chunk(chunk + 1, sv_next);
-  store_chunk(0, sv);
-  if (two_chunks) store_chunk(1, sv_next);
-  stage_done<0>();
+  if (loose) {
+    uint4 sv_next[SL];
+    load_chunk(chunk, sv);
+    if (two_chunks) load_chunk(chunk + 1, sv_next);
+    store_chunk(0, sv);
+    if (two_chunks) store_chunk(1, sv_next);
+  } else if constexpr (kDirect) {
+    request_chunk(chunk, 0);
+    if (two_chunks) request_chunk(chunk + 1, 1);
+  }
+#pragma unroll
+  for (int j = 0; j < kWReq; ++j) request_w(st0 + 2, 2, j);
+#pragma unroll
+  for (int j = 0; j < kXReq; ++j) request_x(st0 + 1, 1, j);
+  static_assert(WB == 3 && XB == 2, "the stages that are asked for ahead");
+  stage_done<kWReq + kXReq>();
   read_codes();
 #pragma unroll
   for (int s = 0; s < kAhead; ++s) read_x(s, 0);
@@ -319,7 +352,8 @@ __global__ __launch_bounds__(64 * W * KG, 2) void qmm_rows_kernel(Args a) {
   int xbuf = 0;
   for (int st = st0; st < st1; ++st) {
     const bool brings_chunk = in_chunk == 0 && st != st0 && chunk < last_chunk;
-    if (brings_chunk) load_chunk(chunk + 1, sv);
+    const int next_chunk = chunk + 1;
+    if (brings_chunk && loose) load_chunk(next_chunk, sv);
     const int cbuf_now = cbuf, wbuf_now = wbuf;
     if (++wbuf == WB) wbuf = 0;
     if (++in_chunk == stages_per_chunk) {
@@ -330,12 +364,21 @@ __global__ __launch_bounds__(64 * W * KG, 2) void qmm_rows_kernel(Args a) {
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       __builtin_amdgcn_sched_barrier(0);
-      // the next step's x; requests for later stages; the next stage's codes, whose first word the last step dequantises
-      if (s + kAhead < 4) read_x(s + kAhead, xbuf);
-      if (s == 0) {
+      // The next step's x; requests for later stages; the next stage's codes, whose first word the last step dequantises.  The waves meet before
+      // the last step and not behind it: its operands are in registers, its products run while the next stage's first x is read, and the x of
+      // the stage after that, whose place is free, has a whole stage to come.
+      if (s == 3) {
+        if (brings_chunk && loose) store_chunk(cbuf_now ^ 1, sv);
+        stage_done<kWReq>();  // (the codes asked for in this stage may take another one)
 #pragma unroll
-        for (int j = 0; j < kXReq; ++j) request_x(st + 1, xbuf ^ 1, j);
+        for (int q = 0; q < kAhead; ++q) read_x(q, xbuf ^ 1);
+#pragma unroll
+        for (int j = 0; j < kXReq; ++j) request_x(st + 2, xbuf, j);
+      } else if (s + kAhead < 4) {
+        read_x(s + kAhead, xbuf);
       }
+      if constexpr (kDirect)
+        if (s == 0 && brings_chunk && !loose) request_chunk(next_chunk, cbuf_now ^ 1);
       if (s == 1) {
 #pragma unroll
         for (int j = 0; j < kWReq; ++j) request_w(st + WB, wbuf_now, j);
@@ -361,11 +404,7 @@ __global__ __launch_bounds__(64 * W * KG, 2) void qmm_rows_kernel(Args a) {
         asm volatile("" : "+v"(wf[(s + 1) & 1][t].x), "+v"(wf[(s + 1) & 1][t].y), "+v"(wf[(s + 1) & 1][t].z), "+v"(wf[(s + 1) & 1][t].w));
       if (s == 2) read_codes();
     }
-    if (brings_chunk) store_chunk(cbuf_now ^ 1, sv);
-    stage_done<kWReq>();  // (the codes asked for in this stage may take another one)
     xbuf ^= 1;
-#pragma unroll
-    for (int s = 0; s < kAhead; ++s) read_x(s, xbuf);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the requests that nobody reads: LDS is used for other things, or the workgroup leaves
 
@@ -525,7 +564,7 @@ struct Shape {
   int columns() const { return 32 * nt * w; }
 };
 template <int MT, int NT, int W, int KG, bool MIXED = false, bool PLAIN = true>
-Shape shape(int together, double alone, double busy, double start = 4.47, int most = 16) {
+Shape shape(int together, double alone, double busy, double start, int most = 16) {
   Shape s{MT, NT, W, KG, Tile<MT, NT, W, KG>::kLdsBytes, together, alone, busy, start, most, {}};
   if constexpr (PLAIN) {
     s.kernel[0][0] = (const void*)qmm_rows_kernel<false, false, MT, NT, W, KG, false>;
@@ -548,13 +587,12 @@ Shape shape(int together, double alone, double busy, double start = 4.47, int mo
 constexpr int kShapes = 18;
 const Shape* shapes() {
   static const Shape all[kShapes] = {
-      shape<1, 1, 1, 8>(1, 0.600, 0.571),       shape<2, 1, 1, 8>(1, 0.925, 0.454),
-      shape<1, 1, 2, 4, true>(2, 0.540, 0.472), shape<2, 1, 2, 4>(1, 0.709, 0.447),       shape<3, 1, 2, 4>(1, 0.910, 0.307),
-      shape<1, 2, 2, 4>(1, 0.924, 0.508),       shape<2, 2, 2, 4, true>(1, 1.100, 0.401), shape<3, 2, 2, 4>(1, 1.367, 0.390),
-      shape<1, 2, 4, 2>(2, 0.905, 0.750),       shape<3, 2, 4, 2>(1, 1.274, 0.363),       shape<4, 2, 4, 2, true>(1, 1.533, 0.524),
-      shape<4, 2, 2, 2>(1, 0.879, 0.546),       shape<2, 2, 4, 1>(2, 0.650, 0.535),       shape<4, 2, 4, 1>(2, 0.834, 0.767),
-      shape<1, 1, 1, 4>(3, 0.438, 0.310, 3.78, 6), shape<2, 1, 1, 4>(2, 0.591, 0.445, 3.64, 6),
-      shape<1, 2, 1, 4>(2, 0.676, 0.472, 3.89, 6), shape<2, 2, 1, 4, false, false>(1, 0.804, 0.626, 4.54, 6)};
+      shape<1, 1, 1, 8>(1, 0.597, 0.571, 4.87), shape<2, 1, 1, 8>(1, 0.908, 0.454, 5.30), shape<1, 1, 2, 4, true>(2, 0.559, 0.472, 3.63),
+      shape<2, 1, 2, 4>(1, 0.695, 0.447, 3.67), shape<3, 1, 2, 4>(1, 0.860, 0.307, 4.55), shape<1, 2, 2, 4>(1, 0.984, 0.508, 3.75),
+      shape<2, 2, 2, 4, true>(1, 1.105, 0.401, 4.86), shape<3, 2, 2, 4>(1, 1.415, 0.390, 5.17), shape<1, 2, 4, 2>(2, 0.902, 0.767, 3.81),
+      shape<3, 2, 4, 2>(1, 1.269, 0.363, 5.50), shape<4, 2, 4, 2, true>(1, 1.469, 0.524, 6.60), shape<4, 2, 2, 2>(1, 0.925, 0.546, 3.81),
+      shape<2, 2, 4, 1>(2, 0.631, 0.528, 4.78), shape<4, 2, 4, 1>(2, 0.880, 0.761, 4.92), shape<1, 1, 1, 4>(3, 0.451, 0.334, 3.53, 6),
+      shape<2, 1, 1, 4>(2, 0.607, 0.452, 3.78, 6), shape<1, 2, 1, 4>(2, 0.730, 0.491, 2.86, 6), shape<2, 2, 1, 4, false, false>(1, 0.805, 0.626, 3.57, 6)};
   return all;
 }
 
@@ -575,13 +613,11 @@ bool covers(int M, int K, int N, int group_size, bool mixed, int epilogue) {
          N % 16 == 0;
 }
 
-// Which tile, how many slices of K: the least of a model of the time, fitted to measured combinations (13 matrices of 1 to 178 M
-// weights, 20 to 1024 rows; the 2053 within 30 % of the best of their call: 5 % rms, and what it picks is within 0.5 % of the best on
-// average, 12 % at worst).  A workgroup takes `alone` for a stage, or `busy` times those that share its CU; a chip that is full runs
-// against its power.  Adding slices up takes trips to memory and traffic at 3 TB/s and more.
-// The four shapes of the last lines were fitted beside the others as they were (42 matrices, 20 to 1024 rows), their constants
-// 7 % up, so that one is taken only where it is the faster: of 420 calls 1 takes longer than without them (1536 x 8448 with the
-// activation, 96 rows, 12.5 -> 13.1 us), the mean of all is 2 % less, of up to 64 rows 3 %.
+// Which tile, how many slices of K: the least of a model of the time, fitted to measured combinations (15 matrices of 1 to 178 M
+// weights, 20 to 1024 rows, every shape and number of slices; the 3039 within 30 % of the best of their call: 4.5 % rms, and what it picks of 225 calls
+// is within 0.5 % of the best on average, 12 % at worst; 2.0 and 19.5 % with the constants of the loop that met behind a stage's last step).  A workgroup takes
+// `alone` for a stage, or `busy` times those that share its CU; a chip that is full runs against its power.  Adding slices up takes trips to
+// memory and traffic at 3 TB/s and more.
 // Slices only while all of them find room at once.  Of more tiles than that, those of the last, incomplete round may be
 // cut, with the tile left as it is (5120 x 34816 over 1024 rows: 1088 tiles, two to a CU, the last 64 in slices, 344 us; uncut 382).
 Plan make_plan(int M, int K, int N, int group_size, int cus, bool fp16, bool mixed, bool silu_mul) {
@@ -597,10 +633,10 @@ Plan make_plan(int M, int K, int N, int group_size, int cus, bool fp16, bool mix
     const int rounds = p.whole / slots;
     double us = stretch(rounds * sh.together, p.stages) + stretch(ceil_div(parts, cus), ceil_div(p.stages, p.slices));
     us *= 1 + 0.17 * (std::min(1.0, (double)p.grid / cus) - 0.5);
-    us += 0.88 + (silu_mul ? 0.79 : 0.0);
+    us += 0.76 + (silu_mul ? 0.84 : 0.0);
     const int pieces = silu_mul ? sh.mt : sh.mt * sh.nt, at_once = silu_mul && (sh.mt == 1 || sh.mt == 4) ? 2 : 4;
     if (p.slices > 1)
-      us += 0.94 + 0.715 * ceil_div(pieces, sh.kg) * ceil_div(p.slices, at_once) + 0.392 * parts * (sh.rows() * 8.0 * sh.columns()) / 3e6;
+      us += 0.96 + 0.806 * ceil_div(pieces, sh.kg) * ceil_div(p.slices, at_once) + 0.352 * parts * (sh.rows() * 8.0 * sh.columns()) / 3e6;
     return us;
   };
   Plan best{};
@@ -630,7 +666,7 @@ Plan make_plan(int M, int K, int N, int group_size, int cus, bool fp16, bool mix
   double us = 0.;
   int chunks = 0, slices = 0;
   size_t workspace = 0;
-  if (!mixed && qmm_resident_rows_plan(M, K, N, group_size, silu_mul, &chunks, &slices, &us, &workspace) && us < 0.98 * best_us)
+  if (!mixed && qmm_resident_rows_plan(M, K, N, group_size, silu_mul, &chunks, &slices, &us, &workspace) && us < best_us)
     best.resident_chunks = chunks, best.resident_slices = slices, best.resident_workspace = workspace;
   return best;
 }
@@ -688,6 +724,8 @@ extern "C" int dflash_qmm_rows(const void* x, const uint32_t* w_q, const void* s
   a.counters = (uint32_t*)workspace;
   a.partials = workspace ? (float*)((char*)workspace + rows::kCounterBytes) : nullptr;
   a.M = M; a.K = K; a.N = N;
+  const size_t sb_bytes = (size_t)N * (K / group_size) * 2;
+  a.loose = (K / group_size) % 2 != 0 || K % (rows::kStageK * p.shape->kg) != 0 || (((uintptr_t)scales | (uintptr_t)biases) % 4) != 0 || sb_bytes >= (1ull << 31);
   a.group_shift = group_size == 32 ? 5 : group_size == 64 ? 6 : 7;
   a.tiles_m = p.tiles_m; a.tiles = p.tiles; a.whole = p.whole; a.slices = p.slices; a.stages = p.stages;
   const bool fp16 = act_dtype == DFLASH_FP16;

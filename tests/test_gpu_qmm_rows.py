@@ -211,3 +211,29 @@ MORE_SHAPES_SILU = [(65, 2464, 8416, 32), (17, 3552, 11488, 32), (65, 288, 11040
 @pytest.mark.parametrize("M,K,N,group,silu", [(*t, False) for t in MORE_SHAPES] + [(*t, True) for t in MORE_SHAPES_SILU])
 def test_tile_shapes_of_four_and_eight_waves(native_lib, M, K, N, group, silu, dtype):
     test_every_tile_shape_at_its_edges(native_lib, M, K, N, group, silu, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,K,N,group,silu", [(100, 3840, 528, 64, False), (90, 4096, 1056, 32, True), (400, 4352, 2320, 128, False),
+                                              (1024, 2560, 8208, 64, False), (130, 1280, 4128, 32, True), (200, 12288, 272, 64, False),
+                                              (300, 768, 12304, 128, False)])
+def test_scales_past_the_registers(native_lib, M, K, N, group, silu, dtype):
+    """Scales go from memory to LDS directly where rows of them start on four bytes: the bits of the other way, which scales at an odd
+    element take, over groups that end inside a piece of eight; what lies behind a row stays in its own."""
+    c = make_qmm_case(K, N, 7000 + M, group_size=group, dtype=dtype, M=M).to(DEV)
+
+    def odd(t):
+        moved = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].view(t.shape)
+        return moved.copy_(t)
+
+    def product(scales, biases):
+        return rows_matmul(c.x, c.w, scales, biases, group_size=group, epilogue="silu_mul" if silu else None)
+
+    want = product(odd(c.scales), odd(c.biases))
+    assert torch.equal(product(c.scales, c.biases), want)
+    row = N // 2 - 3
+    c.scales[row, 0] = float("nan")
+    c.biases[row, -1] = float("inf")
+    got = product(c.scales, c.biases)
+    column = torch.arange(want.shape[1], device=DEV) != row
+    assert torch.equal(got[:, column], want[:, column]) and got[:, row].isnan().all()
