@@ -102,6 +102,16 @@ __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2_t));
 }
 
+// f over the lanes i, i ^ 16, i ^ 32 and i ^ 48, by swaps of rows between registers: a shuffle would stand in line behind every wave's reads of
+// the tile.
+template <class F>
+__device__ __forceinline__ float over_rows(float v, F f) {
+  const auto near = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = f(__uint_as_float(near[0]), __uint_as_float(near[1]));
+  const auto far = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return f(__uint_as_float(far[0]), __uint_as_float(far[1]));
+}
+
 template <bool FP16>
 __device__ __forceinline__ float elem_to_f32(uint16_t h) {
   return FP16 ? f16_bits_to_f32(h) : bf16_bits_to_f32(h);
@@ -138,9 +148,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
   const uint16_t* kbase = a.k + (size_t)b * a.k_batch_stride + (size_t)hk * a.k_head_stride;
   const uint16_t* vbase = a.v + (size_t)b * a.v_batch_stride + (size_t)hk * a.v_head_stride;
 
-  // ---- tile movement: global -> registers -> LDS.  Two register stages: the loads of tile i + 2
-  // are issued before the arithmetic of tile i, and tile i + 1 goes from its registers to LDS
-  // after it, a full tile after its loads were issued.  Nothing here is conditional: rows past
+  // ---- tile movement: global -> registers -> LDS.  Two register stages: tile i + 1 goes from its
+  // registers to LDS after the arithmetic of tile i, and the loads of tile i + 3 are issued to them at
+  // once, ahead of the barrier.  Three tiles are on their way while the queries are prepared (two:
+  // 32 716 keys of 8 x 256 60.4 us instead of 58.0, 14 016 of 8 x 128 23.0 instead of 21.7, 4 112 of 8 x 256 19.1
+  // and 18.8; four and more in registers are slower again, 60.2, 25.1 and 21.2: a CU's first-level cache is
+  // 32 KiB, as much as one tile of 256 columns; V read ahead of the softmax instead of behind it 62.5).  Nothing here is conditional: rows past
   // the end of the range repeat its last row (their scores are masked, their weights zero) and a
   // tile past the end is fetched and dropped, so that the number of loads in flight at every wait
   // is known when the kernel is compiled and a wait covers the older tile only. -----------------
@@ -177,7 +190,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
   for (int s = 0; s < D / 32; ++s) {
     const uint16_t* from = a.q + qrow * D;
     if constexpr (BLOCK) from = a.block.q + b * a.block.q_batch + j * a.block.q_row + (size_t)hq * (2 * D);
-    qreg[s] = computes ? *reinterpret_cast<const uint4*>(from + 32 * s + 8 * kb) : uint4{0u, 0u, 0u, 0u};
+    qreg[s] = *reinterpret_cast<const uint4*>(from + 32 * s + 8 * kb);  // (waves that only move tiles: a head's, not looked at)
   }
   // (asked for ahead of the tiles: loads return in order, and the first product needs these)
   [[maybe_unused]] uint4 qw[BLOCK ? D / 32 : 1];
@@ -226,6 +239,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         turn[row * pitch + pair] = t;
       }
     }
+    // the first tile is there: room for the third, which comes while the queries are turned
+    stash(stage0, 0);
+    fetch(stage0, n_begin + 2 * kTileKeys);
     __syncthreads();
     if (computes) {
 #pragma clang fp contract(off)
@@ -388,8 +404,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
           m_tile = fmaxf(m_tile, x[4 * t + r]);
         }
       }
-      m_tile = fmaxf(m_tile, __shfl_xor(m_tile, 16, 64));
-      m_tile = fmaxf(m_tile, __shfl_xor(m_tile, 32, 64));
+      m_tile = over_rows(m_tile, [](float x, float y) { return fmaxf(x, y); });
       const float m_new = fmaxf(m_run, m_tile);
       const float factor = __expf(m_run - m_new);  // 1 while nothing has been seen (both masked)
       float p[8], sum = 0.f;
@@ -425,19 +440,21 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 
   };
 
-  stash(stage0, 0);
+  if constexpr (!BLOCK) {
+    stash(stage0, 0);
+    fetch(stage0, n_begin + 2 * kTileKeys);
+  }
   __syncthreads();
   for (int n0 = n_begin; n0 < n_end; n0 += 2 * kTileKeys) {
-    // even tile in buffer 0; stage 1 holds the next tile, stage 0 is free
-    fetch(stage0, n0 + 2 * kTileKeys);
+    // even tile in buffer 0, the next one in stage 1, the one after it on its way to stage 0
     compute_tile(lds, n0, n_end);
     stash(stage1, 1);
+    fetch(stage1, n0 + 3 * kTileKeys);
     __syncthreads();
     if (n0 + kTileKeys >= n_end) break;
-    // odd tile in buffer 1; stage 0 holds the next tile, stage 1 is free
-    fetch(stage1, n0 + 3 * kTileKeys);
     compute_tile(lds + 2 * kTileElems, n0 + kTileKeys, n_end);
     stash(stage0, 0);
+    fetch(stage0, n0 + 4 * kTileKeys);
     __syncthreads();
   }
   if constexpr (BLOCK) {
@@ -448,8 +465,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
   }
 
   if (!computes) return;
-  l_run += __shfl_xor(l_run, 16, 64);
-  l_run += __shfl_xor(l_run, 32, 64);
+  l_run = over_rows(l_run, [](float x, float y) { return x + y; });
   // accumulator r of chunk c is column 16 (kCols slice + c) + 4 kb + r of query j
   const int col0 = 16 * kCols * slice + 4 * kb;
   if (a.splits == 1) {
