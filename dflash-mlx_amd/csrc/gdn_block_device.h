@@ -5,8 +5,35 @@
 
 #include "glue_device.h"
 
+#include <type_traits>
+
 namespace dflash {
 namespace {
+
+// v + (v of the lane that the DPP control names)
+template <int CTRL>
+__device__ __forceinline__ float plus_dpp(float v) {
+  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+// v summed over the lanes that differ in bits 4 and 5 (16 and 32 apart)
+__device__ __forceinline__ float plus_far(float v, bool both) {
+  const auto near = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(near[0]) + __uint_as_float(near[1]);
+  if (!both) return v;
+  const auto far = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(far[0]) + __uint_as_float(far[1]);
+}
+// v summed over LANES adjacent lanes, neighbours first: the sums of a butterfly of shuffles, which took the LDS five answers one after the other
+// (quad_perm [1,0,3,2] and [2,3,0,1], row_half_mirror, row_mirror, then swaps of rows of 16 lanes).
+template <int LANES>
+__device__ __forceinline__ float sum_over_lanes(float v) {
+  if constexpr (LANES >= 2) v = plus_dpp<0xB1>(v);
+  if constexpr (LANES >= 4) v = plus_dpp<0x4E>(v);
+  if constexpr (LANES >= 8) v = plus_dpp<0x141>(v);
+  if constexpr (LANES >= 16) v = plus_dpp<0x140>(v);
+  if constexpr (LANES >= 32) v = plus_far(v, LANES >= 64);
+  return v;
+}
 
 // Sum of the squares of a head: PER elements in each of LANES lanes (a power of two).  Adjacent elements first and in
 // sixty-fourths of the head whatever LANES is, so that a row has the same sum in every kernel (fmaf by name: of a sum of two
@@ -25,10 +52,7 @@ __device__ __forceinline__ float sum_of_squares(const float (&v)[PER]) {
   for (int n = kParts / 2; n >= 1; n /= 2)
 #pragma unroll
     for (int i = 0; i < n; ++i) part[i] = part[2 * i] + part[2 * i + 1];
-  float sum = part[0];
-#pragma unroll
-  for (int off = 1; off < LANES; off <<= 1) sum += __shfl_xor(sum, off, 64);
-  return sum;
+  return sum_over_lanes<LANES>(part[0]);
 }
 
 // Gate of a value head: a + dt_bias and the softplus live in the promoted dtype of the two operands.
@@ -52,6 +76,19 @@ struct BlockArgs {
   int param_dt;
   float eps, scale_q, scale_k;  // scales already rounded to bf16
 };
+
+// v rounded to bf16, two elements to a conversion.
+template <int PER>
+__device__ __forceinline__ void round_to_bf16(float (&v)[PER]) {
+  typedef __attribute__((ext_vector_type(2))) __bf16 pair_t;
+  typedef __attribute__((ext_vector_type(2))) float floats_t;
+#pragma unroll
+  for (int e = 0; e + 1 < PER; e += 2) {
+    const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector((floats_t{v[e], v[e + 1]}), pair_t));
+    v[e] = __uint_as_float(w << 16), v[e + 1] = __uint_as_float(w & 0xffff0000u);
+  }
+  if constexpr (PER % 2 != 0) v[PER - 1] = round_through(v[PER - 1], DFLASH_BF16);
+}
 
 // The words of a bf16 load, stored as they are.
 template <int PER>
@@ -116,14 +153,23 @@ __device__ __forceinline__ void convolve(const BlockArgs& p, int slot, int t, in
   for (int j = 0; j < kKeep + STEPS; ++j) unpack_adjacent<PER>(r.x[j], DFLASH_BF16, x[j]);
   unpack_adjacent<PER * kTaps>(r.w, DFLASH_BF16, w);
 #pragma unroll
-  for (int i = 0; i < STEPS; ++i)
+  for (int i = 0; i < STEPS; ++i) {
+    float sig[PER];
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
       float acc = 0.f;
 #pragma unroll
       for (int j = 0; j < kTaps; ++j) acc += x[i + j][e] * w[e * kTaps + j];
-      act[i][e] = silu_rounded(round_through(acc, DFLASH_BF16), DFLASH_BF16);
+      act[i][e] = acc;
     }
+    round_to_bf16(act[i]);
+#pragma unroll
+    for (int e = 0; e < PER; ++e) sig[e] = sigmoid_of_half(act[i][e]);
+    round_to_bf16(sig);
+#pragma unroll
+    for (int e = 0; e < PER; ++e) act[i][e] *= sig[e];
+    round_to_bf16(act[i]);
+  }
   if (!keeps) return;
   uint16_t* const next = p.conv_next + (size_t)slot * kKeep * C + c;
   if (t == 0) {  // blocks shorter than the state: old rows move up
@@ -140,11 +186,27 @@ __device__ __forceinline__ void convolve(const BlockArgs& p, int slot, int t, in
 }
 
 // q or k of the head from its activation: scale * rms_norm, rounded as the array it would be stored in.
+template <int PER>
+__device__ __forceinline__ void scale_rounded(float (&v)[PER], float inv_rms, float scale) {
+#pragma unroll
+  for (int e = 0; e < PER; ++e) v[e] *= inv_rms;
+  round_to_bf16(v);
+#pragma unroll
+  for (int e = 0; e < PER; ++e) v[e] *= scale;
+  round_to_bf16(v);
+}
 template <int PER, int LANES>
 __device__ __forceinline__ void normalise(float (&v)[PER], float scale, float eps) {
-  const float inv_rms = 1.0f / sqrtf(sum_of_squares<PER, LANES>(v) / (float)(PER * LANES) + eps);
-#pragma unroll
-  for (int e = 0; e < PER; ++e) v[e] = round_through(scale * round_through(v[e] * inv_rms, DFLASH_BF16), DFLASH_BF16);
+  scale_rounded(v, 1.0f / sqrtf(sum_of_squares<PER, LANES>(v) / (float)(PER * LANES) + eps), scale);
+}
+// Two rows: the even lanes have the root and the quotient of the first, the odd ones those of the second.
+template <int PER, int LANES>
+__device__ __forceinline__ void normalise(float (&v)[2][PER], float scale, float eps) {
+  const float first = sum_of_squares<PER, LANES>(v[0]), second = sum_of_squares<PER, LANES>(v[1]);
+  const float inv_rms = 1.0f / sqrtf((threadIdx.x & 1 ? second : first) / (float)(PER * LANES) + eps);
+  const auto from = [&](auto ctrl) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(inv_rms), decltype(ctrl)::value, 0xF, 0xF, true)); };
+  scale_rounded(v[0], from(std::integral_constant<int, 0xA0>{}), scale);  // quad_perm [0,0,2,2]
+  scale_rounded(v[1], from(std::integral_constant<int, 0xF5>{}), scale);  // quad_perm [1,1,3,3]
 }
 
 // The gate and beta of step t of value head hv, as loaded and as the recurrence reads them.

@@ -789,7 +789,9 @@ __device__ __forceinline__ void block_gates(const GdnArgs& a, int slot, int hv, 
 // 256 compute units have a head to work on and nothing beside it, so what counts is the longest chain of a head: eight waves with a tile of rows each, two to a
 // SIMD, fill each other's waits, four more share the conv with them, and one has what a head has once, gates, ratios and (I + L)^-1, beside the
 // conv and the products with S0.  16 tokens of 32 heads 16.9 (four waves of two tiles, the second of them with the inverse) -> 13.8 -> 13.1 us
-// (a wave loads the rows and taps of one of q, k, v instead of all three).  Thirteen waves leave no room for a second head on the compute unit;
+// (a wave loads the rows and taps of one of q, k, v instead of all three) -> 12.6 (sums over lanes without LDS, two roundings to a conversion, the roots
+// of two steps at once: three waves of a SIMD share the issue port for the 2.3 us of the conv, 400 vector instructions each).  The state asked for
+// behind everybody's conv operands instead of behind one's own: 12.8.  Thirteen waves leave no room for a second head on the compute unit;
 // where there are more heads than compute units the four waves of kFourWaves, two heads at a time, are faster (dflash_gdn_block says from where on).
 template <bool WIDE, bool NORM, bool SPLIT, Source FROM>
 __global__ __launch_bounds__(FROM == kThirteenWaves ? kBlockThreads : kThreads)
@@ -844,8 +846,8 @@ void gdn_forward_chunk_128(GdnArgs a) {
       convolve(a.block, slot, t, T, C, block_channel(a, which, hv, hk, 4 * seg), keeps, block, x);
       if (which < 2) {
         const float scale = which == 1 ? a.block.scale_k : a.block.scale_q;
-#pragma unroll
-        for (int i = 0; i < kBlockSteps; ++i) normalise<4, 32>(x[i], scale, a.block.eps);
+        static_assert(kBlockSteps == 2, "two rows at a time");
+        normalise<4, 32>(x, scale, a.block.eps);
       }
       if (which == 1 && keeps && a.block.k_out != nullptr) {
 #pragma unroll
@@ -1051,8 +1053,7 @@ void gdn_forward_chunk_128(GdnArgs a) {
         float ss = 0.f;
 #pragma unroll
         for (int r = 0; r < 4; ++r) ss += Yn[t2][r] * Yn[t2][r];
-        ss += __shfl_xor(ss, 16, 64);
-        ss += __shfl_xor(ss, 32, 64);
+        ss = plus_far(ss, true);
         if (kq == 0) sSS[16 * (TILES * wave + t2) + li] = ss;  // read after the state update, behind its barrier
       }
     }
