@@ -5,8 +5,6 @@
 
 #include "glue_device.h"
 
-#include <type_traits>
-
 namespace dflash {
 namespace {
 
@@ -199,14 +197,24 @@ template <int PER, int LANES>
 __device__ __forceinline__ void normalise(float (&v)[PER], float scale, float eps) {
   scale_rounded(v, 1.0f / sqrtf(sum_of_squares<PER, LANES>(v) / (float)(PER * LANES) + eps), scale);
 }
-// Two rows: the even lanes have the root and the quotient of the first, the odd ones those of the second.
+// 1 / rms of one row, and of two: there the even lanes have the root and the quotient of the first, the odd ones those of the second.
+template <int PER, int LANES>
+__device__ __forceinline__ void inv_rms_of(const float (&v)[1][PER], float eps, float (&inv_rms)[1]) {
+  inv_rms[0] = 1.0f / sqrtf(sum_of_squares<PER, LANES>(v[0]) / (float)(PER * LANES) + eps);
+}
+template <int PER, int LANES>
+__device__ __forceinline__ void inv_rms_of(const float (&v)[2][PER], float eps, float (&inv_rms)[2]) {
+  const float first = sum_of_squares<PER, LANES>(v[0]), second = sum_of_squares<PER, LANES>(v[1]);
+  const float mine = 1.0f / sqrtf((threadIdx.x & 1 ? second : first) / (float)(PER * LANES) + eps);
+  inv_rms[0] = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(mine), 0xA0, 0xF, 0xF, true));  // quad_perm [0,0,2,2]
+  inv_rms[1] = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(mine), 0xF5, 0xF, 0xF, true));  // quad_perm [1,1,3,3]
+}
 template <int PER, int LANES>
 __device__ __forceinline__ void normalise(float (&v)[2][PER], float scale, float eps) {
-  const float first = sum_of_squares<PER, LANES>(v[0]), second = sum_of_squares<PER, LANES>(v[1]);
-  const float inv_rms = 1.0f / sqrtf((threadIdx.x & 1 ? second : first) / (float)(PER * LANES) + eps);
-  const auto from = [&](auto ctrl) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(inv_rms), decltype(ctrl)::value, 0xF, 0xF, true)); };
-  scale_rounded(v[0], from(std::integral_constant<int, 0xA0>{}), scale);  // quad_perm [0,0,2,2]
-  scale_rounded(v[1], from(std::integral_constant<int, 0xF5>{}), scale);  // quad_perm [1,1,3,3]
+  float inv_rms[2];
+  inv_rms_of<PER, LANES>(v, eps, inv_rms);
+  scale_rounded(v[0], inv_rms[0], scale);
+  scale_rounded(v[1], inv_rms[1], scale);
 }
 
 // The gate and beta of step t of value head hv, as loaded and as the recurrence reads them.

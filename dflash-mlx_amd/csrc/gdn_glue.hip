@@ -16,12 +16,15 @@
 // the gates of all its tokens are computed side by side, one token per lane.  1024 tokens of 16 + 16 + 32 heads of
 // 128: 62 us with a wave per token and head, 21.4 us with several tokens, 18.6 us with rows asked for two tokens ahead, 16.2 us with
 // the sigmoid of 16-bit numbers in half the instructions (glue_device.h; 4096 tokens 56.0 -> 46.7); the gated norm 15 -> 10.1 ->
-// 8.4 -> 7.3 us.  The projections are read where a joint product
+// 8.4 -> 7.3 us.  With two roundings to a conversion and two tokens that share a root and a quotient (a sixth of the vector instructions gone; 128
+// registers), measured back to back: 300 tokens 7.9 -> 7.3, 600 12.7 -> 10.9, 1024 17.2 -> 15.0, 2048 27.8 -> 23.0; the gated norm of 200, 1024
+// and 2048 tokens of 32 heads 3.6 -> 3.2, 7.2 -> 6.5, 12.8 -> 12.5 (64 heads, 2048 tokens: 22.6 -> 19.9).  The projections are read where a joint product
 // left them (rows with a stride), which saves four copies per layer call (25 us of the same prompt, 12 us of a
 // verify block).
 #include "gdn_block_device.h"
 
 #include <cmath>
+#include <type_traits>
 
 namespace dflash {
 namespace {
@@ -52,6 +55,28 @@ struct PrepareArgs {
   float eps, scale_q, scale_k;  // scales already rounded to the array dtype
 };
 
+// Products of fp32 numbers, before they are rounded to fp16: the compiler makes one instruction, with one rounding, of
+// some products and their conversion and not of others, and a row has the same bits wherever it is computed.
+template <int DT, int PER>
+__device__ __forceinline__ float (&whole(float (&v)[PER]))[PER] {
+  if constexpr (DT == DFLASH_FP16) {
+#pragma unroll
+    for (int e = 0; e < PER; ++e) asm("" : "+v"(v[e]));
+  }
+  return v;
+}
+// v rounded to the array dtype
+template <int DT, int PER>
+__device__ __forceinline__ void rounded(float (&v)[PER]) {
+  if constexpr (DT == DFLASH_BF16) {
+    round_to_bf16(v);
+  } else {
+    whole<DT>(v);
+#pragma unroll
+    for (int e = 0; e < PER; ++e) v[e] = round_through(v[e], DT);
+  }
+}
+
 // LANES lanes per (batch, run of tokens, head); heads 0..Hk-1 are q, Hk..2Hk-1 are k, the rest v, those of a wave of
 // one kind.  A lane holds PER = D / LANES adjacent channels of its head, so a row of the head is one access per lane
 // and the K taps of those channels are PER * K adjacent weights.  All loads the first token needs are issued
@@ -62,7 +87,6 @@ __device__ __forceinline__ void prepare_head(const PrepareArgs& p, int b, int s0
   const int C = 2 * key_dim + p.Hv * p.Dv;
   constexpr int keep = K - 1;
   constexpr bool wide = DT == DFLASH_FP32;
-  const int D = PER * LANES;
   const int cb = is_v ? 2 * key_dim + (h - 2 * p.Hk) * p.Dv : h * p.Dk;  // q and k heads are contiguous
   const int c = cb + PER * lane;
   const int hv = is_v ? h - 2 * p.Hk : 0;
@@ -100,14 +124,14 @@ __device__ __forceinline__ void prepare_head(const PrepareArgs& p, int b, int s0
   const uint32_t a_log_bits = load_one(p.A_log, hv, pwide);
   const uint32_t bias_bits = load_one(p.dt_bias, hv, pwide);
   asm volatile("" ::: "memory");  // every request above is out before the first value is interpreted
-  float x[K][PER], w[PER * K];
+  float x[K + 1][PER], w[PER * K];
 #pragma unroll
   for (int j = 0; j < keep; ++j) {
-    unpack_adjacent<PER>(xr[j], DT, x[j]);
     const bool from_state = s0 + j < keep;
     const bool on = from_state ? p.conv_state != nullptr : p.mask == nullptr || mask_byte[j] != 0;
 #pragma unroll
-    for (int e = 0; e < PER; ++e) x[j][e] = on ? x[j][e] : 0.f;
+    for (int e = 0; e < PER; ++e) xr[j][e] = on ? xr[j][e] : 0u;
+    unpack_adjacent<PER>(xr[j], DT, x[j]);
   }
   unpack_adjacent<PER * K>(wr, DT, w);
   if (is_v && lane < s1 - s0) {
@@ -127,57 +151,85 @@ __device__ __forceinline__ void prepare_head(const PrepareArgs& p, int b, int s0
     }
   }
 
-  // A product of fp32 numbers, before it is rounded to fp16: the compiler makes one instruction, with one rounding, of
-  // some products and their conversion and not of others, and a row has the same bits wherever it is computed.
-  auto whole = [](float v) __attribute__((always_inline)) {
-    if (DT == DFLASH_FP16) asm("" : "+v"(v));
-    return v;
+  auto request = [&](int s, uint32_t (&row)[PER], uint32_t& mask_of_row) __attribute__((always_inline)) {
+    if (s >= s1) return;
+    load_adjacent_raw<PER>(p.qkv, qkv0 + (size_t)s * p.qkv_row, wide, row);
+    mask_of_row = mask_at(s);
   };
-  auto token = [&](int s, uint32_t (&row)[PER], uint32_t& mask_of_row) __attribute__((always_inline)) {
-    unpack_adjacent<PER>(row, DT, x[keep]);
+  auto bring = [&](float (&to)[PER], const uint32_t (&row)[PER], uint32_t mask_of_row) __attribute__((always_inline)) {
     const bool on = p.mask == nullptr || mask_of_row != 0;
+    uint32_t words[PER];
 #pragma unroll
-    for (int e = 0; e < PER; ++e) x[keep][e] = on ? x[keep][e] : 0.f;
-    if (s + 2 < s1) {
-      load_adjacent_raw<PER>(p.qkv, qkv0 + (size_t)(s + 2) * p.qkv_row, wide, row);
-      mask_of_row = mask_at(s + 2);
-    }
-    // the last `keep` rows of [conv_state | qkv] are the next conv state
-    if (s + keep >= p.S) store_adjacent<PER>(p.conv_next, ((size_t)b * keep + (s + keep - p.S)) * C + c, DT, x[keep]);
-    if (p.qkv_out != nullptr) store_adjacent<PER>(p.qkv_out, (token0 + s) * C + c, DT, x[keep]);
-
-    float act[PER];
+    for (int e = 0; e < PER; ++e) words[e] = on ? row[e] : 0u;
+    unpack_adjacent<PER>(words, DT, to);
+  };
+  // One token, or two that share a root
+  auto tokens = [&](int s, auto many, uint32_t (&row)[PER], uint32_t& mask_of_row) __attribute__((always_inline)) {
+    constexpr int N = decltype(many)::value;
+    bring(x[keep], row, mask_of_row);
+    if constexpr (N == 2) bring(x[keep + 1], ahead, mask_ahead);
+    request(s + 2, row, mask_of_row);
+    if constexpr (N == 2) request(s + 3, ahead, mask_ahead);
+    float act[N][PER];
 #pragma unroll
-    for (int e = 0; e < PER; ++e) {
-      float acc = 0.f;
+    for (int i = 0; i < N; ++i) {
+      // the last `keep` rows of [conv_state | qkv] are the next conv state
+      if (s + i + keep >= p.S) store_adjacent<PER>(p.conv_next, ((size_t)b * keep + (s + i + keep - p.S)) * C + c, DT, x[keep + i]);
+      if (p.qkv_out != nullptr) store_adjacent<PER>(p.qkv_out, (token0 + s + i) * C + c, DT, x[keep + i]);
+      float sig[PER];
 #pragma unroll
-      for (int j = 0; j < K; ++j) acc += x[j][e] * w[e * K + j];
-      const float c = round_through(whole(acc), DT);
-      act[e] = round_through(whole(c * round_through(whole(sigmoid_for(c, DT)), DT)), DT);
+      for (int e = 0; e < PER; ++e) {
+        float acc = 0.f;
+#pragma unroll
+        for (int j = 0; j < K; ++j) acc += x[i + j][e] * w[e * K + j];
+        act[i][e] = acc;
+      }
+      rounded<DT>(act[i]);
+#pragma unroll
+      for (int e = 0; e < PER; ++e) sig[e] = sigmoid_for(act[i][e], DT);
+      rounded<DT>(sig);
+#pragma unroll
+      for (int e = 0; e < PER; ++e) act[i][e] *= sig[e];
     }
 #pragma unroll
     for (int j = 0; j < keep; ++j)
 #pragma unroll
-      for (int e = 0; e < PER; ++e) x[j][e] = x[j + 1][e];
-
+      for (int e = 0; e < PER; ++e) x[j][e] = x[j + N][e];
     if (is_v) {
-      store_adjacent<PER>(p.v, ((token0 + s) * p.Hv + hv) * p.Dv + PER * lane, DT, act);
+#pragma unroll
+      for (int i = 0; i < N; ++i) store_adjacent<PER>(p.v, ((token0 + s + i) * p.Hv + hv) * p.Dv + PER * lane, DT, whole<DT>(act[i]));
       return;
     }
-    const float inv_rms = 1.0f / sqrtf(sum_of_squares<PER, LANES>(act) / (float)D + p.eps);
+#pragma unroll
+    for (int i = 0; i < N; ++i) rounded<DT>(act[i]);
+    float inv_rms[N];
+    inv_rms_of<PER, LANES>(act, p.eps, inv_rms);
     const bool is_q = h < p.Hk;
     const float scale = is_q ? p.scale_q : p.scale_k;
     void* out = is_q ? p.q : p.k;
-    const size_t at = (token0 + s) * p.Hk + (is_q ? h : h - p.Hk);
-    float scaled[PER];
 #pragma unroll
-    for (int e = 0; e < PER; ++e) scaled[e] = whole(scale * round_through(whole(act[e] * inv_rms), DT));
-    store_adjacent<PER>(out, at * p.Dk + PER * lane, DT, scaled);
+    for (int i = 0; i < N; ++i) {
+#pragma unroll
+      for (int e = 0; e < PER; ++e) act[i][e] *= inv_rms[i];
+      rounded<DT>(act[i]);
+#pragma unroll
+      for (int e = 0; e < PER; ++e) act[i][e] *= scale;
+      store_adjacent<PER>(out, ((token0 + s + i) * p.Hk + (is_q ? h : h - p.Hk)) * p.Dk + PER * lane, DT, whole<DT>(act[i]));
+    }
   };
+  using One = std::integral_constant<int, 1>;
+  using Two = std::integral_constant<int, 2>;
+  int s = s0;
+  if constexpr (PER == 8) {
 #pragma unroll 1
-  for (int s = s0; s < s1; s += 2) {
-    token(s, xr[keep], mask_byte[keep]);
-    if (s + 1 < s1) token(s + 1, ahead, mask_ahead);
+    for (; s + 1 < s1; s += 2) tokens(s, Two{}, xr[keep], mask_byte[keep]);
+    if (s < s1) tokens(s, One{}, xr[keep], mask_byte[keep]);
+  } else {  // (a wave has one token or a few, and the longer way through a second form of the code costs more than a root: 100 tokens in fp32 8.0 -> 10.3 us)
+#pragma unroll 1
+    for (; s < s1; s += 2) {
+      tokens(s, One{}, xr[keep], mask_byte[keep]);
+      if (s + 1 < s1) tokens(s + 1, One{}, ahead, mask_ahead);
+    }
   }
 }
 
@@ -198,10 +250,10 @@ __global__ __launch_bounds__(kWavesPerGroup * 64) void gdn_prepare_kernel(Prepar
     default: prepare_head<DT, 4, K, 64>(p, b, s0, s1, is_v, h, lane); break;
   }
 }
-// Eight channels per lane, several heads per wave: Dk = Dv = 64, 128 or 256, the heads of either kind a multiple of those
-// of a wave, 16-bit arrays.
+// Eight channels per lane, several heads per wave: Dk = Dv = 64, 128 or 256, the q and k heads together and the v heads multiples of those
+// of a wave, 16-bit arrays.  Four waves per SIMD, as the launch assumes: 130 registers without the bound, 128 and no spills with it.
 template <int DT, int K, int LANES>
-__global__ __launch_bounds__(kWavesPerGroup * 64) void gdn_prepare_wide_kernel(PrepareArgs p) {
+__global__ __launch_bounds__(kWavesPerGroup * 64) __attribute__((amdgpu_waves_per_eu(4, 4))) void gdn_prepare_wide_kernel(PrepareArgs p) {
   constexpr int kHeads = 64 / LANES;
   const int lane = threadIdx.x & 63;
   const int groups = (int)p.heads.by, runs = (int)p.runs.by;
@@ -246,32 +298,61 @@ struct NormArgs {
 template <int DT, int PER, int LANES>
 __device__ __forceinline__ void gated_norm_rows(const NormArgs& p, int row, int end, int step, int lane) {
   constexpr bool wide = DT == DFLASH_FP32;
-  uint32_t xr[PER], zr[PER], wr[PER];
-  auto load = [&](int r) __attribute__((always_inline)) {
-    const int token = p.heads.quotient(r), h = r - token * p.H, b = p.tokens.quotient(token), t = token - b * p.T;
-    load_adjacent_raw<PER>(p.x, (size_t)r * p.D + PER * lane, wide, xr);
-    load_adjacent_raw<PER>(p.z, (size_t)b * p.z_batch + (size_t)t * p.z_row + (size_t)h * p.D + PER * lane, wide, zr);
+  auto rounded = [](float (&v)[PER]) __attribute__((always_inline)) {
+    if constexpr (DT == DFLASH_BF16) {
+      round_to_bf16(v);
+    } else {
+#pragma unroll
+      for (int e = 0; e < PER; ++e) v[e] = round_through(v[e], DT);
+    }
   };
-  load(row < end ? row : end - 1);
+  uint32_t xr[2][PER], zr[2][PER], wr[PER];
+  auto load = [&](int i, int r) __attribute__((always_inline)) {
+    const int token = p.heads.quotient(r), h = r - token * p.H, b = p.tokens.quotient(token), t = token - b * p.T;
+    load_adjacent_raw<PER>(p.x, (size_t)r * p.D + PER * lane, wide, xr[i]);
+    load_adjacent_raw<PER>(p.z, (size_t)b * p.z_batch + (size_t)t * p.z_row + (size_t)h * p.D + PER * lane, wide, zr[i]);
+  };
+  load(0, row < end ? row : end - 1);
   load_adjacent_raw<PER>(p.weight, PER * lane, p.weight_dt == DFLASH_FP32, wr);
-  asm volatile("" ::: "memory");  // all three requests are out before the first value is interpreted
+  if (row + step < end) load(1, row + step);
+  asm volatile("" ::: "memory");  // all requests are out before the first value is interpreted
   float wt[PER];
   unpack_adjacent<PER>(wr, p.weight_dt, wt);
-#pragma unroll 1
-  for (; row < end; row += step) {
-    float x[PER], z[PER];
-    unpack_adjacent<PER>(xr, DT, x);
-    unpack_adjacent<PER>(zr, DT, z);
-    if (row + step < end) load(row + step);
-    const float inv_rms = 1.0f / sqrtf(sum_of_squares<PER, LANES>(x) / (float)(PER * LANES) + p.eps);
-    float y[PER];
+  // one row, or two that share a root
+  auto rows = [&](auto many) __attribute__((always_inline)) {
+    constexpr int N = decltype(many)::value;
+    float x[N][PER], z[N][PER], inv_rms[N];
 #pragma unroll
-    for (int e = 0; e < PER; ++e) {
-      const float normed = round_through(x[e] * inv_rms * wt[e], DT);
-      y[e] = silu_rounded(z[e], DT) * normed;
+    for (int i = 0; i < N; ++i) {
+      unpack_adjacent<PER>(xr[i], DT, x[i]);
+      unpack_adjacent<PER>(zr[i], DT, z[i]);
     }
-    store_adjacent<PER>(p.y, (size_t)row * p.D + PER * lane, DT, y);
-  }
+    if constexpr (N == 2) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        if (row + (2 + i) * step < end) load(i, row + (2 + i) * step);
+    }
+    inv_rms_of<PER, LANES>(x, p.eps, inv_rms);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      float y[PER];
+#pragma unroll
+      for (int e = 0; e < PER; ++e) y[e] = sigmoid_for(z[i][e], DT);
+      rounded(y);
+#pragma unroll
+      for (int e = 0; e < PER; ++e) y[e] *= z[i][e];
+      rounded(y);
+#pragma unroll
+      for (int e = 0; e < PER; ++e) x[i][e] = x[i][e] * inv_rms[i] * wt[e];
+      rounded(x[i]);
+#pragma unroll
+      for (int e = 0; e < PER; ++e) y[e] *= x[i][e];
+      store_adjacent<PER>(p.y, (size_t)row * p.D + (size_t)i * step * p.D + PER * lane, DT, y);
+    }
+  };
+#pragma unroll 1
+  for (; row + step < end; row += 2 * step) rows(std::integral_constant<int, 2>{});
+  if (row < end) rows(std::integral_constant<int, 1>{});
 }
 
 template <int DT>
@@ -364,9 +445,12 @@ extern "C" int dflash_gdn_prepare_rows(const void* qkv, const void* conv_state, 
   // waves on (16 + 16 + 32 heads of 128, us, a head and several per wave: 32 tokens 4.6 / 4.8, 40 tokens 5.3 / 4.7, 128 tokens
   // 9.7 / 5.4, 200 tokens 13.8 / 7.2, 1024 tokens 22.3 / 16.3), and as many tokens each as leave the 4 waves per SIMD that fit: a
   // few more would run by themselves at the end (3072 and 8192 waves / 4096: 512 tokens 11.3 and 13.0 / 11.2, 1024 tokens 17.8 and
-  // 17.1 / 16.3).
+  // 17.1 / 16.3).  A wave may have heads of q and of k: 4 + 4 + 8 heads of 64, a head per wave and eight, 320 tokens 5.9 / 3.7, 1024 tokens
+  // 8.5 / 4.5; 2 + 2 + 8 heads of 128, 700 tokens 9.0 / 5.6.  Its accesses are of 8 bytes.
   const int per_wave = 512 / Dk;  // heads
-  const bool wide = dtype != DFLASH_FP32 && Dk == Dv && Dk != 192 && Hk % per_wave == 0 && Hv % per_wave == 0 &&
+  const uintptr_t places = (uintptr_t)qkv | (uintptr_t)conv_state | (uintptr_t)conv_w | (uintptr_t)conv_next | (uintptr_t)q | (uintptr_t)k |
+                           (uintptr_t)v | (uintptr_t)qkv_out | (uintptr_t)(2 * (strides[0] | strides[1]));
+  const bool wide = dtype != DFLASH_FP32 && Dk == Dv && Dk != 192 && 2 * Hk % per_wave == 0 && Hv % per_wave == 0 && places % 8 == 0 &&
                     (long long)B * S * heads / per_wave >= 640;
   if (wide) {
     const long long each = ((long long)B * S * heads / per_wave + 4095) / 4096, most = Dk / 8 < 16 ? Dk / 8 : 16;

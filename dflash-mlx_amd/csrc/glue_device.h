@@ -103,6 +103,20 @@ __device__ __forceinline__ void store_adjacent(void* p, size_t i, int dt, const 
     for (int e = 0; e < PER; ++e) dst[e] = v[e];
     return;
   }
+  if (dt == DFLASH_BF16 && PER % 2 == 0) {  // two elements to a conversion
+    typedef __attribute__((ext_vector_type(2))) __bf16 pair_t;
+    typedef __attribute__((ext_vector_type(2))) float floats_t;
+    uint32_t words[PER];
+#pragma unroll
+    for (int e = 0; e + 1 < PER; e += 2) words[e / 2] = __builtin_bit_cast(uint32_t, __builtin_convertvector((floats_t{v[e], v[e + 1]}), pair_t));
+    uint16_t* const dst = (uint16_t*)p + i;
+#pragma unroll
+    for (int e = 0; e + 1 < PER; e += PER % 4 == 0 ? 4 : 2) {
+      if constexpr (PER % 4 == 0) *reinterpret_cast<uint2*>(dst + e) = uint2{words[e / 2], words[e / 2 + 1]};
+      else *reinterpret_cast<uint32_t*>(dst + e) = words[e / 2];
+    }
+    return;
+  }
   uint32_t h[PER];
 #pragma unroll
   for (int e = 0; e < PER; ++e) h[e] = dt == DFLASH_BF16 ? f32_to_bf16_bits(v[e]) : f32_to_f16_bits(v[e]);

@@ -380,6 +380,13 @@ def test_several_heads_per_wave(native_lib, B, S, Hk, Hv, D, K, masked):
         test_long_prompts_and_strided_projections(native_lib, name, B, S, Hk, Hv, D, D, K, masked)
 
 
+@pytest.mark.parametrize("B,S,Hk,Hv,D,K,masked", [(1, 321, 4, 8, 64, 4, False), (1, 700, 4, 8, 64, 3, True), (1, 645, 2, 4, 128, 4, True), (2, 643, 1, 2, 256, 2, False)])
+def test_query_and_key_heads_in_one_wave(native_lib, B, S, Hk, Hv, D, K, masked):
+    """Fewer q heads than a wave has room for: the same bits."""
+    for name in ("bf16", "fp16"):
+        test_long_prompts_and_strided_projections(native_lib, name, B, S, Hk, Hv, D, D, K, masked)
+
+
 @pytest.mark.parametrize("name", ["bf16", "fp16"])
 def test_activations_of_every_16_bit_number(native_lib, name):
     """The sigmoid behind beta, the conv's and the norm's silu and the attention's gate, for all 65536 numbers of the type.  Its fp32
