@@ -120,7 +120,13 @@ int qmm_resident_launch(const void* x, const void* w, const void* scales, const 
   return DFLASH_OK;
 }
 
-// 17 to 80 rows: the slices of K that take the least time by a model fitted to 328 combinations of 25 matrices, 32 to 80 rows and 1 to 6
+// Tiles of 16 rows: two at least, which is what a call of up to 16 rows takes whose K or columns the kernel for those does not serve (rows that are not
+// there are read as zeros and not stored).  16 rows, us, through the any-rows product
+// and here: 10496 x 352 12.1 / 7.3, 4096 x 3936 in groups of 32 10.9 / 7.9, 2688 x 2880 in groups of 32 9.8 / 6.4, 1536 x 1632 with the activation 8.7 / 5.2;
+// three rows of 10752 x 320 11.2 / 7.0.
+int row_tiles_of(int M) { return M <= 32 ? 2 : (M + 15) / 16; }
+
+// Up to 80 rows: the slices of K that take the least time by a model fitted to 328 combinations of 25 matrices, 32 to 80 rows and 1 to 6
 // slices (4.7 % rms, what it picks is within 3 % of the best of its call).  The caller takes this kernel where that is less than what the any-rows
 // product is expected to take: 17 - 32 rows of most matrices (4096 x 4096 10.3 -> 7.5 us, 4096 x 12288 19.9 -> 12.9, 5120 x 34816 with the activation 40.7 -> 30.5),
 // 33 - 48 of those but the largest (4096 x 6144 15.1 -> 11.1), up to 80 of fewer (80 rows of 4096 x 6144 17.5 -> 13.8).  The others stay there (4096 x 24576
@@ -128,8 +134,8 @@ int qmm_resident_launch(const void* x, const void* w, const void* scales, const 
 // Of 193 calls of 18 matrices what is taken is within 0.2 % of the better of the two in the mean and 4 % at most (2.5 and 33 % before the factor below).
 bool qmm_resident_rows_plan(int M, int K, int N, int group_size, bool silu_mul, int* chunks_out, int* slices_out, double* us_out, size_t* workspace) {
   using namespace resident;
-  const int row_tiles = (M + 15) / 16, step = group_size == 128 ? 2 : 1;
-  if (row_tiles < 2 || row_tiles > kMostRowTiles || K % (kChunk * step) != 0 || N % 16 != 0 || (long long)N * K / 2 >= (1ll << 31) - (1 << 24))
+  const int row_tiles = row_tiles_of(M), step = group_size == 128 ? 2 : 1;
+  if (M < 1 || row_tiles > kMostRowTiles || K % (kChunk * step) != 0 || N % 16 != 0 || (long long)N * K / 2 >= (1ll << 31) - (1 << 24))
     return false;
   const int pieces = K / (kChunk * step), tiles = N / 16, cus = qmm_stream_grid(), most = most_chunks(group_size, row_tiles);
   if (cus > kRowCounters) return false;
@@ -152,7 +158,7 @@ bool qmm_resident_rows_plan(int M, int K, int N, int group_size, bool silu_mul, 
 int qmm_resident_rows_launch(const void* x, const void* w, const void* scales, const void* biases, void* y, void* workspace, int M, int K,
                              int N, int group_size, int dtype, bool silu_mul, int chunks, int slices, hipStream_t stream) {
   using namespace resident;
-  const int row_tiles = (M + 15) / 16;
+  const int row_tiles = row_tiles_of(M);
   const bool h16 = dtype == DFLASH_FP16;
   const Kernel k = h16 ? fp16_rows_kernel(row_tiles, group_size, chunks, silu_mul) : bf16_rows_kernel(row_tiles, group_size, chunks, silu_mul);
   DFLASH_REQUIRE(k.fn != nullptr, DFLASH_ERR_SHAPE, "dflash_qmm_rows: no kernel for M=%d K=%d N=%d gs=%d", M, K, N, group_size);

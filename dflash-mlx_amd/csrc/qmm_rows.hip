@@ -46,7 +46,7 @@
 
 namespace dflash {
 int qmm_stream_grid();
-// qmm_resident.hip: 17 to 80 rows
+// qmm_resident.hip: up to 80 rows
 bool qmm_resident_rows_plan(int M, int K, int N, int group_size, bool silu_mul, int* chunks, int* slices, double* us, size_t* workspace);
 int qmm_resident_rows_launch(const void* x, const void* w, const void* scales, const void* biases, void* y, void* workspace, int M, int K,
                              int N, int group_size, int dtype, bool silu_mul, int chunks, int slices, hipStream_t stream);
@@ -559,13 +559,14 @@ struct Shape {
   double alone, busy;  // us per stage: of one workgroup on a CU, and of each where they share it
   double start;        // us before the first product and behind the last one
   int most;            // slices
+  double loose;        // us more where scales come through registers
   const void* kernel[2][3];  // [fp16][plain, scales of the other type, silu-mul]; null: there is none, or it was never the one to take
   int rows() const { return 32 * mt; }
   int columns() const { return 32 * nt * w; }
 };
 template <int MT, int NT, int W, int KG, bool MIXED = false, bool PLAIN = true>
-Shape shape(int together, double alone, double busy, double start, int most = 16) {
-  Shape s{MT, NT, W, KG, Tile<MT, NT, W, KG>::kLdsBytes, together, alone, busy, start, most, {}};
+Shape shape(int together, double alone, double busy, double start, int most = 16, double loose = 0.0) {
+  Shape s{MT, NT, W, KG, Tile<MT, NT, W, KG>::kLdsBytes, together, alone, busy, start, most, loose, {}};
   if constexpr (PLAIN) {
     s.kernel[0][0] = (const void*)qmm_rows_kernel<false, false, MT, NT, W, KG, false>;
     s.kernel[1][0] = (const void*)qmm_rows_kernel<true, true, MT, NT, W, KG, false>;
@@ -587,12 +588,13 @@ Shape shape(int together, double alone, double busy, double start, int most = 16
 constexpr int kShapes = 18;
 const Shape* shapes() {
   static const Shape all[kShapes] = {
-      shape<1, 1, 1, 8>(1, 0.597, 0.571, 4.87), shape<2, 1, 1, 8>(1, 0.908, 0.454, 5.30), shape<1, 1, 2, 4, true>(2, 0.559, 0.472, 3.63),
-      shape<2, 1, 2, 4>(1, 0.695, 0.447, 3.67), shape<3, 1, 2, 4>(1, 0.860, 0.307, 4.55), shape<1, 2, 2, 4>(1, 0.984, 0.508, 3.75),
-      shape<2, 2, 2, 4, true>(1, 1.105, 0.401, 4.86), shape<3, 2, 2, 4>(1, 1.415, 0.390, 5.17), shape<1, 2, 4, 2>(2, 0.902, 0.767, 3.81),
+      shape<1, 1, 1, 8>(1, 0.597, 0.571, 4.87, 16, 0.17), shape<2, 1, 1, 8>(1, 0.908, 0.454, 5.30),
+      shape<1, 1, 2, 4, true>(2, 0.559, 0.472, 3.63, 16, 2.02), shape<2, 1, 2, 4>(1, 0.695, 0.447, 3.67, 16, 1.08),
+      shape<3, 1, 2, 4>(1, 0.860, 0.307, 4.55, 16, 1.8), shape<1, 2, 2, 4>(1, 0.984, 0.508, 3.75, 16, 1.14),
+      shape<2, 2, 2, 4, true>(1, 1.105, 0.401, 4.86, 16, 0.81), shape<3, 2, 2, 4>(1, 1.415, 0.390, 5.17), shape<1, 2, 4, 2>(2, 0.902, 0.767, 3.81, 16, 0.75),
       shape<3, 2, 4, 2>(1, 1.269, 0.363, 5.50), shape<4, 2, 4, 2, true>(1, 1.469, 0.524, 6.60), shape<4, 2, 2, 2>(1, 0.925, 0.546, 3.81),
-      shape<2, 2, 4, 1>(2, 0.631, 0.528, 4.78), shape<4, 2, 4, 1>(2, 0.880, 0.761, 4.92), shape<1, 1, 1, 4>(3, 0.451, 0.334, 3.53, 6),
-      shape<2, 1, 1, 4>(2, 0.607, 0.452, 3.78, 6), shape<1, 2, 1, 4>(2, 0.730, 0.491, 2.86, 6), shape<2, 2, 1, 4, false, false>(1, 0.805, 0.626, 3.57, 6)};
+      shape<2, 2, 4, 1>(2, 0.631, 0.528, 4.78), shape<4, 2, 4, 1>(2, 0.880, 0.761, 4.92), shape<1, 1, 1, 4>(3, 0.451, 0.334, 3.53, 6, 0.36),
+      shape<2, 1, 1, 4>(2, 0.607, 0.452, 3.78, 6, 0.45), shape<1, 2, 1, 4>(2, 0.730, 0.491, 2.86, 6, 0.62), shape<2, 2, 1, 4, false, false>(1, 0.805, 0.626, 3.57, 6)};
   return all;
 }
 
@@ -613,11 +615,21 @@ bool covers(int M, int K, int N, int group_size, bool mixed, int epilogue) {
          N % 16 == 0;
 }
 
+// A row's scales do not start on four bytes, or K does not fill the stages.  (Also where the arrays do not, which a plan does not know.)
+bool scales_through_registers(int K, int group_size, int kg) { return (K / group_size) % 2 != 0 || K % (kStageK * kg) != 0; }
+
 // Which tile, how many slices of K: the least of a model of the time, fitted to measured combinations (15 matrices of 1 to 178 M
 // weights, 20 to 1024 rows, every shape and number of slices; the 3039 within 30 % of the best of their call: 4.5 % rms, and what it picks of 225 calls
 // is within 0.5 % of the best on average, 12 % at worst; 2.0 and 19.5 % with the constants of the loop that met behind a stage's last step).  A workgroup takes
 // `alone` for a stage, or `busy` times those that share its CU; a chip that is full runs against its power.  Adding slices up takes trips to
 // memory and traffic at 3 TB/s and more.
+// What a shape takes more where scales come through registers (`loose`) is fitted to 4600 combinations of 120 calls with such K (odd multiples of
+// 128 from 1664 to 11904, 320 to 3072 columns, 16 to 200 rows): what is picked of them is within 1.3 % of the best on average and 10 % at worst, without
+// it 7.5 and 26 % (17 rows of 7808 x 1024 in groups of 128 11.4 -> 9.9 us, 64 of 10112 x 320 12.5 -> 11.0, 100 of 11904 x 2048 19.1 -> 17.6).
+// Four waves along K with no more than four stages and nothing to add up start sooner than the line through longer calls has it: 64 calls of K up to 1472 within
+// 2 % of the best, 4 % without that (24 rows of 384 x 224 5.4 -> 4.5 us, 24 of 512 x 1024 5.2 -> 4.6); and so do eight with one column of tiles each (58 rows of
+// 3072 x 4000 in groups of 128 10.9 -> 9.2; 116 calls of layers of 1024 to 5120 columns, 33 to 450 rows: within 0.8 % of the best in the mean).  Against the kernel whose waves met behind a stage's last step, 600 calls of such
+// layers: 0.96 of its time in the mean; up to 4 % more for K = 512 (0.15 us), up to 10 % for single ones whose choice is not the best (142 rows of 3968 x 1792).
 // Slices only while all of them find room at once.  Of more tiles than that, those of the last, incomplete round may be
 // cut, with the tile left as it is (5120 x 34816 over 1024 rows: 1088 tiles, two to a CU, the last 64 in slices, 344 us; uncut 382).
 Plan make_plan(int M, int K, int N, int group_size, int cus, bool fp16, bool mixed, bool silu_mul) {
@@ -634,6 +646,8 @@ Plan make_plan(int M, int K, int N, int group_size, int cus, bool fp16, bool mix
     double us = stretch(rounds * sh.together, p.stages) + stretch(ceil_div(parts, cus), ceil_div(p.stages, p.slices));
     us *= 1 + 0.17 * (std::min(1.0, (double)p.grid / cus) - 0.5);
     us += 0.76 + (silu_mul ? 0.84 : 0.0);
+    if (scales_through_registers(K, group_size, sh.kg)) us += sh.loose;
+    if (p.slices == 1 && sh.w == 1 && sh.nt == 1 && (sh.kg == 4 ? p.stages <= 4 : sh.mt == 1)) us -= 0.35;
     const int pieces = silu_mul ? sh.mt : sh.mt * sh.nt, at_once = silu_mul && (sh.mt == 1 || sh.mt == 4) ? 2 : 4;
     if (p.slices > 1)
       us += 0.96 + 0.806 * ceil_div(pieces, sh.kg) * ceil_div(p.slices, at_once) + 0.352 * parts * (sh.rows() * 8.0 * sh.columns()) / 3e6;
@@ -725,7 +739,7 @@ extern "C" int dflash_qmm_rows(const void* x, const uint32_t* w_q, const void* s
   a.partials = workspace ? (float*)((char*)workspace + rows::kCounterBytes) : nullptr;
   a.M = M; a.K = K; a.N = N;
   const size_t sb_bytes = (size_t)N * (K / group_size) * 2;
-  a.loose = (K / group_size) % 2 != 0 || K % (rows::kStageK * p.shape->kg) != 0 || (((uintptr_t)scales | (uintptr_t)biases) % 4) != 0 || sb_bytes >= (1ull << 31);
+  a.loose = rows::scales_through_registers(K, group_size, p.shape->kg) || (((uintptr_t)scales | (uintptr_t)biases) % 4) != 0 || sb_bytes >= (1ull << 31);
   a.group_shift = group_size == 32 ? 5 : group_size == 64 ? 6 : 7;
   a.tiles_m = p.tiles_m; a.tiles = p.tiles; a.whole = p.whole; a.slices = p.slices; a.stages = p.stages;
   const bool fp16 = act_dtype == DFLASH_FP16;

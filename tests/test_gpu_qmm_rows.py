@@ -237,3 +237,11 @@ def test_scales_past_the_registers(native_lib, M, K, N, group, silu, dtype):
     got = product(c.scales, c.biases)
     column = torch.arange(want.shape[1], device=DEV) != row
     assert torch.equal(got[:, column], want[:, column]) and got[:, row].isnan().all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,K,N,group,silu", [(1, 1152, 160, 64, False), (16, 10496, 352, 64, False), (15, 4480, 224, 32, True), (8, 17024, 96, 64, False),
+                                              (16, 2688, 2880, 32, False), (3, 1280, 1600, 32, True)])
+def test_up_to_sixteen_rows_with_weights_in_registers(native_lib, M, K, N, group, silu, dtype):
+    """K that the verify block's kernel does not take (an odd multiple of 128), or columns: rows that are not there, whole and in slices of K."""
+    test_every_tile_shape_at_its_edges(native_lib, M, K, N, group, silu, dtype)
