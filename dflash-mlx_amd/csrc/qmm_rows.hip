@@ -336,6 +336,8 @@ __global__ __launch_bounds__(64 * W * KG, 2) void qmm_rows_kernel(Args a) {
     request_chunk(chunk, 0);
     if (two_chunks) request_chunk(chunk + 1, 1);
   }
+  // (behind the scales in either form: asked for before those that come through registers, 9 of 64 calls differed from run to run, 33 rows of 3168 x 4112 in
+  // groups of 32 among them; in this order none of 64 in 200 runs each)
 #pragma unroll
   for (int j = 0; j < kWReq; ++j) request_w(st0 + 2, 2, j);
 #pragma unroll
