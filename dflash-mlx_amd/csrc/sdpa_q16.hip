@@ -136,8 +136,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
   const int bh = a.ranges.quotient((int)blockIdx.x), split = (int)blockIdx.x - bh * a.splits;
   const int b = a.key_heads.quotient(bh), hk = bh - b * a.Hk;
   const int n_begin = split * a.keys_per_split;
-  const int cached = BLOCK ? a.N - 16 : a.N;  // (a last range may have none of them)
-  const int n_end = n_begin + a.keys_per_split < cached ? n_begin + a.keys_per_split : cached;
+  const int n_end = n_begin + a.keys_per_split < a.N ? n_begin + a.keys_per_split : a.N;
+  // BLOCK: keys from here on are the block's own, which the cache does not hold yet; a last range of fewer than 16 keys
+  // leaves some of them to the one before it.
+  const int cached = BLOCK ? a.N - 16 : a.N;
+  const bool has_block = BLOCK && n_end > cached;
+  const int n_there = n_end < cached ? n_end : cached;  // (may be n_begin or less)
+  const int full = !has_block ? n_end : n_begin < cached ? n_begin + (cached - n_begin) / kTileKeys * kTileKeys : n_begin;
   const int j = lane & 15, kb = lane >> 4;
   const bool computes = wave < a.G * CS;  // the other waves only move tiles
   int slice = 0, of_group = computes ? wave : 0;  // wave / G, wave % G
@@ -167,7 +172,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     for (int i = 0; i < kLoads; ++i) {
       const int c = tid + i * kThreads;
       const int key = c / (D / 8), piece = c % (D / 8);
-      const int n = n0 + key < n_end ? n0 + key : n_end - 1;
+      const int n = n0 + key < n_there ? n0 + key : n_there - 1;
       st.k[i] = *reinterpret_cast<const u32x4_t*>(kbase + (size_t)n * a.k_seq_stride + 8 * piece);
       st.v[i] = *reinterpret_cast<const u32x4_t*>(vbase + (size_t)n * a.v_seq_stride + 8 * piece);
     }
@@ -202,12 +207,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
   fetch(stage0, n_begin);
   fetch(stage1, n_begin + kTileKeys);
 
-  [[maybe_unused]] const bool has_block = BLOCK && split == a.splits - 1;
-  [[maybe_unused]] uint16_t* const block_k = lds + 4 * kTileElems;  // the block's own tile, its upper half zeros
-  [[maybe_unused]] uint16_t* const block_v = block_k + kTileElems;
+  [[maybe_unused]] uint16_t* const block_k = lds + 4 * kTileElems;  // the block's own 16 rows
+  [[maybe_unused]] uint16_t* const block_v = block_k + 16 * P;
   if constexpr (BLOCK) {
-    // Norm and rotation of the queries by the waves that multiply with them, of the block's keys by the last range, which also
-    // writes them to the cache; all while the first tiles are on their way.  A launch of its own for it (attn_prepare_kernel,
+    // Norm and rotation of the queries by the waves that multiply with them, of the block's keys by the ranges that have some of
+    // them, the last of which also writes them to the cache; all while the first tiles are on their way.  A launch of its own for it (attn_prepare_kernel,
     // whose bits these are) took 4 to 5 us and its place in the queue.  Here every range does it again, bound by its vector
     // instructions: 1.5 us of a launch with heads of 128, 3.2 of 256 (4.7 with one wave for all of a head's queries and the
     // powers computed by every thread).  Layer calls, us, before and with it: 4 112 keys of 8 x 256 48.1 -> 46.4, 32 716 89.5 ->
@@ -215,7 +219,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     constexpr int PER = D / 64, kRowsPerWave = 16 / (kThreads / 64);
     const BlockArgs& p = a.block;
     const int half = p.half, pitch = half + kTurnPad;
-    float2* const turn = reinterpret_cast<float2*>(lds + 6 * kTileElems);  // cosine and sine, [token][pair]
+    float2* const turn = reinterpret_cast<float2*>(lds + 5 * kTileElems);  // cosine and sine, [token][pair]
     float* const frequency = reinterpret_cast<float*>(turn + 16 * pitch);
     uint32_t k_raw[kRowsPerWave][PER], v_raw[kRowsPerWave][PER], kw_raw[PER];
     if (has_block) {
@@ -352,13 +356,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         norm_and_turn<PER>(x, w, p.k_eps, cs, sn, rotates, upper, other, dt);
         const long long at = b * a.k_batch_stride + hk * a.k_head_stride + (a.N - 16 + row) * a.k_seq_stride + c;
         const long long vat = b * a.v_batch_stride + hk * a.v_head_stride + (a.N - 16 + row) * a.v_seq_stride + c;
-        store_adjacent<PER>(p.k_cache, (size_t)at, dt, x);
         store_adjacent<PER>(block_k, (size_t)(row * P + c), dt, x);
-        store_raw<PER>(p.v_cache + vat, v_raw[u]);
         store_raw<PER>(block_v + row * P + c, v_raw[u]);
-        const uint32_t zero[PER] = {};
-        store_raw<PER>(block_k + (16 + row) * P + c, zero);
-        store_raw<PER>(block_v + (16 + row) * P + c, zero);
+        if (split == a.splits - 1) {
+          store_adjacent<PER>(p.k_cache, (size_t)at, dt, x);
+          store_raw<PER>(p.v_cache + vat, v_raw[u]);
+        }
       }
     }
   }
@@ -368,16 +371,24 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
   for (int c = 0; c < kCols; ++c) O[c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   float m_run = kMasked, l_run = 0.f;  // l_run: this lane's keys only, merged at the end
 
-  auto compute_tile = [&](const uint16_t* sk, int n0, int n_end) __attribute__((always_inline)) {
+  // OWN: a tile with keys of the block, which are read where they were prepared.  Where they take their places among the cached ones,
+  // ranges and tiles are those of a block whose rows were in the cache before the launch, and so are the results' bits.
+  auto compute_tile = [&](const uint16_t* sk, int n0, auto own) __attribute__((always_inline)) {
+    constexpr bool OWN = decltype(own)::value;
     if (computes) {
       const uint16_t* sv = sk + kTileElems;
+      auto row_of = [&](const uint16_t* tile, const uint16_t* block, int i) __attribute__((always_inline)) {  // of key n0 + i
+        if constexpr (!OWN) return tile + i * P;
+        const int at = n0 + i - cached;
+        return at < 0 ? tile + i * P : block + (at < 16 ? at : 15) * P;  // (behind the last key: that one, not counted)
+      };
       // S^T = K Q^T for the two 16-key halves of the tile
       // (all reads of the tile are issued before the first product: one LDS latency, not sixteen)
       uint4 kf[2][D / 32];
 #pragma unroll
       for (int s = 0; s < D / 32; ++s)
 #pragma unroll
-        for (int t = 0; t < 2; ++t) kf[t][s] = *reinterpret_cast<const uint4*>(sk + (16 * t + j) * P + 32 * s + 8 * kb);
+        for (int t = 0; t < 2; ++t) kf[t][s] = *reinterpret_cast<const uint4*>(row_of(sk, block_k, 16 * t + j) + 32 * s + 8 * kb);
       f32x4_t st[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
       for (int s = 0; s < D / 32; ++s)
@@ -423,13 +434,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
                         pack2<FP16>(p[6], p[7])};
       // O^T += V^T P^T, 16 columns of V at a time
       const int src = lane & 15;  // source lane inside the group of 16: key 4 kb + src / 4, columns 4 (src % 4) ..+3
-      const uint16_t* vrow = sv + (4 * kb + (src >> 2)) * P + 4 * (src & 3) + 16 * kCols * slice;
+      const int piece = 4 * (src & 3) + 16 * kCols * slice;
+      const uint16_t* const vlow = row_of(sv, block_v, 4 * kb + (src >> 2)) + piece;
+      const uint16_t* const vhigh = row_of(sv, block_v, 16 + 4 * kb + (src >> 2)) + piece;
       typedef __attribute__((address_space(3))) s16x4_t lds_s16x4;
       s16x4_t lo[kCols], hi[kCols];
 #pragma unroll
       for (int c = 0; c < kCols; ++c) {
-        lo[c] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(vrow + 16 * c));
-        hi[c] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(vrow + 16 * P + 16 * c));
+        lo[c] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(vlow + 16 * c));
+        hi[c] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(vhigh + 16 * c));
       }
 #pragma unroll
       for (int c = 0; c < kCols; ++c) {
@@ -445,22 +458,24 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     fetch(stage0, n_begin + 2 * kTileKeys);
   }
   __syncthreads();
-  for (int n0 = n_begin; n0 < n_end; n0 += 2 * kTileKeys) {
+  for (int n0 = n_begin; n0 < full; n0 += 2 * kTileKeys) {
     // even tile in buffer 0, the next one in stage 1, the one after it on its way to stage 0
-    compute_tile(lds, n0, n_end);
+    compute_tile(lds, n0, std::false_type{});
     stash(stage1, 1);
     fetch(stage1, n0 + 3 * kTileKeys);
     __syncthreads();
-    if (n0 + kTileKeys >= n_end) break;
-    compute_tile(lds + 2 * kTileElems, n0 + kTileKeys, n_end);
+    if (n0 + kTileKeys >= full) break;
+    compute_tile(lds + 2 * kTileElems, n0 + kTileKeys, std::false_type{});
     stash(stage0, 0);
     fetch(stage0, n0 + 4 * kTileKeys);
     __syncthreads();
   }
   if constexpr (BLOCK) {
     if (has_block) {
-      __syncthreads();  // (a range without cached keys has met nowhere since the block's tile was written)
-      compute_tile(block_k, a.N - 16, a.N);
+      // the first of these tiles may begin with cached keys and is in the buffer of its turn; a second one is the block's alone
+      const uint16_t* const from = lds + ((full - n_begin) / kTileKeys & 1) * 2 * kTileElems;
+#pragma unroll 1
+      for (int n0 = full; n0 < n_end; n0 += kTileKeys) compute_tile(from, n0, std::true_type{});
     }
   }
 
@@ -582,7 +597,6 @@ __global__ __launch_bounds__(256) void sdpa_q16_merge_kernel(SdpaArgs a, int D) 
   }
 }
 
-// keys: that the ranges are to share.
 int pick_splits(int B, int Hk, int N, int* keys_per_split) {
   // About one workgroup per compute unit, and never less than 128 keys per split: every split
   // adds B * Hq * 16 * (2 D + 8) bytes of partial results, written once and read once.
@@ -598,10 +612,6 @@ int pick_splits(int B, int Hk, int N, int* keys_per_split) {
   *keys_per_split = per;
   return (N + per - 1) / per;  // no empty split
 }
-
-// A block that its launch prepares: the last range has these keys fewer than the others, for the block's own tile and for
-// what stands before it.
-constexpr int kBlockKeys = 48;
 
 size_t partial_bytes(int splits, int B, int Hq, int D) {
   return splits == 1 ? 0 : (size_t)splits * B * Hq * 16 * (D * sizeof(uint16_t) + 2 * sizeof(float));
@@ -619,9 +629,7 @@ extern "C" size_t dflash_sdpa_q16_workspace_bytes(int B, int Hq, int Hk, int N, 
 
 extern "C" size_t dflash_attn_block_workspace_bytes(int B, int Hq, int Hk, int N, int D) {
   using namespace dflash;
-  if (B <= 0 || Hq <= 0 || Hk <= 0 || N <= 16 || D <= 0) return 0;
-  int per = 0;
-  return partial_bytes(pick_splits(B, Hk, N - 16 + kBlockKeys, &per), B, Hq, D);
+  return N > 16 ? dflash_sdpa_q16_workspace_bytes(B, Hq, Hk, N, D) : 0;
 }
 
 namespace dflash {
@@ -654,7 +662,7 @@ int sdpa_launch(const void* q, const void* k, const void* v, const void* mask, c
   a.k_batch_stride = k_batch_stride; a.k_head_stride = k_head_stride; a.k_seq_stride = k_seq_stride;
   a.v_batch_stride = v_batch_stride; a.v_head_stride = v_head_stride; a.v_seq_stride = v_seq_stride;
   a.B = B; a.Hq = Hq; a.Hk = Hk; a.N = N; a.G = Hq / Hk;
-  a.splits = pick_splits(B, Hk, block ? N - 16 + kBlockKeys : N, &a.keys_per_split);
+  a.splits = pick_splits(B, Hk, N, &a.keys_per_split);
   if (block) a.block = *block;
   a.ranges = Divisor::of(a.splits); a.key_heads = Divisor::of(Hk); a.heads = Divisor::of(Hq);
   a.scale = scale;
@@ -676,7 +684,7 @@ int sdpa_launch(const void* q, const void* k, const void* v, const void* mask, c
   hipStream_t s = (hipStream_t)stream;
   // column split: as many waves as fit eight, in powers of two
   const int cs = a.G <= 2 ? 4 : a.G <= 4 ? 2 : 1;
-  const int tiles = block ? 6 : 4;
+  const int tiles = block ? 5 : 4;  // (a block's rows: half a tile of keys, half of values)
   const size_t lds_bytes = (size_t)tiles * kTileKeys * (D + kPadElems) * sizeof(uint16_t) +
                            (block ? turn_bytes(block->half) : 0);
   const size_t lds_most = (size_t)tiles * kTileKeys * (D + kPadElems) * sizeof(uint16_t) +

@@ -561,7 +561,7 @@ int dflash_sdpa_q16_gated(const void* q, const void* k, const void* v, const voi
  * dflash_attn_prepare and dflash_sdpa_q16_gated of a block of 16 tokens behind N - 16 cached ones, without a mask, in the
  * launches of the attention alone: q [B, 16, Hq, 2 D] (a head's queries, then its gate), k, v [B, 16, Hk, D] as the projections
  * gave them, through strides (elements); k_cache, v_cache [B, Hk, N.., D] through strides, rows N - 16 .. N - 1 of them written
- * here with the bits that dflash_attn_prepare leaves; out [B, 16, Hq, D].
+ * here with the bits that dflash_attn_prepare leaves; out [B, 16, Hq, D] has those of the two calls.
  * D 128 or 256, rope_dims 64, 128 or 256; norm weights of the activations' dtype; q, k, v, their rows and the weights 16-byte
  * aligned; more than one range of keys (a workspace size of 0: there is no form).  workspace as for dflash_sdpa_q16.
  */

@@ -226,35 +226,43 @@ def _block_layer(*args):
     (1, 16, 2, 128, 128, 1025, torch.float16, True),    # eight heads of a key head, an odd prefix
     (2, 3, 1, 128, 64, 1039, torch.bfloat16, False),    # three heads, half of the features turned
     (1, 4, 4, 256, 64, 130, torch.float16, False),      # waves share a head four ways
-    (1, 6, 2, 256, 128, 90, torch.bfloat16, True),      # two ranges, the last one without a cached key
-    (1, 4, 2, 128, 128, 112, torch.bfloat16, True),     # ... with one tile of them
+    (1, 6, 2, 256, 128, 90, torch.bfloat16, True),      # one range: the launch has no form
+    (1, 4, 2, 128, 128, 112, torch.bfloat16, True),
+    (1, 6, 2, 256, 128, 1024, torch.bfloat16, True),    # the last range without a cached key
+    (1, 4, 2, 128, 128, 1020, torch.bfloat16, True),    # ... with 12 of the block's own, four are the range's before it
+    (2, 16, 2, 128, 64, 1015, torch.bfloat16, True),    # ... with seven
+    (1, 8, 2, 256, 256, 250, torch.float16, False),     # the block's keys begin in one tile and end in the next
+    (1, 32, 8, 256, 256, 32700, torch.bfloat16, True),
 ])
 def test_block_from_its_projections_in_the_launch_of_its_attention(monkeypatch, B, Hq, Hk, D, dims, prefix, dtype, joint):
-    """Against the launch of its own for norms, rotation and cache rows: the same rows in the cache, an attention that is as
-    close to 64 bits as that one's."""
+    """Against the launch of its own for norms, rotation and cache rows, which is what a cache without room for the block
+    takes: the same rows in the cache and the same bits of the attention, as close to 64 bits."""
     gen = torch.Generator(device="cuda").manual_seed(21)
     attn, outs = _block_layer(B, 16, Hq, Hk, D, dims, dtype, dtype, gen, joint)
     x = torch.empty((B, 16, 8), device="cuda")
     before = [torch.randn((B, Hk, prefix, D), generator=gen, device="cuda").to(dtype) for _ in range(2)]
     fused, real = [], A._native.host().attn_block
     results = []
-    for in_one in (True, False):
-        if not in_one:
+    for in_one in (True, None, False):  # (None: no room)
+        if in_one is False:
             monkeypatch.setattr(A, "_attend_in_one", lambda *a: None)
-        else:
+        elif in_one:
             spy = type("H", (), {"__getattr__": lambda self, n, h=A._native.host(): getattr(h, n),
                                  "attn_block": lambda self, *a: fused.append(real(*a)) or fused[-1]})()
             monkeypatch.setattr(A._native, "host", lambda: spy)
         cache = KVCache()
         cache.update_and_fetch(*before)
-        if cache.keys.shape[2] < prefix + 16:
+        if in_one is None:
+            cache.keys, cache.values = (t[:, :, :prefix].contiguous() for t in (cache.keys, cache.values))
+        elif cache.keys.shape[2] < prefix + 16:
             cache._make_room(B, Hk, 16, D, D, *before)
         y = attn(x, mask="causal" if in_one else None, cache=cache)
         assert cache.offset == prefix + 16
         results.append((y, *cache.state))
-    assert fused and fused[-1] is not None
-    (got, keys, values), (ref, ref_keys, ref_values) = results
+    assert fused and (fused[-1] is not None) == (prefix + 16 > 128)
+    (got, keys, values), grown, (ref, ref_keys, ref_values) = results
     assert torch.equal(keys, ref_keys) and torch.equal(values, ref_values)
+    assert torch.equal(got, ref) and all(torch.equal(a, b) for a, b in zip(grown, results[2]))
     q = A.rms_norm_ops(outs[0].reshape(B, 16, Hq, 2 * D)[..., :D], attn.q_norm.weight, attn.q_norm.eps).transpose(1, 2)
     q = attn.rope(q, offset=prefix).double()
     k, v = (t.double().repeat_interleave(Hq // Hk, dim=1) for t in (ref_keys, ref_values))
@@ -263,8 +271,7 @@ def test_block_from_its_projections_in_the_launch_of_its_attention(monkeypatch, 
     o = torch.matmul(torch.softmax(scores.masked_fill(late, float("-inf")), dim=-1), v).transpose(1, 2)
     exact = (o * torch.sigmoid(outs[0].reshape(B, 16, Hq, 2 * D)[..., D:].double())).reshape(B, 16, Hq * D)
     err = [((t.double() - exact).norm() / exact.norm()).item() for t in (got, ref)]
-    # (partial outputs, the output, the gate and their product are rounded to the type, each by eps / sqrt(48) on average, and other
-    # ranges of keys have other partial outputs)
+    # (partial outputs, the output, the gate and their product are rounded to the type, each by eps / sqrt(48) on average)
     assert err[0] <= max(1.1 * err[1], 4 * torch.finfo(dtype).eps / 48 ** 0.5), err
 
 
