@@ -146,6 +146,13 @@ __device__ __forceinline__ void store_raw(uint16_t* dst, const uint32_t (&raw)[P
   }
 }
 
+// A number of 32 bits that is one before it is rounded to fp16: the compiler makes one instruction with one rounding
+// (v_fma_mixlo_f16) of some products and their conversion, where it knows the type, and not of others.
+__device__ __forceinline__ float in_full(float v) {
+  asm("" : "+v"(v));
+  return v;
+}
+
 // Norm and rotation of one head by a wave, a lane on PER adjacent features: x <- turned(round(x rsqrt(mean x^2 + eps) w)), the
 // products and sums of the rotation rounded one by one, as the array operators do it.  other: the lane of the pair's other half.
 template <int PER>
@@ -159,11 +166,11 @@ __device__ __forceinline__ void norm_and_turn(float (&x)[PER], const float (&w)[
   const float inv_rms = 1.0f / sqrtf(wave_sum(ss) * (1.0f / (float)(64 * PER)) + eps);
 #pragma unroll
   for (int e = 0; e < PER; ++e) {
-    x[e] = round_through(x[e] * inv_rms * w[e], dt);
+    x[e] = round_through(in_full(x[e] * inv_rms * w[e]), dt);
     const float y = __shfl(x[e], other, 64);  // the other half's feature of the pair
     if (rotates) {
       const float a = x[e] * cs[e], d = y * sn[e];
-      x[e] = upper ? d + a : a - d;
+      x[e] = in_full(upper ? d + a : a - d);
     }
   }
 }

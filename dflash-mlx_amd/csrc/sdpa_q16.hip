@@ -288,6 +288,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
       auto word = [](const uint4& v, int w) __attribute__((always_inline)) { return w == 0 ? v.x : w == 1 ? v.y : w == 2 ? v.z : v.w; };
       auto low = [](uint32_t w) __attribute__((always_inline)) { return elem_to_f32<FP16>((uint16_t)w); };
       auto high = [](uint32_t w) __attribute__((always_inline)) { return elem_to_f32<FP16>((uint16_t)(w >> 16)); };
+      auto rounded = [](float x, float y) __attribute__((always_inline)) {
+        return FP16 ? pack2<FP16>(in_full(x), in_full(y)) : pack2<FP16>(x, y);
+      };
 #pragma unroll
       for (int s = 0; s < S; ++s)
 #pragma unroll
@@ -299,7 +302,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             asm("" : "+v"(other_x), "+v"(other_w));  // (a choice of values: of addresses, the pieces would go to memory)
             x = slice == c ? other_x : x, w = slice == c ? other_w : w;
           }
-          mine[s][i] = pack2<FP16>(low(x) * inv_rms * low(w), high(x) * inv_rms * high(w));
+          mine[s][i] = rounded(low(x) * inv_rms * low(w), high(x) * inv_rms * high(w));
         }
       // features i and i + half, in pieces s and s + half / 32 of one lane
       auto rotate = [&](auto apart) __attribute__((always_inline)) {
@@ -313,8 +316,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
               const f32x4_t t = *reinterpret_cast<const f32x4_t*>(turn + j * pitch + 32 * s + 8 * kb + 2 * (kWords * slice + i));
               const uint32_t xw = mine[s][i], yw = mine[s + A][i];
               const float x0 = low(xw), x1 = high(xw), y0 = low(yw), y1 = high(yw);
-              mine[s][i] = pack2<FP16>(x0 * t[0] - y0 * t[1], x1 * t[2] - y1 * t[3]);
-              mine[s + A][i] = pack2<FP16>(x0 * t[1] + y0 * t[0], x1 * t[3] + y1 * t[2]);
+              mine[s][i] = rounded(x0 * t[0] - y0 * t[1], x1 * t[2] - y1 * t[3]);
+              mine[s + A][i] = rounded(x0 * t[1] + y0 * t[0], x1 * t[3] + y1 * t[2]);
             }
         }
       };

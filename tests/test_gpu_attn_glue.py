@@ -233,6 +233,8 @@ def _block_layer(*args):
     (2, 16, 2, 128, 64, 1015, torch.bfloat16, True),    # ... with seven
     (1, 8, 2, 256, 256, 250, torch.float16, False),     # the block's keys begin in one tile and end in the next
     (1, 32, 8, 256, 256, 32700, torch.bfloat16, True),
+    (2, 16, 2, 128, 64, 1015, torch.float16, True),     # a key feature whose product falls between two numbers of fp16 once in fp32
+    (8, 16, 16, 256, 64, 200, torch.float16, True),     # 524288 key features, one in 8192 of them such a one
 ])
 def test_block_from_its_projections_in_the_launch_of_its_attention(monkeypatch, B, Hq, Hk, D, dims, prefix, dtype, joint):
     """Against the launch of its own for norms, rotation and cache rows, which is what a cache without room for the block
