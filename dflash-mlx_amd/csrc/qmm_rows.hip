@@ -117,7 +117,9 @@ __device__ __forceinline__ f32x16_t mfma32(uint4 w, uint4 x, f32x16_t c) {
 }
 
 // Lane i of the wave: 16 bytes from rsrc + voff + soff to LDS at lds + 16 i, past the registers.  The compiler counts neither the
-// request nor what it writes: whoever reads that place waits with stage_done() first.
+// request nor what it writes: whoever reads that place waits with stage_done() first, and whoever asks for it to be filled again
+// has met every wave that read it since (stage_done() or all_read(), whose clobber keeps reads on their side).  Requests and
+// these two stay in the order they are written in, all being volatile.
 __device__ __forceinline__ void request16(__amdgpu_buffer_rsrc_t rsrc, uint32_t lds, uint32_t voff, uint32_t soff) {
   asm volatile("s_mov_b32 m0, %0\n s_nop 0\n buffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "m0");
 }
@@ -126,6 +128,9 @@ template <int LEFT>
 __device__ __forceinline__ void stage_done() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n s_barrier" ::"n"(LEFT) : "memory");
 }
+
+// What this wave has read from LDS is in registers, and so is what every other wave has.
+__device__ __forceinline__ void all_read() { asm volatile("s_waitcnt lgkmcnt(0)\n s_barrier" ::: "memory"); }
 
 template <int MT, int NT, int W, int KG>
 struct Tile {
@@ -221,10 +226,14 @@ __global__ __launch_bounds__(64 * W * KG, 2) void qmm_rows_kernel(Args a) {
   };
   // a chunk is the scales and biases of kGroups groups of every row, 16 bytes for eight of them
   constexpr int kSbPieces = kGroups / 4 * BN, SL = (kSbPieces + kThreads - 1) / kThreads;
+  static_assert(kSbPieces % 64 == 0, "whole waves of pieces");
+  auto has_piece = [&](int i) __attribute__((always_inline)) { return kSbPieces % kThreads == 0 || 64 * wid + kThreads * i < kSbPieces; };
   uint4 sv[SL];
   auto load_chunk = [&](int chunk, uint4 (&sv)[SL]) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < SL; ++i) {
+      if (!has_piece(i)) break;  // (no load that its wave never looks at: the compiler waits for those where it next writes their registers.  33
+                                  // rows of 3168 x 4112 in groups of 32 14.6 -> 13.6 us, 100 of 11904 x 2048 in groups of 128 20.5 -> 19.6)
       const int e = tid + kThreads * i, p = e % BN, g0 = kGroups * chunk + (e / (2 * BN)) * 8;
       int n = first_row(p >> 5) + row_in_tile(p & 31);
       const int end = SILU_MUL && ((p >> 5) & 1) ? a.N : out_cols;
@@ -244,10 +253,8 @@ __global__ __launch_bounds__(64 * W * KG, 2) void qmm_rows_kernel(Args a) {
   };
   auto store_chunk = [&](int buf, const uint4 (&sv)[SL]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < SL; ++i) {
-      const int e = tid + kThreads * i;
-      if (kSbPieces % kThreads == 0 || e < kSbPieces) *reinterpret_cast<uint4*>(sb_lds + buf * T::kSbBytes + e * 16) = sv[i];
-    }
+    for (int i = 0; i < SL; ++i)
+      if (has_piece(i)) *reinterpret_cast<uint4*>(sb_lds + buf * T::kSbBytes + (tid + kThreads * i) * 16) = sv[i];
   };
   // The same past the registers, a request for 64 rows at a time: scales in registers made the compiler wait for every request in flight, codes
   // of the next stages included.  What is asked for behind the end of a row is never read (a.loose: where it would be, and where rows start
@@ -336,8 +343,7 @@ __global__ __launch_bounds__(64 * W * KG, 2) void qmm_rows_kernel(Args a) {
     request_chunk(chunk, 0);
     if (two_chunks) request_chunk(chunk + 1, 1);
   }
-  // (behind the scales in either form: asked for before those that come through registers, 9 of 64 calls differed from run to run, 33 rows of 3168 x 4112 in
-  // groups of 32 among them; in this order none of 64 in 200 runs each)
+  // (behind the scales in either form: the wait for those in registers is one for everything that was asked for before them)
 #pragma unroll
   for (int j = 0; j < kWReq; ++j) request_w(st0 + 2, 2, j);
 #pragma unroll
@@ -347,6 +353,12 @@ __global__ __launch_bounds__(64 * W * KG, 2) void qmm_rows_kernel(Args a) {
   read_codes();
 #pragma unroll
   for (int s = 0; s < kAhead; ++s) read_x(s, 0);
+  // The first stage asks for codes into the buffer that was just read, before its own meeting: the codes of a row of 2 KG pieces come
+  // by requests of other waves than those that read them.  Without this meeting a wave that was held up between the two
+  // multiplied with codes of stage st0 + 3 (seen while the requests stood before scales in registers, for whose registers the compiler
+  // put a wait for all of memory right there: 9 of 64 calls differed from run to run).  It takes 0.1 us (100 rows of 512 x 2048 5.3 -> 5.4,
+  // 150 of 2048 x 8192 14.1 -> 14.3, 200 of 4096 x 4096 18.6 -> 19.1, long calls as before).
+  if constexpr (KG > 1) all_read();
   take_scales();
 #pragma unroll
   for (int t = 0; t < NT; ++t) wf[0][t] = dequant8<FP16>(wc[t].x, sc[t], sc16[t], bc[t], mask0, mask4);
@@ -371,7 +383,8 @@ __global__ __launch_bounds__(64 * W * KG, 2) void qmm_rows_kernel(Args a) {
       // the stage after that, whose place is free, has a whole stage to come.
       if (s == 3) {
         if (brings_chunk && loose) store_chunk(cbuf_now ^ 1, sv);
-        stage_done<kWReq>();  // (the codes asked for in this stage may take another one)
+        // (the codes asked for in this stage may take another one; loads of scales among the requests make the wait longer, never shorter)
+        stage_done<kWReq>();
 #pragma unroll
         for (int q = 0; q < kAhead; ++q) read_x(q, xbuf ^ 1);
 #pragma unroll

@@ -14,6 +14,8 @@ cycle after it has been issued; where the compiler places such a store it also p
 states, but it cannot see one inside a hand-written block, so every such store in a block must
 be followed by wait states of its own (seen on the device as partial tiles whose upper two
 words were those of whatever the next instruction wrote).
+``check_refills``: in the any-rows kernels whose waves read codes that other waves asked for, the waves meet
+between the prologue's reads of the first buffer and the first stage, whose requests fill it again.
 """
 from __future__ import annotations
 
@@ -40,6 +42,9 @@ KERNELS = (
 # source, number of counter bumps (arrival counters; the chained kernel's per-problem and exit counters too)
 ARRIVALS = (("qmm_m16.hip", 24), ("qmm_m16_stream.hip", 0), ("qmm_m16_chain.hip", 64), ("qmm_resident_bf16.hip", 0),
             ("qmm_resident_fp16.hip", 0), ("qmm_resident_rows_bf16.hip", 42), ("qmm_resident_rows_fp16.hip", 42))
+
+# source, mangled-name prefix of the any-rows kernel, instantiations
+REFILLS = ("qmm_rows.hip", "_ZN6dflash4rows15qmm_rows_kernel", 62)
 
 
 def _regs(text: str) -> set:
@@ -156,17 +161,34 @@ def check_wide_stores(text: str, source: str) -> int:
     return found
 
 
+def check_refills(text: str, prefix: str, count: int) -> None:
+    """``prefix`` up to the template arguments, of which the last integer but one flag is the number of sets of waves."""
+    kernels = re.findall(rf"^({prefix}\w+):", text, flags=re.M)
+    if len(kernels) != count:
+        raise AssertionError(f"{prefix}: {len(kernels)} instantiations, expected {count}")
+    for name in kernels:
+        if re.findall(r"Li(\d+)E", name)[-1] == "1":  # a wave reads what it asked for itself
+            continue
+        body = text[text.index(name + ":"):]
+        ops = re.findall(r"s_barrier|ds_read_b128|v_mfma", body[:body.index(".Lfunc_end")])
+        # the first stage is there; its first product is before its first request (whose block may stand anywhere in the text)
+        first = ops[ops.index("s_barrier") + 1:ops.index("v_mfma")]
+        if "ds_read_b128" not in first or "s_barrier" not in first[first.index("ds_read_b128"):]:
+            raise AssertionError(f"{name}: a buffer is asked for again before every wave has read it")
+
+
 def check_all() -> None:
     """Every check on every source; raises AssertionError on the first finding."""
     from concurrent.futures import ThreadPoolExecutor
 
-    sources = sorted({s for s, *_ in KERNELS} | {s for s, _ in ARRIVALS})
+    sources = sorted({s for s, *_ in KERNELS} | {s for s, _ in ARRIVALS} | {REFILLS[0]})
     with ThreadPoolExecutor(max_workers=7) as pool:
         isa = dict(zip(sources, pool.map(compile_to_isa, sources)))
     for source, prefix, count, min_reads in KERNELS:
         check_kernels(isa[source], prefix, count, min_reads)
     for source, arrivals in ARRIVALS:
         check_arrivals(isa[source], source, arrivals)
+    check_refills(isa[REFILLS[0]], *REFILLS[1:])
     for source in ("qmm_m16_stream.hip", "qmm_m16_chain.hip", "qmm_resident_bf16.hip", "qmm_resident_fp16.hip",
                    "qmm_resident_rows_bf16.hip", "qmm_resident_rows_fp16.hip"):
         if check_wide_stores(isa[source], source) == 0:

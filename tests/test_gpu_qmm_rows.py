@@ -245,3 +245,18 @@ def test_scales_past_the_registers(native_lib, M, K, N, group, silu, dtype):
 def test_up_to_sixteen_rows_with_weights_in_registers(native_lib, M, K, N, group, silu, dtype):
     """K that the verify block's kernel does not take (an odd multiple of 128), or columns: rows that are not there, whole and in slices of K."""
     test_every_tile_shape_at_its_edges(native_lib, M, K, N, group, silu, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,K,N,group,silu", [
+    (33, 3168, 4112, 32, False), (33, 3232, 2064, 32, False),           # an odd number of groups, K that ends inside a stage: sliced, whole
+    (17, 10112, 416, 128, False), (100, 11904, 2048, 128, False),       # slices that begin inside a chunk of scales
+    (100, 5440, 1040, 64, False), (70, 6432, 528, 32, False), (45, 4128, 1056, 32, True), (400, 4352, 2320, 128, False)])
+def test_the_same_bits_call_after_call(native_lib, M, K, N, group, silu, dtype):
+    """Waves read codes that other waves asked for: none of them may be filled again before.  Against fp64 once, then against itself."""
+    test_every_tile_shape_at_its_edges(native_lib, M, K, N, group, silu, dtype)
+    c = make_qmm_case(K, N, 8000 + M, group_size=group, dtype=dtype, M=M).to(DEV)
+    want = rows_matmul(c.x, c.w, c.scales, c.biases, group_size=group, epilogue="silu_mul" if silu else None)
+    for i in range(60):
+        got = rows_matmul(c.x, c.w, c.scales, c.biases, group_size=group, epilogue="silu_mul" if silu else None)
+        assert torch.equal(got, want), i

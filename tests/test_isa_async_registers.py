@@ -52,6 +52,20 @@ def test_checks_flag_what_they_are_for():
     assert isa_check.check_wide_stores("global_store_dwordx4 v[2:3], v[4:7], off\nv_mov_b32 v6, v9\n", "x.hip") == 0
 
 
+def test_a_buffer_that_is_asked_for_again_too_early_is_found():
+    name, fill, read = "_ZN1kILb0ELi2ELi1ELi2ELi4ELb0EEEv", "buffer_load_dwordx4 v1, s[0:3], s4 offen lds\n", "ds_read_b128 v[4:7], v1\n"
+    early = f"{name}:\n{fill}s_barrier\n{read}v_mfma\n{fill}s_barrier\n{read}.Lfunc_end0:\n"
+    with pytest.raises(AssertionError, match="asked for again"):
+        isa_check.check_refills(early, "_ZN1kI", 1)
+    isa_check.check_refills(early.replace("v_mfma", "s_barrier\nv_mfma"), "_ZN1kI", 1)
+    isa_check.check_refills(early.replace("Li4E", "Li1E"), "_ZN1kI", 1)  # its own requests
+
+
+@needs_hipcc
+def test_any_rows_kernels_meet_between_the_first_reads_and_the_first_refill():
+    isa_check.check_refills(_text(isa_check.REFILLS[0]), *isa_check.REFILLS[1:])
+
+
 @needs_hipcc
 @pytest.mark.parametrize("source,prefix,count,min_reads", isa_check.KERNELS)
 def test_no_instruction_touches_registers_of_reads_in_flight(source, prefix, count, min_reads):
