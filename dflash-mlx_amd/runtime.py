@@ -109,10 +109,10 @@ def _arm_target_rollback(cache_entries: List[Any]) -> None:
 
 
 def _arm_target_rollback_with_prefix(cache_entries: List[Any], *, prefix_len: int) -> None:
-    prefix_len = int(prefix_len)
-    for cache_entry in cache_entries:
-        arm = getattr(cache_entry, "arm_rollback", None)
-        if arm is not None:
+    armed = [c.arm_rollback for c in cache_entries if hasattr(c, "arm_rollback")]
+    if armed:  # (without a recurrent layer the length is nobody's, and may be anything)
+        prefix_len = int(prefix_len)
+        for arm in armed:
             arm(prefix_len=prefix_len)
 
 

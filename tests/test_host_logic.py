@@ -275,6 +275,17 @@ def test_restore_follows_plan():
                 assert c.offset == 4112
 
 
+def test_arming_asks_nothing_of_a_prefix_that_no_cache_takes():
+    R._arm_target_rollback_with_prefix([KVCache(), object()], prefix_len=None)
+    cache = RecurrentRollbackCache()
+    R._arm_target_rollback_with_prefix([KVCache(), cache], prefix_len=np.int64(7))
+    assert cache._armed
+    broken = RecurrentRollbackCache()
+    broken.arm_rollback = None
+    with pytest.raises(TypeError):
+        R._arm_target_rollback_with_prefix([broken], prefix_len=7)
+
+
 def test_rollback_cache_state_machine_on_host():
     """CPU tensors take the array-op replay (as the reference does without its GPU)."""
     rng = np.random.default_rng(18)
