@@ -490,6 +490,35 @@ def test_arena_takes_per_batch_row_acceptance_and_other_tape_dtypes(native_lib):
         arena.rollback_all(torch.zeros(5, dtype=torch.int32, device=DEV))
 
 
+def test_every_way_back_clears_what_a_cache_holds_for_a_rollback(native_lib, monkeypatch):
+    """The arena's rollback, that of several caches in one launch and a cache's own, with a field that was not there when they were written."""
+    from dflash_mlx_amd import recurrent_rollback_cache as M
+
+    monkeypatch.setitem(M._NO_TRANSIENTS, "_later", None)
+    L, T, Hk, Hv, C = 2, 16, 2, 4, 2 * 2 * 128 + 4 * 128
+    case = make_replay_case(L, batch=1, T=T, Hk=Hk, Hv=Hv, steps=T, seed=175)
+    qkv, conv0 = torch.randn((1, T, C)).to(torch.bfloat16).to(DEV), torch.randn((1, 3, C)).to(torch.bfloat16).to(DEV)
+    arena = RollbackArena(L, batch=1, max_steps=T, Hk=Hk, Hv=Hv, Dk=128, Dv=128, conv_dim=C, device=DEV)
+
+    def armed(caches):
+        for l, c in enumerate(caches):
+            if c._arena is None:
+                c[0], c[1] = conv0, case.state[l].to(DEV)
+            c.arm_rollback()
+            c.record_tape(tape=case.tape[l].to(DEV).float(), k=case.k[l].to(DEV), g=case.g[l].to(DEV), qkv=qkv)
+            c._later = "held"
+        return caches
+
+    own = armed([RecurrentRollbackCache(size=2, conv_kernel_size=4) for _ in range(L)])
+    assert M.rollback_together(own, 3)
+    armed(arena.caches())
+    arena.rollback_all(3)
+    alone = armed([RecurrentRollbackCache(size=2, conv_kernel_size=4)])
+    alone[0].rollback(3)
+    for c in (*own, *arena.caches(), *alone):
+        assert {n: getattr(c, n) for n in M._NO_TRANSIENTS} == M._NO_TRANSIENTS
+
+
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("Dk,Dv,layers,T", [(128, 32, 2, 16), (128, 96, 1, 5), (128, 128, 3, 16), (128, 128, 130, 16), (64, 32, 2, 16),
                                             (64, 64, 3, 1), (64, 192, 2, 16), (64, 64, 130, 9)])
