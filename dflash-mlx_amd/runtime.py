@@ -109,11 +109,15 @@ def _arm_target_rollback(cache_entries: List[Any]) -> None:
 
 
 def _arm_target_rollback_with_prefix(cache_entries: List[Any], *, prefix_len: int) -> None:
-    armed = [c.arm_rollback for c in cache_entries if hasattr(c, "arm_rollback")]
-    if armed:  # (without a recurrent layer the length is nobody's, and may be anything)
-        prefix_len = int(prefix_len)
-        for arm in armed:
-            arm(prefix_len=prefix_len)
+    length = None
+    for cache_entry in cache_entries:
+        try:
+            arm = cache_entry.arm_rollback
+        except AttributeError:
+            continue
+        if length is None:  # (without a recurrent layer it is nobody's, and may be anything)
+            length = int(prefix_len)
+        arm(prefix_len=length)
 
 
 def _clear_rollback_state(cache_entry: Any) -> None:
