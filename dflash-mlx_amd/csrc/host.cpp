@@ -17,7 +17,10 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/Context.h>
 #include <ATen/EmptyTensor.h>
+#include <ATen/record_function.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
@@ -101,11 +104,18 @@ int released(F&& work) {
   return work();
 }
 
-// A new tensor beside `like`: at::empty without the way through the dispatcher, half of its 0.5 us.  A verify block of a recurrent layer
-// with its rollback makes ten.
+// Somebody looks at what goes through the dispatcher - a dispatch mode, a transform, a trace, the profiler - or wants new memory filled.
+bool watched() {
+  return !(c10::impl::tls_local_dispatch_key_set().included_ - c10::default_included_set).empty() || at::hasCallbacks() ||
+         (at::globalContext().deterministicAlgorithms() && at::globalContext().deterministicFillUninitializedMemory());
+}
+
+// A new tensor beside `like`: at::empty without the way through the dispatcher, half of its 0.5 us, where nobody is there to see it.  A verify
+// block of a recurrent layer with its rollback makes ten.
 Tensor fresh(at::IntArrayRef shape, const Tensor& like, at::ScalarType type) {
   c10::Allocator* const allocator = like.storage().allocator();
-  if (allocator == nullptr || c10::hip::current_device() != like.device().index()) return at::empty(shape, like.options().dtype(type));
+  if (allocator == nullptr || c10::hip::current_device() != like.device().index() || watched())
+    return at::empty(shape, like.options().dtype(type));
   return Tensor(at::detail::empty_generic(shape, allocator, c10::DispatchKeySet(c10::DispatchKey::CUDA), type, std::nullopt));
 }
 Tensor fresh(at::IntArrayRef shape, const Tensor& like) { return fresh(shape, like, like.scalar_type()); }

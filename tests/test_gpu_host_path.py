@@ -325,6 +325,37 @@ def test_block_from_the_joint_product(monkeypatch, B, S, Hk, Hv, D, record):
 
 
 @pytest.mark.gpu
+def test_results_go_through_the_dispatcher_where_somebody_looks(monkeypatch):
+    """A dispatch mode and the profiler see the results that the launches make, and memory is filled where that is asked for."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    monkeypatch.setenv("DFLASH_VERIFY_QMM", "1")
+    w, s, b = _triple(1024, 512, 64, BF)
+    x = _rows((1, 16), 1024, BF)
+    want = VQ.verify_matmul(x, w, s, b)
+    seen = []
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    with Mode():
+        got = VQ.verify_matmul(x, w, s, b)
+    assert torch.equal(got, want) and any(name.startswith("aten.empty") for name in seen)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+        got = VQ.verify_matmul(x, w, s, b)
+    assert torch.equal(got, want) and any(e.key == "aten::empty" for e in prof.key_averages())
+    before = torch.are_deterministic_algorithms_enabled()
+    torch.use_deterministic_algorithms(True)
+    try:
+        got = VQ.verify_matmul(x, w, s, b)
+    finally:
+        torch.use_deterministic_algorithms(before)
+    assert torch.equal(got, want)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("rows", [1, 15, 16, 17, 40])
 @pytest.mark.parametrize("N", [16, 32, 48, 512])
 def test_projection_module(monkeypatch, rows, N):
