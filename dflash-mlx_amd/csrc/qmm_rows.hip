@@ -573,6 +573,7 @@ struct Shape {
   int together;        // workgroups that a CU has room for
   double alone, busy;  // us per stage: of one workgroup on a CU, and of each where they share it
   double start;        // us before the first product and behind the last one
+  double brief;        // the same of a call of up to kBriefK
   int most;            // slices
   double loose;        // us more where scales come through registers
   const void* kernel[2][3];  // [fp16][plain, scales of the other type, silu-mul]; null: there is none, or it was never the one to take
@@ -580,8 +581,8 @@ struct Shape {
   int columns() const { return 32 * nt * w; }
 };
 template <int MT, int NT, int W, int KG, bool MIXED = false, bool PLAIN = true>
-Shape shape(int together, double alone, double busy, double start, int most = 16, double loose = 0.0) {
-  Shape s{MT, NT, W, KG, Tile<MT, NT, W, KG>::kLdsBytes, together, alone, busy, start, most, loose, {}};
+Shape shape(int together, double alone, double busy, double start, double brief, int most = 16, double loose = 0.0) {
+  Shape s{MT, NT, W, KG, Tile<MT, NT, W, KG>::kLdsBytes, together, alone, busy, start, brief, most, loose, {}};
   if constexpr (PLAIN) {
     s.kernel[0][0] = (const void*)qmm_rows_kernel<false, false, MT, NT, W, KG, false>;
     s.kernel[1][0] = (const void*)qmm_rows_kernel<true, true, MT, NT, W, KG, false>;
@@ -603,13 +604,15 @@ Shape shape(int together, double alone, double busy, double start, int most = 16
 constexpr int kShapes = 18;
 const Shape* shapes() {
   static const Shape all[kShapes] = {
-      shape<1, 1, 1, 8>(1, 0.597, 0.571, 4.87, 16, 0.17), shape<2, 1, 1, 8>(1, 0.908, 0.454, 5.30),
-      shape<1, 1, 2, 4, true>(2, 0.559, 0.472, 3.63, 16, 2.02), shape<2, 1, 2, 4>(1, 0.695, 0.447, 3.67, 16, 1.08),
-      shape<3, 1, 2, 4>(1, 0.860, 0.307, 4.55, 16, 1.8), shape<1, 2, 2, 4>(1, 0.984, 0.508, 3.75, 16, 1.14),
-      shape<2, 2, 2, 4, true>(1, 1.105, 0.401, 4.86, 16, 0.81), shape<3, 2, 2, 4>(1, 1.415, 0.390, 5.17), shape<1, 2, 4, 2>(2, 0.902, 0.767, 3.81, 16, 0.75),
-      shape<3, 2, 4, 2>(1, 1.269, 0.363, 5.50), shape<4, 2, 4, 2, true>(1, 1.469, 0.524, 6.60), shape<4, 2, 2, 2>(1, 0.925, 0.546, 3.81),
-      shape<2, 2, 4, 1>(2, 0.631, 0.528, 4.78), shape<4, 2, 4, 1>(2, 0.880, 0.761, 4.92), shape<1, 1, 1, 4>(3, 0.451, 0.334, 3.53, 6, 0.36),
-      shape<2, 1, 1, 4>(2, 0.607, 0.452, 3.78, 6, 0.45), shape<1, 2, 1, 4>(2, 0.730, 0.491, 2.86, 6, 0.62), shape<2, 2, 1, 4, false, false>(1, 0.805, 0.626, 3.57, 6)};
+      shape<1, 1, 1, 8>(1, 0.597, 0.571, 4.87, 4.74, 16, 0.17), shape<2, 1, 1, 8>(1, 0.908, 0.454, 5.30, 5.51),
+      shape<1, 1, 2, 4, true>(2, 0.559, 0.472, 3.63, 4.33, 16, 2.02), shape<2, 1, 2, 4>(1, 0.695, 0.447, 3.67, 4.81, 16, 1.08),
+      shape<3, 1, 2, 4>(1, 0.860, 0.307, 4.55, 5.32, 16, 1.8), shape<1, 2, 2, 4>(1, 0.984, 0.508, 3.75, 5.05, 16, 1.14),
+      shape<2, 2, 2, 4, true>(1, 1.105, 0.401, 4.86, 5.96, 16, 0.81), shape<3, 2, 2, 4>(1, 1.415, 0.390, 5.17, 6.86),
+      shape<1, 2, 4, 2>(2, 0.902, 0.767, 3.81, 4.77, 16, 0.75), shape<3, 2, 4, 2>(1, 1.269, 0.363, 5.50, 6.39),
+      shape<4, 2, 4, 2, true>(1, 1.469, 0.524, 6.60, 7.93), shape<4, 2, 2, 2>(1, 0.925, 0.546, 3.81, 5.77),
+      shape<2, 2, 4, 1>(2, 0.631, 0.528, 4.78, 4.93), shape<4, 2, 4, 1>(2, 0.880, 0.761, 4.92, 5.68),
+      shape<1, 1, 1, 4>(3, 0.451, 0.334, 3.53, 3.89, 6, 0.36), shape<2, 1, 1, 4>(2, 0.607, 0.452, 3.78, 4.35, 6, 0.45),
+      shape<1, 2, 1, 4>(2, 0.730, 0.491, 2.86, 4.29, 6, 0.62), shape<2, 2, 1, 4, false, false>(1, 0.805, 0.626, 3.57, 4.95, 6)};
   return all;
 }
 
@@ -623,6 +626,7 @@ struct Plan {
 };
 
 constexpr size_t kCounterBytes = 64 * 1024;
+constexpr int kBriefK = 640;
 
 bool covers(int M, int K, int N, int group_size, bool mixed, int epilogue) {
   if (epilogue != DFLASH_QMM_EPILOGUE_NONE && (epilogue != DFLASH_QMM_EPILOGUE_SILU_MUL || mixed || N % 32 != 0)) return false;
@@ -642,9 +646,16 @@ bool scales_through_registers(int K, int group_size, int kg) { return (K / group
 // 128 from 1664 to 11904, 320 to 3072 columns, 16 to 200 rows): what is picked of them is within 1.3 % of the best on average and 10 % at worst, without
 // it 7.5 and 26 % (17 rows of 7808 x 1024 in groups of 128 11.4 -> 9.9 us, 64 of 10112 x 320 12.5 -> 11.0, 100 of 11904 x 2048 19.1 -> 17.6).
 // Four waves along K with no more than four stages and nothing to add up start sooner than the line through longer calls has it: 64 calls of K up to 1472 within
-// 2 % of the best, 4 % without that (24 rows of 384 x 224 5.4 -> 4.5 us, 24 of 512 x 1024 5.2 -> 4.6); and so do eight with one column of tiles each (58 rows of
-// 3072 x 4000 in groups of 128 10.9 -> 9.2; 116 calls of layers of 1024 to 5120 columns, 33 to 450 rows: within 0.8 % of the best in the mean).  Against the kernel whose waves met behind a stage's last step, 600 calls of such
-// layers: 0.96 of its time in the mean; up to 4 % more for K = 512 (0.15 us), up to 10 % for single ones whose choice is not the best (142 rows of 3968 x 1792).
+// 2 % of the best, 4 % without that; and so do eight with one column of tiles each (58 rows of
+// 3072 x 4000 in groups of 128 10.9 -> 9.2; 116 calls of layers of 1024 to 5120 columns, 33 to 450 rows: within 0.8 % of the best in the mean).
+// Calls of up to kBriefK are a start, an end and a few stages, and the line through longer calls has their starts wrong by -0.1 to 1.8 us, as the shape is
+// (300 rows of 640 x 4096 8.7 -> 10.3 us, 450 of 512 x 4096 with the activation 9.0 -> 10.8 when that line was fitted anew): a line of their own, fitted to the whole
+// products of 394 such calls, 17 to 1000 rows, 256 to 8640 columns.  What it picks of 260 others is within 0.3 % of the best in the mean and 9 % at worst, by the
+// line of longer calls of the 244 first ones 3.8 and 25 %.
+// Against the kernel whose waves met behind a stage's last step, 620 calls of layers of 1024 to 5120 columns and of K 256 to 1024, 17 to 1024 rows: 0.96 of its time in
+// the mean, 15 of them slower by more than 3 %, 9 % at most (21 rows of 1792 x 1952 in groups of 128 6.8 -> 7.4; 80 of 15488 x 4608 30.0 -> 31.7, 40 of 4096 x 23552 with the
+// activation 24.7 -> 26.1: the line has another shape, or the kernel with weights in registers, too fast).  K of 384 and 640, where four waves along K bring their scales
+// through registers, up to 6 % (64 rows of 384 x 8192 5.2 -> 5.5).
 // Slices only while all of them find room at once.  Of more tiles than that, those of the last, incomplete round may be
 // cut, with the tile left as it is (5120 x 34816 over 1024 rows: 1088 tiles, two to a CU, the last 64 in slices, 344 us; uncut 382).
 Plan make_plan(int M, int K, int N, int group_size, int cus, bool fp16, bool mixed, bool silu_mul) {
@@ -658,11 +669,18 @@ Plan make_plan(int M, int K, int N, int group_size, int cus, bool fp16, bool mix
       return rounds * sh.start + stages * std::max(sh.alone * rounds, sh.busy * on_a_cu);
     };
     const int rounds = p.whole / slots;
-    double us = stretch(rounds * sh.together, p.stages) + stretch(ceil_div(parts, cus), ceil_div(p.stages, p.slices));
-    us *= 1 + 0.17 * (std::min(1.0, (double)p.grid / cus) - 0.5);
-    us += 0.76 + (silu_mul ? 0.84 : 0.0);
-    if (scales_through_registers(K, group_size, sh.kg)) us += sh.loose;
-    if (p.slices == 1 && sh.w == 1 && sh.nt == 1 && (sh.kg == 4 ? p.stages <= 4 : sh.mt == 1)) us -= 0.35;
+    const double loops = stretch(rounds * sh.together, p.stages) + stretch(ceil_div(parts, cus), ceil_div(p.stages, p.slices));
+    const double full = std::min(1.0, (double)p.grid / cus);
+    double us;
+    if (K <= kBriefK) {
+      const int on_a_cu = rounds * sh.together + ceil_div(parts, cus), in_turn = rounds + ceil_div(ceil_div(parts, cus), sh.together);
+      us = sh.brief + 1.95 * (in_turn - 1) + 0.45 * (on_a_cu - in_turn) + 1.08 * (loops - in_turn * sh.start) + 0.65 * full + (silu_mul ? 0.74 : 0.0);
+      if (scales_through_registers(K, group_size, sh.kg)) us += 0.16;
+    } else {
+      us = loops * (1 + 0.17 * (full - 0.5)) + 0.76 + (silu_mul ? 0.84 : 0.0);
+      if (scales_through_registers(K, group_size, sh.kg)) us += sh.loose;
+    }
+    if (K > kBriefK && p.slices == 1 && sh.w == 1 && sh.nt == 1 && (sh.kg == 4 ? p.stages <= 4 : sh.mt == 1)) us -= 0.35;
     const int pieces = silu_mul ? sh.mt : sh.mt * sh.nt, at_once = silu_mul && (sh.mt == 1 || sh.mt == 4) ? 2 : 4;
     if (p.slices > 1)
       us += 0.96 + 0.806 * ceil_div(pieces, sh.kg) * ceil_div(p.slices, at_once) + 0.352 * parts * (sh.rows() * 8.0 * sh.columns()) / 3e6;
