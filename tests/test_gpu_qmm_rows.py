@@ -34,7 +34,7 @@ def test_rows_against_fp64(native_lib, M, K, N, group, dtype):
     assert (y.double() - exact).norm() <= eps * exact.norm()
 
 
-# (with MORE_SHAPES) a call for every tile shape there is: K that ends inside a stage, N and M that end inside a tile, whole and sliced
+# (with MORE_SHAPES and REST_SHAPES) a call for every tile shape there is: K that ends inside a stage, N and M that end inside a tile, whole and sliced
 TILE_SHAPES = [(17, 288, 16, 32), (17, 2080, 48, 32), (20, 96, 528, 32), (17, 160, 8208, 32), (17, 96, 6160, 32), (33, 288, 2064, 32),
                (45, 96, 2064, 32), (33, 160, 12432, 32), (65, 160, 3088, 32), (129, 160, 6160, 32), (129, 96, 12432, 32), (65, 96, 1552, 32),
                (400, 160, 8208, 32), (300, 96, 12432, 32), (97, 4416, 2064, 64), (200, 3136, 1552, 64), (1000, 1664, 5136, 128)]
@@ -210,6 +210,20 @@ MORE_SHAPES_SILU = [(65, 2464, 8416, 32), (17, 3552, 11488, 32), (65, 288, 11040
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M,K,N,group,silu", [(*t, False) for t in MORE_SHAPES] + [(*t, True) for t in MORE_SHAPES_SILU])
 def test_tile_shapes_of_four_and_eight_waves(native_lib, M, K, N, group, silu, dtype):
+    test_every_tile_shape_at_its_edges(native_lib, M, K, N, group, silu, dtype)
+
+
+# the shapes, whole and sliced, that the lists above do not reach as the choice is fitted now
+REST_SHAPES = [(400, 5760, 144, 64), (65, 3616, 4240, 32), (97, 416, 8592, 32), (33, 5728, 5488, 32), (130, 960, 10992, 32), (17, 4416, 10912, 64),
+               (400, 736, 13712, 32), (600, 1376, 13216, 32), (600, 96, 6432, 32), (97, 2880, 8288, 32), (300, 192, 1632, 32), (33, 5600, 1376, 32)]
+REST_SHAPES_SILU = [(17, 192, 16736, 32), (33, 416, 17696, 32), (33, 3872, 8416, 32), (65, 992, 15136, 32), (65, 4672, 2848, 32),
+                    (17, 2592, 16416, 32), (193, 224, 18720, 32), (65, 3424, 16608, 32), (200, 736, 22176, 32), (97, 4128, 16928, 32),
+                    (65, 352, 21984, 32), (97, 3008, 8416, 64), (33, 4960, 16480, 32), (1000, 704, 16544, 32)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,K,N,group,silu", [(*t, False) for t in REST_SHAPES] + [(*t, True) for t in REST_SHAPES_SILU])
+def test_tile_shapes_that_the_choice_has_for_other_sizes(native_lib, M, K, N, group, silu, dtype):
     test_every_tile_shape_at_its_edges(native_lib, M, K, N, group, silu, dtype)
 
 
