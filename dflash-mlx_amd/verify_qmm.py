@@ -166,8 +166,10 @@ def _launch(x2: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: tor
 
 def verify_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
                   *, transpose: bool = True, group_size: int = 64, bits: int = 4) -> torch.Tensor:
-    # (the native call looks at sizes, types and rows itself, and answers None to what is not its own)
-    if x.is_cuda and bits == 4 and transpose and is_enabled() and _native.env(b"DFLASH_VERIFY_VARIANT") is None:
+    # (the native call looks at sizes, types and rows itself, and answers None to what is not its own; without a library a call outside the
+    # gate is still the stock operator's)
+    if (x.is_cuda and bits == 4 and transpose and is_enabled() and _native.env(b"DFLASH_VERIFY_VARIANT") is None
+            and _native.is_built()):
         y = _native.host().qmm_m16(x, w, scales, biases, group_size, _kernel_select(), _WORKSPACES)
         if y is not None:
             return y

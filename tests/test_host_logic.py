@@ -92,6 +92,22 @@ def test_eligible_call_on_host_tensors_fails_loudly(verify_env):
         VQ.verify_matmul(c.x, c.w, c.scales, c.biases)
 
 
+def test_ineligible_call_on_a_device_asks_nothing_of_a_library_that_is_not_there(verify_env, monkeypatch, tmp_path):
+    """Calls outside the verify gate go to the stock operator's array form; eligible ones fail loudly as above."""
+    class OnDevice(torch.Tensor):
+        is_cuda = property(lambda self: True)
+
+    for name, value in (("_lib", None), ("_host", None), ("LIB_PATH", str(tmp_path / "nope.so"))):
+        monkeypatch.setattr(nat, name, value)
+    for rows in (4, 40):
+        c = make_qmm_case(256, 32, 7, M=rows)
+        got = VQ.verify_matmul(c.x.as_subclass(OnDevice), c.w, c.scales, c.biases)
+        assert torch.equal(got.as_subclass(torch.Tensor), quantized_matmul(c.x, c.w, c.scales, c.biases))
+    c = make_qmm_case(512, 64, 7)
+    with pytest.raises(nat.NativeLibraryError):
+        VQ.verify_matmul(c.x.as_subclass(OnDevice), c.w, c.scales, c.biases)
+
+
 def test_verify_qmm_takes_group_size_and_bits_positionally(verify_env):
     """verify_qmm(x, w_packed, scales, biases, group_size, bits): the spelling of the hot path's
     name; ineligible calls (4 rows here) go to the stock operator like verify_matmul's."""
