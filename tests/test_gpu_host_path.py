@@ -322,6 +322,7 @@ def test_block_from_the_joint_product(monkeypatch, B, S, Hk, Hv, D, record):
     assert made(wide.half()) is None and made(wide[0]) is None and made(wide[..., :cut[-1] - 1]) is None
     assert made(wide, bounds=bounds[:3]) is None and made(wide, bounds=[(lo + 4, hi + 4) for lo, hi in bounds]) is None
     assert made(wide, bounds=bounds[:3] + [(cut[-1], cut[-1] + 99)]) is None and made(_at(wide, 1)) is None
+    assert made(wide, bounds=[(lo - 8, hi - 8) for lo, hi in bounds]) is None  # (of the right widths, before the product)
 
 
 @pytest.mark.gpu
