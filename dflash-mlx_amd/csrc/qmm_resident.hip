@@ -129,7 +129,7 @@ int row_tiles_of(int M) { return M <= 32 ? 2 : (M + 15) / 16; }
 // Up to 80 rows: the slices of K that take the least time by a model fitted to 328 combinations of 25 matrices, 32 to 80 rows and 1 to 6
 // slices (4.7 % rms, what it picks is within 3 % of the best of its call).  The caller takes this kernel where that is less than what the any-rows
 // product is expected to take: 17 - 32 rows of most matrices (4096 x 4096 10.3 -> 7.5 us, 4096 x 12288 19.9 -> 12.9, 5120 x 34816 with the activation 40.7 -> 30.5),
-// 33 - 48 of those but the largest (4096 x 6144 15.1 -> 11.1), up to 80 of fewer (80 rows of 4096 x 6144 17.5 -> 13.8).  The others stay there (4096 x 24576
+// 33 - 48 of those too (4096 x 6144 15.1 -> 11.1; of 5120 x 34816 with the activation as long as there, 44), up to 80 of fewer (80 rows of 4096 x 6144 17.5 -> 13.8).  The others stay there (4096 x 24576
 // with the activation, 80 rows: 30.8 there, 33.8 here: sums of eight waves for every 16 x 16 piece, and x of 80 rows leaves room for two chunks a wave only).
 // Of 193 calls of 18 matrices what is taken is within 0.2 % of the better of the two in the mean and 4 % at most (2.5 and 33 % before the factor below).
 bool qmm_resident_rows_plan(int M, int K, int N, int group_size, bool silu_mul, int* chunks_out, int* slices_out, double* us_out, size_t* workspace) {

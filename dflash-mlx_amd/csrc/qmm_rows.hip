@@ -30,15 +30,16 @@
 // Measured (us, group 64; before: 16 x 16 x 32 instructions, loads to registers): 1024 rows of 5120 x 34816 with the
 // activation 398 -> 335 (1.09 PFLOP/s), 17408 x 5120 207 -> 184, 5120 x 12352 164 -> 134; 200 rows of 4096 x 4096 22.6 -> 17.5; 77 rows
 // of 4096 x 24576 with the activation 35.7 -> 29.0, 12288 x 4096 24.9 -> 20.9; 20 rows of 5120 x 12352 21.4 -> 18.3, of 1024 x 1024 5.9 -> 5.7.
-// Still slower than that form: 17 to 32 rows of squares of 2048 to 5120 4 to 6 %, 17 to 48 rows of 5120 x 34816 with the activation
-// 2 to 9 % (40 rows 40.4 -> 43.9), 77 to 128 rows of 3072 x 1024 6 to 9 %.
+// Slower than that form: 77 to 128 rows of 3072 x 1024, 6 to 9 % when that was measured.  (17 to 48 rows of nearly every matrix are now the kernel's with
+// weights in registers, qmm_resident.hip.)
 // With the waves meeting before a stage's last step, and scales that go past the registers, before / after: 400 rows of 4096 x 2304 19.5 -> 16.9, 600
 // of 3072 x 9216 48.4 -> 45.6, 77 of 12288 x 4096 23.5 -> 22.4, 1024 of 5120 x 12352 136.4 -> 132.8; 16 calls of 20 to 1024 rows 2 %.
-// What bounds it at many rows: the matrix pipes are busy for 60 to 66 % of the cycles at 2.0 to 2.1 of 2.4 GHz (power); with no requests
-// to memory at all the same loop is 15 to 20 % faster, with no dequantisation on top 2 to 10 %.  At few rows:
-// 3300 cycles of setup, requests and their latency before the first product, 5000 and more for the slices, and between them the issue port: two waves
-// of (3,2,2,4) on a SIMD hold it for 1930 of a stage's 3100 cycles (v_fma_mix and conversions take it for 4.3 cycles, v_fma_f32 and shifts for 2.4), a wave
-// that is alone there issues every 5 cycles.  Turns at priority between the two change nothing.
+// What bounds it at many rows: the matrix pipes are busy for 60 to 67 % of the cycles at 2.0 to 2.1 of 2.4 GHz (power); with no requests
+// to memory at all the loop that met behind a stage's last step was 15 to 20 % faster, with no dequantisation on top 2 to 10 %.  At few rows, by stamps
+// in that loop: 3300 cycles of setup, requests and their latency before the first product, 5000 and more for the slices, and between them the issue port: two
+// waves of (3,2,2,4) on a SIMD held it for 1930 of a stage's 3100 cycles (v_fma_mix and conversions take it for 4.3 cycles, v_fma_f32 and shifts for 2.4), a
+// wave that is alone there issues every 5 cycles.  Turns at priority between the two changed nothing.  Counters of the loop as it is, 77 rows of
+// 4096 x 24576 with the activation / of 12288 x 4096: vector 47 / 34 % of the time that the SIMDs hold waves, matrix 39 / 23, waves wait 32 / 44.
 #include "glue_device.h"
 
 #include "qmm_stream_device.h"

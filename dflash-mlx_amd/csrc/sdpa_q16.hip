@@ -214,8 +214,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     // them, the last of which also writes them to the cache; all while the first tiles are on their way.  A launch of its own for it (attn_prepare_kernel,
     // whose bits these are) took 4 to 5 us and its place in the queue.  Here every range does it again, bound by its vector
     // instructions: 1.5 us of a launch with heads of 128, 3.2 of 256 (4.7 with one wave for all of a head's queries and the
-    // powers computed by every thread).  Layer calls, us, before and with it: 4 112 keys of 8 x 256 48.1 -> 46.4, 32 716 89.5 ->
-    // 88.7; of calls that the host bounds (five launches, now four) 8 299 keys of 8 x 128 43.4 -> 36.0, 2 016 of 2 x 256 43.2 -> 35.8.
+    // powers computed by every thread).  Layer calls, us, before and with it: 4 112 keys of 8 x 256 48.5 -> 46.9, 32 716 92.3 ->
+    // 89.1 (with the third tile on its way); of calls that the host bounds (five launches, now four) 9 152 keys of 8 x 128 43.3 -> 36.1, 2 343 of 2 x 256 43.1 -> 34.8.
     constexpr int PER = D / 64, kRowsPerWave = 16 / (kThreads / 64);
     const BlockArgs& p = a.block;
     const int half = p.half, pitch = half + kTurnPad;
